@@ -245,6 +245,23 @@ __device__ __forceinline__ void build_tile_lists(uint32_t U, uint32_t p0, uint32
     }
 }
 #endif
+// the tile lists as a launch of their own, for callers whose pair sort did not write them
+hipError_t launch_build_tiles(const uint32_t *expert_start, const uint32_t *n_unique, uint32_t n_pairs, const TileLists &tl, hipStream_t s);
+// A chunk on experts without tile-major copies (redhip_tiles.hip): raw GGUF rows or packed IQ2_XXS rows (`packed`), every matrix 16-byte
+// aligned. Expert uid[u]: gate matrix at gate + uid[u] * stride, up matrix up_delta behind it, down matrix at down + uid[u] * down_stride;
+// the shared expert's slot gate | up | down at `shared` when tl.shared_ntok asks for its tiles. x as fp16 halves in; act: f32
+// [ntok * top_k + shared tokens][ffn] scratch; outputs tmp / sh_tmp as launch_prefill_packed leaves them for launch_batch_combine.
+struct StagedExperts {
+    const void *gate, *down, *shared;
+    uint64_t stride, down_stride, up_delta;
+    uint32_t gate_up_type, down_type;
+    const int8_t *gate_up_grid, *down_grid;
+    bool packed;
+};
+bool staged_tiles_supported(uint32_t gate_up_type, uint32_t down_type, uint32_t hidden, uint32_t ffn, uint32_t n_expert, bool packed);
+hipError_t launch_staged_tiles(const StagedExperts &x, const uint32_t *uid, const uint32_t *expert_start, const uint32_t *pair_token, const uint32_t *n_unique,
+                               const TileLists &tl, bool tiles_built, const void *xh, const void *xl, const int *xexp, float *act, float *tmp, float *sh_tmp,
+                               uint32_t hidden, uint32_t ffn, uint32_t top_k, uint32_t ntok, uint32_t n_expert, hipStream_t s);
 // Device scratch of the pair sort of large chunks (more than 512 tokens), which runs as three launches over blocks of kGroupSpan tokens:
 // count_blk / blk_off [blocks][n_expert], first_key / expert_base [n_expert]. All zero before the first use (the sort leaves first_key
 // zero again); `blocks` = the capacity in blocks.

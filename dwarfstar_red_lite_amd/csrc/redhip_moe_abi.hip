@@ -177,15 +177,22 @@ struct Moe {
         const bool gu_cb = gu_type == T_IQ2_XS || gu_type == T_IQ1_M, dn_cb = dn_type == T_IQ2_XS || dn_type == T_IQ1_M;
         return mixed && gu_cb && dn_cb && (cfg.ffn == 256u || cfg.ffn == 512u) && cfg.hidden / 512u <= 4u && cfg.max_tokens > 8u;
     }
-    // a chunk on a mixed layout that has no tile kernels (ffn > 512, or IQ2_XS / IQ1_M gate/up beside another down format) runs as slices
-    // of 8 tokens on the grouped small-batch kernels, far ahead of the generic per-pair kernels on raw rows
+    // a chunk on a layout without tile-major copies (ffn > 512, or IQ2_XS / IQ1_M gate/up beside another down format): the tile kernels that
+    // take rows through LDS - the raw ones of mixed layouts, the packed row-major ones of all-IQ2_XXS layers
+    bool staged_chunk(uint32_t ntok) const {
+        if (ntok <= 8u || tiles_resident() || stream_tiles_resident()) return false;
+        return fused ? rowmajor_down() && staged_tiles_supported(gu_type, dn_type, cfg.hidden, cfg.ffn, cfg.n_expert, true)
+                     : mixed && keep_raw() && staged_tiles_supported(gu_type, dn_type, cfg.hidden, cfg.ffn, cfg.n_expert, false);
+    }
+    // a chunk on a mixed layout that has no tile kernels at all runs as slices of 8 tokens on the grouped small-batch kernels, far ahead of
+    // the generic per-pair kernels on raw rows
     static constexpr uint32_t kSlice = 8u;
     // So does every layout from 9 to 16 tokens: two small batches are quicker than one chunk, whose tile kernels leave most workgroups
     // without work at that size.
     bool sliced(uint32_t ntok) const {
         if (ntok <= kSlice || small_batch(ntok, true)) return false;      // (one small batch: up to 32 tokens behind the layer's own router)
         if (ntok <= 2u * kSlice && (small_batch(kSlice) || grouped_mixed(kSlice))) return true;
-        return mixed && !tiles_resident() && !stream_chunk(ntok) && grouped_mixed(kSlice);
+        return mixed && !tiles_resident() && !stream_chunk(ntok) && !staged_chunk(ntok) && grouped_mixed(kSlice);
     }
     // the workspace entries a caller can read back (redhip_moe_last_route) of the slice that starts at token t0 sit at their place in the chunk
     void shift_route_outputs(int64_t t0) {
@@ -300,10 +307,11 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
         // the shared expert as dense f32 products on the fp32 matrix units, started before the pair sort (one workgroup on an idle machine;
         // the many-workgroup sort of a large chunk then queues behind the dense tiles - 73 against 22 us at 2048 tokens - but started
         // behind the sort the dense products slow the down tiles by more: 787 against 760 us per chunk)
-        const bool dense_shared = (stream_tiles || (m->mixed_chunk(ntok) && Ld.dense_gu && m->side));
+        const bool staged = !stream_tiles && m->staged_chunk(ntok);
+        const bool dense_shared = (stream_tiles || ((m->mixed_chunk(ntok) || (staged && m->mixed)) && Ld.dense_gu && m->side));
         if (dense_shared && !fork_shared_dense(m, Ld, x, ntok, s)) return 0;
         // the pair sort also writes the tile lists of the tile kernels that follow (all-IQ2_XXS layers: with the shared expert's tiles)
-        const bool tile_path = !m->small_batch(ntok) && (m->packed_path(ntok) || stream_tiles || m->mixed_chunk(ntok));
+        const bool tile_path = !m->small_batch(ntok) && (m->packed_path(ntok) || stream_tiles || staged || m->mixed_chunk(ntok));
         const TileLists tl{m->tile_group, m->tile_pair0, m->tile_n, m->n_tiles, prefill_tile_bound(ntok, c.top_k, c.n_expert), m->packed_path(ntok) ? ntok : 0u};
         const bool tiles_built = !grouped && tile_path;
         if (!grouped) {
@@ -319,6 +327,19 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
             return 1;
         }
         if (m->small_batch(ntok)) { moe_err("internal: a small batch reached the expert kernels without its pass list"); return 0; }
+        if (staged && (m->fused || dense_shared)) {
+            const Layer &L = Ld;
+            const uint8_t *rows = m->fused ? L.packed : L.experts;
+            const uint64_t stride = m->fused ? m->packed_stride : m->expert_stride;
+            const StagedExperts x{rows, rows + 2u * m->gate_bytes, m->fused ? L.shared_packed : nullptr, stride, stride, m->gate_bytes, m->gu_type, m->dn_type, m->gu_grid, m->dn_grid, m->fused};
+            HIP_OK(launch_staged_tiles(x, m->uid, m->expert_start, m->pair_token, m->n_unique, tl, tiles_built, m->xh, m->xl, m->xexp, m->act, m->tmp, m->sh_tmp,
+                                       c.hidden, c.ffn, c.top_k, ntok, c.n_expert, s), "staged tile launch");
+            if (dense_shared && !join_shared_dense(m, s)) return 0;
+            prof_set_stage(ST_BATCH_COMBINE);
+            HIP_OK(launch_batch_combine(m->tmp, m->pair_weight, m->tok_pair, ntok, c.top_k, m->sh_tmp, m->scalar, c.hidden, out, s), "batched combine launch");
+            prof_set_stage(ST_OTHER);
+            return 1;
+        }
         if (m->packed_path(ntok)) {     // prefill chunk: tiles of 16 pairs per expert on the MFMA units
             const Layer &L = m->layers[layer];
             HIP_OK(launch_prefill_packed(L.packed, m->expert_stride, L.shared_packed, L.tiled, L.shared_tiled, m->uid, m->expert_start, m->pair_token, m->n_unique,
@@ -885,7 +906,7 @@ int redhip_moe_experts(redhip_moe_t h, uint32_t layer, const float *x_dev, uint3
         GuardScope(uint32_t n, uint32_t *st) { route_guard() = RouteGuard{n, st}; }
         ~GuardScope() { route_guard() = RouteGuard{}; }
     } guard_scope(m->cfg.n_expert, m->status);
-    if (m->packed_path(ntok) || m->small_batch_mixed(ntok) || m->mixed_chunk(ntok) || m->stream_chunk(ntok)) {
+    if (m->packed_path(ntok) || m->small_batch_mixed(ntok) || m->mixed_chunk(ntok) || m->stream_chunk(ntok) || m->staged_chunk(ntok)) {
         const Layer &L = m->layers[layer];
         const uint32_t nv = m->cfg.hidden / 256u;
         // batches whose pairs are grouped by expert next: the pair sort rides in the same launch as one more workgroup

@@ -34,6 +34,11 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const uint32_t *exper
     build_tile_lists(U, p0, n, P, tl, wave_total);
 }
 
+hipError_t launch_build_tiles(const uint32_t *expert_start, const uint32_t *n_unique, uint32_t n_pairs, const TileLists &tl, hipStream_t s) {
+    REDHIP_LAUNCH(build_tiles_kernel, dim3(1), dim3(1024), 0, s, expert_start, n_unique, n_pairs, tl);
+    return hipGetLastError();
+}
+
 struct PrefillArgs {
     const uint8_t *experts;
     uint64_t stride;
@@ -1368,8 +1373,7 @@ hipError_t launch_prefill_gateup_tiled(const void *tiled_experts, uint64_t strid
     if (!tiles_built) {
         prof_set_stage(ST_GROUP);
         const TileLists tl{tile_group, tile_pair0, tile_n, n_tiles, prefill_tile_bound(ntok, top_k, n_expert), 0u};      // no shared tiles
-        REDHIP_LAUNCH(build_tiles_kernel, dim3(1), dim3(1024), 0, s, expert_start, n_unique, P, tl);
-        e = hipGetLastError();
+        e = launch_build_tiles(expert_start, n_unique, P, tl, s);
         if (e != hipSuccess) return e;
     }
     PrefillArgs a{nullptr, stride, nullptr, uid, pair_token, n_unique, tile_group, tile_pair0, tile_n, n_tiles, static_cast<const _Float16 *>(xh),
@@ -1397,8 +1401,7 @@ hipError_t launch_prefill_streams(uint32_t gate_up_type, const int8_t *gate_up_g
     if (!tiles_built) {
         prof_set_stage(ST_GROUP);
         const TileLists tl{tile_group, tile_pair0, tile_n, n_tiles, prefill_tile_bound(ntok, top_k, n_expert), 0u};      // no shared tiles
-        REDHIP_LAUNCH(build_tiles_kernel, dim3(1), dim3(1024), 0, s, expert_start, n_unique, P, tl);
-        e = hipGetLastError();
+        e = launch_build_tiles(expert_start, n_unique, P, tl, s);
         if (e != hipSuccess) return e;
     }
     PrefillArgs a{nullptr, packed_stride, nullptr, uid, pair_token, n_unique, tile_group, tile_pair0, tile_n, n_tiles, static_cast<const _Float16 *>(xh),
@@ -1452,8 +1455,7 @@ hipError_t launch_prefill_packed(const void *experts, uint64_t stride, const voi
     if (!tiles_built) {
         prof_set_stage(ST_GROUP);
         const TileLists tl{tile_group, tile_pair0, tile_n, n_tiles, prefill_tile_bound(ntok, top_k, n_expert), with_shared ? ntok : 0u};
-        REDHIP_LAUNCH(build_tiles_kernel, dim3(1), dim3(1024), 0, s, expert_start, n_unique, P, tl);
-        e = hipGetLastError();
+        e = launch_build_tiles(expert_start, n_unique, P, tl, s);
         if (e != hipSuccess) return e;
     }
     PrefillArgs a{static_cast<const uint8_t *>(experts), stride, static_cast<const uint8_t *>(shared), uid, pair_token, n_unique,

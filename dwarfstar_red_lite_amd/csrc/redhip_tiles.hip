@@ -1,0 +1,630 @@
+// Chunks of tokens on experts that have no tile-major copy: the (token, expert) pairs of one expert are cut into tiles of up to 32 pairs
+// (build_tile_lists) and multiplied on v_mfma_f32_16x16x32_f16 straight from rows as they lie in memory - raw GGUF blocks of IQ2_XXS,
+// IQ2_XS, IQ1_M and (down) IQ3_S, or packed IQ2_XXS rows.
+//
+// What bounds these kernels is the decode (LDS table reads and vector issue; every weight is decoded once per tile), so the rows must cost
+// nothing extra. GGUF rows are 2-byte aligned blocks of 56 .. 110 bytes: fetched by the lanes that multiply them, a wave-wide load would
+// touch 16 rows x 32 bytes and every line several times. Instead the workgroup copies whole rows - 16 or more consecutive ones are one
+// contiguous run - to LDS with 16-byte loads that bypass the registers, one unit ahead of the arithmetic, and each lane picks its fields
+// from LDS.
+//
+// K is cut into KP parts of 32 NG columns, and NRT = 8 / KP row tiles of 16 rows are in work beside each other. A unit is two halves
+// ("m") of 16 NRT rows: the gate and the up rows of 16 NRT FFN columns, or 32 NRT rows of a down matrix. A wave keeps the activations of its
+// K part for the whole tile in registers (fp16 hi and lo halves, 22 significant bits); the K parts meet in LDS. Tiles of up to 16 pairs
+// run sixteen waves, one half each (64 registers of activations, four waves per SIMD: the reads and the arithmetic of different waves
+// overlap; eight waves with both halves each took 158 us for the gate/up of 512 tokens x 10 over 512 raw
+// IQ2_XXS experts, sixteen 150), tiles of 17 .. 32 pairs eight waves with both halves
+// and two sets of pairs per decoded weight, as a launch of their own.
+// The SwiGLU activations go to the down kernel as f32, so work is cut at any unit, not at groups of columns that share an exponent; the
+// down kernel splits them per pair and K part when it loads them.
+//
+// Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights of row r (one
+// 32-column group per instruction), D[i = 4q .. 4q + 3][j = r]: the lane's own row against four pairs.
+#include <hip/hip_runtime.h>
+
+#include "redhip_mfma.h"
+
+namespace redhip {
+
+namespace {
+
+template <int SETS> constexpr uint32_t staged_waves() { return SETS == 1 ? 16u : 8u; }
+template <int SETS> constexpr uint32_t staged_threads() { return 64u * staged_waves<SETS>(); }
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+union H8 { uint4 u; half8_t v; half2_t p[4]; _Float16 e[8]; };
+
+// row sources
+enum : int { S_XXS = 0, S_XS = 1, S_M = 2, S_IQ3 = 3, S_PACKED_XXS = 4 };
+template <int SRC> constexpr uint32_t src_block() { return SRC == S_XXS ? 66u : SRC == S_XS ? 74u : SRC == S_M ? 56u : SRC == S_IQ3 ? 110u : 64u; }      // bytes per 256 columns
+
+// Decode tables in LDS.
+//   IQ2_XXS: the eight fp16 magnitudes of every grid entry times every group scale 2 s + 1 (64 KB, exact), at entry * 256 + s * 16: the address is
+//   the entry's byte over the top byte of the group's second word, one byte permute and one mask; IQ3_S likewise (four magnitudes, by scale)
+//   IQ2_XS: the fp16 codebook eight times, lane l reading copy l % 8 - a wave's 16-byte reads then hit every bank evenly (random entries of
+//   one copy: 2.6 times the cycles); IQ1_M: its fp16 codebook twice
+//   signs: bit 15 - i / 31 - i of the word of a sign field = signs of weights 2i and 2i + 1, so a pair's signs are one shift and one and-or;
+//   replicated so that the reads are (nearly) free of conflicts. (Sign masks as 16-byte entries save three shifts per eight weights and cost
+//   a second conflicting 16-byte read: LDS, the tighter of the two pipes, loses more.)
+template <int SRC> constexpr uint32_t sign_copies() { return SRC == S_M ? 0u : SRC == S_IQ3 ? 4u : 16u; }
+template <int SRC> constexpr uint32_t sign_bytes() { return (SRC == S_IQ3 ? 256u : 128u) * sign_copies<SRC>() * 4u; }
+constexpr uint32_t kEntryBytes = 65536u;
+
+__device__ __forceinline__ uint32_t two_halves(float lo, float hi) {
+    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
+}
+
+template <int SRC, uint32_t T>          // by all T threads of the workgroup
+__device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *signs, uint32_t tid, const int8_t *grid) {
+    if constexpr (SRC == S_XXS || SRC == S_PACKED_XXS) {
+        for (uint32_t e = tid; e < 16u * 256u; e += T) {
+            const uint64_t ge = redhip_iq2xxs_grid[e >> 4];
+            const float f = (float)(2u * (e & 15u) + 1u);
+            uint32_t w4[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w4[i] = two_halves(f * (float)((uint32_t)(ge >> (16 * i)) & 255u), f * (float)((uint32_t)(ge >> (16 * i + 8)) & 255u));
+            *reinterpret_cast<uint4 *>(entries + (size_t)e * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+        }
+    } else if constexpr (SRC == S_XS || SRC == S_M) {
+        constexpr uint32_t kCopies = SRC == S_XS ? 8u : 2u, kEntries = kEntryBytes / (16u * kCopies);
+        for (uint32_t e = tid; e < kEntries; e += T) {
+            const uint64_t ge = reinterpret_cast<const uint64_t *>(grid)[e];
+            uint32_t w4[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w4[i] = two_halves((float)(int8_t)(ge >> (16 * i)), (float)(int8_t)(ge >> (16 * i + 8)));
+            for (uint32_t c = 0; c < kCopies; ++c) *reinterpret_cast<uint4 *>(entries + ((size_t)e * kCopies + c) * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+        }
+    } else {
+        for (uint32_t e = tid; e < 16u * 512u; e += T) {
+            const uint32_t gw = redhip_iq3s_grid[e & 511u];
+            const float f = (float)(1u + 2u * (e >> 9));
+            *reinterpret_cast<uint2 *>(entries + (size_t)e * 8u) =
+                make_uint2(two_halves(f * (float)(gw & 255u), f * (float)((gw >> 8) & 255u)), two_halves(f * (float)((gw >> 16) & 255u), f * (float)(gw >> 24)));
+        }
+    }
+    if constexpr (SRC != S_M) {
+        constexpr uint32_t R = sign_copies<SRC>(), N = sign_bytes<SRC>() / 4u;
+        for (uint32_t i = tid; i < N; i += T) {
+            const uint32_t s = i / R, s8 = SRC == S_IQ3 ? s : s | ((__popc(s) & 1u) << 7);
+            uint32_t w = 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) w |= (((s8 >> (2u * k)) & 1u) << (15u - k)) | (((s8 >> (2u * k + 1u)) & 1u) << (31u - k));
+            signs[i] = w;
+        }
+    }
+}
+
+// fields of one 32-column group of the lane's row, as staged in LDS
+struct GroupWords { uint32_t a, b; };
+__device__ __forceinline__ uint32_t lds_u32_a2(const uint8_t *p) { uint32_t v; __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 4); return v; }
+__device__ __forceinline__ uint32_t lds_u16(const uint8_t *p) { return *reinterpret_cast<const uint16_t *>(p); }
+
+// IQ2_XXS rows are not staged as they lie: 16-byte LDS reads of 66-byte blocks are unaligned (more than half of the LDS cycles of the kernel
+// were unaligned stalls), and packed rows (512 bytes apart) would all start in one bank. A thread carries one 16-byte piece (two groups)
+// of a block through registers to an aligned place: piece (row R, block b, part) at ((R nb + b') 4 + (part ^ x)) 16 with b' and x functions
+// of the row that spread the sixteen rows a wave reads together over all banks. The block scales follow as f32.
+template <int SRC> constexpr bool src_pieces() { return SRC == S_XXS || SRC == S_PACKED_XXS; }
+__device__ __forceinline__ uint32_t piece_at(uint32_t R, uint32_t b, uint32_t part, uint32_t nb) {
+    const uint32_t r = R & 15u;
+    if (nb == 4u || nb == 8u) return (((R * nb + ((b + r) & (nb - 1u))) << 2) + (part ^ (r >> 2))) << 4;
+    if (nb == 2u) return (((R * 2u + (b ^ (r >> 3))) << 2) + (part ^ ((r >> 1) & 3u))) << 4;
+    return (((R * nb + b) << 2) + (part ^ (r >> 2))) << 4;
+}
+
+// blk: the block in LDS, sub: the group inside it (0 .. 7)
+template <int SRC>
+__device__ __forceinline__ GroupWords group_words(const uint8_t *blk, uint32_t sub, uint32_t q) {
+    if constexpr (SRC == S_XS) {
+        return GroupWords{lds_u16(blk + 2u + 8u * sub + 2u * q), blk[66u + sub]};
+    } else if constexpr (SRC == S_M) {      // b: the qh byte of the lane's entry | scale word of the group's 64 columns << 8
+        return GroupWords{blk[4u * sub + q], blk[32u + 2u * sub + (q >> 1)] | (lds_u16(blk + 48u + 2u * (sub >> 1)) >> (6u * (sub & 1u))) << 8};
+    } else {                                // IQ3_S. b: sign byte | qh byte << 8 | scale byte << 16
+        return GroupWords{lds_u16(blk + 2u + 8u * sub + 2u * q),
+                          blk[74u + 4u * sub + q] | ((uint32_t)blk[66u + sub] << 8) | (((uint32_t)blk[106u + (sub >> 1)] >> (4u * (sub & 1u))) << 16)};
+    }
+}
+template <int SRC>
+__device__ __forceinline__ float block_d(const uint8_t *blk) {
+    if constexpr (SRC == S_M) {
+        const uint32_t s01 = lds_u32_a2(blk + 48u), s23 = lds_u32_a2(blk + 52u);
+        return scale_to_f32(((s01 >> 12) & 0x000fu) | ((s01 >> 24) & 0x00f0u) | ((s23 >> 4) & 0x0f00u) | ((s23 >> 16) & 0xf000u));
+    } else
+        return scale_to_f32(lds_u16(blk));
+}
+
+// odd integer 2 s + 1 (s < 16) as two equal fp16 halves: 1024 + (2 s + 1) by integer arithmetic, minus 1024, exact
+__device__ __forceinline__ half2_t odd_splat(uint32_t s) {
+    const half2_t big = {(_Float16)1024.0f, (_Float16)1024.0f};
+    return __builtin_bit_cast(half2_t, __umul24(s, 0x20002u) + 0x64016401u) - big;
+}
+
+// lane constants of the tables: addresses of the lane's copy
+struct LaneTables { const uint8_t *entries; const uint8_t *signs; };
+
+// table reads of entry q (eight columns) of a group, then the arithmetic on what they return: the eight signed, scaled fp16 weights
+struct Entry { uint4 m; uint32_t s; };
+template <int SRC>
+__device__ __forceinline__ Entry fetch_entry(const GroupWords &w, uint32_t q, const LaneTables &t) {
+    Entry e;
+    if constexpr (SRC == S_XXS || SRC == S_PACKED_XXS) {
+        const uint32_t s7 = __builtin_amdgcn_ubfe(w.b, 7u * q, 7u);
+        // bytes 0 .. 3 of the permute's second operand are the entries, 7 the top byte of the first
+        e.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_perm(w.b, w.a, 0x0c0c0007u | (q << 8)) & 0xfff0u));
+        e.s = *reinterpret_cast<const uint32_t *>(t.signs + (s7 << 6));
+    } else if constexpr (SRC == S_XS) {
+        e.m = *reinterpret_cast<const uint4 *>(t.entries + ((w.a & 511u) << 7));
+        e.s = *reinterpret_cast<const uint32_t *>(t.signs + ((w.a >> 9) << 6));
+    } else if constexpr (SRC == S_M) {
+        const uint32_t nib = __builtin_amdgcn_ubfe(w.b, 4u * (q & 1u), 4u);
+        e.m = *reinterpret_cast<const uint4 *>(t.entries + ((w.a | ((nib & 7u) << 8)) << 5));
+        e.s = nib;
+    } else {
+        const uint32_t scale = (w.b & 0xf0000u) >> 4;                 // nibble * 512 entries * 8 bytes
+        const uint32_t ha = (w.b << (8u - 2u * q)) >> 5, hb = (w.b << (7u - 2u * q)) >> 5;      // bit 8 + 2q / 9 + 2q of b -> bit 11
+        const uint2 ma = *reinterpret_cast<const uint2 *>(t.entries + (((w.a & 255u) << 3) | (ha & 2048u) | scale));
+        const uint2 mb = *reinterpret_cast<const uint2 *>(t.entries + (((w.a >> 8) << 3) | (hb & 2048u) | scale));
+        e.m = make_uint4(ma.x, ma.y, mb.x, mb.y);
+        e.s = *reinterpret_cast<const uint32_t *>(t.signs + ((w.b & 255u) << 4));
+    }
+    return e;
+}
+template <int SRC>
+__device__ __forceinline__ half8_t finish_entry(const Entry &e, const GroupWords &w, uint32_t q) {
+    H8 r;
+    if constexpr (SRC == S_M) {
+        const half2_t f = odd_splat(__builtin_amdgcn_ubfe(w.b, 8u + 3u * (q >> 1), 3u));
+        // (2 s + 1) / 8 with the sign of the offset: three exponent steps down (2 s + 1 >= 1 is a normal number), sign bit by xor
+        const uint32_t neg = (e.s & 8u) << 12;
+        const half2_t off = __builtin_bit_cast(half2_t, (__builtin_bit_cast(uint32_t, f) - 0x0c000c00u) ^ (neg | (neg << 16)));
+        r.u = e.m;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * f + off;
+    } else {
+        constexpr uint32_t kSign = 0x80008000u;
+        r.u = e.m;
+        if constexpr (SRC == S_XS) {        // entries are signed bytes in general: the sign goes to the (positive) scale
+            const uint32_t f = __builtin_bit_cast(uint32_t, odd_splat(__builtin_amdgcn_ubfe(w.b, 4u * (q >> 1), 4u)));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * __builtin_bit_cast(half2_t, f | ((e.s << i) & kSign));
+        } else {
+            r.u.x |= e.s & kSign; r.u.y |= (e.s << 1) & kSign; r.u.z |= (e.s << 2) & kSign; r.u.w |= (e.s << 3) & kSign;
+        }
+    }
+    return r.v;
+}
+
+struct StagedArgs {
+    const uint8_t *experts, *shared;       // first matrix of expert uid[u] at experts + uid[u] * stride; of group n_unique[0] at `shared`
+    uint64_t stride, mat_step;             // mat_step: gate/up, distance of the up matrix
+    uint64_t d_off;                        // packed rows: the block scales [row][K / 256] behind the rows of a matrix
+    const uint32_t *uid, *pair_token, *n_unique, *tile_group, *tile_pair0, *tile_n, *n_tiles;
+    const _Float16 *xh, *xl;               // gate/up in: [ntok][K]
+    const int *xexp;                       // [ntok]
+    float *act;                            // [P + shared tokens][rows]: gate/up out; down in as [..][K]
+    float *tmp, *sh_tmp;                   // down out: [P][rows] routed pairs, [ntok][rows] shared expert
+    const int8_t *grid;                    // codebook of IQ2_XS / IQ1_M
+    uint32_t rows, P, list_stride;
+};
+
+__device__ __forceinline__ void wave_lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// 16 bytes per lane from src to LDS at dst (wave-uniform) + 16 * lane, past the registers. Written as an instruction of its own because the
+// compiler, which cannot tell the two halves of the stage apart, otherwise waits for it before the next read of the stage: the copy of the
+// next unit would be waited for before this unit is multiplied. Completion: s_waitcnt vmcnt(0) + barrier at the head of the next unit.
+__device__ __forceinline__ void copy16_to_lds(uint32_t dst, const uint8_t *src) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory");
+}
+typedef __attribute__((address_space(3))) uint8_t *lptr_t;
+
+// Hides from the compiler that v is the same in every trip of a loop: what is cheap to form again from it must not be kept in registers
+// (which the activations need) across the loop.
+__device__ __forceinline__ uint32_t each_trip(uint32_t v) { asm volatile("" : "+v"(v)); return v; }
+
+// `pieces` 16-byte pieces from src to dst in LDS, by the whole workgroup of T threads
+template <uint32_t T>
+__device__ __forceinline__ void stage_run(uint8_t *dst, const uint8_t *src, uint32_t pieces, uint32_t wave, uint32_t lane) {
+    for (uint32_t p = 64u * wave; p < pieces; p += T)
+        if (p + lane < pieces)
+            copy16_to_lds(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)dst + p * 16u), src + (uint64_t)(p + lane) * 16u);
+}
+
+// units u0 .. u1 - 1 (unit = tile * units per tile + unit of the tile) of a tile list; SETS sets of 16 pairs per tile
+template <int SRC, int NG, bool DOWN, int SETS, uint32_t KPS>          // KP = 1 << KPS parts of K
+__device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t *tile_group, const uint32_t *tile_pair0, const uint32_t *tile_n, uint32_t u0,
+                                             uint32_t u1, uint8_t *stage, float *part, const LaneTables &lt) {
+    if (u0 >= u1) return;
+    constexpr uint32_t BB = src_block<SRC>(), RUN = NG == 8 ? 8u : 2u;      // groups of one block per wave: all of them, or in pairs that never straddle blocks
+    constexpr uint32_t M = SETS == 1 ? 1u : 2u, T = staged_threads<SETS>();      // M: halves per wave
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), w8 = wave & 7u, m_first = SETS == 1 ? wave >> 3 : 0u;
+    constexpr uint32_t KP = 1u << KPS, NRT = 8u >> KPS, K = 32u * NG * KP, nb = K / 256u;
+    constexpr uint32_t RB = nb * BB, seg_rows = 16u * NRT, seg = seg_rows * RB, blocks = seg_rows * nb;
+    const uint32_t kc = w8 & (KP - 1u), rt = w8 >> KPS;
+    constexpr uint32_t segs = src_pieces<SRC>() ? blocks * 68u : seg;      // bytes of a half in LDS (pieces: 64 bytes + the scale per block)
+    const uint32_t upt = a.rows / ((DOWN ? 2u : 1u) * seg_rows), U = a.n_unique[0];
+    const auto matrix_of = [&](uint32_t tile) {
+        const uint32_t u = tile_group[tile];
+        return u == U ? a.shared : a.experts + (uint64_t)a.uid[u] * a.stride;
+    };
+    const auto run_of = [&](const uint8_t *mat, uint32_t j, uint32_t m) {      // rows of half m of unit j
+        return mat + (DOWN ? (uint64_t)(2u * j + m) * seg : m * a.mat_step + (uint64_t)j * seg);
+    };
+    const auto scales_of = [&](const uint8_t *mat, uint32_t j, uint32_t m) {   // packed rows: their block scales
+        return mat + a.d_off + (DOWN ? (uint64_t)(2u * j + m) * blocks * 2u : m * a.mat_step + (uint64_t)j * blocks * 2u);
+    };
+    // IQ2_XXS: this thread's piece (of either half), on its way through registers (plain variables and unconditional loads: an array filled
+    // under a condition ends up in scratch memory)
+    const uint32_t my_half = SETS == 1 ? wave >> 3 : 0u, my_at = my_half * segs + piece_at(((tid & 511u) >> 2) / nb, ((tid & 511u) >> 2) % nb, tid & 3u, nb);
+    uint4 piece0, piece1;
+    uint32_t scale0, scale1;
+    const auto request = [&](const uint8_t *mat, uint32_t j, uint8_t *buf) {
+        const uint8_t *run0 = run_of(mat, j, my_half), *run1 = SETS == 2 ? run_of(mat, j, 1u) : nullptr;
+        const uint32_t t = each_trip(tid & 511u), my_part = t & 3u, from_block = t >> 2 < blocks ? t >> 2 : 0u;
+        if constexpr (SRC == S_XXS) {
+            const uint32_t at = from_block * 66u, pt = at + 2u + 16u * my_part;
+            __builtin_memcpy(&piece0, __builtin_assume_aligned(run0 + pt, 2), 16);
+            scale0 = *reinterpret_cast<const uint16_t *>(run0 + at);
+            if constexpr (SETS == 2) {
+                __builtin_memcpy(&piece1, __builtin_assume_aligned(run1 + pt, 2), 16);
+                scale1 = *reinterpret_cast<const uint16_t *>(run1 + at);
+            }
+        } else if constexpr (SRC == S_PACKED_XXS) {
+            const uint32_t at = from_block * 64u + 16u * my_part;
+            piece0 = *reinterpret_cast<const uint4 *>(run0 + at);
+            scale0 = *reinterpret_cast<const uint16_t *>(scales_of(mat, j, my_half) + 2u * from_block);
+            if constexpr (SETS == 2) {
+                piece1 = *reinterpret_cast<const uint4 *>(run1 + at);
+                scale1 = *reinterpret_cast<const uint16_t *>(scales_of(mat, j, 1u) + 2u * from_block);
+            }
+        } else {
+            stage_run<T>(buf, run_of(mat, j, 0u), seg / 16u, wave, lane);
+            stage_run<T>(buf + segs, run_of(mat, j, 1u), seg / 16u, wave, lane);
+        }
+    };
+    const auto deliver = [&](uint8_t *buf) {
+        if constexpr (src_pieces<SRC>()) {
+            const uint32_t t = each_trip(tid & 511u), my_scale_at = my_half * segs + blocks * 64u + t;      // (threads of part 0: 4 bytes per block)
+            if (t >> 2 >= blocks) return;
+            *reinterpret_cast<uint4 *>(buf + my_at) = piece0;
+            if constexpr (SETS == 2) *reinterpret_cast<uint4 *>(buf + segs + my_at) = piece1;
+            if (t & 3u) return;
+            *reinterpret_cast<float *>(buf + my_scale_at) = scale_to_f32(scale0);
+            if constexpr (SETS == 2) *reinterpret_cast<float *>(buf + segs + my_scale_at) = scale_to_f32(scale1);
+        }
+    };
+    H8 xa[SETS][NG], xb[SETS][NG];
+    float ps[SETS][4];
+    // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
+    const auto load_tile = [&](uint32_t p0, uint32_t n) {
+#pragma unroll
+        for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
+            __builtin_amdgcn_sched_barrier(0);             // one set at a time: both at once do not fit the registers
+            const uint32_t l = each_trip(lane), q8 = 8u * (l >> 4), i = 16u * s + (l & 15u), p = i < n ? p0 + i : p0;
+            float scale = SRC == S_M || SRC == S_IQ3 ? 1.0f : 0.125f;      // (the d / 8 of the IQ2 formats)
+            if constexpr (!DOWN) {
+                const uint32_t tok = p < a.P ? a.pair_token[p] : p - a.P;
+                scale *= exp2i(a.xexp[tok]);
+                const uint64_t base = (uint64_t)tok * K + 32u * NG * kc + q8;
+                const _Float16 *hp = a.xh + base, *lp = a.xl + base;
+#pragma unroll
+                for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
+                    xa[s][g].u = *reinterpret_cast<const uint4 *>(hp + 32u * g);
+                    xb[s][g].u = *reinterpret_cast<const uint4 *>(lp + 32u * g);
+                }
+                // the low halves are stored times 2^11: back to their own scale (exact, the largest |x| of a token sits in [2^13, 2^14)), so that a
+                // product's high and low parts add up in one accumulator
+#pragma unroll
+                for (uint32_t g = 0; g < (uint32_t)NG; ++g) xb[s][g].v = xb[s][g].v * (_Float16)4.8828125e-4f;
+            } else {
+                // f32 activations of pair p, columns of this wave's K part: one exponent for them, then the fp16 halves
+                const float *src = a.act + (uint64_t)p * K + 32u * NG * kc + q8;
+                float amax = 0.0f;
+#pragma unroll
+                for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
+                    const float4 v0 = *reinterpret_cast<const float4 *>(src + 32u * g), v1 = *reinterpret_cast<const float4 *>(src + 32u * g + 4u);
+                    xa[s][g].u = __builtin_bit_cast(uint4, v0);
+                    xb[s][g].u = __builtin_bit_cast(uint4, v1);
+                }
+#pragma unroll
+                for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
+                    const float4 v0 = __builtin_bit_cast(float4, xa[s][g].u), v1 = __builtin_bit_cast(float4, xb[s][g].u);
+                    amax = fmaxf(amax, fmaxf(fmaxf(fmaxf(fabsf(v0.x), fabsf(v0.y)), fmaxf(fabsf(v0.z), fabsf(v0.w))), fmaxf(fmaxf(fabsf(v1.x), fabsf(v1.y)), fmaxf(fabsf(v1.z), fabsf(v1.w)))));
+                }
+                amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+                amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+                const int e = prescale_exp(amax);
+                const float inv = exp2i(-e);
+                scale *= exp2i(e);
+#pragma unroll
+                for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
+                    const float4 v0 = __builtin_bit_cast(float4, xa[s][g].u), v1 = __builtin_bit_cast(float4, xb[s][g].u);
+                    const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+                    H8 hi, lo;
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const float t = f[k] * inv;
+                        const _Float16 h = (_Float16)t;
+                        hi.e[k] = h;
+                        lo.e[k] = (_Float16)(t - (float)h);
+                    }
+                    xa[s][g].u = hi.u;
+                    xb[s][g].u = lo.u;
+                }
+            }
+#pragma unroll
+            for (uint32_t t = 0; t < 4u; ++t) ps[s][t] = __shfl(scale, (int)(q8 / 2u + t), 64);
+        }
+    };
+    // partial sums of the waves: [row tile, K part][m][set][lane] float4
+    constexpr uint32_t kWavePart = 2u * SETS * 256u, kPart = 8u * kWavePart;
+    const auto reduce = [&](uint32_t j, uint32_t p0, uint32_t n, const float *pt, uint32_t turn) {
+        const uint32_t t = each_trip(tid);
+        if constexpr (DOWN) {
+            // V consecutive floats (pairs of one row) per thread
+            constexpr uint32_t V = SETS == 1 ? 2u : 4u, PB = 256u / V, N = PB * SETS * 2u * NRT;
+            float *out = (p0 < a.P ? a.tmp + (uint64_t)p0 * a.rows : a.sh_tmp + (uint64_t)(p0 - a.P) * a.rows) + j * 2u * seg_rows;      // (a tile is routed or shared as a whole)
+#pragma unroll
+            for (uint32_t base = 0; base < N; base += T) {
+                const uint32_t it = base + t;
+                if (N % T != 0u && it >= N) continue;
+                const uint32_t at = (it & (PB - 1u)) * V, b = it / PB, set = b & (SETS - 1u), m = (b / SETS) & 1u, slot = b / (2u * SETS);
+                const float *src = pt + (slot << KPS) * kWavePart + (m * SETS + set) * 256u + at;
+                float s[V];
+#pragma unroll
+                for (uint32_t v = 0; v < V; ++v) s[v] = src[v];
+#pragma unroll
+                for (uint32_t k = 1; k < KP; ++k)
+#pragma unroll
+                    for (uint32_t v = 0; v < V; ++v) s[v] += src[k * kWavePart + v];
+                const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u);
+                float *o = out + (uint64_t)i * a.rows + m * seg_rows + 16u * slot + ((at >> 2) & 15u);
+#pragma unroll
+                for (uint32_t v = 0; v < V; ++v)
+                    if (i + v < n) o[(uint64_t)v * a.rows] = s[v];
+            }
+        } else {
+            // one (pair, column) element per thread; where the elements are fewer than the threads, the waves take turns
+            constexpr uint32_t N = 256u * SETS * NRT;
+            const uint32_t lead = N < T ? (turn % (T / N)) * N : 0u;
+#pragma unroll
+            for (uint32_t base = 0; base < N; base += T) {
+                const uint32_t e = base + t - lead;
+                if (N < T && e >= N) continue;             // (wave-uniform)
+                const uint32_t at = e & 255u, b = e >> 8, set = b & (SETS - 1u), slot = b / SETS;
+                const float *src = pt + (slot << KPS) * kWavePart + set * 256u + at;
+                float s0 = src[0], s1 = src[SETS * 256u];
+#pragma unroll
+                for (uint32_t k = 1; k < KP; ++k) {
+                    s0 += src[k * kWavePart];
+                    s1 += src[k * kWavePart + SETS * 256u];
+                }
+                const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u);
+                if (i < n) a.act[(uint64_t)(p0 + i) * a.rows + j * seg_rows + 16u * slot + ((at >> 2) & 15u)] = (s0 / (1.0f + expf(-s0))) * s1;
+            }
+        }
+    };
+    // offsets of the lane's pieces and block scales inside a half
+    uint32_t piece_off[NG / 2], d_off[NG / RUN];
+#pragma unroll
+    for (uint32_t g2 = 0; g2 < NG / 2u; ++g2) {
+        const uint32_t gg = kc * NG + 2u * g2;
+        piece_off[g2] = src_pieces<SRC>() ? m_first * segs + piece_at(16u * rt + r, gg >> 3, (gg & 7u) >> 1, nb) : 0u;
+    }
+#pragma unroll
+    for (uint32_t b = 0; b < NG / RUN; ++b) d_off[b] = src_pieces<SRC>() ? m_first * segs + blocks * 64u + 4u * ((16u * rt + r) * nb + ((kc * NG + RUN * b) >> 3)) : 0u;
+
+    uint32_t tile = u0 / upt, j = u0 % upt, p0 = tile_pair0[tile], n = tile_n[tile];
+    uint32_t pj = 0u, pp0 = 0u, pn = 0u;                   // the unit before, whose partial sums wait in LDS
+    const uint8_t *mat = matrix_of(tile);
+    bool fresh = true;
+    request(mat, j, stage);
+    deliver(stage);
+    for (uint32_t u = u0; u < u1; ++u) {
+        const uint32_t buf = (u - u0) & 1u;
+        if (fresh) { load_tile(p0, n); fresh = false; }
+        const bool more = u + 1u < u1, next_tile = j + 1u == upt;
+        const uint32_t nj = next_tile ? 0u : j + 1u;
+        uint32_t np0 = p0, nn = n;
+        const uint8_t *nmat = mat;
+        if (more && next_tile) { nmat = matrix_of(tile + 1u); np0 = tile_pair0[tile + 1u]; nn = tile_n[tile + 1u]; }
+        if constexpr (!src_pieces<SRC>()) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's share of the unit has landed
+        wave_lds_barrier();                                // everybody's has; the unit before is multiplied and its partial sums are written (first time: the tables too)
+        if (u > u0) reduce(pj, pp0, pn, part + (SETS == 1 ? (buf ^ 1u) * kPart : 0u), u);
+        // the next unit's rows, behind the stores of reduce, which have the unit's time to drain. (Pieces unconditionally - the last unit
+        // fetches its own again: registers filled under a condition would be live all around the loop.)
+        if (src_pieces<SRC>() || more) request(more ? nmat : mat, more ? nj : j, stage + (buf ^ 1u) * 2u * segs);
+
+        const uint8_t *half = stage + buf * 2u * segs, *rows = half + m_first * segs + (16u * rt + r) * RB;
+        float4_t tot[M][SETS], acc[M][SETS];
+        GroupWords gw[M][NG];
+        const auto block_of = [&](uint32_t g) { return (NG == 8 ? kc : (kc * NG + g) >> 3); };
+        const auto sub_of = [&](uint32_t g) { return NG == 8 ? g : (kc * NG + g) & 7u; };
+        const auto words_of = [&](uint32_t g) {            // groups g and g + 1
+#pragma unroll
+            for (uint32_t m = 0; m < M; ++m) {
+                if constexpr (src_pieces<SRC>()) {
+                    const uint4 v = *reinterpret_cast<const uint4 *>(half + m * segs + piece_off[g / 2u]);
+                    gw[m][g] = GroupWords{v.x, v.y};
+                    gw[m][g + 1u] = GroupWords{v.z, v.w};
+                } else {
+                    gw[m][g] = group_words<SRC>(rows + m * segs + block_of(g) * BB, sub_of(g), q);
+                    gw[m][g + 1u] = group_words<SRC>(rows + m * segs + block_of(g + 1u) * BB, sub_of(g + 1u), q);
+                }
+            }
+        };
+        words_of(0u);
+        words_of(2u);
+#pragma unroll
+        for (uint32_t m = 0; m < M; ++m)
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) { tot[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f}; acc[m][s] = tot[m][s]; }
+        Entry e0[M], e1[M];
+#pragma unroll
+        for (uint32_t m = 0; m < M; ++m) { e0[m] = fetch_entry<SRC>(gw[m][0], q, lt); e1[m] = fetch_entry<SRC>(gw[m][1], q, lt); }
+#pragma unroll
+        for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
+            // fields run four groups ahead of the arithmetic, table reads two
+            __builtin_amdgcn_sched_barrier(0);
+            if ((g & 1u) == 0u && g + 4u < (uint32_t)NG) words_of(g + 4u);
+            half8_t w[M];
+#pragma unroll
+            for (uint32_t m = 0; m < M; ++m) {
+                w[m] = finish_entry<SRC>(g & 1u ? e1[m] : e0[m], gw[m][g], q);
+                if (g + 2u < (uint32_t)NG) { if (g & 1u) e1[m] = fetch_entry<SRC>(gw[m][g + 2u], q, lt); else e0[m] = fetch_entry<SRC>(gw[m][g + 2u], q, lt); }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
+#pragma unroll
+                for (uint32_t m = 0; m < M; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[s][g].v, w[m], acc[m][s], 0, 0, 0);
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
+#pragma unroll
+                for (uint32_t m = 0; m < M; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[s][g].v, w[m], acc[m][s], 0, 0, 0);
+            if ((g + 1u) % RUN == 0u) {
+#pragma unroll
+                for (uint32_t m = 0; m < M; ++m) {
+                    float d;
+                    if constexpr (src_pieces<SRC>()) d = *reinterpret_cast<const float *>(half + m * segs + d_off[g / RUN]);
+                    else d = block_d<SRC>(rows + m * segs + block_of(g) * BB);
+#pragma unroll
+                    for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) tot[m][s][t] = fmaf(acc[m][s][t], d * ps[s][t], tot[m][s][t]);
+                        acc[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+                }
+            }
+        }
+        if constexpr (SETS == 2) wave_lds_barrier();       // one buffer of partial sums: those of the unit before have been read
+        float *mine = part + (SETS == 1 ? buf * kPart : 0u) + w8 * kWavePart + m_first * SETS * 256u + 4u * lane;
+#pragma unroll
+        for (uint32_t m = 0; m < M; ++m)
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) = tot[m][s];
+        deliver(stage + (buf ^ 1u) * 2u * segs);           // (free since the barrier at this unit's head)
+        pj = j; pp0 = p0; pn = n;
+        if (next_tile && more) { ++tile; fresh = true; p0 = np0; n = nn; mat = nmat; }
+        j = nj;
+    }
+    wave_lds_barrier();
+    reduce(pj, pp0, pn, part + (SETS == 1 ? ((u1 - 1u - u0) & 1u) * kPart : 0u), 0u);
+}
+
+// SETS 1: the narrow tiles (list 2) of a chunk, SETS 2: the wide ones (list 1). Persistent workgroups, each with an equal run of the units.
+// A launch that finds few wide tiles leaves them: the narrow one then takes every pair in tiles of 16 (list 0). A wide launch costs 20 us
+// however few tiles it has (tables, the first tile's activations), one more tile on the narrow kernels 0.3 us of the whole device.
+constexpr uint32_t kFewWide = 48u;
+template <int SRC, int NG, bool DOWN, int SETS, uint32_t KPS>
+__global__ __launch_bounds__(staged_threads<SETS>()) void staged_tiles_kernel(StagedArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t stage[];        // two buffers of two halves of a unit
+    __shared__ __attribute__((aligned(16))) uint8_t entries[kEntryBytes];   // static: table reads take immediate offsets
+    __shared__ __attribute__((aligned(16))) uint32_t signs[sign_bytes<SRC>() / 4u + 4u];
+    __shared__ __attribute__((aligned(16))) float part[2u * 8u * 2u * 256u];
+    const bool few = a.n_tiles[1] < kFewWide;
+    if (SETS == 2 && few) return;
+    const uint32_t tid = threadIdx.x, l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
+    const uint32_t units = a.n_tiles[l] * (a.rows / ((DOWN ? 32u : 16u) * (8u >> KPS)));
+    // workgroups are dealt round-robin over the eight XCDs: neighbouring runs (which share tiles) go to one XCD's L2
+    const uint32_t G = gridDim.x, at = G % 8u == 0u ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
+    const uint32_t u0 = (uint32_t)((uint64_t)at * units / G), u1 = (uint32_t)((uint64_t)(at + 1u) * units / G);
+    if (u0 >= u1) return;
+    build_staged_tables<SRC, staged_threads<SETS>()>(entries, signs, tid, a.grid);
+    const LaneTables lt{entries + (SRC == S_XS ? (tid & 7u) * 16u : SRC == S_M ? (tid & 1u) * 16u : 0u),
+                        reinterpret_cast<const uint8_t *>(signs) + (SRC == S_IQ3 ? (tid & 3u) * 4u : SRC == S_M ? 0u : (tid & 15u) * 4u)};
+    staged_units<SRC, NG, DOWN, SETS, KPS>(a, a.tile_group + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, stage, part, lt);
+}
+
+template <int SRC, int NG, bool DOWN, int SETS, uint32_t KPS>
+hipError_t launch_staged_list(const StagedArgs &a, uint32_t grid, hipStream_t s) {
+    constexpr size_t lds = (size_t)4u * 16u * (8u >> KPS) * (NG << KPS) / 8u * (src_pieces<SRC>() ? 68u : src_block<SRC>());
+    static bool attr = false;
+    if (!attr) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(staged_tiles_kernel<SRC, NG, DOWN, SETS, KPS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    REDHIP_LAUNCH((staged_tiles_kernel<SRC, NG, DOWN, SETS, KPS>), dim3(grid), dim3(staged_threads<SETS>()), lds, s, a);
+    return hipGetLastError();
+}
+// wide: the chunk can have tiles of more than 16 pairs
+template <int SRC, int NG, bool DOWN, uint32_t KPS>
+hipError_t launch_staged_lists(const StagedArgs &a, uint32_t grid, bool wide, hipStream_t s) {
+    const hipError_t e = wide ? launch_staged_list<SRC, NG, DOWN, 2, KPS>(a, grid, s) : hipSuccess;
+    return e == hipSuccess ? launch_staged_list<SRC, NG, DOWN, 1, KPS>(a, grid, s) : e;
+}
+template <int SRC>
+hipError_t launch_staged_gateup(const StagedArgs &a, uint32_t hidden, uint32_t grid, bool wide, hipStream_t s) {
+    return hidden == 512u    ? launch_staged_lists<SRC, 8, false, 1>(a, grid, wide, s)
+           : hidden == 1024u ? launch_staged_lists<SRC, 8, false, 2>(a, grid, wide, s)
+                             : launch_staged_lists<SRC, 8, false, 3>(a, grid, wide, s);
+}
+template <int SRC>
+hipError_t launch_staged_down(const StagedArgs &a, uint32_t ffn, uint32_t grid, bool wide, hipStream_t s) {
+    return ffn == 256u   ? launch_staged_lists<SRC, 8, true, 0>(a, grid, wide, s)
+           : ffn == 512u ? launch_staged_lists<SRC, 8, true, 1>(a, grid, wide, s)
+           : ffn == 768u ? launch_staged_lists<SRC, 6, true, 2>(a, grid, wide, s)
+                         : launch_staged_lists<SRC, 8, true, 2>(a, grid, wide, s);
+}
+
+int staged_src(uint32_t type, bool packed) {
+    if (packed) return type == T_IQ2_XXS ? S_PACKED_XXS : -1;
+    return type == T_IQ2_XXS ? S_XXS : type == T_IQ2_XS ? S_XS : type == T_IQ1_M ? S_M : type == T_IQ3_S ? S_IQ3 : -1;
+}
+
+}  // namespace
+
+// hidden: one K part of 256 columns per wave, two to eight of them; ffn: 256, 512, 1024 likewise, 768 as four parts of 192
+bool staged_tiles_supported(uint32_t gate_up_type, uint32_t down_type, uint32_t hidden, uint32_t ffn, uint32_t n_expert, bool packed) {
+    const int g = staged_src(gate_up_type, packed), d = staged_src(down_type, packed);
+    return g >= 0 && g != S_IQ3 && d >= 0 && (hidden == 512u || hidden == 1024u || hidden == 2048u) && (ffn == 256u || ffn == 512u || ffn == 768u || ffn == 1024u) && n_expert <= 1024u;
+}
+
+hipError_t launch_staged_tiles(const StagedExperts &x, const uint32_t *uid, const uint32_t *expert_start, const uint32_t *pair_token, const uint32_t *n_unique,
+                               const TileLists &tl, bool tiles_built, const void *xh, const void *xl, const int *xexp, float *act, float *tmp, float *sh_tmp,
+                               uint32_t hidden, uint32_t ffn, uint32_t top_k, uint32_t ntok, uint32_t n_expert, hipStream_t s) {
+    if (!staged_tiles_supported(x.gate_up_type, x.down_type, hidden, ffn, n_expert, x.packed) || !ntok || (tl.shared_ntok && (!x.shared || !sh_tmp))) return hipErrorInvalidValue;
+    const uint32_t P = ntok * top_k;
+    if (!tiles_built) {
+        prof_set_stage(ST_GROUP);
+        const hipError_t e = launch_build_tiles(expert_start, n_unique, P, tl, s);
+        if (e != hipSuccess) return e;
+    }
+    const uint32_t bound = prefill_tile_bound(ntok, top_k, n_expert), grid = 4u * bound < 256u ? 4u * bound : 256u;
+    StagedArgs a{static_cast<const uint8_t *>(x.gate), static_cast<const uint8_t *>(x.shared), x.stride, x.up_delta, (uint64_t)ffn * (hidden / 32u) * 8u,
+                 uid, pair_token, n_unique, tl.tile_group, tl.tile_pair0, tl.tile_n, tl.n_tiles, static_cast<const _Float16 *>(xh), static_cast<const _Float16 *>(xl), xexp,
+                 act, tmp, sh_tmp, x.gate_up_grid, ffn, P, tl.list_stride};
+    const bool wide = P > kPrefillTile;
+    hipError_t e = hipErrorInvalidValue;
+    prof_set_stage(ST_PREFILL_GATEUP);
+    switch (staged_src(x.gate_up_type, x.packed)) {
+        case S_XXS: e = launch_staged_gateup<S_XXS>(a, hidden, grid, wide, s); break;
+        case S_XS: e = launch_staged_gateup<S_XS>(a, hidden, grid, wide, s); break;
+        case S_M: e = launch_staged_gateup<S_M>(a, hidden, grid, wide, s); break;
+        case S_PACKED_XXS: e = launch_staged_gateup<S_PACKED_XXS>(a, hidden, grid, wide, s); break;
+    }
+    if (e != hipSuccess) return e;
+    a.experts = static_cast<const uint8_t *>(x.down);
+    a.stride = x.down_stride;
+    a.mat_step = 0u;
+    if (x.shared) a.shared += 2u * x.up_delta;
+    a.d_off = (uint64_t)hidden * (ffn / 32u) * 8u;
+    a.grid = x.down_grid;
+    a.rows = hidden;
+    prof_set_stage(ST_PREFILL_DOWN);
+    switch (staged_src(x.down_type, x.packed)) {
+        case S_XXS: return launch_staged_down<S_XXS>(a, ffn, grid, wide, s);
+        case S_XS: return launch_staged_down<S_XS>(a, ffn, grid, wide, s);
+        case S_M: return launch_staged_down<S_M>(a, ffn, grid, wide, s);
+        case S_IQ3: return launch_staged_down<S_IQ3>(a, ffn, grid, wide, s);
+        case S_PACKED_XXS: return launch_staged_down<S_PACKED_XXS>(a, ffn, grid, wide, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace redhip

@@ -329,26 +329,41 @@ bool enqueue_pairs(TopkPool *p, hipStream_t s, const std::vector<uint64_t> &gate
     return true;
 }
 
-// The same pairs on the prefill tile kernels, for slots that hold tile-major copies: x split to fp16 halves per token, tiles of up to 32
-// pairs per expert on the MFMA units (gate / up + SwiGLU, then down rows into tmp[pair]), combine in selection order. An expert is named
-// by the distance of its slot from the lowest slot of the call, in units of 256 bytes (slots are 4096-aligned, HBM is far below 1 TB).
-bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const std::vector<uint64_t> &slot_addr, uint32_t n_expert, uint32_t hidden, uint32_t ffn,
+// The same pairs on the tile kernels: x split to fp16 halves per token, tiles of up to 32 pairs per expert on the MFMA units (gate / up +
+// SwiGLU, then down rows into tmp[pair]), combine in selection order. `copies`: slots that hold tile-major copies, on the kernels that
+// read those; otherwise the kernels that take raw rows through LDS. Expert u is number uid[u] of the arrays that `ex` describes.
+struct PairExperts {
+    const uint8_t *gate, *down;
+    uint64_t stride, down_stride, up_delta;
+    std::vector<uint32_t> uid;
+};
+// slots: an expert is named by the distance of its slot from the lowest slot of the call, in units of 256 bytes (slots are 4096-aligned,
+// HBM is far below 1 TB)
+bool slot_experts(const std::vector<uint64_t> &slot_addr, uint64_t gate_bytes, PairExperts *ex) {
+    uint64_t lowest = slot_addr[0];
+    for (uint64_t a : slot_addr) lowest = a < lowest ? a : lowest;
+    for (uint64_t a : slot_addr) {
+        const uint64_t d = a - lowest;
+        if ((d & 255u) || (d >> 8) > 0xffffffffull) { TOPK_ERR("top-k slots of one call lie too far apart"); return false; }
+        ex->uid.push_back((uint32_t)(d >> 8));
+    }
+    ex->gate = reinterpret_cast<const uint8_t *>(lowest);
+    ex->down = ex->gate + 2u * gate_bytes;
+    ex->stride = ex->down_stride = 256u;
+    ex->up_delta = gate_bytes;
+    return true;
+}
+bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const PairExperts &ex, bool copies, uint32_t type_word, uint32_t n_expert, uint32_t hidden, uint32_t ffn,
                          uint32_t tok_first, uint32_t ntok, uint32_t top_k, uint32_t n_pairs, const uint32_t *pair_token, const float *pair_weight,
                          const uint32_t *expert_start, const uint32_t *tok_pair, const float *x, float *out) {
     std::lock_guard<std::recursive_mutex> lk(p->enc_mu);
-    if (!bind_grids(p, p->fs.word)) return false;
-    uint64_t lowest = slot_addr[0];
-    for (uint64_t a : slot_addr) lowest = a < lowest ? a : lowest;
+    if (!bind_grids(p, type_word)) return false;
     std::vector<uint32_t> u;
     u.reserve((size_t)n_pairs * 2u + 2u * n_expert + 2u);
     u.insert(u.end(), pair_token, pair_token + n_pairs);
     u.insert(u.end(), expert_start, expert_start + n_expert + 1u);
     u.insert(u.end(), tok_pair, tok_pair + (size_t)ntok * top_k);
-    for (uint64_t a : slot_addr) {
-        const uint64_t d = a - lowest;
-        if ((d & 255u) || (d >> 8) > 0xffffffffull) { TOPK_ERR("top-k slots of one call lie too far apart"); return false; }
-        u.push_back((uint32_t)(d >> 8));
-    }
+    u.insert(u.end(), ex.uid.begin(), ex.uid.end());
     u.push_back(n_expert);
     // scratch of the call: rows of x up to the last token of the call, n_pairs activation rows
     const size_t rows = (size_t)tok_first + ntok, arows = (size_t)n_pairs + ntok;
@@ -375,10 +390,15 @@ bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const std::vector<uint64_t>
     if (!stage_lists(p, s, {}, pair_weight, n_pairs, u, &st)) return false;
     const uint32_t *d_pair_token = st.u, *d_start = st.u + n_pairs, *d_tok_pair = d_start + n_expert + 1u, *d_uid = d_tok_pair + (size_t)ntok * top_k, *d_unique = d_uid + n_expert;
     float *tmp = static_cast<float *>(p->tmp_b.p);
-    const uint8_t *tiles = reinterpret_cast<const uint8_t *>(lowest + p->fs.tile_off);
+    const uint8_t *tiles = ex.gate + p->fs.tile_off;
     // (the split kernel also forms a gate logit per row from a second vector: x itself stands in, the result is not used)
     hipError_t e = launch_prep(x, x, (uint32_t)rows, hidden, xh, xl, xexp, gate_unused, s, nullptr, nullptr);
-    if (e == hipSuccess && p->fs.kind == 0u)
+    if (e == hipSuccess && !copies) {
+        const uint32_t gu = word_gate_up(type_word), dn = word_down(type_word);
+        const StagedExperts rows{ex.gate, ex.down, nullptr, ex.stride, ex.down_stride, ex.up_delta, gu, dn, caller_grid_device(gu), caller_grid_device(dn), false};
+        e = launch_staged_tiles(rows, d_uid, d_start, d_pair_token, d_unique, TileLists{tile_group, tile_pair0, tile_n, n_tiles, bound, 0u}, false, xh, xl, xexp,
+                                static_cast<float *>(act_h), tmp, nullptr, hidden, ffn, top_k, ntok, n_expert, s);      // (act_h | act_l: as many bytes as f32)
+    } else if (e == hipSuccess && p->fs.kind == 0u)
         e = launch_prefill_packed(nullptr, 256u, nullptr, tiles, nullptr, d_uid, d_start, d_pair_token, d_unique, tile_group, tile_pair0, tile_n, n_tiles,
                                   xh, xl, xexp, act_h, act_l, act_exp, tmp, nullptr, hidden, ffn, top_k, ntok, n_expert, s, false, false);
     else if (e == hipSuccess && p->fs.kind == 1u) {      // IQ2_XXS gate / up tiles, then the IQ3_S down tiles
@@ -899,11 +919,15 @@ int redmetal_topk_pool_encode_batched(redmetal_topk_pool_t h, void *stream, cons
         std::lock_guard<std::mutex> lk(p->mu);
         for (uint32_t i = 0; i < n_expert; ++i) tiles = tiles && p->shadow_ok[slot_ids[i]];
     }
-    if (tiles ? !enqueue_pairs_tiles(p, static_cast<hipStream_t>(stream), table, n_expert, hidden_size, ffn_size, tok_first, ntok, top_k, n_pairs, pair_token,
-                                     pair_weight, expert_start, tok_pair, at(input_dev, input_offset), at(output_dev, output_offset))
-              : !enqueue_pairs(p, static_cast<hipStream_t>(stream), table, table, gate_bytes[0], gate_bytes[0] + up_bytes[0], n_expert, ggml_type,
-                               hidden_size, ffn_size, tok_first, ntok, top_k, n_pairs, pair_token, pair_weight, expert_start, tok_pair,
-                               at(input_dev, input_offset), at(output_dev, output_offset))) return 0;
+    // slots without tile-major copies: the tile kernels on their raw rows, for the formats and shapes those take
+    const bool staged = !tiles && staged_tiles_supported(word_gate_up(ggml_type), word_down(ggml_type), hidden_size, ffn_size, n_expert, false);
+    PairExperts ex;
+    if (tiles || staged ? !slot_experts(table, gate_bytes[0], &ex) ||
+                              !enqueue_pairs_tiles(p, static_cast<hipStream_t>(stream), ex, tiles, ggml_type, n_expert, hidden_size, ffn_size, tok_first, ntok, top_k, n_pairs,
+                                                   pair_token, pair_weight, expert_start, tok_pair, at(input_dev, input_offset), at(output_dev, output_offset))
+                        : !enqueue_pairs(p, static_cast<hipStream_t>(stream), table, table, gate_bytes[0], gate_bytes[0] + up_bytes[0], n_expert, ggml_type,
+                                         hidden_size, ffn_size, tok_first, ntok, top_k, n_pairs, pair_token, pair_weight, expert_start, tok_pair,
+                                         at(input_dev, input_offset), at(output_dev, output_offset))) return 0;
     p->mark(slot_ids, n_expert, +1);
     return 1;
 }
@@ -922,6 +946,13 @@ int redmetal_topk_pool_encode_mapped(redmetal_topk_pool_t h, void *stream,
         down_bytes != (uint64_t)hidden_size * pool_row_bytes(word_down(ggml_type), ffn_size)) { TOPK_ERR("mapped top-k matrix byte mismatch"); return 0; }
     if (!pool_shape_ok(hidden_size, ffn_size, true)) return 0;
     if (!pair_layout_ok("mapped", n_expert, tok_first, ntok, top_k, n_pairs, pair_token, expert_start, tok_pair)) return 0;
+    if (((gate_addr0 | up_addr0 | down_addr0 | gate_bytes | down_bytes) & 15u) == 0u &&
+        staged_tiles_supported(word_gate_up(ggml_type), word_down(ggml_type), hidden_size, ffn_size, n_expert, false)) {
+        const PairExperts ex{reinterpret_cast<const uint8_t *>(gate_addr0), reinterpret_cast<const uint8_t *>(down_addr0), gate_bytes, down_bytes, up_addr0 - gate_addr0,
+                             std::vector<uint32_t>(expert_ids, expert_ids + n_expert)};
+        return enqueue_pairs_tiles(p, static_cast<hipStream_t>(stream), ex, false, ggml_type, n_expert, hidden_size, ffn_size, tok_first, ntok, top_k, n_pairs, pair_token,
+                                   pair_weight, expert_start, tok_pair, at(input_dev, input_offset), at(output_dev, output_offset)) ? 1 : 0;
+    }
     std::vector<uint64_t> gate(n_expert), down(n_expert);
     for (uint32_t i = 0; i < n_expert; ++i) {
         gate[i] = gate_addr0 + (uint64_t)expert_ids[i] * gate_bytes;

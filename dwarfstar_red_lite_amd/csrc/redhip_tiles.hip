@@ -4,22 +4,23 @@
 //
 // What bounds these kernels is the decode (LDS table reads and vector issue; every weight is decoded once per tile), so the rows must cost
 // nothing extra. GGUF rows are 2-byte aligned blocks of 56 .. 110 bytes: fetched by the lanes that multiply them, a wave-wide load would
-// touch 16 rows x 32 bytes and every line several times. Instead the workgroup copies whole rows - 16 or more consecutive ones are one
-// contiguous run - to LDS with 16-byte loads that bypass the registers, one unit ahead of the arithmetic, and each lane picks its fields
-// from LDS.
+// touch 16 rows x 32 bytes and every line several times; staged as they lie, 16-byte LDS reads of them are unaligned (more than half of the
+// kernel's LDS cycles were unaligned stalls). Instead every thread of the workgroup carries the fields of a quarter block (64 columns) through
+// its registers, one unit ahead of the arithmetic, to an aligned place in LDS.
 //
-// K is cut into KP parts of 32 NG columns, and NRT = 8 / KP row tiles of 16 rows are in work beside each other. A unit is two halves
-// ("m") of 16 NRT rows: the gate and the up rows of 16 NRT FFN columns, or 32 NRT rows of a down matrix. A wave keeps the activations of its
-// K part for the whole tile in registers (fp16 hi and lo halves, 22 significant bits); the K parts meet in LDS. Tiles of up to 16 pairs
-// run sixteen waves, one half each (64 registers of activations, four waves per SIMD: the reads and the arithmetic of different waves
-// overlap; eight waves with both halves each took 158 us for the gate/up of 512 tokens x 10 over 512 raw
-// IQ2_XXS experts, sixteen 150), tiles of 17 .. 32 pairs eight waves with both halves
-// and two sets of pairs per decoded weight, as a launch of their own.
-// The SwiGLU activations go to the down kernel as f32, so work is cut at any unit, not at groups of columns that share an exponent; the
-// down kernel splits them per pair and K part when it loads them.
+// K is cut into KP blocks of 256 columns, and NRT row tiles of 16 rows are in work beside each other (KP * NRT = 8; 6 with three
+// blocks). A unit is two halves ("m") of 16 NRT rows: the gate and the up rows of 16 NRT FFN columns, or 32 NRT rows of a down matrix.
+// A wave keeps the activations of its block for the whole tile in registers (fp16 hi and lo halves, 22 significant bits); the blocks
+// meet in LDS. Tiles of up to 16 pairs run sixteen waves, one half each (64 registers of activations, four waves per SIMD: the reads and
+// the arithmetic of different waves overlap), tiles of 17 .. 32 pairs eight waves with both halves and two sets of pairs per decoded
+// weight, as a launch of their own. The SwiGLU activations go to the down kernel as f32, so work is cut at any unit, not at groups of
+// columns that share an exponent; the down kernel splits them per pair and block when it loads them.
 //
-// Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights of row r (one
-// 32-column group per instruction), D[i = 4q .. 4q + 3][j = r]: the lane's own row against four pairs.
+// Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights of row r,
+// D[i = 4q .. 4q + 3][j = r]: the lane's own row against four pairs. Which columns the instruction's k stand for is free as long as both
+// operands agree: step s of a block takes columns 64 q + 8 s .. + 7 of it, so lane (r, q) decodes quarter q of its row's block and
+// nothing else - its fields are one aligned 16-byte read (XS 4, IQ3_S 12 more bytes), every bit position is a constant, and a scale
+// (per 16 or 32 columns) is formed once for the entries that share it.
 #include <hip/hip_runtime.h>
 
 #include "redhip_mfma.h"
@@ -28,8 +29,8 @@ namespace redhip {
 
 namespace {
 
-template <int SETS> constexpr uint32_t staged_waves() { return SETS == 1 ? 16u : 8u; }
-template <int SETS> constexpr uint32_t staged_threads() { return 64u * staged_waves<SETS>(); }
+constexpr uint32_t staged_nrt(uint32_t KP) { return KP == 3u ? 2u : 8u / KP; }
+constexpr uint32_t staged_threads(int sets, uint32_t KP) { return 64u * KP * staged_nrt(KP) * (sets == 1 ? 2u : 1u); }
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
@@ -95,42 +96,48 @@ __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *
     }
 }
 
-// fields of one 32-column group of the lane's row, as staged in LDS
-struct GroupWords { uint32_t a, b; };
-__device__ __forceinline__ uint32_t lds_u32_a2(const uint8_t *p) { uint32_t v; __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 4); return v; }
-__device__ __forceinline__ uint32_t lds_u16(const uint8_t *p) { return *reinterpret_cast<const uint16_t *>(p); }
+// fields of a quarter block (two 32-column groups) of a row: what a lane multiplies
+//   IQ2_XXS  a: the two groups' words                     IQ2_XS  a: eight 16-bit entries, c: two scale bytes
+//   IQ1_M    a: 8 index bytes | 4 bytes of nibbles | scale word     IQ3_S   a: 16 index bytes, b: 8 sign bytes, c: two qh bytes | scale byte << 16
+struct Quarter { uint4 a; uint2 b; uint32_t c; };
+template <int SRC> constexpr uint32_t quarter_b() { return SRC == S_IQ3 ? 8u : 0u; }                       // bytes of b and c in LDS
+template <int SRC> constexpr uint32_t quarter_c() { return SRC == S_IQ3 || SRC == S_XS ? 4u : 0u; }
+template <int SRC> constexpr uint32_t staged_block_bytes() { return 4u * (16u + quarter_b<SRC>() + quarter_c<SRC>()) + 4u; }      // of a block in LDS: its quarters, then d as f32
 
-// IQ2_XXS rows are not staged as they lie: 16-byte LDS reads of 66-byte blocks are unaligned (more than half of the LDS cycles of the kernel
-// were unaligned stalls), and packed rows (512 bytes apart) would all start in one bank. A thread carries one 16-byte piece (two groups)
-// of a block through registers to an aligned place: piece (row R, block b, part) at ((R nb + b') 4 + (part ^ x)) 16 with b' and x functions
-// of the row that spread the sixteen rows a wave reads together over all banks. The block scales follow as f32.
-template <int SRC> constexpr bool src_pieces() { return SRC == S_XXS || SRC == S_PACKED_XXS; }
-__device__ __forceinline__ uint32_t piece_at(uint32_t R, uint32_t b, uint32_t part, uint32_t nb) {
-    const uint32_t r = R & 15u;
-    if (nb == 4u || nb == 8u) return (((R * nb + ((b + r) & (nb - 1u))) << 2) + (part ^ (r >> 2))) << 4;
-    if (nb == 2u) return (((R * 2u + (b ^ (r >> 3))) << 2) + (part ^ ((r >> 1) & 3u))) << 4;
-    return (((R * nb + b) << 2) + (part ^ (r >> 2))) << 4;
-}
+template <class T> __device__ __forceinline__ T load_a2(const uint8_t *p) { T v; __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), sizeof(T)); return v; }
 
-// blk: the block in LDS, sub: the group inside it (0 .. 7)
+// quarter `part` of the block at bp, and what its d is made from (dp: packed rows keep their d elsewhere)
 template <int SRC>
-__device__ __forceinline__ GroupWords group_words(const uint8_t *blk, uint32_t sub, uint32_t q) {
-    if constexpr (SRC == S_XS) {
-        return GroupWords{lds_u16(blk + 2u + 8u * sub + 2u * q), blk[66u + sub]};
-    } else if constexpr (SRC == S_M) {      // b: the qh byte of the lane's entry | scale word of the group's 64 columns << 8
-        return GroupWords{blk[4u * sub + q], blk[32u + 2u * sub + (q >> 1)] | (lds_u16(blk + 48u + 2u * (sub >> 1)) >> (6u * (sub & 1u))) << 8};
-    } else {                                // IQ3_S. b: sign byte | qh byte << 8 | scale byte << 16
-        return GroupWords{lds_u16(blk + 2u + 8u * sub + 2u * q),
-                          blk[74u + 4u * sub + q] | ((uint32_t)blk[66u + sub] << 8) | (((uint32_t)blk[106u + (sub >> 1)] >> (4u * (sub & 1u))) << 16)};
+__device__ __forceinline__ void load_quarter(const uint8_t *bp, const uint8_t *dp, uint32_t part, Quarter &v, uint2 &d) {
+    if constexpr (SRC == S_XXS || SRC == S_XS || SRC == S_IQ3) {
+        v.a = load_a2<uint4>(bp + 2u + 16u * part);
+        d.x = load_a2<uint16_t>(bp);
+    } else if constexpr (SRC == S_PACKED_XXS) {
+        v.a = *reinterpret_cast<const uint4 *>(bp + 16u * part);
+        d.x = *reinterpret_cast<const uint16_t *>(dp);
+    } else {
+        const uint2 qs = load_a2<uint2>(bp + 8u * part);
+        v.a = make_uint4(qs.x, qs.y, load_a2<uint32_t>(bp + 32u + 4u * part), load_a2<uint16_t>(bp + 48u + 2u * part));
+        d = load_a2<uint2>(bp + 48u);
+    }
+    if constexpr (SRC == S_XS) v.c = load_a2<uint16_t>(bp + 66u + 2u * part);
+    if constexpr (SRC == S_IQ3) {
+        v.b = load_a2<uint2>(bp + 74u + 8u * part);
+        v.c = load_a2<uint16_t>(bp + 66u + 2u * part) | ((uint32_t)bp[106u + part] << 16);
     }
 }
 template <int SRC>
-__device__ __forceinline__ float block_d(const uint8_t *blk) {
-    if constexpr (SRC == S_M) {
-        const uint32_t s01 = lds_u32_a2(blk + 48u), s23 = lds_u32_a2(blk + 52u);
-        return scale_to_f32(((s01 >> 12) & 0x000fu) | ((s01 >> 24) & 0x00f0u) | ((s23 >> 4) & 0x0f00u) | ((s23 >> 16) & 0xf000u));
-    } else
-        return scale_to_f32(lds_u16(blk));
+__device__ __forceinline__ float quarter_d(uint2 d) {
+    if constexpr (SRC == S_M) return scale_to_f32(((d.x >> 12) & 0x000fu) | ((d.x >> 24) & 0x00f0u) | ((d.y >> 4) & 0x0f00u) | ((d.y >> 16) & 0xf000u));
+    else return scale_to_f32(d.x);
+}
+// Where a quarter lies in LDS, in quarters: rotated blocks and exclusive-or'ed quarters spread what a wave reads together (one block of
+// sixteen rows) over all banks.
+__device__ __forceinline__ uint32_t quarter_at(uint32_t R, uint32_t b, uint32_t part, uint32_t nb) {
+    const uint32_t r = R & 15u;
+    if (nb == 4u || nb == 8u) return ((R * nb + ((b + r) & (nb - 1u))) << 2) + (part ^ (r >> 2));
+    if (nb == 2u) return ((R * 2u + (b ^ (r >> 3))) << 2) + (part ^ ((r >> 1) & 3u));
+    return ((R * nb + b) << 2) + (part ^ (r >> 2));
 }
 
 // odd integer 2 s + 1 (s < 16) as two equal fp16 halves: 1024 + (2 s + 1) by integer arithmetic, minus 1024, exact
@@ -142,54 +149,61 @@ __device__ __forceinline__ half2_t odd_splat(uint32_t s) {
 // lane constants of the tables: addresses of the lane's copy
 struct LaneTables { const uint8_t *entries; const uint8_t *signs; };
 
-// table reads of entry q (eight columns) of a group, then the arithmetic on what they return: the eight signed, scaled fp16 weights
+// Table reads of step s (eight columns) of a quarter, then the arithmetic on what they return: the eight signed, scaled fp16 weights.
+// s is a constant after unrolling.
 struct Entry { uint4 m; uint32_t s; };
+__device__ __forceinline__ uint32_t word_of(const uint4 &v, uint32_t i) { return i == 0u ? v.x : i == 1u ? v.y : i == 2u ? v.z : v.w; }
 template <int SRC>
-__device__ __forceinline__ Entry fetch_entry(const GroupWords &w, uint32_t q, const LaneTables &t) {
-    Entry e;
+__device__ __forceinline__ Entry fetch_entry(const Quarter &v, uint32_t s, const LaneTables &t) {
+    const uint32_t h = s >> 2, e = s & 3u;                 // group of the quarter, entry of the group
+    Entry r;
     if constexpr (SRC == S_XXS || SRC == S_PACKED_XXS) {
-        const uint32_t s7 = __builtin_amdgcn_ubfe(w.b, 7u * q, 7u);
+        const uint32_t wa = h ? v.a.z : v.a.x, wb = h ? v.a.w : v.a.y;
         // bytes 0 .. 3 of the permute's second operand are the entries, 7 the top byte of the first
-        e.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_perm(w.b, w.a, 0x0c0c0007u | (q << 8)) & 0xfff0u));
-        e.s = *reinterpret_cast<const uint32_t *>(t.signs + (s7 << 6));
+        r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_perm(wb, wa, 0x0c0c0007u | (e << 8)) & 0xfff0u));
+        r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(wb, 7u * e, 7u) << 6));
     } else if constexpr (SRC == S_XS) {
-        e.m = *reinterpret_cast<const uint4 *>(t.entries + ((w.a & 511u) << 7));
-        e.s = *reinterpret_cast<const uint32_t *>(t.signs + ((w.a >> 9) << 6));
+        const uint32_t w = word_of(v.a, 2u * h + (e >> 1)), o = 16u * (e & 1u);
+        r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_ubfe(w, o, 9u) << 7));
+        r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(w, o + 9u, 7u) << 6));
     } else if constexpr (SRC == S_M) {
-        const uint32_t nib = __builtin_amdgcn_ubfe(w.b, 4u * (q & 1u), 4u);
-        e.m = *reinterpret_cast<const uint4 *>(t.entries + ((w.a | ((nib & 7u) << 8)) << 5));
-        e.s = nib;
+        r.s = __builtin_amdgcn_ubfe(v.a.z, 16u * h + 4u * e, 4u);
+        r.m = *reinterpret_cast<const uint4 *>(t.entries + ((__builtin_amdgcn_ubfe(h ? v.a.y : v.a.x, 8u * e, 8u) | ((r.s & 7u) << 8)) << 5));
     } else {
-        const uint32_t scale = (w.b & 0xf0000u) >> 4;                 // nibble * 512 entries * 8 bytes
-        const uint32_t ha = (w.b << (8u - 2u * q)) >> 5, hb = (w.b << (7u - 2u * q)) >> 5;      // bit 8 + 2q / 9 + 2q of b -> bit 11
-        const uint2 ma = *reinterpret_cast<const uint2 *>(t.entries + (((w.a & 255u) << 3) | (ha & 2048u) | scale));
-        const uint2 mb = *reinterpret_cast<const uint2 *>(t.entries + (((w.a >> 8) << 3) | (hb & 2048u) | scale));
-        e.m = make_uint4(ma.x, ma.y, mb.x, mb.y);
-        e.s = *reinterpret_cast<const uint32_t *>(t.signs + ((w.b & 255u) << 4));
+        const uint32_t w = word_of(v.a, 2u * h + (e >> 1)), o = 16u * (e & 1u);
+        const uint32_t scale = h ? (v.c >> 8) & 0xf000u : (v.c >> 4) & 0xf000u;      // nibble * 512 entries * 8 bytes
+        const uint32_t ba = 8u * h + 2u * e, bb = ba + 1u;     // qh bits of the two entries -> bit 11
+        const uint32_t ha = (ba > 11u ? v.c >> (ba - 11u) : v.c << (11u - ba)) & 2048u, hb = (bb > 11u ? v.c >> (bb - 11u) : v.c << (11u - bb)) & 2048u;
+        const uint2 ma = *reinterpret_cast<const uint2 *>(t.entries + ((__builtin_amdgcn_ubfe(w, o, 8u) << 3) | ha | scale));
+        const uint2 mb = *reinterpret_cast<const uint2 *>(t.entries + ((__builtin_amdgcn_ubfe(w, o + 8u, 8u) << 3) | hb | scale));
+        r.m = make_uint4(ma.x, ma.y, mb.x, mb.y);
+        r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(h ? v.b.y : v.b.x, 8u * e, 8u) << 4));
     }
-    return e;
+    return r;
+}
+// f: the scale of the step's sixteen columns (IQ2_XS, IQ1_M), formed by step_scale
+template <int SRC>
+__device__ __forceinline__ half2_t step_scale(const Quarter &v, uint32_t s) {
+    const uint32_t h = s >> 2, e = s & 3u;
+    if constexpr (SRC == S_XS) return odd_splat(__builtin_amdgcn_ubfe(v.c, 8u * h + 4u * (e >> 1), 4u));
+    else return odd_splat(__builtin_amdgcn_ubfe(v.a.w, 6u * h + 3u * (e >> 1), 3u));
 }
 template <int SRC>
-__device__ __forceinline__ half8_t finish_entry(const Entry &e, const GroupWords &w, uint32_t q) {
+__device__ __forceinline__ half8_t finish_entry(const Entry &e, half2_t f) {
+    constexpr uint32_t kSign = 0x80008000u;
     H8 r;
+    r.u = e.m;
     if constexpr (SRC == S_M) {
-        const half2_t f = odd_splat(__builtin_amdgcn_ubfe(w.b, 8u + 3u * (q >> 1), 3u));
         // (2 s + 1) / 8 with the sign of the offset: three exponent steps down (2 s + 1 >= 1 is a normal number), sign bit by xor
         const uint32_t neg = (e.s & 8u) << 12;
         const half2_t off = __builtin_bit_cast(half2_t, (__builtin_bit_cast(uint32_t, f) - 0x0c000c00u) ^ (neg | (neg << 16)));
-        r.u = e.m;
 #pragma unroll
         for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * f + off;
-    } else {
-        constexpr uint32_t kSign = 0x80008000u;
-        r.u = e.m;
-        if constexpr (SRC == S_XS) {        // entries are signed bytes in general: the sign goes to the (positive) scale
-            const uint32_t f = __builtin_bit_cast(uint32_t, odd_splat(__builtin_amdgcn_ubfe(w.b, 4u * (q >> 1), 4u)));
+    } else if constexpr (SRC == S_XS) {     // entries are signed bytes in general: the sign goes to the (positive) scale
 #pragma unroll
-            for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * __builtin_bit_cast(half2_t, f | ((e.s << i) & kSign));
-        } else {
-            r.u.x |= e.s & kSign; r.u.y |= (e.s << 1) & kSign; r.u.z |= (e.s << 2) & kSign; r.u.w |= (e.s << 3) & kSign;
-        }
+        for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * __builtin_bit_cast(half2_t, __builtin_bit_cast(uint32_t, f) | ((e.s << i) & kSign));
+    } else {
+        r.u.x |= e.s & kSign; r.u.y |= (e.s << 1) & kSign; r.u.z |= (e.s << 2) & kSign; r.u.w |= (e.s << 3) & kSign;
     }
     return r.v;
 }
@@ -213,39 +227,19 @@ __device__ __forceinline__ void wave_lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
-// 16 bytes per lane from src to LDS at dst (wave-uniform) + 16 * lane, past the registers. Written as an instruction of its own because the
-// compiler, which cannot tell the two halves of the stage apart, otherwise waits for it before the next read of the stage: the copy of the
-// next unit would be waited for before this unit is multiplied. Completion: s_waitcnt vmcnt(0) + barrier at the head of the next unit.
-__device__ __forceinline__ void copy16_to_lds(uint32_t dst, const uint8_t *src) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory");
-}
-typedef __attribute__((address_space(3))) uint8_t *lptr_t;
-
 // Hides from the compiler that v is the same in every trip of a loop: what is cheap to form again from it must not be kept in registers
 // (which the activations need) across the loop.
 __device__ __forceinline__ uint32_t each_trip(uint32_t v) { asm volatile("" : "+v"(v)); return v; }
 
-// `pieces` 16-byte pieces from src to dst in LDS, by the whole workgroup of T threads
-template <uint32_t T>
-__device__ __forceinline__ void stage_run(uint8_t *dst, const uint8_t *src, uint32_t pieces, uint32_t wave, uint32_t lane) {
-    for (uint32_t p = 64u * wave; p < pieces; p += T)
-        if (p + lane < pieces)
-            copy16_to_lds(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)dst + p * 16u), src + (uint64_t)(p + lane) * 16u);
-}
-
 // units u0 .. u1 - 1 (unit = tile * units per tile + unit of the tile) of a tile list; SETS sets of 16 pairs per tile
-template <int SRC, int NG, bool DOWN, int SETS, uint32_t KPS>          // KP = 1 << KPS parts of K
+template <int SRC, bool DOWN, int SETS, uint32_t KP>
 __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t *tile_group, const uint32_t *tile_pair0, const uint32_t *tile_n, uint32_t u0,
                                              uint32_t u1, uint8_t *stage, float *part, const LaneTables &lt) {
-    if (u0 >= u1) return;
-    constexpr uint32_t BB = src_block<SRC>(), RUN = NG == 8 ? 8u : 2u;      // groups of one block per wave: all of them, or in pairs that never straddle blocks
-    constexpr uint32_t M = SETS == 1 ? 1u : 2u, T = staged_threads<SETS>();      // M: halves per wave
+    constexpr uint32_t NRT = staged_nrt(KP), WV = KP * NRT, T = staged_threads(SETS, KP), M = SETS == 1 ? 1u : 2u;      // M: halves per wave
+    constexpr uint32_t K = 256u * KP, RB = KP * src_block<SRC>(), seg_rows = 16u * NRT, seg = seg_rows * RB, blocks = seg_rows * KP;
+    constexpr uint32_t B_AT = blocks * 64u, C_AT = B_AT + blocks * 4u * quarter_b<SRC>(), D_AT = C_AT + blocks * 4u * quarter_c<SRC>(), segs = blocks * staged_block_bytes<SRC>();      // a half in LDS
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), w8 = wave & 7u, m_first = SETS == 1 ? wave >> 3 : 0u;
-    constexpr uint32_t KP = 1u << KPS, NRT = 8u >> KPS, K = 32u * NG * KP, nb = K / 256u;
-    constexpr uint32_t RB = nb * BB, seg_rows = 16u * NRT, seg = seg_rows * RB, blocks = seg_rows * nb;
-    const uint32_t kc = w8 & (KP - 1u), rt = w8 >> KPS;
-    constexpr uint32_t segs = src_pieces<SRC>() ? blocks * 68u : seg;      // bytes of a half in LDS (pieces: 64 bytes + the scale per block)
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), w8 = wave % WV, m_first = SETS == 1 ? wave / WV : 0u, kc = w8 % KP, rt = w8 / KP;
     const uint32_t upt = a.rows / ((DOWN ? 2u : 1u) * seg_rows), U = a.n_unique[0];
     const auto matrix_of = [&](uint32_t tile) {
         const uint32_t u = tile_group[tile];
@@ -257,81 +251,63 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
     const auto scales_of = [&](const uint8_t *mat, uint32_t j, uint32_t m) {   // packed rows: their block scales
         return mat + a.d_off + (DOWN ? (uint64_t)(2u * j + m) * blocks * 2u : m * a.mat_step + (uint64_t)j * blocks * 2u);
     };
-    // IQ2_XXS: this thread's piece (of either half), on its way through registers (plain variables and unconditional loads: an array filled
-    // under a condition ends up in scratch memory)
-    const uint32_t my_half = SETS == 1 ? wave >> 3 : 0u, my_at = my_half * segs + piece_at(((tid & 511u) >> 2) / nb, ((tid & 511u) >> 2) % nb, tid & 3u, nb);
-    uint4 piece0, piece1;
-    uint32_t scale0, scale1;
-    const auto request = [&](const uint8_t *mat, uint32_t j, uint8_t *buf) {
-        const uint8_t *run0 = run_of(mat, j, my_half), *run1 = SETS == 2 ? run_of(mat, j, 1u) : nullptr;
-        const uint32_t t = each_trip(tid & 511u), my_part = t & 3u, from_block = t >> 2 < blocks ? t >> 2 : 0u;
-        if constexpr (SRC == S_XXS) {
-            const uint32_t at = from_block * 66u, pt = at + 2u + 16u * my_part;
-            __builtin_memcpy(&piece0, __builtin_assume_aligned(run0 + pt, 2), 16);
-            scale0 = *reinterpret_cast<const uint16_t *>(run0 + at);
-            if constexpr (SETS == 2) {
-                __builtin_memcpy(&piece1, __builtin_assume_aligned(run1 + pt, 2), 16);
-                scale1 = *reinterpret_cast<const uint16_t *>(run1 + at);
-            }
-        } else if constexpr (SRC == S_PACKED_XXS) {
-            const uint32_t at = from_block * 64u + 16u * my_part;
-            piece0 = *reinterpret_cast<const uint4 *>(run0 + at);
-            scale0 = *reinterpret_cast<const uint16_t *>(scales_of(mat, j, my_half) + 2u * from_block);
-            if constexpr (SETS == 2) {
-                piece1 = *reinterpret_cast<const uint4 *>(run1 + at);
-                scale1 = *reinterpret_cast<const uint16_t *>(scales_of(mat, j, 1u) + 2u * from_block);
-            }
-        } else {
-            stage_run<T>(buf, run_of(mat, j, 0u), seg / 16u, wave, lane);
-            stage_run<T>(buf + segs, run_of(mat, j, 1u), seg / 16u, wave, lane);
-        }
+    // This thread's quarter (of either half), on its way through registers: plain variables and unconditional loads (an array filled under
+    // a condition ends up in scratch memory). 4 * blocks quarters per half, as many as threads of a half.
+    static_assert(4u * blocks == 64u * WV, "a quarter per thread and half");
+    const uint32_t my_half = m_first, my_t = tid - 64u * WV * my_half, my_at = quarter_at((my_t >> 2) / KP, (my_t >> 2) % KP, my_t & 3u, KP);
+    Quarter q0, q1;
+    uint2 d0, d1;
+    const auto request = [&](const uint8_t *mat, uint32_t j) {
+        const uint32_t t = each_trip(my_t);
+        load_quarter<SRC>(run_of(mat, j, my_half) + (t >> 2) * src_block<SRC>(), scales_of(mat, j, my_half) + (t >> 2) * 2u, t & 3u, q0, d0);
+        if constexpr (SETS == 2) load_quarter<SRC>(run_of(mat, j, 1u) + (t >> 2) * src_block<SRC>(), scales_of(mat, j, 1u) + (t >> 2) * 2u, t & 3u, q1, d1);
     };
     const auto deliver = [&](uint8_t *buf) {
-        if constexpr (src_pieces<SRC>()) {
-            const uint32_t t = each_trip(tid & 511u), my_scale_at = my_half * segs + blocks * 64u + t;      // (threads of part 0: 4 bytes per block)
-            if (t >> 2 >= blocks) return;
-            *reinterpret_cast<uint4 *>(buf + my_at) = piece0;
-            if constexpr (SETS == 2) *reinterpret_cast<uint4 *>(buf + segs + my_at) = piece1;
-            if (t & 3u) return;
-            *reinterpret_cast<float *>(buf + my_scale_at) = scale_to_f32(scale0);
-            if constexpr (SETS == 2) *reinterpret_cast<float *>(buf + segs + my_scale_at) = scale_to_f32(scale1);
-        }
+        const uint32_t t = each_trip(my_t);
+        const auto put = [&](uint8_t *half, const Quarter &v, uint2 d) {
+            *reinterpret_cast<uint4 *>(half + 16u * my_at) = v.a;
+            if constexpr (quarter_b<SRC>()) *reinterpret_cast<uint2 *>(half + B_AT + 8u * my_at) = v.b;
+            if constexpr (quarter_c<SRC>()) *reinterpret_cast<uint32_t *>(half + C_AT + 4u * my_at) = v.c;
+            if ((t & 3u) == 0u) *reinterpret_cast<float *>(half + D_AT + t) = quarter_d<SRC>(d);      // (4 bytes per block)
+        };
+        put(buf + my_half * segs, q0, d0);
+        if constexpr (SETS == 2) put(buf + segs, q1, d1);
     };
-    H8 xa[SETS][NG], xb[SETS][NG];
+    H8 xa[SETS][8], xb[SETS][8];
     float ps[SETS][4];
     // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
     const auto load_tile = [&](uint32_t p0, uint32_t n) {
 #pragma unroll
         for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
             __builtin_amdgcn_sched_barrier(0);             // one set at a time: both at once do not fit the registers
-            const uint32_t l = each_trip(lane), q8 = 8u * (l >> 4), i = 16u * s + (l & 15u), p = i < n ? p0 + i : p0;
+            const uint32_t l = each_trip(lane), q64 = 64u * (l >> 4), i = 16u * s + (l & 15u), p = i < n ? p0 + i : p0;
             float scale = SRC == S_M || SRC == S_IQ3 ? 1.0f : 0.125f;      // (the d / 8 of the IQ2 formats)
             if constexpr (!DOWN) {
                 const uint32_t tok = p < a.P ? a.pair_token[p] : p - a.P;
                 scale *= exp2i(a.xexp[tok]);
-                const uint64_t base = (uint64_t)tok * K + 32u * NG * kc + q8;
+                const uint64_t base = (uint64_t)tok * K + 256u * kc + q64;
                 const _Float16 *hp = a.xh + base, *lp = a.xl + base;
 #pragma unroll
-                for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
-                    xa[s][g].u = *reinterpret_cast<const uint4 *>(hp + 32u * g);
-                    xb[s][g].u = *reinterpret_cast<const uint4 *>(lp + 32u * g);
+                for (uint32_t g = 0; g < 8u; ++g) {
+                    xa[s][g].u = *reinterpret_cast<const uint4 *>(hp + 8u * g);
+                    xb[s][g].u = *reinterpret_cast<const uint4 *>(lp + 8u * g);
                 }
                 // the low halves are stored times 2^11: back to their own scale (exact, the largest |x| of a token sits in [2^13, 2^14)), so that a
                 // product's high and low parts add up in one accumulator
 #pragma unroll
-                for (uint32_t g = 0; g < (uint32_t)NG; ++g) xb[s][g].v = xb[s][g].v * (_Float16)4.8828125e-4f;
+                for (uint32_t g = 0; g < 8u; ++g) xb[s][g].v = xb[s][g].v * (_Float16)4.8828125e-4f;
             } else {
                 // f32 activations of pair p, columns of this wave's K part: one exponent for them, then the fp16 halves
-                const float *src = a.act + (uint64_t)p * K + 32u * NG * kc + q8;
+                const float *src = a.act + (uint64_t)p * K + 256u * kc + q64;
                 float amax = 0.0f;
 #pragma unroll
-                for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
-                    const float4 v0 = *reinterpret_cast<const float4 *>(src + 32u * g), v1 = *reinterpret_cast<const float4 *>(src + 32u * g + 4u);
+                for (uint32_t g = 0; g < 8u; ++g) {
+                    const float4 v0 = *reinterpret_cast<const float4 *>(src + 8u * g), v1 = *reinterpret_cast<const float4 *>(src + 8u * g + 4u);
                     xa[s][g].u = __builtin_bit_cast(uint4, v0);
                     xb[s][g].u = __builtin_bit_cast(uint4, v1);
                 }
 #pragma unroll
-                for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
+                for (uint32_t g = 0; g < 8u; ++g) {
                     const float4 v0 = __builtin_bit_cast(float4, xa[s][g].u), v1 = __builtin_bit_cast(float4, xb[s][g].u);
                     amax = fmaxf(amax, fmaxf(fmaxf(fmaxf(fabsf(v0.x), fabsf(v0.y)), fmaxf(fabsf(v0.z), fabsf(v0.w))), fmaxf(fmaxf(fabsf(v1.x), fabsf(v1.y)), fmaxf(fabsf(v1.z), fabsf(v1.w)))));
                 }
@@ -341,7 +317,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 const float inv = exp2i(-e);
                 scale *= exp2i(e);
 #pragma unroll
-                for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
+                for (uint32_t g = 0; g < 8u; ++g) {
                     const float4 v0 = __builtin_bit_cast(float4, xa[s][g].u), v1 = __builtin_bit_cast(float4, xb[s][g].u);
                     const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
                     H8 hi, lo;
@@ -357,11 +333,11 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 }
             }
 #pragma unroll
-            for (uint32_t t = 0; t < 4u; ++t) ps[s][t] = __shfl(scale, (int)(q8 / 2u + t), 64);
+            for (uint32_t t = 0; t < 4u; ++t) ps[s][t] = __shfl(scale, (int)(q64 / 16u + t), 64);
         }
     };
     // partial sums of the waves: [row tile, K part][m][set][lane] float4
-    constexpr uint32_t kWavePart = 2u * SETS * 256u, kPart = 8u * kWavePart;
+    constexpr uint32_t kWavePart = 2u * SETS * 256u, kPart = WV * kWavePart;
     const auto reduce = [&](uint32_t j, uint32_t p0, uint32_t n, const float *pt, uint32_t turn) {
         const uint32_t t = each_trip(tid);
         if constexpr (DOWN) {
@@ -373,7 +349,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 const uint32_t it = base + t;
                 if (N % T != 0u && it >= N) continue;
                 const uint32_t at = (it & (PB - 1u)) * V, b = it / PB, set = b & (SETS - 1u), m = (b / SETS) & 1u, slot = b / (2u * SETS);
-                const float *src = pt + (slot << KPS) * kWavePart + (m * SETS + set) * 256u + at;
+                const float *src = pt + slot * KP * kWavePart + (m * SETS + set) * 256u + at;
                 float s[V];
 #pragma unroll
                 for (uint32_t v = 0; v < V; ++v) s[v] = src[v];
@@ -396,7 +372,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 const uint32_t e = base + t - lead;
                 if (N < T && e >= N) continue;             // (wave-uniform)
                 const uint32_t at = e & 255u, b = e >> 8, set = b & (SETS - 1u), slot = b / SETS;
-                const float *src = pt + (slot << KPS) * kWavePart + set * 256u + at;
+                const float *src = pt + slot * KP * kWavePart + set * 256u + at;
                 float s0 = src[0], s1 = src[SETS * 256u];
 #pragma unroll
                 for (uint32_t k = 1; k < KP; ++k) {
@@ -408,21 +384,14 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
             }
         }
     };
-    // offsets of the lane's pieces and block scales inside a half
-    uint32_t piece_off[NG / 2], d_off[NG / RUN];
-#pragma unroll
-    for (uint32_t g2 = 0; g2 < NG / 2u; ++g2) {
-        const uint32_t gg = kc * NG + 2u * g2;
-        piece_off[g2] = src_pieces<SRC>() ? m_first * segs + piece_at(16u * rt + r, gg >> 3, (gg & 7u) >> 1, nb) : 0u;
-    }
-#pragma unroll
-    for (uint32_t b = 0; b < NG / RUN; ++b) d_off[b] = src_pieces<SRC>() ? m_first * segs + blocks * 64u + 4u * ((16u * rt + r) * nb + ((kc * NG + RUN * b) >> 3)) : 0u;
+    // the lane's quarter and block scale inside a half
+    const uint32_t lane_at = quarter_at(16u * rt + r, kc, q, KP), lane_d = D_AT + 4u * ((16u * rt + r) * KP + kc);
 
     uint32_t tile = u0 / upt, j = u0 % upt, p0 = tile_pair0[tile], n = tile_n[tile];
     uint32_t pj = 0u, pp0 = 0u, pn = 0u;                   // the unit before, whose partial sums wait in LDS
     const uint8_t *mat = matrix_of(tile);
     bool fresh = true;
-    request(mat, j, stage);
+    request(mat, j);
     deliver(stage);
     for (uint32_t u = u0; u < u1; ++u) {
         const uint32_t buf = (u - u0) & 1u;
@@ -432,81 +401,62 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
         uint32_t np0 = p0, nn = n;
         const uint8_t *nmat = mat;
         if (more && next_tile) { nmat = matrix_of(tile + 1u); np0 = tile_pair0[tile + 1u]; nn = tile_n[tile + 1u]; }
-        if constexpr (!src_pieces<SRC>()) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's share of the unit has landed
-        wave_lds_barrier();                                // everybody's has; the unit before is multiplied and its partial sums are written (first time: the tables too)
+        wave_lds_barrier();                                // the unit's rows are in place; the unit before is multiplied and its partial sums are written (first time: the tables too)
         if (u > u0) reduce(pj, pp0, pn, part + (SETS == 1 ? (buf ^ 1u) * kPart : 0u), u);
-        // the next unit's rows, behind the stores of reduce, which have the unit's time to drain. (Pieces unconditionally - the last unit
-        // fetches its own again: registers filled under a condition would be live all around the loop.)
-        if (src_pieces<SRC>() || more) request(more ? nmat : mat, more ? nj : j, stage + (buf ^ 1u) * 2u * segs);
+        // the next unit's rows, behind the stores of reduce, which have the unit's time to drain (the last unit fetches its own again:
+        // registers filled under a condition would be live all around the loop)
+        request(more ? nmat : mat, more ? nj : j);
 
-        const uint8_t *half = stage + buf * 2u * segs, *rows = half + m_first * segs + (16u * rt + r) * RB;
-        float4_t tot[M][SETS], acc[M][SETS];
-        GroupWords gw[M][NG];
-        const auto block_of = [&](uint32_t g) { return (NG == 8 ? kc : (kc * NG + g) >> 3); };
-        const auto sub_of = [&](uint32_t g) { return NG == 8 ? g : (kc * NG + g) & 7u; };
-        const auto words_of = [&](uint32_t g) {            // groups g and g + 1
+        const uint8_t *half = stage + buf * 2u * segs + m_first * segs;
+        Quarter v[M];
+        float4_t acc[M][SETS];
 #pragma unroll
-            for (uint32_t m = 0; m < M; ++m) {
-                if constexpr (src_pieces<SRC>()) {
-                    const uint4 v = *reinterpret_cast<const uint4 *>(half + m * segs + piece_off[g / 2u]);
-                    gw[m][g] = GroupWords{v.x, v.y};
-                    gw[m][g + 1u] = GroupWords{v.z, v.w};
-                } else {
-                    gw[m][g] = group_words<SRC>(rows + m * segs + block_of(g) * BB, sub_of(g), q);
-                    gw[m][g + 1u] = group_words<SRC>(rows + m * segs + block_of(g + 1u) * BB, sub_of(g + 1u), q);
-                }
-            }
-        };
-        words_of(0u);
-        words_of(2u);
+        for (uint32_t m = 0; m < M; ++m) {
+            v[m].a = *reinterpret_cast<const uint4 *>(half + m * segs + 16u * lane_at);
+            if constexpr (quarter_b<SRC>()) v[m].b = *reinterpret_cast<const uint2 *>(half + m * segs + B_AT + 8u * lane_at);
+            if constexpr (quarter_c<SRC>()) v[m].c = *reinterpret_cast<const uint32_t *>(half + m * segs + C_AT + 4u * lane_at);
 #pragma unroll
-        for (uint32_t m = 0; m < M; ++m)
-#pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) { tot[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f}; acc[m][s] = tot[m][s]; }
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) acc[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
         Entry e0[M], e1[M];
+        half2_t f[M];
 #pragma unroll
-        for (uint32_t m = 0; m < M; ++m) { e0[m] = fetch_entry<SRC>(gw[m][0], q, lt); e1[m] = fetch_entry<SRC>(gw[m][1], q, lt); }
+        for (uint32_t m = 0; m < M; ++m) { e0[m] = fetch_entry<SRC>(v[m], 0u, lt); e1[m] = fetch_entry<SRC>(v[m], 1u, lt); }
 #pragma unroll
-        for (uint32_t g = 0; g < (uint32_t)NG; ++g) {
-            // fields run four groups ahead of the arithmetic, table reads two
+        for (uint32_t s8 = 0; s8 < 8u; ++s8) {
+            // table reads run two steps ahead of the arithmetic
             __builtin_amdgcn_sched_barrier(0);
-            if ((g & 1u) == 0u && g + 4u < (uint32_t)NG) words_of(g + 4u);
             half8_t w[M];
 #pragma unroll
             for (uint32_t m = 0; m < M; ++m) {
-                w[m] = finish_entry<SRC>(g & 1u ? e1[m] : e0[m], gw[m][g], q);
-                if (g + 2u < (uint32_t)NG) { if (g & 1u) e1[m] = fetch_entry<SRC>(gw[m][g + 2u], q, lt); else e0[m] = fetch_entry<SRC>(gw[m][g + 2u], q, lt); }
+                if constexpr (SRC == S_XS || SRC == S_M) { if ((s8 & 1u) == 0u) f[m] = step_scale<SRC>(v[m], s8); }
+                w[m] = finish_entry<SRC>(s8 & 1u ? e1[m] : e0[m], f[m]);
+                if (s8 + 2u < 8u) { if (s8 & 1u) e1[m] = fetch_entry<SRC>(v[m], s8 + 2u, lt); else e0[m] = fetch_entry<SRC>(v[m], s8 + 2u, lt); }
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
-                for (uint32_t m = 0; m < M; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[s][g].v, w[m], acc[m][s], 0, 0, 0);
+                for (uint32_t m = 0; m < M; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[s][s8].v, w[m], acc[m][s], 0, 0, 0);
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
-                for (uint32_t m = 0; m < M; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[s][g].v, w[m], acc[m][s], 0, 0, 0);
-            if ((g + 1u) % RUN == 0u) {
+                for (uint32_t m = 0; m < M; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[s][s8].v, w[m], acc[m][s], 0, 0, 0);
+        }
 #pragma unroll
-                for (uint32_t m = 0; m < M; ++m) {
-                    float d;
-                    if constexpr (src_pieces<SRC>()) d = *reinterpret_cast<const float *>(half + m * segs + d_off[g / RUN]);
-                    else d = block_d<SRC>(rows + m * segs + block_of(g) * BB);
+        for (uint32_t m = 0; m < M; ++m) {
+            const float d = *reinterpret_cast<const float *>(half + m * segs + lane_d);
 #pragma unroll
-                    for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) tot[m][s][t] = fmaf(acc[m][s][t], d * ps[s][t], tot[m][s][t]);
-                        acc[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                    }
-                }
-            }
+                for (int t = 0; t < 4; ++t) acc[m][s][t] *= d * ps[s][t];
         }
         if constexpr (SETS == 2) wave_lds_barrier();       // one buffer of partial sums: those of the unit before have been read
         float *mine = part + (SETS == 1 ? buf * kPart : 0u) + w8 * kWavePart + m_first * SETS * 256u + 4u * lane;
 #pragma unroll
         for (uint32_t m = 0; m < M; ++m)
 #pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) = tot[m][s];
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) = acc[m][s];
         deliver(stage + (buf ^ 1u) * 2u * segs);           // (free since the barrier at this unit's head)
         pj = j; pp0 = p0; pn = n;
         if (next_tile && more) { ++tile; fresh = true; p0 = np0; n = nn; mat = nmat; }
@@ -520,56 +470,56 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
 // A launch that finds few wide tiles leaves them: the narrow one then takes every pair in tiles of 16 (list 0). A wide launch costs 20 us
 // however few tiles it has (tables, the first tile's activations), one more tile on the narrow kernels 0.3 us of the whole device.
 constexpr uint32_t kFewWide = 48u;
-template <int SRC, int NG, bool DOWN, int SETS, uint32_t KPS>
-__global__ __launch_bounds__(staged_threads<SETS>()) void staged_tiles_kernel(StagedArgs a) {
+template <int SRC, bool DOWN, int SETS, uint32_t KP>
+__global__ __launch_bounds__(staged_threads(SETS, KP)) void staged_tiles_kernel(StagedArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t stage[];        // two buffers of two halves of a unit
     __shared__ __attribute__((aligned(16))) uint8_t entries[kEntryBytes];   // static: table reads take immediate offsets
     __shared__ __attribute__((aligned(16))) uint32_t signs[sign_bytes<SRC>() / 4u + 4u];
-    __shared__ __attribute__((aligned(16))) float part[2u * 8u * 2u * 256u];
+    __shared__ __attribute__((aligned(16))) float part[2u * KP * staged_nrt(KP) * 2u * 256u];
     const bool few = a.n_tiles[1] < kFewWide;
     if (SETS == 2 && few) return;
     const uint32_t tid = threadIdx.x, l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
-    const uint32_t units = a.n_tiles[l] * (a.rows / ((DOWN ? 32u : 16u) * (8u >> KPS)));
+    const uint32_t units = a.n_tiles[l] * (a.rows / ((DOWN ? 32u : 16u) * staged_nrt(KP)));
     // workgroups are dealt round-robin over the eight XCDs: neighbouring runs (which share tiles) go to one XCD's L2
     const uint32_t G = gridDim.x, at = G % 8u == 0u ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
     const uint32_t u0 = (uint32_t)((uint64_t)at * units / G), u1 = (uint32_t)((uint64_t)(at + 1u) * units / G);
     if (u0 >= u1) return;
-    build_staged_tables<SRC, staged_threads<SETS>()>(entries, signs, tid, a.grid);
+    build_staged_tables<SRC, staged_threads(SETS, KP)>(entries, signs, tid, a.grid);
     const LaneTables lt{entries + (SRC == S_XS ? (tid & 7u) * 16u : SRC == S_M ? (tid & 1u) * 16u : 0u),
                         reinterpret_cast<const uint8_t *>(signs) + (SRC == S_IQ3 ? (tid & 3u) * 4u : SRC == S_M ? 0u : (tid & 15u) * 4u)};
-    staged_units<SRC, NG, DOWN, SETS, KPS>(a, a.tile_group + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, stage, part, lt);
+    staged_units<SRC, DOWN, SETS, KP>(a, a.tile_group + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, stage, part, lt);
 }
 
-template <int SRC, int NG, bool DOWN, int SETS, uint32_t KPS>
+template <int SRC, bool DOWN, int SETS, uint32_t KP>
 hipError_t launch_staged_list(const StagedArgs &a, uint32_t grid, hipStream_t s) {
-    constexpr size_t lds = (size_t)4u * 16u * (8u >> KPS) * (NG << KPS) / 8u * (src_pieces<SRC>() ? 68u : src_block<SRC>());
+    constexpr size_t lds = (size_t)4u * 16u * staged_nrt(KP) * KP * staged_block_bytes<SRC>();
     static bool attr = false;
     if (!attr) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(staged_tiles_kernel<SRC, NG, DOWN, SETS, KPS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(staged_tiles_kernel<SRC, DOWN, SETS, KP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         attr = true;
     }
-    REDHIP_LAUNCH((staged_tiles_kernel<SRC, NG, DOWN, SETS, KPS>), dim3(grid), dim3(staged_threads<SETS>()), lds, s, a);
+    REDHIP_LAUNCH((staged_tiles_kernel<SRC, DOWN, SETS, KP>), dim3(grid), dim3(staged_threads(SETS, KP)), lds, s, a);
     return hipGetLastError();
 }
 // wide: the chunk can have tiles of more than 16 pairs
-template <int SRC, int NG, bool DOWN, uint32_t KPS>
+template <int SRC, bool DOWN, uint32_t KP>
 hipError_t launch_staged_lists(const StagedArgs &a, uint32_t grid, bool wide, hipStream_t s) {
-    const hipError_t e = wide ? launch_staged_list<SRC, NG, DOWN, 2, KPS>(a, grid, s) : hipSuccess;
-    return e == hipSuccess ? launch_staged_list<SRC, NG, DOWN, 1, KPS>(a, grid, s) : e;
+    const hipError_t e = wide ? launch_staged_list<SRC, DOWN, 2, KP>(a, grid, s) : hipSuccess;
+    return e == hipSuccess ? launch_staged_list<SRC, DOWN, 1, KP>(a, grid, s) : e;
 }
 template <int SRC>
 hipError_t launch_staged_gateup(const StagedArgs &a, uint32_t hidden, uint32_t grid, bool wide, hipStream_t s) {
-    return hidden == 512u    ? launch_staged_lists<SRC, 8, false, 1>(a, grid, wide, s)
-           : hidden == 1024u ? launch_staged_lists<SRC, 8, false, 2>(a, grid, wide, s)
-                             : launch_staged_lists<SRC, 8, false, 3>(a, grid, wide, s);
+    return hidden == 512u    ? launch_staged_lists<SRC, false, 2>(a, grid, wide, s)
+           : hidden == 1024u ? launch_staged_lists<SRC, false, 4>(a, grid, wide, s)
+                             : launch_staged_lists<SRC, false, 8>(a, grid, wide, s);
 }
 template <int SRC>
 hipError_t launch_staged_down(const StagedArgs &a, uint32_t ffn, uint32_t grid, bool wide, hipStream_t s) {
-    return ffn == 256u   ? launch_staged_lists<SRC, 8, true, 0>(a, grid, wide, s)
-           : ffn == 512u ? launch_staged_lists<SRC, 8, true, 1>(a, grid, wide, s)
-           : ffn == 768u ? launch_staged_lists<SRC, 6, true, 2>(a, grid, wide, s)
-                         : launch_staged_lists<SRC, 8, true, 2>(a, grid, wide, s);
+    return ffn == 256u   ? launch_staged_lists<SRC, true, 1>(a, grid, wide, s)
+           : ffn == 512u ? launch_staged_lists<SRC, true, 2>(a, grid, wide, s)
+           : ffn == 768u ? launch_staged_lists<SRC, true, 3>(a, grid, wide, s)
+                         : launch_staged_lists<SRC, true, 4>(a, grid, wide, s);
 }
 
 int staged_src(uint32_t type, bool packed) {
@@ -579,7 +529,7 @@ int staged_src(uint32_t type, bool packed) {
 
 }  // namespace
 
-// hidden: one K part of 256 columns per wave, two to eight of them; ffn: 256, 512, 1024 likewise, 768 as four parts of 192
+// one block of 256 columns per wave: two to eight of them (hidden), one to four (ffn)
 bool staged_tiles_supported(uint32_t gate_up_type, uint32_t down_type, uint32_t hidden, uint32_t ffn, uint32_t n_expert, bool packed) {
     const int g = staged_src(gate_up_type, packed), d = staged_src(down_type, packed);
     return g >= 0 && g != S_IQ3 && d >= 0 && (hidden == 512u || hidden == 1024u || hidden == 2048u) && (ffn == 256u || ffn == 512u || ffn == 768u || ffn == 1024u) && n_expert <= 1024u;

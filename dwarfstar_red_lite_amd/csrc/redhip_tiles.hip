@@ -3,25 +3,25 @@
 // IQ2_XS, IQ1_M and (down) IQ3_S, or packed IQ2_XXS rows.
 //
 // What bounds these kernels is the decode (LDS table reads and vector issue; every weight is decoded once per tile), so the rows must cost
-// nothing extra. GGUF rows are 2-byte aligned blocks of 56 .. 110 bytes: fetched by the lanes that multiply them, a wave-wide load would
-// touch 16 rows x 32 bytes and every line several times; staged as they lie, 16-byte LDS reads of them are unaligned (more than half of the
-// kernel's LDS cycles were unaligned stalls). Instead every thread of the workgroup carries the fields of a quarter block (64 columns) through
-// its registers, one unit ahead of the arithmetic, to an aligned place in LDS.
+// nothing extra. Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights
+// of row r, D[i = 4q .. 4q + 3][j = r]: the lane's own row against four pairs. Which columns the instruction's k stand for is free as
+// long as both operands agree: step s of a block of 256 columns takes columns 64 q + 8 s .. + 7 of it, so lane (r, q) decodes quarter q of
+// its row's block and nothing else. Its fields are one 16-byte load (XS 4, IQ3_S 12 more bytes) that no other lane repeats, the four lanes
+// of a row read 64 consecutive bytes, every bit position is a constant, and a scale (per 16 or 32 columns) is formed once for the
+// entries that share it. (With step s = group s of the block, every lane of a row loaded all of it: four times the requests; rows staged in LDS
+// as they lie, 2-byte aligned: more than half of the LDS cycles were unaligned stalls.)
 //
 // K is cut into KP blocks of 256 columns, and NRT row tiles of 16 rows are in work beside each other (KP * NRT = 8; 6 with three
 // blocks). A unit is two halves ("m") of 16 NRT rows: the gate and the up rows of 16 NRT FFN columns, or 32 NRT rows of a down matrix.
-// A wave keeps the activations of its block for the whole tile in registers (fp16 hi and lo halves, 22 significant bits); the blocks
-// meet in LDS. Tiles of up to 16 pairs run sixteen waves, one half each (64 registers of activations, four waves per SIMD: the reads and
-// the arithmetic of different waves overlap), tiles of 17 .. 32 pairs eight waves with both halves and two sets of pairs per decoded
-// weight, as a launch of their own. The SwiGLU activations go to the down kernel as f32, so work is cut at any unit, not at groups of
-// columns that share an exponent; the down kernel splits them per pair and block when it loads them.
-//
-// Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights of row r,
-// D[i = 4q .. 4q + 3][j = r]: the lane's own row against four pairs. Which columns the instruction's k stand for is free as long as both
-// operands agree: step s of a block takes columns 64 q + 8 s .. + 7 of it, so lane (r, q) decodes quarter q of its row's block and
-// nothing else - its fields are one aligned 16-byte read (XS 4, IQ3_S 12 more bytes), every bit position is a constant, and a scale
-// (per 16 or 32 columns) is formed once for the entries that share it.
+// A wave keeps the activations of its block for the whole tile in registers (fp16 hi and lo halves, 22 significant bits) and the rows of
+// the next two units on their way; the blocks meet in LDS, one barrier per two units. Tiles of up to 16 pairs run sixteen waves, one half
+// each (64 registers of activations, four waves per SIMD: the reads and the arithmetic of different waves overlap), tiles of 17 .. 32
+// pairs eight waves with both halves and two sets of pairs per decoded weight, as a launch of their own. The SwiGLU activations go to
+// the down kernel as f32, so work is cut at any unit, not at groups of columns that share an exponent; the down kernel splits them per
+// pair and block when it loads them.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "redhip_mfma.h"
 
@@ -100,9 +100,6 @@ __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *
 //   IQ2_XXS  a: the two groups' words                     IQ2_XS  a: eight 16-bit entries, c: two scale bytes
 //   IQ1_M    a: 8 index bytes | 4 bytes of nibbles | scale word     IQ3_S   a: 16 index bytes, b: 8 sign bytes, c: two qh bytes | scale byte << 16
 struct Quarter { uint4 a; uint2 b; uint32_t c; };
-template <int SRC> constexpr uint32_t quarter_b() { return SRC == S_IQ3 ? 8u : 0u; }                       // bytes of b and c in LDS
-template <int SRC> constexpr uint32_t quarter_c() { return SRC == S_IQ3 || SRC == S_XS ? 4u : 0u; }
-template <int SRC> constexpr uint32_t staged_block_bytes() { return 4u * (16u + quarter_b<SRC>() + quarter_c<SRC>()) + 4u; }      // of a block in LDS: its quarters, then d as f32
 
 template <class T> __device__ __forceinline__ T load_a2(const uint8_t *p) { T v; __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), sizeof(T)); return v; }
 
@@ -131,15 +128,6 @@ __device__ __forceinline__ float quarter_d(uint2 d) {
     if constexpr (SRC == S_M) return scale_to_f32(((d.x >> 12) & 0x000fu) | ((d.x >> 24) & 0x00f0u) | ((d.y >> 4) & 0x0f00u) | ((d.y >> 16) & 0xf000u));
     else return scale_to_f32(d.x);
 }
-// Where a quarter lies in LDS, in quarters: rotated blocks and exclusive-or'ed quarters spread what a wave reads together (one block of
-// sixteen rows) over all banks.
-__device__ __forceinline__ uint32_t quarter_at(uint32_t R, uint32_t b, uint32_t part, uint32_t nb) {
-    const uint32_t r = R & 15u;
-    if (nb == 4u || nb == 8u) return ((R * nb + ((b + r) & (nb - 1u))) << 2) + (part ^ (r >> 2));
-    if (nb == 2u) return ((R * 2u + (b ^ (r >> 3))) << 2) + (part ^ ((r >> 1) & 3u));
-    return ((R * nb + b) << 2) + (part ^ (r >> 2));
-}
-
 // odd integer 2 s + 1 (s < 16) as two equal fp16 halves: 1024 + (2 s + 1) by integer arithmetic, minus 1024, exact
 __device__ __forceinline__ half2_t odd_splat(uint32_t s) {
     const half2_t big = {(_Float16)1024.0f, (_Float16)1024.0f};
@@ -231,19 +219,24 @@ __device__ __forceinline__ void wave_lds_barrier() {
 // (which the activations need) across the loop.
 __device__ __forceinline__ uint32_t each_trip(uint32_t v) { asm volatile("" : "+v"(v)); return v; }
 
+// What the units of a workgroup need to know of their tiles, fetched once at the kernel's head (a tile's entry, its expert's address, its
+// pairs' tokens and their exponents are four dependent trips to memory); tiles beyond the first kTileInfos are looked up when they begin.
+constexpr uint32_t kTileInfos = 32u;
+struct TileInfo { uint64_t mat; uint32_t p0, n; };      // mat: distance of the expert's first matrix from StagedArgs::experts
+struct PairInfo { uint32_t tok; float scale; };      // gate/up: token of a pair, its power of two (with the d / 8 of the IQ2 formats)
+
 // units u0 .. u1 - 1 (unit = tile * units per tile + unit of the tile) of a tile list; SETS sets of 16 pairs per tile
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
 __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t *tile_group, const uint32_t *tile_pair0, const uint32_t *tile_n, uint32_t u0,
-                                             uint32_t u1, uint8_t *stage, float *part, const LaneTables &lt) {
+                                             uint32_t u1, float *part, TileInfo *tiles, PairInfo *pairs, uint8_t *entries, uint32_t *signs, const LaneTables &lt) {
     constexpr uint32_t NRT = staged_nrt(KP), WV = KP * NRT, T = staged_threads(SETS, KP), M = SETS == 1 ? 1u : 2u;      // M: halves per wave
     constexpr uint32_t K = 256u * KP, RB = KP * src_block<SRC>(), seg_rows = 16u * NRT, seg = seg_rows * RB, blocks = seg_rows * KP;
-    constexpr uint32_t B_AT = blocks * 64u, C_AT = B_AT + blocks * 4u * quarter_b<SRC>(), D_AT = C_AT + blocks * 4u * quarter_c<SRC>(), segs = blocks * staged_block_bytes<SRC>();      // a half in LDS
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), w8 = wave % WV, m_first = SETS == 1 ? wave / WV : 0u, kc = w8 % KP, rt = w8 / KP;
     const uint32_t upt = a.rows / ((DOWN ? 2u : 1u) * seg_rows), U = a.n_unique[0];
     const auto matrix_of = [&](uint32_t tile) {
         const uint32_t u = tile_group[tile];
-        return u == U ? a.shared : a.experts + (uint64_t)a.uid[u] * a.stride;
+        return u == U ? (uint64_t)(a.shared - a.experts) : (uint64_t)a.uid[u] * a.stride;
     };
     const auto run_of = [&](const uint8_t *mat, uint32_t j, uint32_t m) {      // rows of half m of unit j
         return mat + (DOWN ? (uint64_t)(2u * j + m) * seg : m * a.mat_step + (uint64_t)j * seg);
@@ -251,41 +244,52 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
     const auto scales_of = [&](const uint8_t *mat, uint32_t j, uint32_t m) {   // packed rows: their block scales
         return mat + a.d_off + (DOWN ? (uint64_t)(2u * j + m) * blocks * 2u : m * a.mat_step + (uint64_t)j * blocks * 2u);
     };
-    // This thread's quarter (of either half), on its way through registers: plain variables and unconditional loads (an array filled under
-    // a condition ends up in scratch memory). 4 * blocks quarters per half, as many as threads of a half.
-    static_assert(4u * blocks == 64u * WV, "a quarter per thread and half");
-    const uint32_t my_half = m_first, my_t = tid - 64u * WV * my_half, my_at = quarter_at((my_t >> 2) / KP, (my_t >> 2) % KP, my_t & 3u, KP);
-    Quarter q0, q1;
-    uint2 d0, d1;
-    const auto request = [&](const uint8_t *mat, uint32_t j) {
-        const uint32_t t = each_trip(my_t);
-        load_quarter<SRC>(run_of(mat, j, my_half) + (t >> 2) * src_block<SRC>(), scales_of(mat, j, my_half) + (t >> 2) * 2u, t & 3u, q0, d0);
-        if constexpr (SETS == 2) load_quarter<SRC>(run_of(mat, j, 1u) + (t >> 2) * src_block<SRC>(), scales_of(mat, j, 1u) + (t >> 2) * 2u, t & 3u, q1, d1);
+    // the lane's quarters of a unit, and what their d are made from
+    struct Carried { Quarter v[M]; uint2 d[M]; };
+    const uint32_t lane_block = (16u * rt + r) * KP + kc;
+    const auto request = [&](Carried &c, const uint8_t *mat, uint32_t j) {
+        const uint32_t b = each_trip(lane_block);
+#pragma unroll
+        for (uint32_t m = 0; m < M; ++m) load_quarter<SRC>(run_of(mat, j, m_first + m) + b * src_block<SRC>(), scales_of(mat, j, m_first + m) + b * 2u, q, c.v[m], c.d[m]);
     };
-    const auto deliver = [&](uint8_t *buf) {
-        const uint32_t t = each_trip(my_t);
-        const auto put = [&](uint8_t *half, const Quarter &v, uint2 d) {
-            *reinterpret_cast<uint4 *>(half + 16u * my_at) = v.a;
-            if constexpr (quarter_b<SRC>()) *reinterpret_cast<uint2 *>(half + B_AT + 8u * my_at) = v.b;
-            if constexpr (quarter_c<SRC>()) *reinterpret_cast<uint32_t *>(half + C_AT + 4u * my_at) = v.c;
-            if ((t & 3u) == 0u) *reinterpret_cast<float *>(half + D_AT + t) = quarter_d<SRC>(d);      // (4 bytes per block)
-        };
-        put(buf + my_half * segs, q0, d0);
-        if constexpr (SETS == 2) put(buf + segs, q1, d1);
+    const uint32_t tile0 = u0 / upt, n_info = (u1 - 1u) / upt + 1u - tile0 < kTileInfos ? (u1 - 1u) / upt + 1u - tile0 : kTileInfos;
+    const auto pair_info = [&](uint32_t p0, uint32_t n, uint32_t i) {          // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
+        const uint32_t p = i < n ? p0 + i : p0, tok = p < a.P ? a.pair_token[p] : p - a.P;
+        return PairInfo{tok, (SRC == S_M || SRC == S_IQ3 ? 1.0f : 0.125f) * exp2i(a.xexp[tok])};
+    };
+    {
+        TileInfo ti{};
+        PairInfo pi{};
+        const uint32_t pt = tid / (16u * SETS), pk = tid % (16u * SETS);      // (T >= 384 threads serve at least 12 tiles per round)
+        if (tid < n_info) ti = TileInfo{matrix_of(tile0 + tid), tile_pair0[tile0 + tid], tile_n[tile0 + tid]};
+        if (!DOWN && pt < n_info) pi = pair_info(tile_pair0[tile0 + pt], tile_n[tile0 + pt], pk);
+        build_staged_tables<SRC, T>(entries, signs, tid, a.grid);
+        if (tid < n_info) tiles[tid] = ti;
+        if (!DOWN && pt < n_info) pairs[tid] = pi;
+        if constexpr (!DOWN)
+            for (uint32_t k = tid + T; k < n_info * 16u * SETS; k += T) pairs[k] = pair_info(tile_pair0[tile0 + k / (16u * SETS)], tile_n[tile0 + k / (16u * SETS)], k % (16u * SETS));
+    }
+    __syncthreads();
+    const auto uniform64 = [](uint64_t v) {
+        return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
+    };
+    const auto info_of = [&](uint32_t tile) {
+        if (tile - tile0 >= kTileInfos) return TileInfo{matrix_of(tile), tile_pair0[tile], tile_n[tile]};
+        const TileInfo ti = tiles[tile - tile0];
+        return TileInfo{uniform64(ti.mat), (uint32_t)__builtin_amdgcn_readfirstlane(ti.p0), (uint32_t)__builtin_amdgcn_readfirstlane(ti.n)};
     };
     H8 xa[SETS][8], xb[SETS][8];
     float ps[SETS][4];
-    // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
-    const auto load_tile = [&](uint32_t p0, uint32_t n) {
+    const auto load_tile = [&](uint32_t tile, uint32_t p0, uint32_t n) {
 #pragma unroll
         for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
             __builtin_amdgcn_sched_barrier(0);             // one set at a time: both at once do not fit the registers
-            const uint32_t l = each_trip(lane), q64 = 64u * (l >> 4), i = 16u * s + (l & 15u), p = i < n ? p0 + i : p0;
-            float scale = SRC == S_M || SRC == S_IQ3 ? 1.0f : 0.125f;      // (the d / 8 of the IQ2 formats)
+            const uint32_t l = each_trip(lane), q64 = 64u * (l >> 4), i = 16u * s + (l & 15u);
+            float scale;
             if constexpr (!DOWN) {
-                const uint32_t tok = p < a.P ? a.pair_token[p] : p - a.P;
-                scale *= exp2i(a.xexp[tok]);
-                const uint64_t base = (uint64_t)tok * K + 256u * kc + q64;
+                const PairInfo pi = tile - tile0 < kTileInfos ? pairs[(tile - tile0) * 16u * SETS + i] : pair_info(p0, n, i);
+                scale = pi.scale;
+                const uint64_t base = (uint64_t)pi.tok * K + 256u * kc + q64;
                 const _Float16 *hp = a.xh + base, *lp = a.xl + base;
 #pragma unroll
                 for (uint32_t g = 0; g < 8u; ++g) {
@@ -296,9 +300,10 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 // product's high and low parts add up in one accumulator
 #pragma unroll
                 for (uint32_t g = 0; g < 8u; ++g) xb[s][g].v = xb[s][g].v * (_Float16)4.8828125e-4f;
+                if (s + 1u == (uint32_t)SETS) __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): waited for here, once per tile, not (by count) where the loop uses them
             } else {
                 // f32 activations of pair p, columns of this wave's K part: one exponent for them, then the fp16 halves
-                const float *src = a.act + (uint64_t)p * K + 256u * kc + q64;
+                const float *src = a.act + (uint64_t)(i < n ? p0 + i : p0) * K + 256u * kc + q64;
                 float amax = 0.0f;
 #pragma unroll
                 for (uint32_t g = 0; g < 8u; ++g) {
@@ -315,7 +320,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
                 const int e = prescale_exp(amax);
                 const float inv = exp2i(-e);
-                scale *= exp2i(e);
+                scale = (SRC == S_M || SRC == S_IQ3 ? 1.0f : 0.125f) * exp2i(e);
 #pragma unroll
                 for (uint32_t g = 0; g < 8u; ++g) {
                     const float4 v0 = __builtin_bit_cast(float4, xa[s][g].u), v1 = __builtin_bit_cast(float4, xb[s][g].u);
@@ -328,6 +333,8 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                         hi.e[k] = h;
                         lo.e[k] = (_Float16)(t - (float)h);
                     }
+                    // group by group (the compiler otherwise works on several at once and spills)
+                    asm volatile("" : "+v"(hi.u.x), "+v"(hi.u.y), "+v"(hi.u.z), "+v"(hi.u.w), "+v"(lo.u.x), "+v"(lo.u.y), "+v"(lo.u.z), "+v"(lo.u.w));
                     xa[s][g].u = hi.u;
                     xb[s][g].u = lo.u;
                 }
@@ -337,91 +344,90 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
         }
     };
     // partial sums of the waves: [row tile, K part][m][set][lane] float4
-    constexpr uint32_t kWavePart = 2u * SETS * 256u, kPart = WV * kWavePart;
-    const auto reduce = [&](uint32_t j, uint32_t p0, uint32_t n, const float *pt, uint32_t turn) {
+    constexpr uint32_t kWavePart = 2u * SETS * 256u, kPart = WV * kWavePart;      // (kPart: of a unit)
+    struct Done { uint32_t j, p0, n; };                    // a unit whose partial sums are in LDS
+    // The sums of UNITS units (w[0], and w[1] behind it). No wave and no lane may skip a store: the loads of the next units are in flight
+    // behind it, and the compiler, which waits for them by counting memory operations in order, can count only what every path issues
+    // (with a branch around it, every unit waited for the newest of its loads). Pairs beyond a tile's n fall out of the buffer's range.
+    const auto tile_buffer = [&](float *base, uint32_t n) { return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)(n * a.rows * 4u), 0x00027000); };
+    const auto reduce = [&](auto units, const Done *w, const float *pt) {
+        constexpr uint32_t UNITS = decltype(units)::value;
         const uint32_t t = each_trip(tid);
         if constexpr (DOWN) {
-            // V consecutive floats (pairs of one row) per thread
+            // V consecutive floats (pairs of one row) per thread; threads beyond the last repeat it
             constexpr uint32_t V = SETS == 1 ? 2u : 4u, PB = 256u / V, N = PB * SETS * 2u * NRT;
-            float *out = (p0 < a.P ? a.tmp + (uint64_t)p0 * a.rows : a.sh_tmp + (uint64_t)(p0 - a.P) * a.rows) + j * 2u * seg_rows;      // (a tile is routed or shared as a whole)
 #pragma unroll
-            for (uint32_t base = 0; base < N; base += T) {
-                const uint32_t it = base + t;
-                if (N % T != 0u && it >= N) continue;
-                const uint32_t at = (it & (PB - 1u)) * V, b = it / PB, set = b & (SETS - 1u), m = (b / SETS) & 1u, slot = b / (2u * SETS);
-                const float *src = pt + slot * KP * kWavePart + (m * SETS + set) * 256u + at;
-                float s[V];
+            for (uint32_t un = 0; un < UNITS; ++un) {
+                const bool routed = w[un].p0 < a.P;        // (a tile is routed or shared as a whole)
+                const auto buf = tile_buffer((routed ? a.tmp + (uint64_t)w[un].p0 * a.rows : a.sh_tmp + (uint64_t)(w[un].p0 - a.P) * a.rows), w[un].n);
 #pragma unroll
-                for (uint32_t v = 0; v < V; ++v) s[v] = src[v];
+                for (uint32_t base = 0; base < N; base += T) {
+                    const uint32_t it = N % T ? min(base + t, N - 1u) : base + t;
+                    const uint32_t at = (it & (PB - 1u)) * V, b = it / PB, set = b & (SETS - 1u), m = (b / SETS) & 1u, slot = b / (2u * SETS);
+                    const float *src = pt + un * kPart + slot * KP * kWavePart + (m * SETS + set) * 256u + at;
+                    float s[V];
 #pragma unroll
-                for (uint32_t k = 1; k < KP; ++k)
+                    for (uint32_t v = 0; v < V; ++v) s[v] = src[v];
 #pragma unroll
-                    for (uint32_t v = 0; v < V; ++v) s[v] += src[k * kWavePart + v];
-                const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u);
-                float *o = out + (uint64_t)i * a.rows + m * seg_rows + 16u * slot + ((at >> 2) & 15u);
+                    for (uint32_t k = 1; k < KP; ++k)
 #pragma unroll
-                for (uint32_t v = 0; v < V; ++v)
-                    if (i + v < n) o[(uint64_t)v * a.rows] = s[v];
+                        for (uint32_t v = 0; v < V; ++v) s[v] += src[k * kWavePart + v];
+                    const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u), off = 4u * (i * a.rows + w[un].j * 2u * seg_rows + m * seg_rows + 16u * slot + ((at >> 2) & 15u));
+#pragma unroll
+                    for (uint32_t v = 0; v < V; ++v) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s[v]), buf, off + 4u * v * a.rows, 0, 0);
+                }
             }
         } else {
-            // one (pair, column) element per thread; where the elements are fewer than the threads, the waves take turns
-            constexpr uint32_t N = 256u * SETS * NRT;
-            const uint32_t lead = N < T ? (turn % (T / N)) * N : 0u;
+            // (pair, column) elements; L lanes of a wave (halves of it) share one where there are fewer elements than threads
+            constexpr uint32_t N = 256u * SETS * NRT * UNITS, L = N < T ? T / N : 1u;
+            static_assert(L <= 4u && KP % L == 0u, "K parts per lane");
 #pragma unroll
             for (uint32_t base = 0; base < N; base += T) {
-                const uint32_t e = base + t - lead;
-                if (N < T && e >= N) continue;             // (wave-uniform)
-                const uint32_t at = e & 255u, b = e >> 8, set = b & (SETS - 1u), slot = b / SETS;
-                const float *src = pt + slot * KP * kWavePart + set * 256u + at;
+                const uint32_t ln = t & 63u, e = base + (L == 1u ? t : (t >> 6) * (64u / L) + (ln & (64u / L - 1u))), k0 = L == 1u ? 0u : (ln / (64u / L)) * (KP / L);
+                const uint32_t at = e & 255u, b = (e >> 8) % (SETS * NRT), un = (e >> 8) / (SETS * NRT), set = b & (SETS - 1u), slot = b / SETS;
+                const float *src = pt + un * kPart + (slot * KP + k0) * kWavePart + set * 256u + at;
                 float s0 = src[0], s1 = src[SETS * 256u];
 #pragma unroll
-                for (uint32_t k = 1; k < KP; ++k) {
+                for (uint32_t k = 1; k < KP / L; ++k) {
                     s0 += src[k * kWavePart];
                     s1 += src[k * kWavePart + SETS * 256u];
                 }
+                if constexpr (L >= 2u) { s0 += __shfl_xor(s0, 32, 64); s1 += __shfl_xor(s1, 32, 64); }
+                if constexpr (L == 4u) { s0 += __shfl_xor(s0, 16, 64); s1 += __shfl_xor(s1, 16, 64); }
+                // (the wave's elements are of one unit)
+                const uint32_t uw = UNITS == 1u ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(un);
+                const Done d = uw ? w[UNITS - 1u] : w[0];
+                const auto buf = tile_buffer(a.act + (uint64_t)d.p0 * a.rows, d.n);
                 const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u);
-                if (i < n) a.act[(uint64_t)(p0 + i) * a.rows + j * seg_rows + 16u * slot + ((at >> 2) & 15u)] = (s0 / (1.0f + expf(-s0))) * s1;
+                // (of the lanes that share an element the first stores; the others' offset lies beyond every buffer)
+                const uint32_t off = k0 == 0u ? 4u * (i * a.rows + d.j * seg_rows + 16u * slot + ((at >> 2) & 15u)) : 0x7fffffffu;
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((s0 / (1.0f + expf(-s0))) * s1), buf, off, 0, 0);
             }
         }
     };
-    // the lane's quarter and block scale inside a half
-    const uint32_t lane_at = quarter_at(16u * rt + r, kc, q, KP), lane_d = D_AT + 4u * ((16u * rt + r) * KP + kc);
-
-    uint32_t tile = u0 / upt, j = u0 % upt, p0 = tile_pair0[tile], n = tile_n[tile];
-    uint32_t pj = 0u, pp0 = 0u, pn = 0u;                   // the unit before, whose partial sums wait in LDS
-    const uint8_t *mat = matrix_of(tile);
-    bool fresh = true;
-    request(mat, j);
-    deliver(stage);
-    for (uint32_t u = u0; u < u1; ++u) {
-        const uint32_t buf = (u - u0) & 1u;
-        if (fresh) { load_tile(p0, n); fresh = false; }
-        const bool more = u + 1u < u1, next_tile = j + 1u == upt;
-        const uint32_t nj = next_tile ? 0u : j + 1u;
-        uint32_t np0 = p0, nn = n;
-        const uint8_t *nmat = mat;
-        if (more && next_tile) { nmat = matrix_of(tile + 1u); np0 = tile_pair0[tile + 1u]; nn = tile_n[tile + 1u]; }
-        wave_lds_barrier();                                // the unit's rows are in place; the unit before is multiplied and its partial sums are written (first time: the tables too)
-        if (u > u0) reduce(pj, pp0, pn, part + (SETS == 1 ? (buf ^ 1u) * kPart : 0u), u);
-        // the next unit's rows, behind the stores of reduce, which have the unit's time to drain (the last unit fetches its own again:
-        // registers filled under a condition would be live all around the loop)
-        request(more ? nmat : mat, more ? nj : j);
-
-        const uint8_t *half = stage + buf * 2u * segs + m_first * segs;
-        Quarter v[M];
+    uint32_t tile = tile0, j = u0 % upt, ftile = tile0, fj = j, fleft = u1 - u0;      // f..: the unit to be requested next
+    TileInfo cur = info_of(tile);
+    uint64_t fmat = cur.mat;
+    const auto request_next = [&](Carried &c) {            // (the last units fetch theirs again: registers filled under a condition would be live all around the loop)
+        request(c, a.experts + fmat, fj);
+        if (fleft <= 1u) return;
+        --fleft;
+        if (++fj == upt) { fj = 0u; fmat = info_of(++ftile).mat; }
+    };
+    // multiplies the unit whose rows are in c into partial sums at pt and requests the unit two after it in their place
+    const auto unit = [&](uint32_t u, Carried &c, float *pt) {
         float4_t acc[M][SETS];
+        float d[M];
 #pragma unroll
         for (uint32_t m = 0; m < M; ++m) {
-            v[m].a = *reinterpret_cast<const uint4 *>(half + m * segs + 16u * lane_at);
-            if constexpr (quarter_b<SRC>()) v[m].b = *reinterpret_cast<const uint2 *>(half + m * segs + B_AT + 8u * lane_at);
-            if constexpr (quarter_c<SRC>()) v[m].c = *reinterpret_cast<const uint32_t *>(half + m * segs + C_AT + 4u * lane_at);
+            d[m] = quarter_d<SRC>(c.d[m]);
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s) acc[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
         Entry e0[M], e1[M];
         half2_t f[M];
 #pragma unroll
-        for (uint32_t m = 0; m < M; ++m) { e0[m] = fetch_entry<SRC>(v[m], 0u, lt); e1[m] = fetch_entry<SRC>(v[m], 1u, lt); }
+        for (uint32_t m = 0; m < M; ++m) { e0[m] = fetch_entry<SRC>(c.v[m], 0u, lt); e1[m] = fetch_entry<SRC>(c.v[m], 1u, lt); }
 #pragma unroll
         for (uint32_t s8 = 0; s8 < 8u; ++s8) {
             // table reads run two steps ahead of the arithmetic
@@ -429,11 +435,12 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
             half8_t w[M];
 #pragma unroll
             for (uint32_t m = 0; m < M; ++m) {
-                if constexpr (SRC == S_XS || SRC == S_M) { if ((s8 & 1u) == 0u) f[m] = step_scale<SRC>(v[m], s8); }
+                if constexpr (SRC == S_XS || SRC == S_M) { if ((s8 & 1u) == 0u) f[m] = step_scale<SRC>(c.v[m], s8); }
                 w[m] = finish_entry<SRC>(s8 & 1u ? e1[m] : e0[m], f[m]);
-                if (s8 + 2u < 8u) { if (s8 & 1u) e1[m] = fetch_entry<SRC>(v[m], s8 + 2u, lt); else e0[m] = fetch_entry<SRC>(v[m], s8 + 2u, lt); }
+                if (s8 + 2u < 8u) { if (s8 & 1u) e1[m] = fetch_entry<SRC>(c.v[m], s8 + 2u, lt); else e0[m] = fetch_entry<SRC>(c.v[m], s8 + 2u, lt); }
             }
             __builtin_amdgcn_sched_barrier(0);
+            if (s8 == 6u) request_next(c);                 // (the quarters' last use is behind)
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
@@ -443,27 +450,49 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
 #pragma unroll
                 for (uint32_t m = 0; m < M; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[s][s8].v, w[m], acc[m][s], 0, 0, 0);
         }
-#pragma unroll
-        for (uint32_t m = 0; m < M; ++m) {
-            const float d = *reinterpret_cast<const float *>(half + m * segs + lane_d);
-#pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) acc[m][s][t] *= d * ps[s][t];
-        }
-        if constexpr (SETS == 2) wave_lds_barrier();       // one buffer of partial sums: those of the unit before have been read
-        float *mine = part + (SETS == 1 ? buf * kPart : 0u) + w8 * kWavePart + m_first * SETS * 256u + 4u * lane;
+        float *mine = pt + w8 * kWavePart + m_first * SETS * 256u + 4u * lane;
 #pragma unroll
         for (uint32_t m = 0; m < M; ++m)
 #pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) = acc[m][s];
-        deliver(stage + (buf ^ 1u) * 2u * segs);           // (free since the barrier at this unit's head)
-        pj = j; pp0 = p0; pn = n;
-        if (next_tile && more) { ++tile; fresh = true; p0 = np0; n = nn; mat = nmat; }
-        j = nj;
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) acc[m][s][t] *= d[m] * ps[s][t];
+                *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) = acc[m][s];
+            }
+        const Done done{j, cur.p0, cur.n};
+        if (++j == upt && u + 1u < u1) { j = 0u; cur = info_of(++tile); load_tile(tile, cur.p0, cur.n); }
+        return done;
+    };
+    Carried ca, cb;
+    request_next(ca);
+    request_next(cb);
+    load_tile(tile, cur.p0, cur.n);
+    // narrow: two units per barrier, four buffers of partial sums; wide: one, two buffers (as large). A buffer is written again two
+    // barriers after its sums were complete; whoever adds them has passed one in between.
+    constexpr std::integral_constant<uint32_t, 1u> one{};
+    constexpr std::integral_constant<uint32_t, 2u> two{};
+    uint32_t u = u0;
+    float *pt = part;
+    for (; u + 1u < u1; u += 2u) {
+        Done w[2];
+        w[0] = unit(u, ca, pt);
+        if constexpr (SETS == 2) {
+            wave_lds_barrier();
+            reduce(one, w, pt);
+        }
+        w[1] = unit(u + 1u, cb, pt + kPart);
+        wave_lds_barrier();
+        if constexpr (SETS == 2) reduce(one, w + 1, pt + kPart);
+        else {
+            reduce(two, w, pt);
+            pt = pt == part ? part + 2u * kPart : part;
+        }
     }
-    wave_lds_barrier();
-    reduce(pj, pp0, pn, part + (SETS == 1 ? ((u1 - 1u - u0) & 1u) * kPart : 0u), 0u);
+    if (u < u1) {
+        const Done w = unit(u, ca, pt);
+        wave_lds_barrier();
+        reduce(one, &w, pt);
+    }
 }
 
 // SETS 1: the narrow tiles (list 2) of a chunk, SETS 2: the wide ones (list 1). Persistent workgroups, each with an equal run of the units.
@@ -472,10 +501,9 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
 constexpr uint32_t kFewWide = 48u;
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
 __global__ __launch_bounds__(staged_threads(SETS, KP)) void staged_tiles_kernel(StagedArgs a) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t stage[];        // two buffers of two halves of a unit
     __shared__ __attribute__((aligned(16))) uint8_t entries[kEntryBytes];   // static: table reads take immediate offsets
     __shared__ __attribute__((aligned(16))) uint32_t signs[sign_bytes<SRC>() / 4u + 4u];
-    __shared__ __attribute__((aligned(16))) float part[2u * KP * staged_nrt(KP) * 2u * 256u];
+    __shared__ __attribute__((aligned(16))) float part[4u * KP * staged_nrt(KP) * 2u * 256u];
     const bool few = a.n_tiles[1] < kFewWide;
     if (SETS == 2 && few) return;
     const uint32_t tid = threadIdx.x, l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
@@ -484,22 +512,16 @@ __global__ __launch_bounds__(staged_threads(SETS, KP)) void staged_tiles_kernel(
     const uint32_t G = gridDim.x, at = G % 8u == 0u ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
     const uint32_t u0 = (uint32_t)((uint64_t)at * units / G), u1 = (uint32_t)((uint64_t)(at + 1u) * units / G);
     if (u0 >= u1) return;
-    build_staged_tables<SRC, staged_threads(SETS, KP)>(entries, signs, tid, a.grid);
+    __shared__ TileInfo tiles[kTileInfos];
+    __shared__ PairInfo pairs[DOWN ? 1u : kTileInfos * 16u * SETS];
     const LaneTables lt{entries + (SRC == S_XS ? (tid & 7u) * 16u : SRC == S_M ? (tid & 1u) * 16u : 0u),
                         reinterpret_cast<const uint8_t *>(signs) + (SRC == S_IQ3 ? (tid & 3u) * 4u : SRC == S_M ? 0u : (tid & 15u) * 4u)};
-    staged_units<SRC, DOWN, SETS, KP>(a, a.tile_group + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, stage, part, lt);
+    staged_units<SRC, DOWN, SETS, KP>(a, a.tile_group + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, part, tiles, pairs, entries, signs, lt);
 }
 
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
 hipError_t launch_staged_list(const StagedArgs &a, uint32_t grid, hipStream_t s) {
-    constexpr size_t lds = (size_t)4u * 16u * staged_nrt(KP) * KP * staged_block_bytes<SRC>();
-    static bool attr = false;
-    if (!attr) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(staged_tiles_kernel<SRC, DOWN, SETS, KP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
-    REDHIP_LAUNCH((staged_tiles_kernel<SRC, DOWN, SETS, KP>), dim3(grid), dim3(staged_threads(SETS, KP)), lds, s, a);
+    REDHIP_LAUNCH((staged_tiles_kernel<SRC, DOWN, SETS, KP>), dim3(grid), dim3(staged_threads(SETS, KP)), 0, s, a);
     return hipGetLastError();
 }
 // wide: the chunk can have tiles of more than 16 pairs

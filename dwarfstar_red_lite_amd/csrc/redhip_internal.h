@@ -152,41 +152,15 @@ hipError_t launch_f32_tiles(const float *w, const float *extra_row, const float 
 hipError_t launch_swiglu_rows(const float *gu, uint32_t gu_stride, uint32_t ntok, uint32_t ffn, float *act, hipStream_t s);
 hipError_t launch_router_f32_tiles(const float *w, const float *gate_inp, const float *x, uint32_t ntok, uint32_t hidden, uint32_t n_expert,
                                    float *logits, void *xh, void *xl, int *xexp, hipStream_t s);
-// prefill chunk on packed IQ2_XXS experts: tiles of 16 pairs per distinct expert, 16x16x16 fp16 MFMA. Needs the pair
-// grouping (uid, expert_start, pair_token, n_unique); writes tmp [pairs][hidden] and sh_tmp [ntok][hidden] for
-// launch_batch_combine. tile_* hold prefill_tile_bound() entries.
+// entries of a tile list of a chunk, at most
 inline uint32_t prefill_tile_bound(uint32_t ntok, uint32_t top_k, uint32_t n_expert) {
     const uint32_t P = ntok * top_k;
     return (P < n_expert ? P : n_expert) + P / 16u + (ntok + 15u) / 16u + 1u;
 }
-// tiled_experts / tiled_shared: optional tile-major copies (launch_tile_packed) of the same matrices, same stride and offsets; with
-// them and ffn <= 512 the kernels that keep a tile's activations in registers run.
+// tile-major copies: of packed rows (with_sc: an IQ2_XS stream with its scale bytes), of raw IQ3_S rows (one 32-bit word per eight weights)
 hipError_t launch_tile_packed(const void *packed, uint64_t packed_stride, uint32_t count, uint32_t nrows, uint32_t K, void *tiled, uint64_t tiled_stride,
                               hipStream_t s, bool with_sc = false);
-// routed gate/up + SwiGLU of a chunk on the tile-major copy of packed IQ2_XXS gate/up matrices (mixed layouts); act: f32 [pairs][ffn], or
-// nullptr for fp16 halves + two exponents per pair in act_h / act_l / act_exp
-hipError_t launch_prefill_gateup_tiled(const void *tiled_experts, uint64_t stride, const uint32_t *uid, const uint32_t *expert_start,
-                                       const uint32_t *pair_token, const uint32_t *n_unique, uint32_t *tile_group, uint32_t *tile_pair0, uint32_t *tile_n,
-                                       uint32_t *n_tiles, const void *xh, const void *xl, const int *xexp, float *act, void *act_h, void *act_l,
-                                       int *act_exp, uint32_t hidden, uint32_t ffn, uint32_t top_k, uint32_t ntok, uint32_t n_expert, hipStream_t s, bool tiles_built = false);      // tiles_built: launch_group_pairs wrote the tile lists
-// tile-major IQ3_S matrices (one 32-bit word per eight weights) from raw GGUF rows, and the routed down projection of a chunk on them
 hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count, uint32_t nrows, uint32_t K, void *tiled, uint64_t tiled_stride, hipStream_t s);
-// routed matrices of a chunk whose experts are IQ2_XS / IQ1_M: tile kernels on the row-major streams (gate | up at `packed`, down at `down`)
-hipError_t launch_prefill_streams(uint32_t gate_up_type, const int8_t *gate_up_grid, const void *packed, uint64_t packed_stride, uint32_t down_type,
-                                  const int8_t *down_grid, const void *down, uint64_t down_stride, const uint32_t *uid, const uint32_t *expert_start,
-                                  const uint32_t *pair_token, const uint32_t *n_unique, uint32_t *tile_group, uint32_t *tile_pair0, uint32_t *tile_n,
-                                  uint32_t *n_tiles, const void *xh, const void *xl, const int *xexp, void *act_h, void *act_l, int *act_exp, float *tmp,
-                                  uint32_t hidden, uint32_t ffn, uint32_t top_k, uint32_t ntok, uint32_t n_expert, hipStream_t s, bool tiles_built = false);      // tiles_built: launch_group_pairs wrote the tile lists
-hipError_t launch_prefill_down_iq3s(const void *tiled_down, uint64_t stride, const uint32_t *uid, const uint32_t *n_unique, const uint32_t *tile_group,
-                                    const uint32_t *tile_pair0, const uint32_t *tile_n, const uint32_t *n_tiles, const void *act_h, const void *act_l,
-                                    const int *act_exp, float *tmp, uint32_t hidden, uint32_t ffn, uint32_t top_k, uint32_t ntok, uint32_t n_expert,
-                                    hipStream_t s);
-hipError_t launch_prefill_packed(const void *experts, uint64_t stride, const void *shared, const void *tiled_experts, const void *tiled_shared,
-                                 const uint32_t *uid, const uint32_t *expert_start,
-                                 const uint32_t *pair_token, const uint32_t *n_unique, uint32_t *tile_group, uint32_t *tile_pair0,
-                                 uint32_t *tile_n, uint32_t *n_tiles, const void *xh, const void *xl, const int *xexp, void *act_h, void *act_l,
-                                 int *act_exp, float *tmp, float *sh_tmp, uint32_t hidden, uint32_t ffn, uint32_t top_k, uint32_t ntok,
-                                 uint32_t n_expert, hipStream_t s, bool tiles_built = false, bool with_shared = true);      // without: no shared expert's tiles (shared, tiled_shared, sh_tmp unused)      // tiles_built: launch_group_pairs wrote the tile lists
 // Tile lists of a chunk for the prefill kernels. Groups 0..U-1 are the distinct routed experts (pairs expert_start[u] ..
 // expert_start[u + 1]), group U is the shared expert with pairs P .. P + shared_ntok (0: no shared tiles). A tile = (group, first pair,
 // number of pairs). Three lists in the same arrays, list l from entry l * list_stride on (list_stride = prefill_tile_bound of the call),
@@ -247,21 +221,30 @@ __device__ __forceinline__ void build_tile_lists(uint32_t U, uint32_t p0, uint32
 #endif
 // the tile lists as a launch of their own, for callers whose pair sort did not write them
 hipError_t launch_build_tiles(const uint32_t *expert_start, const uint32_t *n_unique, uint32_t n_pairs, const TileLists &tl, hipStream_t s);
-// A chunk on experts without tile-major copies (redhip_tiles.hip): raw GGUF rows or packed IQ2_XXS rows (`packed`), every matrix 16-byte
-// aligned. Expert uid[u]: gate matrix at gate + uid[u] * stride, up matrix up_delta behind it, down matrix at down + uid[u] * down_stride;
-// the shared expert's slot gate | up | down at `shared` when tl.shared_ntok asks for its tiles. x as fp16 halves in; act: f32
-// [ntok * top_k + shared tokens][ffn] scratch; outputs tmp / sh_tmp as launch_prefill_packed leaves them for launch_batch_combine.
-struct StagedExperts {
-    const void *gate, *down, *shared;
-    uint64_t stride, down_stride, up_delta;
-    uint32_t gate_up_type, down_type;
-    const int8_t *gate_up_grid, *down_grid;
-    bool packed;
+// A chunk's experts on the tile kernels (redhip_tiles.hip). `raw`: GGUF rows; `rows`: packed IQ2_XXS rows; `tiled`: tile-major copies
+// (launch_tile_packed, launch_tile_iq3s; ffn <= 512). Matrices are 16-byte aligned, the first of expert uid[u] at experts + uid[u] * stride
+// (gate/up: the up matrix up_delta behind it), of the shared expert at `shared` when tl.shared_ntok asks for its tiles.
+enum class RowLayout : uint32_t { raw, rows, tiled };
+struct StagedMatrices {
+    uint32_t type;
+    RowLayout layout;
+    const void *experts, *shared;
+    uint64_t stride, up_delta;
+    const int8_t *grid;                     // codebook of IQ2_XS / IQ1_M
 };
-bool staged_tiles_supported(uint32_t gate_up_type, uint32_t down_type, uint32_t hidden, uint32_t ffn, uint32_t n_expert, bool packed);
-hipError_t launch_staged_tiles(const StagedExperts &x, const uint32_t *uid, const uint32_t *expert_start, const uint32_t *pair_token, const uint32_t *n_unique,
-                               const TileLists &tl, bool tiles_built, const void *xh, const void *xl, const int *xexp, float *act, float *tmp, float *sh_tmp,
-                               uint32_t hidden, uint32_t ffn, uint32_t top_k, uint32_t ntok, uint32_t n_expert, hipStream_t s);
+struct StagedChunk {                        // the pair sort of the call, its tile lists among it
+    const uint32_t *uid, *pair_token, *n_unique;
+    TileLists tl;
+    uint32_t ntok, top_k, n_expert;
+    uint32_t wide_tiles = 0xffffffffu;      // tiles of more than kPrefillTile pairs, where the host knows their number
+};
+bool staged_gateup_supported(uint32_t type, RowLayout lay, uint32_t hidden, uint32_t ffn);
+bool staged_down_supported(uint32_t type, RowLayout lay, uint32_t hidden, uint32_t ffn);
+// x as fp16 halves in; act out: f32 [ntok * top_k + shared tokens][ffn], SwiGLU of every pair
+hipError_t launch_staged_gateup(const StagedMatrices &m, const StagedChunk &c, const void *xh, const void *xl, const int *xexp, float *act, uint32_t hidden, uint32_t ffn,
+                                hipStream_t s);
+// act in; out tmp [ntok * top_k][hidden] and sh_tmp [shared tokens][hidden], for launch_batch_combine
+hipError_t launch_staged_down(const StagedMatrices &m, const StagedChunk &c, const float *act, float *tmp, float *sh_tmp, uint32_t hidden, uint32_t ffn, hipStream_t s);
 // Device scratch of the pair sort of large chunks (more than 512 tokens), which runs as three launches over blocks of kGroupSpan tokens:
 // count_blk / blk_off [blocks][n_expert], first_key / expert_base [n_expert]. All zero before the first use (the sort leaves first_key
 // zero again); `blocks` = the capacity in blocks.
@@ -275,7 +258,7 @@ inline GroupScratch group_scratch_at(void *base, uint32_t max_tokens, uint32_t n
     uint32_t *p = static_cast<uint32_t *>(base);
     return GroupScratch{p, p + (size_t)nb * n_expert, p + (size_t)2u * nb * n_expert, p + (size_t)2u * nb * n_expert + n_expert, nb};
 }
-// tiles: also write the tile lists of the chunk (the prefill launchers then take tiles_built = true and launch no build_tiles_kernel)
+// tiles: also write the tile lists of the chunk
 // scratch: when given, chunks of more than 512 tokens are sorted by many workgroups (three launches) instead of one
 hipError_t launch_group_pairs(const uint32_t *ids, const float *weights, uint32_t ntok, uint32_t top_k, uint32_t n_expert,
                               uint32_t *uid, uint32_t *expert_start, uint32_t *pair_token, float *pair_weight,

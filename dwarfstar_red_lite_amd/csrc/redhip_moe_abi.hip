@@ -99,8 +99,6 @@ struct Moe {
     bool tiled_router(uint32_t ntok) const { return packed_gu() && ntok >= 40u && (cfg.router_type == T_F32 || mixed); }
     uint64_t tiled_stride() const { return fused ? expert_stride : packed_stride; }      // bytes between experts in `tiled`
     bool tiles_resident() const { return packed_gu() && gu_type == T_IQ2_XXS && cfg.max_tokens > 8u && cfg.ffn <= 512u && cfg.hidden / 512u <= 4u; }
-    // a chunk on a mixed layout: the routed gate/up matrices (packed IQ2_XXS) run on the prefill tiles, the rest on raw rows
-    bool mixed_chunk(uint32_t ntok) const { return mixed && ntok > 8u && tiles_resident(); }
     uint64_t words_down_stride() const {
         return ((dn_type == T_IQ3_S ? iq3s_words_bytes(cfg.hidden, cfg.ffn) : packed_matrix_bytes(dn_type, cfg.hidden, cfg.ffn)) + 255u) & ~255ull;
     }
@@ -169,20 +167,18 @@ struct Moe {
         return small_batch_mixed(ntok) && ntok >= from && (words || cfg.ffn <= 768u) &&
                (words || (quant_supported(dn_type) && (8u * rbd) % 16u == 0u && (8u * rbs) % 16u == 0u && (2u * gate_bytes) % 16u == 0u && (2u * sh_gate_bytes) % 16u == 0u));
     }
-    // a chunk on a layout whose experts are IQ2_XS / IQ1_M: the tile kernels on the row-major streams of the routed matrices, the shared
-    // expert and the router as dense f32 products
-    bool stream_chunk(uint32_t ntok) const { return ntok > 8u && stream_tiles_resident(); }
-    // ... such a handle keeps tile-major copies of the gate | up streams (`tiled`) and of the down streams (`tiled_down`)
+    // a handle that takes chunks on IQ2_XS / IQ1_M experts keeps tile-major copies of the gate | up streams (`tiled`) and of the down streams (`tiled_down`)
     bool stream_tiles_resident() const {
         const bool gu_cb = gu_type == T_IQ2_XS || gu_type == T_IQ1_M, dn_cb = dn_type == T_IQ2_XS || dn_type == T_IQ1_M;
         return mixed && gu_cb && dn_cb && (cfg.ffn == 256u || cfg.ffn == 512u) && cfg.hidden / 512u <= 4u && cfg.max_tokens > 8u;
     }
-    // a chunk on a layout without tile-major copies (ffn > 512, or IQ2_XS / IQ1_M gate/up beside another down format): the tile kernels that
-    // take rows through LDS - the raw ones of mixed layouts, the packed row-major ones of all-IQ2_XXS layers
-    bool staged_chunk(uint32_t ntok) const {
-        if (ntok <= 8u || tiles_resident() || stream_tiles_resident()) return false;
-        return fused ? rowmajor_down() && staged_tiles_supported(gu_type, dn_type, cfg.hidden, cfg.ffn, cfg.n_expert, true)
-                     : mixed && keep_raw() && staged_tiles_supported(gu_type, dn_type, cfg.hidden, cfg.ffn, cfg.n_expert, false);
+    // a chunk runs on the tile kernels: tile-major copies of gate/up (and of down where its format has them), else the packed rows of
+    // all-IQ2_XXS layers or the raw ones of mixed layouts (ffn > 512, IQ2_XS / IQ1_M gate/up beside another down format)
+    bool tile_chunk(uint32_t ntok) const {
+        if (ntok <= 8u || !(fused || mixed)) return false;
+        if (tiles_resident() || stream_tiles_resident()) return true;
+        if (fused) return rowmajor_down() && staged_gateup_supported(gu_type, RowLayout::rows, cfg.hidden, cfg.ffn) && staged_down_supported(dn_type, RowLayout::rows, cfg.hidden, cfg.ffn);
+        return keep_raw() && staged_gateup_supported(gu_type, RowLayout::raw, cfg.hidden, cfg.ffn) && staged_down_supported(dn_type, RowLayout::raw, cfg.hidden, cfg.ffn);
     }
     // a chunk on a mixed layout that has no tile kernels at all runs as slices of 8 tokens on the grouped small-batch kernels, far ahead of
     // the generic per-pair kernels on raw rows
@@ -192,7 +188,7 @@ struct Moe {
     bool sliced(uint32_t ntok) const {
         if (ntok <= kSlice || small_batch(ntok, true)) return false;      // (one small batch: up to 32 tokens behind the layer's own router)
         if (ntok <= 2u * kSlice && (small_batch(kSlice) || grouped_mixed(kSlice))) return true;
-        return mixed && !tiles_resident() && !stream_chunk(ntok) && !staged_chunk(ntok) && grouped_mixed(kSlice);
+        return mixed && !tile_chunk(ntok) && grouped_mixed(kSlice);
     }
     // the workspace entries a caller can read back (redhip_moe_last_route) of the slice that starts at token t0 sit at their place in the chunk
     void shift_route_outputs(int64_t t0) {
@@ -303,22 +299,20 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
         const uint32_t P = ntok * c.top_k, n_groups = P < c.n_expert ? P : c.n_expert;
         const ExpertSet ex = m->routed(layer), sh = m->shared(layer);
         const Layer &Ld = m->layers[layer];
-        const bool stream_tiles = m->stream_chunk(ntok) && Ld.tiled && Ld.tiled_down && Ld.dense_gu && m->side;
         // the shared expert as dense f32 products on the fp32 matrix units, started before the pair sort (one workgroup on an idle machine;
         // the many-workgroup sort of a large chunk then queues behind the dense tiles - 73 against 22 us at 2048 tokens - but started
         // behind the sort the dense products slow the down tiles by more: 787 against 760 us per chunk)
-        const bool staged = !stream_tiles && m->staged_chunk(ntok);
-        const bool dense_shared = (stream_tiles || ((m->mixed_chunk(ntok) || (staged && m->mixed)) && Ld.dense_gu && m->side));
+        const bool tile_path = !m->small_batch(ntok) && !(m->small_batch(ntok, true) && grouped) && m->tile_chunk(ntok);
+        const bool dense_shared = tile_path && m->mixed && Ld.dense_gu && m->side;
         if (dense_shared && !fork_shared_dense(m, Ld, x, ntok, s)) return 0;
         // the pair sort also writes the tile lists of the tile kernels that follow (all-IQ2_XXS layers: with the shared expert's tiles)
-        const bool tile_path = !m->small_batch(ntok) && (m->packed_path(ntok) || stream_tiles || staged || m->mixed_chunk(ntok));
-        const TileLists tl{m->tile_group, m->tile_pair0, m->tile_n, m->n_tiles, prefill_tile_bound(ntok, c.top_k, c.n_expert), m->packed_path(ntok) ? ntok : 0u};
-        const bool tiles_built = !grouped && tile_path;
+        const TileLists tl{m->tile_group, m->tile_pair0, m->tile_n, m->n_tiles, prefill_tile_bound(ntok, c.top_k, c.n_expert), m->fused ? ntok : 0u};
         if (!grouped) {
             prof_set_stage(ST_GROUP);
             HIP_OK(launch_group_pairs(ids, weights, ntok, c.top_k, c.n_expert, m->uid, m->expert_start, m->pair_token, m->pair_weight,
                                       m->tok_pair, m->n_unique, s, tile_path ? &tl : nullptr, m->group_scratch_ptr()), "grouping launch");
-        }
+        } else if (tile_path)
+            HIP_OK(launch_build_tiles(m->expert_start, m->n_unique, P, tl, s), "tile list launch");
         if (m->small_batch(ntok, true) && grouped && !select_here) {     // routing sorted (with its pass list) by the prep or the selection launch: expert slices per pass
             const Layer &L = m->layers[layer];
             HIP_OK(launch_batch_slices(L.packed, m->packed_stride, L.down_cm, m->down_cm_stride(), L.shared_packed, L.shared_down_cm, m->pass_list, m->n_pass,
@@ -327,65 +321,45 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
             return 1;
         }
         if (m->small_batch(ntok)) { moe_err("internal: a small batch reached the expert kernels without its pass list"); return 0; }
-        if (staged && (m->fused || dense_shared)) {
+        if (tile_path) {
+            // gate/up + SwiGLU and down on the tile kernels: tile-major copies where the layout has them, else packed rows (all-IQ2_XXS) or raw ones
             const Layer &L = Ld;
-            const uint8_t *rows = m->fused ? L.packed : L.experts;
-            const uint64_t stride = m->fused ? m->packed_stride : m->expert_stride;
-            const StagedExperts x{rows, rows + 2u * m->gate_bytes, m->fused ? L.shared_packed : nullptr, stride, stride, m->gate_bytes, m->gu_type, m->dn_type, m->gu_grid, m->dn_grid, m->fused};
-            HIP_OK(launch_staged_tiles(x, m->uid, m->expert_start, m->pair_token, m->n_unique, tl, tiles_built, m->xh, m->xl, m->xexp, m->act, m->tmp, m->sh_tmp,
-                                       c.hidden, c.ffn, c.top_k, ntok, c.n_expert, s), "staged tile launch");
-            if (dense_shared && !join_shared_dense(m, s)) return 0;
+            const bool tiles_gu = L.tiled != nullptr, tiles_dn = m->fused ? L.tiled != nullptr : L.tiled_down != nullptr;
+            const RowLayout rows = m->fused ? RowLayout::rows : RowLayout::raw;
+            const uint8_t *plain = m->fused ? L.packed : L.experts;
+            const StagedMatrices gu{m->gu_type, tiles_gu ? RowLayout::tiled : rows, tiles_gu ? L.tiled : plain, tiles_gu ? L.shared_tiled : L.shared_packed,
+                                    tiles_gu ? m->tiled_stride() : m->fused ? m->packed_stride : m->expert_stride, tiles_gu ? m->pk_gate_bytes : m->gate_bytes, m->gu_grid};
+            const StagedChunk chunk{m->uid, m->pair_token, m->n_unique, tl, ntok, c.top_k, c.n_expert};
+            if (!gu.experts) { moe_err("internal: no rows for the tile kernels (layer %u)", layer); return 0; }
+            HIP_OK(launch_staged_gateup(gu, chunk, m->xh, m->xl, m->xexp, m->act, c.hidden, c.ffn, s), "gate/up tile launch");
+            const uint8_t *dn_rows = m->fused ? (tiles_dn ? L.tiled : L.packed) + 2u * m->gate_bytes : tiles_dn ? L.tiled_down : L.experts ? L.experts + 2u * m->gate_bytes : nullptr;
+            const uint8_t *dn_shared = !m->fused ? nullptr : (tiles_dn ? L.shared_tiled : L.shared_packed) + 2u * m->gate_bytes;
+            const uint64_t dn_stride = m->fused ? (tiles_dn ? m->tiled_stride() : m->packed_stride) : !tiles_dn ? m->expert_stride : m->dn_type == T_IQ3_S ? m->tiled_down_stride() : m->words_down_stride();
+            const StagedMatrices dn{m->dn_type, tiles_dn ? RowLayout::tiled : rows, dn_rows, dn_shared, dn_stride, 0u, m->dn_grid};
+            prof_set_stage(ST_BATCH_DOWN);
+            if (staged_down_supported(dn.type, dn.layout, c.hidden, c.ffn) && dn_rows)
+                HIP_OK(launch_staged_down(dn, chunk, m->act, m->tmp, m->sh_tmp, c.hidden, c.ffn, s), "down tile launch");
+            else if (!raw_rows(m, layer)) return 0;
+            else HIP_OK(launch_batch_down(ex, m->uid, m->expert_start, m->n_unique, n_groups, P, c.hidden, c.ffn, m->act, m->tmp, s), "batched down launch");
+            prof_set_stage(ST_BATCH_DOWN);
+            if (dense_shared) {
+                if (!join_shared_dense(m, s)) return 0;
+            } else if (!m->fused) {
+                HIP_OK(launch_batch_gateup(sh, nullptr, nullptr, nullptr, nullptr, 1u, ntok, c.hidden, c.ffn, x, m->sh_act, s), "batched shared gate/up launch");
+                HIP_OK(launch_batch_down(sh, nullptr, nullptr, nullptr, 1u, ntok, c.hidden, c.ffn, m->sh_act, m->sh_tmp, s), "batched shared down launch");
+            }
             prof_set_stage(ST_BATCH_COMBINE);
             HIP_OK(launch_batch_combine(m->tmp, m->pair_weight, m->tok_pair, ntok, c.top_k, m->sh_tmp, m->scalar, c.hidden, out, s), "batched combine launch");
             prof_set_stage(ST_OTHER);
             return 1;
         }
-        if (m->packed_path(ntok)) {     // prefill chunk: tiles of 16 pairs per expert on the MFMA units
-            const Layer &L = m->layers[layer];
-            HIP_OK(launch_prefill_packed(L.packed, m->expert_stride, L.shared_packed, L.tiled, L.shared_tiled, m->uid, m->expert_start, m->pair_token, m->n_unique,
-                                         m->tile_group, m->tile_pair0, m->tile_n, m->n_tiles, m->xh, m->xl, m->xexp, m->act_h, m->act_l,
-                                         m->act_exp, m->tmp, m->sh_tmp, c.hidden, c.ffn, c.top_k, ntok, c.n_expert, s, tiles_built), "prefill launch");
-            prof_set_stage(ST_BATCH_COMBINE);
-            HIP_OK(launch_batch_combine(m->tmp, m->pair_weight, m->tok_pair, ntok, c.top_k, m->sh_tmp, m->scalar, c.hidden, out, s), "batched combine launch");
-            prof_set_stage(ST_OTHER);
-            return 1;
-        }
-        if (stream_tiles) {
-            const Layer &L = Ld;
-            prof_set_stage(ST_BATCH_GATEUP);
-            HIP_OK(launch_prefill_streams(m->gu_type, m->gu_grid, L.tiled, m->packed_stride, m->dn_type, m->dn_grid, L.tiled_down, m->words_down_stride(), m->uid,
-                                          m->expert_start, m->pair_token, m->n_unique, m->tile_group, m->tile_pair0, m->tile_n, m->n_tiles, m->xh, m->xl, m->xexp,
-                                          m->act_h, m->act_l, m->act_exp, m->tmp, c.hidden, c.ffn, c.top_k, ntok, c.n_expert, s, tiles_built), "stream tile launch");
-            if (!join_shared_dense(m, s)) return 0;
-            prof_set_stage(ST_BATCH_COMBINE);
-            HIP_OK(launch_batch_combine(m->tmp, m->pair_weight, m->tok_pair, ntok, c.top_k, m->sh_tmp, m->scalar, c.hidden, out, s), "batched combine launch");
-            prof_set_stage(ST_OTHER);
-            return 1;
-        }
+        if (!raw_rows(m, layer)) return 0;                 // (the per-pair kernels below read raw rows)
         prof_set_stage(ST_BATCH_GATEUP);
-        const bool tiled_down = m->mixed_chunk(ntok) && m->layers[layer].tiled_down;      // then the activations stay fp16 halves for the IQ3_S tile kernel
-        if (!(m->mixed_chunk(ntok) && tiled_down) && !raw_rows(m, layer)) return 0;       // (the per-pair kernels below read raw rows)
-        if (m->mixed_chunk(ntok))      // xh / xl / xexp come from the router kernel or the prep kernel
-            HIP_OK(launch_prefill_gateup_tiled(m->layers[layer].tiled, m->packed_stride, m->uid, m->expert_start, m->pair_token, m->n_unique, m->tile_group,
-                                               m->tile_pair0, m->tile_n, m->n_tiles, m->xh, m->xl, m->xexp, tiled_down ? nullptr : m->act, m->act_h, m->act_l,
-                                               m->act_exp, c.hidden, c.ffn, c.top_k, ntok, c.n_expert, s, tiles_built), "tiled gate/up launch");
-        else
-            HIP_OK(launch_batch_gateup(ex, m->uid, m->expert_start, m->pair_token, m->n_unique, n_groups, P, c.hidden, c.ffn, x, m->act, s), "batched gate/up launch");
-        prof_set_stage(ST_BATCH_GATEUP);
-        if (!dense_shared) {
-            HIP_OK(launch_batch_gateup(sh, nullptr, nullptr, nullptr, nullptr, 1u, ntok, c.hidden, c.ffn, x, m->sh_act, s), "batched shared gate/up launch");
-        }
+        HIP_OK(launch_batch_gateup(ex, m->uid, m->expert_start, m->pair_token, m->n_unique, n_groups, P, c.hidden, c.ffn, x, m->act, s), "batched gate/up launch");
+        HIP_OK(launch_batch_gateup(sh, nullptr, nullptr, nullptr, nullptr, 1u, ntok, c.hidden, c.ffn, x, m->sh_act, s), "batched shared gate/up launch");
         prof_set_stage(ST_BATCH_DOWN);
-        if (tiled_down)
-            HIP_OK(launch_prefill_down_iq3s(Ld.tiled_down, m->tiled_down_stride(), m->uid, m->n_unique, m->tile_group, m->tile_pair0, m->tile_n, m->n_tiles,
-                                            m->act_h, m->act_l, m->act_exp, m->tmp, c.hidden, c.ffn, c.top_k, ntok, c.n_expert, s), "tiled IQ3_S down launch");
-        else
-            HIP_OK(launch_batch_down(ex, m->uid, m->expert_start, m->n_unique, n_groups, P, c.hidden, c.ffn, m->act, m->tmp, s), "batched down launch");
-        prof_set_stage(ST_BATCH_DOWN);
-        if (dense_shared) {
-            if (!join_shared_dense(m, s)) return 0;
-        } else
-            HIP_OK(launch_batch_down(sh, nullptr, nullptr, nullptr, 1u, ntok, c.hidden, c.ffn, m->sh_act, m->sh_tmp, s), "batched shared down launch");
+        HIP_OK(launch_batch_down(ex, m->uid, m->expert_start, m->n_unique, n_groups, P, c.hidden, c.ffn, m->act, m->tmp, s), "batched down launch");
+        HIP_OK(launch_batch_down(sh, nullptr, nullptr, nullptr, 1u, ntok, c.hidden, c.ffn, m->sh_act, m->sh_tmp, s), "batched shared down launch");
         prof_set_stage(ST_BATCH_COMBINE);
         HIP_OK(launch_batch_combine(m->tmp, m->pair_weight, m->tok_pair, ntok, c.top_k, m->sh_tmp, m->scalar, c.hidden, out, s), "batched combine launch");
         prof_set_stage(ST_OTHER);
@@ -906,7 +880,7 @@ int redhip_moe_experts(redhip_moe_t h, uint32_t layer, const float *x_dev, uint3
         GuardScope(uint32_t n, uint32_t *st) { route_guard() = RouteGuard{n, st}; }
         ~GuardScope() { route_guard() = RouteGuard{}; }
     } guard_scope(m->cfg.n_expert, m->status);
-    if (m->packed_path(ntok) || m->small_batch_mixed(ntok) || m->mixed_chunk(ntok) || m->stream_chunk(ntok) || m->staged_chunk(ntok)) {
+    if (m->packed_path(ntok) || m->small_batch_mixed(ntok) || m->tile_chunk(ntok)) {
         const Layer &L = m->layers[layer];
         const uint32_t nv = m->cfg.hidden / 256u;
         // batches whose pairs are grouped by expert next: the pair sort rides in the same launch as one more workgroup

@@ -1,6 +1,8 @@
-// Chunks of tokens on experts that have no tile-major copy: the (token, expert) pairs of one expert are cut into tiles of up to 32 pairs
-// (build_tile_lists) and multiplied on v_mfma_f32_16x16x32_f16 straight from rows as they lie in memory - raw GGUF blocks of IQ2_XXS,
-// IQ2_XS, IQ1_M and (down) IQ3_S, or packed IQ2_XXS rows.
+// Chunks of tokens (prefill): the (token, expert) pairs of one expert are cut into tiles of up to 32 pairs (build_tile_lists) and multiplied
+// on v_mfma_f32_16x16x32_f16. Experts as raw GGUF rows (IQ2_XXS, IQ2_XS, IQ1_M, down also IQ3_S), as packed IQ2_XXS rows, or as tile-major
+// copies of these formats (redhip_prefill.hip).
+// Reference behaviour this replaces: native/redmetal_engine_prefill.m:1246-1330 (grouped GEMM over expert slices)
+// with the arithmetic of native/redlite_native_reference.c:251-382.
 //
 // What bounds these kernels is the decode (LDS table reads and vector issue; every weight is decoded once per tile), so the rows must cost
 // nothing extra. Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights
@@ -36,9 +38,20 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 union H8 { uint4 u; half8_t v; half2_t p[4]; _Float16 e[8]; };
 
-// row sources
-enum : int { S_XXS = 0, S_XS = 1, S_M = 2, S_IQ3 = 3, S_PACKED_XXS = 4 };
-template <int SRC> constexpr uint32_t src_block() { return SRC == S_XXS ? 66u : SRC == S_XS ? 74u : SRC == S_M ? 56u : SRC == S_IQ3 ? 110u : 64u; }      // bytes per 256 columns
+// row sources: format (low half, what the decode goes by) and layout
+enum : int { F_XXS = 0, F_XS = 1, F_M = 2, F_IQ3 = 3, F_IQ3_WORDS = 4, L_RAW = 0, L_ROWS = 8, L_TILED = 16 };
+enum : int { S_XXS = F_XXS, S_XS = F_XS, S_M = F_M, S_IQ3 = F_IQ3, S_ROWS_XXS = F_XXS | L_ROWS, S_TILED_XXS = F_XXS | L_TILED, S_TILED_XS = F_XS | L_TILED,
+             S_TILED_M = F_M | L_TILED, S_TILED_IQ3 = F_IQ3_WORDS | L_TILED };
+template <int SRC> constexpr int fmt() { return SRC & 7; }
+template <int SRC> constexpr int layout() { return SRC & 24; }
+// bytes per 256 columns of a row: raw blocks; the quarters of the other layouts (their block scales lie apart)
+template <int SRC> constexpr uint32_t src_block() {
+    return layout<SRC>() != L_RAW ? (fmt<SRC>() == F_IQ3_WORDS ? 128u : 64u) : SRC == S_XXS ? 66u : SRC == S_XS ? 74u : SRC == S_M ? 56u : 110u;
+}
+template <int SRC> constexpr float format_scale() { return fmt<SRC>() == F_XXS || fmt<SRC>() == F_XS ? 0.125f : 1.0f; }      // the d / 8 of the IQ2 formats
+// first of the eight columns that lane quarter q multiplies in step s of a block: its own quarter, in order - or, where the lane reads entry q
+// of every group (tile-major IQ3_S words), that entry
+template <int SRC> __device__ __forceinline__ uint32_t step_column(uint32_t s, uint32_t q) { return fmt<SRC>() == F_IQ3_WORDS ? 128u * (s >> 2) + 32u * (s & 3u) + 8u * q : 64u * q + 8u * s; }
 
 // Decode tables in LDS.
 //   IQ2_XXS: the eight fp16 magnitudes of every grid entry times every group scale 2 s + 1 (64 KB, exact), at entry * 256 + s * 16: the address is
@@ -48,8 +61,9 @@ template <int SRC> constexpr uint32_t src_block() { return SRC == S_XXS ? 66u : 
 //   signs: bit 15 - i / 31 - i of the word of a sign field = signs of weights 2i and 2i + 1, so a pair's signs are one shift and one and-or;
 //   replicated so that the reads are (nearly) free of conflicts. (Sign masks as 16-byte entries save three shifts per eight weights and cost
 //   a second conflicting 16-byte read: LDS, the tighter of the two pipes, loses more.)
-template <int SRC> constexpr uint32_t sign_copies() { return SRC == S_M ? 0u : SRC == S_IQ3 ? 4u : 16u; }
-template <int SRC> constexpr uint32_t sign_bytes() { return (SRC == S_IQ3 ? 256u : 128u) * sign_copies<SRC>() * 4u; }
+template <int SRC> constexpr bool is_iq3() { return fmt<SRC>() == F_IQ3 || fmt<SRC>() == F_IQ3_WORDS; }
+template <int SRC> constexpr uint32_t sign_copies() { return fmt<SRC>() == F_M ? 0u : is_iq3<SRC>() ? 4u : 16u; }
+template <int SRC> constexpr uint32_t sign_bytes() { return (is_iq3<SRC>() ? 256u : 128u) * sign_copies<SRC>() * 4u; }
 constexpr uint32_t kEntryBytes = 65536u;
 
 __device__ __forceinline__ uint32_t two_halves(float lo, float hi) {
@@ -58,7 +72,7 @@ __device__ __forceinline__ uint32_t two_halves(float lo, float hi) {
 
 template <int SRC, uint32_t T>          // by all T threads of the workgroup
 __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *signs, uint32_t tid, const int8_t *grid) {
-    if constexpr (SRC == S_XXS || SRC == S_PACKED_XXS) {
+    if constexpr (fmt<SRC>() == F_XXS) {
         for (uint32_t e = tid; e < 16u * 256u; e += T) {
             const uint64_t ge = redhip_iq2xxs_grid[e >> 4];
             const float f = (float)(2u * (e & 15u) + 1u);
@@ -67,8 +81,8 @@ __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *
             for (int i = 0; i < 4; ++i) w4[i] = two_halves(f * (float)((uint32_t)(ge >> (16 * i)) & 255u), f * (float)((uint32_t)(ge >> (16 * i + 8)) & 255u));
             *reinterpret_cast<uint4 *>(entries + (size_t)e * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
         }
-    } else if constexpr (SRC == S_XS || SRC == S_M) {
-        constexpr uint32_t kCopies = SRC == S_XS ? 8u : 2u, kEntries = kEntryBytes / (16u * kCopies);
+    } else if constexpr (fmt<SRC>() == F_XS || fmt<SRC>() == F_M) {
+        constexpr uint32_t kCopies = fmt<SRC>() == F_XS ? 8u : 2u, kEntries = kEntryBytes / (16u * kCopies);
         for (uint32_t e = tid; e < kEntries; e += T) {
             const uint64_t ge = reinterpret_cast<const uint64_t *>(grid)[e];
             uint32_t w4[4];
@@ -84,10 +98,10 @@ __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *
                 make_uint2(two_halves(f * (float)(gw & 255u), f * (float)((gw >> 8) & 255u)), two_halves(f * (float)((gw >> 16) & 255u), f * (float)(gw >> 24)));
         }
     }
-    if constexpr (SRC != S_M) {
+    if constexpr (fmt<SRC>() != F_M) {
         constexpr uint32_t R = sign_copies<SRC>(), N = sign_bytes<SRC>() / 4u;
         for (uint32_t i = tid; i < N; i += T) {
-            const uint32_t s = i / R, s8 = SRC == S_IQ3 ? s : s | ((__popc(s) & 1u) << 7);
+            const uint32_t s = i / R, s8 = is_iq3<SRC>() ? s : s | ((__popc(s) & 1u) << 7);
             uint32_t w = 0u;
 #pragma unroll
             for (uint32_t k = 0; k < 4u; ++k) w |= (((s8 >> (2u * k)) & 1u) << (15u - k)) | (((s8 >> (2u * k + 1u)) & 1u) << (31u - k));
@@ -99,28 +113,49 @@ __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *
 // fields of a quarter block (two 32-column groups) of a row: what a lane multiplies
 //   IQ2_XXS  a: the two groups' words                     IQ2_XS  a: eight 16-bit entries, c: two scale bytes
 //   IQ1_M    a: 8 index bytes | 4 bytes of nibbles | scale word     IQ3_S   a: 16 index bytes, b: 8 sign bytes, c: two qh bytes | scale byte << 16
-struct Quarter { uint4 a; uint2 b; uint32_t c; };
+//   tile-major IQ3_S   a, b: entry q of the first and the last four groups of the block, a word each
+struct Quarter { uint4 a, b; uint32_t c; };
 
 template <class T> __device__ __forceinline__ T load_a2(const uint8_t *p) { T v; __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), sizeof(T)); return v; }
 
-// quarter `part` of the block at bp, and what its d is made from (dp: packed rows keep their d elsewhere)
-template <int SRC>
-__device__ __forceinline__ void load_quarter(const uint8_t *bp, const uint8_t *dp, uint32_t part, Quarter &v, uint2 &d) {
-    if constexpr (SRC == S_XXS || SRC == S_XS || SRC == S_IQ3) {
-        v.a = load_a2<uint4>(bp + 2u + 16u * part);
-        d.x = load_a2<uint16_t>(bp);
-    } else if constexpr (SRC == S_PACKED_XXS) {
-        v.a = *reinterpret_cast<const uint4 *>(bp + 16u * part);
-        d.x = *reinterpret_cast<const uint16_t *>(dp);
+// Quarter q of block kc of row r of a tile of 16 rows, and what its d is made from. tile: the tile's rows (raw and packed rows 16 KP blocks,
+// tile-major its KP * 2 chunks of 16 rows), ds: its block scales, scs: tile-major IQ2_XS, its scale bytes.
+//   tile-major: chunk c (128 columns) of row r at (c * 16 + r) * 32 (IQ3_S words * 64), scale of block b at (b * 16 + r) * 2, the scale
+//   bytes of a chunk at (c * 16 + r) * 4: a wave's load is two runs of 512 bytes
+template <int SRC, uint32_t KP>
+__device__ __forceinline__ void load_quarter(const uint8_t *tile, const uint8_t *ds, const uint8_t *scs, uint32_t r, uint32_t kc, uint32_t q, Quarter &v, uint2 &d) {
+    const uint32_t block = r * KP + kc;
+    if constexpr (layout<SRC>() == L_TILED) {
+        const uint32_t chunk = (2u * kc + (q >> 1)) * 16u + r;
+        if constexpr (fmt<SRC>() == F_IQ3_WORDS) {
+            v.a = *reinterpret_cast<const uint4 *>(tile + (32u * kc + r) * 64u + 16u * q);
+            v.b = *reinterpret_cast<const uint4 *>(tile + (32u * kc + 16u + r) * 64u + 16u * q);
+        } else if constexpr (fmt<SRC>() == F_M) {      // stream words: four index bytes | nibbles, two 3-bit scales from bit 16 on
+            const uint4 w = *reinterpret_cast<const uint4 *>(tile + chunk * 32u + 16u * (q & 1u));
+            v.a = make_uint4(w.x, w.z, (w.y & 0xffffu) | (w.w << 16), __builtin_amdgcn_ubfe(w.y, 16u, 6u) | (__builtin_amdgcn_ubfe(w.w, 16u, 6u) << 6));
+        } else
+            v.a = *reinterpret_cast<const uint4 *>(tile + chunk * 32u + 16u * (q & 1u));
+        if constexpr (fmt<SRC>() == F_XS) v.c = *reinterpret_cast<const uint16_t *>(scs + chunk * 4u + 2u * (q & 1u));
+        d.x = *reinterpret_cast<const uint16_t *>(ds + (kc * 16u + r) * 2u);
+    } else if constexpr (layout<SRC>() == L_ROWS) {
+        v.a = *reinterpret_cast<const uint4 *>(tile + block * 64u + 16u * q);
+        d.x = *reinterpret_cast<const uint16_t *>(ds + block * 2u);
     } else {
-        const uint2 qs = load_a2<uint2>(bp + 8u * part);
-        v.a = make_uint4(qs.x, qs.y, load_a2<uint32_t>(bp + 32u + 4u * part), load_a2<uint16_t>(bp + 48u + 2u * part));
-        d = load_a2<uint2>(bp + 48u);
-    }
-    if constexpr (SRC == S_XS) v.c = load_a2<uint16_t>(bp + 66u + 2u * part);
-    if constexpr (SRC == S_IQ3) {
-        v.b = load_a2<uint2>(bp + 74u + 8u * part);
-        v.c = load_a2<uint16_t>(bp + 66u + 2u * part) | ((uint32_t)bp[106u + part] << 16);
+        const uint8_t *bp = tile + block * src_block<SRC>();
+        if constexpr (SRC == S_M) {
+            const uint2 qs = load_a2<uint2>(bp + 8u * q);
+            v.a = make_uint4(qs.x, qs.y, load_a2<uint32_t>(bp + 32u + 4u * q), load_a2<uint16_t>(bp + 48u + 2u * q));
+            d = load_a2<uint2>(bp + 48u);
+        } else {
+            v.a = load_a2<uint4>(bp + 2u + 16u * q);
+            d.x = load_a2<uint16_t>(bp);
+        }
+        if constexpr (SRC == S_XS) v.c = load_a2<uint16_t>(bp + 66u + 2u * q);
+        if constexpr (SRC == S_IQ3) {
+            const uint2 sg = load_a2<uint2>(bp + 74u + 8u * q);
+            v.b.x = sg.x; v.b.y = sg.y;
+            v.c = load_a2<uint16_t>(bp + 66u + 2u * q) | ((uint32_t)bp[106u + q] << 16);
+        }
     }
 }
 template <int SRC>
@@ -128,6 +163,7 @@ __device__ __forceinline__ float quarter_d(uint2 d) {
     if constexpr (SRC == S_M) return scale_to_f32(((d.x >> 12) & 0x000fu) | ((d.x >> 24) & 0x00f0u) | ((d.y >> 4) & 0x0f00u) | ((d.y >> 16) & 0xf000u));
     else return scale_to_f32(d.x);
 }
+
 // odd integer 2 s + 1 (s < 16) as two equal fp16 halves: 1024 + (2 s + 1) by integer arithmetic, minus 1024, exact
 __device__ __forceinline__ half2_t odd_splat(uint32_t s) {
     const half2_t big = {(_Float16)1024.0f, (_Float16)1024.0f};
@@ -145,16 +181,22 @@ template <int SRC>
 __device__ __forceinline__ Entry fetch_entry(const Quarter &v, uint32_t s, const LaneTables &t) {
     const uint32_t h = s >> 2, e = s & 3u;                 // group of the quarter, entry of the group
     Entry r;
-    if constexpr (SRC == S_XXS || SRC == S_PACKED_XXS) {
+    if constexpr (fmt<SRC>() == F_XXS) {
         const uint32_t wa = h ? v.a.z : v.a.x, wb = h ? v.a.w : v.a.y;
         // bytes 0 .. 3 of the permute's second operand are the entries, 7 the top byte of the first
         r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_perm(wb, wa, 0x0c0c0007u | (e << 8)) & 0xfff0u));
         r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(wb, 7u * e, 7u) << 6));
-    } else if constexpr (SRC == S_XS) {
+    } else if constexpr (fmt<SRC>() == F_XS) {
         const uint32_t w = word_of(v.a, 2u * h + (e >> 1)), o = 16u * (e & 1u);
         r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_ubfe(w, o, 9u) << 7));
         r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(w, o + 9u, 7u) << 6));
-    } else if constexpr (SRC == S_M) {
+    } else if constexpr (fmt<SRC>() == F_IQ3_WORDS) {
+        const uint32_t w = word_of(h ? v.b : v.a, e), scale = (w >> 14) & 0xf000u;      // nibble * 512 entries * 8 bytes
+        const uint2 ma = *reinterpret_cast<const uint2 *>(t.entries + (((w << 3) & 0xff8u) | scale));
+        const uint2 mb = *reinterpret_cast<const uint2 *>(t.entries + (((w >> 6) & 0xff8u) | scale));
+        r.m = make_uint4(ma.x, ma.y, mb.x, mb.y);
+        r.s = *reinterpret_cast<const uint32_t *>(t.signs + ((w >> 14) & 0xff0u));
+    } else if constexpr (fmt<SRC>() == F_M) {
         r.s = __builtin_amdgcn_ubfe(v.a.z, 16u * h + 4u * e, 4u);
         r.m = *reinterpret_cast<const uint4 *>(t.entries + ((__builtin_amdgcn_ubfe(h ? v.a.y : v.a.x, 8u * e, 8u) | ((r.s & 7u) << 8)) << 5));
     } else {
@@ -173,7 +215,7 @@ __device__ __forceinline__ Entry fetch_entry(const Quarter &v, uint32_t s, const
 template <int SRC>
 __device__ __forceinline__ half2_t step_scale(const Quarter &v, uint32_t s) {
     const uint32_t h = s >> 2, e = s & 3u;
-    if constexpr (SRC == S_XS) return odd_splat(__builtin_amdgcn_ubfe(v.c, 8u * h + 4u * (e >> 1), 4u));
+    if constexpr (fmt<SRC>() == F_XS) return odd_splat(__builtin_amdgcn_ubfe(v.c, 8u * h + 4u * (e >> 1), 4u));
     else return odd_splat(__builtin_amdgcn_ubfe(v.a.w, 6u * h + 3u * (e >> 1), 3u));
 }
 template <int SRC>
@@ -181,13 +223,13 @@ __device__ __forceinline__ half8_t finish_entry(const Entry &e, half2_t f) {
     constexpr uint32_t kSign = 0x80008000u;
     H8 r;
     r.u = e.m;
-    if constexpr (SRC == S_M) {
+    if constexpr (fmt<SRC>() == F_M) {
         // (2 s + 1) / 8 with the sign of the offset: three exponent steps down (2 s + 1 >= 1 is a normal number), sign bit by xor
         const uint32_t neg = (e.s & 8u) << 12;
         const half2_t off = __builtin_bit_cast(half2_t, (__builtin_bit_cast(uint32_t, f) - 0x0c000c00u) ^ (neg | (neg << 16)));
 #pragma unroll
         for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * f + off;
-    } else if constexpr (SRC == S_XS) {     // entries are signed bytes in general: the sign goes to the (positive) scale
+    } else if constexpr (fmt<SRC>() == F_XS) {     // entries are signed bytes in general: the sign goes to the (positive) scale
 #pragma unroll
         for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * __builtin_bit_cast(half2_t, __builtin_bit_cast(uint32_t, f) | ((e.s << i) & kSign));
     } else {
@@ -199,7 +241,7 @@ __device__ __forceinline__ half8_t finish_entry(const Entry &e, half2_t f) {
 struct StagedArgs {
     const uint8_t *experts, *shared;       // first matrix of expert uid[u] at experts + uid[u] * stride; of group n_unique[0] at `shared`
     uint64_t stride, mat_step;             // mat_step: gate/up, distance of the up matrix
-    uint64_t d_off;                        // packed rows: the block scales [row][K / 256] behind the rows of a matrix
+    uint64_t d_off;                        // not raw rows: the block scales behind the quarters of a matrix (tile-major IQ2_XS: the scale bytes behind them)
     const uint32_t *uid, *pair_token, *n_unique, *tile_group, *tile_pair0, *tile_n, *n_tiles;
     const _Float16 *xh, *xl;               // gate/up in: [ntok][K]
     const int *xexp;                       // [ntok]
@@ -230,7 +272,7 @@ template <int SRC, bool DOWN, int SETS, uint32_t KP>
 __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t *tile_group, const uint32_t *tile_pair0, const uint32_t *tile_n, uint32_t u0,
                                              uint32_t u1, float *part, TileInfo *tiles, PairInfo *pairs, uint8_t *entries, uint32_t *signs, const LaneTables &lt) {
     constexpr uint32_t NRT = staged_nrt(KP), WV = KP * NRT, T = staged_threads(SETS, KP), M = SETS == 1 ? 1u : 2u;      // M: halves per wave
-    constexpr uint32_t K = 256u * KP, RB = KP * src_block<SRC>(), seg_rows = 16u * NRT, seg = seg_rows * RB, blocks = seg_rows * KP;
+    constexpr uint32_t K = 256u * KP, seg_rows = 16u * NRT, tile_bytes = 16u * KP * src_block<SRC>();
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), w8 = wave % WV, m_first = SETS == 1 ? wave / WV : 0u, kc = w8 % KP, rt = w8 / KP;
     const uint32_t upt = a.rows / ((DOWN ? 2u : 1u) * seg_rows), U = a.n_unique[0];
@@ -238,24 +280,20 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
         const uint32_t u = tile_group[tile];
         return u == U ? (uint64_t)(a.shared - a.experts) : (uint64_t)a.uid[u] * a.stride;
     };
-    const auto run_of = [&](const uint8_t *mat, uint32_t j, uint32_t m) {      // rows of half m of unit j
-        return mat + (DOWN ? (uint64_t)(2u * j + m) * seg : m * a.mat_step + (uint64_t)j * seg);
-    };
-    const auto scales_of = [&](const uint8_t *mat, uint32_t j, uint32_t m) {   // packed rows: their block scales
-        return mat + a.d_off + (DOWN ? (uint64_t)(2u * j + m) * blocks * 2u : m * a.mat_step + (uint64_t)j * blocks * 2u);
-    };
     // the lane's quarters of a unit, and what their d are made from
     struct Carried { Quarter v[M]; uint2 d[M]; };
-    const uint32_t lane_block = (16u * rt + r) * KP + kc;
     const auto request = [&](Carried &c, const uint8_t *mat, uint32_t j) {
-        const uint32_t b = each_trip(lane_block);
 #pragma unroll
-        for (uint32_t m = 0; m < M; ++m) load_quarter<SRC>(run_of(mat, j, m_first + m) + b * src_block<SRC>(), scales_of(mat, j, m_first + m) + b * 2u, q, c.v[m], c.d[m]);
+        for (uint32_t m = 0; m < M; ++m) {
+            const uint32_t half = m_first + m, row_tile = (DOWN ? 2u * j + half : j) * NRT + rt;
+            const uint8_t *mm = mat + (DOWN ? 0u : half * a.mat_step), *ds = mm + a.d_off + row_tile * (KP * 32u);
+            load_quarter<SRC, KP>(mm + (uint64_t)row_tile * tile_bytes, ds, fmt<SRC>() == F_XS ? mm + a.d_off + (uint64_t)a.rows * KP * 2u + row_tile * (KP * 128u) : nullptr, r, kc, q, c.v[m], c.d[m]);
+        }
     };
     const uint32_t tile0 = u0 / upt, n_info = (u1 - 1u) / upt + 1u - tile0 < kTileInfos ? (u1 - 1u) / upt + 1u - tile0 : kTileInfos;
     const auto pair_info = [&](uint32_t p0, uint32_t n, uint32_t i) {          // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
         const uint32_t p = i < n ? p0 + i : p0, tok = p < a.P ? a.pair_token[p] : p - a.P;
-        return PairInfo{tok, (SRC == S_M || SRC == S_IQ3 ? 1.0f : 0.125f) * exp2i(a.xexp[tok])};
+        return PairInfo{tok, format_scale<SRC>() * exp2i(a.xexp[tok])};
     };
     {
         TileInfo ti{};
@@ -284,17 +322,17 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
 #pragma unroll
         for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
             __builtin_amdgcn_sched_barrier(0);             // one set at a time: both at once do not fit the registers
-            const uint32_t l = each_trip(lane), q64 = 64u * (l >> 4), i = 16u * s + (l & 15u);
+            const uint32_t l = each_trip(lane), lq = l >> 4, i = 16u * s + (l & 15u);
             float scale;
             if constexpr (!DOWN) {
                 const PairInfo pi = tile - tile0 < kTileInfos ? pairs[(tile - tile0) * 16u * SETS + i] : pair_info(p0, n, i);
                 scale = pi.scale;
-                const uint64_t base = (uint64_t)pi.tok * K + 256u * kc + q64;
+                const uint64_t base = (uint64_t)pi.tok * K + 256u * kc;
                 const _Float16 *hp = a.xh + base, *lp = a.xl + base;
 #pragma unroll
                 for (uint32_t g = 0; g < 8u; ++g) {
-                    xa[s][g].u = *reinterpret_cast<const uint4 *>(hp + 8u * g);
-                    xb[s][g].u = *reinterpret_cast<const uint4 *>(lp + 8u * g);
+                    xa[s][g].u = *reinterpret_cast<const uint4 *>(hp + step_column<SRC>(g, lq));
+                    xb[s][g].u = *reinterpret_cast<const uint4 *>(lp + step_column<SRC>(g, lq));
                 }
                 // the low halves are stored times 2^11: back to their own scale (exact, the largest |x| of a token sits in [2^13, 2^14)), so that a
                 // product's high and low parts add up in one accumulator
@@ -303,11 +341,11 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 if (s + 1u == (uint32_t)SETS) __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): waited for here, once per tile, not (by count) where the loop uses them
             } else {
                 // f32 activations of pair p, columns of this wave's K part: one exponent for them, then the fp16 halves
-                const float *src = a.act + (uint64_t)(i < n ? p0 + i : p0) * K + 256u * kc + q64;
+                const float *src = a.act + (uint64_t)(i < n ? p0 + i : p0) * K + 256u * kc;
                 float amax = 0.0f;
 #pragma unroll
                 for (uint32_t g = 0; g < 8u; ++g) {
-                    const float4 v0 = *reinterpret_cast<const float4 *>(src + 8u * g), v1 = *reinterpret_cast<const float4 *>(src + 8u * g + 4u);
+                    const float4 v0 = *reinterpret_cast<const float4 *>(src + step_column<SRC>(g, lq)), v1 = *reinterpret_cast<const float4 *>(src + step_column<SRC>(g, lq) + 4u);
                     xa[s][g].u = __builtin_bit_cast(uint4, v0);
                     xb[s][g].u = __builtin_bit_cast(uint4, v1);
                 }
@@ -320,7 +358,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
                 const int e = prescale_exp(amax);
                 const float inv = exp2i(-e);
-                scale = (SRC == S_M || SRC == S_IQ3 ? 1.0f : 0.125f) * exp2i(e);
+                scale = format_scale<SRC>() * exp2i(e);
 #pragma unroll
                 for (uint32_t g = 0; g < 8u; ++g) {
                     const float4 v0 = __builtin_bit_cast(float4, xa[s][g].u), v1 = __builtin_bit_cast(float4, xb[s][g].u);
@@ -340,7 +378,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 }
             }
 #pragma unroll
-            for (uint32_t t = 0; t < 4u; ++t) ps[s][t] = __shfl(scale, (int)(q64 / 16u + t), 64);
+            for (uint32_t t = 0; t < 4u; ++t) ps[s][t] = __shfl(scale, (int)(4u * lq + t), 64);
         }
     };
     // partial sums of the waves: [row tile, K part][m][set][lane] float4
@@ -435,7 +473,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
             half8_t w[M];
 #pragma unroll
             for (uint32_t m = 0; m < M; ++m) {
-                if constexpr (SRC == S_XS || SRC == S_M) { if ((s8 & 1u) == 0u) f[m] = step_scale<SRC>(c.v[m], s8); }
+                if constexpr (fmt<SRC>() == F_XS || fmt<SRC>() == F_M) { if ((s8 & 1u) == 0u) f[m] = step_scale<SRC>(c.v[m], s8); }
                 w[m] = finish_entry<SRC>(s8 & 1u ? e1[m] : e0[m], f[m]);
                 if (s8 + 2u < 8u) { if (s8 & 1u) e1[m] = fetch_entry<SRC>(c.v[m], s8 + 2u, lt); else e0[m] = fetch_entry<SRC>(c.v[m], s8 + 2u, lt); }
             }
@@ -514,8 +552,8 @@ __global__ __launch_bounds__(staged_threads(SETS, KP)) void staged_tiles_kernel(
     if (u0 >= u1) return;
     __shared__ TileInfo tiles[kTileInfos];
     __shared__ PairInfo pairs[DOWN ? 1u : kTileInfos * 16u * SETS];
-    const LaneTables lt{entries + (SRC == S_XS ? (tid & 7u) * 16u : SRC == S_M ? (tid & 1u) * 16u : 0u),
-                        reinterpret_cast<const uint8_t *>(signs) + (SRC == S_IQ3 ? (tid & 3u) * 4u : SRC == S_M ? 0u : (tid & 15u) * 4u)};
+    const LaneTables lt{entries + (fmt<SRC>() == F_XS ? (tid & 7u) * 16u : fmt<SRC>() == F_M ? (tid & 1u) * 16u : 0u),
+                        reinterpret_cast<const uint8_t *>(signs) + (is_iq3<SRC>() ? (tid & 3u) * 4u : fmt<SRC>() == F_M ? 0u : (tid & 15u) * 4u)};
     staged_units<SRC, DOWN, SETS, KP>(a, a.tile_group + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, part, tiles, pairs, entries, signs, lt);
 }
 
@@ -531,70 +569,104 @@ hipError_t launch_staged_lists(const StagedArgs &a, uint32_t grid, bool wide, hi
     return e == hipSuccess ? launch_staged_list<SRC, DOWN, 1, KP>(a, grid, s) : e;
 }
 template <int SRC>
-hipError_t launch_staged_gateup(const StagedArgs &a, uint32_t hidden, uint32_t grid, bool wide, hipStream_t s) {
+hipError_t staged_gateup(const StagedArgs &a, uint32_t hidden, uint32_t grid, bool wide, hipStream_t s) {
     return hidden == 512u    ? launch_staged_lists<SRC, false, 2>(a, grid, wide, s)
            : hidden == 1024u ? launch_staged_lists<SRC, false, 4>(a, grid, wide, s)
                              : launch_staged_lists<SRC, false, 8>(a, grid, wide, s);
 }
 template <int SRC>
-hipError_t launch_staged_down(const StagedArgs &a, uint32_t ffn, uint32_t grid, bool wide, hipStream_t s) {
-    return ffn == 256u   ? launch_staged_lists<SRC, true, 1>(a, grid, wide, s)
-           : ffn == 512u ? launch_staged_lists<SRC, true, 2>(a, grid, wide, s)
-           : ffn == 768u ? launch_staged_lists<SRC, true, 3>(a, grid, wide, s)
-                         : launch_staged_lists<SRC, true, 4>(a, grid, wide, s);
+hipError_t staged_down(const StagedArgs &a, uint32_t ffn, uint32_t grid, bool wide, hipStream_t s) {
+    if (ffn == 256u) return launch_staged_lists<SRC, true, 1>(a, grid, wide, s);
+    if (ffn == 512u) return launch_staged_lists<SRC, true, 2>(a, grid, wide, s);
+    if constexpr (layout<SRC>() == L_TILED) return hipErrorInvalidValue;      // (tile-major copies are made for ffn <= 512)
+    else return ffn == 768u ? launch_staged_lists<SRC, true, 3>(a, grid, wide, s) : launch_staged_lists<SRC, true, 4>(a, grid, wide, s);
 }
 
-int staged_src(uint32_t type, bool packed) {
-    if (packed) return type == T_IQ2_XXS ? S_PACKED_XXS : -1;
+int staged_src(uint32_t type, RowLayout lay) {
+    if (lay == RowLayout::rows) return type == T_IQ2_XXS ? S_ROWS_XXS : -1;
+    if (lay == RowLayout::tiled) return type == T_IQ2_XXS ? S_TILED_XXS : type == T_IQ2_XS ? S_TILED_XS : type == T_IQ1_M ? S_TILED_M : type == T_IQ3_S ? S_TILED_IQ3 : -1;
     return type == T_IQ2_XXS ? S_XXS : type == T_IQ2_XS ? S_XS : type == T_IQ1_M ? S_M : type == T_IQ3_S ? S_IQ3 : -1;
+}
+
+StagedArgs staged_args(const StagedMatrices &m, const StagedChunk &c, uint32_t K, uint32_t rows) {
+    const int src = staged_src(m.type, m.layout);
+    StagedArgs a{};
+    a.experts = static_cast<const uint8_t *>(m.experts);
+    a.shared = static_cast<const uint8_t *>(m.shared);
+    a.stride = m.stride;
+    a.mat_step = m.up_delta;
+    a.d_off = src == S_TILED_IQ3 ? (uint64_t)rows * (K / 32u) * 16u : (uint64_t)rows * (K / 32u) * 8u;
+    a.uid = c.uid; a.pair_token = c.pair_token; a.n_unique = c.n_unique;
+    a.tile_group = c.tl.tile_group; a.tile_pair0 = c.tl.tile_pair0; a.tile_n = c.tl.tile_n; a.n_tiles = c.tl.n_tiles;
+    a.list_stride = c.tl.list_stride;
+    a.grid = m.grid;
+    a.rows = rows;
+    a.P = c.ntok * c.top_k;
+    return a;
+}
+// persistent workgroups, one per compute unit; fewer where a chunk cannot have as many units as that
+uint32_t staged_grid(const StagedChunk &c) {
+    const uint32_t bound = 4u * prefill_tile_bound(c.ntok, c.top_k, c.n_expert);
+    return bound < 256u ? bound : 256u;
+}
+bool staged_wide(const StagedChunk &c) {               // a wide tile has 17 pairs or more
+    const uint32_t most = c.ntok * c.top_k / (kPrefillTile + 1u) + c.tl.shared_ntok / (kPrefillTile + 1u);
+    return (c.wide_tiles < most ? c.wide_tiles : most) >= kFewWide;
 }
 
 }  // namespace
 
+bool staged_gateup_supported(uint32_t type, RowLayout lay, uint32_t hidden, uint32_t ffn) {
+    const int src = staged_src(type, lay);
+    return src >= 0 && type != T_IQ3_S && (hidden == 512u || hidden == 1024u || hidden == 2048u) && ffn && ffn % 128u == 0u;
+}
 // one block of 256 columns per wave: two to eight of them (hidden), one to four (ffn)
-bool staged_tiles_supported(uint32_t gate_up_type, uint32_t down_type, uint32_t hidden, uint32_t ffn, uint32_t n_expert, bool packed) {
-    const int g = staged_src(gate_up_type, packed), d = staged_src(down_type, packed);
-    return g >= 0 && g != S_IQ3 && d >= 0 && (hidden == 512u || hidden == 1024u || hidden == 2048u) && (ffn == 256u || ffn == 512u || ffn == 768u || ffn == 1024u) && n_expert <= 1024u;
+bool staged_down_supported(uint32_t type, RowLayout lay, uint32_t hidden, uint32_t ffn) {
+    return staged_src(type, lay) >= 0 && hidden && hidden % 256u == 0u && (ffn == 256u || ffn == 512u || (lay != RowLayout::tiled && (ffn == 768u || ffn == 1024u)));
 }
 
-hipError_t launch_staged_tiles(const StagedExperts &x, const uint32_t *uid, const uint32_t *expert_start, const uint32_t *pair_token, const uint32_t *n_unique,
-                               const TileLists &tl, bool tiles_built, const void *xh, const void *xl, const int *xexp, float *act, float *tmp, float *sh_tmp,
-                               uint32_t hidden, uint32_t ffn, uint32_t top_k, uint32_t ntok, uint32_t n_expert, hipStream_t s) {
-    if (!staged_tiles_supported(x.gate_up_type, x.down_type, hidden, ffn, n_expert, x.packed) || !ntok || (tl.shared_ntok && (!x.shared || !sh_tmp))) return hipErrorInvalidValue;
-    const uint32_t P = ntok * top_k;
-    if (!tiles_built) {
-        prof_set_stage(ST_GROUP);
-        const hipError_t e = launch_build_tiles(expert_start, n_unique, P, tl, s);
-        if (e != hipSuccess) return e;
-    }
-    const uint32_t bound = prefill_tile_bound(ntok, top_k, n_expert), grid = 4u * bound < 256u ? 4u * bound : 256u;
-    StagedArgs a{static_cast<const uint8_t *>(x.gate), static_cast<const uint8_t *>(x.shared), x.stride, x.up_delta, (uint64_t)ffn * (hidden / 32u) * 8u,
-                 uid, pair_token, n_unique, tl.tile_group, tl.tile_pair0, tl.tile_n, tl.n_tiles, static_cast<const _Float16 *>(xh), static_cast<const _Float16 *>(xl), xexp,
-                 act, tmp, sh_tmp, x.gate_up_grid, ffn, P, tl.list_stride};
-    const bool wide = P > kPrefillTile;
-    hipError_t e = hipErrorInvalidValue;
+hipError_t launch_staged_gateup(const StagedMatrices &m, const StagedChunk &c, const void *xh, const void *xl, const int *xexp, float *act, uint32_t hidden, uint32_t ffn,
+                                hipStream_t s) {
+    if (!staged_gateup_supported(m.type, m.layout, hidden, ffn) || !c.ntok || (c.tl.shared_ntok && !m.shared)) return hipErrorInvalidValue;
+    StagedArgs a = staged_args(m, c, hidden, ffn);
+    a.xh = static_cast<const _Float16 *>(xh);
+    a.xl = static_cast<const _Float16 *>(xl);
+    a.xexp = xexp;
+    a.act = act;
+    const uint32_t grid = staged_grid(c);
+    const bool wide = staged_wide(c);
     prof_set_stage(ST_PREFILL_GATEUP);
-    switch (staged_src(x.gate_up_type, x.packed)) {
-        case S_XXS: e = launch_staged_gateup<S_XXS>(a, hidden, grid, wide, s); break;
-        case S_XS: e = launch_staged_gateup<S_XS>(a, hidden, grid, wide, s); break;
-        case S_M: e = launch_staged_gateup<S_M>(a, hidden, grid, wide, s); break;
-        case S_PACKED_XXS: e = launch_staged_gateup<S_PACKED_XXS>(a, hidden, grid, wide, s); break;
+    switch (staged_src(m.type, m.layout)) {
+        case S_XXS: return staged_gateup<S_XXS>(a, hidden, grid, wide, s);
+        case S_XS: return staged_gateup<S_XS>(a, hidden, grid, wide, s);
+        case S_M: return staged_gateup<S_M>(a, hidden, grid, wide, s);
+        case S_ROWS_XXS: return staged_gateup<S_ROWS_XXS>(a, hidden, grid, wide, s);
+        case S_TILED_XXS: return staged_gateup<S_TILED_XXS>(a, hidden, grid, wide, s);
+        case S_TILED_XS: return staged_gateup<S_TILED_XS>(a, hidden, grid, wide, s);
+        case S_TILED_M: return staged_gateup<S_TILED_M>(a, hidden, grid, wide, s);
     }
-    if (e != hipSuccess) return e;
-    a.experts = static_cast<const uint8_t *>(x.down);
-    a.stride = x.down_stride;
-    a.mat_step = 0u;
-    if (x.shared) a.shared += 2u * x.up_delta;
-    a.d_off = (uint64_t)hidden * (ffn / 32u) * 8u;
-    a.grid = x.down_grid;
-    a.rows = hidden;
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_staged_down(const StagedMatrices &m, const StagedChunk &c, const float *act, float *tmp, float *sh_tmp, uint32_t hidden, uint32_t ffn, hipStream_t s) {
+    if (!staged_down_supported(m.type, m.layout, hidden, ffn) || !c.ntok || (c.tl.shared_ntok && (!m.shared || !sh_tmp))) return hipErrorInvalidValue;
+    StagedArgs a = staged_args(m, c, ffn, hidden);
+    a.act = const_cast<float *>(act);
+    a.tmp = tmp;
+    a.sh_tmp = sh_tmp;
+    const uint32_t grid = staged_grid(c);
+    const bool wide = staged_wide(c);
     prof_set_stage(ST_PREFILL_DOWN);
-    switch (staged_src(x.down_type, x.packed)) {
-        case S_XXS: return launch_staged_down<S_XXS>(a, ffn, grid, wide, s);
-        case S_XS: return launch_staged_down<S_XS>(a, ffn, grid, wide, s);
-        case S_M: return launch_staged_down<S_M>(a, ffn, grid, wide, s);
-        case S_IQ3: return launch_staged_down<S_IQ3>(a, ffn, grid, wide, s);
-        case S_PACKED_XXS: return launch_staged_down<S_PACKED_XXS>(a, ffn, grid, wide, s);
+    switch (staged_src(m.type, m.layout)) {
+        case S_XXS: return staged_down<S_XXS>(a, ffn, grid, wide, s);
+        case S_XS: return staged_down<S_XS>(a, ffn, grid, wide, s);
+        case S_M: return staged_down<S_M>(a, ffn, grid, wide, s);
+        case S_IQ3: return staged_down<S_IQ3>(a, ffn, grid, wide, s);
+        case S_ROWS_XXS: return staged_down<S_ROWS_XXS>(a, ffn, grid, wide, s);
+        case S_TILED_XXS: return staged_down<S_TILED_XXS>(a, ffn, grid, wide, s);
+        case S_TILED_XS: return staged_down<S_TILED_XS>(a, ffn, grid, wide, s);
+        case S_TILED_M: return staged_down<S_TILED_M>(a, ffn, grid, wide, s);
+        case S_TILED_IQ3: return staged_down<S_TILED_IQ3>(a, ffn, grid, wide, s);
     }
     return hipErrorInvalidValue;
 }

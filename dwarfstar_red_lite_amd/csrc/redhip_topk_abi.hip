@@ -337,6 +337,9 @@ struct PairExperts {
     uint64_t stride, down_stride, up_delta;
     std::vector<uint32_t> uid;
 };
+bool rows_on_tiles(uint32_t type_word, uint32_t hidden, uint32_t ffn, uint32_t n_expert) {
+    return n_expert <= 1024u && staged_gateup_supported(word_gate_up(type_word), RowLayout::raw, hidden, ffn) && staged_down_supported(word_down(type_word), RowLayout::raw, hidden, ffn);
+}
 // slots: an expert is named by the distance of its slot from the lowest slot of the call, in units of 256 bytes (slots are 4096-aligned,
 // HBM is far below 1 TB)
 bool slot_experts(const std::vector<uint64_t> &slot_addr, uint64_t gate_bytes, PairExperts *ex) {
@@ -366,11 +369,11 @@ bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const PairExperts &ex, bool
     u.insert(u.end(), ex.uid.begin(), ex.uid.end());
     u.push_back(n_expert);
     // scratch of the call: rows of x up to the last token of the call, n_pairs activation rows
-    const size_t rows = (size_t)tok_first + ntok, arows = (size_t)n_pairs + ntok;
+    const size_t rows = (size_t)tok_first + ntok;
     const uint32_t bound = prefill_tile_bound(ntok, top_k, n_expert);
     auto a256 = [](size_t v) { return (v + 255u) & ~(size_t)255u; };
-    const size_t x_half = a256(rows * hidden * 2u), x_exp = a256(rows * 4u), a_half = a256(arows * ffn * 2u), a_exp = a256(arows * (ffn / 32u) * 4u), tl = a256(12u * (size_t)bound);
-    if (!p->chunk.reserve(2u * x_half + 2u * x_exp + 2u * a_half + a_exp + 4u * tl) || !p->tmp_b.reserve((size_t)n_pairs * hidden * sizeof(float))) {
+    const size_t x_half = a256(rows * hidden * 2u), x_exp = a256(rows * 4u), a_bytes = a256((size_t)n_pairs * ffn * 4u), tl = a256(12u * (size_t)bound);
+    if (!p->chunk.reserve(2u * x_half + 2u * x_exp + a_bytes + 4u * tl) || !p->tmp_b.reserve((size_t)n_pairs * hidden * sizeof(float))) {
         TOPK_ERR("failed to allocate top-k activation buffers");
         return false;
     }
@@ -379,9 +382,7 @@ bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const PairExperts &ex, bool
     void *xl = w; w += x_half;
     int *xexp = reinterpret_cast<int *>(w); w += x_exp;
     float *gate_unused = reinterpret_cast<float *>(w); w += x_exp;
-    void *act_h = w; w += a_half;
-    void *act_l = w; w += a_half;
-    int *act_exp = reinterpret_cast<int *>(w); w += a_exp;
+    float *act = reinterpret_cast<float *>(w); w += a_bytes;
     uint32_t *tile_group = reinterpret_cast<uint32_t *>(w); w += tl;
     uint32_t *tile_pair0 = reinterpret_cast<uint32_t *>(w); w += tl;
     uint32_t *tile_n = reinterpret_cast<uint32_t *>(w); w += tl;
@@ -390,28 +391,23 @@ bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const PairExperts &ex, bool
     if (!stage_lists(p, s, {}, pair_weight, n_pairs, u, &st)) return false;
     const uint32_t *d_pair_token = st.u, *d_start = st.u + n_pairs, *d_tok_pair = d_start + n_expert + 1u, *d_uid = d_tok_pair + (size_t)ntok * top_k, *d_unique = d_uid + n_expert;
     float *tmp = static_cast<float *>(p->tmp_b.p);
-    const uint8_t *tiles = ex.gate + p->fs.tile_off;
     // (the split kernel also forms a gate logit per row from a second vector: x itself stands in, the result is not used)
     hipError_t e = launch_prep(x, x, (uint32_t)rows, hidden, xh, xl, xexp, gate_unused, s, nullptr, nullptr);
-    if (e == hipSuccess && !copies) {
-        const uint32_t gu = word_gate_up(type_word), dn = word_down(type_word);
-        const StagedExperts rows{ex.gate, ex.down, nullptr, ex.stride, ex.down_stride, ex.up_delta, gu, dn, caller_grid_device(gu), caller_grid_device(dn), false};
-        e = launch_staged_tiles(rows, d_uid, d_start, d_pair_token, d_unique, TileLists{tile_group, tile_pair0, tile_n, n_tiles, bound, 0u}, false, xh, xl, xexp,
-                                static_cast<float *>(act_h), tmp, nullptr, hidden, ffn, top_k, ntok, n_expert, s);      // (act_h | act_l: as many bytes as f32)
-    } else if (e == hipSuccess && p->fs.kind == 0u)
-        e = launch_prefill_packed(nullptr, 256u, nullptr, tiles, nullptr, d_uid, d_start, d_pair_token, d_unique, tile_group, tile_pair0, tile_n, n_tiles,
-                                  xh, xl, xexp, act_h, act_l, act_exp, tmp, nullptr, hidden, ffn, top_k, ntok, n_expert, s, false, false);
-    else if (e == hipSuccess && p->fs.kind == 1u) {      // IQ2_XXS gate / up tiles, then the IQ3_S down tiles
-        e = launch_prefill_gateup_tiled(tiles, 256u, d_uid, d_start, d_pair_token, d_unique, tile_group, tile_pair0, tile_n, n_tiles, xh, xl, xexp, nullptr, act_h, act_l,
-                                        act_exp, hidden, ffn, top_k, ntok, n_expert, s, false);
-        if (e == hipSuccess)
-            e = launch_prefill_down_iq3s(tiles + 2u * p->fs.gate_copy, 256u, d_uid, d_unique, tile_group, tile_pair0, tile_n, n_tiles, act_h, act_l, act_exp, tmp, hidden, ffn,
-                                         top_k, ntok, n_expert, s);
-    } else if (e == hipSuccess) {      // IQ2_XS / IQ1_M: the same tile kernels on the tile-major streams, through the pool's codebooks
-        const uint32_t t = word_gate_up(p->fs.word);
-        e = launch_prefill_streams(t, caller_grid_device(t), tiles, 256u, t, caller_grid_device(t), tiles + 2u * p->fs.gate_copy, 256u, d_uid, d_start, d_pair_token,
-                                   d_unique, tile_group, tile_pair0, tile_n, n_tiles, xh, xl, xexp, act_h, act_l, act_exp, tmp, hidden, ffn, top_k, ntok, n_expert, s, false);
+    const TileLists lists{tile_group, tile_pair0, tile_n, n_tiles, bound, 0u};
+    if (e == hipSuccess) e = launch_build_tiles(d_start, d_unique, n_pairs, lists, s);
+    uint32_t wide = 0u;
+    for (uint32_t i = 0; i < n_expert; ++i) {
+        const uint32_t m = expert_start[i + 1u] - expert_start[i];
+        wide += m / kPrefillWideTile + (m % kPrefillWideTile > kPrefillTile ? 1u : 0u);
     }
+    const uint32_t gu = word_gate_up(type_word), dn = word_down(type_word);
+    const RowLayout lay = copies ? RowLayout::tiled : RowLayout::raw;
+    const uint8_t *tiles = ex.gate + p->fs.tile_off;
+    const StagedChunk chunk{d_uid, d_pair_token, d_unique, lists, ntok, top_k, n_expert, wide};
+    const StagedMatrices gate_up{gu, lay, copies ? tiles : ex.gate, nullptr, ex.stride, copies ? p->fs.gate_copy : ex.up_delta, caller_grid_device(gu)};
+    const StagedMatrices down{dn, lay, copies ? tiles + 2u * p->fs.gate_copy : ex.down, nullptr, ex.down_stride, 0u, caller_grid_device(dn)};
+    if (e == hipSuccess) e = launch_staged_gateup(gate_up, chunk, xh, xl, xexp, act, hidden, ffn, s);
+    if (e == hipSuccess) e = launch_staged_down(down, chunk, act, tmp, nullptr, hidden, ffn, s);
     if (e == hipSuccess) e = launch_batch_combine(tmp, st.w, d_tok_pair, ntok, top_k, nullptr, nullptr, hidden, out + (uint64_t)tok_first * hidden, s);
     stage_done(st, s);
     if (e != hipSuccess) { TOPK_ERR("batched top-k HIP command failed: %s", hipGetErrorString(e)); return false; }
@@ -920,7 +916,7 @@ int redmetal_topk_pool_encode_batched(redmetal_topk_pool_t h, void *stream, cons
         for (uint32_t i = 0; i < n_expert; ++i) tiles = tiles && p->shadow_ok[slot_ids[i]];
     }
     // slots without tile-major copies: the tile kernels on their raw rows, for the formats and shapes those take
-    const bool staged = !tiles && staged_tiles_supported(word_gate_up(ggml_type), word_down(ggml_type), hidden_size, ffn_size, n_expert, false);
+    const bool staged = !tiles && rows_on_tiles(ggml_type, hidden_size, ffn_size, n_expert);
     PairExperts ex;
     if (tiles || staged ? !slot_experts(table, gate_bytes[0], &ex) ||
                               !enqueue_pairs_tiles(p, static_cast<hipStream_t>(stream), ex, tiles, ggml_type, n_expert, hidden_size, ffn_size, tok_first, ntok, top_k, n_pairs,
@@ -947,7 +943,7 @@ int redmetal_topk_pool_encode_mapped(redmetal_topk_pool_t h, void *stream,
     if (!pool_shape_ok(hidden_size, ffn_size, true)) return 0;
     if (!pair_layout_ok("mapped", n_expert, tok_first, ntok, top_k, n_pairs, pair_token, expert_start, tok_pair)) return 0;
     if (((gate_addr0 | up_addr0 | down_addr0 | gate_bytes | down_bytes) & 15u) == 0u &&
-        staged_tiles_supported(word_gate_up(ggml_type), word_down(ggml_type), hidden_size, ffn_size, n_expert, false)) {
+        rows_on_tiles(ggml_type, hidden_size, ffn_size, n_expert)) {
         const PairExperts ex{reinterpret_cast<const uint8_t *>(gate_addr0), reinterpret_cast<const uint8_t *>(down_addr0), gate_bytes, down_bytes, up_addr0 - gate_addr0,
                              std::vector<uint32_t>(expert_ids, expert_ids + n_expert)};
         return enqueue_pairs_tiles(p, static_cast<hipStream_t>(stream), ex, false, ggml_type, n_expert, hidden_size, ffn_size, tok_first, ntok, top_k, n_pairs, pair_token,

@@ -161,24 +161,23 @@ inline uint32_t prefill_tile_bound(uint32_t ntok, uint32_t top_k, uint32_t n_exp
 hipError_t launch_tile_packed(const void *packed, uint64_t packed_stride, uint32_t count, uint32_t nrows, uint32_t K, void *tiled, uint64_t tiled_stride,
                               hipStream_t s, bool with_sc = false);
 hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count, uint32_t nrows, uint32_t K, void *tiled, uint64_t tiled_stride, hipStream_t s);
-// Tile lists of a chunk for the prefill kernels. Groups 0..U-1 are the distinct routed experts (pairs expert_start[u] ..
-// expert_start[u + 1]), group U is the shared expert with pairs P .. P + shared_ntok (0: no shared tiles). A tile = (group, first pair,
-// number of pairs). Three lists in the same arrays, list l from entry l * list_stride on (list_stride = prefill_tile_bound of the call),
+// Tile lists of a chunk for the tile kernels. Groups 0..U-1 are the distinct routed experts (pairs expert_start[u] ..
+// expert_start[u + 1]), the last is the shared expert with pairs P .. P + shared_ntok (0: no shared tiles). A tile = (expert id or
+// kSharedTile, first pair, number of pairs). Three lists in the same arrays, list l from entry l * list_stride on (list_stride = prefill_tile_bound of the call),
 // its length in n_tiles[l]:
-//   0  tiles of kPrefillTile pairs (the down kernels; the gate/up kernel of hidden 512)
+//   0  tiles of kPrefillTile pairs
 //   1  "wide" tiles of 17 .. kPrefillWideTile pairs: a group's runs of 32 pairs, and its remainder when that is more than 16
 //   2  "narrow" tiles: the remainders of 1 .. 16 pairs
-// Lists 1 and 2 together cover every pair once: the gate/up kernel takes the wide tiles on the path that multiplies two sets of 16 pairs
-// with every decoded weight, the narrow ones on the path for 16.
-constexpr uint32_t kPrefillTile = 16u, kPrefillWideTile = 32u;
+// List 0 covers every pair once, and so do lists 1 and 2 together: wide tiles multiply two sets of 16 pairs with every decoded weight.
+constexpr uint32_t kPrefillTile = 16u, kPrefillWideTile = 32u, kSharedTile = 0xffffffffu;
 struct TileLists {
-    uint32_t *tile_group, *tile_pair0, *tile_n, *n_tiles;
+    uint32_t *tile_expert, *tile_pair0, *tile_n, *n_tiles;
     uint32_t list_stride, shared_ntok;
 };
 #ifdef __HIPCC__
-// By all 1024 threads of one workgroup: thread u < U brings its group's run (first pair p0, n pairs), the others n = 0; wave_total:
-// LDS scratch. Exclusive prefix sums of the tiles per group, then every group writes its tiles.
-__device__ __forceinline__ void build_tile_lists(uint32_t U, uint32_t p0, uint32_t n, uint32_t P, const TileLists &tl, uint32_t (*wave_total)[16]) {
+// By all 1024 threads of one workgroup: thread u < U brings its group's expert and run (first pair p0, n pairs), the others n = 0;
+// wave_total: LDS scratch. Exclusive prefix sums of the tiles per group, then every group writes its tiles.
+__device__ __forceinline__ void build_tile_lists(uint32_t expert, uint32_t p0, uint32_t n, uint32_t P, const TileLists &tl, uint32_t (*wave_total)[16]) {
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
     auto counts = [](uint32_t m, uint32_t *c) {            // tiles of m pairs in the three lists
         const uint32_t rem = m % kPrefillWideTile;
@@ -207,22 +206,22 @@ __device__ __forceinline__ void build_tile_lists(uint32_t U, uint32_t p0, uint32
         for (uint32_t w = 0; w < 16u; ++w) { if (w < wave) base += wave_total[l][w]; routed_tiles += wave_total[l][w]; }
         const uint32_t off = (uint32_t)l * tl.list_stride, first = off + base + scan[l] - mine[l];
         // tile t of a run of m pairs that starts at pair q0, in list l
-        auto put = [&](uint32_t at, uint32_t group, uint32_t q0, uint32_t m, uint32_t t) {
+        auto put = [&](uint32_t at, uint32_t e, uint32_t q0, uint32_t m, uint32_t t) {
             const uint32_t size = l == 0 ? kPrefillTile : kPrefillWideTile, start = l == 2 ? m - m % kPrefillWideTile : size * t;
-            tl.tile_group[at] = group;
+            tl.tile_expert[at] = e;
             tl.tile_pair0[at] = q0 + start;
             tl.tile_n[at] = m - start < size ? m - start : size;
         };
-        for (uint32_t t = 0; t < mine[l]; ++t) put(first + t, tid, p0, n, t);
-        for (uint32_t t = tid; t < sh[l]; t += 1024u) put(off + routed_tiles + t, U, P, tl.shared_ntok, t);
+        for (uint32_t t = 0; t < mine[l]; ++t) put(first + t, expert, p0, n, t);
+        for (uint32_t t = tid; t < sh[l]; t += 1024u) put(off + routed_tiles + t, kSharedTile, P, tl.shared_ntok, t);
         if (tid == 0u) tl.n_tiles[l] = routed_tiles + sh[l];
     }
 }
 #endif
 // the tile lists as a launch of their own, for callers whose pair sort did not write them
-hipError_t launch_build_tiles(const uint32_t *expert_start, const uint32_t *n_unique, uint32_t n_pairs, const TileLists &tl, hipStream_t s);
+hipError_t launch_build_tiles(const uint32_t *uid, const uint32_t *expert_start, const uint32_t *n_unique, uint32_t n_pairs, const TileLists &tl, hipStream_t s);
 // A chunk's experts on the tile kernels (redhip_tiles.hip). `raw`: GGUF rows; `rows`: packed IQ2_XXS rows; `tiled`: tile-major copies
-// (launch_tile_packed, launch_tile_iq3s; ffn <= 512). Matrices are 16-byte aligned, the first of expert uid[u] at experts + uid[u] * stride
+// (launch_tile_packed, launch_tile_iq3s; ffn <= 512). Matrices are 16-byte aligned, the first of expert e at experts + e * stride
 // (gate/up: the up matrix up_delta behind it), of the shared expert at `shared` when tl.shared_ntok asks for its tiles.
 enum class RowLayout : uint32_t { raw, rows, tiled };
 struct StagedMatrices {
@@ -233,7 +232,7 @@ struct StagedMatrices {
     const int8_t *grid;                     // codebook of IQ2_XS / IQ1_M
 };
 struct StagedChunk {                        // the pair sort of the call, its tile lists among it
-    const uint32_t *uid, *pair_token, *n_unique;
+    const uint32_t *pair_token;
     TileLists tl;
     uint32_t ntok, top_k, n_expert;
     uint32_t wide_tiles = 0xffffffffu;      // tiles of more than kPrefillTile pairs, where the host knows their number

@@ -967,7 +967,7 @@ __global__ __launch_bounds__(1024) void group_pairs_kernel(const uint32_t *ids, 
         for (uint32_t p = tid; p < P; p += 1024u) place(p, id_of(p), weights[p]);
     }
     // the tile lists of the prefill kernels, from the group starts still in LDS: no launch of their own
-    if (tiles.tile_group) build_tile_lists(U, tid < U ? start[tid] : 0u, tid < U ? start[tid + 1u] - start[tid] : 0u, P, tiles, tile_tot);
+    if (tiles.tile_expert) build_tile_lists(tid < U ? uid_l[tid] : 0u, tid < U ? start[tid] : 0u, tid < U ? start[tid + 1u] - start[tid] : 0u, P, tiles, tile_tot);
 }
 
 // The same sort for chunks of more than 512 tokens, whose token bitmaps per expert would not fit the LDS (2048 tokens x 512 experts: 128
@@ -1065,7 +1065,7 @@ __global__ __launch_bounds__(1024) void group_pairs_blocked_kernel(const uint32_
         if (tid < n_expert) cursor[tid] += block_count;
     }
     __syncthreads();
-    if (tiles.tile_group) build_tile_lists(U, tid < U ? start[tid] : 0u, tid < U ? start[tid + 1u] - start[tid] : 0u, P, tiles, tile_tot);
+    if (tiles.tile_expert) build_tile_lists(tid < U ? uid_l[tid] : 0u, tid < U ? start[tid] : 0u, tid < U ? start[tid + 1u] - start[tid] : 0u, P, tiles, tile_tot);
 }
 
 // ---- the same sort by many workgroups, for large chunks: spans of kGroupSpan tokens, three launches
@@ -1129,7 +1129,7 @@ __global__ __launch_bounds__(1024) void group_plan_kernel(GroupScratch gs, uint3
     if (tid < U) { start[tid] = my_start; expert_start[tid] = my_start; gs.expert_base[uid_l[tid]] = my_start; }
     if (tid == 0u) { start[U] = all; expert_start[U] = all; n_unique[0] = U; }
     __syncthreads();
-    if (tiles.tile_group) build_tile_lists(U, tid < U ? start[tid] : 0u, tid < U ? start[tid + 1u] - start[tid] : 0u, P, tiles, tile_tot);
+    if (tiles.tile_expert) build_tile_lists(tid < U ? uid_l[tid] : 0u, tid < U ? start[tid] : 0u, tid < U ? start[tid + 1u] - start[tid] : 0u, P, tiles, tile_tot);
 }
 
 __global__ __launch_bounds__(256) void group_place_kernel(const uint32_t *ids, const float *weights, uint32_t ntok, uint32_t top_k, uint32_t top_k_magic,

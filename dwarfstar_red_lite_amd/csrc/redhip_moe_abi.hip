@@ -115,7 +115,7 @@ struct Moe {
     bool shared_gu_ready = false;            // the router launch of this forward() has left the shared expert's gate / up products in `act`
     // batched path (ntok > 1): pairs grouped by expert
     uint32_t *uid = nullptr, *expert_start = nullptr, *pair_token = nullptr, *tok_pair = nullptr, *n_unique = nullptr;
-    uint32_t *tile_group = nullptr, *tile_pair0 = nullptr, *tile_n = nullptr, *n_tiles = nullptr;      // prefill tiles
+    uint32_t *tile_expert = nullptr, *tile_pair0 = nullptr, *tile_n = nullptr, *n_tiles = nullptr;      // prefill tiles
     void *group_mem = nullptr;               // handles that take more than 512 tokens: scratch of the pair sort by many workgroups
     GroupScratch group_scratch{};
     const GroupScratch *group_scratch_ptr() const { return group_mem ? &group_scratch : nullptr; }
@@ -306,13 +306,13 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
         const bool dense_shared = tile_path && m->mixed && Ld.dense_gu && m->side;
         if (dense_shared && !fork_shared_dense(m, Ld, x, ntok, s)) return 0;
         // the pair sort also writes the tile lists of the tile kernels that follow (all-IQ2_XXS layers: with the shared expert's tiles)
-        const TileLists tl{m->tile_group, m->tile_pair0, m->tile_n, m->n_tiles, prefill_tile_bound(ntok, c.top_k, c.n_expert), m->fused ? ntok : 0u};
+        const TileLists tl{m->tile_expert, m->tile_pair0, m->tile_n, m->n_tiles, prefill_tile_bound(ntok, c.top_k, c.n_expert), m->fused ? ntok : 0u};
         if (!grouped) {
             prof_set_stage(ST_GROUP);
             HIP_OK(launch_group_pairs(ids, weights, ntok, c.top_k, c.n_expert, m->uid, m->expert_start, m->pair_token, m->pair_weight,
                                       m->tok_pair, m->n_unique, s, tile_path ? &tl : nullptr, m->group_scratch_ptr()), "grouping launch");
         } else if (tile_path)
-            HIP_OK(launch_build_tiles(m->expert_start, m->n_unique, P, tl, s), "tile list launch");
+            HIP_OK(launch_build_tiles(m->uid, m->expert_start, m->n_unique, P, tl, s), "tile list launch");
         if (m->small_batch(ntok, true) && grouped && !select_here) {     // routing sorted (with its pass list) by the prep or the selection launch: expert slices per pass
             const Layer &L = m->layers[layer];
             HIP_OK(launch_batch_slices(L.packed, m->packed_stride, L.down_cm, m->down_cm_stride(), L.shared_packed, L.shared_down_cm, m->pass_list, m->n_pass,
@@ -329,7 +329,7 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
             const uint8_t *plain = m->fused ? L.packed : L.experts;
             const StagedMatrices gu{m->gu_type, tiles_gu ? RowLayout::tiled : rows, tiles_gu ? L.tiled : plain, tiles_gu ? L.shared_tiled : L.shared_packed,
                                     tiles_gu ? m->tiled_stride() : m->fused ? m->packed_stride : m->expert_stride, tiles_gu ? m->pk_gate_bytes : m->gate_bytes, m->gu_grid};
-            const StagedChunk chunk{m->uid, m->pair_token, m->n_unique, tl, ntok, c.top_k, c.n_expert};
+            const StagedChunk chunk{m->pair_token, tl, ntok, c.top_k, c.n_expert};
             if (!gu.experts) { moe_err("internal: no rows for the tile kernels (layer %u)", layer); return 0; }
             HIP_OK(launch_staged_gateup(gu, chunk, m->xh, m->xl, m->xexp, m->act, c.hidden, c.ffn, s), "gate/up tile launch");
             const uint8_t *dn_rows = m->fused ? (tiles_dn ? L.tiled : L.packed) + 2u * m->gate_bytes : tiles_dn ? L.tiled_down : L.experts ? L.experts + 2u * m->gate_bytes : nullptr;
@@ -599,7 +599,7 @@ redhip_moe_t redhip_moe_create(const redhip_moe_config *cfg) {
         m->tmp = reinterpret_cast<float *>(w); w += align256(4u * T * c.top_k * c.hidden);
         m->sh_tmp = reinterpret_cast<float *>(w); w += align256(4u * T * c.hidden);
         const size_t tw = align256(12u * (size_t)prefill_tile_bound(c.max_tokens, c.top_k, c.n_expert));
-        m->tile_group = reinterpret_cast<uint32_t *>(w); w += tw;
+        m->tile_expert = reinterpret_cast<uint32_t *>(w); w += tw;
         m->tile_pair0 = reinterpret_cast<uint32_t *>(w); w += tw;
         m->tile_n = reinterpret_cast<uint32_t *>(w); w += tw;
         m->n_tiles = reinterpret_cast<uint32_t *>(w);

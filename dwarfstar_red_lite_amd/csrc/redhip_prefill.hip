@@ -9,16 +9,16 @@ namespace redhip {
 // ---------------------------------------------------------------- tile list
 
 // the tile lists (TileLists) as a launch of their own, for callers whose pair sort did not write them
-__global__ __launch_bounds__(1024) void build_tiles_kernel(const uint32_t *expert_start, const uint32_t *n_unique, uint32_t P, TileLists tl) {
+__global__ __launch_bounds__(1024) void build_tiles_kernel(const uint32_t *uid, const uint32_t *expert_start, const uint32_t *n_unique, uint32_t P, TileLists tl) {
     __shared__ uint32_t wave_total[3][16];
     const uint32_t tid = threadIdx.x, U = n_unique[0];
-    uint32_t p0 = 0u, n = 0u;
-    if (tid < U) { p0 = expert_start[tid]; n = expert_start[tid + 1u] - p0; }
-    build_tile_lists(U, p0, n, P, tl, wave_total);
+    uint32_t e = 0u, p0 = 0u, n = 0u;
+    if (tid < U) { e = uid[tid]; p0 = expert_start[tid]; n = expert_start[tid + 1u] - p0; }
+    build_tile_lists(e, p0, n, P, tl, wave_total);
 }
 
-hipError_t launch_build_tiles(const uint32_t *expert_start, const uint32_t *n_unique, uint32_t n_pairs, const TileLists &tl, hipStream_t s) {
-    REDHIP_LAUNCH(build_tiles_kernel, dim3(1), dim3(1024), 0, s, expert_start, n_unique, n_pairs, tl);
+hipError_t launch_build_tiles(const uint32_t *uid, const uint32_t *expert_start, const uint32_t *n_unique, uint32_t n_pairs, const TileLists &tl, hipStream_t s) {
+    REDHIP_LAUNCH(build_tiles_kernel, dim3(1), dim3(1024), 0, s, uid, expert_start, n_unique, n_pairs, tl);
     return hipGetLastError();
 }
 

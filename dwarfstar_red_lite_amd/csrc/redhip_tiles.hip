@@ -70,16 +70,20 @@ __device__ __forceinline__ uint32_t two_halves(float lo, float hi) {
     return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
 }
 
-template <int SRC, uint32_t T>          // by all T threads of the workgroup
+template <int SRC, uint32_t T>          // by T threads
 __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *signs, uint32_t tid, const int8_t *grid) {
     if constexpr (fmt<SRC>() == F_XXS) {
-        for (uint32_t e = tid; e < 16u * 256u; e += T) {
-            const uint64_t ge = redhip_iq2xxs_grid[e >> 4];
-            const float f = (float)(2u * (e & 15u) + 1u);
-            uint32_t w4[4];
+        for (uint32_t e4 = tid; e4 < 4u * 256u; e4 += T) {
+            const uint64_t ge = redhip_iq2xxs_grid[e4 >> 2];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) w4[i] = two_halves(f * (float)((uint32_t)(ge >> (16 * i)) & 255u), f * (float)((uint32_t)(ge >> (16 * i + 8)) & 255u));
-            *reinterpret_cast<uint4 *>(entries + (size_t)e * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+            for (uint32_t k = 0; k < 4u; ++k) {
+                const uint32_t e = 4u * e4 + k;
+                const float f = (float)(2u * (e & 15u) + 1u);
+                uint32_t w4[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w4[i] = two_halves(f * (float)((uint32_t)(ge >> (16 * i)) & 255u), f * (float)((uint32_t)(ge >> (16 * i + 8)) & 255u));
+                *reinterpret_cast<uint4 *>(entries + (size_t)e * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+            }
         }
     } else if constexpr (fmt<SRC>() == F_XS || fmt<SRC>() == F_M) {
         constexpr uint32_t kCopies = fmt<SRC>() == F_XS ? 8u : 2u, kEntries = kEntryBytes / (16u * kCopies);
@@ -239,10 +243,10 @@ __device__ __forceinline__ half8_t finish_entry(const Entry &e, half2_t f) {
 }
 
 struct StagedArgs {
-    const uint8_t *experts, *shared;       // first matrix of expert uid[u] at experts + uid[u] * stride; of group n_unique[0] at `shared`
+    const uint8_t *experts, *shared;       // first matrix of expert e at experts + e * stride, of the shared expert at `shared`
     uint64_t stride, mat_step;             // mat_step: gate/up, distance of the up matrix
     uint64_t d_off;                        // not raw rows: the block scales behind the quarters of a matrix (tile-major IQ2_XS: the scale bytes behind them)
-    const uint32_t *uid, *pair_token, *n_unique, *tile_group, *tile_pair0, *tile_n, *n_tiles;
+    const uint32_t *pair_token, *tile_expert, *tile_pair0, *tile_n, *n_tiles;
     const _Float16 *xh, *xl;               // gate/up in: [ntok][K]
     const int *xexp;                       // [ntok]
     float *act;                            // [P + shared tokens][rows]: gate/up out; down in as [..][K]
@@ -261,24 +265,23 @@ __device__ __forceinline__ void wave_lds_barrier() {
 // (which the activations need) across the loop.
 __device__ __forceinline__ uint32_t each_trip(uint32_t v) { asm volatile("" : "+v"(v)); return v; }
 
-// What the units of a workgroup need to know of their tiles, fetched once at the kernel's head (a tile's entry, its expert's address, its
-// pairs' tokens and their exponents are four dependent trips to memory); tiles beyond the first kTileInfos are looked up when they begin.
+// What the units of a workgroup need to know of their tiles (gate/up: the pairs' tokens among it), fetched at the kernel's head by its
+// first wave while the others build the tables; tiles beyond the first kTileInfos are looked up when they begin.
 constexpr uint32_t kTileInfos = 32u;
 struct TileInfo { uint64_t mat; uint32_t p0, n; };      // mat: distance of the expert's first matrix from StagedArgs::experts
-struct PairInfo { uint32_t tok; float scale; };      // gate/up: token of a pair, its power of two (with the d / 8 of the IQ2 formats)
 
 // units u0 .. u1 - 1 (unit = tile * units per tile + unit of the tile) of a tile list; SETS sets of 16 pairs per tile
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
-__device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t *tile_group, const uint32_t *tile_pair0, const uint32_t *tile_n, uint32_t u0,
-                                             uint32_t u1, float *part, TileInfo *tiles, PairInfo *pairs, uint8_t *entries, uint32_t *signs, const LaneTables &lt) {
+__device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t *tile_expert, const uint32_t *tile_pair0, const uint32_t *tile_n, uint32_t u0,
+                                             uint32_t u1, float *part, TileInfo *tiles, uint32_t *tokens, uint8_t *entries, uint32_t *signs, const LaneTables &lt) {
     constexpr uint32_t NRT = staged_nrt(KP), WV = KP * NRT, T = staged_threads(SETS, KP), M = SETS == 1 ? 1u : 2u;      // M: halves per wave
     constexpr uint32_t K = 256u * KP, seg_rows = 16u * NRT, tile_bytes = 16u * KP * src_block<SRC>();
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), w8 = wave % WV, m_first = SETS == 1 ? wave / WV : 0u, kc = w8 % KP, rt = w8 / KP;
-    const uint32_t upt = a.rows / ((DOWN ? 2u : 1u) * seg_rows), U = a.n_unique[0];
+    const uint32_t upt = a.rows / ((DOWN ? 2u : 1u) * seg_rows);
     const auto matrix_of = [&](uint32_t tile) {
-        const uint32_t u = tile_group[tile];
-        return u == U ? (uint64_t)(a.shared - a.experts) : (uint64_t)a.uid[u] * a.stride;
+        const uint32_t e = tile_expert[tile];
+        return e == kSharedTile ? (uint64_t)(a.shared - a.experts) : (uint64_t)e * a.stride;
     };
     // the lane's quarters of a unit, and what their d are made from
     struct Carried { Quarter v[M]; uint2 d[M]; };
@@ -291,22 +294,16 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
         }
     };
     const uint32_t tile0 = u0 / upt, n_info = (u1 - 1u) / upt + 1u - tile0 < kTileInfos ? (u1 - 1u) / upt + 1u - tile0 : kTileInfos;
-    const auto pair_info = [&](uint32_t p0, uint32_t n, uint32_t i) {          // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
-        const uint32_t p = i < n ? p0 + i : p0, tok = p < a.P ? a.pair_token[p] : p - a.P;
-        return PairInfo{tok, format_scale<SRC>() * exp2i(a.xexp[tok])};
+    const auto token_of = [&](uint32_t p0, uint32_t n, uint32_t i) {           // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
+        const uint32_t p = i < n ? p0 + i : p0;
+        return p < a.P ? a.pair_token[p] : p - a.P;
     };
-    {
-        TileInfo ti{};
-        PairInfo pi{};
-        const uint32_t pt = tid / (16u * SETS), pk = tid % (16u * SETS);      // (T >= 384 threads serve at least 12 tiles per round)
-        if (tid < n_info) ti = TileInfo{matrix_of(tile0 + tid), tile_pair0[tile0 + tid], tile_n[tile0 + tid]};
-        if (!DOWN && pt < n_info) pi = pair_info(tile_pair0[tile0 + pt], tile_n[tile0 + pt], pk);
-        build_staged_tables<SRC, T>(entries, signs, tid, a.grid);
-        if (tid < n_info) tiles[tid] = ti;
-        if (!DOWN && pt < n_info) pairs[tid] = pi;
+    if (tid < 64u) {
+        if (tid < n_info) tiles[tid] = TileInfo{matrix_of(tile0 + tid), tile_pair0[tile0 + tid], tile_n[tile0 + tid]};
         if constexpr (!DOWN)
-            for (uint32_t k = tid + T; k < n_info * 16u * SETS; k += T) pairs[k] = pair_info(tile_pair0[tile0 + k / (16u * SETS)], tile_n[tile0 + k / (16u * SETS)], k % (16u * SETS));
-    }
+            for (uint32_t k = tid; k < n_info * 16u * SETS; k += 64u) tokens[k] = token_of(tile_pair0[tile0 + k / (16u * SETS)], tile_n[tile0 + k / (16u * SETS)], k % (16u * SETS));
+    } else
+        build_staged_tables<SRC, T - 64u>(entries, signs, tid - 64u, a.grid);
     __syncthreads();
     const auto uniform64 = [](uint64_t v) {
         return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
@@ -325,9 +322,9 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
             const uint32_t l = each_trip(lane), lq = l >> 4, i = 16u * s + (l & 15u);
             float scale;
             if constexpr (!DOWN) {
-                const PairInfo pi = tile - tile0 < kTileInfos ? pairs[(tile - tile0) * 16u * SETS + i] : pair_info(p0, n, i);
-                scale = pi.scale;
-                const uint64_t base = (uint64_t)pi.tok * K + 256u * kc;
+                const uint32_t tok = tile - tile0 < kTileInfos ? tokens[(tile - tile0) * 16u * SETS + i] : token_of(p0, n, i);
+                scale = format_scale<SRC>() * exp2i(a.xexp[tok]);
+                const uint64_t base = (uint64_t)tok * K + 256u * kc;
                 const _Float16 *hp = a.xh + base, *lp = a.xl + base;
 #pragma unroll
                 for (uint32_t g = 0; g < 8u; ++g) {
@@ -542,19 +539,20 @@ __global__ __launch_bounds__(staged_threads(SETS, KP)) void staged_tiles_kernel(
     __shared__ __attribute__((aligned(16))) uint8_t entries[kEntryBytes];   // static: table reads take immediate offsets
     __shared__ __attribute__((aligned(16))) uint32_t signs[sign_bytes<SRC>() / 4u + 4u];
     __shared__ __attribute__((aligned(16))) float part[4u * KP * staged_nrt(KP) * 2u * 256u];
-    const bool few = a.n_tiles[1] < kFewWide;
+    const uint32_t n0 = a.n_tiles[0], n1 = a.n_tiles[1], n2 = a.n_tiles[2];      // (one trip)
+    const bool few = n1 < kFewWide;
     if (SETS == 2 && few) return;
     const uint32_t tid = threadIdx.x, l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
-    const uint32_t units = a.n_tiles[l] * (a.rows / ((DOWN ? 32u : 16u) * staged_nrt(KP)));
+    const uint32_t units = (SETS == 2 ? n1 : few ? n0 : n2) * (a.rows / ((DOWN ? 32u : 16u) * staged_nrt(KP)));
     // workgroups are dealt round-robin over the eight XCDs: neighbouring runs (which share tiles) go to one XCD's L2
     const uint32_t G = gridDim.x, at = G % 8u == 0u ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
     const uint32_t u0 = (uint32_t)((uint64_t)at * units / G), u1 = (uint32_t)((uint64_t)(at + 1u) * units / G);
     if (u0 >= u1) return;
     __shared__ TileInfo tiles[kTileInfos];
-    __shared__ PairInfo pairs[DOWN ? 1u : kTileInfos * 16u * SETS];
+    __shared__ uint32_t tokens[DOWN ? 1u : kTileInfos * 16u * SETS];
     const LaneTables lt{entries + (fmt<SRC>() == F_XS ? (tid & 7u) * 16u : fmt<SRC>() == F_M ? (tid & 1u) * 16u : 0u),
                         reinterpret_cast<const uint8_t *>(signs) + (is_iq3<SRC>() ? (tid & 3u) * 4u : fmt<SRC>() == F_M ? 0u : (tid & 15u) * 4u)};
-    staged_units<SRC, DOWN, SETS, KP>(a, a.tile_group + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, part, tiles, pairs, entries, signs, lt);
+    staged_units<SRC, DOWN, SETS, KP>(a, a.tile_expert + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, part, tiles, tokens, entries, signs, lt);
 }
 
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
@@ -596,8 +594,8 @@ StagedArgs staged_args(const StagedMatrices &m, const StagedChunk &c, uint32_t K
     a.stride = m.stride;
     a.mat_step = m.up_delta;
     a.d_off = src == S_TILED_IQ3 ? (uint64_t)rows * (K / 32u) * 16u : (uint64_t)rows * (K / 32u) * 8u;
-    a.uid = c.uid; a.pair_token = c.pair_token; a.n_unique = c.n_unique;
-    a.tile_group = c.tl.tile_group; a.tile_pair0 = c.tl.tile_pair0; a.tile_n = c.tl.tile_n; a.n_tiles = c.tl.n_tiles;
+    a.pair_token = c.pair_token;
+    a.tile_expert = c.tl.tile_expert; a.tile_pair0 = c.tl.tile_pair0; a.tile_n = c.tl.tile_n; a.n_tiles = c.tl.n_tiles;
     a.list_stride = c.tl.list_stride;
     a.grid = m.grid;
     a.rows = rows;

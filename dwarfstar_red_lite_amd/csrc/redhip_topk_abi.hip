@@ -383,7 +383,7 @@ bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const PairExperts &ex, bool
     int *xexp = reinterpret_cast<int *>(w); w += x_exp;
     float *gate_unused = reinterpret_cast<float *>(w); w += x_exp;
     float *act = reinterpret_cast<float *>(w); w += a_bytes;
-    uint32_t *tile_group = reinterpret_cast<uint32_t *>(w); w += tl;
+    uint32_t *tile_expert = reinterpret_cast<uint32_t *>(w); w += tl;
     uint32_t *tile_pair0 = reinterpret_cast<uint32_t *>(w); w += tl;
     uint32_t *tile_n = reinterpret_cast<uint32_t *>(w); w += tl;
     uint32_t *n_tiles = reinterpret_cast<uint32_t *>(w);
@@ -393,8 +393,8 @@ bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const PairExperts &ex, bool
     float *tmp = static_cast<float *>(p->tmp_b.p);
     // (the split kernel also forms a gate logit per row from a second vector: x itself stands in, the result is not used)
     hipError_t e = launch_prep(x, x, (uint32_t)rows, hidden, xh, xl, xexp, gate_unused, s, nullptr, nullptr);
-    const TileLists lists{tile_group, tile_pair0, tile_n, n_tiles, bound, 0u};
-    if (e == hipSuccess) e = launch_build_tiles(d_start, d_unique, n_pairs, lists, s);
+    const TileLists lists{tile_expert, tile_pair0, tile_n, n_tiles, bound, 0u};
+    if (e == hipSuccess) e = launch_build_tiles(d_uid, d_start, d_unique, n_pairs, lists, s);
     uint32_t wide = 0u;
     for (uint32_t i = 0; i < n_expert; ++i) {
         const uint32_t m = expert_start[i + 1u] - expert_start[i];
@@ -403,7 +403,7 @@ bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const PairExperts &ex, bool
     const uint32_t gu = word_gate_up(type_word), dn = word_down(type_word);
     const RowLayout lay = copies ? RowLayout::tiled : RowLayout::raw;
     const uint8_t *tiles = ex.gate + p->fs.tile_off;
-    const StagedChunk chunk{d_uid, d_pair_token, d_unique, lists, ntok, top_k, n_expert, wide};
+    const StagedChunk chunk{d_pair_token, lists, ntok, top_k, n_expert, wide};
     const StagedMatrices gate_up{gu, lay, copies ? tiles : ex.gate, nullptr, ex.stride, copies ? p->fs.gate_copy : ex.up_delta, caller_grid_device(gu)};
     const StagedMatrices down{dn, lay, copies ? tiles + 2u * p->fs.gate_copy : ex.down, nullptr, ex.down_stride, 0u, caller_grid_device(dn)};
     if (e == hipSuccess) e = launch_staged_gateup(gate_up, chunk, xh, xl, xexp, act, hidden, ffn, s);

@@ -9,7 +9,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libredmetal_hip.so")
-SOURCES = ["redhip_kernels.hip", "redhip_fused.hip", "redhip_prefill.hip", "redhip_tiles.hip", "redhip_pool_abi.hip", "redhip_moe_abi.hip",
+SOURCES = ["redhip_kernels.hip", "redhip_fused.hip", "redhip_prefill.hip", "redhip_tiles.hip", "redhip_token.hip", "redhip_pool_abi.hip", "redhip_moe_abi.hip",
            "redhip_gguf.hip", "redhip_profile.hip", "redhip_topk_abi.hip"]
 # -packed-fp32-ops off: v_pk_*_f32 forms are not used on this pool of machines
 # -amdgpu-kernarg-preload-count: the leading scalar / pointer arguments of a kernel (up to 14 dwords) are handed to every wave in

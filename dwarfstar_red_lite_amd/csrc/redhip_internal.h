@@ -117,6 +117,15 @@ struct ExpertSet {               // where the experts of one layer live (raw GGU
                                        // reads its expert at table[i]; base, stride and the ids / uid arrays are not used
 };
 
+// One token on raw rows (redhip_token.hip), the experts of ex in slot order: the activations of n_slot experts (from x_split on x1, when
+// given, is read), and rows row_start .. of the weighted sum of their down products (weights == nullptr: one expert, weight 1), with a tail
+// the layer's last step. Callers ask token_rows_supported first.
+struct TokenTail { const float *resid, *shared, *scalar; float *x, *layer_out; };
+bool token_rows_supported(uint32_t gate_up_type, uint32_t down_type, uint32_t top_k, uint32_t hidden, uint32_t ffn, const float *x, const float *x1);
+hipError_t launch_token_gateup(const ExpertSet &ex, uint32_t n_slot, uint32_t hidden, uint32_t ffn, const float *x, const float *x1, uint32_t x_split, float *act, hipStream_t s);
+hipError_t launch_token_down(const ExpertSet &ex, const float *weights, uint32_t top_k, uint32_t ffn, uint32_t row_start, uint32_t row_count, const float *act, float *out,
+                             const TokenTail *tail, hipStream_t s);
+
 // act[slot][r] = SiLU(gate_e[r] . x) * (up_e[r] . x) for slot < n_slot, e = ids ? ids[slot] : slot
 // With x1, slots from x_split on read x1 instead of x (two activation vectors in one launch).
 hipError_t launch_moe_gateup(const ExpertSet &ex, const uint32_t *ids, uint32_t n_slot, uint32_t hidden, uint32_t ffn,

@@ -14,7 +14,8 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 // power-of-two pre-scale: largest |v| lands in [2^13, 2^14)
 __device__ __forceinline__ int prescale_exp(float amax) {
     if (!(amax > 0.0f) || isinf(amax) || isnan(amax)) return 0;
-    return (int)((__float_as_uint(amax) >> 23) & 255u) - 127 - 13;
+    const int e = (int)((__float_as_uint(amax) >> 23) & 255u) - 127 - 13;
+    return e < -126 ? -126 : e;                     // (its inverse has to be a float)
 }
 __device__ __forceinline__ float exp2i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }   // e in [-126, 127]
 

@@ -1,0 +1,275 @@
+// Rows of the expert formats, decoded a quarter block (64 of 256 columns) per lane into eight signed, scaled fp16 weights at a time: what
+// the MFMA kernels on tiles of tokens and on one token share.
+#pragma once
+#include "redhip_mfma.h"
+
+namespace redhip {
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+union H8 { uint4 u; half8_t v; half2_t p[4]; _Float16 e[8]; };
+
+// row sources: format (low half, what the decode goes by) and layout
+enum : int { F_XXS = 0, F_XS = 1, F_M = 2, F_IQ3 = 3, F_IQ3_WORDS = 4, L_RAW = 0, L_ROWS = 8, L_TILED = 16 };
+enum : int { S_XXS = F_XXS, S_XS = F_XS, S_M = F_M, S_IQ3 = F_IQ3, S_ROWS_XXS = F_XXS | L_ROWS, S_TILED_XXS = F_XXS | L_TILED, S_TILED_XS = F_XS | L_TILED,
+             S_TILED_M = F_M | L_TILED, S_TILED_IQ3 = F_IQ3_WORDS | L_TILED };
+// a kernel on one token uses every table entry about once: small tables, quickly built
+enum : int { SMALL_TABLES = 32 };
+template <int SRC> constexpr bool small_tables() { return (SRC & SMALL_TABLES) != 0; }
+template <int SRC> constexpr int fmt() { return SRC & 7; }
+template <int SRC> constexpr int layout() { return SRC & 24; }
+// bytes per 256 columns of a row: raw blocks; the quarters of the other layouts (their block scales lie apart)
+template <int SRC> constexpr uint32_t src_block() {
+    return layout<SRC>() != L_RAW ? (fmt<SRC>() == F_IQ3_WORDS ? 128u : 64u) : fmt<SRC>() == F_XXS ? 66u : fmt<SRC>() == F_XS ? 74u : fmt<SRC>() == F_M ? 56u : 110u;
+}
+template <int SRC> constexpr float format_scale() { return fmt<SRC>() == F_XXS || fmt<SRC>() == F_XS ? 0.125f : 1.0f; }      // the d / 8 of the IQ2 formats
+// first of the eight columns that lane quarter q multiplies in step s of a block: its own quarter, in order - or, where the lane reads entry q
+// of every group (tile-major IQ3_S words), that entry
+template <int SRC> __device__ __forceinline__ uint32_t step_column(uint32_t s, uint32_t q) { return fmt<SRC>() == F_IQ3_WORDS ? 128u * (s >> 2) + 32u * (s & 3u) + 8u * q : 64u * q + 8u * s; }
+
+// Decode tables in LDS.
+//   IQ2_XXS: the eight fp16 magnitudes of every grid entry times every group scale 2 s + 1 (64 KB, exact), at entry * 256 + s * 16: the address is
+//   the entry's byte over the top byte of the group's second word, one byte permute and one mask; IQ3_S likewise (four magnitudes, by scale)
+//   IQ2_XS: the fp16 codebook eight times, lane l reading copy l % 8 - a wave's 16-byte reads then hit every bank evenly (random entries of
+//   one copy: 2.6 times the cycles); IQ1_M: its fp16 codebook twice
+//   Small tables (32 KB, IQ3_S 16): IQ2_XXS and IQ3_S without the scales, eight and four copies; IQ2_XS four copies, IQ1_M one
+//   signs: bit 15 - i / 31 - i of the word of a sign field = signs of weights 2i and 2i + 1, so a pair's signs are one shift and one and-or;
+//   replicated so that the reads are (nearly) free of conflicts. (Sign masks as 16-byte entries save three shifts per eight weights and cost
+//   a second conflicting 16-byte read: LDS, the tighter of the two pipes, loses more.)
+template <int SRC> constexpr bool is_iq3() { return fmt<SRC>() == F_IQ3 || fmt<SRC>() == F_IQ3_WORDS; }
+template <int SRC> constexpr uint32_t sign_copies() { return fmt<SRC>() == F_M ? 0u : (is_iq3<SRC>() ? 4u : 16u) / (small_tables<SRC>() ? is_iq3<SRC>() ? 2u : 4u : 1u); }
+template <int SRC> constexpr uint32_t sign_shift() { return sign_copies<SRC>() == 16u ? 6u : sign_copies<SRC>() == 4u ? 4u : 3u; }
+template <int SRC> constexpr uint32_t sign_bytes() { return (is_iq3<SRC>() ? 256u : 128u) * sign_copies<SRC>() * 4u; }
+constexpr uint32_t kEntryBytes = 65536u;
+
+__device__ __forceinline__ uint32_t two_halves(float lo, float hi) {
+    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
+}
+
+template <int SRC, uint32_t T>          // by T threads
+__device__ __forceinline__ void build_signs(uint32_t *signs, uint32_t tid) {
+    if constexpr (fmt<SRC>() != F_M) {
+        constexpr uint32_t R = sign_copies<SRC>(), N = sign_bytes<SRC>() / 4u;
+        for (uint32_t i = tid; i < N; i += T) {
+            const uint32_t s = i / R, s8 = is_iq3<SRC>() ? s : s | ((__popc(s) & 1u) << 7);
+            uint32_t w = 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) w |= (((s8 >> (2u * k)) & 1u) << (15u - k)) | (((s8 >> (2u * k + 1u)) & 1u) << (31u - k));
+            signs[i] = w;
+        }
+    }
+}
+
+template <int SRC, uint32_t T>
+__device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *signs, uint32_t tid, const int8_t *grid) {
+    if constexpr (fmt<SRC>() == F_XXS) {
+        for (uint32_t e4 = tid; e4 < 4u * 256u; e4 += T) {
+            const uint64_t ge = redhip_iq2xxs_grid[e4 >> 2];
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) {
+                const uint32_t e = 4u * e4 + k;
+                const float f = (float)(2u * (e & 15u) + 1u);
+                uint32_t w4[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w4[i] = two_halves(f * (float)((uint32_t)(ge >> (16 * i)) & 255u), f * (float)((uint32_t)(ge >> (16 * i + 8)) & 255u));
+                *reinterpret_cast<uint4 *>(entries + (size_t)e * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+            }
+        }
+    } else if constexpr (fmt<SRC>() == F_XS || fmt<SRC>() == F_M) {
+        constexpr uint32_t kCopies = fmt<SRC>() == F_XS ? 8u : 2u, kEntries = kEntryBytes / (16u * kCopies);
+        for (uint32_t e = tid; e < kEntries; e += T) {
+            const uint64_t ge = reinterpret_cast<const uint64_t *>(grid)[e];
+            uint32_t w4[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w4[i] = two_halves((float)(int8_t)(ge >> (16 * i)), (float)(int8_t)(ge >> (16 * i + 8)));
+            for (uint32_t c = 0; c < kCopies; ++c) *reinterpret_cast<uint4 *>(entries + ((size_t)e * kCopies + c) * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+        }
+    } else {
+        for (uint32_t e = tid; e < 16u * 512u; e += T) {
+            const uint32_t gw = redhip_iq3s_grid[e & 511u];
+            const float f = (float)(1u + 2u * (e >> 9));
+            *reinterpret_cast<uint2 *>(entries + (size_t)e * 8u) =
+                make_uint2(two_halves(f * (float)(gw & 255u), f * (float)((gw >> 8) & 255u)), two_halves(f * (float)((gw >> 16) & 255u), f * (float)(gw >> 24)));
+        }
+    }
+    build_signs<SRC, T>(signs, tid);
+}
+
+// The small tables, by T threads in two parts: a thread's codebook entries are requested (before the rows, which the second part must not
+// wait for), then written. Tables with copies are written by two threads per entry, half of the copies each.
+template <int SRC> constexpr uint32_t codebook_entries() { return fmt<SRC>() == F_XXS ? 256u : fmt<SRC>() == F_M ? 2048u : 512u; }
+template <int SRC> constexpr uint32_t small_copies() { return fmt<SRC>() == F_XXS ? 8u : fmt<SRC>() == F_M ? 1u : 4u; }
+template <int SRC> constexpr uint32_t entry_shift() { return !small_tables<SRC>() ? (fmt<SRC>() == F_M ? 5u : 7u) : fmt<SRC>() == F_XXS ? 7u : fmt<SRC>() == F_XS ? 6u : fmt<SRC>() == F_M ? 4u : 5u; }
+template <int SRC> constexpr uint32_t small_entry_bytes() { return codebook_entries<SRC>() << entry_shift<SRC>(); }
+template <int SRC, uint32_t T> struct SmallSeeds {
+    static constexpr uint32_t kHalves = small_copies<SRC>() > 1u ? 2u : 1u, kItems = codebook_entries<SRC>() * kHalves, N = (kItems + T - 1u) / T;
+    uint64_t e[N];
+    __device__ __forceinline__ void request(uint32_t tid, const int8_t *grid) {
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n) {
+            const uint32_t i = (min(tid + n * T, kItems - 1u)) / kHalves;
+            if constexpr (is_iq3<SRC>()) e[n] = redhip_iq3s_grid[i];
+            else if constexpr (fmt<SRC>() == F_XXS) e[n] = redhip_iq2xxs_grid[i];
+            else e[n] = reinterpret_cast<const uint64_t *>(grid)[i];
+        }
+    }
+    __device__ __forceinline__ void store(uint8_t *entries, uint32_t *signs, uint32_t tid) const {
+        constexpr uint32_t kCopies = small_copies<SRC>(), kMine = kCopies / kHalves;
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n) {
+            const uint32_t i = min(tid + n * T, kItems - 1u), first = ((i / kHalves) * kCopies + (i % kHalves) * kMine);      // (surplus threads repeat the last)
+            if constexpr (is_iq3<SRC>()) {
+                const uint32_t g = (uint32_t)e[n];
+                const uint2 v = make_uint2(two_halves((float)(g & 255u), (float)((g >> 8) & 255u)), two_halves((float)((g >> 16) & 255u), (float)(g >> 24)));
+#pragma unroll
+                for (uint32_t c = 0; c < kMine; ++c) *reinterpret_cast<uint2 *>(entries + (size_t)(first + c) * 8u) = v;
+            } else {
+                uint32_t w4[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if constexpr (fmt<SRC>() == F_XXS) w4[k] = two_halves((float)((uint32_t)(e[n] >> (16 * k)) & 255u), (float)((uint32_t)(e[n] >> (16 * k + 8)) & 255u));
+                    else w4[k] = two_halves((float)(int8_t)(e[n] >> (16 * k)), (float)(int8_t)(e[n] >> (16 * k + 8)));
+                }
+#pragma unroll
+                for (uint32_t c = 0; c < kMine; ++c) *reinterpret_cast<uint4 *>(entries + (size_t)(first + c) * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+            }
+        }
+        build_signs<SRC, T>(signs, tid);
+    }
+};
+
+// fields of a quarter block (two 32-column groups) of a row: what a lane multiplies
+//   IQ2_XXS  a: the two groups' words                     IQ2_XS  a: eight 16-bit entries, c: two scale bytes
+//   IQ1_M    a: 8 index bytes | 4 bytes of nibbles | scale word     IQ3_S   a: 16 index bytes, b: 8 sign bytes, c: two qh bytes | scale byte << 16
+//   tile-major IQ3_S   a, b: entry q of the first and the last four groups of the block, a word each
+struct Quarter { uint4 a, b; uint32_t c; };
+
+template <class T> __device__ __forceinline__ T load_a2(const uint8_t *p) { T v; __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), sizeof(T)); return v; }
+
+// Quarter q of block kc of row r of a tile of 16 rows, and what its d is made from. tile: the tile's rows (raw and packed rows 16 KP blocks,
+// tile-major its KP * 2 chunks of 16 rows), ds: its block scales, scs: tile-major IQ2_XS, its scale bytes.
+//   tile-major: chunk c (128 columns) of row r at (c * 16 + r) * 32 (IQ3_S words * 64), scale of block b at (b * 16 + r) * 2, the scale
+//   bytes of a chunk at (c * 16 + r) * 4: a wave's load is two runs of 512 bytes
+template <int SRC, uint32_t KP>
+__device__ __forceinline__ void load_quarter(const uint8_t *tile, const uint8_t *ds, const uint8_t *scs, uint32_t r, uint32_t kc, uint32_t q, Quarter &v, uint2 &d) {
+    const uint32_t block = r * KP + kc;
+    if constexpr (layout<SRC>() == L_TILED) {
+        const uint32_t chunk = (2u * kc + (q >> 1)) * 16u + r;
+        if constexpr (fmt<SRC>() == F_IQ3_WORDS) {
+            v.a = *reinterpret_cast<const uint4 *>(tile + (32u * kc + r) * 64u + 16u * q);
+            v.b = *reinterpret_cast<const uint4 *>(tile + (32u * kc + 16u + r) * 64u + 16u * q);
+        } else if constexpr (fmt<SRC>() == F_M) {      // stream words: four index bytes | nibbles, two 3-bit scales from bit 16 on
+            const uint4 w = *reinterpret_cast<const uint4 *>(tile + chunk * 32u + 16u * (q & 1u));
+            v.a = make_uint4(w.x, w.z, (w.y & 0xffffu) | (w.w << 16), __builtin_amdgcn_ubfe(w.y, 16u, 6u) | (__builtin_amdgcn_ubfe(w.w, 16u, 6u) << 6));
+        } else
+            v.a = *reinterpret_cast<const uint4 *>(tile + chunk * 32u + 16u * (q & 1u));
+        if constexpr (fmt<SRC>() == F_XS) v.c = *reinterpret_cast<const uint16_t *>(scs + chunk * 4u + 2u * (q & 1u));
+        d.x = *reinterpret_cast<const uint16_t *>(ds + (kc * 16u + r) * 2u);
+    } else if constexpr (layout<SRC>() == L_ROWS) {
+        v.a = *reinterpret_cast<const uint4 *>(tile + block * 64u + 16u * q);
+        d.x = *reinterpret_cast<const uint16_t *>(ds + block * 2u);
+    } else {
+        const uint8_t *bp = tile + block * src_block<SRC>();
+        if constexpr (fmt<SRC>() == F_M && layout<SRC>() == L_RAW) {
+            const uint2 qs = load_a2<uint2>(bp + 8u * q);
+            v.a = make_uint4(qs.x, qs.y, load_a2<uint32_t>(bp + 32u + 4u * q), load_a2<uint16_t>(bp + 48u + 2u * q));
+            d = load_a2<uint2>(bp + 48u);
+        } else {
+            v.a = load_a2<uint4>(bp + 2u + 16u * q);
+            d.x = load_a2<uint16_t>(bp);
+        }
+        if constexpr (fmt<SRC>() == F_XS) v.c = load_a2<uint16_t>(bp + 66u + 2u * q);
+        if constexpr (fmt<SRC>() == F_IQ3) {
+            const uint2 sg = load_a2<uint2>(bp + 74u + 8u * q);
+            v.b.x = sg.x; v.b.y = sg.y;
+            v.c = load_a2<uint16_t>(bp + 66u + 2u * q) | ((uint32_t)bp[106u + q] << 16);
+        }
+    }
+}
+template <int SRC>
+__device__ __forceinline__ float quarter_d(uint2 d) {
+    if constexpr (fmt<SRC>() == F_M && layout<SRC>() == L_RAW) return scale_to_f32(((d.x >> 12) & 0x000fu) | ((d.x >> 24) & 0x00f0u) | ((d.y >> 4) & 0x0f00u) | ((d.y >> 16) & 0xf000u));
+    else return scale_to_f32(d.x);
+}
+
+// odd integer 2 s + 1 (s < 16) as two equal fp16 halves: 1024 + (2 s + 1) by integer arithmetic, minus 1024, exact
+__device__ __forceinline__ half2_t odd_splat(uint32_t s) {
+    const half2_t big = {(_Float16)1024.0f, (_Float16)1024.0f};
+    return __builtin_bit_cast(half2_t, __umul24(s, 0x20002u) + 0x64016401u) - big;
+}
+
+// lane constants of the tables: addresses of the lane's copy
+struct LaneTables { const uint8_t *entries; const uint8_t *signs; };
+
+// Table reads of step s (eight columns) of a quarter, then the arithmetic on what they return: the eight signed, scaled fp16 weights.
+// s is a constant after unrolling.
+struct Entry { uint4 m; uint32_t s; };
+__device__ __forceinline__ uint32_t word_of(const uint4 &v, uint32_t i) { return i == 0u ? v.x : i == 1u ? v.y : i == 2u ? v.z : v.w; }
+template <int SRC>
+__device__ __forceinline__ Entry fetch_entry(const Quarter &v, uint32_t s, const LaneTables &t) {
+    const uint32_t h = s >> 2, e = s & 3u;                 // group of the quarter, entry of the group
+    Entry r;
+    if constexpr (fmt<SRC>() == F_XXS) {
+        const uint32_t wa = h ? v.a.z : v.a.x, wb = h ? v.a.w : v.a.y;
+        // bytes 0 .. 3 of the permute's second operand are the entries, 7 the top byte of the first
+        if constexpr (small_tables<SRC>()) r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_ubfe(wa, 8u * e, 8u) << entry_shift<SRC>()));
+        else r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_perm(wb, wa, 0x0c0c0007u | (e << 8)) & 0xfff0u));
+        r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(wb, 7u * e, 7u) << sign_shift<SRC>()));
+    } else if constexpr (fmt<SRC>() == F_XS) {
+        const uint32_t w = word_of(v.a, 2u * h + (e >> 1)), o = 16u * (e & 1u);
+        r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_ubfe(w, o, 9u) << entry_shift<SRC>()));
+        r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(w, o + 9u, 7u) << sign_shift<SRC>()));
+    } else if constexpr (fmt<SRC>() == F_IQ3_WORDS) {
+        const uint32_t w = word_of(h ? v.b : v.a, e), scale = (w >> 14) & 0xf000u;      // nibble * 512 entries * 8 bytes
+        const uint2 ma = *reinterpret_cast<const uint2 *>(t.entries + (((w << 3) & 0xff8u) | scale));
+        const uint2 mb = *reinterpret_cast<const uint2 *>(t.entries + (((w >> 6) & 0xff8u) | scale));
+        r.m = make_uint4(ma.x, ma.y, mb.x, mb.y);
+        r.s = *reinterpret_cast<const uint32_t *>(t.signs + ((w >> 14) & 0xff0u));
+    } else if constexpr (fmt<SRC>() == F_M) {
+        r.s = __builtin_amdgcn_ubfe(v.a.z, 16u * h + 4u * e, 4u);
+        r.m = *reinterpret_cast<const uint4 *>(t.entries + ((__builtin_amdgcn_ubfe(h ? v.a.y : v.a.x, 8u * e, 8u) | ((r.s & 7u) << 8)) << entry_shift<SRC>()));
+    } else {
+        const uint32_t w = word_of(v.a, 2u * h + (e >> 1)), o = 16u * (e & 1u);
+        const uint32_t scale = h ? (v.c >> 8) & 0xf000u : (v.c >> 4) & 0xf000u;      // nibble * 512 entries * 8 bytes
+        const uint32_t ba = 8u * h + 2u * e, bb = ba + 1u;     // qh bits of the two entries -> bit 11
+        const uint32_t ha = (ba > 11u ? v.c >> (ba - 11u) : v.c << (11u - ba)) & 2048u, hb = (bb > 11u ? v.c >> (bb - 11u) : v.c << (11u - bb)) & 2048u;
+        uint32_t ia = (__builtin_amdgcn_ubfe(w, o, 8u) << 3) | ha, ib = (__builtin_amdgcn_ubfe(w, o + 8u, 8u) << 3) | hb;      // entry * 8
+        if constexpr (small_tables<SRC>()) { ia <<= 2; ib <<= 2; }
+        else { ia |= scale; ib |= scale; }
+        const uint2 ma = *reinterpret_cast<const uint2 *>(t.entries + ia), mb = *reinterpret_cast<const uint2 *>(t.entries + ib);
+        r.m = make_uint4(ma.x, ma.y, mb.x, mb.y);
+        r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(h ? v.b.y : v.b.x, 8u * e, 8u) << sign_shift<SRC>()));
+    }
+    return r;
+}
+// f: the scale of the step's columns where the table does not hold it (sixteen columns IQ2_XS, IQ1_M; 32 the others, small tables)
+template <int SRC> constexpr uint32_t steps_per_scale() { return fmt<SRC>() == F_XS || fmt<SRC>() == F_M ? 2u : small_tables<SRC>() ? 4u : 0u; }
+template <int SRC>
+__device__ __forceinline__ half2_t step_scale(const Quarter &v, uint32_t s) {
+    const uint32_t h = s >> 2, e = s & 3u;
+    if constexpr (fmt<SRC>() == F_XS) return odd_splat(__builtin_amdgcn_ubfe(v.c, 8u * h + 4u * (e >> 1), 4u));
+    else if constexpr (fmt<SRC>() == F_M) return odd_splat(__builtin_amdgcn_ubfe(v.a.w, 6u * h + 3u * (e >> 1), 3u));
+    else if constexpr (fmt<SRC>() == F_XXS) return odd_splat((h ? v.a.w : v.a.y) >> 28);
+    else return odd_splat(__builtin_amdgcn_ubfe(v.c, 16u + 4u * h, 4u));
+}
+template <int SRC>
+__device__ __forceinline__ half8_t finish_entry(const Entry &e, half2_t f) {
+    constexpr uint32_t kSign = 0x80008000u;
+    H8 r;
+    r.u = e.m;
+    if constexpr (fmt<SRC>() == F_M) {
+        // (2 s + 1) / 8 with the sign of the offset: three exponent steps down (2 s + 1 >= 1 is a normal number), sign bit by xor
+        const uint32_t neg = (e.s & 8u) << 12;
+        const half2_t off = __builtin_bit_cast(half2_t, (__builtin_bit_cast(uint32_t, f) - 0x0c000c00u) ^ (neg | (neg << 16)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * f + off;
+    } else if constexpr (fmt<SRC>() == F_XS || small_tables<SRC>()) {     // IQ2_XS entries are signed bytes in general: the sign goes to the (positive) scale
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * __builtin_bit_cast(half2_t, __builtin_bit_cast(uint32_t, f) | ((e.s << i) & kSign));
+    } else {
+        r.u.x |= e.s & kSign; r.u.y |= (e.s << 1) & kSign; r.u.z |= (e.s << 2) & kSign; r.u.w |= (e.s << 3) & kSign;
+    }
+    return r.v;
+}
+
+}  // namespace redhip

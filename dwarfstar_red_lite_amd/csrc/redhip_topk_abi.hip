@@ -195,7 +195,7 @@ bool ensure_scratch(TopkPool *p, uint32_t n_act_rows, uint32_t hidden, uint32_t 
 // the three launches of one token over a device slot table: gate/up + SwiGLU per expert, down rows per expert into tmp[e][r],
 // weighted sum in list order (native/redmetal_topk.m:1338-1415 and :1858-1943). x1: experts from x_split on read it. With
 // out == nullptr the sum is left to the caller; with a tail the last launch also adds the residual and the shared expert.
-struct Tail { const float *resid, *shared, *scalar; float *x, *layer_out; };
+using Tail = TokenTail;
 constexpr uint32_t kFastMaxTopK = 64u;             // experts per call on the slice kernels (sizes the partial vectors)
 
 __global__ __launch_bounds__(256) void topk_tail_kernel(const float *tmp, const float *weights, uint32_t top_k, uint32_t n,
@@ -229,6 +229,13 @@ bool enqueue_token(TopkPool *p, hipStream_t s, const uint64_t *table_dev, const 
     ExpertSet ex{nullptr, 0, gate_bytes, up_bytes, word_gate_up(type_word), word_down(type_word)};
     ex.table = table_dev;
     float *act = static_cast<float *>(p->act.p), *tmp = static_cast<float *>(p->tmp.p);
+    if ((out || tail) && token_rows_supported(ex.gate_up_type, ex.down_type, top_k, hidden, ffn, x, x1)) {
+        hipError_t e = launch_token_gateup(ex, top_k, hidden, ffn, x, x1, x_split, act, s);
+        if (e == hipSuccess) e = launch_token_down(ex, weights_dev, top_k, ffn, row_start, row_count, act, out, tail, s);
+        if (e != hipSuccess) { TOPK_ERR("top-k HIP command failed: %s", hipGetErrorString(e)); return false; }
+        return true;
+    }
+    // Q6_K rows, more experts than the kernels above hold, or the per-expert results wanted
     hipError_t e = launch_moe_gateup(ex, nullptr, top_k, hidden, ffn, x, act, s, x1, x_split);
     // one group per expert with exactly one pair: pair e reads act[e], writes tmp[e]
     if (e == hipSuccess) e = launch_batch_down(ex, nullptr, p->iota, nullptr, top_k, top_k, hidden, ffn, act, tmp, s);

@@ -120,9 +120,8 @@ struct Moe {
     GroupScratch group_scratch{};
     const GroupScratch *group_scratch_ptr() const { return group_mem ? &group_scratch : nullptr; }
     float *pair_weight = nullptr, *tmp = nullptr, *sh_tmp = nullptr;
-    // chunks on mixed layouts: the shared expert's dense products (x -> sh_gu -> sh_act -> sh_tmp) run on a stream of their own beside
+    // chunks on mixed layouts: the shared expert's dense products (x -> sh_act -> sh_tmp) run on a stream of their own beside
     // the routed experts' tile kernels, which leave most of the machine's issue slots free; forked and joined with events
-    float *sh_gu = nullptr;                  // [max_tokens][2 ffn]
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     void *act_h = nullptr, *act_l = nullptr; // fp16 [top_k + 1][ffn] each
@@ -245,14 +244,13 @@ __global__ __launch_bounds__(256) void resid_rms_kernel(const float *x, const fl
 }
 
 // The shared expert of a chunk on a mixed layout as dense f32 products (gate | up, SwiGLU, down) on the side stream: forked from s here,
-// joined by join_shared_dense before the combine. Reads x, writes sh_gu, sh_act, sh_tmp, which nothing on s touches in between.
+// joined by join_shared_dense before the combine. Reads x, writes sh_act, sh_tmp, which nothing on s touches in between.
 int fork_shared_dense(Moe *m, const Layer &L, const float *x, uint32_t ntok, hipStream_t s) {
     const redhip_moe_config &c = m->cfg;
     HIP_OK(hipEventRecord(m->ev_fork, s), "fork event");
     HIP_OK(hipStreamWaitEvent(m->side, m->ev_fork, 0), "fork wait");
     prof_set_stage(ST_BATCH_GATEUP);
-    HIP_OK(launch_f32_tiles(L.dense_gu, nullptr, x, ntok, c.hidden, 2u * c.ffn, m->sh_gu, 2u * c.ffn, nullptr, nullptr, nullptr, m->side), "shared gate/up tiles");
-    HIP_OK(launch_swiglu_rows(m->sh_gu, 2u * c.ffn, ntok, c.ffn, m->sh_act, m->side), "shared SwiGLU");
+    HIP_OK(launch_f32_swiglu_tiles(L.dense_gu, x, ntok, c.hidden, c.ffn, m->sh_act, m->side), "shared gate/up tiles");
     prof_set_stage(ST_BATCH_DOWN);
     HIP_OK(launch_f32_tiles(L.dense_down, nullptr, m->sh_act, ntok, c.ffn, c.hidden, m->sh_tmp, c.hidden, nullptr, nullptr, nullptr, m->side), "shared down tiles");
     HIP_OK(hipEventRecord(m->ev_join, m->side), "join event");
@@ -552,7 +550,6 @@ redhip_moe_t redhip_moe_create(const redhip_moe_config *cfg) {
                             align256(T * c.top_k * c.ffn * 4u) + align256(T * c.ffn * 4u) +
                             2u * align256(2u * T * c.hidden) + align256(4u * T) + 2u * align256(2u * T * (c.top_k + 1u) * c.ffn) +
                             align256(4u * T * (c.top_k + 1u) * (c.ffn / 32u)) +
-                            (T > 8u && m->mixed ? align256(8u * T * c.ffn) : 0u) +
                             (T > 1u ? 6u * align256(4u * (T * c.top_k + 2u)) + align256(4u * T * c.top_k * c.hidden) + align256(4u * T * c.hidden) +
                                           4u * align256(12u * (size_t)prefill_tile_bound(c.max_tokens, c.top_k, c.n_expert)) : 0u);      // (three tile lists)
     ok = ok && hipMalloc(reinterpret_cast<void **>(&m->ws), ws_bytes) == hipSuccess;
@@ -580,7 +577,6 @@ redhip_moe_t redhip_moe_create(const redhip_moe_config *cfg) {
     m->act_l = w; w += align256(2u * T * (c.top_k + 1u) * c.ffn);
     m->act_exp = reinterpret_cast<int *>(w); w += align256(4u * T * (c.top_k + 1u) * (c.ffn / 32u));
     if (T > 8u && m->mixed) {
-        m->sh_gu = reinterpret_cast<float *>(w); w += align256(8u * T * c.ffn);
         if (hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking) != hipSuccess || hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&m->ev_join, hipEventDisableTiming) != hipSuccess) {
             moe_err("failed to create the side stream of the shared expert");

@@ -97,76 +97,78 @@ hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count
 
 // ---------------------------------------------------------------- router logits of a token chunk
 
-// logits[tok][e] = W[e] . x[tok] for an f32 router as a tiled product on v_mfma_f32_16x16x4_f32 (full fp32 multiply-add): a workgroup
-// owns 32 rows x 32 tokens, wave (wr, wt) the 16 x 16 block of rows 16 wr .. and tokens 16 wt .. over the whole hidden dimension. Both
-// operands pass through LDS in slices of 64 k (double-buffered, one barrier per slice: the next two slices are in registers while this one
-// is multiplied), so a row or an activation vector is read from L2 once per workgroup instead of once per 16 x 16 block. Lane
-// (r = l % 16, q = l / 16) reads four consecutive k of row r and of token r per 16 k and feeds them to four MFMAs (A[i = r][k = q],
-// B[k = q][j = r], D[i = 4q .. 4q + 3][j = r]; the order of k inside a slice does not matter as long as both operands agree). With
-// `gate_inp` set, row E is that vector (the shared expert's gate). A second kind of workgroup (blockIdx.x beyond the row tiles,
-// launched when xh is set) does the fp16 split of its tokens' activations; it then also multiplies them with the gate vector, so the
-// row tiles cover the E matrix rows only (512 experts x 512 tokens: 16 x 16 tiles, one per compute unit, instead of a seventeenth row of
-// tiles for the one vector). The same kernel multiplies any f32 matrix [E][H] with a chunk of activations (dense shared expert).
-constexpr uint32_t kGemmTile = 32u, kGemmK = 64u, kGemmRow = kGemmK + 4u;      // LDS row of 68 floats: the eight lanes of a 16-byte read pass hit different banks
+// out[tok][row] = W[row] . x[tok] for an f32 matrix W (a router, the dense shared expert of mixed layouts) and a chunk of activations, on
+// v_mfma_f32_16x16x4_f32 (full fp32 multiply-add). A workgroup owns BR = 16 MR WR rows x BT = 16 MT WT tokens; a wave MR blocks of 16 rows times
+// MT of 16 tokens, and half of k: the waves come in two sets, one for the even slices of 64 k, one for the odd ones, whose sums meet in LDS at
+// the end. Both operands pass through LDS (SLICE k of either half per round, double-buffered, the next two rounds in registers). Lane
+// (r = l % 16, q = l / 16) reads four consecutive k of row r and of token r and feeds them to four MFMAs (A[i = r][k = q], B[k = q][j = r],
+// D[i = 4q .. 4q + 3][j = r]; the order of k does not matter as long as both operands agree).
+// What bounds it: the matrix pipe where a tile is large (64 x 64: 16 bytes of L2 per clock and compute unit; tiles of 32 x 32 for every size
+// needed 32, and waited for them), the number of workgroups where a chunk is small. So the tile is chosen by the launch (f32_tile_choice).
+// The order in which an output's products are added is the same for every tile.
+// SWIGLU: W holds gate rows, then as many up rows; two row blocks beside each other are the gate and the up rows of 16 columns, and out gets
+// silu(gate) * up of them: no pass of its own over the products.
+// Launches with xh get workgroups behind the tiles that write the fp16 halves of the activations (a wave per token, split_token) and multiply them
+// with gate_inp, if there is one, as row n_rows; without xh the tiles have it as a further row.
 
-// Eight waves: waves 0..3 take the even slices of 64 k, waves 4..7 the odd ones (each set one 16 x 16 block per wave, as described above);
-// the two partial blocks meet in LDS at the end. Two waves per SIMD, so one's MFMAs run while the other waits at the barrier or for LDS,
-// and half as many barriers as slices.
-__global__ __launch_bounds__(512) void router_f32_tile_kernel(const float *w, const float *gate_inp, const float *x, float *logits, uint32_t out_stride,
-                                                              _Float16 *xh, _Float16 *xl, int *xexp, uint32_t H, uint32_t E, uint32_t ntok) {
-    __shared__ __attribute__((aligned(16))) float ws[2][2][kGemmTile][kGemmRow], xs[2][2][kGemmTile][kGemmRow];      // [buffer][k half]
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
-    const uint32_t n_rows = E + (gate_inp && !xh ? 1u : 0u), row_tiles = (n_rows + kGemmTile - 1u) / kGemmTile, tok_tiles = (ntok + kGemmTile - 1u) / kGemmTile;
-    const uint32_t n_tile = row_tiles * tok_tiles;
-    if (blockIdx.x >= n_tile) {                            // split job: one wave per token, 8 tokens per workgroup
-        const uint32_t tok = 8u * (blockIdx.x - n_tile) + wave;
-        if (tok >= ntok) return;
-        // the vector as float4 per lane, eight requested at a time (2048 elements per pass: one round trip for the usual widths)
-        const float4 *xt = reinterpret_cast<const float4 *>(x + (uint64_t)tok * H), *gv = reinterpret_cast<const float4 *>(gate_inp);
-        const uint32_t H4 = H / 4u;
-        float amax = 0.0f, gate = 0.0f;
-        for (uint32_t base = 0; base < H4; base += 512u) {
-            float4 v[8], g[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const uint32_t i = base + 64u * k + lane;
-                v[k] = i < H4 ? xt[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                g[k] = gate_inp && i < H4 ? gv[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+__device__ __forceinline__ void split_token(const float *gate_inp, const float *x, float *logits, uint32_t out_stride, _Float16 *xh, _Float16 *xl, int *xexp, uint32_t H,
+                                            uint32_t E, uint32_t tok, uint32_t lane) {
+            // the vector as float4 per lane, eight requested at a time (2048 elements per pass: one round trip for the usual widths)
+            const float4 *xt = reinterpret_cast<const float4 *>(x + (uint64_t)tok * H), *gv = reinterpret_cast<const float4 *>(gate_inp);
+            const uint32_t H4 = H / 4u;
+            float amax = 0.0f, gate = 0.0f;
+            for (uint32_t base = 0; base < H4; base += 512u) {
+                float4 v[8], g[8];
+    #pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const uint32_t i = base + 64u * k + lane;
+                    v[k] = i < H4 ? xt[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    g[k] = gate_inp && i < H4 ? gv[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                }
+    #pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    amax = fmaxf(fmaxf(amax, fmaxf(fabsf(v[k].x), fabsf(v[k].y))), fmaxf(fabsf(v[k].z), fabsf(v[k].w)));
+                    gate = fmaf(g[k].w, v[k].w, fmaf(g[k].z, v[k].z, fmaf(g[k].y, v[k].y, fmaf(g[k].x, v[k].x, gate))));
+                }
             }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                amax = fmaxf(fmaxf(amax, fmaxf(fabsf(v[k].x), fabsf(v[k].y))), fmaxf(fabsf(v[k].z), fabsf(v[k].w)));
-                gate = fmaf(g[k].w, v[k].w, fmaf(g[k].z, v[k].z, fmaf(g[k].y, v[k].y, fmaf(g[k].x, v[k].x, gate))));
+    #pragma unroll
+            for (int o = 32; o > 0; o >>= 1) { amax = fmaxf(amax, __shfl_xor(amax, o, 64)); gate += __shfl_xor(gate, o, 64); }
+            const int e = prescale_exp(amax);
+            const float inv = exp2i(-e);
+            for (uint32_t base = 0; base < H4; base += 512u) {
+                float4 v[8];
+    #pragma unroll
+                for (int k = 0; k < 8; ++k) { const uint32_t i = base + 64u * k + lane; v[k] = xt[i < H4 ? i : 0u]; }
+    #pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const uint32_t i = base + 64u * k + lane;
+                    if (i >= H4) continue;
+                    const float f[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+                    half4_t h4, l4;
+    #pragma unroll
+                    for (int c = 0; c < 4; ++c) { _Float16 hh, ll; split_hi_lo(f[c], inv, &hh, &ll); h4[c] = hh; l4[c] = ll; }
+                    *reinterpret_cast<half4_t *>(xh + (uint64_t)tok * H + 4u * i) = h4;
+                    *reinterpret_cast<half4_t *>(xl + (uint64_t)tok * H + 4u * i) = l4;
+                }
             }
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) { amax = fmaxf(amax, __shfl_xor(amax, o, 64)); gate += __shfl_xor(gate, o, 64); }
-        const int e = prescale_exp(amax);
-        const float inv = exp2i(-e);
-        for (uint32_t base = 0; base < H4; base += 512u) {
-            float4 v[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) { const uint32_t i = base + 64u * k + lane; v[k] = xt[i < H4 ? i : 0u]; }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const uint32_t i = base + 64u * k + lane;
-                if (i >= H4) continue;
-                const float f[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-                half4_t h4, l4;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) { _Float16 hh, ll; split_hi_lo(f[c], inv, &hh, &ll); h4[c] = hh; l4[c] = ll; }
-                *reinterpret_cast<half4_t *>(xh + (uint64_t)tok * H + 4u * i) = h4;
-                *reinterpret_cast<half4_t *>(xl + (uint64_t)tok * H + 4u * i) = l4;
+            if (lane == 0u) {
+                xexp[tok] = e;
+                if (gate_inp) logits[(uint64_t)tok * out_stride + E] = gate;
             }
-        }
-        if (lane == 0u) {
-            xexp[tok] = e;
-            if (gate_inp) logits[(uint64_t)tok * out_stride + E] = gate;
-        }
+}
+
+template <int MR, int MT, uint32_t WR, uint32_t WT, uint32_t SLICE, bool SWIGLU>
+__global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w, const float *gate_inp, const float *x, float *out, uint32_t out_stride, _Float16 *xh,
+                                                                  _Float16 *xl, int *xexp, uint32_t K, uint32_t n_rows, uint32_t ntok) {
+    constexpr uint32_t BR = 16u * MR * WR, BT = 16u * MT * WT, T = 128u * WR * WT, P = SLICE / 4u, D = T / (2u * P), NW = BR / D, NX = BT / D;      // P pieces of 16 bytes per row, D rows per pass of the threads
+    __shared__ __attribute__((aligned(16))) float lds[2][2][BR + BT][SLICE + 4u];      // [buffer][k half][W rows, then tokens]
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t all_rows = n_rows + (gate_inp && !xh ? 1u : 0u), row_tiles = (all_rows + BR - 1u) / BR, tok_tiles = (ntok + BT - 1u) / BT, n_tile = row_tiles * tok_tiles;
+    if (blockIdx.x >= n_tile) {
+        const uint32_t tok = T / 64u * (blockIdx.x - n_tile) + wave;
+        if (tok < ntok) split_token(gate_inp, x, out, out_stride, xh, xl, xexp, K, n_rows, tok, lane);
         return;
     }
-    // staging: thread t of k half h = t / 256 moves rows (t % 256) / 16 and + 16 of both operands, 16 bytes at column 4 (t % 16) of its half's
-    // slice; rows beyond the last one repeat another and are not stored
     // Workgroups are dealt to the eight XCDs in turn, each with its own L2: workgroup i lands on XCD i % 8. The tiles of one XCD form a
     // compact block of the tile grid (a quarter of the row tiles x half of the token tiles), so that an XCD fetches a quarter of the
     // matrix and half of the activations instead of all of both. (A different dealing order would only cost this locality.)
@@ -176,103 +178,164 @@ __global__ __launch_bounds__(512) void router_f32_tile_kernel(const float *w, co
         tile_r = (xcd & 3u) * br + slot % br;
         tile_t = (xcd >> 2) * bt + slot / br;
     }
-    const uint32_t kh = tid >> 8, srow = (tid & 255u) >> 4, scol = 4u * (tid & 15u);
-    const uint32_t row_a = kGemmTile * tile_r + srow, row_b = row_a + 16u, tok_a = kGemmTile * tile_t + srow, tok_b = tok_a + 16u;
-    const float *wsrc_a = (row_a < E ? w + (uint64_t)row_a * H : gate_inp ? gate_inp : w) + scol + kh * kGemmK;
-    const float *wsrc_b = (row_b < E ? w + (uint64_t)row_b * H : gate_inp ? gate_inp : w) + scol + kh * kGemmK;
-    const float *xsrc_a = x + (uint64_t)(tok_a < ntok ? tok_a : ntok - 1u) * H + scol + kh * kGemmK;
-    const float *xsrc_b = x + (uint64_t)(tok_b < ntok ? tok_b : ntok - 1u) * H + scol + kh * kGemmK;
-    const uint32_t wr = wave & 1u, wt = (wave >> 1) & 1u, n_round = H / (2u * kGemmK);      // hidden is a multiple of 256: an even number of rounds
-    constexpr uint32_t kStep = 2u * kGemmK;                // k per round
-    // two register sets, one per LDS buffer: the loads of round rd + 2 are issued while round rd is multiplied, so a round trip has two
-    // rounds of arithmetic to hide behind (plain variables: arrays of them end up in scratch memory)
-    float4 w0a = *reinterpret_cast<const float4 *>(wsrc_a), w0b = *reinterpret_cast<const float4 *>(wsrc_b);
-    float4 x0a = *reinterpret_cast<const float4 *>(xsrc_a), x0b = *reinterpret_cast<const float4 *>(xsrc_b);
-    float4 w1a = *reinterpret_cast<const float4 *>(wsrc_a + kStep), w1b = *reinterpret_cast<const float4 *>(wsrc_b + kStep);
-    float4 x1a = *reinterpret_cast<const float4 *>(xsrc_a + kStep), x1b = *reinterpret_cast<const float4 *>(xsrc_b + kStep);
-    float4_t acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
-    const uint32_t mh = wave >> 2;                         // the k half this wave multiplies
-    auto multiply = [&](uint32_t buf) {
+    // staging: thread t moves the 16 bytes t % P of k half (t / P) % 2 of rows t / 2P, t / 2P + D, ..; rows and tokens beyond the last repeat
+    // another and are not stored. (LDS rows of SLICE + 4 floats: the sixteen lanes of a 16-byte read pass hit different banks)
+    const uint32_t scol = 4u * (tid % P), kh = (tid / P) & 1u, srow = tid / (2u * P);
+    const auto source = [&](uint32_t n) -> const float * {      // (n < NW: matrix rows, then tokens)
+        const uint32_t l = srow + n * D;
+        if (n >= NW) return x + (uint64_t)min(tile_t * BT + l - BR, ntok - 1u) * K + kh * 64u + scol;
+        const uint32_t row = SWIGLU ? ((l >> 4) & 1u) * (n_rows / 2u) + tile_r * (BR / 2u) + (l >> 5) * 16u + (l & 15u) : tile_r * BR + l;
+        return (row < n_rows ? w + (uint64_t)row * K : gate_inp ? gate_inp : w) + kh * 64u + scol;
+    };
+    constexpr uint32_t N = NW + NX;
+    static_assert(N >= 3u && N <= 6u && NW * D == BR && NX * D == BT && (SLICE == 32u || SLICE == 64u), "16-byte pieces per thread and round");
+    const float *src0 = source(0u), *src1 = source(1u), *src2 = source(2u), *src3 = source(3u < N ? 3u : 0u), *src4 = source(4u < N ? 4u : 0u), *src5 = source(5u < N ? 5u : 0u);
+    const uint32_t n_round = K / (2u * SLICE);             // even: K is a multiple of 256
+    struct Staged { float4_t v0, v1, v2, v3, v4, v5; };    // (as an array, or of float4 objects, these end up in scratch memory)
+    const auto request = [&](Staged &st, uint32_t rd) {    // (the last rounds request themselves again: no branch around the loads)
+        const uint32_t at = SLICE == 64u ? rd * 128u : (rd >> 1) * 128u + (rd & 1u) * 32u;
+        st.v0 = *reinterpret_cast<const float4_t *>(src0 + at);
+        st.v1 = *reinterpret_cast<const float4_t *>(src1 + at);
+        st.v2 = *reinterpret_cast<const float4_t *>(src2 + at);
+        if constexpr (N > 3u) st.v3 = *reinterpret_cast<const float4_t *>(src3 + at);
+        if constexpr (N > 4u) st.v4 = *reinterpret_cast<const float4_t *>(src4 + at);
+        if constexpr (N > 5u) st.v5 = *reinterpret_cast<const float4_t *>(src5 + at);
+    };
+    const auto place = [&](const Staged &st, uint32_t buf) {      // (tokens follow the rows)
+        *reinterpret_cast<float4_t *>(&lds[buf][kh][srow][scol]) = st.v0;
+        *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + D][scol]) = st.v1;
+        *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + 2u * D][scol]) = st.v2;
+        if constexpr (N > 3u) *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + 3u * D][scol]) = st.v3;
+        if constexpr (N > 4u) *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + 4u * D][scol]) = st.v4;
+        if constexpr (N > 5u) *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + 5u * D][scol]) = st.v5;
+    };
+    const uint32_t mh = wave / (WR * WT), block = wave % (WR * WT), wr = block % WR, wt = block / WR;
+    float4_t acc[MR][MT][2];
 #pragma unroll
-        for (uint32_t u = 0; u < kGemmK / 16u; ++u) {
-            const float4 av = *reinterpret_cast<const float4 *>(&ws[buf][mh][16u * wr + r][16u * u + 4u * q]);
-            const float4 bv = *reinterpret_cast<const float4 *>(&xs[buf][mh][16u * wt + r][16u * u + 4u * q]);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.x, bv.x, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.y, bv.y, acc1, 0, 0, 0);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.z, bv.z, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.w, bv.w, acc1, 0, 0, 0);
+    for (int m = 0; m < MR; ++m)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[m][t][0] = acc[m][t][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    const auto multiply = [&](uint32_t buf) {
+#pragma unroll
+        for (uint32_t u = 0; u < SLICE / 16u; ++u) {
+            float4 a[MR], b[MT];
+#pragma unroll
+            for (int m = 0; m < MR; ++m) a[m] = *reinterpret_cast<const float4 *>(&lds[buf][mh][16u * (MR * wr + m) + r][16u * u + 4u * q]);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) b[t] = *reinterpret_cast<const float4 *>(&lds[buf][mh][BR + 16u * (MT * wt + t) + r][16u * u + 4u * q]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int m = 0; m < MR; ++m)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+                        acc[m][t][k & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k == 0 ? a[m].x : k == 1 ? a[m].y : k == 2 ? a[m].z : a[m].w,
+                                                                                k == 0 ? b[t].x : k == 1 ? b[t].y : k == 2 ? b[t].z : b[t].w, acc[m][t][k & 1], 0, 0, 0);
         }
     };
+    Staged s0, s1;
+    request(s0, 0u);
+    request(s1, 1u);
     for (uint32_t rd = 0; rd < n_round; rd += 2u) {
-        *reinterpret_cast<float4 *>(&ws[0][kh][srow][scol]) = w0a;
-        *reinterpret_cast<float4 *>(&ws[0][kh][srow + 16u][scol]) = w0b;
-        *reinterpret_cast<float4 *>(&xs[0][kh][srow][scol]) = x0a;
-        *reinterpret_cast<float4 *>(&xs[0][kh][srow + 16u][scol]) = x0b;
+        place(s0, 0u);
         __syncthreads();                                   // round rd is in place; the readers of the other buffer (round rd - 1) are past their barrier
-        const uint32_t k2 = (rd + 2u < n_round ? rd + 2u : rd) * kStep;          // the last rounds reload themselves: no branch around the loads
-        w0a = *reinterpret_cast<const float4 *>(wsrc_a + k2);
-        w0b = *reinterpret_cast<const float4 *>(wsrc_b + k2);
-        x0a = *reinterpret_cast<const float4 *>(xsrc_a + k2);
-        x0b = *reinterpret_cast<const float4 *>(xsrc_b + k2);
+        request(s0, rd + 2u < n_round ? rd + 2u : rd);
         multiply(0u);
-        *reinterpret_cast<float4 *>(&ws[1][kh][srow][scol]) = w1a;
-        *reinterpret_cast<float4 *>(&ws[1][kh][srow + 16u][scol]) = w1b;
-        *reinterpret_cast<float4 *>(&xs[1][kh][srow][scol]) = x1a;
-        *reinterpret_cast<float4 *>(&xs[1][kh][srow + 16u][scol]) = x1b;
+        place(s1, 1u);
         __syncthreads();
-        const uint32_t k3 = (rd + 3u < n_round ? rd + 3u : rd + 1u) * kStep;
-        w1a = *reinterpret_cast<const float4 *>(wsrc_a + k3);
-        w1b = *reinterpret_cast<const float4 *>(wsrc_b + k3);
-        x1a = *reinterpret_cast<const float4 *>(xsrc_a + k3);
-        x1b = *reinterpret_cast<const float4 *>(xsrc_b + k3);
+        request(s1, rd + 3u < n_round ? rd + 3u : rd + 1u);
         multiply(1u);
     }
-    // the odd slices' blocks go through LDS (buffer 0 was last read two barriers ago) to the waves that hold the even ones
-    float *meet = &ws[0][0][0][0];                         // [4 blocks][64 lanes] float4
+    // the odd slices' sums go through LDS to the waves that hold the even ones; SWIGLU with one row block per wave: then the up products to
+    // the wave of their gate rows
+    float4_t *meet = reinterpret_cast<float4_t *>(&lds[0][0][0][0]);
+    static_assert(sizeof(lds) >= (size_t)WR * WT * MR * MT * 64u * 16u, "the sums fit the staging buffers");
+    const auto at = [&](uint32_t b, int m, int t) { return ((b * MR + m) * MT + t) * 64u + lane; };
     __syncthreads();
-    if (mh == 1u) *reinterpret_cast<float4 *>(meet + ((wave & 3u) * 64u + lane) * 4u) = make_float4(acc0[0] + acc1[0], acc0[1] + acc1[1], acc0[2] + acc1[2], acc0[3] + acc1[3]);
-    __syncthreads();
-    if (mh == 1u) return;
-    const float4 other = *reinterpret_cast<const float4 *>(meet + (wave * 64u + lane) * 4u);
-    const float oth[4] = {other.x, other.y, other.z, other.w};
-    const uint32_t out_tok = kGemmTile * tile_t + 16u * wt + r;
+    if (mh == 1u) {
 #pragma unroll
-    for (uint32_t t = 0; t < 4u; ++t) {
-        const uint32_t out_row = kGemmTile * tile_r + 16u * wr + 4u * q + t;
-        if (out_tok < ntok && out_row < n_rows) logits[(uint64_t)out_tok * out_stride + out_row] = (acc0[t] + acc1[t]) + oth[t];
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) meet[at(block, m, t)] = acc[m][t][0] + acc[m][t][1];
     }
+    __syncthreads();
+    if (mh == 0u) {
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[m][t][0] = (acc[m][t][0] + acc[m][t][1]) + meet[at(block, m, t)];
+    }
+    if constexpr (SWIGLU && MR == 1) {
+        if (mh == 0u && (wr & 1u)) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) meet[at(block, 0, t)] = acc[0][t][0];      // (its own place: nobody else reads it before)
+        }
+        __syncthreads();
+    }
+    if (mh == 1u || (SWIGLU && MR == 1 && (wr & 1u))) return;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const uint32_t tok = tile_t * BT + 16u * (MT * wt + t) + r;
+        if (tok >= ntok) continue;
+        if constexpr (SWIGLU) {
+            float4_t y;
+            const float4_t g = acc[0][t][0], u = MR == 1 ? meet[at(block + 1u, 0, t)] : acc[MR - 1][t][0];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = (g[i] / (1.0f + expf(-g[i]))) * u[i];
+            *reinterpret_cast<float4_t *>(out + (uint64_t)tok * out_stride + tile_r * (BR / 2u) + 16u * (MR == 1 ? wr / 2u : wr) + 4u * q) = y;
+        } else {
+#pragma unroll
+            for (int m = 0; m < MR; ++m)
+#pragma unroll
+                for (uint32_t i = 0; i < 4u; ++i) {
+                    const uint32_t row = tile_r * BR + 16u * (MR * wr + m) + 4u * q + i;
+                    if (row < all_rows) out[(uint64_t)tok * out_stride + row] = acc[m][t][0][i];
+                }
+        }
+    }
+}
+
+// The largest tile that costs no more rounds of the device (256 compute units, workgroups of equal length) than a quarter above the best
+// tile: large tiles read less, small ones fill the device when a chunk has few outputs.
+template <bool SWIGLU>
+hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out, uint32_t out_stride, void *xh, void *xl,
+                     int *xexp, hipStream_t s) {
+    if (!ntok || !K || K % 256u || !n_rows || !w || !x || !out || (SWIGLU && n_rows % 128u)) return hipErrorInvalidValue;
+    const uint32_t all_rows = n_rows + (extra_row && !xh ? 1u : 0u);
+    static constexpr struct { uint32_t br, bt; } kTiles[4] = {{64u, 64u}, {64u, 32u}, {32u, 32u}, {32u, 16u}};
+    uint64_t n[4], cost[4], best = ~0ull;
+    for (int i = 0; i < 4; ++i) {
+        n[i] = (uint64_t)((all_rows + kTiles[i].br - 1u) / kTiles[i].br) * ((ntok + kTiles[i].bt - 1u) / kTiles[i].bt);
+        cost[i] = (n[i] + 255u) / 256u * (kTiles[i].br * kTiles[i].bt);
+        if (cost[i] < best) best = cost[i];
+    }
+    int pick = 0;
+    while (4u * cost[pick] > 5u * best) ++pick;
+    const uint32_t waves = pick < 3 ? 8u : 4u, split_wgs = xh ? (ntok + waves - 1u) / waves : 0u;      // (behind the tiles)
+    if (n[pick] + split_wgs > 0x7fffffffull) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)n[pick] + split_wgs), block(64u * waves);
+    _Float16 *h = static_cast<_Float16 *>(xh), *l = static_cast<_Float16 *>(xl);
+    if (pick == 0) REDHIP_LAUNCH((f32_tiles_kernel<2, 2, 2u, 2u, 32u, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    else if (pick == 1) REDHIP_LAUNCH((f32_tiles_kernel<2, 1, 2u, 2u, 32u, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    else if (pick == 2) REDHIP_LAUNCH((f32_tiles_kernel<1, 1, 2u, 2u, 64u, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    else REDHIP_LAUNCH((f32_tiles_kernel<1, 1, 2u, 1u, 64u, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    return hipGetLastError();
 }
 
 // out[tok][row] = W[row] . x[tok] for an f32 matrix W [n_rows][K] and a chunk of activations x [ntok][K]; extra_row (optional) is one more
 // row behind the matrix; xh / xl / xexp (optional): also write the fp16 halves of x
 hipError_t launch_f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out,
                             uint32_t out_stride, void *xh, void *xl, int *xexp, hipStream_t s) {
-    if (!ntok || !K || K % 256u || !n_rows || !w || !x || !out) return hipErrorInvalidValue;
-    const uint32_t row_tiles = (n_rows + (extra_row && !xh ? 1u : 0u) + kGemmTile - 1u) / kGemmTile, tok_tiles = (ntok + kGemmTile - 1u) / kGemmTile;      // (as in the kernel)
-    if ((uint64_t)row_tiles * tok_tiles + ntok > 0x7fffffffull) return hipErrorInvalidValue;
-    const uint32_t split_wgs = xh ? (ntok + 7u) / 8u : 0u;            // behind the tiles
-    REDHIP_LAUNCH(router_f32_tile_kernel, dim3(row_tiles * tok_tiles + split_wgs), dim3(512), 0, s, w, extra_row, x, out, out_stride,
-                  static_cast<_Float16 *>(xh), static_cast<_Float16 *>(xl), xexp, K, n_rows, ntok);
-    return hipGetLastError();
+    return f32_tiles<false>(w, extra_row, x, ntok, K, n_rows, out, out_stride, xh, xl, xexp, s);
+}
+// act[tok][c] = silu(W[c] . x[tok]) * (W[ffn + c] . x[tok])
+hipError_t launch_f32_swiglu_tiles(const float *w, const float *x, uint32_t ntok, uint32_t K, uint32_t ffn, float *act, hipStream_t s) {
+    return f32_tiles<true>(w, nullptr, x, ntok, K, 2u * ffn, act, ffn, nullptr, nullptr, nullptr, s);
 }
 
 hipError_t launch_router_f32_tiles(const float *w, const float *gate_inp, const float *x, uint32_t ntok, uint32_t hidden, uint32_t n_expert,
                                    float *logits, void *xh, void *xl, int *xexp, hipStream_t s) {
     return launch_f32_tiles(w, gate_inp, x, ntok, hidden, n_expert, logits, n_expert + 1u, xh, xl, xexp, s);
 }
-
-// act[tok][c] = silu(gu[tok][c]) * gu[tok][ffn + c]
-__global__ void swiglu_rows_kernel(const float *gu, uint32_t gu_stride, uint32_t ffn, float *act) {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x, tok = blockIdx.y;
-    if (c >= ffn) return;
-    const float g = gu[(uint64_t)tok * gu_stride + c], u = gu[(uint64_t)tok * gu_stride + ffn + c];
-    act[(uint64_t)tok * ffn + c] = (g / (1.0f + expf(-g))) * u;
-}
-
-hipError_t launch_swiglu_rows(const float *gu, uint32_t gu_stride, uint32_t ntok, uint32_t ffn, float *act, hipStream_t s) {
-    REDHIP_LAUNCH(swiglu_rows_kernel, dim3((ffn + 255u) / 256u, ntok), dim3(256), 0, s, gu, gu_stride, ffn, act);
-    return hipGetLastError();
-}
-
 
 }  // namespace redhip

@@ -1806,7 +1806,8 @@ template <int REP, int MIX> constexpr uint32_t slice_table_bytes() {
     return MIX == 2 ? 512u * 16u : MIX == 3 ? 2048u * 16u : (uint32_t)(REP + 1) * kMagBytes + 128u * 4u * (uint32_t)kSliceLut;
 }
 constexpr uint32_t kSliceSharedParts = 4u;      // workgroups per 32 columns of a dense shared expert (mixed layouts)
-template <int NKC, int REP, bool SLOTS = false, int MIX = 0>        // hidden = 512 * NKC; MIX as in batch_slice_kernel
+// MANY: one grid layer per token (a template flag: reading the token's index costs the one-token launch of mixed layouts 0.3 us)
+template <int NKC, int REP, bool SLOTS = false, int MIX = 0, bool MANY = false>        // hidden = 512 * NKC; MIX as in batch_slice_kernel
 __global__ __launch_bounds__(kWaves * 64) void expert_slice_kernel(const void *p0_first, uint32_t n_expert_first, uint32_t top_k_first, const void *p1_first,
                                                                    const void *p2_first, uint32_t u0_first, uint32_t hidden_first, uint32_t ffn_first, SliceArgs a) {
     constexpr int NW = kWaves;
@@ -1827,11 +1828,13 @@ __global__ __launch_bounds__(kWaves * 64) void expert_slice_kernel(const void *p
     const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63u, blk = lane >> 2, j = lane & 3u;
     // Mixed layouts: the shared expert's dense slice is kSliceSharedParts workgroups (a quarter of the output rows each: 16 x hidden bytes of f32
     // per row-quarter would otherwise be the longest-running workgroup); they come first in the grid, the routed slots behind them
+    const uint32_t tok = MANY ? blockIdx.z : 0u;
     const uint32_t g = blockIdx.x, slot = MIX != 0 && !SLOTS ? (blockIdx.y < kSliceSharedParts ? top_k_first : blockIdx.y - kSliceSharedParts) : blockIdx.y;
     // The leading kernel arguments repeat what the first requests of the kernel need - a.logits, a.xh, a.xl (SLOTS: a.slot_table, a.x,
     // a.x1 and a.x_split), a.n_expert, a.top_k: leading scalar arguments can be handed to a wave in registers at its start, so these
     // requests do not wait for the argument block to come from memory.
-    const float *logits_first = SLOTS ? nullptr : static_cast<const float *>(p0_first);
+    const float *logits_first = SLOTS ? nullptr : static_cast<const float *>(p0_first);      // (MANY: always given)
+    if constexpr (MANY) logits_first += tok * (n_expert_first + 1u);
     const bool is_shared = slot >= top_k_first;
     const bool selecting = !SLOTS && !is_shared && logits_first;
     REDHIP_STAMP(0);
@@ -1841,17 +1844,17 @@ __global__ __launch_bounds__(kWaves * 64) void expert_slice_kernel(const void *p
     if constexpr (MIX != 0 && !SLOTS) {
         if (is_shared) {       // the shared expert's slice from dense f32 data: SwiGLU of the 32 columns, then their part of every output row
             if (tid < 32u) {
-                const float *gu = a.shared_gu + 32u * g + tid;
+                const float *gu = a.shared_gu + tok * 2u * F + 32u * g + tid;
                 const float gv = gu[0], uv = gu[F];
                 part[tid] = (gv / (1.0f + expf(-gv))) * uv;
             }
-            const float gate = logits_first ? 1.0f / (1.0f + expf(-logits_first[n_expert_first])) : a.scalar_in[0];
+            const float gate = logits_first ? 1.0f / (1.0f + expf(-logits_first[n_expert_first])) : a.scalar_in[tok];
             __syncthreads();
             // eight lanes per output row, each lane four of the 32 columns: a wave-wide load reads the 128-byte slices of eight rows whole
             const uint32_t sub = tid & 7u;
             const float4 av = *reinterpret_cast<const float4 *>(part + 4u * sub);
             constexpr uint32_t kRows = (uint32_t)NW * 8u;      // rows per round of the workgroup
-            float *out = a.partial + ((uint64_t)slot * FG + g) * H;
+            float *out = a.partial + ((uint64_t)(tok * (top_k_first + 1u) + slot) * FG + g) * H;
             const uint32_t h_end = (blockIdx.y + 1u) * (H / kSliceSharedParts);      // (hidden is a multiple of 512)
             for (uint32_t h0 = blockIdx.y * (H / kSliceSharedParts) + (tid >> 3); h0 < h_end; h0 += 4u * kRows) {      // four rounds' loads in flight
                 float4 w4[4];
@@ -1894,7 +1897,7 @@ __global__ __launch_bounds__(kWaves * 64) void expert_slice_kernel(const void *p
         amax = wave_max(amax);                         // waves kc = 0 .. NKC - 1 cover the whole vector between them
         if (lane == 0u) reinterpret_cast<float *>(sel)[wave] = amax;
     } else {
-        const _Float16 *xh_g = static_cast<const _Float16 *>(p1_first) + 32u * G, *xl_g = static_cast<const _Float16 *>(p2_first) + 32u * G;
+        const _Float16 *xh_g = static_cast<const _Float16 *>(p1_first) + tok * hidden_first + 32u * G, *xl_g = static_cast<const _Float16 *>(p2_first) + tok * hidden_first + 32u * G;
         // The selecting wave asks for the logits before anything else and for its activations only behind the selection (requested together,
         // the logits were measured to arrive 0.5 us later: the wave then waits for all its loads); the barrier behind the selection
         // waits for LDS only, so those late activations do not hold the workgroup up.
@@ -1940,19 +1943,19 @@ __global__ __launch_bounds__(kWaves * 64) void expert_slice_kernel(const void *p
             }
         }
     } else if (is_shared) {
-        comb = logits_first ? 1.0f / (1.0f + expf(-logits_first[n_expert_first])) : a.scalar_in[0];
+        comb = logits_first ? 1.0f / (1.0f + expf(-logits_first[n_expert_first])) : a.scalar_in[tok];
         __syncthreads();                               // table
     } else if (logits_first) {
         lds_barrier();                                 // selection (by wave 0, at the kernel's head) and table: both in LDS
         expert = __builtin_amdgcn_readfirstlane(sel->ids[slot]);      // the same in every lane: the weights' base addresses stay scalar
         comb = sel->w[slot];
         if (g == 0u && slot == 0u) {
-            if (tid < a.top_k) { a.ids_out[tid] = sel->ids[tid]; a.weights_out[tid] = sel->w[tid]; }
-            if (tid == 0u) a.scalar_out[0] = sel->scalar;
+            if (tid < a.top_k) { a.ids_out[tok * a.top_k + tid] = sel->ids[tid]; a.weights_out[tok * a.top_k + tid] = sel->w[tid]; }
+            if (tid == 0u) a.scalar_out[tok] = sel->scalar;
         }
     } else {
-        expert = __builtin_amdgcn_readfirstlane(guarded_id(a.ids_in[slot], a.n_expert, a.status));
-        comb = a.weights_in[slot];
+        expert = __builtin_amdgcn_readfirstlane(guarded_id(a.ids_in[tok * a.top_k + slot], a.n_expert, a.status));
+        comb = a.weights_in[tok * a.top_k + slot];
         __syncthreads();                               // table
     }
     REDHIP_STAMP(1);                                   // selection (or the caller's routing) and tables are here
@@ -2015,7 +2018,7 @@ __global__ __launch_bounds__(kWaves * 64) void expert_slice_kernel(const void *p
         float gsum = 0.0f, usum = 0.0f;
 #pragma unroll
         for (int c = 0; c < NKC; ++c) { gsum += part[c * 64 + tid]; usum += part[c * 64 + 32 + tid]; }
-        const float xs = (MIX == 3 ? 1.0f : 0.125f) * exp2i(SLOTS ? x_exp : a.xexp[0]);      // d / 8 (an IQ1_M weight is d (2 s + 1) (entry +- 1/8): none) and the pre-scale of x
+        const float xs = (MIX == 3 ? 1.0f : 0.125f) * exp2i(SLOTS ? x_exp : a.xexp[tok]);      // d / 8 (an IQ1_M weight is d (2 s + 1) (entry +- 1/8): none) and the pre-scale of x
         gsum *= xs;
         usum *= xs;
         const float act = (gsum / (1.0f + expf(-gsum))) * usum;
@@ -2040,7 +2043,7 @@ __global__ __launch_bounds__(kWaves * 64) void expert_slice_kernel(const void *p
         }
     }
     const float post = act_scale[0] * comb * (MIX == 1 || MIX == 3 ? 1.0f : 0.125f);     // the activations' pre-scale, the slot's weight, d / 8 (an IQ3_S weight is d (1 + 2 nibble) grid byte: no 1 / 8)
-    float *out = a.partial + ((uint64_t)slot * FG + g) * H;
+    float *out = a.partial + ((uint64_t)(tok * (top_k_first + 1u) + slot) * FG + g) * H;
 #pragma unroll
     for (int k = 0; k < DU; ++k) {
         const uint32_t unit = wave + NW * k;
@@ -2385,33 +2388,37 @@ hipError_t launch_expert_slices(const void *experts, uint64_t stride, const void
                                 const float *logits, const uint32_t *ids_in, const float *weights_in, const float *scalar_in, uint32_t *ids_out,
                                 float *weights_out, float *scalar_out, const void *xh, const void *xl, const int *xexp, float *partial, float *out,
                                 uint32_t hidden, uint32_t ffn, uint32_t n_expert, uint32_t top_k, hipStream_t s, const float *shared_gu, const float *shared_dense,
-                                uint32_t stream_type, const int8_t *grid) {
-    if (!fused_iq2_supported(hidden, ffn) || top_k + 1u > (uint32_t)kWaves || n_expert > 1024u || hidden % 32u) return hipErrorInvalidValue;
+                                uint32_t stream_type, const int8_t *grid, uint32_t ntok) {
+    if (!ntok || !fused_iq2_supported(hidden, ffn) || top_k + 1u > (uint32_t)kWaves || n_expert > 1024u || hidden % 32u) return hipErrorInvalidValue;
     if (!logits && (!ids_in || !weights_in || !scalar_in)) return hipErrorInvalidValue;
     const bool mix = shared_gu != nullptr;             // down slices of another format (column-sliced) and the dense shared expert
     if (mix && (!shared_dense || ffn % 256u)) return hipErrorInvalidValue;
     // 1: IQ2_XXS gate / up with IQ3_S words; 2 / 3: IQ2_XS / IQ1_M streams throughout
     const int kind = !mix ? 0 : stream_type == T_IQ2_XS ? 2 : stream_type == T_IQ1_M ? 3 : 1;
-    if (kind >= 2 && !grid) return hipErrorInvalidValue;
+    if ((kind >= 2 && !grid) || (ntok > 1u && (kind == 0 || !logits))) return hipErrorInvalidValue;      // (all-IQ2_XXS layers take batches as passes)
     const SliceArgs a{static_cast<const uint8_t *>(experts), stride, static_cast<const uint8_t *>(down_cm), down_stride, static_cast<const uint8_t *>(shared),
                       static_cast<const uint8_t *>(shared_down_cm), logits, ids_in, weights_in, scalar_in, ids_out, weights_out, scalar_out,
                       static_cast<const _Float16 *>(xh), static_cast<const _Float16 *>(xl), xexp, partial, hidden, ffn, n_expert, top_k, route_guard().status,
                       nullptr, 0u, nullptr, nullptr, 0u, shared_gu, shared_dense, grid};
-    const dim3 grid_dim(ffn / 32u, top_k + (mix ? kSliceSharedParts : 1u));
-#define REDHIP_SLICE_MIX(NKC, MIX)                                                                                                     \
+    const dim3 grid_dim(ffn / 32u, top_k + (mix ? kSliceSharedParts : 1u), ntok);
+#define REDHIP_SLICE_MANY(NKC, MIX, MANY)                                                                                              \
     do {                                                                                                                               \
         static bool attr = false;                                                                                                       \
         const size_t dyn = slice_lds_bytes<MIX>(NKC);                                                                                \
         if (!attr) {                                                                                                                    \
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(expert_slice_kernel<NKC, kSliceRep, false, MIX>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn); \
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(expert_slice_kernel<NKC, kSliceRep, false, MIX, MANY>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn); \
             if (e != hipSuccess) return e;                                                                                              \
             attr = true;                                                                                                                \
         }                                                                                                                               \
-        REDHIP_LAUNCH((expert_slice_kernel<NKC, kSliceRep, false, MIX>), grid_dim, dim3(kWaves * 64), dyn, s, (const void *)a.logits, a.n_expert, a.top_k, (const void *)a.xh, (const void *)a.xl, 0u, a.hidden, a.ffn, a); \
+        REDHIP_LAUNCH((expert_slice_kernel<NKC, kSliceRep, false, MIX, MANY>), grid_dim, dim3(kWaves * 64), dyn, s, (const void *)a.logits, a.n_expert, a.top_k, (const void *)a.xh, (const void *)a.xl, 0u, a.hidden, a.ffn, a); \
+    } while (0)
+#define REDHIP_SLICE_MIX(NKC, MIX)                                                                                                     \
+    do {                                                                                                                               \
+        if (ntok > 1u) REDHIP_SLICE_MANY(NKC, MIX, true); else REDHIP_SLICE_MANY(NKC, MIX, false);                                     \
     } while (0)
 #define REDHIP_SLICE(NKC)                                                                                                              \
     do {                                                                                                                               \
-        if (kind == 3) REDHIP_SLICE_MIX(NKC, 3); else if (kind == 2) REDHIP_SLICE_MIX(NKC, 2); else if (kind == 1) REDHIP_SLICE_MIX(NKC, 1); else REDHIP_SLICE_MIX(NKC, 0); \
+        if (kind == 3) REDHIP_SLICE_MIX(NKC, 3); else if (kind == 2) REDHIP_SLICE_MIX(NKC, 2); else if (kind == 1) REDHIP_SLICE_MIX(NKC, 1); else REDHIP_SLICE_MANY(NKC, 0, false); \
     } while (0)
     prof_set_stage(ST_FUSED_EXPERTS);
     switch (hidden / 512u) {
@@ -2423,10 +2430,11 @@ hipError_t launch_expert_slices(const void *experts, uint64_t stride, const void
     }
 #undef REDHIP_SLICE
 #undef REDHIP_SLICE_MIX
+#undef REDHIP_SLICE_MANY
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     prof_set_stage(ST_SLICE_SUM);
-    REDHIP_LAUNCH(slice_sum_kernel, dim3(hidden / 32u), dim3(256), 0, s, partial, (top_k + 1u) * (ffn / 32u), hidden, out, block_context().resid_a, block_context().resid_b, SumTail{nullptr, nullptr, nullptr, nullptr});
+    REDHIP_LAUNCH(slice_sum_kernel, dim3(hidden / 32u, ntok), dim3(256), 0, s, partial, (top_k + 1u) * (ffn / 32u), hidden, out, block_context().resid_a, block_context().resid_b, SumTail{nullptr, nullptr, nullptr, nullptr});
     return hipGetLastError();
 }
 

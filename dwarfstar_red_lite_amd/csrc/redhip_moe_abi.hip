@@ -149,8 +149,12 @@ struct Moe {
         return mixed_slices && ntok <= 8u && ntok * cfg.top_k <= 128u && ntok * (cfg.top_k + 1u) <= 144u;
     }
     // ... with the layer's own router: on a mixed layout two tokens are quicker on the single-token kernels (three launches, the selection
-    // inside the gate/up kernel) than as slices behind a selection + pair sort launch of their own (four): 30.7 against 32.7 us
+    // inside the expert kernel) than as slices behind a selection + pair sort launch of their own (four): 30.7 against 32.7 us
     bool slices_after_router(uint32_t ntok) const { return small_batch(ntok, true) && (fused || ntok >= kGroupedMin); }
+    // ... of which layouts with slices take the single-token slices, one grid layer per token: two tokens of IQ2_XS / IQ1_M / IQ2_XXS + IQ3_S
+    // layers 30.9 / 30.1 / 30.3 -> 27.6 / 26.1 / 27.6 us per layer against gateup_select_kernel + down_combine_words_kernel. (448 workgroups,
+    // two per compute unit; three tokens would need a second round, and all-IQ2_XXS tables leave room for one workgroup.)
+    bool token_slices(uint32_t ntok) const { return ntok == 2u && mixed_slices && dense_routed && small_batch(ntok, true); }
     // the same batches on a mixed layout run on the single-token kernels, one grid layer per token (tokens rarely share an
     // expert at these sizes, so reading a shared expert twice costs less than the pair sort and the per-pair kernels)
     bool small_batch_mixed(uint32_t ntok) const {
@@ -371,13 +375,13 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
         prof_set_stage(ST_OTHER);
         return 1;
     }
-    if (m->mixed_slices && ntok == 1u && m->shared_gu_ready && m->layers[layer].dense_down) {
+    if (m->mixed_slices && (ntok == 1u || (select_here && m->token_slices(ntok))) && m->shared_gu_ready && m->layers[layer].dense_down) {
         // one token on a mixed layout whose small batches run as slices: the same slices, the down matrices from their column-sliced copy, the
         // shared expert from its products (m->act, left by the router launch) and the dense copy of its down matrix
         const Layer &L = m->layers[layer];
         HIP_OK(launch_expert_slices(L.packed, m->packed_stride, L.down_cm, m->down_cm_stride(), nullptr, nullptr, select_here ? m->logits : nullptr,
                                     ids, weights, m->scalar, m->ids, m->weights, m->scalar, m->xh, m->xl, m->xexp, m->partial, out, c.hidden, c.ffn, c.n_expert,
-                                    c.top_k, s, m->act, L.dense_down, m->sliced_streams() ? m->dn_type : 0u, m->sliced_streams() ? m->dn_grid : nullptr), "expert slice launch");
+                                    c.top_k, s, m->act, L.dense_down, m->sliced_streams() ? m->dn_type : 0u, m->sliced_streams() ? m->dn_grid : nullptr, ntok), "expert slice launch");
         prof_set_stage(ST_OTHER);
         return 1;
     }

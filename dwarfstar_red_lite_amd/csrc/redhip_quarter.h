@@ -213,7 +213,7 @@ __device__ __forceinline__ Entry fetch_entry(const Quarter &v, uint32_t s, const
         const uint32_t wa = h ? v.a.z : v.a.x, wb = h ? v.a.w : v.a.y;
         // bytes 0 .. 3 of the permute's second operand are the entries, 7 the top byte of the first
         if constexpr (small_tables<SRC>()) r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_ubfe(wa, 8u * e, 8u) << entry_shift<SRC>()));
-        else r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_perm(wb, wa, 0x0c0c0007u | (e << 8)) & 0xfff0u));
+        else r.m = *reinterpret_cast<const uint4 *>(t.entries + __builtin_amdgcn_perm(wb & 0xf0000000u, wa, 0x0c0c0007u | (e << 8)));
         r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(wb, 7u * e, 7u) << sign_shift<SRC>()));
     } else if constexpr (fmt<SRC>() == F_XS) {
         const uint32_t w = word_of(v.a, 2u * h + (e >> 1)), o = 16u * (e & 1u);

@@ -323,16 +323,17 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
 }
 
 // SETS 1: the narrow tiles (list 2) of a chunk, SETS 2: the wide ones (list 1). Persistent workgroups, each with an equal run of the units.
-// A launch that finds few wide tiles leaves them: the narrow one then takes every pair in tiles of 16 (list 0). A wide launch costs 20 us
-// however few tiles it has (tables, the first tile's activations), one more tile on the narrow kernels 0.3 us of the whole device.
-constexpr uint32_t kFewWide = 48u;
+// A launch that finds few wide tiles leaves them: the narrow one then takes every pair in tiles of 16 (list 0). A wide launch costs 10 us
+// however few tiles it has (tables, the first tile's activations); beyond that a wide tile took 0.32 us of the device (gate/up, hidden 2048,
+// ffn 512) where two narrow ones take 0.43, 0.21 against 0.26 in the down kernels, 0.24 against 0.27 with IQ3_S words.
+template <int SRC, bool DOWN> constexpr uint32_t few_wide() { return !DOWN ? 90u : is_iq3<SRC>() ? 330u : 190u; }
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
 __global__ __launch_bounds__(staged_threads(SETS, KP)) void staged_tiles_kernel(StagedArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t entries[kEntryBytes];   // static: table reads take immediate offsets
     __shared__ __attribute__((aligned(16))) uint32_t signs[sign_bytes<SRC>() / 4u + 4u];
     __shared__ __attribute__((aligned(16))) float part[4u * KP * staged_nrt(KP) * 2u * 256u];
     const uint32_t n0 = a.n_tiles[0], n1 = a.n_tiles[1], n2 = a.n_tiles[2];      // (one trip)
-    const bool few = n1 < kFewWide;
+    const bool few = n1 < few_wide<SRC, DOWN>();
     if (SETS == 2 && few) return;
     const uint32_t tid = threadIdx.x, l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
     const uint32_t units = (SETS == 2 ? n1 : few ? n0 : n2) * (a.rows / ((DOWN ? 32u : 16u) * staged_nrt(KP)));
@@ -352,20 +353,20 @@ hipError_t launch_staged_list(const StagedArgs &a, uint32_t grid, hipStream_t s)
     REDHIP_LAUNCH((staged_tiles_kernel<SRC, DOWN, SETS, KP>), dim3(grid), dim3(staged_threads(SETS, KP)), 0, s, a);
     return hipGetLastError();
 }
-// wide: the chunk can have tiles of more than 16 pairs
+// wide: wide tiles that the chunk can have at most
 template <int SRC, bool DOWN, uint32_t KP>
-hipError_t launch_staged_lists(const StagedArgs &a, uint32_t grid, bool wide, hipStream_t s) {
-    const hipError_t e = wide ? launch_staged_list<SRC, DOWN, 2, KP>(a, grid, s) : hipSuccess;
+hipError_t launch_staged_lists(const StagedArgs &a, uint32_t grid, uint32_t wide, hipStream_t s) {
+    const hipError_t e = wide >= few_wide<SRC, DOWN>() ? launch_staged_list<SRC, DOWN, 2, KP>(a, grid, s) : hipSuccess;
     return e == hipSuccess ? launch_staged_list<SRC, DOWN, 1, KP>(a, grid, s) : e;
 }
 template <int SRC>
-hipError_t staged_gateup(const StagedArgs &a, uint32_t hidden, uint32_t grid, bool wide, hipStream_t s) {
+hipError_t staged_gateup(const StagedArgs &a, uint32_t hidden, uint32_t grid, uint32_t wide, hipStream_t s) {
     return hidden == 512u    ? launch_staged_lists<SRC, false, 2>(a, grid, wide, s)
            : hidden == 1024u ? launch_staged_lists<SRC, false, 4>(a, grid, wide, s)
                              : launch_staged_lists<SRC, false, 8>(a, grid, wide, s);
 }
 template <int SRC>
-hipError_t staged_down(const StagedArgs &a, uint32_t ffn, uint32_t grid, bool wide, hipStream_t s) {
+hipError_t staged_down(const StagedArgs &a, uint32_t ffn, uint32_t grid, uint32_t wide, hipStream_t s) {
     if (ffn == 256u) return launch_staged_lists<SRC, true, 1>(a, grid, wide, s);
     if (ffn == 512u) return launch_staged_lists<SRC, true, 2>(a, grid, wide, s);
     if constexpr (layout<SRC>() == L_TILED) return hipErrorInvalidValue;      // (tile-major copies are made for ffn <= 512)
@@ -399,9 +400,9 @@ uint32_t staged_grid(const StagedChunk &c) {
     const uint32_t bound = 4u * prefill_tile_bound(c.ntok, c.top_k, c.n_expert);
     return bound < 256u ? bound : 256u;
 }
-bool staged_wide(const StagedChunk &c) {               // a wide tile has 17 pairs or more
+uint32_t staged_wide(const StagedChunk &c) {           // a wide tile has 17 pairs or more
     const uint32_t most = c.ntok * c.top_k / (kPrefillTile + 1u) + c.tl.shared_ntok / (kPrefillTile + 1u);
-    return (c.wide_tiles < most ? c.wide_tiles : most) >= kFewWide;
+    return c.wide_tiles < most ? c.wide_tiles : most;
 }
 
 }  // namespace
@@ -424,7 +425,7 @@ hipError_t launch_staged_gateup(const StagedMatrices &m, const StagedChunk &c, c
     a.xexp = xexp;
     a.act = act;
     const uint32_t grid = staged_grid(c);
-    const bool wide = staged_wide(c);
+    const uint32_t wide = staged_wide(c);
     prof_set_stage(ST_PREFILL_GATEUP);
     switch (staged_src(m.type, m.layout)) {
         case S_XXS: return staged_gateup<S_XXS>(a, hidden, grid, wide, s);
@@ -445,7 +446,7 @@ hipError_t launch_staged_down(const StagedMatrices &m, const StagedChunk &c, con
     a.tmp = tmp;
     a.sh_tmp = sh_tmp;
     const uint32_t grid = staged_grid(c);
-    const bool wide = staged_wide(c);
+    const uint32_t wide = staged_wide(c);
     prof_set_stage(ST_PREFILL_DOWN);
     switch (staged_src(m.type, m.layout)) {
         case S_XXS: return staged_down<S_XXS>(a, ffn, grid, wide, s);

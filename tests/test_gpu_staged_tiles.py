@@ -48,11 +48,11 @@ def test_pool_slots(tmp_path, grids, layout, hidden, ffn, many_wide):
     n_expert, top_k = 12, 4
     c = Case(tmp_path, grids, layout, hidden=hidden, ffn=ffn, n_expert=n_expert, seed=811)
     rng = np.random.default_rng(3)
-    if many_wide:      # 12 experts with 133 or 134 pairs: 48 or more tiles of 32, remainders of 5 and 6; one expert with a wide remainder
-        ntok = 402
-        counts = [134] * n_expert
-        counts[0] += 23
-        counts[1] -= 23
+    if many_wide:      # 12 experts with about 900 pairs: enough tiles of 32 for the wide launches of every format, remainders of 4, two wide remainders
+        ntok = 2700
+        counts = [900] * n_expert
+        counts[0] += 15
+        counts[1] -= 15
     else:
         counts, ntok = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 3, 0], 73
     ids = routing_with(counts, ntok, top_k, rng)

@@ -873,6 +873,8 @@ __device__ __forceinline__ uint32_t block_scan_1024(uint32_t v, uint32_t *wave_t
 // compute unit, so the instruction count is what it costs: the token of a pair comes from a multiply-high by
 // ceil(2^32 / top_k) (exact while pairs * top_k < 2^32), and with PREFIX the bit counts of the words below a token's word come
 // from a table made once per expert (which also yields the expert's pair count) instead of a loop per pair.
+// An expert's words lie an odd number of words behind the last one's: the pairs of a wave belong to tokens near each other, so they all
+// use the same word of their experts, and with sixteen words per expert (512 tokens) these were in a few LDS banks.
 template <bool PREFIX>
 __global__ __launch_bounds__(1024) void group_pairs_kernel(const uint32_t *ids, const float *weights, uint32_t ntok, uint32_t top_k, uint32_t top_k_magic,
                                                            uint32_t n_expert, uint32_t *uid, uint32_t *expert_start,
@@ -880,16 +882,16 @@ __global__ __launch_bounds__(1024) void group_pairs_kernel(const uint32_t *ids, 
                                                            uint32_t *n_unique, uint32_t *status, uint32_t cache_ids, TileLists tiles) {
     extern __shared__ uint32_t sm[];
     __shared__ uint32_t tile_tot[3][16];
-    const uint32_t words = (ntok + 31u) / 32u, P = ntok * top_k, tid = threadIdx.x;
+    const uint32_t words = (ntok + 31u) / 32u, stride = words | 1u, P = ntok * top_k, tid = threadIdx.x;
     uint32_t *first = sm;                          // [n_expert]
     uint32_t *count = first + n_expert;            // [n_expert]
     uint32_t *dense = count + n_expert;            // [n_expert]
     uint32_t *start = dense + n_expert;            // [n_expert + 1] by dense index
     uint32_t *uid_l = start + n_expert + 1u;       // [1024] experts by dense index (n_expert <= 1024)
     uint32_t *wave_tot = uid_l + 1024u;            // [17]
-    uint32_t *member = wave_tot + 17u;             // [n_expert][words]
-    uint32_t *below = member + n_expert * words;   // [n_expert][words] when PREFIX: members in the words before this one
-    uint32_t *ids_l = cache_ids ? below + (PREFIX ? n_expert * words : 0u) : nullptr;      // [P] the clamped ids, when LDS has room: the later passes need no second trip to device memory
+    uint32_t *member = wave_tot + 17u;             // [n_expert][stride]
+    uint32_t *below = member + n_expert * stride;  // [n_expert][stride] when PREFIX: members in the words before this one
+    uint32_t *ids_l = cache_ids ? below + (PREFIX ? n_expert * stride : 0u) : nullptr;      // [P] the clamped ids, when LDS has room: the later passes need no second trip to device memory
     auto token_of = [&](uint32_t p) { return top_k == 1u ? p : __umulhi(p, top_k_magic); };
     // the ids are the caller's: clamped into the tables (reported once, in the first pass)
     auto id_of = [&](uint32_t p) { if (ids_l) return ids_l[p]; const uint32_t e = ids[p]; return e < n_expert ? e : n_expert - 1u; };
@@ -908,14 +910,14 @@ __global__ __launch_bounds__(1024) void group_pairs_kernel(const uint32_t *ids, 
         }
     }
     for (uint32_t i = tid; i < n_expert; i += 1024u) { first[i] = 0xffffffffu; count[i] = 0u; dense[i] = 0u; }
-    for (uint32_t i = tid; i < n_expert * words; i += 1024u) member[i] = 0u;
+    for (uint32_t i = tid; i < n_expert * stride; i += 1024u) member[i] = 0u;
     __syncthreads();
     auto enter = [&](uint32_t p, uint32_t raw) {
         const uint32_t e = guarded_id(raw, n_expert, status), t = token_of(p);
         if (ids_l) ids_l[p] = e;
         atomicMin(&first[e], p);
         if constexpr (!PREFIX) atomicAdd(&count[e], 1u);
-        if ((atomicOr(&member[e * words + (t >> 5)], 1u << (t & 31u)) & (1u << (t & 31u))) && status) atomicOr(status, 2u);      // the token names this expert twice
+        if ((atomicOr(&member[e * stride + (t >> 5)], 1u << (t & 31u)) & (1u << (t & 31u))) && status) atomicOr(status, 2u);      // the token names this expert twice
         return e;
     };
     if (in_regs) {
@@ -928,7 +930,7 @@ __global__ __launch_bounds__(1024) void group_pairs_kernel(const uint32_t *ids, 
     if constexpr (PREFIX) {
         for (uint32_t e = tid; e < n_expert; e += 1024u) {
             uint32_t run = 0u;
-            for (uint32_t w = 0; w < words; ++w) { below[e * words + w] = run; run += __popc(member[e * words + w]); }
+            for (uint32_t w = 0; w < words; ++w) { below[e * stride + w] = run; run += __popc(member[e * stride + w]); }
             count[e] = run;
         }
     }
@@ -951,9 +953,9 @@ __global__ __launch_bounds__(1024) void group_pairs_kernel(const uint32_t *ids, 
     __syncthreads();
     auto place = [&](uint32_t p, uint32_t e, float wt) {
         const uint32_t t = token_of(p);
-        const uint32_t *bits = member + e * words;
+        const uint32_t *bits = member + e * stride;
         uint32_t rank = __popc(bits[t >> 5] & ((1u << (t & 31u)) - 1u));
-        if constexpr (PREFIX) rank += below[e * words + (t >> 5)];
+        if constexpr (PREFIX) rank += below[e * stride + (t >> 5)];
         else for (uint32_t w = 0; w < (t >> 5); ++w) rank += __popc(bits[w]);
         const uint32_t pos = start[dense[e]] + rank;
         pair_token[pos] = t;
@@ -1096,7 +1098,7 @@ __global__ __launch_bounds__(256) void group_count_kernel(const uint32_t *ids, u
 
 __global__ __launch_bounds__(1024) void group_plan_kernel(GroupScratch gs, uint32_t nb, uint32_t n_expert, uint32_t P, uint32_t *uid, uint32_t *expert_start,
                                                           uint32_t *n_unique, TileLists tiles) {
-    __shared__ uint32_t key_l[1024], cnt[1024], uid_l[1024], start[1025], wave_tot[17];
+    __shared__ uint32_t firsts[1024], below[1024], cnt[1024], uid_l[1024], start[1025], wave_tot[17];
     __shared__ uint32_t tile_tot[3][16];
     const uint32_t tid = threadIdx.x;
     uint32_t my_key = 0u, total = 0u;
@@ -1114,14 +1116,25 @@ __global__ __launch_bounds__(1024) void group_plan_kernel(GroupScratch gs, uint3
             }
         }
     }
-    key_l[tid] = my_key;
     cnt[tid] = total;
-    __syncthreads();
-    // first-appearance order: the experts with an earlier first pair (a larger key) come before this one
-    uint32_t d = 0u;
-    if (my_key) for (uint32_t e = 0; e < n_expert; ++e) d += key_l[e] > my_key ? 1u : 0u;
-    uint32_t U = 0u;
-    (void)block_scan_1024(my_key ? 1u : 0u, wave_tot, U);
+    // first-appearance order: an expert's number is how many first pairs lie before its own - a bitmap of them and the counts below its words,
+    // 32768 pairs at a time (a comparison with every other expert's first pair instead: several hundred steps per thread)
+    const uint32_t first = ~my_key;
+    uint32_t d = 0u, U = 0u;
+    for (uint32_t base = 0u; base < P; base += 32768u) {
+        const bool here = my_key && first - base < 32768u;
+        const uint32_t word = here ? (first - base) >> 5 : 0u, bit = here ? first & 31u : 0u;
+        firsts[tid] = 0u;
+        __syncthreads();
+        if (here) atomicOr(&firsts[word], 1u << bit);
+        __syncthreads();
+        uint32_t n = 0u;
+        below[tid] = block_scan_1024(__popc(firsts[tid]), wave_tot, n);
+        __syncthreads();
+        if (here) d = U + below[word] + __popc(firsts[word] & ((1u << bit) - 1u));
+        U += n;
+        __syncthreads();
+    }
     if (my_key) { uid_l[d] = tid; uid[d] = tid; }
     __syncthreads();
     uint32_t all = 0u;
@@ -1182,9 +1195,9 @@ hipError_t launch_group_pairs(const uint32_t *ids, const float *weights, uint32_
     if (!ntok || !top_k || !n_expert || n_expert > 1024u || (uint64_t)ntok * top_k * top_k >= (1ull << 32)) return hipErrorInvalidValue;
     const TileLists tl = tiles ? *tiles : TileLists{};
     const uint32_t words = (ntok + 31u) / 32u;
-    const size_t lds = sizeof(uint32_t) * ((size_t)4u * n_expert + 1u + 1024u + 17u + (size_t)n_expert * words);
+    const size_t lds = sizeof(uint32_t) * ((size_t)4u * n_expert + 1u + 1024u + 17u + (size_t)n_expert * (words | 1u));
     constexpr size_t kGroupDynLds = 159u * 1024u;      // (the kernel has a little static LDS beside it)
-    const size_t lds_prefix = lds + sizeof(uint32_t) * (size_t)n_expert * words;
+    const size_t lds_prefix = lds + sizeof(uint32_t) * (size_t)n_expert * (words | 1u);
     const uint32_t magic = (uint32_t)(((1ull << 32) + top_k - 1u) / top_k);      // top_k == 1 needs none (and would not fit)
     static bool attr_set = false;
     if (!attr_set) {

@@ -191,3 +191,18 @@ def test_grouping_matches_host_sort():
     for a, b in zip(got, want):
         assert np.array_equal(a.cpu().numpy().view(b.dtype), b)
     m.close()
+
+
+@pytest.mark.parametrize("ntok,E,K", [(97, 512, 10), (256, 512, 10), (480, 300, 7), (512, 1024, 4), (2049, 512, 16), (2100, 600, 16)])
+def test_grouping_numbers_late_experts(ntok, E, K):
+    """even and odd counts of bitmap words per expert; chunks of more than 32768 pairs, with experts that first appear behind them"""
+    from dwarfstar_red_lite_amd import moe
+    m = moe.ResidentMoe(synth.layer_config(hidden=256, ffn=256, n_expert=E, top_k=K), n_layer=1, max_tokens=ntok)
+    rng = np.random.default_rng(ntok)
+    ids = np.argsort(rng.random((ntok, E - 40)), axis=1)[:, :K].astype(np.uint32)
+    ids[-1] = E - 1 - np.arange(K)                      # never named before
+    ids[ntok // 2] = E - 40 + np.arange(K)
+    w = rng.random((ntok, K)).astype(np.float32)
+    for got, want in zip(m.group(dev(ids.astype(np.int32)), dev(w)), orc.group_pairs(ids, w, E)):
+        assert np.array_equal(got.cpu().numpy().view(want.dtype), want)
+    m.close()

@@ -15,8 +15,8 @@
 //
 // K is cut into KP blocks of 256 columns, and NRT row tiles of 16 rows are in work beside each other (KP * NRT = 8; 6 with three
 // blocks). A unit is two halves ("m") of 16 NRT rows: the gate and the up rows of 16 NRT FFN columns, or 32 NRT rows of a down matrix.
-// A wave keeps the activations of its block for the whole tile in registers (fp16 hi and lo halves, 22 significant bits) and the rows of
-// the next two units on their way; the blocks meet in LDS, one barrier per two units. Tiles of up to 16 pairs run sixteen waves, one half
+// A wave keeps the activations of its block for the whole tile in registers (fp16 halves hi + lo 2^-11, 22 significant bits of every value
+// down to 2^-28 of the largest) and the rows of the next two units on their way; the blocks meet in LDS, one barrier per two units. Tiles of up to 16 pairs run sixteen waves, one half
 // each (64 registers of activations, four waves per SIMD: the reads and the arithmetic of different waves overlap), tiles of 17 .. 32
 // pairs eight waves with both halves and two sets of pairs per decoded weight, as a launch of their own. The SwiGLU activations go to
 // the down kernel as f32, so work is cut at any unit, not at groups of columns that share an exponent; the down kernel splits them per
@@ -65,7 +65,7 @@ struct TileInfo { uint64_t mat; uint32_t p0, n; };      // mat: distance of the 
 // units u0 .. u1 - 1 (unit = tile * units per tile + unit of the tile) of a tile list; SETS sets of 16 pairs per tile
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
 __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t *tile_expert, const uint32_t *tile_pair0, const uint32_t *tile_n, uint32_t u0,
-                                             uint32_t u1, float *part, TileInfo *tiles, uint32_t *tokens, uint8_t *entries, uint32_t *signs, const LaneTables &lt) {
+                                             uint32_t u1, float *part, float *scales, TileInfo *tiles, uint32_t *tokens, uint8_t *entries, uint32_t *signs, const LaneTables &lt) {
     constexpr uint32_t NRT = staged_nrt(KP), WV = KP * NRT, T = staged_threads(SETS, KP), M = SETS == 1 ? 1u : 2u;      // M: halves per wave
     constexpr uint32_t K = 256u * KP, seg_rows = 16u * NRT, tile_bytes = 16u * KP * src_block<SRC>();
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
@@ -105,8 +105,20 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
         const TileInfo ti = tiles[tile - tile0];
         return TileInfo{uniform64(ti.mat), (uint32_t)__builtin_amdgcn_readfirstlane(ti.p0), (uint32_t)__builtin_amdgcn_readfirstlane(ti.n)};
     };
+    // Precision. The matrix unit rounds a sum four times per instruction (once per eight products), so what a block's sum loses goes with the
+    // length of its chain of instructions: the low halves have a chain of their own, and the high ones one per kChain steps, added up in
+    // f32 (in the registers, or where these are full in the LDS that takes the block's sum anyway). A chunk of normal rows comes out 1.9e-7
+    // off (f32 multiplications: 2.1e-7); with one chain for everything it was 2.9e-7, in 3 .. 5 % less time. Packed rows (all-IQ2_XXS, ffn
+    // above 512) take two steps per chain: 1.75e-7 instead of 1.9e-7, 5 % of the time.
+    constexpr uint32_t kChain = layout<SRC>() == L_ROWS ? 2u : 4u;
+    constexpr bool kSumInLds = SETS == 1 ? SRC == S_IQ3 : fmt<SRC>() != F_XXS || layout<SRC>() == L_ROWS;
+    // units on their way: two, one where the registers hold no second (a spill to scratch memory would be counted among the loads that the waits count)
+    constexpr uint32_t kCarried = SRC == S_IQ3 || (SETS == 2 && SRC == S_M) ? 1u : 2u;
     H8 xa[SETS][8], xb[SETS][8];
-    float ps[SETS][4];
+    // Powers of two that the products of a pair are multiplied with. Down: of this wave's block. Gate/up: of the token, so the sums over the
+    // blocks take them; a tile's stand in row tile % 4: a tile has two units or
+    // more, so the first wave is at most two tiles ahead of the one that still adds sums up.
+    float *pair_scale = scales + (DOWN ? wave * 16u * SETS : 0u);
     const auto load_tile = [&](uint32_t tile, uint32_t p0, uint32_t n) {
 #pragma unroll
         for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
@@ -123,10 +135,6 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                     xa[s][g].u = *reinterpret_cast<const uint4 *>(hp + step_column<SRC>(g, lq));
                     xb[s][g].u = *reinterpret_cast<const uint4 *>(lp + step_column<SRC>(g, lq));
                 }
-                // the low halves are stored times 2^11: back to their own scale (exact, the largest |x| of a token sits in [2^13, 2^14)), so that a
-                // product's high and low parts add up in one accumulator
-#pragma unroll
-                for (uint32_t g = 0; g < 8u; ++g) xb[s][g].v = xb[s][g].v * (_Float16)4.8828125e-4f;
                 if (s + 1u == (uint32_t)SETS) __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): waited for here, once per tile, not (by count) where the loop uses them
             } else {
                 // f32 activations of pair p, columns of this wave's K part: one exponent for them, then the fp16 halves
@@ -158,7 +166,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                         const float t = f[k] * inv;
                         const _Float16 h = (_Float16)t;
                         hi.e[k] = h;
-                        lo.e[k] = (_Float16)(t - (float)h);
+                        lo.e[k] = (_Float16)((t - (float)h) * 2048.0f);
                     }
                     // group by group (the compiler otherwise works on several at once and spills)
                     asm volatile("" : "+v"(hi.u.x), "+v"(hi.u.y), "+v"(hi.u.z), "+v"(hi.u.w), "+v"(lo.u.x), "+v"(lo.u.y), "+v"(lo.u.z), "+v"(lo.u.w));
@@ -166,17 +174,17 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                     xb[s][g].u = lo.u;
                 }
             }
-#pragma unroll
-            for (uint32_t t = 0; t < 4u; ++t) ps[s][t] = __shfl(scale, (int)(4u * lq + t), 64);
+            pair_scale[(DOWN ? 0u : (tile & 3u) * 16u * SETS) + i] = scale;      // (every lane and wave that has pair i writes the same)
         }
     };
     // partial sums of the waves: [row tile, K part][m][set][lane] float4
     constexpr uint32_t kWavePart = 2u * SETS * 256u, kPart = WV * kWavePart;      // (kPart: of a unit)
-    struct Done { uint32_t j, p0, n; };                    // a unit whose partial sums are in LDS
+    struct Done { uint32_t tile, j, p0, n; };              // a unit whose partial sums are in LDS
     // The sums of UNITS units (w[0], and w[1] behind it). No wave and no lane may skip a store: the loads of the next units are in flight
     // behind it, and the compiler, which waits for them by counting memory operations in order, can count only what every path issues
     // (with a branch around it, every unit waited for the newest of its loads). Pairs beyond a tile's n fall out of the buffer's range.
     const auto tile_buffer = [&](float *base, uint32_t n) { return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)(n * a.rows * 4u), 0x00027000); };
+    using Sum = std::conditional_t<(KP > 2u), double, float>;      // (a row's partial sums are added here one after the other)
     const auto reduce = [&](auto units, const Done *w, const float *pt) {
         constexpr uint32_t UNITS = decltype(units)::value;
         const uint32_t t = each_trip(tid);
@@ -192,7 +200,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                     const uint32_t it = N % T ? min(base + t, N - 1u) : base + t;
                     const uint32_t at = (it & (PB - 1u)) * V, b = it / PB, set = b & (SETS - 1u), m = (b / SETS) & 1u, slot = b / (2u * SETS);
                     const float *src = pt + un * kPart + slot * KP * kWavePart + (m * SETS + set) * 256u + at;
-                    float s[V];
+                    Sum s[V];
 #pragma unroll
                     for (uint32_t v = 0; v < V; ++v) s[v] = src[v];
 #pragma unroll
@@ -201,7 +209,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                         for (uint32_t v = 0; v < V; ++v) s[v] += src[k * kWavePart + v];
                     const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u), off = 4u * (i * a.rows + w[un].j * 2u * seg_rows + m * seg_rows + 16u * slot + ((at >> 2) & 15u));
 #pragma unroll
-                    for (uint32_t v = 0; v < V; ++v) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s[v]), buf, off + 4u * v * a.rows, 0, 0);
+                    for (uint32_t v = 0; v < V; ++v) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((float)s[v]), buf, off + 4u * v * a.rows, 0, 0);
                 }
             }
         } else {
@@ -213,7 +221,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 const uint32_t ln = t & 63u, e = base + (L == 1u ? t : (t >> 6) * (64u / L) + (ln & (64u / L - 1u))), k0 = L == 1u ? 0u : (ln / (64u / L)) * (KP / L);
                 const uint32_t at = e & 255u, b = (e >> 8) % (SETS * NRT), un = (e >> 8) / (SETS * NRT), set = b & (SETS - 1u), slot = b / SETS;
                 const float *src = pt + un * kPart + (slot * KP + k0) * kWavePart + set * 256u + at;
-                float s0 = src[0], s1 = src[SETS * 256u];
+                Sum s0 = src[0], s1 = src[SETS * 256u];
 #pragma unroll
                 for (uint32_t k = 1; k < KP / L; ++k) {
                     s0 += src[k * kWavePart];
@@ -226,9 +234,10 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                 const Done d = uw ? w[UNITS - 1u] : w[0];
                 const auto buf = tile_buffer(a.act + (uint64_t)d.p0 * a.rows, d.n);
                 const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u);
+                const float scale = pair_scale[(d.tile & 3u) * 16u * SETS + i], g = (float)s0 * scale, up = (float)s1 * scale;
                 // (of the lanes that share an element the first stores; the others' offset lies beyond every buffer)
                 const uint32_t off = k0 == 0u ? 4u * (i * a.rows + d.j * seg_rows + 16u * slot + ((at >> 2) & 15u)) : 0x7fffffffu;
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((s0 / (1.0f + expf(-s0))) * s1), buf, off, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((g / (1.0f + expf(-g))) * up), buf, off, 0, 0);
             }
         }
     };
@@ -243,31 +252,42 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
     };
     // multiplies the unit whose rows are in c into partial sums at pt and requests the unit two after it in their place
     const auto unit = [&](uint32_t u, Carried &c, float *pt) {
-        float4_t acc[M][SETS];
+        float4_t acc[M][SETS], low[M][SETS], sum[M][SETS];
         float d[M];
 #pragma unroll
         for (uint32_t m = 0; m < M; ++m) {
             d[m] = quarter_d<SRC>(c.d[m]);
 #pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) acc[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) acc[m][s] = low[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
-        Entry e0[M], e1[M];
+        float *mine = pt + w8 * kWavePart + m_first * SETS * 256u + 4u * lane;
+        Entry e[M];
         half2_t f[M];
 #pragma unroll
-        for (uint32_t m = 0; m < M; ++m) { e0[m] = fetch_entry<SRC>(c.v[m], 0u, lt); e1[m] = fetch_entry<SRC>(c.v[m], 1u, lt); }
+        for (uint32_t m = 0; m < M; ++m) e[m] = fetch_entry<SRC>(c.v[m], 0u, lt);
 #pragma unroll
         for (uint32_t s8 = 0; s8 < 8u; ++s8) {
-            // table reads run two steps ahead of the arithmetic
+            // table reads run a step ahead of the products (two steps ahead takes five registers more per row and was no quicker)
             __builtin_amdgcn_sched_barrier(0);
             half8_t w[M];
 #pragma unroll
             for (uint32_t m = 0; m < M; ++m) {
                 if constexpr (steps_per_scale<SRC>() != 0u) { if (s8 % steps_per_scale<SRC>() == 0u) f[m] = step_scale<SRC>(c.v[m], s8); }
-                w[m] = finish_entry<SRC>(s8 & 1u ? e1[m] : e0[m], f[m]);
-                if (s8 + 2u < 8u) { if (s8 & 1u) e1[m] = fetch_entry<SRC>(c.v[m], s8 + 2u, lt); else e0[m] = fetch_entry<SRC>(c.v[m], s8 + 2u, lt); }
+                w[m] = finish_entry<SRC>(e[m], f[m]);
+                if (s8 < 7u) e[m] = fetch_entry<SRC>(c.v[m], s8 + 1u, lt);
             }
             __builtin_amdgcn_sched_barrier(0);
             if (s8 == 6u) request_next(c);                 // (the quarters' last use is behind)
+            if (s8 && s8 % kChain == 0u) {                 // put the sums so far aside
+#pragma unroll
+                for (uint32_t m = 0; m < M; ++m)
+#pragma unroll
+                    for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
+                        float4_t &so_far = kSumInLds ? *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) : sum[m][s];
+                        so_far = s8 == kChain ? acc[m][s] : so_far + acc[m][s];
+                        acc[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+            }
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
@@ -275,24 +295,27 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
-                for (uint32_t m = 0; m < M; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[s][s8].v, w[m], acc[m][s], 0, 0, 0);
+                for (uint32_t m = 0; m < M; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[s][s8].v, w[m], low[m][s], 0, 0, 0);
         }
-        float *mine = pt + w8 * kWavePart + m_first * SETS * 256u + 4u * lane;
 #pragma unroll
         for (uint32_t m = 0; m < M; ++m)
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
+                float4_t *at = reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u);
+                if constexpr (kSumInLds) sum[m][s] = *at;
+                float4_t factor = {d[m], d[m], d[m], d[m]};
+                if constexpr (DOWN) factor *= *reinterpret_cast<const float4_t *>(pair_scale + 16u * s + 4u * q);
 #pragma unroll
-                for (int t = 0; t < 4; ++t) acc[m][s][t] *= d[m] * ps[s][t];
-                *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) = acc[m][s];
+                for (int t = 0; t < 4; ++t) acc[m][s][t] = fmaf(low[m][s][t], 4.8828125e-4f, sum[m][s][t] + acc[m][s][t]) * factor[t];
+                *at = acc[m][s];
             }
-        const Done done{j, cur.p0, cur.n};
+        const Done done{tile, j, cur.p0, cur.n};
         if (++j == upt && u + 1u < u1) { j = 0u; cur = info_of(++tile); load_tile(tile, cur.p0, cur.n); }
         return done;
     };
-    Carried ca, cb;
-    request_next(ca);
-    request_next(cb);
+    Carried c[kCarried];
+#pragma unroll
+    for (uint32_t k = 0; k < kCarried; ++k) request_next(c[k]);
     load_tile(tile, cur.p0, cur.n);
     // narrow: two units per barrier, four buffers of partial sums; wide: one, two buffers (as large). A buffer is written again two
     // barriers after its sums were complete; whoever adds them has passed one in between.
@@ -302,12 +325,12 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
     float *pt = part;
     for (; u + 1u < u1; u += 2u) {
         Done w[2];
-        w[0] = unit(u, ca, pt);
+        w[0] = unit(u, c[0], pt);
         if constexpr (SETS == 2) {
             wave_lds_barrier();
             reduce(one, w, pt);
         }
-        w[1] = unit(u + 1u, cb, pt + kPart);
+        w[1] = unit(u + 1u, c[kCarried - 1u], pt + kPart);
         wave_lds_barrier();
         if constexpr (SETS == 2) reduce(one, w + 1, pt + kPart);
         else {
@@ -316,7 +339,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
         }
     }
     if (u < u1) {
-        const Done w = unit(u, ca, pt);
+        const Done w = unit(u, c[0], pt);
         wave_lds_barrier();
         reduce(one, &w, pt);
     }
@@ -343,9 +366,10 @@ __global__ __launch_bounds__(staged_threads(SETS, KP)) void staged_tiles_kernel(
     if (u0 >= u1) return;
     __shared__ TileInfo tiles[kTileInfos];
     __shared__ uint32_t tokens[DOWN ? 1u : kTileInfos * 16u * SETS];
+    __shared__ __attribute__((aligned(16))) float scales[(DOWN ? staged_threads(SETS, KP) / 64u : 4u) * 16u * SETS];
     const LaneTables lt{entries + (fmt<SRC>() == F_XS ? (tid & 7u) * 16u : fmt<SRC>() == F_M ? (tid & 1u) * 16u : 0u),
                         reinterpret_cast<const uint8_t *>(signs) + (is_iq3<SRC>() ? (tid & 3u) * 4u : fmt<SRC>() == F_M ? 0u : (tid & 15u) * 4u)};
-    staged_units<SRC, DOWN, SETS, KP>(a, a.tile_expert + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, part, tiles, tokens, entries, signs, lt);
+    staged_units<SRC, DOWN, SETS, KP>(a, a.tile_expert + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, part, scales, tiles, tokens, entries, signs, lt);
 }
 
 template <int SRC, bool DOWN, int SETS, uint32_t KP>

@@ -105,7 +105,9 @@ hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count
 // D[i = 4q .. 4q + 3][j = r]; the order of k does not matter as long as both operands agree).
 // What bounds it: the matrix pipe where a tile is large (64 x 64: 16 bytes of L2 per clock and compute unit; tiles of 32 x 32 for every size
 // needed 32, and waited for them), the number of workgroups where a chunk is small. So the tile is chosen by the launch (f32_tile_choice).
-// The order in which an output's products are added is the same for every tile.
+// The order in which an output's products are added is the same for every tile. The matrix unit rounds with every product, so the dense
+// products leave it after 32 columns and are added up in double: of a shared expert's 2048-column rows 0.9e-7 is lost instead of 3.5e-7 (and of
+// the output of an IQ1_M layer 1.6e-7 instead of 6e-7). A router keeps two plain chains: nothing but the selection hangs on its last bits.
 // SWIGLU: W holds gate rows, then as many up rows; two row blocks beside each other are the gate and the up rows of 16 columns, and out gets
 // silu(gate) * up of them: no pass of its own over the products.
 // Launches with xh get workgroups behind the tiles that write the fp16 halves of the activations (a wave per token, split_token) and multiply them
@@ -157,7 +159,7 @@ __device__ __forceinline__ void split_token(const float *gate_inp, const float *
             }
 }
 
-template <int MR, int MT, uint32_t WR, uint32_t WT, uint32_t SLICE, bool SWIGLU>
+template <int MR, int MT, uint32_t WR, uint32_t WT, uint32_t SLICE, bool SWIGLU, bool ROUTER>
 __global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w, const float *gate_inp, const float *x, float *out, uint32_t out_stride, _Float16 *xh,
                                                                   _Float16 *xl, int *xexp, uint32_t K, uint32_t n_rows, uint32_t ntok) {
     constexpr uint32_t BR = 16u * MR * WR, BT = 16u * MT * WT, T = 128u * WR * WT, P = SLICE / 4u, D = T / (2u * P), NW = BR / D, NX = BT / D;      // P pieces of 16 bytes per row, D rows per pass of the threads
@@ -210,11 +212,18 @@ __global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w
         if constexpr (N > 5u) *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + 5u * D][scol]) = st.v5;
     };
     const uint32_t mh = wave / (WR * WT), block = wave % (WR * WT), wr = block % WR, wt = block / WR;
-    float4_t acc[MR][MT][2];
+    constexpr int CH = ROUTER ? 2 : 1;
+    float4_t acc[MR][MT][CH];
+    double total[MR][MT][4];
 #pragma unroll
     for (int m = 0; m < MR; ++m)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) acc[m][t][0] = acc[m][t][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) acc[m][t][c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) total[m][t][i] = 0.0;
+        }
     const auto multiply = [&](uint32_t buf) {
 #pragma unroll
         for (uint32_t u = 0; u < SLICE / 16u; ++u) {
@@ -229,8 +238,19 @@ __global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w
                 for (int m = 0; m < MR; ++m)
 #pragma unroll
                     for (int t = 0; t < MT; ++t)
-                        acc[m][t][k & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k == 0 ? a[m].x : k == 1 ? a[m].y : k == 2 ? a[m].z : a[m].w,
-                                                                                k == 0 ? b[t].x : k == 1 ? b[t].y : k == 2 ? b[t].z : b[t].w, acc[m][t][k & 1], 0, 0, 0);
+                        acc[m][t][k % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(k == 0 ? a[m].x : k == 1 ? a[m].y : k == 2 ? a[m].z : a[m].w,
+                                                                                k == 0 ? b[t].x : k == 1 ? b[t].y : k == 2 ? b[t].z : b[t].w, acc[m][t][k % CH], 0, 0, 0);
+            if constexpr (!ROUTER)
+                if (u & 1u) {
+#pragma unroll
+                    for (int m = 0; m < MR; ++m)
+#pragma unroll
+                        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) total[m][t][i] += acc[m][t][0][i];
+                            acc[m][t][0] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                        }
+                }
         }
     };
     Staged s0, s1;
@@ -246,6 +266,14 @@ __global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w
         request(s1, rd + 3u < n_round ? rd + 3u : rd + 1u);
         multiply(1u);
     }
+    float4_t sum[MR][MT];
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[m][t][i] = ROUTER ? acc[m][t][0][i] + acc[m][t][CH - 1][i] : (float)total[m][t][i];
+        }
     // the odd slices' sums go through LDS to the waves that hold the even ones; SWIGLU with one row block per wave: then the up products to
     // the wave of their gate rows
     float4_t *meet = reinterpret_cast<float4_t *>(&lds[0][0][0][0]);
@@ -256,19 +284,19 @@ __global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w
 #pragma unroll
         for (int m = 0; m < MR; ++m)
 #pragma unroll
-            for (int t = 0; t < MT; ++t) meet[at(block, m, t)] = acc[m][t][0] + acc[m][t][1];
+            for (int t = 0; t < MT; ++t) meet[at(block, m, t)] = sum[m][t];
     }
     __syncthreads();
     if (mh == 0u) {
 #pragma unroll
         for (int m = 0; m < MR; ++m)
 #pragma unroll
-            for (int t = 0; t < MT; ++t) acc[m][t][0] = (acc[m][t][0] + acc[m][t][1]) + meet[at(block, m, t)];
+            for (int t = 0; t < MT; ++t) sum[m][t] += meet[at(block, m, t)];
     }
     if constexpr (SWIGLU && MR == 1) {
         if (mh == 0u && (wr & 1u)) {
 #pragma unroll
-            for (int t = 0; t < MT; ++t) meet[at(block, 0, t)] = acc[0][t][0];      // (its own place: nobody else reads it before)
+            for (int t = 0; t < MT; ++t) meet[at(block, 0, t)] = sum[0][t];      // (its own place: nobody else reads it before)
         }
         __syncthreads();
     }
@@ -279,7 +307,7 @@ __global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w
         if (tok >= ntok) continue;
         if constexpr (SWIGLU) {
             float4_t y;
-            const float4_t g = acc[0][t][0], u = MR == 1 ? meet[at(block + 1u, 0, t)] : acc[MR - 1][t][0];
+            const float4_t g = sum[0][t], u = MR == 1 ? meet[at(block + 1u, 0, t)] : sum[MR - 1][t];
 #pragma unroll
             for (int i = 0; i < 4; ++i) y[i] = (g[i] / (1.0f + expf(-g[i]))) * u[i];
             *reinterpret_cast<float4_t *>(out + (uint64_t)tok * out_stride + tile_r * (BR / 2u) + 16u * (MR == 1 ? wr / 2u : wr) + 4u * q) = y;
@@ -289,7 +317,7 @@ __global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w
 #pragma unroll
                 for (uint32_t i = 0; i < 4u; ++i) {
                     const uint32_t row = tile_r * BR + 16u * (MR * wr + m) + 4u * q + i;
-                    if (row < all_rows) out[(uint64_t)tok * out_stride + row] = acc[m][t][0][i];
+                    if (row < all_rows) out[(uint64_t)tok * out_stride + row] = sum[m][t][i];
                 }
         }
     }
@@ -297,7 +325,7 @@ __global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w
 
 // The largest tile that costs no more rounds of the device (256 compute units, workgroups of equal length) than a quarter above the best
 // tile: large tiles read less, small ones fill the device when a chunk has few outputs.
-template <bool SWIGLU>
+template <bool SWIGLU, bool ROUTER>
 hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out, uint32_t out_stride, void *xh, void *xl,
                      int *xexp, hipStream_t s) {
     if (!ntok || !K || K % 256u || !n_rows || !w || !x || !out || (SWIGLU && n_rows % 128u)) return hipErrorInvalidValue;
@@ -315,10 +343,10 @@ hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uin
     if (n[pick] + split_wgs > 0x7fffffffull) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)n[pick] + split_wgs), block(64u * waves);
     _Float16 *h = static_cast<_Float16 *>(xh), *l = static_cast<_Float16 *>(xl);
-    if (pick == 0) REDHIP_LAUNCH((f32_tiles_kernel<2, 2, 2u, 2u, 32u, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
-    else if (pick == 1) REDHIP_LAUNCH((f32_tiles_kernel<2, 1, 2u, 2u, 32u, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
-    else if (pick == 2) REDHIP_LAUNCH((f32_tiles_kernel<1, 1, 2u, 2u, 64u, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
-    else REDHIP_LAUNCH((f32_tiles_kernel<1, 1, 2u, 1u, 64u, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    if (pick == 0) REDHIP_LAUNCH((f32_tiles_kernel<2, 2, 2u, 2u, 32u, SWIGLU, ROUTER>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    else if (pick == 1) REDHIP_LAUNCH((f32_tiles_kernel<2, 1, 2u, 2u, 32u, SWIGLU, ROUTER>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    else if (pick == 2) REDHIP_LAUNCH((f32_tiles_kernel<1, 1, 2u, 2u, 64u, SWIGLU, ROUTER>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    else REDHIP_LAUNCH((f32_tiles_kernel<1, 1, 2u, 1u, 64u, SWIGLU, ROUTER>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
     return hipGetLastError();
 }
 
@@ -326,16 +354,16 @@ hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uin
 // row behind the matrix; xh / xl / xexp (optional): also write the fp16 halves of x
 hipError_t launch_f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out,
                             uint32_t out_stride, void *xh, void *xl, int *xexp, hipStream_t s) {
-    return f32_tiles<false>(w, extra_row, x, ntok, K, n_rows, out, out_stride, xh, xl, xexp, s);
+    return f32_tiles<false, false>(w, extra_row, x, ntok, K, n_rows, out, out_stride, xh, xl, xexp, s);
 }
 // act[tok][c] = silu(W[c] . x[tok]) * (W[ffn + c] . x[tok])
 hipError_t launch_f32_swiglu_tiles(const float *w, const float *x, uint32_t ntok, uint32_t K, uint32_t ffn, float *act, hipStream_t s) {
-    return f32_tiles<true>(w, nullptr, x, ntok, K, 2u * ffn, act, ffn, nullptr, nullptr, nullptr, s);
+    return f32_tiles<true, false>(w, nullptr, x, ntok, K, 2u * ffn, act, ffn, nullptr, nullptr, nullptr, s);
 }
 
 hipError_t launch_router_f32_tiles(const float *w, const float *gate_inp, const float *x, uint32_t ntok, uint32_t hidden, uint32_t n_expert,
                                    float *logits, void *xh, void *xl, int *xexp, hipStream_t s) {
-    return launch_f32_tiles(w, gate_inp, x, ntok, hidden, n_expert, logits, n_expert + 1u, xh, xl, xexp, s);
+    return f32_tiles<false, true>(w, gate_inp, x, ntok, hidden, n_expert, logits, n_expert + 1u, xh, xl, xexp, s);
 }
 
 }  // namespace redhip

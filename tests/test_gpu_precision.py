@@ -86,3 +86,27 @@ def test_small_activations_beside_large_ones(tmp_path, grids, layout, wide, monk
     pick = rng.choice(ntok, 24, replace=False)
     assert pool_chunk(c, hidden, ffn, counts, ntok, 4, x, rng, pick) <= F32_CHUNK
     c.pool.close()
+
+
+@pytest.mark.parametrize("layout", ["f2", "m"])
+def test_wide_experts_of_a_mixed_layer(layout, grids):
+    """ffn 768: routed experts on raw rows, the shared expert's dense f32 rows on the matrix unit's f32 products (on IQ1_M layers the larger part of the output)"""
+    H, F, E, K, ntok = 2048, 768, 16, 4, 40
+    cfg = synth.layer_config(hidden=H, ffn=F, n_expert=E, top_k=K, layout=layout)
+    lay = synth.make_layer(61, cfg)
+    m = moe_api.ResidentMoe(cfg, n_layer=1, max_tokens=ntok)
+    m.load_layer(0, lay)
+    rng = np.random.default_rng(62)
+    x = synth.normed_x(rng, ntok, H)
+    ids = np.stack([rng.permutation(E)[:K] for _ in range(ntok)]).astype(np.uint32)
+    w = rng.random((ntok, K)).astype(np.float32)
+    w /= w.sum(axis=1, keepdims=True)
+    got = m.experts(0, torch.from_numpy(x).cuda(), torch.from_numpy(ids.astype(np.int32)).cuda(), torch.from_numpy(w).cuda()).cpu().numpy()
+    pick = range(0, ntok, 4)
+    want = []
+    for t in pick:
+        y = sum(float(w[t, k]) * orc.expert_ffn(cfg["gate_up_type"], cfg["down_type"], lay["gate"][e], lay["up"][e], lay["down"][e], H, F, x[t]) for k, e in enumerate(ids[t]))
+        gate = 1.0 / (1.0 + np.exp(-float(np.dot(lay["sh_gate_inp"].astype(np.float64), x[t].astype(np.float64)))))
+        want.append(y + gate * orc.expert_ffn(cfg["sh_gate_up_type"], cfg["sh_down_type"], lay["sh_gate"], lay["sh_up"], lay["sh_down"], H, F, x[t]))
+    assert rel(got[list(pick)], np.stack(want)) <= F32_CHUNK
+    m.close()

@@ -7,7 +7,7 @@
 // built while the rows are on their way, and no wave has more than one or two units: 16 rows times a block of 256 columns. The products run on v_mfma_f32_16x16x32_f16 with the
 // weights as one operand, a quarter block of its row per lane (redhip_quarter.h); three of the 16 columns of the other operand hold the
 // activation as fp16 terms x = t0 + t1 2^-11 + t2 2^-22, which is every bit of the f32 value, at no cost - one token leaves these
-// columns empty.
+// columns empty. (Every bit down to 2^-26 of the block's largest value; below that the terms run out of exponents.)
 // A token through ten IQ2_XS experts of 2048 x 512: gate/up 12.9 -> 9.1 us, down + sum 8.0 + 3.7 -> 6.4 us against one row per wave
 // with scalar products, 32 columns per lane (the arithmetic on 2-byte-aligned pieces, and a grid entry looked up in memory behind the weights, took most of it).
 #include <hip/hip_runtime.h>
@@ -59,14 +59,15 @@ __device__ __forceinline__ half8_t term_operand(const _Float16 *planes, uint32_t
 // one unit: 16 rows (row r of lanes r, r + 16, ..) times a block; the sum of row r in lanes 0 .. 15
 template <int SRC>
 __device__ __forceinline__ float unit_product(const Quarter &v, uint2 d, const _Float16 *planes, uint32_t i, uint32_t q, const LaneTables &lt) {
-    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4_t acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};      // (half of the block each: half as many roundings behind one another)
     half2_t f{};
 #pragma unroll
     for (uint32_t s = 0; s < 8u; ++s) {
         if (s % steps_per_scale<SRC>() == 0u) f = step_scale<SRC>(v, s);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(term_operand(planes, s, i, q), finish_entry<SRC>(fetch_entry<SRC>(v, s, lt), f), acc, 0, 0, 0);
+        acc[s >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(term_operand(planes, s, i, q), finish_entry<SRC>(fetch_entry<SRC>(v, s, lt), f), acc[s >> 2], 0, 0, 0);
     }
-    return (acc[0] + (acc[1] + acc[2] * 4.8828125e-4f) * 4.8828125e-4f) * quarter_d<SRC>(d);
+    acc[0] += acc[1];
+    return (acc[0][0] + (acc[0][1] + acc[0][2] * 4.8828125e-4f) * 4.8828125e-4f) * quarter_d<SRC>(d);
 }
 
 template <int SRC> __device__ __forceinline__ LaneTables lane_tables(const uint8_t *entries, const uint32_t *signs, uint32_t tid) {

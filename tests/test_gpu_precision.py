@@ -19,7 +19,7 @@ from test_gpu_topk_pool import Case
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
-F32_CHUNK = 2.3e-7
+F32_CHUNK, F32_TOKEN = 2.3e-7, 2.1e-7
 
 
 @pytest.fixture(scope="module")
@@ -110,3 +110,17 @@ def test_wide_experts_of_a_mixed_layer(layout, grids):
         want.append(y + gate * orc.expert_ffn(cfg["sh_gate_up_type"], cfg["sh_down_type"], lay["sh_gate"], lay["sh_up"], lay["sh_down"], H, F, x[t]))
     assert rel(got[list(pick)], np.stack(want)) <= F32_CHUNK
     m.close()
+
+
+@pytest.mark.parametrize("layout", ["iq2", "f2", "xs", "m"])
+def test_one_token(tmp_path, grids, layout):
+    hidden, ffn = 2048, 512
+    c = Case(tmp_path, grids, layout, hidden=hidden, ffn=ffn, n_expert=16, seed=825)
+    rng = np.random.default_rng(12)
+    got, want = [], []
+    for _ in range(6):
+        experts, w, x = rng.permutation(16)[:10], rng.random(10).astype(np.float32) + 0.05, synth.normed_x(rng, 1, hidden)[0]
+        got.append(c.pool.execute([c.slot_of[int(e)] for e in experts], [c.layouts[e] for e in experts], w, c.word, hidden, ffn, 0, hidden, x)[0])
+        want.append(c.want(experts, w, x))
+    assert rel(np.stack(got), np.stack(want)) <= F32_TOKEN
+    c.pool.close()

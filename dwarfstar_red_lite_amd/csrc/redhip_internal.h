@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include <mutex>
+#include <vector>
 
 namespace redhip {
 
@@ -34,6 +35,33 @@ void forget_caller_grids(const void *owner);
 constexpr const char *kCodebookConflict = "IQ2_XS / IQ1_M codebooks differ from the ones this process holds while pools or resident layers that decode through them are alive";
 const int8_t *caller_grid_device(uint32_t type);      // device address of the process's codebook of IQ2_XS / IQ1_M, nullptr for other types
 bool caller_grid_present(uint32_t type);       // true for the formats that carry their own tables
+// Kernels on the matrix units hold a weight without its block's d as fp16, eleven bits: an IQ2_XS weight is entry x (2 s + 1) with s < 16, an
+// IQ1_M weight (8 entry +- 1) x (2 s + 1) / 8 with s < 8. True if they hold every weight of this codebook exactly.
+inline bool codebook_fits_fp16(uint32_t type, const int8_t *grid, size_t n) {
+    for (size_t i = 0; i < n; ++i) {
+        int v = grid[i] < 0 ? -grid[i] : grid[i];
+        if (type == T_IQ1_M ? v > 16 : (v >> __builtin_ctz(v | 256)) * 31 > 2048) return false;      // (trailing zero bits cost an fp16 nothing)
+    }
+    return true;
+}
+// The two codebooks of a pool, as the caller gave them
+struct PoolCodebooks {
+    std::vector<int8_t> iq2_xs, iq1_m;
+    bool xs_fp16 = true, m_fp16 = true, xs_signed = false;
+    void assign(const int8_t *xs, size_t n_xs, const int8_t *m, size_t n_m) {
+        iq2_xs.assign(xs, xs + n_xs);
+        iq1_m.assign(m, m + n_m);
+        xs_fp16 = codebook_fits_fp16(T_IQ2_XS, xs, n_xs);
+        m_fp16 = codebook_fits_fp16(T_IQ1_M, m, n_m);
+        for (size_t i = 0; i < n_xs; ++i) xs_signed = xs_signed || xs[i] < 0;
+    }
+    // may experts of these types run on the matrix units? (other codebooks: the kernels that decode to f32)
+    bool fp16_rows(uint32_t gate_up, uint32_t down) const {
+        return (xs_fp16 || (gate_up != T_IQ2_XS && down != T_IQ2_XS)) && (m_fp16 || (gate_up != T_IQ1_M && down != T_IQ1_M));
+    }
+    // ... from re-laid copies? The slice kernels place the sign bits beside IQ2_XS magnitudes.
+    bool fp16_copies(uint32_t gate_up, uint32_t down) const { return fp16_rows(gate_up, down) && !(xs_signed && (gate_up == T_IQ2_XS || down == T_IQ2_XS)); }
+};
 inline uint64_t row_bytes(uint32_t t, uint32_t ncols) {
     if (!ncols) return 0;
     if (t == T_F32) return 4ull * ncols;

@@ -43,7 +43,7 @@ struct FfnPool {
     PinnedBuf in{hipHostMallocNonCoherent}, out{hipHostMallocCoherent};      // an execute's input and output rows
     uint64_t bytes_read = 0, read_calls = 0;
     double read_ms = 0.0;
-    std::vector<int8_t> iq2_xs, iq1_m;            // the caller's codebooks (the reference keeps them in two device buffers per pool)
+    PoolCodebooks books;                          // (the reference keeps them in two device buffers per pool)
 
     uint8_t *slot_base(uint32_t slot) {           // nullptr + message on failure
         if (slot >= capacity) { FFN_ERR("FFN slot %u exceeds capacity %u", slot, capacity); return nullptr; }
@@ -120,8 +120,9 @@ bool floats_arrived(const void *p, size_t n) {
 }
 
 // gate/up + SwiGLU into act, then the down rows asked for
-hipError_t enqueue_expert(const ExpertSet &ex, uint32_t hidden, uint32_t ffn, uint32_t row_start, uint32_t row_count, const float *x, float *act, float *out, hipStream_t s) {
-    const bool token = token_rows_supported(ex.gate_up_type, ex.down_type, 1u, hidden, ffn, x, nullptr);      // (Q6_K rows and a misaligned input go the other way)
+hipError_t enqueue_expert(const PoolCodebooks &books, const ExpertSet &ex, uint32_t hidden, uint32_t ffn, uint32_t row_start, uint32_t row_count, const float *x, float *act, float *out, hipStream_t s) {
+    // (Q6_K rows, a misaligned input and codebooks of large values go the other way)
+    const bool token = books.fp16_rows(ex.gate_up_type, ex.down_type) && token_rows_supported(ex.gate_up_type, ex.down_type, 1u, hidden, ffn, x, nullptr);
     const hipError_t e = token ? launch_token_gateup(ex, 1u, hidden, ffn, x, nullptr, 0u, act, s) : launch_moe_gateup(ex, nullptr, 1u, hidden, ffn, x, act, s);
     if (e != hipSuccess) return e;
     return token ? launch_token_down(ex, nullptr, 1u, ffn, row_start, row_count, act, out, nullptr, s)
@@ -153,8 +154,7 @@ redmetal_ffn_pool_t redmetal_ffn_pool_create(const char *model_path, uint64_t bu
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) { FFN_ERR("no HIP device available"); return nullptr; }
     if (!scratch_of_current_device(g_ffn_error, sizeof(g_ffn_error))) return nullptr;      // set-up of the entry point that allocates nothing
     FfnPool *p = new FfnPool();
-    p->iq2_xs.assign(iq2_xs_grid, iq2_xs_grid + iq2_xs_grid_count);      // uploaded when an IQ2_XS / IQ1_M expert is executed
-    p->iq1_m.assign(iq1_m_grid, iq1_m_grid + iq1_m_grid_count);
+    p->books.assign(iq2_xs_grid, iq2_xs_grid_count, iq1_m_grid, iq1_m_grid_count);      // uploaded when an IQ2_XS / IQ1_M expert is executed
     p->slot_bytes = aligned;
     p->budget = budget_bytes;
     const uint64_t cap64 = budget_bytes / aligned;
@@ -311,14 +311,14 @@ int redmetal_ffn_pool_execute_expert(redmetal_ffn_pool_t h, uint32_t slot_id, ui
     memcpy(p->in.p, input, n_x * sizeof(float));
     expect_floats(p->out.p, n_out);
     if (gu == T_IQ2_XS || gu == T_IQ1_M || dn == T_IQ2_XS || dn == T_IQ1_M) {      // this pool's codebooks on the device (free when they already are)
-        const hipError_t e = set_caller_grids(p->iq2_xs.data(), p->iq1_m.data(), p);
+        const hipError_t e = set_caller_grids(p->books.iq2_xs.data(), p->books.iq1_m.data(), p);
         if (e == hipErrorContextAlreadyInUse) { FFN_ERR("%s", kCodebookConflict); return 0; }
         if (e != hipSuccess) { FFN_ERR("failed to upload the IQ2_XS / IQ1_M codebooks: %s", hipGetErrorString(e)); return 0; }
     }
     p->mark(slot_id, 1);
     const double t0 = now_ms();
     const ExpertSet ex{base, 0, gate_bytes, up_bytes, gu, dn};
-    hipError_t e = enqueue_expert(ex, hidden_size, ffn_size, output_row_start, output_row_count, reinterpret_cast<const float *>(p->in.dev), dact,
+    hipError_t e = enqueue_expert(p->books, ex, hidden_size, ffn_size, output_row_start, output_row_count, reinterpret_cast<const float *>(p->in.dev), dact,
                                   reinterpret_cast<float *>(p->out.dev), nullptr);
     if (e == hipSuccess && !floats_arrived(p->out.p, n_out)) e = hipStreamSynchronize(nullptr);
     const double ms = now_ms() - t0;
@@ -379,7 +379,7 @@ int redmetal_ffn_pool_execute_expert_noalloc(redmetal_ffn_pool_t h, uint32_t slo
     hipStream_t s = static_cast<hipStream_t>(stream);
     // gate/up + SwiGLU writes act[0 .. ffn), the down rows read exactly that range: nothing in the scratch has to start at zero
     const ExpertSet ex{base, 0, gate_bytes, up_bytes, gu, dn};
-    const hipError_t e = enqueue_expert(ex, hidden_size, ffn_size, output_row_start, output_row_count, input_dev, act, output_dev, s);
+    const hipError_t e = enqueue_expert(p->books, ex, hidden_size, ffn_size, output_row_start, output_row_count, input_dev, act, output_dev, s);
     if (e != hipSuccess) { FFN_ERR("FFN HIP command failed: %s", hipGetErrorString(e)); return 0; }
     return 1;
 }

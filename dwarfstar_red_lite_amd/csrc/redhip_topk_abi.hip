@@ -40,7 +40,7 @@ struct TopkPool {
     std::recursive_mutex enc_mu;                  // an encode call sizes and fills buffers of the pool: host side one call at a time
     uint64_t bytes_read = 0, read_calls = 0;
     double read_ms = 0.0;
-    std::vector<int8_t> iq2_xs, iq1_m;
+    PoolCodebooks books;
     // buffers between the launches of a call (grow-only)
     DevBuf act, tmp, io;
     // the batched / mapped forms keep buffers of their own (the reference's _tmpB): growing them for a large chunk never moves `tmp`,
@@ -109,7 +109,7 @@ struct TopkPool {
     }
     // may calls of this shape run on the slice kernels? (the copies of the slots they name are checked by the caller where it knows them)
     bool fast_shape(uint32_t word, uint32_t hidden, uint32_t ffn) const {
-        return fast && hidden == fs.hidden && ffn == fs.ffn && word_gate_up(word) == word_gate_up(fs.word) && word_down(word) == word_down(fs.word);
+        return fast && books.fp16_copies(word_gate_up(word), word_down(word)) && hidden == fs.hidden && ffn == fs.ffn && word_gate_up(word) == word_gate_up(fs.word) && word_down(word) == word_down(fs.word);
     }
     void mark(const uint32_t *slots, uint32_t n, int delta) {
         std::lock_guard<std::mutex> lk(mu);
@@ -141,7 +141,7 @@ bool type_word_ok(uint32_t w) { return !(w >> 16) && pool_quant_supported(word_g
 bool bind_grids(TopkPool *p, uint32_t type_word) {
     const uint32_t gu = word_gate_up(type_word), dn = word_down(type_word);
     if (gu != T_IQ2_XS && gu != T_IQ1_M && dn != T_IQ2_XS && dn != T_IQ1_M) return true;
-    const hipError_t e = set_caller_grids(p->iq2_xs.data(), p->iq1_m.data(), p);
+    const hipError_t e = set_caller_grids(p->books.iq2_xs.data(), p->books.iq1_m.data(), p);
     if (e == hipErrorContextAlreadyInUse) { TOPK_ERR("%s", kCodebookConflict); return false; }
     if (e != hipSuccess) { TOPK_ERR("failed to upload the IQ2_XS / IQ1_M codebooks: %s", hipGetErrorString(e)); return false; }
     return true;
@@ -229,13 +229,13 @@ bool enqueue_token(TopkPool *p, hipStream_t s, const uint64_t *table_dev, const 
     ExpertSet ex{nullptr, 0, gate_bytes, up_bytes, word_gate_up(type_word), word_down(type_word)};
     ex.table = table_dev;
     float *act = static_cast<float *>(p->act.p), *tmp = static_cast<float *>(p->tmp.p);
-    if ((out || tail) && token_rows_supported(ex.gate_up_type, ex.down_type, top_k, hidden, ffn, x, x1)) {
+    if ((out || tail) && p->books.fp16_rows(ex.gate_up_type, ex.down_type) && token_rows_supported(ex.gate_up_type, ex.down_type, top_k, hidden, ffn, x, x1)) {
         hipError_t e = launch_token_gateup(ex, top_k, hidden, ffn, x, x1, x_split, act, s);
         if (e == hipSuccess) e = launch_token_down(ex, weights_dev, top_k, ffn, row_start, row_count, act, out, tail, s);
         if (e != hipSuccess) { TOPK_ERR("top-k HIP command failed: %s", hipGetErrorString(e)); return false; }
         return true;
     }
-    // Q6_K rows, more experts than the kernels above hold, or the per-expert results wanted
+    // Q6_K rows, codebooks of large values, more experts than the kernels above hold, or the per-expert results wanted
     hipError_t e = launch_moe_gateup(ex, nullptr, top_k, hidden, ffn, x, act, s, x1, x_split);
     // one group per expert with exactly one pair: pair e reads act[e], writes tmp[e]
     if (e == hipSuccess) e = launch_batch_down(ex, nullptr, p->iota, nullptr, top_k, top_k, hidden, ffn, act, tmp, s);
@@ -338,14 +338,15 @@ bool enqueue_pairs(TopkPool *p, hipStream_t s, const std::vector<uint64_t> &gate
 
 // The same pairs on the tile kernels: x split to fp16 halves per token, tiles of up to 32 pairs per expert on the MFMA units (gate / up +
 // SwiGLU, then down rows into tmp[pair]), combine in selection order. `copies`: slots that hold tile-major copies, on the kernels that
-// read those; otherwise the kernels that take raw rows through LDS. Expert u is number uid[u] of the arrays that `ex` describes.
+// read those; otherwise on the raw rows. Expert u is number uid[u] of the arrays that `ex` describes.
 struct PairExperts {
     const uint8_t *gate, *down;
     uint64_t stride, down_stride, up_delta;
     std::vector<uint32_t> uid;
 };
-bool rows_on_tiles(uint32_t type_word, uint32_t hidden, uint32_t ffn, uint32_t n_expert) {
-    return n_expert <= 1024u && staged_gateup_supported(word_gate_up(type_word), RowLayout::raw, hidden, ffn) && staged_down_supported(word_down(type_word), RowLayout::raw, hidden, ffn);
+bool rows_on_tiles(const TopkPool *p, uint32_t type_word, uint32_t hidden, uint32_t ffn, uint32_t n_expert) {
+    const uint32_t gu = word_gate_up(type_word), dn = word_down(type_word);
+    return n_expert <= 1024u && p->books.fp16_rows(gu, dn) && staged_gateup_supported(gu, RowLayout::raw, hidden, ffn) && staged_down_supported(dn, RowLayout::raw, hidden, ffn);
 }
 // slots: an expert is named by the distance of its slot from the lowest slot of the call, in units of 256 bytes (slots are 4096-aligned,
 // HBM is far below 1 TB)
@@ -477,8 +478,7 @@ redmetal_topk_pool_t redmetal_topk_pool_create(const char *model_path, uint64_t 
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) { TOPK_ERR("no HIP device available"); return nullptr; }
     TopkPool *p = new TopkPool();
-    p->iq2_xs.assign(iq2_xs_grid, iq2_xs_grid + iq2_xs_grid_count);
-    p->iq1_m.assign(iq1_m_grid, iq1_m_grid + iq1_m_grid_count);
+    p->books.assign(iq2_xs_grid, iq2_xs_grid_count, iq1_m_grid, iq1_m_grid_count);
     p->budget = budget_bytes;
     const uint64_t cap64 = budget_bytes / aligned;
     p->capacity = cap64 > 0xffffffffull ? 0xffffffffu : (uint32_t)cap64;
@@ -923,7 +923,7 @@ int redmetal_topk_pool_encode_batched(redmetal_topk_pool_t h, void *stream, cons
         for (uint32_t i = 0; i < n_expert; ++i) tiles = tiles && p->shadow_ok[slot_ids[i]];
     }
     // slots without tile-major copies: the tile kernels on their raw rows, for the formats and shapes those take
-    const bool staged = !tiles && rows_on_tiles(ggml_type, hidden_size, ffn_size, n_expert);
+    const bool staged = !tiles && rows_on_tiles(p, ggml_type, hidden_size, ffn_size, n_expert);
     PairExperts ex;
     if (tiles || staged ? !slot_experts(table, gate_bytes[0], &ex) ||
                               !enqueue_pairs_tiles(p, static_cast<hipStream_t>(stream), ex, tiles, ggml_type, n_expert, hidden_size, ffn_size, tok_first, ntok, top_k, n_pairs,
@@ -950,7 +950,7 @@ int redmetal_topk_pool_encode_mapped(redmetal_topk_pool_t h, void *stream,
     if (!pool_shape_ok(hidden_size, ffn_size, true)) return 0;
     if (!pair_layout_ok("mapped", n_expert, tok_first, ntok, top_k, n_pairs, pair_token, expert_start, tok_pair)) return 0;
     if (((gate_addr0 | up_addr0 | down_addr0 | gate_bytes | down_bytes) & 15u) == 0u &&
-        rows_on_tiles(ggml_type, hidden_size, ffn_size, n_expert)) {
+        rows_on_tiles(p, ggml_type, hidden_size, ffn_size, n_expert)) {
         const PairExperts ex{reinterpret_cast<const uint8_t *>(gate_addr0), reinterpret_cast<const uint8_t *>(down_addr0), gate_bytes, down_bytes, up_addr0 - gate_addr0,
                              std::vector<uint32_t>(expert_ids, expert_ids + n_expert)};
         return enqueue_pairs_tiles(p, static_cast<hipStream_t>(stream), ex, false, ggml_type, n_expert, hidden_size, ffn_size, tok_first, ntok, top_k, n_pairs, pair_token,

@@ -132,7 +132,9 @@ int redhip_moe_group(redhip_moe_t moe, const uint32_t *ids_dev, const float *wei
  * redmetal_ffn_pool_create and redmetal_quant_rows (native/redmetal_ffn.h:9-18, native/redmetal_quant.h:9-27), which upload
  * them too. Process-wide and synchronous: the process holds one pair of tables. Resident layers with such experts, and pools that have run
  * one, are bound to the tables' content: while any of them is alive, a call (here, or through a pool / redmetal_quant_rows) that brings
- * different tables fails with a message instead of changing what they decode through; the same content again is free. */
+ * different tables fails with a message instead of changing what they decode through; the same content again is free.
+ * Resident layers multiply weights as fp16 without their block's d and take IQ2_XS entries as magnitudes: entries have to be 0 .. 66
+ * (IQ2_XS) and -16 .. 16 (IQ1_M), which the formats' own tables are. (Pools, redmetal_quant_rows and the taps below take any int8 values.) */
 int redhip_set_codebooks(const int8_t *iq2_xs_grid, uint32_t iq2_xs_count, const int8_t *iq1_m_grid, uint32_t iq1_m_count);
 
 /* Parity tap: f32 dequantisation of `rows` rows of `ncols` weights of raw GGUF blocks (device pointers). */

@@ -144,8 +144,9 @@ int redmetal_topk_pool_encode_device_tail(redmetal_topk_pool_t pool, void *strea
  * (slots) serve n_pairs = ntok * top_k (expert, token) pairs sorted by expert (expert_start[n_expert + 1] prefix sums;
  * pair_token / pair_weight per pair; tok_pair[ntok * top_k] lists each token's pairs in router selection order; all four are
  * host arrays). Input rows are hidden_size floats per token at input_dev + input_offset (token index = pair_token), output
- * rows likewise for tokens tok_first .. tok_first + ntok - 1. Every expert's weights are decoded once per eight of its
- * pairs. Marks the slots in flight; release with redmetal_topk_pool_release(slot_ids, n_expert). */
+ * rows likewise for tokens tok_first .. tok_first + ntok - 1. Every expert's weights are decoded once per 16 or 32 of its
+ * pairs (hidden_size 512, 1024 or 2048 with ffn_size 256 .. 1024 on IQ2_XXS, IQ2_XS, IQ1_M or IQ3_S rows; other shapes, Q6_K rows and
+ * codebooks of large values: once per eight). Marks the slots in flight; release with redmetal_topk_pool_release(slot_ids, n_expert). */
 int redmetal_topk_pool_encode_batched(redmetal_topk_pool_t pool, void *stream, const uint32_t *slot_ids,
     const uint64_t *gate_bytes, const uint64_t *up_bytes, const uint64_t *down_bytes, uint32_t n_expert,
     uint32_t ggml_type, uint32_t hidden_size, uint32_t ffn_size, uint32_t tok_first, uint32_t ntok, uint32_t top_k,
@@ -178,7 +179,8 @@ int redmetal_topk_pool_encode_mapped(redmetal_topk_pool_t pool, void *stream,
  * pool's slots loaded with experts of the declared shape. flags: REDHIP_TOPK_FAST_TILES (hidden_size <= 2048 and ffn_size <= 512)
  * adds a third copy per slot, tile-major as this library's prefill kernels read it (the slot class grows to three times the expert's
  * bytes); redmetal_topk_pool_encode_batched of that shape then runs on those kernels - tiles of up to 32 pairs per expert on the
- * matrix units - when every slot it names holds its copies; 0: none. Returns 1, or 0 with redmetal_topk_last_error(). */
+ * matrix units - when every slot it names holds its copies; 0: none. (Codebooks with IQ2_XS entries
+ * beyond 0 .. 66 or IQ1_M entries beyond +-16 leave every call on the raw rows, decoded to f32.) Returns 1, or 0 with redmetal_topk_last_error(). */
 #define REDHIP_TOPK_FAST_TILES 1u
 int redhip_topk_pool_enable_fast_path(redmetal_topk_pool_t pool, uint32_t ggml_type, uint32_t hidden_size, uint32_t ffn_size, uint32_t flags);
 

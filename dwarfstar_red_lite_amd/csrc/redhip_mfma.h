@@ -11,20 +11,23 @@ namespace redhip {
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-// power-of-two pre-scale: largest |v| lands in [2^13, 2^14)
+// power-of-two pre-scale: largest |v| lands in [2^13, 2^14); beside an infinity every finite value stays below 2^13
 __device__ __forceinline__ int prescale_exp(float amax) {
-    if (!(amax > 0.0f) || isinf(amax) || isnan(amax)) return 0;
+    if (!(amax > 0.0f)) return 0;
     const int e = (int)((__float_as_uint(amax) >> 23) & 255u) - 127 - 13;
     return e < -126 ? -126 : e;                     // (its inverse has to be a float)
 }
 __device__ __forceinline__ float exp2i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }   // e in [-126, 127]
 
+// What t, the value that h was rounded from, has beyond h, times 2^11. Of an infinity: something finite (and not inf - inf), so that the
+// product of an infinity stays one.
+__device__ __forceinline__ float split_rest(float t, _Float16 h) { return __builtin_amdgcn_fmed3f((t - (float)h) * 2048.0f, -16384.0f, 16384.0f); }
 // v = hi + lo * 2^-11 (to 22 significant bits) after scaling by 2^-e
 __device__ __forceinline__ void split_hi_lo(float v, float inv_scale, _Float16 *hi, _Float16 *lo) {
     const float t = v * inv_scale;
     const _Float16 h = (_Float16)t;
     *hi = h;
-    *lo = (_Float16)((t - (float)h) * 2048.0f);
+    *lo = (_Float16)split_rest(t, h);
 }
 
 

@@ -166,7 +166,7 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
                         const float t = f[k] * inv;
                         const _Float16 h = (_Float16)t;
                         hi.e[k] = h;
-                        lo.e[k] = (_Float16)((t - (float)h) * 2048.0f);
+                        lo.e[k] = (_Float16)split_rest(t, h);
                     }
                     // group by group (the compiler otherwise works on several at once and spills)
                     asm volatile("" : "+v"(hi.u.x), "+v"(hi.u.y), "+v"(hi.u.z), "+v"(hi.u.w), "+v"(lo.u.x), "+v"(lo.u.y), "+v"(lo.u.z), "+v"(lo.u.w));

@@ -43,7 +43,7 @@ __device__ __forceinline__ float store_terms(float4 x, _Float16 *planes, uint32_
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             t[k].h[i] = (_Float16)rest;
-            rest = (rest - (float)t[k].h[i]) * 2048.0f;
+            rest = split_rest(rest, t[k].h[i]);
         }
     }
 #pragma unroll

@@ -68,16 +68,14 @@ struct DevBuf {                       // grow-only device scratch
     ~DevBuf() { if (p) (void)hipFree(p); }
 };
 
-struct PinnedBuf {                    // grow-only pinned host memory that kernels read or write
-    const unsigned flags;             // hipHostMallocNonCoherent (the device caches what it reads) or hipHostMallocCoherent (its stores are seen before the kernel ends)
-    explicit PinnedBuf(unsigned f) : flags(f) {}
+struct PinnedBuf {                    // grow-only pinned host memory that kernels read or write, coherent: either side sees the other's stores without a wait for the stream
     uint8_t *p = nullptr, *dev = nullptr;
     size_t cap = 0;
     bool reserve(size_t n) {
         if (n <= cap) return true;
         release();
         void *h = nullptr, *d = nullptr;
-        if (hipHostMalloc(&h, n, hipHostMallocMapped | hipHostMallocPortable | flags) != hipSuccess) return false;
+        if (hipHostMalloc(&h, n, hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) return false;
         if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) { (void)hipHostFree(h); return false; }
         p = static_cast<uint8_t *>(h);
         dev = static_cast<uint8_t *>(d);

@@ -369,18 +369,20 @@ bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const PairExperts &ex, bool
                          const uint32_t *expert_start, const uint32_t *tok_pair, const float *x, float *out) {
     std::lock_guard<std::recursive_mutex> lk(p->enc_mu);
     if (!bind_grids(p, type_word)) return false;
+    // rows of x from the first to the last that a pair names, which are all that is read of it (a call's tokens mostly lie together)
+    const uint32_t row0 = *std::min_element(pair_token, pair_token + n_pairs), rows = *std::max_element(pair_token, pair_token + n_pairs) + 1u - row0;
+    x += (uint64_t)row0 * hidden;
     std::vector<uint32_t> u;
     u.reserve((size_t)n_pairs * 2u + 2u * n_expert + 2u);
-    u.insert(u.end(), pair_token, pair_token + n_pairs);
+    for (uint32_t i = 0; i < n_pairs; ++i) u.push_back(pair_token[i] - row0);
     u.insert(u.end(), expert_start, expert_start + n_expert + 1u);
     u.insert(u.end(), tok_pair, tok_pair + (size_t)ntok * top_k);
     u.insert(u.end(), ex.uid.begin(), ex.uid.end());
     u.push_back(n_expert);
-    // scratch of the call: rows of x up to the last token of the call, n_pairs activation rows
-    const size_t rows = (size_t)tok_first + ntok;
+    // scratch of the call: the halves of these rows, n_pairs activation rows
     const uint32_t bound = prefill_tile_bound(ntok, top_k, n_expert);
     auto a256 = [](size_t v) { return (v + 255u) & ~(size_t)255u; };
-    const size_t x_half = a256(rows * hidden * 2u), x_exp = a256(rows * 4u), a_bytes = a256((size_t)n_pairs * ffn * 4u), tl = a256(12u * (size_t)bound);
+    const size_t x_half = a256((size_t)rows * hidden * 2u), x_exp = a256((size_t)rows * 4u), a_bytes = a256((size_t)n_pairs * ffn * 4u), tl = a256(12u * (size_t)bound);
     if (!p->chunk.reserve(2u * x_half + 2u * x_exp + a_bytes + 4u * tl) || !p->tmp_b.reserve((size_t)n_pairs * hidden * sizeof(float))) {
         TOPK_ERR("failed to allocate top-k activation buffers");
         return false;
@@ -400,7 +402,7 @@ bool enqueue_pairs_tiles(TopkPool *p, hipStream_t s, const PairExperts &ex, bool
     const uint32_t *d_pair_token = st.u, *d_start = st.u + n_pairs, *d_tok_pair = d_start + n_expert + 1u, *d_uid = d_tok_pair + (size_t)ntok * top_k, *d_unique = d_uid + n_expert;
     float *tmp = static_cast<float *>(p->tmp_b.p);
     // (the split kernel also forms a gate logit per row from a second vector: x itself stands in, the result is not used)
-    hipError_t e = launch_prep(x, x, (uint32_t)rows, hidden, xh, xl, xexp, gate_unused, s, nullptr, nullptr);
+    hipError_t e = launch_prep(x, x, rows, hidden, xh, xl, xexp, gate_unused, s, nullptr, nullptr);
     const TileLists lists{tile_expert, tile_pair0, tile_n, n_tiles, bound, 0u};
     if (e == hipSuccess) e = launch_build_tiles(d_uid, d_start, d_unique, n_pairs, lists, s);
     uint32_t wide = 0u;

@@ -45,6 +45,7 @@ struct StagedArgs {
     float *tmp, *sh_tmp;                   // down out: [P][rows] routed pairs, [ntok][rows] shared expert
     const int8_t *grid;                    // codebook of IQ2_XS / IQ1_M
     uint32_t rows, P, list_stride;
+    uint32_t few;                          // wide tiles that are not worth a launch: fewer than this many
 };
 
 __device__ __forceinline__ void wave_lds_barrier() {
@@ -346,17 +347,27 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
 }
 
 // SETS 1: the narrow tiles (list 2) of a chunk, SETS 2: the wide ones (list 1). Persistent workgroups, each with an equal run of the units.
-// A launch that finds few wide tiles leaves them: the narrow one then takes every pair in tiles of 16 (list 0). A wide launch costs 10 us
-// however few tiles it has (tables, the first tile's activations); beyond that a wide tile took 0.32 us of the device (gate/up, hidden 2048,
-// ffn 512) where two narrow ones take 0.43, 0.21 against 0.26 in the down kernels, 0.24 against 0.27 with IQ3_S words.
-template <int SRC, bool DOWN> constexpr uint32_t few_wide() { return !DOWN ? 90u : is_iq3<SRC>() ? 330u : 190u; }
+// A launch that finds few wide tiles leaves them: the narrow one then takes every pair in tiles of 16 (list 0). Two launches where one would
+// do cost 10 to 20 us (tables, the first tiles' activations, compute units without a unit at both ends); a wide tile saves a second decoding
+// of its rows, which goes with their weights. So the line is a number of weights in wide tiles: 220 million for gate/up, 230 million for
+// IQ2_XXS down rows, 145 million for the other down formats. Both ways measured on chunks of evenly routed tokens, 128 and 512 experts with
+// 12 to 40 pairs on average, 1024 x 256 to 2048 x 768; what was even: gate/up 130 to 240 million on all-IQ2_XXS layers, 300 to 450 on the
+// others, down 118 to 230 IQ2_XXS, 125 to 170 the others. 221 wide tiles of 2048 x 512 (464 / 232 million, IQ2_XS): 260 + 133 us with
+// them, 263 + 154 without; 97 (203 / 102): 105 + 69 against 99 + 54. On mixed layouts the shared expert's products run beside gate/up and
+// finish sooner beside two launches: a layer of 112 wide tiles of 2048 x 512 (235 million) takes 332 us with them, 340 without, one of 195
+// of 1024 x 512 (205) 191 against 183, so these share the all-IQ2_XXS line. Packed IQ2_XXS down rows (ffn above 512) lost 20 us with 57 to
+// 139 wide tiles alike and have none.
+template <int SRC, bool DOWN> constexpr bool has_wide() { return !(DOWN && layout<SRC>() == L_ROWS); }
+template <int SRC, bool DOWN> uint32_t few_wide(uint32_t rows, uint32_t K) {
+    return !has_wide<SRC, DOWN>() ? ~0u : (DOWN ? fmt<SRC>() == F_XXS ? 230000000u : 145000000u : 110000000u) / (rows * K) + 1u;
+}
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
 __global__ __launch_bounds__(staged_threads(SETS, KP)) void staged_tiles_kernel(StagedArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t entries[kEntryBytes];   // static: table reads take immediate offsets
     __shared__ __attribute__((aligned(16))) uint32_t signs[sign_bytes<SRC>() / 4u + 4u];
     __shared__ __attribute__((aligned(16))) float part[4u * KP * staged_nrt(KP) * 2u * 256u];
     const uint32_t n0 = a.n_tiles[0], n1 = a.n_tiles[1], n2 = a.n_tiles[2];      // (one trip)
-    const bool few = n1 < few_wide<SRC, DOWN>();
+    const bool few = n1 < a.few;
     if (SETS == 2 && few) return;
     const uint32_t tid = threadIdx.x, l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
     const uint32_t units = (SETS == 2 ? n1 : few ? n0 : n2) * (a.rows / ((DOWN ? 32u : 16u) * staged_nrt(KP)));
@@ -379,8 +390,12 @@ hipError_t launch_staged_list(const StagedArgs &a, uint32_t grid, hipStream_t s)
 }
 // wide: wide tiles that the chunk can have at most
 template <int SRC, bool DOWN, uint32_t KP>
-hipError_t launch_staged_lists(const StagedArgs &a, uint32_t grid, uint32_t wide, hipStream_t s) {
-    const hipError_t e = wide >= few_wide<SRC, DOWN>() ? launch_staged_list<SRC, DOWN, 2, KP>(a, grid, s) : hipSuccess;
+hipError_t launch_staged_lists(StagedArgs a, uint32_t grid, uint32_t wide, hipStream_t s) {
+    a.few = few_wide<SRC, DOWN>(a.rows, 256u * KP);
+    hipError_t e = hipSuccess;
+    if constexpr (has_wide<SRC, DOWN>()) {
+        if (wide >= a.few) e = launch_staged_list<SRC, DOWN, 2, KP>(a, grid, s);
+    }
     return e == hipSuccess ? launch_staged_list<SRC, DOWN, 1, KP>(a, grid, s) : e;
 }
 template <int SRC>

@@ -52,11 +52,11 @@ def pool_chunk(c, hidden, ffn, counts, ntok, top_k, x, rng, pick):
 
 # raw rows and tile-major copies; tiles of 16 pairs (the first two sizes) and of 32
 @pytest.mark.parametrize("layout", ["iq2", "f2", "xs", "m"])
-@pytest.mark.parametrize("hidden,ffn,tiles,wide", [(2048, 512, False, False), (1024, 256, True, False), (512, 512, False, True), (512, 256, True, True)])
+@pytest.mark.parametrize("hidden,ffn,tiles,wide", [(2048, 512, False, False), (1024, 256, True, False), (512, 512, False, True), (1024, 256, True, True)])
 def test_chunk_of_pairs(tmp_path, grids, layout, hidden, ffn, tiles, wide):
     c = Case(tmp_path, grids, layout, hidden=hidden, ffn=ffn, n_expert=12, seed=821, fast=tiles, tiles=tiles)
     rng = np.random.default_rng(4)
-    ntok, counts = (2700, [900] * 12) if wide else (24, [8] * 12)
+    ntok, counts = (8100, [2700] * 12) if wide else (24, [8] * 12)
     x = synth.normed_x(rng, ntok, hidden)
     pick = rng.choice(ntok, 24, replace=False)
     assert pool_chunk(c, hidden, ffn, counts, ntok, 4, x, rng, pick) <= F32_CHUNK
@@ -80,7 +80,7 @@ def test_small_activations_beside_large_ones(tmp_path, grids, layout, wide, monk
     monkeypatch.setattr(synth, "make_layer", first_block_zero)
     c = Case(tmp_path, grids, layout, hidden=hidden, ffn=ffn, n_expert=12, seed=823)
     rng = np.random.default_rng(6)
-    ntok, counts = (2700, [900] * 12) if wide else (24, [8] * 12)
+    ntok, counts = (8100, [2700] * 12) if wide else (24, [8] * 12)
     x = synth.normed_x(rng, ntok, hidden)
     x[:, :256] *= np.float32(2.0 ** 18)
     pick = rng.choice(ntok, 24, replace=False)

@@ -1,5 +1,5 @@
-"""The tile kernels that take rows through LDS (csrc/redhip_tiles.hip): chunks on the pool's raw slots and on resident layers without
-tile-major copies, against the CPU path. Experts with 1, 15, 16, 17, 31, 32, 33 and more pairs (edges of the 16- and 32-pair tiles), few and
+"""The tile kernels (csrc/redhip_tiles.hip) on raw and packed rows: chunks on the pool's slots and on resident layers without tile-major
+copies, against the CPU path. Experts with 1, 15, 16, 17, 31, 32, 33 and more pairs (edges of the 16- and 32-pair tiles), few and
 many wide tiles (few of them run as tiles of 16), every row format, every split of K."""
 import json
 import os
@@ -37,10 +37,12 @@ def routing_with(counts, ntok, top_k, rng):
     return ids[rng.permutation(ntok)]
 
 
-# (hidden, ffn): K parts 2 / 4 / 8 of the gate/up kernel, 1 / 2 / 4 (768: of 192 columns) / 4 of the down kernel; wide tiles at the smaller shapes
+# (hidden, ffn): K parts 2 / 4 / 8 of the gate/up kernel, 1 / 2 / 3 / 4 of the down kernel
 SHAPES = [("iq2", 512, 256), ("f2", 1024, 512), ("xs", 2048, 768), ("m", 512, 1024), ("iq2", 1024, 768), ("f2", 512, 768), ("xs", 512, 512), ("m", 1024, 256),
           ("f2", 2048, 256), ("xs", 1024, 1024), ("m", 512, 768), ("iq2", 512, 1024), ("f2", 512, 1024)]
-WIDE = [("iq2", 512, 256), ("f2", 1024, 512), ("f2", 512, 768), ("xs", 512, 512), ("m", 1024, 256), ("m", 512, 768)]
+# 1008 wide tiles are above both kernels' lines for these (220 million weights in them for gate/up, 230 / 145 million for down)
+WIDE = [("iq2", 512, 512), ("iq2", 1024, 256), ("f2", 1024, 512), ("f2", 512, 768), ("f2", 1024, 256), ("f2", 512, 1024), ("xs", 512, 512), ("xs", 1024, 1024), ("m", 1024, 256),
+        ("m", 512, 768), ("m", 2048, 512)]
 
 
 @pytest.mark.parametrize("layout,hidden,ffn,many_wide", [s + (False,) for s in SHAPES] + [s + (True,) for s in WIDE])
@@ -48,9 +50,9 @@ def test_pool_slots(tmp_path, grids, layout, hidden, ffn, many_wide):
     n_expert, top_k = 12, 4
     c = Case(tmp_path, grids, layout, hidden=hidden, ffn=ffn, n_expert=n_expert, seed=811)
     rng = np.random.default_rng(3)
-    if many_wide:      # 12 experts with about 900 pairs: enough tiles of 32 for the wide launches of every format, remainders of 4, two wide remainders
-        ntok = 2700
-        counts = [900] * n_expert
+    if many_wide:      # 12 experts with 2700 pairs (84 tiles of 32 each): enough for the wide launches, remainders of 12, one wide remainder
+        ntok = 8100
+        counts = [2700] * n_expert
         counts[0] += 15
         counts[1] -= 15
     else:
@@ -108,4 +110,27 @@ def test_resident_layers(layout, shape, ntok, grids):
     got = m.experts(0, x_dev, torch.from_numpy(ids.astype(np.int32)).cuda(), torch.from_numpy(w).cuda()).cpu().numpy()
     want = oracle_tokens(cfg, lay, xs, ids, w)
     assert max(rel_l2(got[t], want[t]) for t in range(ntok)) <= REL_L2_TOL
+    m.close()
+
+
+def test_resident_packed_rows_in_wide_tiles(grids):
+    """all-IQ2_XXS layers with ffn 768 have no tile-major copies: more than 70 wide tiles of packed gate/up rows, the shared expert's among them"""
+    from dwarfstar_red_lite_amd.moe import ResidentMoe
+    from test_gpu_moe_batch import oracle_tokens
+    H, F, E, K, ntok = 2048, 768, 8, 4, 500
+    cfg = synth.layer_config(hidden=H, ffn=F, n_expert=E, top_k=K, layout="iq2")
+    m = ResidentMoe(cfg, n_layer=1, max_tokens=ntok)
+    lay = synth.make_layer(41, cfg)
+    m.load_layer(0, lay)
+    rng = np.random.default_rng(30)
+    xs = synth.normed_x(rng, ntok, H)
+    ids = np.stack([rng.permutation(E)[:K] for _ in range(ntok)]).astype(np.uint32)
+    w = rng.random((ntok, K)).astype(np.float32)
+    w /= w.sum(axis=1, keepdims=True)
+    n = np.append(np.bincount(ids.ravel(), minlength=E), ntok)
+    assert (n // 32 + (n % 32 > 16)).sum() >= 70
+    got = m.experts(0, torch.from_numpy(xs).cuda(), torch.from_numpy(ids.astype(np.int32)).cuda(), torch.from_numpy(w).cuda()).cpu().numpy()
+    pick = rng.choice(ntok, 12, replace=False)
+    want = oracle_tokens(cfg, lay, xs[pick], ids[pick], w[pick])
+    assert max(rel_l2(got[t], want[i]) for i, t in enumerate(pick)) <= 1e-5
     m.close()

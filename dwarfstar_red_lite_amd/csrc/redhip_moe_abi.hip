@@ -150,11 +150,17 @@ struct Moe {
     }
     // ... with the layer's own router: on a mixed layout two tokens are quicker on the single-token kernels (three launches, the selection
     // inside the expert kernel) than as slices behind a selection + pair sort launch of their own (four): 30.7 against 32.7 us
-    bool slices_after_router(uint32_t ntok) const { return small_batch(ntok, true) && (fused || ntok >= kGroupedMin); }
-    // ... of which layouts with slices take the single-token slices, one grid layer per token: two tokens of IQ2_XS / IQ1_M / IQ2_XXS + IQ3_S
-    // layers 30.9 / 30.1 / 30.3 -> 27.6 / 26.1 / 27.6 us per layer against gateup_select_kernel + down_combine_words_kernel. (448 workgroups,
-    // two per compute unit; three tokens would need a second round, and all-IQ2_XXS tables leave room for one workgroup.)
-    bool token_slices(uint32_t ntok) const { return ntok == 2u && mixed_slices && dense_routed && small_batch(ntok, true); }
+    bool slices_after_router(uint32_t ntok) const { return small_batch(ntok, true) && !token_slices(ntok) && (fused || ntok >= kGroupedMin); }
+    // ... of which layouts with slices take the single-token slices, one grid layer per token, while their workgroups (ffn / 32 for each expert and
+    // four times for the shared one) are about one round of the device, two per compute unit. IQ2_XXS + IQ3_S / IQ2_XS / IQ1_M layers, us per
+    // layer, against the kernels that two tokens had before or the slices behind a selection + pair sort launch: two tokens of 2048 x 512, ten
+    // experts (448 workgroups) 27.5 / 28.3 / 27.3 -> 24.8 / 25.5 / 23.8; of 1024 x 256, eight experts: three (288) 18.5 / 19.3 / 19.2 -> 15.1 /
+    // 15.0 / 14.6, five (480) 22.5 / 22.8 / 22.5 -> 20.0 / 19.7 / 19.2; three of 2048 x 512 (672) 30.4 / 31.0 / 30.4 -> 29.1 / 29.3 / 27.6; four
+    // of 1024 x 512, eight experts (768) 23.0 / 23.4 / 23.4 -> 23.8 / 23.2 / 22.8: even. (All-IQ2_XXS tables leave room for one workgroup only.)
+    static constexpr uint32_t kTokenSliceGroups = 680u;
+    bool token_slices(uint32_t ntok) const {
+        return mixed_slices && dense_routed && small_batch(ntok) && ntok * (cfg.ffn / 32u) * (cfg.top_k + 4u) <= kTokenSliceGroups;
+    }
     // the same batches on a mixed layout run on the single-token kernels, one grid layer per token (tokens rarely share an
     // expert at these sizes, so reading a shared expert twice costs less than the pair sort and the per-pair kernels)
     bool small_batch_mixed(uint32_t ntok) const {
@@ -170,6 +176,8 @@ struct Moe {
         return small_batch_mixed(ntok) && ntok >= from && (words || cfg.ffn <= 768u) &&
                (words || (quant_supported(dn_type) && (8u * rbd) % 16u == 0u && (8u * rbs) % 16u == 0u && (2u * gate_bytes) % 16u == 0u && (2u * sh_gate_bytes) % 16u == 0u));
     }
+    // behind the layer's own router: selection and pair sort in front of the experts' kernels (or inside the grouped gate/up kernel)
+    bool group_in_select(uint32_t ntok) const { return slices_after_router(ntok) || (grouped_mixed(ntok) && !token_slices(ntok)); }
     // a handle that takes chunks on IQ2_XS / IQ1_M experts keeps tile-major copies of the gate | up streams (`tiled`) and of the down streams (`tiled_down`)
     bool stream_tiles_resident() const {
         const bool gu_cb = gu_type == T_IQ2_XS || gu_type == T_IQ1_M, dn_cb = dn_type == T_IQ2_XS || dn_type == T_IQ1_M;
@@ -282,7 +290,7 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
         prof_set_stage(ST_OTHER);
         return 1;
     }
-    if (m->grouped_mixed(ntok, grouped ? 2u : Moe::kGroupedMin) && m->shared_gu_ready) {      // xh / xl / xexp / scalar and the shared gate | up products (m->act) come from the router launch
+    if (m->grouped_mixed(ntok, grouped ? 2u : Moe::kGroupedMin) && m->shared_gu_ready && !(select_here && !grouped)) {      // xh / xl / xexp / scalar and the shared gate | up products (m->act) come from the router launch
         const Layer &L = m->layers[layer];
         if (!grouped) {
             prof_set_stage(ST_GROUP);
@@ -952,7 +960,7 @@ int redhip_moe_forward(redhip_moe_t h, uint32_t layer, const float *x_dev, uint3
         }
         return ok;
     }
-    const bool group_in_select = m->slices_after_router(ntok) || m->grouped_mixed(ntok);
+    const bool group_in_select = m->group_in_select(ntok);
     const bool select_in_gateup = m->packed_gu() && (ntok == 1u || m->small_batch_mixed(ntok)) && !group_in_select;
     m->skip_select = select_in_gateup || group_in_select;      // small batches: the batched gate/up kernel selects and sorts the pairs itself
     const int routed = redhip_moe_route(h, layer, x_dev, ntok, nullptr, nullptr, nullptr, stream);
@@ -994,7 +1002,7 @@ int redhip_moe_forward_block(redhip_moe_t h, uint32_t layer, const float *x_dev,
         if (hipGetLastError() != hipSuccess) { moe_err("residual + norm launch failed"); ok = 0; }
     }
     if (ok) {
-        const bool group_in_select = m->slices_after_router(ntok) || m->grouped_mixed(ntok);
+        const bool group_in_select = m->group_in_select(ntok);
         const bool select_in_gateup = m->packed_gu() && (ntok == 1u || m->small_batch_mixed(ntok)) && !group_in_select;
         m->skip_select = select_in_gateup || group_in_select;
         if (in_router) { bc.branch = branch_dev; bc.norm_w = post_norm_dev; bc.eps = eps; bc.xn_out = m->xn; }

@@ -124,8 +124,8 @@ struct Moe {
     // the routed experts' tile kernels, which leave most of the machine's issue slots free; forked and joined with events
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-    void *act_h = nullptr, *act_l = nullptr; // fp16 [top_k + 1][ffn] each
-    int *act_exp = nullptr;                  // [top_k + 1][ffn / 32]
+    void *act_h = nullptr, *act_l = nullptr; // fp16 [top_k + 1][ffn] each, of up to eight tokens
+    int *act_exp = nullptr;                  // [top_k + 1][ffn / 32], likewise
 
     // mixed layouts whose batches of 2..8 tokens run as expert slices: gate/up packed IQ2_XXS, down IQ3_S (column-sliced words), the shared
     // expert from its dense f32 copies, an f32 router (or the f32 copy of a quantised one) in the launch that leaves the shared gate | up products;
@@ -556,12 +556,13 @@ redhip_moe_t redhip_moe_create(const redhip_moe_config *cfg) {
         }
     }
     const size_t T = c.max_tokens;
+    const size_t TA = T < 8u ? T : 8u;               // tokens with activations as fp16 halves: one, or a small batch (chunks keep them in f32)
     const size_t partial_tokens = m->fused ? Moe::kSmallMaxRouted : Moe::kSmallMaxMixed;      // the largest batch that runs as expert slices
     const size_t partial_bytes = m->fused || m->mixed_slices ? align256((size_t)(c.max_tokens < partial_tokens ? c.max_tokens : partial_tokens) * (c.top_k + 1u) * (c.ffn / 32u) * c.hidden * 4u) : 0u;
     const size_t ws_bytes = partial_bytes + align256(8u * 512u) + align256(4u) + align256(4u) + align256(T * c.hidden * 4u) + align256(T * (c.n_expert + 1u) * 4u) + 2u * align256(T * c.top_k * 4u) + align256(T * 4u) +
                             align256(T * c.top_k * c.ffn * 4u) + align256(T * c.ffn * 4u) +
-                            2u * align256(2u * T * c.hidden) + align256(4u * T) + 2u * align256(2u * T * (c.top_k + 1u) * c.ffn) +
-                            align256(4u * T * (c.top_k + 1u) * (c.ffn / 32u)) +
+                            2u * align256(2u * T * c.hidden) + align256(4u * T) + 2u * align256(2u * TA * (c.top_k + 1u) * c.ffn) +
+                            align256(4u * TA * (c.top_k + 1u) * (c.ffn / 32u)) +
                             (T > 1u ? 6u * align256(4u * (T * c.top_k + 2u)) + align256(4u * T * c.top_k * c.hidden) + align256(4u * T * c.hidden) +
                                           4u * align256(12u * (size_t)prefill_tile_bound(c.max_tokens, c.top_k, c.n_expert)) : 0u);      // (three tile lists)
     ok = ok && hipMalloc(reinterpret_cast<void **>(&m->ws), ws_bytes) == hipSuccess;
@@ -585,9 +586,9 @@ redhip_moe_t redhip_moe_create(const redhip_moe_config *cfg) {
     m->xh = w; w += align256(2u * T * c.hidden);
     m->xl = w; w += align256(2u * T * c.hidden);
     m->xexp = reinterpret_cast<int *>(w); w += align256(4u * T);
-    m->act_h = w; w += align256(2u * T * (c.top_k + 1u) * c.ffn);
-    m->act_l = w; w += align256(2u * T * (c.top_k + 1u) * c.ffn);
-    m->act_exp = reinterpret_cast<int *>(w); w += align256(4u * T * (c.top_k + 1u) * (c.ffn / 32u));
+    m->act_h = w; w += align256(2u * TA * (c.top_k + 1u) * c.ffn);
+    m->act_l = w; w += align256(2u * TA * (c.top_k + 1u) * c.ffn);
+    m->act_exp = reinterpret_cast<int *>(w); w += align256(4u * TA * (c.top_k + 1u) * (c.ffn / 32u));
     if (T > 8u && m->mixed) {
         if (hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking) != hipSuccess || hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&m->ev_join, hipEventDisableTiming) != hipSuccess) {

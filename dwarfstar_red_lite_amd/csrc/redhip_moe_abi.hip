@@ -138,7 +138,8 @@ struct Moe {
     // batches that run as expert slices per pass: 2..8 tokens and at most 128 pairs on mixed layouts (their first launch multiplies the
     // shared expert's gate | up rows for up to eight tokens), 2..16 tokens and at most 256 pairs on all-IQ2_XXS layers - 2..32 tokens and
     // 512 pairs behind the layer's own router (own_router: the selection launch sorts that many; a caller's routing is sorted by one more
-    // workgroup of the launch that splits the activations, up to 256 pairs)
+    // workgroup of the launch that splits the activations, up to 256 pairs). Behind the own router the slices are ahead of the tiles up to
+    // there: 17, 24, 32 tokens 77 / 90, 98 / 111, 124 / 130 us, IQ3_S down 87 / 107, 109 / 122, 135 / 137, IQ2_XS 90 / 117, 114 / 136, 141 / 152
     static constexpr uint32_t kSmallMaxFused = 16u, kSmallMaxRouted = 32u, kSmallMaxGiven = 24u, kSmallMaxMixed = 32u;
     bool dense_routed = false;               // every layer has f32 copies of its router and of the shared expert's gate | up rows (set at creation)
     bool small_batch(uint32_t ntok, bool own_router = false) const {
@@ -930,8 +931,10 @@ int redhip_moe_experts(redhip_moe_t h, uint32_t layer, const float *x_dev, uint3
         }
         if (m->fused && !grouped && !m->small_batch(ntok) && m->small_batch(ntok, true) && ntok <= Moe::kSmallMaxGiven) {
             // 17..24 tokens on an all-IQ2_XXS layer: more pairs than the side job above sorts; one more launch sorts them with their pass list.
-            // (The slices cost a pass per two pairs of an expert, the tile kernels a decode per distinct expert: with 32 hot experts the
-            // slices took 58.5 / 74.2 / 93.2 us at 17 / 24 / 32 tokens against 67.9 / 79.2 / 84.5 us on the tiles.)
+            // (The slices cost a pass per two pairs of an expert, the tile kernels a decode per distinct expert, and the call does not know its
+            // routing. Slices / tiles at 17, 24, 32 tokens, us: evenly routed 69 / 84, 88 / 101, 110 / 111; Zipf popularity 61 / 68, 77 / 79, 98 /
+            // 90; 32 hot experts 57 / 57, 73 / 65, 92 / 75. Mixed layouts (above), IQ2_XS: even 87 / 108, 109 / 124, 135 / 142; Zipf 78 / 94,
+            // 97 / 105, 121 / 113; hot 73 / 80, 91 / 86, 116 / 94.)
             const GroupJob big{ids_dev, weights_dev, ntok, m->cfg.top_k, m->cfg.n_expert, m->uid, m->expert_start, m->pair_token, m->pair_weight, m->tok_pair, m->n_unique,
                                m->status, m->pass_list, m->n_pass};
             prof_set_stage(ST_GROUP);

@@ -4,14 +4,14 @@
 // Reference behaviour this replaces: native/redmetal_engine_prefill.m:1246-1330 (grouped GEMM over expert slices)
 // with the arithmetic of native/redlite_native_reference.c:251-382.
 //
-// What bounds these kernels is the decode (LDS table reads and vector issue; every weight is decoded once per tile), so the rows must cost
-// nothing extra. Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights
+// What bounds these kernels is the decode (every weight is decoded once per tile): 512 raw IQ2_XXS experts with ten pairs each keep the LDS busy
+// 57 % of the gate/up launch (half of that conflicts of the table reads), the vector pipes 61 %, the matrix pipes 22 %, in waves that take
+// turns. So the rows must cost nothing extra. Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights
 // of row r, D[i = 4q .. 4q + 3][j = r]: the lane's own row against four pairs. Which columns the instruction's k stand for is free as
 // long as both operands agree: step s of a block of 256 columns takes columns 64 q + 8 s .. + 7 of it, so lane (r, q) decodes quarter q of
 // its row's block and nothing else. Its fields are one 16-byte load (XS 4, IQ3_S 12 more bytes) that no other lane repeats, the four lanes
 // of a row read 64 consecutive bytes, every bit position is a constant, and a scale (per 16 or 32 columns) is formed once for the
-// entries that share it. (With step s = group s of the block, every lane of a row loaded all of it: four times the requests; rows staged in LDS
-// as they lie, 2-byte aligned: more than half of the LDS cycles were unaligned stalls.)
+// entries that share it. (With step s = group s of the block, every lane of a row would load all of it: four times the requests.)
 //
 // K is cut into KP blocks of 256 columns, and NRT row tiles of 16 rows are in work beside each other (KP * NRT = 8; 6 with three
 // blocks). A unit is two halves ("m") of 16 NRT rows: the gate and the up rows of 16 NRT FFN columns, or 32 NRT rows of a down matrix.

@@ -268,11 +268,12 @@ struct StagedMatrices {
     uint64_t stride, up_delta;
     const int8_t *grid;                     // codebook of IQ2_XS / IQ1_M
 };
+constexpr uint32_t kWideUnknown = 0xffffffffu;
 struct StagedChunk {                        // the pair sort of the call, its tile lists among it
     const uint32_t *pair_token;
     TileLists tl;
     uint32_t ntok, top_k, n_expert;
-    uint32_t wide_tiles = 0xffffffffu;      // tiles of more than kPrefillTile pairs, where the host knows their number
+    uint32_t wide_tiles = kWideUnknown;     // tiles of more than kPrefillTile pairs, where the host knows their number
 };
 bool staged_gateup_supported(uint32_t type, RowLayout lay, uint32_t hidden, uint32_t ffn);
 bool staged_down_supported(uint32_t type, RowLayout lay, uint32_t hidden, uint32_t ffn);

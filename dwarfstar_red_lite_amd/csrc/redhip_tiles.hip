@@ -5,7 +5,7 @@
 // with the arithmetic of native/redlite_native_reference.c:251-382.
 //
 // What bounds these kernels is the decode (every weight is decoded once per tile): 512 raw IQ2_XXS experts with ten pairs each keep the LDS busy
-// 57 % of the gate/up launch (half of that conflicts of the table reads), the vector pipes 61 %, the matrix pipes 22 %, in waves that take
+// 58 % of the gate/up launch (half of that conflicts of the table reads), the vector pipes 67 %, the matrix pipes 24 %, in waves that take
 // turns. So the rows must cost nothing extra. Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights
 // of row r, D[i = 4q .. 4q + 3][j = r]: the lane's own row against four pairs. Which columns the instruction's k stand for is free as
 // long as both operands agree: step s of a block of 256 columns takes columns 64 q + 8 s .. + 7 of it, so lane (r, q) decodes quarter q of
@@ -388,13 +388,14 @@ hipError_t launch_staged_list(const StagedArgs &a, uint32_t grid, hipStream_t s)
     REDHIP_LAUNCH((staged_tiles_kernel<SRC, DOWN, SETS, KP>), dim3(grid), dim3(staged_threads(SETS, KP)), 0, s, a);
     return hipGetLastError();
 }
-// wide: wide tiles that the chunk can have at most
+// wide: wide tiles that the chunk is expected to have
 template <int SRC, bool DOWN, uint32_t KP>
 hipError_t launch_staged_lists(StagedArgs a, uint32_t grid, uint32_t wide, hipStream_t s) {
     a.few = few_wide<SRC, DOWN>(a.rows, 256u * KP);
     hipError_t e = hipSuccess;
+    if (wide < a.few) a.few = ~0u;                         // (without a wide launch the narrow one takes everything)
     if constexpr (has_wide<SRC, DOWN>()) {
-        if (wide >= a.few) e = launch_staged_list<SRC, DOWN, 2, KP>(a, grid, s);
+        if (a.few != ~0u) e = launch_staged_list<SRC, DOWN, 2, KP>(a, grid, s);
     }
     return e == hipSuccess ? launch_staged_list<SRC, DOWN, 1, KP>(a, grid, s) : e;
 }
@@ -439,9 +440,14 @@ uint32_t staged_grid(const StagedChunk &c) {
     const uint32_t bound = 4u * prefill_tile_bound(c.ntok, c.top_k, c.n_expert);
     return bound < 256u ? bound : 256u;
 }
-uint32_t staged_wide(const StagedChunk &c) {           // a wide tile has 17 pairs or more
-    const uint32_t most = c.ntok * c.top_k / (kPrefillTile + 1u) + c.tl.shared_ntok / (kPrefillTile + 1u);
-    return c.wide_tiles < most ? c.wide_tiles : most;
+// Wide tiles that a chunk will have: counted by the caller, or guessed. A launch that finds too few costs 5 us, and a wide tile has 17 pairs or
+// more, so a chunk has at most pairs / 17 of them: 0.37 of that with Zipf-popular experts (512 and 1024 tokens, top 10 of 512), next to none
+// at ten evenly routed pairs per expert, one for nearly every expert from 23 pairs on, a further one per 32 from 42 on.
+uint32_t staged_wide(const StagedChunk &c) {
+    if (c.wide_tiles != kWideUnknown) return c.wide_tiles;
+    const uint32_t pairs = c.ntok * c.top_k, E = c.n_expert, popular = pairs / (kPrefillTile + 1u) * 2u / 5u, first = pairs > 10u * E ? (pairs - 10u * E) / 13u : 0u;
+    const uint32_t routed = (first < E ? first : E) + (pairs > 42u * E ? (pairs - 42u * E) / kPrefillWideTile : 0u);
+    return (routed < popular ? popular : routed) + c.tl.shared_ntok / kPrefillWideTile;
 }
 
 }  // namespace

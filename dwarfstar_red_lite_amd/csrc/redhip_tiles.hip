@@ -112,9 +112,9 @@ __device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t
     // off (f32 multiplications: 2.1e-7); with one chain for everything it was 2.9e-7, in 3 .. 5 % less time. Packed rows (all-IQ2_XXS, ffn
     // above 512) take two steps per chain: 1.75e-7 instead of 1.9e-7, 5 % of the time.
     constexpr uint32_t kChain = layout<SRC>() == L_ROWS ? 2u : 4u;
-    constexpr bool kSumInLds = SETS == 1 ? SRC == S_IQ3 : fmt<SRC>() != F_XXS || layout<SRC>() == L_ROWS;
+    constexpr bool kSumInLds = SRC == S_IQ3 || (SETS == 2 && layout<SRC>() == L_ROWS);
     // units on their way: two, one where the registers hold no second (a spill to scratch memory would be counted among the loads that the waits count)
-    constexpr uint32_t kCarried = SRC == S_IQ3 || (SETS == 2 && SRC == S_M) ? 1u : 2u;
+    constexpr uint32_t kCarried = SRC == S_IQ3 || (SETS == 2 && fmt<SRC>() != F_XXS) ? 1u : 2u;
     H8 xa[SETS][8], xb[SETS][8];
     // Powers of two that the products of a pair are multiplied with. Down: of this wave's block. Gate/up: of the token, so the sums over the
     // blocks take them; a tile's stand in row tile % 4: a tile has two units or

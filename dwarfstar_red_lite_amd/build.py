@@ -1,4 +1,4 @@
-"""Builds libredmetal_hip.so (gfx950) in-tree with hipcc. Run on the CPU-only build machine; the GPU box loads the
+"""Builds libredmetal_hip.so (gfx950) in-tree with hipcc. Run on the CPU-only build machine; the machine with the GPU loads the
 prebuilt library. Every source is compiled to an object of its own (in parallel), then linked."""
 import os
 import subprocess

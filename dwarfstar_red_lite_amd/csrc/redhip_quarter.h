@@ -1,6 +1,9 @@
 // Rows of the expert formats, decoded a quarter block (64 of 256 columns) per lane into eight signed, scaled fp16 weights at a time: what
 // the MFMA kernels on tiles of tokens and on one token share.
 #pragma once
+#include <type_traits>
+#include <utility>
+
 #include "redhip_mfma.h"
 
 namespace redhip {
@@ -8,6 +11,16 @@ namespace redhip {
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 union H8 { uint4 u; half8_t v; half2_t p[4]; _Float16 e[8]; };
+
+// A SIMD takes the simple 32-bit instructions (and, or, xor, bitop3, add, sub, right shifts; f32 add, mul, fma) of two waves side by side as
+// long as every operand is a vector register or an inline constant: 2.2 .. 2.6 cycles each with four waves. With a scalar register or a
+// literal among the operands, and for left shifts, bit-field extracts, permutes, and_or, lshl_or and packed fp16, it is 4.3. So the decode
+// keeps its masks in vector registers, shifts left by additions and merges by bitop3.
+__device__ __forceinline__ uint32_t in_vector(uint32_t k) { asm("" : "+v"(k)); return k; }
+__device__ __forceinline__ uint32_t twice(uint32_t v) { uint32_t r; asm("v_add_u32 %0, %1, %1" : "=v"(r) : "v"(v)); return r; }
+__device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0xea); }
+// bits of w, those at position `from` moved to `to`
+template <uint32_t FROM, uint32_t TO> __device__ __forceinline__ uint32_t moved(uint32_t w) { return FROM >= TO ? w >> (FROM >= TO ? FROM - TO : 0u) : w << (FROM < TO ? TO - FROM : 0u); }
 
 // row sources: format (low half, what the decode goes by) and layout
 enum : int { F_XXS = 0, F_XS = 1, F_M = 2, F_IQ3 = 3, F_IQ3_WORDS = 4, L_RAW = 0, L_ROWS = 8, L_TILED = 16 };
@@ -31,14 +44,14 @@ template <int SRC> __device__ __forceinline__ uint32_t step_column(uint32_t s, u
 //   IQ2_XXS: the eight fp16 magnitudes of every grid entry times every group scale 2 s + 1 (64 KB, exact), at entry * 256 + s * 16: the address is
 //   the entry's byte over the top byte of the group's second word, one byte permute and one mask; IQ3_S likewise (four magnitudes, by scale)
 //   IQ2_XS: the fp16 codebook eight times, lane l reading copy l % 8 - a wave's 16-byte reads then hit every bank evenly (random entries of
-//   one copy: 2.6 times the cycles); IQ1_M: its fp16 codebook twice
+//   one copy: 2.6 times the cycles); IQ1_M: its codebook with the offset of +1/8 and of -1/8, at (offset sign << 15 | entry << 4)
 //   Small tables (32 KB, IQ3_S 16): IQ2_XXS and IQ3_S without the scales, eight and four copies; IQ2_XS four copies, IQ1_M one
 //   signs: bit 15 - i / 31 - i of the word of a sign field = signs of weights 2i and 2i + 1, so a pair's signs are one shift and one and-or;
 //   replicated so that the reads are (nearly) free of conflicts. (Sign masks as 16-byte entries save three shifts per eight weights and cost
 //   a second conflicting 16-byte read: LDS, the tighter of the two pipes, loses more.)
 template <int SRC> constexpr bool is_iq3() { return fmt<SRC>() == F_IQ3 || fmt<SRC>() == F_IQ3_WORDS; }
-template <int SRC> constexpr uint32_t sign_copies() { return fmt<SRC>() == F_M ? 0u : (is_iq3<SRC>() ? 4u : 16u) / (small_tables<SRC>() ? is_iq3<SRC>() ? 2u : 4u : 1u); }
-template <int SRC> constexpr uint32_t sign_shift() { return sign_copies<SRC>() == 16u ? 6u : sign_copies<SRC>() == 4u ? 4u : 3u; }
+template <int SRC> constexpr uint32_t sign_copies() { return fmt<SRC>() == F_M ? 0u : small_tables<SRC>() ? (is_iq3<SRC>() ? 2u : 4u) : is_iq3<SRC>() ? 4u : 32u; }
+template <int SRC> constexpr uint32_t sign_shift() { return sign_copies<SRC>() == 32u ? 7u : sign_copies<SRC>() == 4u ? 4u : 3u; }
 template <int SRC> constexpr uint32_t sign_bytes() { return (is_iq3<SRC>() ? 256u : 128u) * sign_copies<SRC>() * 4u; }
 constexpr uint32_t kEntryBytes = 65536u;
 
@@ -75,8 +88,20 @@ __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *
                 *reinterpret_cast<uint4 *>(entries + (size_t)e * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
             }
         }
-    } else if constexpr (fmt<SRC>() == F_XS || fmt<SRC>() == F_M) {
-        constexpr uint32_t kCopies = fmt<SRC>() == F_XS ? 8u : 2u, kEntries = kEntryBytes / (16u * kCopies);
+    } else if constexpr (fmt<SRC>() == F_M) {
+        for (uint32_t e = tid; e < 2048u; e += T) {
+            const uint64_t ge = reinterpret_cast<const uint64_t *>(grid)[e];
+#pragma unroll
+            for (uint32_t neg = 0; neg < 2u; ++neg) {
+                const float off = neg ? -0.125f : 0.125f;      // (exact: a byte and three bits behind the point)
+                uint32_t w4[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w4[i] = two_halves((float)(int8_t)(ge >> (16 * i)) + off, (float)(int8_t)(ge >> (16 * i + 8)) + off);
+                *reinterpret_cast<uint4 *>(entries + neg * 32768u + e * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+            }
+        }
+    } else if constexpr (fmt<SRC>() == F_XS) {
+        constexpr uint32_t kCopies = 8u, kEntries = kEntryBytes / (16u * kCopies);
         for (uint32_t e = tid; e < kEntries; e += T) {
             const uint64_t ge = reinterpret_cast<const uint64_t *>(grid)[e];
             uint32_t w4[4];
@@ -99,7 +124,7 @@ __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *
 // wait for), then written. Tables with copies are written by two threads per entry, half of the copies each.
 template <int SRC> constexpr uint32_t codebook_entries() { return fmt<SRC>() == F_XXS ? 256u : fmt<SRC>() == F_M ? 2048u : 512u; }
 template <int SRC> constexpr uint32_t small_copies() { return fmt<SRC>() == F_XXS ? 8u : fmt<SRC>() == F_M ? 1u : 4u; }
-template <int SRC> constexpr uint32_t entry_shift() { return !small_tables<SRC>() ? (fmt<SRC>() == F_M ? 5u : 7u) : fmt<SRC>() == F_XXS ? 7u : fmt<SRC>() == F_XS ? 6u : fmt<SRC>() == F_M ? 4u : 5u; }
+template <int SRC> constexpr uint32_t entry_shift() { return !small_tables<SRC>() ? (fmt<SRC>() == F_M ? 4u : 7u) : fmt<SRC>() == F_XXS ? 7u : fmt<SRC>() == F_XS ? 6u : fmt<SRC>() == F_M ? 4u : 5u; }
 template <int SRC> constexpr uint32_t small_entry_bytes() { return codebook_entries<SRC>() << entry_shift<SRC>(); }
 template <int SRC, uint32_t T> struct SmallSeeds {
     static constexpr uint32_t kHalves = small_copies<SRC>() > 1u ? 2u : 1u, kItems = codebook_entries<SRC>() * kHalves, N = (kItems + T - 1u) / T;
@@ -192,82 +217,119 @@ __device__ __forceinline__ float quarter_d(uint2 d) {
     else return scale_to_f32(d.x);
 }
 
-// odd integer 2 s + 1 (s < 16) as two equal fp16 halves: 1024 + (2 s + 1) by integer arithmetic, minus 1024, exact
-__device__ __forceinline__ half2_t odd_splat(uint32_t s) {
-    const half2_t big = {(_Float16)1024.0f, (_Float16)1024.0f};
-    return __builtin_bit_cast(half2_t, __umul24(s, 0x20002u) + 0x64016401u) - big;
+// odd integer 2 s + 1 as two equal fp16 halves, s the BITS bits of w at AT: 1024 + (2 s + 1) by integer arithmetic, minus 1024, exact
+template <uint32_t AT, uint32_t BITS> __device__ __forceinline__ half2_t odd_splat(uint32_t w) {
+    const uint32_t big = and_or(moved<AT, 1u>(w), (2u << BITS) - 2u, 0x6401u);
+    const _Float16 h = __builtin_bit_cast(_Float16, (uint16_t)big);
+    return half2_t{h, h} - half2_t{(_Float16)1024.0f, (_Float16)1024.0f};
 }
 
-// lane constants of the tables: addresses of the lane's copy
-struct LaneTables { const uint8_t *entries; const uint8_t *signs; };
+// f(constant 0) .. f(constant 7): the steps of a quarter block
+template <class F, uint32_t... S> __device__ __forceinline__ void each_step_of(F &&f, std::integer_sequence<uint32_t, S...>) { (f(std::integral_constant<uint32_t, S>{}), ...); }
+template <uint32_t N, class F> __device__ __forceinline__ void each(F &&f) { each_step_of(f, std::make_integer_sequence<uint32_t, N>{}); }
+template <class F> __device__ __forceinline__ void each_step(F &&f) { each_step_of(f, std::make_integer_sequence<uint32_t, 8>{}); }
+
+// lane constants of the tables: addresses of the lane's copy, masks in vector registers
+struct LaneTables {
+    const uint8_t *entries, *signs;        // (signs: the lane's copy is or-ed into the offset)
+    uint32_t entry_mask, sign_mask, sign_lane, scale_mask, sign_bits;
+};
+template <int SRC> constexpr uint32_t entry_copies() { return small_tables<SRC>() ? small_copies<SRC>() : fmt<SRC>() == F_XS ? 8u : 1u; }
+template <int SRC> __device__ __forceinline__ LaneTables lane_tables(const uint8_t *entries, const uint32_t *signs, uint32_t tid) {
+    constexpr uint32_t C = sign_copies<SRC>() ? sign_copies<SRC>() : 1u, E = is_iq3<SRC>() ? 8u : 16u, ES = entry_shift<SRC>();
+    LaneTables t;
+    t.entries = entries + (tid % entry_copies<SRC>()) * E;
+    t.signs = reinterpret_cast<const uint8_t *>(signs);
+    t.sign_lane = (tid % C) * 4u;
+    t.sign_mask = in_vector((is_iq3<SRC>() ? 255u : 127u) << sign_shift<SRC>());
+    t.entry_mask = in_vector(fmt<SRC>() == F_XS ? 511u << ES : fmt<SRC>() == F_XXS ? 255u << ES : fmt<SRC>() == F_M ? 255u << ES : fmt<SRC>() == F_IQ3_WORDS ? 0xff8u : 255u << 3);
+    t.scale_mask = in_vector(0xf000u);
+    t.sign_bits = in_vector(0x80008000u);
+    return t;
+}
 
 // Table reads of step s (eight columns) of a quarter, then the arithmetic on what they return: the eight signed, scaled fp16 weights.
-// s is a constant after unrolling.
 struct Entry { uint4 m; uint32_t s; };
 __device__ __forceinline__ uint32_t word_of(const uint4 &v, uint32_t i) { return i == 0u ? v.x : i == 1u ? v.y : i == 2u ? v.z : v.w; }
-template <int SRC>
-__device__ __forceinline__ Entry fetch_entry(const Quarter &v, uint32_t s, const LaneTables &t) {
-    const uint32_t h = s >> 2, e = s & 3u;                 // group of the quarter, entry of the group
+template <int SRC, uint32_t S>
+__device__ __forceinline__ Entry fetch_entry(const Quarter &v, const LaneTables &t) {
+    constexpr uint32_t h = S >> 2, e = S & 3u, ES = entry_shift<SRC>(), SS = sign_shift<SRC>();                 // group of the quarter, entry of the group
+    const auto entry = [&](uint32_t off) { return *reinterpret_cast<const uint4 *>(t.entries + off); };
+    const auto half_entry = [&](uint32_t off) { return *reinterpret_cast<const uint2 *>(t.entries + off); };
+    const auto sign = [&](uint32_t w) { return *reinterpret_cast<const uint32_t *>(t.signs + and_or(w, t.sign_mask, t.sign_lane)); };
     Entry r;
     if constexpr (fmt<SRC>() == F_XXS) {
         const uint32_t wa = h ? v.a.z : v.a.x, wb = h ? v.a.w : v.a.y;
         // bytes 0 .. 3 of the permute's second operand are the entries, 7 the top byte of the first
-        if constexpr (small_tables<SRC>()) r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_ubfe(wa, 8u * e, 8u) << entry_shift<SRC>()));
-        else r.m = *reinterpret_cast<const uint4 *>(t.entries + __builtin_amdgcn_perm(wb & 0xf0000000u, wa, 0x0c0c0007u | (e << 8)));
-        r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(wb, 7u * e, 7u) << sign_shift<SRC>()));
+        if constexpr (small_tables<SRC>()) r.m = entry(moved<8u * e, ES>(wa) & t.entry_mask);
+        else r.m = entry(__builtin_amdgcn_perm(wb & 0xf0000000u, wa, 0x0c0c0007u | (e << 8)));
+        r.s = sign(moved<7u * e, SS>(wb));
     } else if constexpr (fmt<SRC>() == F_XS) {
-        const uint32_t w = word_of(v.a, 2u * h + (e >> 1)), o = 16u * (e & 1u);
-        r.m = *reinterpret_cast<const uint4 *>(t.entries + (__builtin_amdgcn_ubfe(w, o, 9u) << entry_shift<SRC>()));
-        r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(w, o + 9u, 7u) << sign_shift<SRC>()));
+        const uint32_t w = word_of(v.a, 2u * h + (e >> 1));
+        constexpr uint32_t o = 16u * (e & 1u);
+        r.m = entry(moved<o, ES>(w) & t.entry_mask);
+        r.s = sign(moved<o + 9u, SS>(w));
     } else if constexpr (fmt<SRC>() == F_IQ3_WORDS) {
-        const uint32_t w = word_of(h ? v.b : v.a, e), scale = (w >> 14) & 0xf000u;      // nibble * 512 entries * 8 bytes
-        const uint2 ma = *reinterpret_cast<const uint2 *>(t.entries + (((w << 3) & 0xff8u) | scale));
-        const uint2 mb = *reinterpret_cast<const uint2 *>(t.entries + (((w >> 6) & 0xff8u) | scale));
+        const uint32_t w = word_of(h ? v.b : v.a, e), top = w >> 14, scale = top & t.scale_mask;      // nibble * 512 entries * 8 bytes
+        const uint2 ma = half_entry(and_or(w << 3, t.entry_mask, scale)), mb = half_entry(and_or(w >> 6, t.entry_mask, scale));
         r.m = make_uint4(ma.x, ma.y, mb.x, mb.y);
-        r.s = *reinterpret_cast<const uint32_t *>(t.signs + ((w >> 14) & 0xff0u));
+        r.s = sign(top);
     } else if constexpr (fmt<SRC>() == F_M) {
-        r.s = __builtin_amdgcn_ubfe(v.a.z, 16u * h + 4u * e, 4u);
-        r.m = *reinterpret_cast<const uint4 *>(t.entries + ((__builtin_amdgcn_ubfe(h ? v.a.y : v.a.x, 8u * e, 8u) | ((r.s & 7u) << 8)) << entry_shift<SRC>()));
+        const uint32_t idx = h ? v.a.y : v.a.x;
+        if constexpr (small_tables<SRC>()) {
+            r.s = __builtin_amdgcn_ubfe(v.a.z, 16u * h + 4u * e, 4u);
+            r.m = entry((__builtin_amdgcn_ubfe(idx, 8u * e, 8u) | ((r.s & 7u) << 8)) << ES);
+        } else {
+            r.s = 0u;
+            r.m = entry(and_or(moved<8u * e, 4u>(idx), t.entry_mask, moved<16u * h + 4u * e, 12u>(v.a.z) & t.scale_mask));
+        }
     } else {
-        const uint32_t w = word_of(v.a, 2u * h + (e >> 1)), o = 16u * (e & 1u);
-        const uint32_t scale = h ? (v.c >> 8) & 0xf000u : (v.c >> 4) & 0xf000u;      // nibble * 512 entries * 8 bytes
-        const uint32_t ba = 8u * h + 2u * e, bb = ba + 1u;     // qh bits of the two entries -> bit 11
-        const uint32_t ha = (ba > 11u ? v.c >> (ba - 11u) : v.c << (11u - ba)) & 2048u, hb = (bb > 11u ? v.c >> (bb - 11u) : v.c << (11u - bb)) & 2048u;
-        uint32_t ia = (__builtin_amdgcn_ubfe(w, o, 8u) << 3) | ha, ib = (__builtin_amdgcn_ubfe(w, o + 8u, 8u) << 3) | hb;      // entry * 8
+        const uint32_t w = word_of(v.a, 2u * h + (e >> 1));
+        constexpr uint32_t o = 16u * (e & 1u), ba = 8u * h + 2u * e, bb = ba + 1u;     // qh bits of the two entries -> bit 11
+        const uint32_t scale = moved<h ? 20u : 16u, 12u>(v.c) & t.scale_mask;      // nibble * 512 entries * 8 bytes
+        const uint32_t ha = moved<ba, 11u>(v.c) & 2048u, hb = moved<bb, 11u>(v.c) & 2048u;
+        uint32_t ia = and_or(moved<o, 3u>(w), t.entry_mask, ha), ib = and_or(moved<o + 8u, 3u>(w), t.entry_mask, hb);      // entry * 8
         if constexpr (small_tables<SRC>()) { ia <<= 2; ib <<= 2; }
         else { ia |= scale; ib |= scale; }
-        const uint2 ma = *reinterpret_cast<const uint2 *>(t.entries + ia), mb = *reinterpret_cast<const uint2 *>(t.entries + ib);
+        const uint2 ma = half_entry(ia), mb = half_entry(ib);
         r.m = make_uint4(ma.x, ma.y, mb.x, mb.y);
-        r.s = *reinterpret_cast<const uint32_t *>(t.signs + (__builtin_amdgcn_ubfe(h ? v.b.y : v.b.x, 8u * e, 8u) << sign_shift<SRC>()));
+        r.s = sign(moved<8u * e, SS>(h ? v.b.y : v.b.x));
     }
     return r;
 }
 // f: the scale of the step's columns where the table does not hold it (sixteen columns IQ2_XS, IQ1_M; 32 the others, small tables)
 template <int SRC> constexpr uint32_t steps_per_scale() { return fmt<SRC>() == F_XS || fmt<SRC>() == F_M ? 2u : small_tables<SRC>() ? 4u : 0u; }
-template <int SRC>
-__device__ __forceinline__ half2_t step_scale(const Quarter &v, uint32_t s) {
-    const uint32_t h = s >> 2, e = s & 3u;
-    if constexpr (fmt<SRC>() == F_XS) return odd_splat(__builtin_amdgcn_ubfe(v.c, 8u * h + 4u * (e >> 1), 4u));
-    else if constexpr (fmt<SRC>() == F_M) return odd_splat(__builtin_amdgcn_ubfe(v.a.w, 6u * h + 3u * (e >> 1), 3u));
-    else if constexpr (fmt<SRC>() == F_XXS) return odd_splat((h ? v.a.w : v.a.y) >> 28);
-    else return odd_splat(__builtin_amdgcn_ubfe(v.c, 16u + 4u * h, 4u));
+template <int SRC, uint32_t S>
+__device__ __forceinline__ half2_t step_scale(const Quarter &v) {
+    constexpr uint32_t h = S >> 2, e = S & 3u;
+    if constexpr (fmt<SRC>() == F_XS) return odd_splat<8u * h + 4u * (e >> 1), 4u>(v.c);
+    else if constexpr (fmt<SRC>() == F_M) return odd_splat<6u * h + 3u * (e >> 1), 3u>(v.a.w);
+    else if constexpr (fmt<SRC>() == F_XXS) return odd_splat<28u, 4u>(h ? v.a.w : v.a.y);
+    else return odd_splat<16u + 4u * h, 4u>(v.c);
 }
 template <int SRC>
-__device__ __forceinline__ half8_t finish_entry(const Entry &e, half2_t f) {
-    constexpr uint32_t kSign = 0x80008000u;
+__device__ __forceinline__ half8_t finish_entry(const Entry &e, half2_t f, const LaneTables &t) {
     H8 r;
     r.u = e.m;
-    if constexpr (fmt<SRC>() == F_M) {
+    if constexpr (fmt<SRC>() == F_M && !small_tables<SRC>()) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * f;
+    } else if constexpr (fmt<SRC>() == F_M) {
         // (2 s + 1) / 8 with the sign of the offset: three exponent steps down (2 s + 1 >= 1 is a normal number), sign bit by xor
         const uint32_t neg = (e.s & 8u) << 12;
         const half2_t off = __builtin_bit_cast(half2_t, (__builtin_bit_cast(uint32_t, f) - 0x0c000c00u) ^ (neg | (neg << 16)));
 #pragma unroll
         for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * f + off;
-    } else if constexpr (fmt<SRC>() == F_XS || small_tables<SRC>()) {     // IQ2_XS entries are signed bytes in general: the sign goes to the (positive) scale
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * __builtin_bit_cast(half2_t, __builtin_bit_cast(uint32_t, f) | ((e.s << i) & kSign));
     } else {
-        r.u.x |= e.s & kSign; r.u.y |= (e.s << 1) & kSign; r.u.z |= (e.s << 2) & kSign; r.u.w |= (e.s << 3) & kSign;
+        const uint32_t s1 = twice(e.s), s2 = twice(s1), s3 = twice(s2);
+        if constexpr (fmt<SRC>() == F_XS || small_tables<SRC>()) {     // IQ2_XS entries are signed bytes in general: the sign goes to the (positive) scale
+            const uint32_t fb = __builtin_bit_cast(uint32_t, f);
+            r.p[0] *= __builtin_bit_cast(half2_t, and_or(e.s, t.sign_bits, fb));
+            r.p[1] *= __builtin_bit_cast(half2_t, and_or(s1, t.sign_bits, fb));
+            r.p[2] *= __builtin_bit_cast(half2_t, and_or(s2, t.sign_bits, fb));
+            r.p[3] *= __builtin_bit_cast(half2_t, and_or(s3, t.sign_bits, fb));
+        } else
+            r.u = make_uint4(and_or(e.s, t.sign_bits, e.m.x), and_or(s1, t.sign_bits, e.m.y), and_or(s2, t.sign_bits, e.m.z), and_or(s3, t.sign_bits, e.m.w));
     }
     return r.v;
 }

@@ -4,23 +4,22 @@
 // Reference behaviour this replaces: native/redmetal_engine_prefill.m:1246-1330 (grouped GEMM over expert slices)
 // with the arithmetic of native/redlite_native_reference.c:251-382.
 //
-// What bounds these kernels is the decode (every weight is decoded once per tile): 512 raw IQ2_XXS experts with ten pairs each keep the LDS busy
-// 58 % of the gate/up launch (half of that conflicts of the table reads), the vector pipes 67 %, the matrix pipes 24 %, in waves that take
-// turns. So the rows must cost nothing extra. Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights
+// What bounds these kernels is the decode: every weight is decoded once per tile, eight of them for about ten vector instructions and a table read
+// of 12 LDS cycles (conflicts of random entries), beside which the matrix instructions take 8 issue cycles each. So the rows must cost nothing
+// extra. Operand mapping (lane l, r = l % 16, q = l / 16): A[i = r][k = 8q .. 8q + 7] activations of pair r, B[k][j = r] weights
 // of row r, D[i = 4q .. 4q + 3][j = r]: the lane's own row against four pairs. Which columns the instruction's k stand for is free as
 // long as both operands agree: step s of a block of 256 columns takes columns 64 q + 8 s .. + 7 of it, so lane (r, q) decodes quarter q of
 // its row's block and nothing else. Its fields are one 16-byte load (XS 4, IQ3_S 12 more bytes) that no other lane repeats, the four lanes
 // of a row read 64 consecutive bytes, every bit position is a constant, and a scale (per 16 or 32 columns) is formed once for the
 // entries that share it. (With step s = group s of the block, every lane of a row would load all of it: four times the requests.)
 //
-// K is cut into KP blocks of 256 columns, and NRT row tiles of 16 rows are in work beside each other (KP * NRT = 8; 6 with three
-// blocks). A unit is two halves ("m") of 16 NRT rows: the gate and the up rows of 16 NRT FFN columns, or 32 NRT rows of a down matrix.
-// A wave keeps the activations of its block for the whole tile in registers (fp16 halves hi + lo 2^-11, 22 significant bits of every value
-// down to 2^-28 of the largest) and the rows of the next two units on their way; the blocks meet in LDS, one barrier per two units. Tiles of up to 16 pairs run sixteen waves, one half
-// each (64 registers of activations, four waves per SIMD: the reads and the arithmetic of different waves overlap), tiles of 17 .. 32
-// pairs eight waves with both halves and two sets of pairs per decoded weight, as a launch of their own. The SwiGLU activations go to
-// the down kernel as f32, so work is cut at any unit, not at groups of columns that share an exponent; the down kernel splits them per
-// pair and block when it loads them.
+// K is cut into KP blocks of 256 columns. The activations are fp16 halves hi + lo 2^-11 (22 significant bits of every value down to 2^-28 of the
+// largest). A tile's 16 pairs times 2048 columns fill a quarter of the vector registers, so gate/up keeps them there, split over the waves by
+// columns, and adds the waves' sums up in LDS; the 512 columns of a down tile fit the LDS, so there every wave has whole rows and nothing
+// is added up (with whole rows and the activations of 2048 columns passing through LDS block by block, gate/up took 171 instead of 144 us).
+// The SwiGLU activations go to the down kernel as f32, so work is cut at any unit, not at groups of columns that share an exponent.
+// 512 raw IQ2_XXS experts of 2048 x 512 with ten pairs each: gate/up 144 us (sixteen waves of one block, and the decode on full instruction rate
+// only: 166), down 83 (99, activations in registers too); 77 tokens of IQ1_M layers 96 + 48 (112 + 68).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -30,9 +29,6 @@
 namespace redhip {
 
 namespace {
-
-constexpr uint32_t staged_nrt(uint32_t KP) { return KP == 3u ? 2u : 8u / KP; }
-constexpr uint32_t staged_threads(int sets, uint32_t KP) { return 64u * KP * staged_nrt(KP) * (sets == 1 ? 2u : 1u); }
 
 struct StagedArgs {
     const uint8_t *experts, *shared;       // first matrix of expert e at experts + e * stride, of the shared expert at `shared`
@@ -58,344 +54,486 @@ __device__ __forceinline__ void wave_lds_barrier() {
 // (which the activations need) across the loop.
 __device__ __forceinline__ uint32_t each_trip(uint32_t v) { asm volatile("" : "+v"(v)); return v; }
 
-// What the units of a workgroup need to know of their tiles (gate/up: the pairs' tokens among it), fetched at the kernel's head by its
-// first wave while the others build the tables; tiles beyond the first kTileInfos are looked up when they begin.
+// exchange of two registers' halves between lanes that differ in bit 4 (16) or 5 (32)
+__device__ __forceinline__ void swap16(uint32_t &a, uint32_t &b) { const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false); a = r[0]; b = r[1]; }
+__device__ __forceinline__ void swap32(uint32_t &a, uint32_t &b) { const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false); a = r[0]; b = r[1]; }
+__device__ __forceinline__ void swap16(uint4 &a, uint4 &b) { swap16(a.x, b.x); swap16(a.y, b.y); swap16(a.z, b.z); swap16(a.w, b.w); }
+__device__ __forceinline__ void swap32(uint4 &a, uint4 &b) { swap32(a.x, b.x); swap32(a.y, b.y); swap32(a.z, b.z); swap32(a.w, b.w); }
+
+// What a workgroup needs to know of its tiles, fetched for up to kTileInfos of them at a time.
 constexpr uint32_t kTileInfos = 32u;
 struct TileInfo { uint64_t mat; uint32_t p0, n; };      // mat: distance of the expert's first matrix from StagedArgs::experts
+struct TileList { const uint32_t *expert, *pair0, *n; };
+__device__ __forceinline__ TileInfo tile_info(const StagedArgs &a, const TileList &l, uint32_t tile) {
+    const uint32_t e = l.expert[tile];
+    return TileInfo{e == kSharedTile ? (uint64_t)(a.shared - a.experts) : (uint64_t)e * a.stride, l.pair0[tile], l.n[tile]};
+}
+__device__ __forceinline__ TileInfo uniform_info(const TileInfo &t) {
+    const auto one = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane(v); };
+    return TileInfo{((uint64_t)one((uint32_t)(t.mat >> 32)) << 32) | one((uint32_t)t.mat), one(t.p0), one(t.n)};
+}
+// the lane's quarter of block kc of row tile `row_tile` of a matrix of `rows` rows
+template <int SRC, uint32_t KP>
+__device__ __forceinline__ void request_quarter(const StagedArgs &a, const uint8_t *mat, uint32_t row_tile, uint32_t r, uint32_t kc, uint32_t q, Quarter &v, uint2 &d) {
+    constexpr uint32_t tile_bytes = 16u * KP * src_block<SRC>();
+    load_quarter<SRC, KP>(mat + (uint64_t)row_tile * tile_bytes, mat + a.d_off + row_tile * (KP * 32u),
+                          fmt<SRC>() == F_XS ? mat + a.d_off + (uint64_t)a.rows * KP * 2u + row_tile * (KP * 128u) : nullptr, r, kc, q, v, d);
+}
+// rows `rows` long of the pairs of a tile: stores of pairs beyond n fall out of the range
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pair_rows(float *base, uint32_t n, uint32_t rows) { return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)(n * rows * 4u), 0x00027000); }
 
-// units u0 .. u1 - 1 (unit = tile * units per tile + unit of the tile) of a tile list; SETS sets of 16 pairs per tile
-template <int SRC, bool DOWN, int SETS, uint32_t KP>
-__device__ __forceinline__ void staged_units(const StagedArgs &a, const uint32_t *tile_expert, const uint32_t *tile_pair0, const uint32_t *tile_n, uint32_t u0,
-                                             uint32_t u1, float *part, float *scales, TileInfo *tiles, uint32_t *tokens, uint8_t *entries, uint32_t *signs, const LaneTables &lt) {
-    constexpr uint32_t NRT = staged_nrt(KP), WV = KP * NRT, T = staged_threads(SETS, KP), M = SETS == 1 ? 1u : 2u;      // M: halves per wave
-    constexpr uint32_t K = 256u * KP, seg_rows = 16u * NRT, tile_bytes = 16u * KP * src_block<SRC>();
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), w8 = wave % WV, m_first = SETS == 1 ? wave / WV : 0u, kc = w8 % KP, rt = w8 / KP;
-    const uint32_t upt = a.rows / ((DOWN ? 2u : 1u) * seg_rows);
-    const auto matrix_of = [&](uint32_t tile) {
-        const uint32_t e = tile_expert[tile];
-        return e == kSharedTile ? (uint64_t)(a.shared - a.experts) : (uint64_t)e * a.stride;
-    };
-    // the lane's quarters of a unit, and what their d are made from
-    struct Carried { Quarter v[M]; uint2 d[M]; };
-    const auto request = [&](Carried &c, const uint8_t *mat, uint32_t j) {
-#pragma unroll
-        for (uint32_t m = 0; m < M; ++m) {
-            const uint32_t half = m_first + m, row_tile = (DOWN ? 2u * j + half : j) * NRT + rt;
-            const uint8_t *mm = mat + (DOWN ? 0u : half * a.mat_step), *ds = mm + a.d_off + row_tile * (KP * 32u);
-            load_quarter<SRC, KP>(mm + (uint64_t)row_tile * tile_bytes, ds, fmt<SRC>() == F_XS ? mm + a.d_off + (uint64_t)a.rows * KP * 2u + row_tile * (KP * 128u) : nullptr, r, kc, q, c.v[m], c.d[m]);
-        }
-    };
-    const uint32_t tile0 = u0 / upt, n_info = (u1 - 1u) / upt + 1u - tile0 < kTileInfos ? (u1 - 1u) / upt + 1u - tile0 : kTileInfos;
-    const auto token_of = [&](uint32_t p0, uint32_t n, uint32_t i) {           // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
-        const uint32_t p = i < n ? p0 + i : p0;
-        return p < a.P ? a.pair_token[p] : p - a.P;
-    };
+// ---- gate/up ----
+// Eight waves. A wave keeps the activations of its columns for the whole tile in registers, as fp16 halves: of two blocks of 256 columns for
+// sixteen pairs (SETS 1; it multiplies the gate or the up rows with them), of one block for 32 (SETS 2; both rows). PK such parts make the
+// columns, NRT row tiles of 16 rows are in work beside each other: a unit is the gate and the up rows of 16 NRT FFN columns.
+constexpr uint32_t kGateUpThreads = 512u;
+template <int SETS, uint32_t KP> struct GateUp {
+    static constexpr uint32_t PK = SETS == 1 ? KP / 2u : KP, NRT = SETS == 1 ? 4u / PK : 8u / PK, kUnits = SETS == 1 ? 4u : 1u;      // kUnits: between two barriers
+    static constexpr uint32_t kSums = 512u * (uint32_t)SETS, kPart = NRT * PK * kSums;      // partial sums of a row tile's K part: [gate | up][set][256]; of a unit
+};
+template <int SRC, int SETS, uint32_t KP> struct GateUpLds {
+    uint32_t signs[sign_bytes<SRC>() / 4u];              // the tables first: their reads then take the base as an immediate offset (16 bits)
+    uint8_t entries[kEntryBytes];
+    float part[2u * GateUp<SETS, KP>::kUnits * GateUp<SETS, KP>::kPart];
+    TileInfo tiles[kTileInfos];
+    float scales[kTileInfos * 16u * (uint32_t)SETS];     // powers of two that the sums of a pair are multiplied with
+    uint32_t tokens[kTileInfos * 16u * (uint32_t)SETS];
+};
+
+// units u0 .. u1 - 1 (unit = tile * units per tile + unit of the tile) of a tile list
+template <int SRC, int SETS, uint32_t KP>
+__device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList &list, uint32_t u0, uint32_t u1, GateUpLds<SRC, SETS, KP> &lds, bool tables) {
+    using G = GateUp<SETS, KP>;
+    constexpr uint32_t PK = G::PK, NRT = G::NRT, K = 256u * KP, PAIRS = 16u * SETS, T = kGateUpThreads, UB = G::kUnits;
+    const uint32_t tid = each_trip(threadIdx.x), lane = tid & 63u, r = lane & 15u, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t kp = wave % PK, rt = (wave / PK) % NRT, up = wave / (PK * NRT);      // up: SETS 1, the wave has the up rows
+    const uint32_t upt = a.rows / (16u * NRT), tile0 = u0 / upt, n_info = (u1 - 1u) / upt + 1u - tile0;
     if (tid < 64u) {
-        if (tid < n_info) tiles[tid] = TileInfo{matrix_of(tile0 + tid), tile_pair0[tile0 + tid], tile_n[tile0 + tid]};
-        if constexpr (!DOWN)
-            for (uint32_t k = tid; k < n_info * 16u * SETS; k += 64u) tokens[k] = token_of(tile_pair0[tile0 + k / (16u * SETS)], tile_n[tile0 + k / (16u * SETS)], k % (16u * SETS));
-    } else
-        build_staged_tables<SRC, T - 64u>(entries, signs, tid - 64u, a.grid);
+        if (tid < n_info) lds.tiles[tid] = tile_info(a, list, tile0 + tid);
+        for (uint32_t k = tid; k < n_info * PAIRS; k += 64u) {      // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
+            const uint32_t t = tile0 + k / PAIRS, i = k % PAIRS, p = list.pair0[t] + (i < list.n[t] ? i : 0u), tok = p < a.P ? a.pair_token[p] : p - a.P;
+            lds.tokens[k] = tok;
+            lds.scales[k] = format_scale<SRC>() * exp2i(a.xexp[tok]);
+        }
+    } else if (tables)
+        build_staged_tables<SRC, T - 64u>(lds.entries, lds.signs, tid - 64u, a.grid);
     __syncthreads();
-    const auto uniform64 = [](uint64_t v) {
-        return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
-    };
-    const auto info_of = [&](uint32_t tile) {
-        if (tile - tile0 >= kTileInfos) return TileInfo{matrix_of(tile), tile_pair0[tile], tile_n[tile]};
-        const TileInfo ti = tiles[tile - tile0];
-        return TileInfo{uniform64(ti.mat), (uint32_t)__builtin_amdgcn_readfirstlane(ti.p0), (uint32_t)__builtin_amdgcn_readfirstlane(ti.n)};
+    const LaneTables lt = lane_tables<SRC>(lds.entries, lds.signs, tid);
+    // the lane's two quarters of a unit (SETS 1: of the two blocks, SETS 2: of the gate and the up row), and what their d are made from
+    struct Carried { Quarter v[2]; uint2 d[2]; };
+    const auto request = [&](Carried &c, uint64_t mat, uint32_t j) {
+#pragma unroll
+        for (uint32_t m = 0; m < 2u; ++m) {
+            const uint8_t *mm = a.experts + mat + (SETS == 1 ? up : m) * a.mat_step;
+            request_quarter<SRC, KP>(a, mm, j * NRT + rt, r, SETS == 1 ? 2u * kp + m : kp, q, c.v[m], c.d[m]);
+        }
     };
     // Precision. The matrix unit rounds a sum four times per instruction (once per eight products), so what a block's sum loses goes with the
-    // length of its chain of instructions: the low halves have a chain of their own, and the high ones one per kChain steps, added up in
-    // f32 (in the registers, or where these are full in the LDS that takes the block's sum anyway). A chunk of normal rows comes out 1.9e-7
-    // off (f32 multiplications: 2.1e-7); with one chain for everything it was 2.9e-7, in 3 .. 5 % less time. Packed rows (all-IQ2_XXS, ffn
-    // above 512) take two steps per chain: 1.75e-7 instead of 1.9e-7, 5 % of the time.
+    // length of its chain of instructions: the low halves have a chain of their own, and the high ones one per kChain steps, added up in f32.
     constexpr uint32_t kChain = layout<SRC>() == L_ROWS ? 2u : 4u;
-    constexpr bool kSumInLds = SRC == S_IQ3 || (SETS == 2 && layout<SRC>() == L_ROWS);
-    // Units on their way: two, one where the registers hold no second (a spill to scratch memory would be counted among the loads that the
-    // waits count). Codebook wide tiles with two and the sums in the LDS instead: 2048 tokens IQ1_M 743 against 732 us, IQ2_XS 793 against 782.
-    constexpr uint32_t kCarried = SRC == S_IQ3 || (SETS == 2 && fmt<SRC>() != F_XXS) ? 1u : 2u;
-    H8 xa[SETS][8], xb[SETS][8];
-    // Powers of two that the products of a pair are multiplied with. Down: of this wave's block. Gate/up: of the token, so the sums over the
-    // blocks take them; a tile's stand in row tile % 4: a tile has two units or more, so the first wave is at most two tiles ahead of the
-    // one that still adds sums up.
-    float *pair_scale = scales + (DOWN ? wave * 16u * SETS : 0u);
-    const auto load_tile = [&](uint32_t tile, uint32_t p0, uint32_t n) {
+    H8 xa[2][8], xb[2][8];                                 // SETS 1: [block], SETS 2: [set]
+    const auto load_tile = [&](uint32_t tile) {
 #pragma unroll
-        for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
-            __builtin_amdgcn_sched_barrier(0);             // one set at a time: both at once do not fit the registers
-            const uint32_t l = each_trip(lane), lq = l >> 4, i = 16u * s + (l & 15u);
-            float scale;
-            if constexpr (!DOWN) {
-                const uint32_t tok = tile - tile0 < kTileInfos ? tokens[(tile - tile0) * 16u * SETS + i] : token_of(p0, n, i);
-                scale = format_scale<SRC>() * exp2i(a.xexp[tok]);
-                const uint64_t base = (uint64_t)tok * K + 256u * kc;
-                const _Float16 *hp = a.xh + base, *lp = a.xl + base;
+        for (uint32_t x = 0; x < 2u; ++x) {
+            __builtin_amdgcn_sched_barrier(0);             // one at a time: both at once do not fit the registers
+            const uint32_t tok = lds.tokens[(tile - tile0) * PAIRS + (SETS == 1 ? 0u : 16u * x) + r];
+            const uint64_t base = (uint64_t)tok * K + 256u * (SETS == 1 ? 2u * kp + x : kp) + 8u * q;
+            const _Float16 *hp = a.xh + base, *lp = a.xl + base;
+            // four lanes of a pair take 64 bytes side by side; the exchange makes them each lane's own run
 #pragma unroll
-                for (uint32_t g = 0; g < 8u; ++g) {
-                    xa[s][g].u = *reinterpret_cast<const uint4 *>(hp + step_column<SRC>(g, lq));
-                    xb[s][g].u = *reinterpret_cast<const uint4 *>(lp + step_column<SRC>(g, lq));
-                }
-                if (s + 1u == (uint32_t)SETS) __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): waited for here, once per tile, not (by count) where the loop uses them
-            } else {
-                // f32 activations of pair p, columns of this wave's K part: one exponent for them, then the fp16 halves
-                const float *src = a.act + (uint64_t)(i < n ? p0 + i : p0) * K + 256u * kc;
-                float amax = 0.0f;
-#pragma unroll
-                for (uint32_t g = 0; g < 8u; ++g) {
-                    const float4 v0 = *reinterpret_cast<const float4 *>(src + step_column<SRC>(g, lq)), v1 = *reinterpret_cast<const float4 *>(src + step_column<SRC>(g, lq) + 4u);
-                    xa[s][g].u = __builtin_bit_cast(uint4, v0);
-                    xb[s][g].u = __builtin_bit_cast(uint4, v1);
-                }
-#pragma unroll
-                for (uint32_t g = 0; g < 8u; ++g) {
-                    const float4 v0 = __builtin_bit_cast(float4, xa[s][g].u), v1 = __builtin_bit_cast(float4, xb[s][g].u);
-                    amax = fmaxf(amax, fmaxf(fmaxf(fmaxf(fabsf(v0.x), fabsf(v0.y)), fmaxf(fabsf(v0.z), fabsf(v0.w))), fmaxf(fmaxf(fabsf(v1.x), fabsf(v1.y)), fmaxf(fabsf(v1.z), fabsf(v1.w)))));
-                }
-                amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-                amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-                const int e = prescale_exp(amax);
-                const float inv = exp2i(-e);
-                scale = format_scale<SRC>() * exp2i(e);
-#pragma unroll
-                for (uint32_t g = 0; g < 8u; ++g) {
-                    const float4 v0 = __builtin_bit_cast(float4, xa[s][g].u), v1 = __builtin_bit_cast(float4, xb[s][g].u);
-                    const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-                    H8 hi, lo;
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        const float t = f[k] * inv;
-                        const _Float16 h = (_Float16)t;
-                        hi.e[k] = h;
-                        lo.e[k] = (_Float16)split_rest(t, h);
-                    }
-                    // group by group (the compiler otherwise works on several at once and spills)
-                    asm volatile("" : "+v"(hi.u.x), "+v"(hi.u.y), "+v"(hi.u.z), "+v"(hi.u.w), "+v"(lo.u.x), "+v"(lo.u.y), "+v"(lo.u.z), "+v"(lo.u.w));
-                    xa[s][g].u = hi.u;
-                    xb[s][g].u = lo.u;
-                }
+            for (uint32_t g = 0; g < 8u; ++g) {
+                const uint32_t at = 8u * (16u * ((g >> 1) & 1u) + 8u * (g & 1u) + 4u * (g >> 2));
+                xa[x][g].u = *reinterpret_cast<const uint4 *>(hp + at);
+                xb[x][g].u = *reinterpret_cast<const uint4 *>(lp + at);
             }
-            pair_scale[(DOWN ? 0u : (tile & 3u) * 16u * SETS) + i] = scale;      // (every lane and wave that has pair i writes the same)
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t x = 0; x < 2u; ++x) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t g = 0; g < 8u; g += 2u) { swap16(xa[x][g].u, xa[x][g + 1u].u); swap16(xb[x][g].u, xb[x][g + 1u].u); }
+#pragma unroll
+            for (uint32_t g = 0; g < 8u; ++g) if (!(g & 2u)) { swap32(xa[x][g].u, xa[x][g + 2u].u); swap32(xb[x][g].u, xb[x][g + 2u].u); }
         }
     };
-    // partial sums of the waves: [row tile, K part][m][set][lane] float4
-    constexpr uint32_t kWavePart = 2u * SETS * 256u, kPart = WV * kWavePart;      // (kPart: of a unit)
-    struct Done { uint32_t tile, j, p0, n; };              // a unit whose partial sums are in LDS
-    // The sums of UNITS units (w[0], and w[1] behind it). No wave and no lane may skip a store: the loads of the next units are in flight
-    // behind it, and the compiler, which waits for them by counting memory operations in order, can count only what every path issues
-    // (with a branch around it, every unit waited for the newest of its loads). Pairs beyond a tile's n fall out of the buffer's range.
-    const auto tile_buffer = [&](float *base, uint32_t n) { return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)(n * a.rows * 4u), 0x00027000); };
-    using Sum = std::conditional_t<(KP > 2u), double, float>;      // (a row's partial sums are added here one after the other)
-    const auto reduce = [&](auto units, const Done *w, const float *pt) {
-        constexpr uint32_t UNITS = decltype(units)::value;
-        const uint32_t t = each_trip(tid);
-        if constexpr (DOWN) {
-            // V consecutive floats (pairs of one row) per thread; threads beyond the last repeat it
-            constexpr uint32_t V = SETS == 1 ? 2u : 4u, PB = 256u / V, N = PB * SETS * 2u * NRT;
+    // The sums of UNITS units, the first of them number fj of tile ft, and their SwiGLU. No wave and no lane may skip a store: the loads of the next units are in flight in front of it, and the
+    // compiler, which waits for them by counting memory operations in order, can count only what every path issues.
+    const auto reduce = [&](auto units, uint32_t ft, uint32_t fj, const float *pt) {
+        constexpr uint32_t UNITS = decltype(units)::value, N = 256u * SETS * NRT * UNITS;
 #pragma unroll
-            for (uint32_t un = 0; un < UNITS; ++un) {
-                const bool routed = w[un].p0 < a.P;        // (a tile is routed or shared as a whole)
-                const auto buf = tile_buffer((routed ? a.tmp + (uint64_t)w[un].p0 * a.rows : a.sh_tmp + (uint64_t)(w[un].p0 - a.P) * a.rows), w[un].n);
+        for (uint32_t base = 0; base < N; base += T) {
+            const uint32_t e = N < T ? min(tid, N - 1u) : base + tid;      // (surplus threads repeat the last element)
+            const uint32_t at = e & 255u, b = __builtin_amdgcn_readfirstlane((e >> 8) % (SETS * NRT)), un = __builtin_amdgcn_readfirstlane((e >> 8) / (SETS * NRT)), set = b % SETS, slot = b / SETS;
+            const float *src = pt + un * G::kPart + slot * PK * G::kSums + set * 256u + at;
+            using Sum = std::conditional_t<(PK > 2u), double, float>;      // (a row's parts are added here)
+            Sum g[PK], u[PK];
 #pragma unroll
-                for (uint32_t base = 0; base < N; base += T) {
-                    const uint32_t it = N % T ? min(base + t, N - 1u) : base + t;
-                    const uint32_t at = (it & (PB - 1u)) * V, b = it / PB, set = b & (SETS - 1u), m = (b / SETS) & 1u, slot = b / (2u * SETS);
-                    const float *src = pt + un * kPart + slot * KP * kWavePart + (m * SETS + set) * 256u + at;
-                    Sum s[V];
+            for (uint32_t k = 0; k < PK; ++k) { g[k] = src[k * G::kSums]; u[k] = src[k * G::kSums + SETS * 256u]; }
 #pragma unroll
-                    for (uint32_t v = 0; v < V; ++v) s[v] = src[v];
+            for (uint32_t n = PK / 2u; n; n /= 2u)
 #pragma unroll
-                    for (uint32_t k = 1; k < KP; ++k)
-#pragma unroll
-                        for (uint32_t v = 0; v < V; ++v) s[v] += src[k * kWavePart + v];
-                    const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u), off = 4u * (i * a.rows + w[un].j * 2u * seg_rows + m * seg_rows + 16u * slot + ((at >> 2) & 15u));
-#pragma unroll
-                    for (uint32_t v = 0; v < V; ++v) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((float)s[v]), buf, off + 4u * v * a.rows, 0, 0);
-                }
-            }
-        } else {
-            // (pair, column) elements; L lanes of a wave (halves of it) share one where there are fewer elements than threads
-            constexpr uint32_t N = 256u * SETS * NRT * UNITS, L = N < T ? T / N : 1u;
-            static_assert(L <= 4u && KP % L == 0u, "K parts per lane");
-#pragma unroll
-            for (uint32_t base = 0; base < N; base += T) {
-                const uint32_t ln = t & 63u, e = base + (L == 1u ? t : (t >> 6) * (64u / L) + (ln & (64u / L - 1u))), k0 = L == 1u ? 0u : (ln / (64u / L)) * (KP / L);
-                const uint32_t at = e & 255u, b = (e >> 8) % (SETS * NRT), un = (e >> 8) / (SETS * NRT), set = b & (SETS - 1u), slot = b / SETS;
-                const float *src = pt + un * kPart + (slot * KP + k0) * kWavePart + set * 256u + at;
-                Sum s0 = src[0], s1 = src[SETS * 256u];
-#pragma unroll
-                for (uint32_t k = 1; k < KP / L; ++k) {
-                    s0 += src[k * kWavePart];
-                    s1 += src[k * kWavePart + SETS * 256u];
-                }
-                if constexpr (L >= 2u) { s0 += __shfl_xor(s0, 32, 64); s1 += __shfl_xor(s1, 32, 64); }
-                if constexpr (L == 4u) { s0 += __shfl_xor(s0, 16, 64); s1 += __shfl_xor(s1, 16, 64); }
-                // (the wave's elements are of one unit)
-                const uint32_t uw = UNITS == 1u ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(un);
-                const Done d = uw ? w[UNITS - 1u] : w[0];
-                const auto buf = tile_buffer(a.act + (uint64_t)d.p0 * a.rows, d.n);
-                const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u);
-                const float scale = pair_scale[(d.tile & 3u) * 16u * SETS + i], g = (float)s0 * scale, up = (float)s1 * scale;
-                // (of the lanes that share an element the first stores; the others' offset lies beyond every buffer)
-                const uint32_t off = k0 == 0u ? 4u * (i * a.rows + d.j * seg_rows + 16u * slot + ((at >> 2) & 15u)) : 0x7fffffffu;
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((g / (1.0f + expf(-g))) * up), buf, off, 0, 0);
-            }
+                for (uint32_t k = 0; k < n; ++k) { g[k] += g[k + n]; u[k] += u[k + n]; }
+            uint32_t dt = ft - tile0, dj = fj + un;
+            while (dj >= upt) { dj -= upt; ++dt; }
+            const TileInfo d = uniform_info(lds.tiles[dt]);
+            const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u);
+            const float scale = lds.scales[dt * PAIRS + i], gate = (float)g[0] * scale;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((gate / (1.0f + expf(-gate))) * ((float)u[0] * scale)), pair_rows(a.act + (uint64_t)d.p0 * a.rows, d.n, a.rows),
+                                                  4u * (i * a.rows + dj * 16u * NRT + 16u * slot + ((at >> 2) & 15u)), 0, 0);
         }
     };
     uint32_t tile = tile0, j = u0 % upt, ftile = tile0, fj = j, fleft = u1 - u0;      // f..: the unit to be requested next
-    TileInfo cur = info_of(tile);
-    uint64_t fmat = cur.mat;
-    const auto request_next = [&](Carried &c) {            // (the last units fetch theirs again: registers filled under a condition would be live all around the loop)
-        request(c, a.experts + fmat, fj);
+    uint64_t fmat = uniform_info(lds.tiles[0]).mat;
+    const auto request_rows = [&](Carried &c) { request(c, fmat, fj); };
+    const auto advance = [&] {                             // (the last units fetch theirs again: registers filled under a condition would be live all around the loop)
         if (fleft <= 1u) return;
         --fleft;
-        if (++fj == upt) { fj = 0u; fmat = info_of(++ftile).mat; }
+        if (++fj == upt) { fj = 0u; fmat = uniform_info(lds.tiles[++ftile - tile0]).mat; }
     };
     // multiplies the unit whose rows are in c into partial sums at pt and requests the unit two after it in their place
     const auto unit = [&](uint32_t u, Carried &c, float *pt) {
-        float4_t acc[M][SETS], low[M][SETS], sum[M][SETS];
-        float d[M];
+        float4_t acc[2][SETS], low[2][SETS], sum[2][SETS];
+        float d[2];
+        Entry e[2];
+        half2_t f[2];
 #pragma unroll
-        for (uint32_t m = 0; m < M; ++m) {
+        for (uint32_t m = 0; m < 2u; ++m) {
             d[m] = quarter_d<SRC>(c.d[m]);
+            e[m] = fetch_entry<SRC, 0u>(c.v[m], lt);
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s) acc[m][s] = low[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
-        float *mine = pt + w8 * kWavePart + m_first * SETS * 256u + 4u * lane;
-        Entry e[M];
-        half2_t f[M];
-#pragma unroll
-        for (uint32_t m = 0; m < M; ++m) e[m] = fetch_entry<SRC>(c.v[m], 0u, lt);
-#pragma unroll
-        for (uint32_t s8 = 0; s8 < 8u; ++s8) {
-            // table reads run a step ahead of the products (two steps ahead takes five registers more per row and was no quicker)
+        each_step([&](auto step) {
+            constexpr uint32_t S = decltype(step)::value;
+            // table reads run a step ahead of the products; who is behind goes first
+            if constexpr (S % (SETS == 1 ? 4u : 2u) == 0u) __builtin_amdgcn_s_setprio(SETS == 1 ? 2 - (int)S / 2 : 3 - (int)S / 2);
             __builtin_amdgcn_sched_barrier(0);
-            half8_t w[M];
+            half8_t w[2];
 #pragma unroll
-            for (uint32_t m = 0; m < M; ++m) {
-                if constexpr (steps_per_scale<SRC>() != 0u) { if (s8 % steps_per_scale<SRC>() == 0u) f[m] = step_scale<SRC>(c.v[m], s8); }
-                w[m] = finish_entry<SRC>(e[m], f[m]);
-                if (s8 < 7u) e[m] = fetch_entry<SRC>(c.v[m], s8 + 1u, lt);
+            for (uint32_t m = 0; m < 2u; ++m) {
+                if constexpr (steps_per_scale<SRC>() != 0u) { if constexpr (S % steps_per_scale<SRC>() == 0u) f[m] = step_scale<SRC, S>(c.v[m]); }
+                w[m] = finish_entry<SRC>(e[m], f[m], lt);
+                if constexpr (S < 7u) e[m] = fetch_entry<SRC, S + 1u>(c.v[m], lt);
             }
             __builtin_amdgcn_sched_barrier(0);
-            if (s8 == 6u) request_next(c);                 // (the quarters' last use is behind)
-            if (s8 && s8 % kChain == 0u) {                 // put the sums so far aside
+            if constexpr (S == 6u) request_rows(c);        // (the quarters' last use is behind)
+            if constexpr (S && S % kChain == 0u) {         // put the sums so far aside
 #pragma unroll
-                for (uint32_t m = 0; m < M; ++m)
+                for (uint32_t m = 0; m < 2u; ++m)
 #pragma unroll
                     for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
-                        float4_t &so_far = kSumInLds ? *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) : sum[m][s];
-                        so_far = s8 == kChain ? acc[m][s] : so_far + acc[m][s];
+                        sum[m][s] = S == kChain ? acc[m][s] : sum[m][s] + acc[m][s];
                         acc[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
                     }
             }
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
-                for (uint32_t m = 0; m < M; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[s][s8].v, w[m], acc[m][s], 0, 0, 0);
+                for (uint32_t m = 0; m < 2u; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[SETS == 1 ? m : s][S].v, w[m], acc[m][s], 0, 0, 0);
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
-                for (uint32_t m = 0; m < M; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[s][s8].v, w[m], low[m][s], 0, 0, 0);
+                for (uint32_t m = 0; m < 2u; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[SETS == 1 ? m : s][S].v, w[m], low[m][s], 0, 0, 0);
+        });
+        float *mine = pt + (rt * PK + kp) * G::kSums + 4u * lane;
+#pragma unroll
+        for (uint32_t m = 0; m < 2u; ++m)
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) acc[m][s][t] = fmaf(low[m][s][t], 4.8828125e-4f, sum[m][s][t] + acc[m][s][t]) * d[m];
+        if constexpr (SETS == 1) *reinterpret_cast<float4_t *>(mine + up * 256u) = acc[0][0] + acc[1][0];
+        else {
+#pragma unroll
+            for (uint32_t m = 0; m < 2u; ++m)
+#pragma unroll
+                for (uint32_t s = 0; s < (uint32_t)SETS; ++s) *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) = acc[m][s];
         }
-#pragma unroll
-        for (uint32_t m = 0; m < M; ++m)
-#pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
-                float4_t *at = reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u);
-                if constexpr (kSumInLds) sum[m][s] = *at;
-                float4_t factor = {d[m], d[m], d[m], d[m]};
-                if constexpr (DOWN) factor *= *reinterpret_cast<const float4_t *>(pair_scale + 16u * s + 4u * q);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) acc[m][s][t] = fmaf(low[m][s][t], 4.8828125e-4f, sum[m][s][t] + acc[m][s][t]) * factor[t];
-                *at = acc[m][s];
-            }
-        const Done done{tile, j, cur.p0, cur.n};
-        if (++j == upt && u + 1u < u1) { j = 0u; cur = info_of(++tile); load_tile(tile, cur.p0, cur.n); }
-        return done;
+        advance();
+        if (++j == upt && u + 1u < u1) { j = 0u; load_tile(++tile); }
     };
+    constexpr uint32_t kCarried = SETS == 2 && fmt<SRC>() != F_XXS ? 1u : 2u;      // units on their way: two where the registers hold them
     Carried c[kCarried];
 #pragma unroll
-    for (uint32_t k = 0; k < kCarried; ++k) request_next(c[k]);
-    load_tile(tile, cur.p0, cur.n);
-    // narrow: two units per barrier, four buffers of partial sums; wide: one, two buffers (as large). A buffer is written again two
-    // barriers after its sums were complete; whoever adds them has passed one in between.
+    for (uint32_t k = 0; k < kCarried; ++k) {
+        request_rows(c[k]);
+        advance();
+    }
+    load_tile(tile);
+    // A buffer of partial sums is written again two barriers after its sums were complete; whoever adds them has passed one in between.
     constexpr std::integral_constant<uint32_t, 1u> one{};
-    constexpr std::integral_constant<uint32_t, 2u> two{};
+    constexpr std::integral_constant<uint32_t, UB> all{};
     uint32_t u = u0;
-    float *pt = part;
-    for (; u + 1u < u1; u += 2u) {
-        Done w[2];
-        w[0] = unit(u, c[0], pt);
-        if constexpr (SETS == 2) {
-            wave_lds_barrier();
-            reduce(one, w, pt);
-        }
-        w[1] = unit(u + 1u, c[kCarried - 1u], pt + kPart);
+    float *pt = lds.part;
+    const auto turn = [&] { pt = pt == lds.part ? lds.part + UB * G::kPart : lds.part; };
+    for (; UB > 1u && u + UB <= u1; u += UB) {
+        const uint32_t t = tile, j0 = j;
+#pragma unroll
+        for (uint32_t k = 0; k < UB; ++k) unit(u + k, c[k % kCarried], pt + k * G::kPart);
         wave_lds_barrier();
-        if constexpr (SETS == 2) reduce(one, w + 1, pt + kPart);
-        else {
-            reduce(two, w, pt);
-            pt = pt == part ? part + 2u * kPart : part;
-        }
+        reduce(all, t, j0, pt);
+        turn();
     }
-    if (u < u1) {
-        const Done w = unit(u, c[0], pt);
+    const auto single = [&](Carried &cc) {
+        const uint32_t t = tile, j0 = j;
+        unit(u, cc, pt);
         wave_lds_barrier();
-        reduce(one, &w, pt);
-    }
+        reduce(one, t, j0, pt);
+        turn();
+        return ++u < u1;
+    };
+    if (u < u1) while (single(c[0]) && single(c[kCarried - 1u])) {}
 }
 
-// SETS 1: the narrow tiles (list 2) of a chunk, SETS 2: the wide ones (list 1). Persistent workgroups, each with an equal run of the units.
+// ---- down ----
+// A tile's activations stand in LDS as fp16 halves, split once per tile: per panel (a block of 256 columns of sixteen pairs) and half the 16 bytes
+// that lane l multiplies in step s at 1024 s + 16 l. A wave has whole rows, two row tiles beside each other, so it stores its sums from registers
+// and waits for the others only where a tile begins. Narrow passes may take the end of one tile and the begin of the next where two fit the LDS.
+constexpr uint32_t kPanel = 16384u;
+constexpr uint32_t down_waves(int sets) { return sets == 1 ? 12u : 8u; }
+template <int SETS, uint32_t KP> constexpr uint32_t down_tiles_a_pass() { return SETS == 1 && KP <= 2u ? 2u : 1u; }
+template <int SRC, int SETS, uint32_t KP> struct DownLds {
+    uint32_t signs[sign_bytes<SRC>() / 4u];
+    uint8_t entries[kEntryBytes];
+    uint8_t x[(SETS == 2 ? 2u : down_tiles_a_pass<SETS, KP>()) * KP * kPanel];      // [tile % 2, or set][block]
+    TileInfo tiles[kTileInfos];
+    float scales[2u * KP * 16u * (uint32_t)SETS];        // [tile % 2][block][pair]: powers of two that the sums of a pair's block are multiplied with
+};
+// largest of the sixteen lanes of a row
+__device__ __forceinline__ float row_max(float v) {
+    const auto with = [](float x, auto ctrl) { return fmaxf(x, __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), decltype(ctrl)::value, 0xf, 0xf, false))); };
+    v = with(v, std::integral_constant<int, 0xB1>{});      // quad_perm [1, 0, 3, 2], [2, 3, 0, 1]; row_ror 4, 8
+    v = with(v, std::integral_constant<int, 0x4E>{});
+    v = with(v, std::integral_constant<int, 0x124>{});
+    return with(v, std::integral_constant<int, 0x128>{});
+}
+
+// items i0 .. i1 - 1 of a tile list (item = tile * items per tile + item of the tile; an item: 32 rows, a wave's)
+template <int SRC, int SETS, uint32_t KP>
+__device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &list, uint32_t i0, uint32_t i1, DownLds<SRC, SETS, KP> &lds, bool tables) {
+    constexpr uint32_t WV = down_waves(SETS), T = 64u * WV, PAIRS = 16u * SETS, K = 256u * KP, kPassTiles = down_tiles_a_pass<SETS, KP>();
+    const uint32_t tid = each_trip(threadIdx.x), lane = tid & 63u, r = lane & 15u, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t ipt = a.rows / 32u, tile0 = i0 / ipt, n_info = (i1 - 1u) / ipt + 1u - tile0;
+    if (tid < 64u) {
+        if (tid < n_info) lds.tiles[tid] = tile_info(a, list, tile0 + tid);
+    } else if (tables)
+        build_staged_tables<SRC, T - 64u>(lds.entries, lds.signs, tid - 64u, a.grid);
+    __syncthreads();
+    const LaneTables lt = lane_tables<SRC>(lds.entries, lds.signs, tid);
+    const auto info_of = [&](uint32_t tile) { return uniform_info(lds.tiles[tile - tile0]); };
+    // A pass: an item per wave, of up to kPassTiles tiles
+    struct Pass { uint32_t i, tile, j, n; };               // first item, its tile, its number in the tile, items
+    const auto pass_at = [&](uint32_t i, uint32_t tile, uint32_t j) { return Pass{i, tile, j, (uint32_t)min(min(i1 - i, WV), kPassTiles * ipt - j)}; };
+    const auto following = [&](const Pass &p) {            // (behind the last pass: that one again)
+        if (p.i + p.n >= i1) return p;
+        const uint32_t j = p.j + p.n, over = j >= ipt ? j >= 2u * ipt ? 2u : 1u : 0u;
+        return pass_at(p.i + p.n, p.tile + over, j - over * ipt);
+    };
+    const auto second = [&](const Pass &p) { return kPassTiles == 2u && p.j + min(wave, p.n - 1u) >= ipt ? 1u : 0u; };      // the wave's item is of the pass's second tile
+    // the lane's quarters of a block of the wave's two row tiles, and what their d are made from
+    struct Carried { Quarter v[2]; uint2 d[2]; };
+    struct { Pass p; uint64_t mat; uint32_t kb; } ahead;   // the block to be requested next
+    ahead.p = pass_at(i0, tile0, i0 - tile0 * ipt);
+    ahead.mat = info_of(tile0 + second(ahead.p)).mat;
+    ahead.kb = 0u;
+    Pass p = ahead.p;
+    const auto request = [&](Carried &c) {                 // (a wave without an item requests the pass's last)
+        const uint32_t item = ahead.p.j + min(wave, ahead.p.n - 1u) - second(ahead.p) * ipt;
+#pragma unroll
+        for (uint32_t m = 0; m < 2u; ++m) request_quarter<SRC, KP>(a, a.experts + ahead.mat, 2u * item + m, r, ahead.kb, q, c.v[m], c.d[m]);
+        if (++ahead.kb < KP) return;
+        ahead.kb = 0u;
+        ahead.p = following(ahead.p);
+        ahead.mat = info_of(ahead.p.tile + second(ahead.p)).mat;
+    };
+    // f32 activations of four pairs and a block per wave: one exponent for a pair's block, then the fp16 halves
+    const auto stage = [&](uint32_t tile) {
+        const TileInfo ti = info_of(tile);
+        for (uint32_t w = wave; w < KP * SETS * 4u; w += WV) {
+            const uint32_t block = w / (SETS * 4u), i = (w % (SETS * 4u)) * 4u + q;
+            const float *src = a.act + (uint64_t)(i < ti.n ? ti.p0 + i : ti.p0) * K + 256u * block + 4u * r;
+            float4 v[4];
+            float amax = 0.0f;
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) v[k] = *reinterpret_cast<const float4 *>(src + 64u * k);
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[k].x), fabsf(v[k].y)), fmaxf(fabsf(v[k].z), fabsf(v[k].w))));
+            const int e = prescale_exp(row_max(amax));
+            const float inv = exp2i(-e);
+            if (r == 0u) lds.scales[((tile & 1u) * KP + block) * PAIRS + i] = format_scale<SRC>() * exp2i(e);
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) {
+                const float f[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+                union { uint2 u; _Float16 e[4]; } hi, lo;
+#pragma unroll
+                for (int n = 0; n < 4; ++n) {
+                    const float t = f[n] * inv;
+                    hi.e[n] = (_Float16)t;
+                    lo.e[n] = (_Float16)split_rest(t, hi.e[n]);
+                }
+                // columns 64 k + 4 r .. + 3: eight of step s and lane quarter sq, their half r % 2
+                const uint32_t c8 = 8u * k + r / 2u, s = fmt<SRC>() == F_IQ3_WORDS ? 4u * (c8 >> 4) + ((c8 >> 2) & 3u) : c8 & 7u, sq = fmt<SRC>() == F_IQ3_WORDS ? c8 & 3u : c8 >> 3;
+                uint8_t *at = lds.x + ((SETS == 2 ? i / 16u : kPassTiles == 2u ? tile & 1u : 0u) * KP + block) * kPanel + (s * 64u + sq * 16u + (i & 15u)) * 16u + (r & 1u) * 8u;
+                *reinterpret_cast<uint2 *>(at) = hi.u;
+                *reinterpret_cast<uint2 *>(at + 8192u) = lo.u;
+            }
+        }
+    };
+    // Precision: as in gate/up, but a row's blocks are added up in f32, so the chains are half as long.
+    constexpr uint32_t kChain = 2u;
+    float4_t sum[2][SETS];
+    const auto clear = [&] {
+#pragma unroll
+        for (uint32_t m = 0; m < 2u; ++m)
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) sum[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    // adds the products of the block whose rows are in c
+    const auto multiply = [&](const Carried &c, const uint8_t *x, const float *pair_scale) {
+        const auto operand = [&](uint32_t s, uint32_t half, uint32_t step) { return *reinterpret_cast<const half8_t *>(x + s * KP * kPanel + half * 8192u + 1024u * step); };
+        float4_t acc[2][SETS], low[2][SETS], block[2][SETS];
+        float d[2];
+        Entry e[2];
+        half2_t f[2];
+#pragma unroll
+        for (uint32_t m = 0; m < 2u; ++m) {
+            d[m] = quarter_d<SRC>(c.d[m]);
+            e[m] = fetch_entry<SRC, 0u>(c.v[m], lt);
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) acc[m][s] = low[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        each_step([&](auto step) {
+            constexpr uint32_t S = decltype(step)::value;
+            // table reads run a step ahead of the products
+            __builtin_amdgcn_sched_barrier(0);
+            half8_t w[2], xh[SETS], xl[SETS];
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) { xh[s] = operand(s, 0u, S); xl[s] = operand(s, 1u, S); }
+#pragma unroll
+            for (uint32_t m = 0; m < 2u; ++m) {
+                if constexpr (steps_per_scale<SRC>() != 0u) { if constexpr (S % steps_per_scale<SRC>() == 0u) f[m] = step_scale<SRC, S>(c.v[m]); }
+                w[m] = finish_entry<SRC>(e[m], f[m], lt);
+                __builtin_amdgcn_sched_barrier(0);         // (the entry's registers take the next one)
+                if constexpr (S < 7u) e[m] = fetch_entry<SRC, S + 1u>(c.v[m], lt);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (S && S % kChain == 0u) {
+#pragma unroll
+                for (uint32_t m = 0; m < 2u; ++m)
+#pragma unroll
+                    for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
+                        block[m][s] = S == kChain ? acc[m][s] : block[m][s] + acc[m][s];
+                        acc[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+            }
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
+#pragma unroll
+                for (uint32_t m = 0; m < 2u; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[s], w[m], acc[m][s], 0, 0, 0);
+#pragma unroll
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
+#pragma unroll
+                for (uint32_t m = 0; m < 2u; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[s], w[m], low[m][s], 0, 0, 0);
+        });
+#pragma unroll
+        for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
+            const float4_t ps = *reinterpret_cast<const float4_t *>(pair_scale + 16u * s + 4u * q);
+#pragma unroll
+            for (uint32_t m = 0; m < 2u; ++m)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) sum[m][s][t] = fmaf(fmaf(low[m][s][t], 4.8828125e-4f, block[m][s][t] + acc[m][s][t]), d[m] * ps[t], sum[m][s][t]);
+        }
+    };
+    // No wave may skip a store (as in gate/up): of a wave without an item every one falls out of the range.
+    const auto store_pass = [&] {
+        const uint32_t over = second(p), item = p.j + wave - over * ipt;
+        const TileInfo ti = info_of(p.tile + over);
+        const auto buf = pair_rows(ti.p0 < a.P ? a.tmp + (uint64_t)ti.p0 * a.rows : a.sh_tmp + (uint64_t)(ti.p0 - a.P) * a.rows, wave < p.n ? ti.n : 0u, a.rows);      // (a tile is routed or shared as a whole)
+#pragma unroll
+        for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
+#pragma unroll
+            for (uint32_t m = 0; m < 2u; ++m)
+#pragma unroll
+                for (uint32_t t = 0; t < 4u; ++t)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sum[m][s][t]), buf, 4u * ((16u * s + 4u * q + t) * a.rows + (2u * item + m) * 16u + r), 0, 0);
+    };
+    Carried c[2];
+    request(c[0]);
+    request(c[1]);
+    const uint8_t *x_lane = lds.x + 16u * lane;
+    uint32_t kb = 0u, staged = tile0;                      // staged: tiles below it are in LDS or were
+    const auto last_tile = [&] { return p.tile + (p.j + p.n > ipt ? 1u : 0u); };
+    const auto stage_pass = [&] {
+        for (; staged <= last_tile(); ++staged) stage(staged);
+        wave_lds_barrier();
+    };
+    clear();
+    stage_pass();
+    const auto block = [&](Carried &cc) {                  // false: the last one is done
+        const uint32_t odd = (p.tile + second(p)) & 1u;
+        if (wave < p.n) multiply(cc, x_lane + ((kPassTiles == 2u ? odd : 0u) * KP + kb) * kPanel, lds.scales + (odd * KP + kb) * PAIRS);
+        request(cc);
+        if (++kb < KP) return true;
+        kb = 0u;
+        store_pass();
+        clear();
+        if (p.i + p.n >= i1) return false;
+        p = following(p);
+        if (last_tile() >= staged) {
+            wave_lds_barrier();                            // (nobody needs the tiles before the pass's any more)
+            stage_pass();
+        }
+        return true;
+    };
+    while (block(c[0]) && block(c[1])) {}
+}
+
+// SETS 1: the narrow tiles (list 2) of a chunk, SETS 2: the wide ones (list 1). Persistent workgroups, each with an equal run of the work.
 // A launch that finds few wide tiles leaves them: the narrow one then takes every pair in tiles of 16 (list 0). Two launches where one would
-// do cost 10 to 20 us (tables, the first tiles' activations, compute units without a unit at both ends); a wide tile saves a second decoding
-// of its rows, which goes with their weights. So the line is a number of weights in wide tiles: 220 million for gate/up, 230 million for
-// IQ2_XXS down rows, 145 million for the other down formats. Both ways measured on chunks of evenly routed tokens, 128 and 512 experts with
-// 12 to 40 pairs on average, 1024 x 256 to 2048 x 768; what was even: gate/up 130 to 240 million on all-IQ2_XXS layers, 300 to 450 on the
-// others, down 118 to 230 IQ2_XXS, 125 to 170 the others. 221 wide tiles of 2048 x 512 (464 / 232 million, IQ2_XS): 260 + 133 us with
-// them, 263 + 154 without; 97 (203 / 102): 105 + 69 against 99 + 54. On mixed layouts the shared expert's products run beside gate/up and
-// finish sooner beside two launches: a layer of 112 wide tiles of 2048 x 512 (235 million) takes 332 us with them, 340 without, one of 195
-// of 1024 x 512 (205) 191 against 183, so these share the all-IQ2_XXS line. Packed IQ2_XXS down rows (ffn above 512) lost 20 us with 57 to
-// 139 wide tiles alike and have none.
-template <int SRC, bool DOWN> constexpr bool has_wide() { return !(DOWN && layout<SRC>() == L_ROWS); }
-template <int SRC, bool DOWN> uint32_t few_wide(uint32_t rows, uint32_t K) {
-    return !has_wide<SRC, DOWN>() ? ~0u : (DOWN ? fmt<SRC>() == F_XXS ? 230000000u : 145000000u : 110000000u) / (rows * K) + 1u;
+// do cost 10 to 20 us (tables, the first tiles' activations, compute units without work at both ends); a wide tile saves a second decoding
+// of its rows, which goes with their weights. So the line is a number of weights in wide tiles: 290 million for gate/up, 200 million for
+// down. Whole chunks measured with and without, by weights in wide tiles: gate/up of 235 to 268 million (512 tokens, Zipf-popular or 32 pairs
+// per expert) 7 to 12 us slower with them, 262 million (250 tiles of 1024 x 512) 0 to 4 us quicker, 315 million 15 us quicker, one of 1000 million
+// 20 to 60 us quicker; down of 117 million 5 to 8 us slower, 131 to 157 million 1 to 3 us slower, 230 million 4 us quicker, 500 million 6 to
+// 24. Down matrices of more than two blocks have none: their tiles of 32 pairs do not fit the LDS.
+template <int SRC, bool DOWN, uint32_t KP> constexpr bool has_wide() { return !DOWN || KP <= 2u; }
+template <int SRC, bool DOWN, uint32_t KP> uint32_t few_wide(uint32_t rows, uint32_t K) {
+    return !has_wide<SRC, DOWN, KP>() ? ~0u : (DOWN ? 200000000u : 145000000u) / (rows * K) + 1u;
 }
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
-__global__ __launch_bounds__(staged_threads(SETS, KP)) void staged_tiles_kernel(StagedArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t entries[kEntryBytes];   // static: table reads take immediate offsets
-    __shared__ __attribute__((aligned(16))) uint32_t signs[sign_bytes<SRC>() / 4u + 4u];
-    __shared__ __attribute__((aligned(16))) float part[4u * KP * staged_nrt(KP) * 2u * 256u];
+__global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) void staged_tiles_kernel(StagedArgs a) {
+    __shared__ __attribute__((aligned(16))) std::conditional_t<DOWN, DownLds<SRC, SETS, KP>, GateUpLds<SRC, SETS, KP>> lds;
     const uint32_t n0 = a.n_tiles[0], n1 = a.n_tiles[1], n2 = a.n_tiles[2];      // (one trip)
     const bool few = n1 < a.few;
     if (SETS == 2 && few) return;
-    const uint32_t tid = threadIdx.x, l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
-    const uint32_t units = (SETS == 2 ? n1 : few ? n0 : n2) * (a.rows / ((DOWN ? 32u : 16u) * staged_nrt(KP)));
+    const uint32_t l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
+    const uint32_t per_tile = a.rows / (DOWN ? 32u : 16u * GateUp<SETS, DOWN ? 2u : KP>::NRT), work = (SETS == 2 ? n1 : few ? n0 : n2) * per_tile;
+    const TileList list{a.tile_expert + off, a.tile_pair0 + off, a.tile_n + off};
     // workgroups are dealt round-robin over the eight XCDs: neighbouring runs (which share tiles) go to one XCD's L2
     const uint32_t G = gridDim.x, at = G % 8u == 0u ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
-    const uint32_t u0 = (uint32_t)((uint64_t)at * units / G), u1 = (uint32_t)((uint64_t)(at + 1u) * units / G);
-    if (u0 >= u1) return;
-    __shared__ TileInfo tiles[kTileInfos];
-    __shared__ uint32_t tokens[DOWN ? 1u : kTileInfos * 16u * SETS];
-    __shared__ __attribute__((aligned(16))) float scales[(DOWN ? staged_threads(SETS, KP) / 64u : 4u) * 16u * SETS];
-    const LaneTables lt{entries + (fmt<SRC>() == F_XS ? (tid & 7u) * 16u : fmt<SRC>() == F_M ? (tid & 1u) * 16u : 0u),
-                        reinterpret_cast<const uint8_t *>(signs) + (is_iq3<SRC>() ? (tid & 3u) * 4u : fmt<SRC>() == F_M ? 0u : (tid & 15u) * 4u)};
-    staged_units<SRC, DOWN, SETS, KP>(a, a.tile_expert + off, a.tile_pair0 + off, a.tile_n + off, u0, u1, part, scales, tiles, tokens, entries, signs, lt);
+    const uint32_t w0 = (uint32_t)((uint64_t)at * work / G), w1 = (uint32_t)((uint64_t)(at + 1u) * work / G);
+    for (uint32_t from = w0; from < w1;) {                 // (a run of more than kTileInfos tiles in parts)
+        const uint32_t to = min(w1, (from / per_tile + kTileInfos) * per_tile);
+        if (from != w0) __syncthreads();
+        if constexpr (DOWN) down_items<SRC, SETS, KP>(a, list, from, to, lds, from == w0);
+        else gateup_units<SRC, SETS, KP>(a, list, from, to, lds, from == w0);
+        from = to;
+    }
 }
 
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
 hipError_t launch_staged_list(const StagedArgs &a, uint32_t grid, hipStream_t s) {
-    REDHIP_LAUNCH((staged_tiles_kernel<SRC, DOWN, SETS, KP>), dim3(grid), dim3(staged_threads(SETS, KP)), 0, s, a);
+    REDHIP_LAUNCH((staged_tiles_kernel<SRC, DOWN, SETS, KP>), dim3(grid), dim3(DOWN ? 64u * down_waves(SETS) : kGateUpThreads), 0, s, a);
     return hipGetLastError();
 }
 // wide: wide tiles that the chunk is expected to have
 template <int SRC, bool DOWN, uint32_t KP>
 hipError_t launch_staged_lists(StagedArgs a, uint32_t grid, uint32_t wide, hipStream_t s) {
-    a.few = few_wide<SRC, DOWN>(a.rows, 256u * KP);
+    a.few = few_wide<SRC, DOWN, KP>(a.rows, 256u * KP);
     hipError_t e = hipSuccess;
     if (wide < a.few) a.few = ~0u;                         // (without a wide launch the narrow one takes everything)
-    if constexpr (has_wide<SRC, DOWN>()) {
+    if constexpr (has_wide<SRC, DOWN, KP>()) {
         if (a.few != ~0u) e = launch_staged_list<SRC, DOWN, 2, KP>(a, grid, s);
     }
     return e == hipSuccess ? launch_staged_list<SRC, DOWN, 1, KP>(a, grid, s) : e;

@@ -61,18 +61,13 @@ template <int SRC>
 __device__ __forceinline__ float unit_product(const Quarter &v, uint2 d, const _Float16 *planes, uint32_t i, uint32_t q, const LaneTables &lt) {
     float4_t acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};      // (half of the block each: half as many roundings behind one another)
     half2_t f{};
-#pragma unroll
-    for (uint32_t s = 0; s < 8u; ++s) {
-        if (s % steps_per_scale<SRC>() == 0u) f = step_scale<SRC>(v, s);
-        acc[s >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(term_operand(planes, s, i, q), finish_entry<SRC>(fetch_entry<SRC>(v, s, lt), f), acc[s >> 2], 0, 0, 0);
-    }
+    each_step([&](auto step) {
+        constexpr uint32_t s = decltype(step)::value;
+        if constexpr (s % steps_per_scale<SRC>() == 0u) f = step_scale<SRC, s>(v);
+        acc[s >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(term_operand(planes, s, i, q), finish_entry<SRC>(fetch_entry<SRC, s>(v, lt), f, lt), acc[s >> 2], 0, 0, 0);
+    });
     acc[0] += acc[1];
     return (acc[0][0] + (acc[0][1] + acc[0][2] * 4.8828125e-4f) * 4.8828125e-4f) * quarter_d<SRC>(d);
-}
-
-template <int SRC> __device__ __forceinline__ LaneTables lane_tables(const uint8_t *entries, const uint32_t *signs, uint32_t tid) {
-    constexpr uint32_t C = sign_copies<SRC>() ? sign_copies<SRC>() : 1u;
-    return LaneTables{entries + (tid % small_copies<SRC>()) * (is_iq3<SRC>() ? 8u : 16u), reinterpret_cast<const uint8_t *>(signs) + (tid % C) * 4u};
 }
 
 // act[slot][r] = SiLU(gate[r] . x) * (up[r] . x). Sixteen waves: KP of them, one block of 256 columns each (or every KP-th), share 16 gate

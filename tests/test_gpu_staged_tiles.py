@@ -40,7 +40,7 @@ def routing_with(counts, ntok, top_k, rng):
 # (hidden, ffn): K parts 2 / 4 / 8 of the gate/up kernel, 1 / 2 / 3 / 4 of the down kernel
 SHAPES = [("iq2", 512, 256), ("f2", 1024, 512), ("xs", 2048, 768), ("m", 512, 1024), ("iq2", 1024, 768), ("f2", 512, 768), ("xs", 512, 512), ("m", 1024, 256),
           ("f2", 2048, 256), ("xs", 1024, 1024), ("m", 512, 768), ("iq2", 512, 1024), ("f2", 512, 1024)]
-# 1008 wide tiles are above both kernels' lines for these (220 million weights in them for gate/up, 230 / 145 million for down)
+# 1008 wide tiles are above both kernels' lines for these (290 million weights in them for gate/up, 200 million for down)
 WIDE = [("iq2", 512, 512), ("iq2", 1024, 256), ("f2", 1024, 512), ("f2", 512, 768), ("f2", 1024, 256), ("f2", 512, 1024), ("xs", 512, 512), ("xs", 1024, 1024), ("m", 1024, 256),
         ("m", 512, 768), ("m", 2048, 512)]
 

@@ -1732,7 +1732,7 @@ __device__ const SignWordTable redhip_sign_words = make_sign_words();
 // bits below the entry index and the table bases the bits above it - magnitudes (64 KB-aligned): entry << 8 | (lane % 16) << 4; sign
 // words (aligned to their size): field << (2 + log2 LR) | (lane % LR) << 2 - so that an address is one byte permute resp. a shift and an
 // and-or of the packed group word, with no add.
-struct LaneTables { uint32_t mag_lane, lut_lane; };
+struct LaneTables { uint32_t mag_lane, lut_lane, lut_mask, sign_bits; };      // (the masks in vector registers)
 typedef uint32_t lds_u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const lds_u32x4 *lds_u32x4_ptr;
 typedef __attribute__((address_space(3))) const uint32_t *lds_u32_ptr;
@@ -1740,7 +1740,8 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) { return (uint32_
 template <int REP, int LR>
 __device__ __forceinline__ LaneTables lane_tables(const uint8_t *mag, const uint8_t *lut, uint32_t lane) {
     static_assert(REP == 16 && (LR == 8 || LR == 16 || LR == 32), "address bit layout");
-    return LaneTables{lds_address(mag) + (lane % (uint32_t)REP) * 16u, lds_address(lut) + (lane % (uint32_t)LR) * 4u};
+    return LaneTables{lds_address(mag) + (lane % (uint32_t)REP) * 16u, lds_address(lut) + (lane % (uint32_t)LR) * 4u, in_vector(127u << (LR == 8 ? 5u : LR == 16 ? 6u : 7u)),
+                      in_vector(0x80008000u)};
 }
 // eight signed weights: group word pair q, index / sign field L (0..3)
 template <int REP, int LR, uint32_t L>
@@ -1748,8 +1749,7 @@ __device__ __forceinline__ void signed_weights_lut(const LaneTables &t, uint2 q,
     constexpr uint32_t kLutShift = LR == 8 ? 5u : LR == 16 ? 6u : 7u;      // log2 of the bytes per sign field
     // bytes of the magnitude address: [low byte of the lane's base, index byte L of q.x, upper two bytes of the lane's base]
     const uint32_t mag_at = __builtin_amdgcn_perm(q.x, t.mag_lane, 0x03020000u | ((4u + L) << 8));
-    const uint32_t field = 7u * L < kLutShift ? q.y << (kLutShift - 7u * L) : q.y >> (7u * L - kLutShift);
-    const uint32_t lut_at = (field & (127u << kLutShift)) | t.lut_lane;
+    const uint32_t lut_at = and_or(moved<7u * L, kLutShift>(q.y), t.lut_mask, t.lut_lane);
 #ifdef REDHIP_ABLATE_NO_LDS      // measurement builds only (build.py --ablate): the table reads replaced by register moves, results wrong
     const lds_u32x4 m = {mag_at, lut_at, mag_at ^ 0x1234u, lut_at + 7u};
     const uint32_t e = lut_at ^ mag_at;
@@ -1760,10 +1760,11 @@ __device__ __forceinline__ void signed_weights_lut(const LaneTables &t, uint2 q,
 #ifdef REDHIP_ABLATE_NO_SIGN     // ... the sign placement left out
     b0.u[0] = m.x ^ e; b0.u[1] = m.y; b1.u[0] = m.z; b1.u[1] = m.w;
 #else
-    b0.u[0] = (e & 0x80008000u) | m.x;
-    b0.u[1] = ((e << 1) & 0x80008000u) | m.y;
-    b1.u[0] = ((e << 2) & 0x80008000u) | m.z;
-    b1.u[1] = ((e << 3) & 0x80008000u) | m.w;
+    const uint32_t e1 = twice(e), e2 = twice(e1), e3 = twice(e2);
+    b0.u[0] = and_or(e, t.sign_bits, m.x);
+    b0.u[1] = and_or(e1, t.sign_bits, m.y);
+    b1.u[0] = and_or(e2, t.sign_bits, m.z);
+    b1.u[1] = and_or(e3, t.sign_bits, m.w);
 #endif
 }
 template <int REP, int LR, uint32_t L>

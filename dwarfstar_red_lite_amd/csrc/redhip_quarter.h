@@ -12,16 +12,6 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 union H8 { uint4 u; half8_t v; half2_t p[4]; _Float16 e[8]; };
 
-// A SIMD takes the simple 32-bit instructions (and, or, xor, bitop3, add, sub, right shifts; f32 add, mul, fma) of two waves side by side as
-// long as every operand is a vector register or an inline constant: 2.2 .. 2.6 cycles each with four waves. With a scalar register or a
-// literal among the operands, and for left shifts, bit-field extracts, permutes, and_or, lshl_or and packed fp16, it is 4.3. So the decode
-// keeps its masks in vector registers, shifts left by additions and merges by bitop3.
-__device__ __forceinline__ uint32_t in_vector(uint32_t k) { asm("" : "+v"(k)); return k; }
-__device__ __forceinline__ uint32_t twice(uint32_t v) { uint32_t r; asm("v_add_u32 %0, %1, %1" : "=v"(r) : "v"(v)); return r; }
-__device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0xea); }
-// bits of w, those at position `from` moved to `to`
-template <uint32_t FROM, uint32_t TO> __device__ __forceinline__ uint32_t moved(uint32_t w) { return FROM >= TO ? w >> (FROM >= TO ? FROM - TO : 0u) : w << (FROM < TO ? TO - FROM : 0u); }
-
 // row sources: format (low half, what the decode goes by) and layout
 enum : int { F_XXS = 0, F_XS = 1, F_M = 2, F_IQ3 = 3, F_IQ3_WORDS = 4, L_RAW = 0, L_ROWS = 8, L_TILED = 16 };
 enum : int { S_XXS = F_XXS, S_XS = F_XS, S_M = F_M, S_IQ3 = F_IQ3, S_ROWS_XXS = F_XXS | L_ROWS, S_TILED_XXS = F_XXS | L_TILED, S_TILED_XS = F_XS | L_TILED,

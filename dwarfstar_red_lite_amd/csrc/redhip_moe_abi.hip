@@ -138,15 +138,30 @@ struct Moe {
     // batches that run as expert slices per pass: 2..8 tokens and at most 128 pairs on mixed layouts (their first launch multiplies the
     // shared expert's gate | up rows for up to eight tokens), 2..16 tokens and at most 256 pairs on all-IQ2_XXS layers - 2..32 tokens and
     // 512 pairs behind the layer's own router (own_router: the selection launch sorts that many; a caller's routing is sorted by one more
-    // workgroup of the launch that splits the activations, up to 256 pairs). Behind the own router the slices are ahead of the tiles up to
-    // there: 17, 24, 32 tokens 77 / 90, 98 / 111, 124 / 130 us, IQ3_S down 87 / 107, 109 / 122, 135 / 137, IQ2_XS 90 / 117, 114 / 136, 141 / 152
+    // workgroup of the launch that splits the activations, up to 256 pairs)
     static constexpr uint32_t kSmallMaxFused = 16u, kSmallMaxRouted = 32u, kSmallMaxGiven = 24u, kSmallMaxMixed = 32u;
+    // ... unless the tiles are ahead from fewer tokens on. The slices cost a pass per two pairs of an expert, the tiles a decode per distinct expert,
+    // so the line lies lower where a unit of the tiles' decode is cheap (IQ2_XXS everywhere, IQ1_M everywhere) and the experts are large
+    // enough to fill their launches; a call with given routing does not know how it is spread. Slices / tiles, us per layer of 2048 x 512, 512 experts, ten a token:
+    //   own router: IQ2_XXS 20, 24, 28, 32 tokens 85 / 86, 97 / 94, 109 / 102, 121 / 110; IQ1_M 24, 26, 28, 32: 108 / 111, 116 / 114, 120 / 117, 134 / 123;
+    //     IQ3_S down 28, 32: 121 / 127, 134 / 128; IQ2_XS 28, 32: 129 / 136, 142 / 147
+    //   given, evenly / with Zipf popularity / on 32 hot experts: IQ2_XXS 18 tokens 69 / 72, 61 / 58, 58 / 51, 20: 75 / 75, 67 / 59, 63 / 53; IQ1_M 22:
+    //     96 / 98, 87 / 81, 82 / 72, 24: 102 / 100, 91 / 84, 86 / 75; IQ3_S down 24: 105 / 108, 94 / 89, 87 / 80; IQ2_XS 24: 109 / 117, 97 / 100, 92 / 84
+    // IQ2_XXS layers of 2048 x 768, 128 experts, eight a token: own router 18, 24 tokens 78 / 81, 95 / 87; evenly given 18, 24: 73 / 73, 88 / 80. Of 1024 x
+    // 512 and less the slices stay ahead (32 tokens of 1024 x 512: 65 / 65).
+    uint32_t slices_up_to(bool own_router) const {
+        if ((size_t)cfg.hidden * cfg.ffn >= (size_t)2048u * 512u) {
+            if (fused && tile_chunk(kSmallMaxRouted)) return own_router ? 22u : 19u;
+            if (gu_type == T_IQ1_M && stream_tiles_resident()) return own_router ? 25u : 22u;
+        }
+        return own_router ? (fused ? kSmallMaxRouted : kSmallMaxMixed) : kSmallMaxGiven;
+    }
     bool dense_routed = false;               // every layer has f32 copies of its router and of the shared expert's gate | up rows (set at creation)
     bool small_batch(uint32_t ntok, bool own_router = false) const {
         if (ntok < 2u || cfg.hidden / 512u > 4u) return false;
-        if (fused) return ntok <= (own_router ? kSmallMaxRouted : kSmallMaxFused) && ntok * cfg.top_k <= (own_router ? 512u : 256u);
+        if (fused) return ntok <= (own_router ? slices_up_to(true) : kSmallMaxFused) && ntok * cfg.top_k <= (own_router ? 512u : 256u);
         // (mixed layouts behind their own router: the router launch is repeated per sixteen tokens, the selection launch sorts up to 512 pairs)
-        if (own_router && ntok > 8u) return mixed_slices && dense_routed && ntok <= kSmallMaxMixed && ntok * cfg.top_k <= 512u;
+        if (own_router && ntok > 8u) return mixed_slices && dense_routed && ntok <= slices_up_to(true) && ntok * cfg.top_k <= 512u;
         return mixed_slices && ntok <= 8u && ntok * cfg.top_k <= 128u && ntok * (cfg.top_k + 1u) <= 144u;
     }
     // ... with the layer's own router: on a mixed layout two tokens are quicker on the single-token kernels (three launches, the selection
@@ -826,7 +841,7 @@ int redhip_moe_route(redhip_moe_t h, uint32_t layer, const float *x_dev, uint32_
                              (m->mixed && m->sh_gu_type == T_Q6_K && c.router_type == T_Q6_K && (ntok == 1u || m->small_batch_mixed(ntok)) && c.top_k >= 2u);
         const bool dense_multi = !dense_small && m->mixed && ntok > 8u && m->small_batch(ntok, true) && router_f32 && m->layers[layer].dense_gu;
         if (dense_multi) {
-            // 9..32 tokens on a mixed layout whose batches run as slices: the launch of the small batches once per sixteen tokens, each
+            // 9 tokens and more on a mixed layout whose batches run as slices: the launch of the small batches once per sixteen tokens, each
             // on its own rows of the activations, logits, fp16 halves and shared products (a block step: of the branch and the normalised rows too)
             BlockContext &bc = block_context();
             const BlockContext saved = bc;
@@ -899,9 +914,9 @@ int redhip_moe_experts(redhip_moe_t h, uint32_t layer, const float *x_dev, uint3
         const GroupJob job{ids_dev, weights_dev, ntok, m->cfg.top_k, m->cfg.n_expert, m->uid, m->expert_start, m->pair_token, m->pair_weight, m->tok_pair, m->n_unique, m->status,
                            m->small_batch(ntok) ? m->pass_list : nullptr, m->small_batch(ntok) ? m->n_pass : nullptr};
         bool grouped = false;
-        const bool mixed_mid = m->mixed_slices && ntok > 8u && ntok <= Moe::kSmallMaxGiven && m->small_batch(ntok, true) && L.dense_gu;
+        const bool mixed_mid = m->mixed_slices && ntok > 8u && ntok <= m->slices_up_to(false) && m->small_batch(ntok, true) && L.dense_gu;
         if (mixed_mid) {
-            // 9..24 tokens on a mixed layout whose batches run as slices: the shared expert's products, the fp16 halves and the scalar gates
+            // 9 tokens and more on a mixed layout whose batches run as slices: the shared expert's products, the fp16 halves and the scalar gates
             // from the launch of the small batches, once per sixteen tokens; then one launch sorts the pairs with their pass list
             prof_set_stage(ST_SHARED_GATEUP);
             const uint32_t per = (size_t)16u * m->cfg.hidden * 4u <= 128u * 1024u ? 16u : 8u;      // tokens whose activations fit the launch's LDS
@@ -929,12 +944,8 @@ int redhip_moe_experts(redhip_moe_t h, uint32_t layer, const float *x_dev, uint3
             prof_set_stage(ST_OTHER);
             HIP_OK(launch_prep(x_dev, L.gate_inp, ntok, m->cfg.hidden, m->xh, m->xl, m->xexp, m->scalar, s, to_group ? &job : nullptr, &grouped), "prep launch");
         }
-        if (m->fused && !grouped && !m->small_batch(ntok) && m->small_batch(ntok, true) && ntok <= Moe::kSmallMaxGiven) {
-            // 17..24 tokens on an all-IQ2_XXS layer: more pairs than the side job above sorts; one more launch sorts them with their pass list.
-            // (The slices cost a pass per two pairs of an expert, the tile kernels a decode per distinct expert, and the call does not know its
-            // routing. Slices / tiles at 17, 24, 32 tokens, us: evenly routed 69 / 84, 88 / 101, 110 / 111; Zipf popularity 61 / 68, 77 / 79, 98 /
-            // 90; 32 hot experts 57 / 57, 73 / 65, 92 / 75. Mixed layouts (above), IQ2_XS: even 87 / 108, 109 / 124, 135 / 142; Zipf 78 / 94,
-            // 97 / 105, 121 / 113; hot 73 / 80, 91 / 86, 116 / 94.)
+        if (m->fused && !grouped && !m->small_batch(ntok) && m->small_batch(ntok, true) && ntok <= m->slices_up_to(false)) {
+            // 17 tokens and more on an all-IQ2_XXS layer: more pairs than the side job above sorts; one more launch sorts them with their pass list
             const GroupJob big{ids_dev, weights_dev, ntok, m->cfg.top_k, m->cfg.n_expert, m->uid, m->expert_start, m->pair_token, m->pair_weight, m->tok_pair, m->n_unique,
                                m->status, m->pass_list, m->n_pass};
             prof_set_stage(ST_GROUP);

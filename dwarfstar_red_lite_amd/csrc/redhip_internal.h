@@ -181,9 +181,9 @@ hipError_t launch_batch_combine(const float *tmp, const float *pair_weight, cons
                                 const float *sh_tmp, const float *scalar, uint32_t hidden, float *out, hipStream_t s);
 
 // pair sort of [ntok][top_k] ids: see redhip_moe_group in include/redhip_moe.h
-// f32 router logits of a chunk of tokens as a tiled fp32 MFMA product (every router row read once per 32 tokens), plus the
+// f32 router logits of a chunk of tokens as a tiled product, three bf16 terms for each f32 (every router row read once per 16 or 32 tokens), plus the
 // fp16 split of the activations; same outputs as launch_router_gemv
-// out[tok][row] = W[row] . x[tok] on the fp32 matrix units: W f32 [n_rows][K] (+ one optional extra row), x f32 [ntok][K]
+// out[tok][row] = W[row] . x[tok] in the same way: W f32 [n_rows][K] (+ one optional extra row), x f32 [ntok][K]
 hipError_t launch_f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out,
                             uint32_t out_stride, void *xh, void *xl, int *xexp, hipStream_t s);
 hipError_t launch_f32_swiglu_tiles(const float *w, const float *x, uint32_t ntok, uint32_t K, uint32_t ffn, float *act, hipStream_t s);

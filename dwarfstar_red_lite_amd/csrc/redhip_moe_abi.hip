@@ -94,8 +94,8 @@ struct Moe {
     static constexpr uint32_t kStageExperts = 64u;
     // handles that can be given chunks keep a tile-major copy for the prefill kernels that hold a tile's activations in registers
     // larger chunks take the router as a tiled f32 product (a quantised router through its f32 copy)
-    // (below 40 tokens the f32 rows are quicker one token per grid layer - 12.1 against 14.0 us at 32 tokens, 14.4 against 13.8 at 40:
-    // 32 x 32 tiles leave most of the chip idle there)
+    // (below 40 tokens the f32 rows are quicker one token per grid layer where a router is small: 33 tokens of 1024 x 96 experts 2.4 us, of 2048 x 128
+    // experts 4.6 us; 512 experts' tiles would be 3 us ahead from 36 tokens on)
     bool tiled_router(uint32_t ntok) const { return packed_gu() && ntok >= 40u && (cfg.router_type == T_F32 || mixed); }
     uint64_t tiled_stride() const { return fused ? expert_stride : packed_stride; }      // bytes between experts in `tiled`
     bool tiles_resident() const { return packed_gu() && gu_type == T_IQ2_XXS && cfg.max_tokens > 8u && cfg.ffn <= 512u && cfg.hidden / 512u <= 4u; }
@@ -325,9 +325,9 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
         const uint32_t P = ntok * c.top_k, n_groups = P < c.n_expert ? P : c.n_expert;
         const ExpertSet ex = m->routed(layer), sh = m->shared(layer);
         const Layer &Ld = m->layers[layer];
-        // the shared expert as dense f32 products on the fp32 matrix units, started before the pair sort (one workgroup on an idle machine;
+        // the shared expert as dense f32 products, started before the pair sort (one workgroup on an idle machine;
         // the many-workgroup sort of a large chunk then queues behind the dense tiles - 73 against 22 us at 2048 tokens - but started
-        // behind the sort the dense products slow the down tiles by more: 787 against 760 us per chunk)
+        // behind the sort the dense products slow the down tiles by more: 787 against 760 us per chunk, both with products on the fp32 units)
         const bool tile_path = !m->small_batch(ntok) && !(m->small_batch(ntok, true) && grouped) && m->tile_chunk(ntok);
         const bool dense_shared = tile_path && m->mixed && Ld.dense_gu && m->side;
         if (dense_shared && !fork_shared_dense(m, Ld, x, ntok, s)) return 0;

@@ -1,8 +1,10 @@
 // What a chunk of tokens (prefill) needs beside its tile kernels (redhip_tiles.hip): the tile lists, the tile-major copies of the experts'
-// matrices, and dense f32 products on the fp32 matrix units (router logits, the shared expert of mixed layouts).
+// matrices, and dense f32 products on the bf16 matrix units, three terms for each f32 (router logits, the shared expert of mixed layouts).
 #include <hip/hip_runtime.h>
 
 #include "redhip_mfma.h"
+
+#include <type_traits>
 
 namespace redhip {
 
@@ -97,19 +99,25 @@ hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count
 
 // ---------------------------------------------------------------- router logits of a token chunk
 
-// out[tok][row] = W[row] . x[tok] for an f32 matrix W (a router, the dense shared expert of mixed layouts) and a chunk of activations, on
-// v_mfma_f32_16x16x4_f32 (full fp32 multiply-add). A workgroup owns BR = 16 MR WR rows x BT = 16 MT WT tokens; a wave MR blocks of 16 rows times
-// MT of 16 tokens, and half of k: the waves come in two sets, one for the even slices of 64 k, one for the odd ones, whose sums meet in LDS at
-// the end. Both operands pass through LDS (SLICE k of either half per round, double-buffered, the next two rounds in registers). Lane
-// (r = l % 16, q = l / 16) reads four consecutive k of row r and of token r and feeds them to four MFMAs (A[i = r][k = q], B[k = q][j = r],
-// D[i = 4q .. 4q + 3][j = r]; the order of k does not matter as long as both operands agree).
-// What bounds it: the matrix pipe where a tile is large (64 x 64: 16 bytes of L2 per clock and compute unit; tiles of 32 x 32 for every size
-// needed 32, and waited for them), the number of workgroups where a chunk is small. So the tile is chosen by the launch (f32_tile_choice).
-// The order in which an output's products are added is the same for every tile. The matrix unit rounds with every product, so the dense
-// products leave it after 32 columns and are added up in double: of a shared expert's 2048-column rows 0.9e-7 is lost instead of 3.5e-7 (and of
-// the output of an IQ1_M layer 1.6e-7 instead of 6e-7). A router keeps two plain chains: nothing but the selection hangs on its last bits.
-// SWIGLU: W holds gate rows, then as many up rows; two row blocks beside each other are the gate and the up rows of 16 columns, and out gets
-// silu(gate) * up of them: no pass of its own over the products.
+// out[tok][row] = W[row] . x[tok] for an f32 matrix W (a router, the dense shared expert of mixed layouts) and a chunk of activations. Every f32
+// is the sum of three bf16 numbers, exactly (its bits cut after 8 and 16 places; two of three operations on it are full-rate ones), and of the
+// nine products of such sums the six that reach 2^-24 of the largest go through v_mfma_f32_16x16x32_bf16: six of those are 96 cycles for 32 columns
+// where the fp32 unit takes 256. The products of the leading terms have accumulators of their own, the other five share one.
+// A workgroup owns BR = 16 MR rows x BT = 16 MT tokens, each of its eight waves an eighth of k for all of them; the eight sums meet in LDS, in
+// double. A wave fetches 32 columns of every row and token straight into LDS (full 128-byte lines: sixteen lanes of a load that name sixteen rows
+// take four times as long, 26 instead of 15 us for 64 x 32 outputs of 2048 columns), takes them into registers as fragments (lane (r = l % 16, q = l / 16):
+// columns 4q .. 4q + 3 and 16 + 4q .. of row r; the 16-byte pieces of a row are permuted by r / 2 so that a read pass meets every bank once),
+// requests the next 32 columns into the same place and multiplies meanwhile. No barrier before the sums meet.
+// What bounds it: the fetch - 96 KB in flight for a tile of 64 x 32, which cover about the 1 .. 1.5 us that they take - then cutting and multiplying
+// (2300 .. 3000 cycles for each 256 columns). us, before (v_mfma_f32_16x16x4_f32, both operands through registers into LDS) -> now:
+// gate/up with SwiGLU of 1024 x 2048: 77 tokens 12.3 -> 7.9, 512: 31 -> 19.7, 2048: 95 -> 81; down 2048 x 512: 77 tokens 6.7 -> 4.7, 512: 16.6 -> 14,
+// 2048: 58 -> 53; router 512 x 2048: 77 tokens 10.5 -> 7.2, 512: 19 -> 11.8, 2048: 48 -> 37.
+// The order in which an output's products are added is the same for every tile. Error against a sum in double, of the rms of the outputs: 2048
+// columns 0.94e-7 (two chains of leading products), 512 columns 0.8e-7, where the fp32 unit with totals in double left 1.04e-7 and 1.1e-7 (and 4.1e-7
+// in a router's plain chains). The gate and up products, which SwiGLU multiplies, leave their chain for a double after every 64 columns: 0.8e-7.
+// An infinity or NaN has no three terms, and an infinite sum may come out as NaN: outputs that are not finite are computed again, product by product.
+// SWIGLU: W holds gate rows, then as many up rows; the upper half of a tile's row blocks are gate rows, the lower half the up rows of the same
+// columns, and out gets silu(gate) * up of them: no pass of its own over the products.
 // Launches with xh get workgroups behind the tiles that write the fp16 halves of the activations (a wave per token, split_token) and multiply them
 // with gate_inp, if there is one, as row n_rows; without xh the tiles have it as a further row.
 
@@ -159,15 +167,34 @@ __device__ __forceinline__ void split_token(const float *gate_inp, const float *
             }
 }
 
-template <int MR, int MT, uint32_t WR, uint32_t WT, uint32_t SLICE, bool SWIGLU, bool ROUTER>
-__global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w, const float *gate_inp, const float *x, float *out, uint32_t out_stride, _Float16 *xh,
-                                                                  _Float16 *xl, int *xexp, uint32_t K, uint32_t n_rows, uint32_t ntok) {
-    constexpr uint32_t BR = 16u * MR * WR, BT = 16u * MT * WT, T = 128u * WR * WT, P = SLICE / 4u, D = T / (2u * P), NW = BR / D, NX = BT / D;      // P pieces of 16 bytes per row, D rows per pass of the threads
-    __shared__ __attribute__((aligned(16))) float lds[2][2][BR + BT][SLICE + 4u];      // [buffer][k half][W rows, then tokens]
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t uint32x4_t __attribute__((ext_vector_type(4)));
+struct ThreeTerms { bf16x8 high, mid, low; };
+// `top` = 0xffff0000 in a vector register
+__device__ __forceinline__ ThreeTerms three_terms(float4_t a, float4_t b, uint32_t top) {
+    const auto cut = [&](float v) { return __uint_as_float(__float_as_uint(v) & top); };
+    const auto tops = [](float v1, float v0) { return __builtin_amdgcn_perm(__float_as_uint(v1), __float_as_uint(v0), 0x07060302u); };
+    uint32x4_t h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float v0 = i < 2 ? a[2 * (i & 1)] : b[2 * (i & 1)], v1 = i < 2 ? a[2 * (i & 1) + 1] : b[2 * (i & 1) + 1];
+        const float r0 = v0 - cut(v0), r1 = v1 - cut(v1), s0 = r0 - cut(r0), s1 = r1 - cut(r1);      // (each exact)
+        h[i] = tops(v1, v0);
+        m[i] = tops(r1, r0);
+        l[i] = tops(s1, s0);
+    }
+    return ThreeTerms{__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+}
+
+template <int MR, int MT, bool SWIGLU>
+__global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const float *gate_inp, const float *x, float *out, uint32_t out_stride, _Float16 *xh,
+                                                        _Float16 *xl, int *xexp, uint32_t K, uint32_t n_rows, uint32_t ntok) {
+    constexpr uint32_t BR = 16u * MR, BT = 16u * MT, NB = MR + MT, PIECES = 2u * NB > MR * MT ? 2u * NB : MR * MT;      // KB per wave: 32 columns of the rows and tokens, later its sums
+    __shared__ __attribute__((aligned(16))) float4_t lds[8][PIECES][64];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t all_rows = n_rows + (gate_inp && !xh ? 1u : 0u), row_tiles = (all_rows + BR - 1u) / BR, tok_tiles = (ntok + BT - 1u) / BT, n_tile = row_tiles * tok_tiles;
     if (blockIdx.x >= n_tile) {
-        const uint32_t tok = T / 64u * (blockIdx.x - n_tile) + wave;
+        const uint32_t tok = 8u * (blockIdx.x - n_tile) + wave;
         if (tok < ntok) split_token(gate_inp, x, out, out_stride, xh, xl, xexp, K, n_rows, tok, lane);
         return;
     }
@@ -180,173 +207,162 @@ __global__ __launch_bounds__(128 * WR * WT) void f32_tiles_kernel(const float *w
         tile_r = (xcd & 3u) * br + slot % br;
         tile_t = (xcd >> 2) * bt + slot / br;
     }
-    // staging: thread t moves the 16 bytes t % P of k half (t / P) % 2 of rows t / 2P, t / 2P + D, ..; rows and tokens beyond the last repeat
-    // another and are not stored. (LDS rows of SLICE + 4 floats: the sixteen lanes of a 16-byte read pass hit different banks)
-    const uint32_t scol = 4u * (tid % P), kh = (tid / P) & 1u, srow = tid / (2u * P);
-    const auto source = [&](uint32_t n) -> const float * {      // (n < NW: matrix rows, then tokens)
-        const uint32_t l = srow + n * D;
-        if (n >= NW) return x + (uint64_t)min(tile_t * BT + l - BR, ntok - 1u) * K + kh * 64u + scol;
-        const uint32_t row = SWIGLU ? ((l >> 4) & 1u) * (n_rows / 2u) + tile_r * (BR / 2u) + (l >> 5) * 16u + (l & 15u) : tile_r * BR + l;
-        return (row < n_rows ? w + (uint64_t)row * K : gate_inp ? gate_inp : w) + kh * 64u + scol;
+    // row block m of the tile starts here; rows and tokens beyond the last repeat another and are not stored
+    const auto block_row = [&](uint32_t m) { return SWIGLU ? (m < MR / 2u ? 0u : n_rows / 2u) + tile_r * (BR / 2u) + 16u * (m % (MR / 2u)) : tile_r * BR + 16u * m; };
+    const auto matrix_row = [&](uint32_t row) { return row < n_rows ? w + (uint64_t)row * K : gate_inp ? gate_inp : w; };
+    // fetch i of a wave: eight rows (or tokens) of 128 bytes; lane l brings piece (l % 8) ^ (row % 16 / 2) of row l / 8
+    const float *src[2u * NB];
+#pragma unroll
+    for (uint32_t i = 0; i < 2u * NB; ++i) {
+        const uint32_t l = 8u * (i & 1u) + (lane >> 3);
+        src[i] = i < 2u * MR ? matrix_row(block_row(i / 2u) + l) : x + (uint64_t)min(tile_t * BT + 16u * (i / 2u - MR) + l, ntok - 1u) * K;
+        src[i] += K / 8u * wave + 4u * ((lane & 7u) ^ (l >> 1));
+    }
+    float4_t *mine = &lds[wave][0][0];
+    const bool in_pieces = (reinterpret_cast<uintptr_t>(x) & 15u) == 0u;      // (the caller's activations may lie at any float)
+    const auto request = [&](uint32_t step) {
+        if (in_pieces) {
+#pragma unroll
+            for (uint32_t i = 0; i < 2u * NB; ++i)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src[i] + 32u * step), (__attribute__((address_space(3))) void *)(mine + 64u * i), 16, 0, 0);
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 2u * NB; ++i) {
+                const float *p = src[i] + 32u * step;
+                mine[64u * i + lane] = float4_t{p[0], p[1], p[2], p[3]};
+            }
+        }
     };
-    constexpr uint32_t N = NW + NX;
-    static_assert(N >= 3u && N <= 6u && NW * D == BR && NX * D == BT && (SLICE == 32u || SLICE == 64u), "16-byte pieces per thread and round");
-    const float *src0 = source(0u), *src1 = source(1u), *src2 = source(2u), *src3 = source(3u < N ? 3u : 0u), *src4 = source(4u < N ? 4u : 0u), *src5 = source(5u < N ? 5u : 0u);
-    const uint32_t n_round = K / (2u * SLICE);             // even: K is a multiple of 256
-    struct Staged { float4_t v0, v1, v2, v3, v4, v5; };    // (as an array, or of float4 objects, these end up in scratch memory)
-    const auto request = [&](Staged &st, uint32_t rd) {    // (the last rounds request themselves again: no branch around the loads)
-        const uint32_t at = SLICE == 64u ? rd * 128u : (rd >> 1) * 128u + (rd & 1u) * 32u;
-        st.v0 = *reinterpret_cast<const float4_t *>(src0 + at);
-        st.v1 = *reinterpret_cast<const float4_t *>(src1 + at);
-        st.v2 = *reinterpret_cast<const float4_t *>(src2 + at);
-        if constexpr (N > 3u) st.v3 = *reinterpret_cast<const float4_t *>(src3 + at);
-        if constexpr (N > 4u) st.v4 = *reinterpret_cast<const float4_t *>(src4 + at);
-        if constexpr (N > 5u) st.v5 = *reinterpret_cast<const float4_t *>(src5 + at);
-    };
-    const auto place = [&](const Staged &st, uint32_t buf) {      // (tokens follow the rows)
-        *reinterpret_cast<float4_t *>(&lds[buf][kh][srow][scol]) = st.v0;
-        *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + D][scol]) = st.v1;
-        *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + 2u * D][scol]) = st.v2;
-        if constexpr (N > 3u) *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + 3u * D][scol]) = st.v3;
-        if constexpr (N > 4u) *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + 4u * D][scol]) = st.v4;
-        if constexpr (N > 5u) *reinterpret_cast<float4_t *>(&lds[buf][kh][srow + 5u * D][scol]) = st.v5;
-    };
-    const uint32_t mh = wave / (WR * WT), block = wave % (WR * WT), wr = block % WR, wt = block / WR;
-    constexpr int CH = ROUTER ? 2 : 1;
-    float4_t acc[MR][MT][CH];
+    constexpr int CH = SWIGLU ? 1 : 2;
+    float4_t high[CH][MR][MT], low[MR][MT];
     double total[MR][MT][4];
 #pragma unroll
     for (int m = 0; m < MR; ++m)
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-#pragma unroll
-            for (int c = 0; c < CH; ++c) acc[m][t][c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            high[0][m][t] = high[CH - 1][m][t] = low[m][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int i = 0; i < 4; ++i) total[m][t][i] = 0.0;
         }
-    const auto multiply = [&](uint32_t buf) {
+    const uint32_t top = in_vector(0xffff0000u), at0 = 8u * r + (q ^ (r >> 1)), at1 = 8u * r + ((q + 4u) ^ (r >> 1)), steps = K / 256u;
+    const auto multiply = [&](uint32_t step, auto chain) {
+        constexpr int C = decltype(chain)::value;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this step's columns are in LDS
+        float4_t v[NB][2];
 #pragma unroll
-        for (uint32_t u = 0; u < SLICE / 16u; ++u) {
-            float4 a[MR], b[MT];
+        for (uint32_t i = 0; i < NB; ++i) { v[i][0] = mine[128u * i + at0]; v[i][1] = mine[128u * i + at1]; }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // and read, before the next ones take their place
+        if (step + 1u < steps) request(step + 1u);
+        __builtin_amdgcn_sched_barrier(0);
+        ThreeTerms b[MT];
 #pragma unroll
-            for (int m = 0; m < MR; ++m) a[m] = *reinterpret_cast<const float4 *>(&lds[buf][mh][16u * (MR * wr + m) + r][16u * u + 4u * q]);
+        for (int t = 0; t < MT; ++t) b[t] = three_terms(v[MR + t][0], v[MR + t][1], top);
 #pragma unroll
-            for (int t = 0; t < MT; ++t) b[t] = *reinterpret_cast<const float4 *>(&lds[buf][mh][BR + 16u * (MT * wt + t) + r][16u * u + 4u * q]);
+        for (int m = 0; m < MR; ++m) {
+            const ThreeTerms a = three_terms(v[m][0], v[m][1], top);
+            const auto add = [&](const bf16x8 &p, const bf16x8 &s, float4_t &to) { to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p, s, to, 0, 0, 0); };
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
+            for (int t = 0; t < MT; ++t) { add(a.high, b[t].high, high[C][m][t]); add(a.low, b[t].high, low[m][t]); }
 #pragma unroll
-                for (int m = 0; m < MR; ++m)
+            for (int t = 0; t < MT; ++t) add(a.mid, b[t].mid, low[m][t]);
 #pragma unroll
-                    for (int t = 0; t < MT; ++t)
-                        acc[m][t][k % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(k == 0 ? a[m].x : k == 1 ? a[m].y : k == 2 ? a[m].z : a[m].w,
-                                                                                k == 0 ? b[t].x : k == 1 ? b[t].y : k == 2 ? b[t].z : b[t].w, acc[m][t][k % CH], 0, 0, 0);
-            if constexpr (!ROUTER)
-                if (u & 1u) {
+            for (int t = 0; t < MT; ++t) add(a.high, b[t].low, low[m][t]);
 #pragma unroll
-                    for (int m = 0; m < MR; ++m)
+            for (int t = 0; t < MT; ++t) add(a.mid, b[t].high, low[m][t]);
 #pragma unroll
-                        for (int t = 0; t < MT; ++t) {
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) total[m][t][i] += acc[m][t][0][i];
-                            acc[m][t][0] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                        }
-                }
+            for (int t = 0; t < MT; ++t) add(a.high, b[t].mid, low[m][t]);
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-    Staged s0, s1;
-    request(s0, 0u);
-    request(s1, 1u);
-    for (uint32_t rd = 0; rd < n_round; rd += 2u) {
-        place(s0, 0u);
-        __syncthreads();                                   // round rd is in place; the readers of the other buffer (round rd - 1) are past their barrier
-        request(s0, rd + 2u < n_round ? rd + 2u : rd);
-        multiply(0u);
-        place(s1, 1u);
-        __syncthreads();
-        request(s1, rd + 3u < n_round ? rd + 3u : rd + 1u);
-        multiply(1u);
+    const auto flush = [&] {
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) total[m][t][i] += high[0][m][t][i];
+                high[0][m][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+    };
+    request(0u);
+    for (uint32_t step = 0; step < steps; step += 2u) {
+        multiply(step, std::integral_constant<int, 0>{});
+        if (step + 1u < steps) multiply(step + 1u, std::integral_constant<int, CH - 1>{});
+        if constexpr (SWIGLU) flush();
     }
-    float4_t sum[MR][MT];
+    __syncthreads();
 #pragma unroll
     for (int m = 0; m < MR; ++m)
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
+            float4_t v;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sum[m][t][i] = ROUTER ? acc[m][t][0][i] + acc[m][t][CH - 1][i] : (float)total[m][t][i];
+            for (int i = 0; i < 4; ++i) v[i] = SWIGLU ? (float)(total[m][t][i] + low[m][t][i]) : high[0][m][t][i] + high[CH - 1][m][t][i] + low[m][t][i];
+            (&lds[0][0][0])[(wave * MR * MT + m * MT + t) * 64u + lane] = v;
         }
-    // the odd slices' sums go through LDS to the waves that hold the even ones; SWIGLU with one row block per wave: then the up products to
-    // the wave of their gate rows
-    float4_t *meet = reinterpret_cast<float4_t *>(&lds[0][0][0][0]);
-    static_assert(sizeof(lds) >= (size_t)WR * WT * MR * MT * 64u * 16u, "the sums fit the staging buffers");
-    const auto at = [&](uint32_t b, int m, int t) { return ((b * MR + m) * MT + t) * 64u + lane; };
     __syncthreads();
-    if (mh == 1u) {
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
-#pragma unroll
-            for (int t = 0; t < MT; ++t) meet[at(block, m, t)] = sum[m][t];
-    }
-    __syncthreads();
-    if (mh == 0u) {
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
-#pragma unroll
-            for (int t = 0; t < MT; ++t) sum[m][t] += meet[at(block, m, t)];
-    }
-    if constexpr (SWIGLU && MR == 1) {
-        if (mh == 0u && (wr & 1u)) {
-#pragma unroll
-            for (int t = 0; t < MT; ++t) meet[at(block, 0, t)] = sum[0][t];      // (its own place: nobody else reads it before)
-        }
-        __syncthreads();
-    }
-    if (mh == 1u || (SWIGLU && MR == 1 && (wr & 1u))) return;
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const uint32_t tok = tile_t * BT + 16u * (MT * wt + t) + r;
+    // a thread: four consecutive rows of a token (D[i = 4q .. 4q + 3][j = r])
+    for (uint32_t o = tid; o < (SWIGLU ? MR / 2u : MR) * MT * 64u; o += 512u) {
+        const uint32_t t = (o >> 6) % MT, m = (o >> 6) / MT, l = o & 63u, tok = tile_t * BT + 16u * t + (l & 15u), row = 4u * (l >> 4);
         if (tok >= ntok) continue;
-        if constexpr (SWIGLU) {
-            float4_t y;
-            const float4_t g = sum[0][t], u = MR == 1 ? meet[at(block + 1u, 0, t)] : sum[MR - 1][t];
+        const auto products = [&](uint32_t mm) {
+            double sum[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) y[i] = (g[i] / (1.0f + expf(-g[i]))) * u[i];
-            *reinterpret_cast<float4_t *>(out + (uint64_t)tok * out_stride + tile_r * (BR / 2u) + 16u * (MR == 1 ? wr / 2u : wr) + 4u * q) = y;
+            for (uint32_t k = 0; k < 8u; ++k) {
+                const float4_t v = (&lds[0][0][0])[(k * MR * MT + mm * MT + t) * 64u + l];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sum[i] += v[i];
+            }
+            float4_t y;
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; ++i) {
+                y[i] = (float)sum[i];
+                if (!(fabsf(y[i]) <= 3.402823466e38f) && block_row(mm) + row + i < all_rows) {
+                    const float *wr = matrix_row(block_row(mm) + row + i), *xr = x + (uint64_t)tok * K;
+                    float again = 0.0f;
+                    for (uint32_t c = 0; c < K; ++c) again = fmaf(wr[c], xr[c], again);
+                    y[i] = again;
+                }
+            }
+            return y;
+        };
+        float4_t y = products(m);
+        if constexpr (SWIGLU) {
+            const float4_t u = products(m + MR / 2u);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = (y[i] / (1.0f + expf(-y[i]))) * u[i];
+            *reinterpret_cast<float4_t *>(out + (uint64_t)tok * out_stride + block_row(m) + row) = y;
         } else {
 #pragma unroll
-            for (int m = 0; m < MR; ++m)
-#pragma unroll
-                for (uint32_t i = 0; i < 4u; ++i) {
-                    const uint32_t row = tile_r * BR + 16u * (MR * wr + m) + 4u * q + i;
-                    if (row < all_rows) out[(uint64_t)tok * out_stride + row] = sum[m][t][i];
-                }
+            for (uint32_t i = 0; i < 4u; ++i)
+                if (block_row(m) + row + i < all_rows) out[(uint64_t)tok * out_stride + block_row(m) + row + i] = y[i];
         }
     }
 }
 
-// The largest tile that costs no more rounds of the device (256 compute units, workgroups of equal length) than a quarter above the best
-// tile: large tiles read less, small ones fill the device when a chunk has few outputs.
-template <bool SWIGLU, bool ROUTER>
+// The tile that costs least: rounds of the device (256 compute units) times what a round of workgroups of it takes, 18, 10 and 7 us for 2048
+// columns of 64 x 32, 32 x 32 and 32 x 16 outputs (gate/up of 512 tokens 19.7 / 23.4 / 26.4 us, of 77 tokens 16.2 / 10.8 / 7.9, down of 77 tokens, 512
+// columns, 6.7 / 4.7 / 5.1, router of 512 tokens 16.9 / 11.8 / 14.2).
+template <bool SWIGLU>
 hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out, uint32_t out_stride, void *xh, void *xl,
                      int *xexp, hipStream_t s) {
     if (!ntok || !K || K % 256u || !n_rows || !w || !x || !out || (SWIGLU && n_rows % 128u)) return hipErrorInvalidValue;
     const uint32_t all_rows = n_rows + (extra_row && !xh ? 1u : 0u);
-    static constexpr struct { uint32_t br, bt; } kTiles[4] = {{64u, 64u}, {64u, 32u}, {32u, 32u}, {32u, 16u}};
-    uint64_t n[4], cost[4], best = ~0ull;
-    for (int i = 0; i < 4; ++i) {
-        n[i] = (uint64_t)((all_rows + kTiles[i].br - 1u) / kTiles[i].br) * ((ntok + kTiles[i].bt - 1u) / kTiles[i].bt);
-        cost[i] = (n[i] + 255u) / 256u * (kTiles[i].br * kTiles[i].bt);
-        if (cost[i] < best) best = cost[i];
-    }
+    static constexpr struct { uint32_t br, bt, round; } kTiles[3] = {{64u, 32u, 18u}, {32u, 32u, 10u}, {32u, 16u, 7u}};
+    uint64_t n[3], best = ~0ull;
     int pick = 0;
-    while (4u * cost[pick] > 5u * best) ++pick;
-    const uint32_t waves = pick < 3 ? 8u : 4u, split_wgs = xh ? (ntok + waves - 1u) / waves : 0u;      // (behind the tiles)
+    for (int i = 0; i < 3; ++i) {
+        n[i] = (uint64_t)((all_rows + kTiles[i].br - 1u) / kTiles[i].br) * ((ntok + kTiles[i].bt - 1u) / kTiles[i].bt);
+        const uint64_t cost = (n[i] + 255u) / 256u * kTiles[i].round;
+        if (cost < best) { best = cost; pick = i; }
+    }
+    const uint32_t split_wgs = xh ? (ntok + 7u) / 8u : 0u;      // (behind the tiles)
     if (n[pick] + split_wgs > 0x7fffffffull) return hipErrorInvalidValue;
-    const dim3 grid((uint32_t)n[pick] + split_wgs), block(64u * waves);
+    const dim3 grid((uint32_t)n[pick] + split_wgs), block(512u);
     _Float16 *h = static_cast<_Float16 *>(xh), *l = static_cast<_Float16 *>(xl);
-    if (pick == 0) REDHIP_LAUNCH((f32_tiles_kernel<2, 2, 2u, 2u, 32u, SWIGLU, ROUTER>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
-    else if (pick == 1) REDHIP_LAUNCH((f32_tiles_kernel<2, 1, 2u, 2u, 32u, SWIGLU, ROUTER>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
-    else if (pick == 2) REDHIP_LAUNCH((f32_tiles_kernel<1, 1, 2u, 2u, 64u, SWIGLU, ROUTER>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
-    else REDHIP_LAUNCH((f32_tiles_kernel<1, 1, 2u, 1u, 64u, SWIGLU, ROUTER>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    if (pick == 0) REDHIP_LAUNCH((f32_tiles_kernel<4, 2, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    else if (pick == 1) REDHIP_LAUNCH((f32_tiles_kernel<2, 2, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    else REDHIP_LAUNCH((f32_tiles_kernel<2, 1, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
     return hipGetLastError();
 }
 
@@ -354,16 +370,16 @@ hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uin
 // row behind the matrix; xh / xl / xexp (optional): also write the fp16 halves of x
 hipError_t launch_f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out,
                             uint32_t out_stride, void *xh, void *xl, int *xexp, hipStream_t s) {
-    return f32_tiles<false, false>(w, extra_row, x, ntok, K, n_rows, out, out_stride, xh, xl, xexp, s);
+    return f32_tiles<false>(w, extra_row, x, ntok, K, n_rows, out, out_stride, xh, xl, xexp, s);
 }
 // act[tok][c] = silu(W[c] . x[tok]) * (W[ffn + c] . x[tok])
 hipError_t launch_f32_swiglu_tiles(const float *w, const float *x, uint32_t ntok, uint32_t K, uint32_t ffn, float *act, hipStream_t s) {
-    return f32_tiles<true, false>(w, nullptr, x, ntok, K, 2u * ffn, act, ffn, nullptr, nullptr, nullptr, s);
+    return f32_tiles<true>(w, nullptr, x, ntok, K, 2u * ffn, act, ffn, nullptr, nullptr, nullptr, s);
 }
 
 hipError_t launch_router_f32_tiles(const float *w, const float *gate_inp, const float *x, uint32_t ntok, uint32_t hidden, uint32_t n_expert,
                                    float *logits, void *xh, void *xl, int *xexp, hipStream_t s) {
-    return f32_tiles<false, true>(w, gate_inp, x, ntok, hidden, n_expert, logits, n_expert + 1u, xh, xl, xexp, s);
+    return f32_tiles<false>(w, gate_inp, x, ntok, hidden, n_expert, logits, n_expert + 1u, xh, xl, xexp, s);
 }
 
 }  // namespace redhip

@@ -27,7 +27,7 @@ def forward_and_check(m, ref, x, pick):
     assert max(rel_l2(got[t], want[i]) for i, t in agree) <= REL_L2_TOL
 
 
-@pytest.mark.parametrize("ntok", [41, 77, 301, 1025, 2047])      # tiles of 32 x 16, 32 x 32, 64 x 32 and 64 x 64, ragged
+@pytest.mark.parametrize("ntok", [41, 77, 301, 1025, 2047])      # tiles of 32 x 16, 32 x 32 and 64 x 32, ragged
 def test_dense_products_of_a_chunk(ntok):
     cfg = synth.layer_config(hidden=512, ffn=256, n_expert=512, top_k=4, layout="f2")
     lay = synth.make_layer(95, cfg)

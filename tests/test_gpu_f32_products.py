@@ -1,0 +1,70 @@
+"""The f32 products of a chunk on the bf16 matrix units (three terms for each f32): every tile they are cut into, activations at any float of
+memory and of any scale, and infinities, against sums in double."""
+import numpy as np
+import pytest
+
+from dwarfstar_red_lite_amd import synth
+from dwarfstar_red_lite_amd.moe import ResidentMoe
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+# of the rms of a token's outputs: 0.94e-7 was measured over 3000 outputs of 2048 columns (six chains of at most eight additions, each rounded to
+# 2^-25 of a partial sum, and the result's own 2^-25); one token's 48 outputs spread by a third around that
+TOL = 2e-7
+
+
+def layer(hidden, n_expert, **kw):
+    cfg = synth.layer_config(hidden=hidden, ffn=256, n_expert=n_expert, top_k=2, layout="iq2", **kw)
+    lay = synth.make_layer(41, cfg)
+    m = ResidentMoe(cfg, n_layer=1, max_tokens=2100)
+    m.load_layer(0, lay)
+    return m, np.frombuffer(np.ascontiguousarray(lay["router"]).tobytes(), np.float32).reshape(n_expert, hidden)
+
+
+def check(logits, x, rows):
+    want = x.astype(np.float64) @ rows.T.astype(np.float64)
+    err = np.sqrt(((logits - want) ** 2).mean(axis=1) / (want ** 2).mean(axis=1))
+    assert err.max() <= TOL, err.max()
+
+
+# 16 rows of 32 x 16, 300 experts' rows (a ragged last block) and tiles of every size: up to 77, 512 and 2048 tokens
+@pytest.mark.parametrize("hidden,n_expert,tokens", [(512, 16, (41, 47)), (1024, 300, (77, 513)), (2048, 512, (40, 77, 512, 2047)), (1536, 48, (49,))])
+def test_logits(hidden, n_expert, tokens):
+    m, rows = layer(hidden, n_expert)
+    for n in tokens:
+        x = synth.normed_x(np.random.default_rng(n), n, hidden)
+        x *= np.float32(10.0) ** np.random.default_rng(1).integers(-28, 29, size=(n, 1)).astype(np.float32)      # a scale per token
+        check(m.route(0, torch.from_numpy(x).cuda())[2].cpu().numpy(), x, rows)
+    m.close()
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_activations_at_any_float(shift):
+    m, rows = layer(1024, 48)
+    n = 45
+    x = synth.normed_x(np.random.default_rng(3), n, 1024)
+    room = torch.zeros(n * 1024 + 4, device="cuda")
+    room[shift:shift + n * 1024] = torch.from_numpy(x).cuda().reshape(-1)
+    aligned = m.route(0, torch.from_numpy(x).cuda())[2].cpu().numpy()
+    got = m.route(0, room[shift:shift + n * 1024].reshape(n, 1024))[2].cpu().numpy()
+    assert np.array_equal(got, aligned)
+    check(got, x, rows)
+    m.close()
+
+
+def test_infinities_and_overflow():
+    m, rows = layer(512, 64)
+    n = 44
+    x = synth.normed_x(np.random.default_rng(4), n, 512)
+    plain = m.route(0, torch.from_numpy(x).cuda())[2].cpu().numpy()
+    y = x.copy()
+    y[3, 100], y[20, 7], y[20, 300], y[43, 11], y[30, 0] = np.inf, 3e38, -np.inf, np.nan, 3.4e38
+    got = m.route(0, torch.from_numpy(y).cuda())[2].cpu().numpy()
+    ok = [t for t in range(n) if t not in (3, 20, 43, 30)]
+    assert np.array_equal(got[ok], plain[ok])
+    assert np.array_equal(got[3], np.where(rows[:, 100] > 0, np.inf, -np.inf).astype(np.float32)) and (rows[:, 100] != 0).all()
+    assert np.array_equal(got[20], np.where(rows[:, 300] > 0, -np.inf, np.inf).astype(np.float32)) and (rows[:, 300] != 0).all()
+    assert np.isnan(got[43]).all()
+    check(got[30:31], y[30:31], rows)
+    m.close()

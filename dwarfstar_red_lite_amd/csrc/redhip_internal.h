@@ -187,6 +187,10 @@ hipError_t launch_batch_combine(const float *tmp, const float *pair_weight, cons
 hipError_t launch_f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out,
                             uint32_t out_stride, void *xh, void *xl, int *xexp, hipStream_t s);
 hipError_t launch_f32_swiglu_tiles(const float *w, const float *x, uint32_t ntok, uint32_t K, uint32_t ffn, float *act, hipStream_t s);
+// the shared expert's gate, up and SwiGLU of a small chunk, its router (n_expert > 0) or gate factor (scalar) and the fp16 halves in one launch
+bool front_tiles_fit(uint32_t ntok, uint32_t ffn, uint32_t n_expert);
+hipError_t launch_front_tiles(const float *gate_up, const float *router, const float *gate_inp, const float *x, uint32_t ntok, uint32_t hidden, uint32_t ffn, uint32_t n_expert,
+                              float *act, float *logits, float *scalar, void *xh, void *xl, int *xexp, hipStream_t s);
 hipError_t launch_router_f32_tiles(const float *w, const float *gate_inp, const float *x, uint32_t ntok, uint32_t hidden, uint32_t n_expert,
                                    float *logits, void *xh, void *xl, int *xexp, hipStream_t s);
 // entries of a tile list of a chunk, at most

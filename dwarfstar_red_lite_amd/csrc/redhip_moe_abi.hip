@@ -96,7 +96,7 @@ struct Moe {
     // larger chunks take the router as a tiled f32 product (a quantised router through its f32 copy)
     // (below 40 tokens the f32 rows are quicker one token per grid layer where a router is small: 33 tokens of 1024 x 96 experts 2.4 us, of 2048 x 128
     // experts 4.6 us; 512 experts' tiles would be 3 us ahead from 36 tokens on)
-    bool tiled_router(uint32_t ntok) const { return packed_gu() && ntok >= 40u && (cfg.router_type == T_F32 || mixed); }
+    bool tiled_router(uint32_t ntok) const { return packed_gu() && (ntok >= 40u || shared_in_front(ntok, true)) && (cfg.router_type == T_F32 || mixed); }
     uint64_t tiled_stride() const { return fused ? expert_stride : packed_stride; }      // bytes between experts in `tiled`
     bool tiles_resident() const { return packed_gu() && gu_type == T_IQ2_XXS && cfg.max_tokens > 8u && cfg.ffn <= 512u && cfg.hidden / 512u <= 4u; }
     uint64_t words_down_stride() const {
@@ -207,6 +207,14 @@ struct Moe {
         if (fused) return rowmajor_down() && staged_gateup_supported(gu_type, RowLayout::rows, cfg.hidden, cfg.ffn) && staged_down_supported(dn_type, RowLayout::rows, cfg.hidden, cfg.ffn);
         return keep_raw() && staged_gateup_supported(gu_type, RowLayout::raw, cfg.hidden, cfg.ffn) && staged_down_supported(dn_type, RowLayout::raw, cfg.hidden, cfg.ffn);
     }
+    // a chunk on a mixed layout so small that its shared expert's gate/up products ride in the launch in front of its routing (own router) or of its
+    // pair sort (routing given), and its down products follow the routed ones, instead of both on a stream of their own
+    bool shared_in_front(uint32_t ntok, bool own_router) const {
+        return mixed && side && tile_chunk(ntok) && !sliced(ntok) && !small_batch(ntok) && !(small_batch(ntok, true) && (own_router || ntok <= slices_up_to(false))) &&
+               front_tiles_fit(ntok, cfg.ffn, own_router ? cfg.n_expert : 0u);
+    }
+    bool shared_act_ready = false;           // this call's front launch left the shared expert's activations in sh_act
+    bool ahead_of_experts = false;           // route() is part of a forward pass
     // a chunk on a mixed layout that has no tile kernels at all runs as slices of 8 tokens on the grouped small-batch kernels, far ahead of
     // the generic per-pair kernels on raw rows
     static constexpr uint32_t kSlice = 8u;
@@ -329,8 +337,8 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
         // the many-workgroup sort of a large chunk then queues behind the dense tiles - 73 against 22 us at 2048 tokens - but started
         // behind the sort the dense products slow the down tiles by more: 787 against 760 us per chunk, both with products on the fp32 units)
         const bool tile_path = !m->small_batch(ntok) && !(m->small_batch(ntok, true) && grouped) && m->tile_chunk(ntok);
-        const bool dense_shared = tile_path && m->mixed && Ld.dense_gu && m->side;
-        if (dense_shared && !fork_shared_dense(m, Ld, x, ntok, s)) return 0;
+        const bool dense_shared = tile_path && m->mixed && Ld.dense_gu && m->side, in_line = dense_shared && m->shared_act_ready;
+        if (dense_shared && !in_line && !fork_shared_dense(m, Ld, x, ntok, s)) return 0;
         // the pair sort also writes the tile lists of the tile kernels that follow (all-IQ2_XXS layers: with the shared expert's tiles)
         const TileLists tl{m->tile_expert, m->tile_pair0, m->tile_n, m->n_tiles, prefill_tile_bound(ntok, c.top_k, c.n_expert), m->fused ? ntok : 0u};
         if (!grouped) {
@@ -368,7 +376,9 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
             else if (!raw_rows(m, layer)) return 0;
             else HIP_OK(launch_batch_down(ex, m->uid, m->expert_start, m->n_unique, n_groups, P, c.hidden, c.ffn, m->act, m->tmp, s), "batched down launch");
             prof_set_stage(ST_BATCH_DOWN);
-            if (dense_shared) {
+            if (in_line) {
+                HIP_OK(launch_f32_tiles(Ld.dense_down, nullptr, m->sh_act, ntok, c.ffn, c.hidden, m->sh_tmp, c.hidden, nullptr, nullptr, nullptr, s), "shared down tiles");
+            } else if (dense_shared) {
                 if (!join_shared_dense(m, s)) return 0;
             } else if (!m->fused) {
                 HIP_OK(launch_batch_gateup(sh, nullptr, nullptr, nullptr, nullptr, 1u, ntok, c.hidden, c.ffn, x, m->sh_act, s), "batched shared gate/up launch");
@@ -858,6 +868,10 @@ int redhip_moe_route(redhip_moe_t h, uint32_t layer, const float *x_dev, uint32_
             }
             bc = saved;
             m->shared_gu_ready = true;
+        } else if (m->ahead_of_experts && m->shared_in_front(ntok, true) && router_f32 && m->layers[layer].dense_gu) {
+            HIP_OK(launch_front_tiles(m->layers[layer].dense_gu, router_f32, m->layers[layer].gate_inp, x_dev, ntok, c.hidden, c.ffn, c.n_expert, m->sh_act, m->logits, nullptr,
+                                      m->xh, m->xl, m->xexp, s), "router and shared gate/up launch");
+            m->shared_act_ready = true;
         } else if (m->tiled_router(ntok))
             HIP_OK(launch_router_f32_tiles(router_f32, m->layers[layer].gate_inp, x_dev, ntok, c.hidden,
                                            c.n_expert, m->logits, m->xh, m->xl, m->xexp, s), "router tile launch");
@@ -940,6 +954,11 @@ int redhip_moe_experts(redhip_moe_t h, uint32_t layer, const float *x_dev, uint3
             HIP_OK(launch_router_gemv(T_F32, L.dense_gu, x_dev, L.gate_inp, ntok, m->cfg.hidden, 0u, m->logits, m->xh, m->xl, m->xexp, nullptr, m->act,
                                       m->cfg.ffn, s, L.dense_gu, m->scalar, to_group ? &job : nullptr, &grouped), "shared gate/up launch");
             m->shared_gu_ready = true;
+        } else if (m->shared_in_front(ntok, false) && L.dense_gu) {
+            prof_set_stage(ST_SHARED_GATEUP);
+            HIP_OK(launch_front_tiles(L.dense_gu, nullptr, L.gate_inp, x_dev, ntok, m->cfg.hidden, m->cfg.ffn, 0u, m->sh_act, nullptr, m->scalar, m->xh, m->xl, m->xexp, s),
+                   "shared gate/up launch");
+            m->shared_act_ready = true;
         } else {
             prof_set_stage(ST_OTHER);
             HIP_OK(launch_prep(x_dev, L.gate_inp, ntok, m->cfg.hidden, m->xh, m->xl, m->xexp, m->scalar, s, to_group ? &job : nullptr, &grouped), "prep launch");
@@ -953,7 +972,7 @@ int redhip_moe_experts(redhip_moe_t h, uint32_t layer, const float *x_dev, uint3
             grouped = true;
         }
         const int ok = experts_enqueue(m, layer, x_dev, ntok, ids_dev, weights_dev, out_dev, s, false, grouped);
-        m->shared_gu_ready = false;
+        m->shared_gu_ready = m->shared_act_ready = false;
         return ok;
     }
     scalar_gate_kernel<<<ntok, 256, 0, s>>>(m->layers[layer].gate_inp, x_dev, m->cfg.hidden, m->scalar);
@@ -978,11 +997,14 @@ int redhip_moe_forward(redhip_moe_t h, uint32_t layer, const float *x_dev, uint3
     const bool group_in_select = m->group_in_select(ntok);
     const bool select_in_gateup = m->packed_gu() && (ntok == 1u || m->small_batch_mixed(ntok)) && !group_in_select;
     m->skip_select = select_in_gateup || group_in_select;      // small batches: the batched gate/up kernel selects and sorts the pairs itself
+    m->ahead_of_experts = true;
     const int routed = redhip_moe_route(h, layer, x_dev, ntok, nullptr, nullptr, nullptr, stream);
-    m->skip_select = false;
-    if (!routed) return 0;
+    m->skip_select = m->ahead_of_experts = false;
+    if (!routed) { m->shared_act_ready = false; return 0; }
     if (m->slices_after_router(ntok)) return select_group_slices(m, layer, x_dev, ntok, out_dev, static_cast<hipStream_t>(stream));
-    return experts_enqueue(m, layer, x_dev, ntok, m->ids, m->weights, out_dev, static_cast<hipStream_t>(stream), select_in_gateup || group_in_select, group_in_select);
+    const int ok = experts_enqueue(m, layer, x_dev, ntok, m->ids, m->weights, out_dev, static_cast<hipStream_t>(stream), select_in_gateup || group_in_select, group_in_select);
+    m->shared_act_ready = false;
+    return ok;
 }
 
 int redhip_moe_forward_block(redhip_moe_t h, uint32_t layer, const float *x_dev, const float *branch_dev, const float *post_norm_dev, float eps,
@@ -1021,16 +1043,18 @@ int redhip_moe_forward_block(redhip_moe_t h, uint32_t layer, const float *x_dev,
         const bool select_in_gateup = m->packed_gu() && (ntok == 1u || m->small_batch_mixed(ntok)) && !group_in_select;
         m->skip_select = select_in_gateup || group_in_select;
         if (in_router) { bc.branch = branch_dev; bc.norm_w = post_norm_dev; bc.eps = eps; bc.xn_out = m->xn; }
+        m->ahead_of_experts = true;
         ok = redhip_moe_route(h, layer, in_router ? x_dev : m->xn, ntok, nullptr, nullptr, nullptr, stream);
         bc.branch = bc.norm_w = nullptr;
         bc.xn_out = nullptr;
-        m->skip_select = false;
+        m->skip_select = m->ahead_of_experts = false;
             if (ok) {
             bc.resid_a = x_dev;                              // the path's last kernel adds x + branch to its output
             bc.resid_b = branch_dev;
             ok = m->slices_after_router(ntok) ? select_group_slices(m, layer, m->xn, ntok, x_out_dev, s)
                                       : experts_enqueue(m, layer, m->xn, ntok, m->ids, m->weights, x_out_dev, s, select_in_gateup || group_in_select, group_in_select);
         }
+        m->shared_act_ready = false;
     }
     bc = BlockContext{};
     return ok;

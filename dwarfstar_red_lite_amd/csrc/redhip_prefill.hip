@@ -122,7 +122,7 @@ hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count
 // with gate_inp, if there is one, as row n_rows; without xh the tiles have it as a further row.
 
 __device__ __forceinline__ void split_token(const float *gate_inp, const float *x, float *logits, uint32_t out_stride, _Float16 *xh, _Float16 *xl, int *xexp, uint32_t H,
-                                            uint32_t E, uint32_t tok, uint32_t lane) {
+                                            uint32_t E, uint32_t tok, uint32_t lane, float *scalar = nullptr) {
             // the vector as float4 per lane, eight requested at a time (2048 elements per pass: one round trip for the usual widths)
             const float4 *xt = reinterpret_cast<const float4 *>(x + (uint64_t)tok * H), *gv = reinterpret_cast<const float4 *>(gate_inp);
             const uint32_t H4 = H / 4u;
@@ -163,7 +163,8 @@ __device__ __forceinline__ void split_token(const float *gate_inp, const float *
             }
             if (lane == 0u) {
                 xexp[tok] = e;
-                if (gate_inp) logits[(uint64_t)tok * out_stride + E] = gate;
+                if (scalar) scalar[tok] = 1.0f / (1.0f + expf(-gate));
+                else if (gate_inp) logits[(uint64_t)tok * out_stride + E] = gate;
             }
 }
 
@@ -186,29 +187,42 @@ __device__ __forceinline__ ThreeTerms three_terms(float4_t a, float4_t b, uint32
     return ThreeTerms{__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
 
-template <int MR, int MT, bool SWIGLU>
+// what a kernel of both kinds multiplies beside its gate and up rows: a router (n_rows may be 0); `scalar`: the shared expert's gate factor instead of row n_rows
+struct RouterRows { const float *w; float *out, *scalar; uint32_t n_rows, out_stride; };
+enum F32Kind { F32_PLAIN, F32_SWIGLU, F32_BOTH };
+template <F32Kind KIND> struct Beside {};
+template <> struct Beside<F32_BOTH> : RouterRows {};
+
+template <int MR, int MT, F32Kind KIND>
 __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const float *gate_inp, const float *x, float *out, uint32_t out_stride, _Float16 *xh,
-                                                        _Float16 *xl, int *xexp, uint32_t K, uint32_t n_rows, uint32_t ntok) {
+                                                        _Float16 *xl, int *xexp, uint32_t K, uint32_t n_rows, uint32_t ntok, Beside<KIND> router) {
     constexpr uint32_t BR = 16u * MR, BT = 16u * MT, NB = MR + MT, PIECES = 2u * NB > MR * MT ? 2u * NB : MR * MT;      // KB per wave: 32 columns of the rows and tokens, later its sums
     __shared__ __attribute__((aligned(16))) float4_t lds[8][PIECES][64];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t all_rows = n_rows + (gate_inp && !xh ? 1u : 0u), row_tiles = (all_rows + BR - 1u) / BR, tok_tiles = (ntok + BT - 1u) / BT, n_tile = row_tiles * tok_tiles;
-    if (blockIdx.x >= n_tile) {
-        const uint32_t tok = 8u * (blockIdx.x - n_tile) + wave;
-        if (tok < ntok) split_token(gate_inp, x, out, out_stride, xh, xl, xexp, K, n_rows, tok, lane);
+    const uint32_t tok_tiles = (ntok + BT - 1u) / BT, first = KIND == F32_BOTH ? n_rows / BR * tok_tiles : 0u;      // tiles of gate and up rows in front of the router's
+    const bool swiglu = KIND == F32_SWIGLU || (KIND == F32_BOTH && blockIdx.x < first);
+    uint32_t tile = blockIdx.x;
+    if constexpr (KIND == F32_BOTH)
+        if (!swiglu) { tile -= first; w = router.w; n_rows = router.n_rows; out = router.out; out_stride = router.out_stride; }
+    const uint32_t all_rows = n_rows + (gate_inp && !xh ? 1u : 0u), row_tiles = (all_rows + BR - 1u) / BR;
+    if (tile >= row_tiles * tok_tiles) {
+        const uint32_t tok = 8u * (tile - row_tiles * tok_tiles) + wave;
+        float *scalar = nullptr;
+        if constexpr (KIND == F32_BOTH) scalar = router.scalar;
+        if (tok < ntok) split_token(gate_inp, x, out, out_stride, xh, xl, xexp, K, n_rows, tok, lane, scalar);
         return;
     }
     // Workgroups are dealt to the eight XCDs in turn, each with its own L2: workgroup i lands on XCD i % 8. The tiles of one XCD form a
     // compact block of the tile grid (a quarter of the row tiles x half of the token tiles), so that an XCD fetches a quarter of the
     // matrix and half of the activations instead of all of both. (A different dealing order would only cost this locality.)
-    uint32_t tile_r = blockIdx.x % row_tiles, tile_t = blockIdx.x / row_tiles;
+    uint32_t tile_r = tile % row_tiles, tile_t = tile / row_tiles;
     if (row_tiles % 4u == 0u && tok_tiles % 2u == 0u) {
-        const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3, br = row_tiles / 4u, bt = tok_tiles / 2u;
+        const uint32_t xcd = tile & 7u, slot = tile >> 3, br = row_tiles / 4u, bt = tok_tiles / 2u;
         tile_r = (xcd & 3u) * br + slot % br;
         tile_t = (xcd >> 2) * bt + slot / br;
     }
     // row block m of the tile starts here; rows and tokens beyond the last repeat another and are not stored
-    const auto block_row = [&](uint32_t m) { return SWIGLU ? (m < MR / 2u ? 0u : n_rows / 2u) + tile_r * (BR / 2u) + 16u * (m % (MR / 2u)) : tile_r * BR + 16u * m; };
+    const auto block_row = [&](uint32_t m) { return swiglu ? (m < MR / 2u ? 0u : n_rows / 2u) + tile_r * (BR / 2u) + 16u * (m % (MR / 2u)) : tile_r * BR + 16u * m; };
     const auto matrix_row = [&](uint32_t row) { return row < n_rows ? w + (uint64_t)row * K : gate_inp ? gate_inp : w; };
     // fetch i of a wave: eight rows (or tokens) of 128 bytes; lane l brings piece (l % 8) ^ (row % 16 / 2) of row l / 8
     const float *src[2u * NB];
@@ -233,7 +247,7 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
             }
         }
     };
-    constexpr int CH = SWIGLU ? 1 : 2;
+    constexpr int CH = KIND == F32_PLAIN ? 2 : 1;
     float4_t high[CH][MR][MT], low[MR][MT];
     double total[MR][MT][4];
 #pragma unroll
@@ -288,7 +302,7 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
     for (uint32_t step = 0; step < steps; step += 2u) {
         multiply(step, std::integral_constant<int, 0>{});
         if (step + 1u < steps) multiply(step + 1u, std::integral_constant<int, CH - 1>{});
-        if constexpr (SWIGLU) flush();
+        if constexpr (KIND != F32_PLAIN) flush();
     }
     __syncthreads();
 #pragma unroll
@@ -297,12 +311,12 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
         for (int t = 0; t < MT; ++t) {
             float4_t v;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = SWIGLU ? (float)(total[m][t][i] + low[m][t][i]) : high[0][m][t][i] + high[CH - 1][m][t][i] + low[m][t][i];
+            for (int i = 0; i < 4; ++i) v[i] = KIND != F32_PLAIN ? (float)(total[m][t][i] + low[m][t][i]) : high[0][m][t][i] + high[CH - 1][m][t][i] + low[m][t][i];
             (&lds[0][0][0])[(wave * MR * MT + m * MT + t) * 64u + lane] = v;
         }
     __syncthreads();
     // a thread: four consecutive rows of a token (D[i = 4q .. 4q + 3][j = r])
-    for (uint32_t o = tid; o < (SWIGLU ? MR / 2u : MR) * MT * 64u; o += 512u) {
+    for (uint32_t o = tid; o < (swiglu ? MR / 2u : MR) * MT * 64u; o += 512u) {
         const uint32_t t = (o >> 6) % MT, m = (o >> 6) / MT, l = o & 63u, tok = tile_t * BT + 16u * t + (l & 15u), row = 4u * (l >> 4);
         if (tok >= ntok) continue;
         const auto products = [&](uint32_t mm) {
@@ -327,7 +341,7 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
             return y;
         };
         float4_t y = products(m);
-        if constexpr (SWIGLU) {
+        if (swiglu) {
             const float4_t u = products(m + MR / 2u);
 #pragma unroll
             for (int i = 0; i < 4; ++i) y[i] = (y[i] / (1.0f + expf(-y[i]))) * u[i];
@@ -343,10 +357,10 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
 // The tile that costs least: rounds of the device (256 compute units) times what a round of workgroups of it takes, 18, 10 and 7 us for 2048
 // columns of 64 x 32, 32 x 32 and 32 x 16 outputs (gate/up of 512 tokens 19.7 / 23.4 / 26.4 us, of 77 tokens 16.2 / 10.8 / 7.9, down of 77 tokens, 512
 // columns, 6.7 / 4.7 / 5.1, router of 512 tokens 16.9 / 11.8 / 14.2).
-template <bool SWIGLU>
+template <F32Kind KIND>
 hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out, uint32_t out_stride, void *xh, void *xl,
                      int *xexp, hipStream_t s) {
-    if (!ntok || !K || K % 256u || !n_rows || !w || !x || !out || (SWIGLU && n_rows % 128u)) return hipErrorInvalidValue;
+    if (!ntok || !K || K % 256u || !n_rows || !w || !x || !out || (KIND == F32_SWIGLU && n_rows % 128u)) return hipErrorInvalidValue;
     const uint32_t all_rows = n_rows + (extra_row && !xh ? 1u : 0u);
     static constexpr struct { uint32_t br, bt, round; } kTiles[3] = {{64u, 32u, 18u}, {32u, 32u, 10u}, {32u, 16u, 7u}};
     uint64_t n[3], best = ~0ull;
@@ -360,9 +374,9 @@ hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uin
     if (n[pick] + split_wgs > 0x7fffffffull) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)n[pick] + split_wgs), block(512u);
     _Float16 *h = static_cast<_Float16 *>(xh), *l = static_cast<_Float16 *>(xl);
-    if (pick == 0) REDHIP_LAUNCH((f32_tiles_kernel<4, 2, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
-    else if (pick == 1) REDHIP_LAUNCH((f32_tiles_kernel<2, 2, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
-    else REDHIP_LAUNCH((f32_tiles_kernel<2, 1, SWIGLU>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok);
+    if (pick == 0) REDHIP_LAUNCH((f32_tiles_kernel<4, 2, KIND>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok, Beside<KIND>{});
+    else if (pick == 1) REDHIP_LAUNCH((f32_tiles_kernel<2, 2, KIND>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok, Beside<KIND>{});
+    else REDHIP_LAUNCH((f32_tiles_kernel<2, 1, KIND>), grid, block, 0, s, w, extra_row, x, out, out_stride, h, l, xexp, K, n_rows, ntok, Beside<KIND>{});
     return hipGetLastError();
 }
 
@@ -370,16 +384,36 @@ hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uin
 // row behind the matrix; xh / xl / xexp (optional): also write the fp16 halves of x
 hipError_t launch_f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out,
                             uint32_t out_stride, void *xh, void *xl, int *xexp, hipStream_t s) {
-    return f32_tiles<false>(w, extra_row, x, ntok, K, n_rows, out, out_stride, xh, xl, xexp, s);
+    return f32_tiles<F32_PLAIN>(w, extra_row, x, ntok, K, n_rows, out, out_stride, xh, xl, xexp, s);
 }
 // act[tok][c] = silu(W[c] . x[tok]) * (W[ffn + c] . x[tok])
 hipError_t launch_f32_swiglu_tiles(const float *w, const float *x, uint32_t ntok, uint32_t K, uint32_t ffn, float *act, hipStream_t s) {
-    return f32_tiles<true>(w, nullptr, x, ntok, K, 2u * ffn, act, ffn, nullptr, nullptr, nullptr, s);
+    return f32_tiles<F32_SWIGLU>(w, nullptr, x, ntok, K, 2u * ffn, act, ffn, nullptr, nullptr, nullptr, s);
 }
 
 hipError_t launch_router_f32_tiles(const float *w, const float *gate_inp, const float *x, uint32_t ntok, uint32_t hidden, uint32_t n_expert,
                                    float *logits, void *xh, void *xl, int *xexp, hipStream_t s) {
-    return f32_tiles<false>(w, gate_inp, x, ntok, hidden, n_expert, logits, n_expert + 1u, xh, xl, xexp, s);
+    return f32_tiles<F32_PLAIN>(w, gate_inp, x, ntok, hidden, n_expert, logits, n_expert + 1u, xh, xl, xexp, s);
+}
+
+// The shared expert of a small chunk as part of the launch that precedes its routing: act = silu(gate) * up as launch_f32_swiglu_tiles, the router's
+// logits (none with n_expert = 0: then the gate's factor goes to scalar) and the fp16 halves of the activations, in tiles of 32 x 16. Where they are less
+// than two rounds of the device the launch takes hardly longer than the router alone, while the same products on a stream of their own cost the chunk
+// 15 us, most of it the fork and the join. Us per layer on the other stream -> here: IQ1_M, 2048 x 512, 28 tokens 113 -> 100, 77 tokens 164 -> 155;
+// IQ3_S down 33 tokens 129 -> 115, 100 tokens (349 workgroups) 177 -> 175, IQ2_XS 160 tokens (500) 226 -> 227; 2048 x 768, 120 tokens (431) 152 -> 145;
+// 1024 x 256, 33 tokens 64 -> 51, 300 tokens (399) 77 -> 72. With the routing given the launch that splits the activations is shorter than a router:
+// IQ1_M 30 tokens 104 -> 97, IQ2_XS 110 tokens (238 workgroups) 199 -> 197, IQ3_S 200 tokens (441) 202 -> 206.
+bool front_tiles_fit(uint32_t ntok, uint32_t ffn, uint32_t n_expert) {
+    return ffn % 64u == 0u && (uint64_t)(ffn / 16u + (n_expert + 31u) / 32u) * ((ntok + 15u) / 16u) + (ntok + 7u) / 8u <= (n_expert ? 448u : 256u);
+}
+hipError_t launch_front_tiles(const float *gate_up, const float *router, const float *gate_inp, const float *x, uint32_t ntok, uint32_t hidden, uint32_t ffn, uint32_t n_expert,
+                              float *act, float *logits, float *scalar, void *xh, void *xl, int *xexp, hipStream_t s) {
+    if (!ntok || !hidden || hidden % 256u || !front_tiles_fit(ntok, ffn, n_expert) || !gate_up || !gate_inp || !x || !act || !xh || !xl || !xexp || (n_expert ? !router || !logits : !scalar))
+        return hipErrorInvalidValue;
+    const dim3 grid((ffn / 16u + (n_expert + 31u) / 32u) * ((ntok + 15u) / 16u) + (ntok + 7u) / 8u);
+    REDHIP_LAUNCH((f32_tiles_kernel<2, 1, F32_BOTH>), grid, dim3(512), 0, s, gate_up, gate_inp, x, act, ffn, static_cast<_Float16 *>(xh), static_cast<_Float16 *>(xl), xexp, hidden,
+                  2u * ffn, ntok, Beside<F32_BOTH>{{router, logits, n_expert ? nullptr : scalar, n_expert, n_expert + 1u}});
+    return hipGetLastError();
 }
 
 }  // namespace redhip

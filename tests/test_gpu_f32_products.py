@@ -68,3 +68,30 @@ def test_infinities_and_overflow():
     assert np.isnan(got[43]).all()
     check(got[30:31], y[30:31], rows)
     m.close()
+
+
+def test_shared_expert_in_front_and_beside(golden_dir):
+    """gate and up products of the shared expert in the launch in front of the routing (up to 448 workgroups: 352 tokens here) or of a given routing
+    (256: 224 tokens), and on a stream of their own beyond: a token gets the same from either"""
+    import oracle_lib as orc
+    from gpu_common import REL_L2_TOL, rel_l2
+    cfg = synth.layer_config(hidden=512, ffn=256, n_expert=64, top_k=4, layout="f2")
+    lay = synth.make_layer(43, cfg)
+    m = ResidentMoe(cfg, n_layer=1, max_tokens=400)
+    m.load_layer(0, lay)
+    x = synth.normed_x(np.random.default_rng(5), 400, 512)
+    x_dev = torch.from_numpy(x).cuda()
+    whole = m.forward(0, x_dev).cpu().numpy()
+    ids, w, _ = m.last_route(400)
+    pick = [0, 7, 32, 33, 39]
+    want, cids, _, _ = orc.Layer(cfg, **lay).forward(np.ascontiguousarray(x[pick]), threads=8)
+    same = [i for i, t in enumerate(pick) if np.array_equal(ids[t], cids[i])]
+    assert len(same) >= len(pick) - 1 and max(rel_l2(whole[pick[i]], want[i]) for i in same) <= REL_L2_TOL
+    ids_dev, w_dev = torch.from_numpy(ids.astype(np.int32)).cuda(), torch.from_numpy(w).cuda()
+    for n in (40, 225, 352, 353, 368, 384):
+        got = m.forward(0, x_dev[:n]).cpu().numpy()
+        assert max(rel_l2(got[t], whole[t]) for t in range(n)) <= 1e-6, n
+    for n in (33, 208, 224, 225, 240):
+        got = m.experts(0, x_dev[:n], ids_dev[:n].contiguous(), w_dev[:n].contiguous()).cpu().numpy()
+        assert max(rel_l2(got[t], whole[t]) for t in range(n)) <= 1e-6, n
+    m.close()

@@ -141,18 +141,30 @@ struct Moe {
     // workgroup of the launch that splits the activations, up to 256 pairs)
     static constexpr uint32_t kSmallMaxFused = 16u, kSmallMaxRouted = 32u, kSmallMaxGiven = 24u, kSmallMaxMixed = 32u;
     // ... unless the tiles are ahead from fewer tokens on. The slices cost a pass per two pairs of an expert, the tiles a decode per distinct expert,
-    // so the line lies lower where a unit of the tiles' decode is cheap (IQ2_XXS everywhere, IQ1_M everywhere) and the experts are large
-    // enough to fill their launches; a call with given routing does not know how it is spread. Slices / tiles, us per layer of 2048 x 512, 512 experts, ten a token:
-    //   own router: IQ2_XXS 20, 24, 28, 32 tokens 85 / 86, 97 / 94, 109 / 102, 121 / 110; IQ1_M 24, 26, 28, 32: 108 / 111, 116 / 114, 120 / 117, 134 / 123;
-    //     IQ3_S down 28, 32: 121 / 127, 134 / 128; IQ2_XS 28, 32: 129 / 136, 142 / 147
-    //   given, evenly / with Zipf popularity / on 32 hot experts: IQ2_XXS 18 tokens 69 / 72, 61 / 58, 58 / 51, 20: 75 / 75, 67 / 59, 63 / 53; IQ1_M 22:
-    //     96 / 98, 87 / 81, 82 / 72, 24: 102 / 100, 91 / 84, 86 / 75; IQ3_S down 24: 105 / 108, 94 / 89, 87 / 80; IQ2_XS 24: 109 / 117, 97 / 100, 92 / 84
-    // IQ2_XXS layers of 2048 x 768, 128 experts, eight a token: own router 18, 24 tokens 78 / 81, 95 / 87; evenly given 18, 24: 73 / 73, 88 / 80. Of 1024 x
-    // 512 and less the slices stay ahead (32 tokens of 1024 x 512: 65 / 65).
+    // so the line lies lower the cheaper a unit of the tiles' decode is and the larger the experts, which have to fill the tiles' launches; a call
+    // with given routing does not know how it is spread. Slices / tiles, us per layer:
+    // 2048 x 512, 512 experts, ten a token, behind the own router:
+    //   IQ2_XXS 20, 24, 28, 32 tokens 85 / 86, 97 / 94, 109 / 102, 121 / 110; IQ1_M 18, 24: 89 / 85, 108 / 95; IQ3_S down 18, 20, 24: 90 / 92, 97 / 96,
+    //   108 / 102; IQ2_XS 20, 24, 28: 101 / 106, 116 / 114, 130 / 121
+    // given, evenly / on 32 hot experts:
+    //   IQ2_XXS 18, 20: 69 / 72 and 58 / 51, 75 / 75 and 63 / 53; IQ1_M 18: 84 / 80 and 71 / 61; IQ3_S down 18, 20: 86 / 89 and 71 / 63, 93 / 92 and
+    //   77 / 67; IQ2_XS 20, 22, 24: 97 / 99 and 81 / 71, 103 / 103 and 87 / 73, 109 / 106 and 93 / 74
+    // 1024 x 512, 200 experts, eight a token, own router: IQ1_M 24, 32: 61 / 62, 75 / 66; IQ3_S down 60 / 66, 75 / 67; IQ2_XS 63 / 69, 78 / 74; IQ2_XXS
+    //   32: 65 / 65; given 18, 24: IQ1_M 47 / 52 and 44 / 47, 56 / 54 and 52 / 48; IQ3_S down 24: 57 / 58 and 51 / 50; IQ2_XS 58 / 59 and 54 / 52
+    // 2048 x 768 (IQ2_XXS, 128 experts, eight a token): own router 18, 24: 78 / 81, 95 / 87; evenly given 73 / 73, 88 / 80
+    // 1024 x 256, 96 experts, six a token, own router 24, 32: IQ1_M 41 / 47, 49 / 48; IQ3_S down 40 / 50, 48 / 51; IQ2_XS 41 / 51, 50 / 52: the slices
     uint32_t slices_up_to(bool own_router) const {
-        if ((size_t)cfg.hidden * cfg.ffn >= (size_t)2048u * 512u) {
-            if (fused && tile_chunk(kSmallMaxRouted)) return own_router ? 22u : 19u;
-            if (gu_type == T_IQ1_M && stream_tiles_resident()) return own_router ? 25u : 22u;
+        const size_t weights = (size_t)cfg.hidden * cfg.ffn;
+        if (weights >= (size_t)1024u * 512u && tile_chunk(kSmallMaxRouted)) {
+            const bool large = weights >= (size_t)2048u * 512u;
+            if (fused) {
+                if (large) return own_router ? 22u : 19u;
+            } else if (gu_type == T_IQ1_M)
+                return large ? 16u : own_router ? 25u : 22u;
+            else if (dn_type == T_IQ3_S)
+                return large ? 19u : own_router ? 28u : kSmallMaxGiven;
+            else
+                return large ? (own_router ? 23u : 22u) : own_router ? 30u : kSmallMaxGiven;
         }
         return own_router ? (fused ? kSmallMaxRouted : kSmallMaxMixed) : kSmallMaxGiven;
     }

@@ -1,5 +1,5 @@
-"""The sizes where batches of large experts leave the slices for the tile kernels (IQ2_XXS: 23 tokens behind the own router, 20 with the routing
-given; IQ1_M: 26 and 23), on both sides of each line, against the CPU path; a token gets the same from either."""
+"""The sizes where batches of large experts leave the slices for the tile kernels, on both sides of each line, against the CPU path; a token
+gets the same from either."""
 import json
 import os
 
@@ -17,9 +17,11 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
-@pytest.mark.parametrize("layout,shape,own,given", [("iq2", (2048, 512, 40, 10), 22, 19), ("iq2", (2048, 768, 24, 8), 22, 19), ("m", (2048, 512, 40, 10), 25, 22)])
+@pytest.mark.parametrize("layout,shape,own,given", [("iq2", (2048, 512, 40, 10), 22, 19), ("iq2", (2048, 768, 24, 8), 22, 19), ("m", (2048, 512, 40, 10), 16, 16),
+                                                    ("f2", (2048, 512, 40, 10), 19, 19), ("xs", (2048, 512, 40, 10), 23, 22), ("m", (1024, 512, 24, 8), 25, 22),
+                                                    ("f2", (1024, 512, 24, 8), 28, 24), ("xs", (1024, 512, 24, 8), 30, 24)])
 def test_both_sides_of_the_line(layout, shape, own, given, golden_dir):
-    if layout == "m":
+    if layout in ("m", "xs"):
         g = json.load(open(os.path.join(golden_dir, "iq_grids.json")))
         grids = [np.frombuffer(bytes.fromhex(g[k]), np.int8) for k in ("iq2_xs", "iq1_m")]
         moe_api.set_codebooks(*grids)

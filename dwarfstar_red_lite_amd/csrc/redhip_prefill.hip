@@ -171,18 +171,18 @@ __device__ __forceinline__ void split_token(const float *gate_inp, const float *
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t uint32x4_t __attribute__((ext_vector_type(4)));
 struct ThreeTerms { bf16x8 high, mid, low; };
-// `top` = 0xffff0000 in a vector register
-__device__ __forceinline__ ThreeTerms three_terms(float4_t a, float4_t b, uint32_t top) {
-    const auto cut = [&](float v) { return __uint_as_float(__float_as_uint(v) & top); };
+// `top` = 0xffff0000, `half` = 0x8000 in vector registers
+__device__ __forceinline__ ThreeTerms three_terms(float4_t a, float4_t b, uint32_t top, uint32_t half) {
+    const auto near = [&](float v) { return __uint_as_float((__float_as_uint(v) + half) & top); };      // (a NaN may lose its mark here; the last term keeps it)
     const auto tops = [](float v1, float v0) { return __builtin_amdgcn_perm(__float_as_uint(v1), __float_as_uint(v0), 0x07060302u); };
     uint32x4_t h, m, l;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float v0 = i < 2 ? a[2 * (i & 1)] : b[2 * (i & 1)], v1 = i < 2 ? a[2 * (i & 1) + 1] : b[2 * (i & 1) + 1];
-        const float r0 = v0 - cut(v0), r1 = v1 - cut(v1), s0 = r0 - cut(r0), s1 = r1 - cut(r1);      // (each exact)
-        h[i] = tops(v1, v0);
-        m[i] = tops(r1, r0);
-        l[i] = tops(s1, s0);
+        const float h0 = near(v0), h1 = near(v1), r0 = v0 - h0, r1 = v1 - h1, m0 = near(r0), m1 = near(r1);      // (each difference exact)
+        h[i] = tops(h1, h0);
+        m[i] = tops(m1, m0);
+        l[i] = tops(r1 - m1, r0 - m0);
     }
     return ThreeTerms{__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
 #pragma unroll
             for (int i = 0; i < 4; ++i) total[m][t][i] = 0.0;
         }
-    const uint32_t top = in_vector(0xffff0000u), at0 = 8u * r + (q ^ (r >> 1)), at1 = 8u * r + ((q + 4u) ^ (r >> 1)), steps = K / 256u;
+    const uint32_t top = in_vector(0xffff0000u), half = in_vector(0x8000u), at0 = 8u * r + (q ^ (r >> 1)), at1 = 8u * r + ((q + 4u) ^ (r >> 1)), steps = K / 256u;
     const auto multiply = [&](uint32_t step, auto chain) {
         constexpr int C = decltype(chain)::value;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this step's columns are in LDS
@@ -270,10 +270,10 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
         __builtin_amdgcn_sched_barrier(0);
         ThreeTerms b[MT];
 #pragma unroll
-        for (int t = 0; t < MT; ++t) b[t] = three_terms(v[MR + t][0], v[MR + t][1], top);
+        for (int t = 0; t < MT; ++t) b[t] = three_terms(v[MR + t][0], v[MR + t][1], top, half);
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
-            const ThreeTerms a = three_terms(v[m][0], v[m][1], top);
+            const ThreeTerms a = three_terms(v[m][0], v[m][1], top, half);
             const auto add = [&](const bf16x8 &p, const bf16x8 &s, float4_t &to) { to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p, s, to, 0, 0, 0); };
 #pragma unroll
             for (int t = 0; t < MT; ++t) { add(a.high, b[t].high, high[C][m][t]); add(a.low, b[t].high, low[m][t]); }

@@ -35,6 +35,7 @@ def test_logits(hidden, n_expert, tokens):
     for n in tokens:
         x = synth.normed_x(np.random.default_rng(n), n, hidden)
         x *= np.float32(10.0) ** np.random.default_rng(1).integers(-28, 29, size=(n, 1)).astype(np.float32)      # a scale per token
+        x[3, 11] *= np.float32(1e5)      # one product that outweighs the others: what its terms leave out (2^-24 of it) is seen undiluted
         check(m.route(0, torch.from_numpy(x).cuda())[2].cpu().numpy(), x, rows)
     m.close()
 

@@ -100,7 +100,7 @@ hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count
 // ---------------------------------------------------------------- router logits of a token chunk
 
 // out[tok][row] = W[row] . x[tok] for an f32 matrix W (a router, the dense shared expert of mixed layouts) and a chunk of activations. Every f32
-// is the sum of three bf16 numbers, exactly (its bits cut after 8 and 16 places; two of three operations on it are full-rate ones), and of the
+// is the sum of three bf16 numbers, exactly (the nearest one, the nearest to the rest, and what is left), and of the
 // nine products of such sums the six that reach 2^-24 of the largest go through v_mfma_f32_16x16x32_bf16: six of those are 96 cycles for 32 columns
 // where the fp32 unit takes 256. The products of the leading terms have accumulators of their own, the other five share one.
 // A workgroup owns BR = 16 MR rows x BT = 16 MT tokens, each of its eight waves an eighth of k for all of them; the eight sums meet in LDS, in
@@ -108,13 +108,14 @@ hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count
 // take four times as long, 26 instead of 15 us for 64 x 32 outputs of 2048 columns), takes them into registers as fragments (lane (r = l % 16, q = l / 16):
 // columns 4q .. 4q + 3 and 16 + 4q .. of row r; the 16-byte pieces of a row are permuted by r / 2 so that a read pass meets every bank once),
 // requests the next 32 columns into the same place and multiplies meanwhile. No barrier before the sums meet.
-// What bounds it: the fetch - 96 KB in flight for a tile of 64 x 32, which cover about the 1 .. 1.5 us that they take - then cutting and multiplying
+// What bounds it: the fetch - 96 KB in flight for a tile of 64 x 32, which cover about the 1 .. 1.5 us that they take - then splitting and multiplying
 // (2300 .. 3000 cycles for each 256 columns). us, before (v_mfma_f32_16x16x4_f32, both operands through registers into LDS) -> now:
-// gate/up with SwiGLU of 1024 x 2048: 77 tokens 12.3 -> 7.9, 512: 31 -> 19.7, 2048: 95 -> 81; down 2048 x 512: 77 tokens 6.7 -> 4.7, 512: 16.6 -> 14,
-// 2048: 58 -> 53; router 512 x 2048: 77 tokens 10.5 -> 7.2, 512: 19 -> 11.8, 2048: 48 -> 37.
+// gate/up with SwiGLU of 1024 x 2048: 77 tokens 12.3 -> 8.2, 512: 31 -> 20, 2048: 94 -> 83; down 2048 x 512: 77 tokens 6.7 -> 5.0, 512: 16.6 -> 15,
+// 2048: 57 -> 57; router 512 x 2048: 77 tokens 10.4 -> 8.2, 512: 18.7 -> 12.7, 2048: 47 -> 41.
 // The order in which an output's products are added is the same for every tile. Error against a sum in double, of the rms of the outputs: 2048
-// columns 0.94e-7 (two chains of leading products), 512 columns 0.8e-7, where the fp32 unit with totals in double left 1.04e-7 and 1.1e-7 (and 4.1e-7
-// in a router's plain chains). The gate and up products, which SwiGLU multiplies, leave their chain for a double after every 64 columns: 0.8e-7.
+// columns 0.74e-7 (two chains of leading products a wave), 512 columns 0.53e-7, where the fp32 unit with totals in double left 1.04e-7 and 1.1e-7 (and
+// 4.1e-7 in a router's plain chains); gate and up products multiplied by SwiGLU 1.1 .. 1.3e-7, 1.6e-7 before. Terms that are cut instead of rounded are
+// a fifth cheaper to make, but leave out products that all have the sign of the whole: 0.94e-7, and twice that where one product outweighs the rest.
 // An infinity or NaN has no three terms, and an infinite sum may come out as NaN: outputs that are not finite are computed again, product by product.
 // SWIGLU: W holds gate rows, then as many up rows; the upper half of a tile's row blocks are gate rows, the lower half the up rows of the same
 // columns, and out gets silu(gate) * up of them: no pass of its own over the products.
@@ -247,17 +248,11 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
             }
         }
     };
-    constexpr int CH = KIND == F32_PLAIN ? 2 : 1;
-    float4_t high[CH][MR][MT], low[MR][MT];
-    double total[MR][MT][4];
+    float4_t high[2][MR][MT], low[MR][MT];
 #pragma unroll
     for (int m = 0; m < MR; ++m)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            high[0][m][t] = high[CH - 1][m][t] = low[m][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) total[m][t][i] = 0.0;
-        }
+        for (int t = 0; t < MT; ++t) high[0][m][t] = high[1][m][t] = low[m][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t top = in_vector(0xffff0000u), half = in_vector(0x8000u), at0 = 8u * r + (q ^ (r >> 1)), at1 = 8u * r + ((q + 4u) ^ (r >> 1)), steps = K / 256u;
     const auto multiply = [&](uint32_t step, auto chain) {
         constexpr int C = decltype(chain)::value;
@@ -288,32 +283,16 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    const auto flush = [&] {
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) total[m][t][i] += high[0][m][t][i];
-                high[0][m][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            }
-    };
     request(0u);
     for (uint32_t step = 0; step < steps; step += 2u) {
         multiply(step, std::integral_constant<int, 0>{});
-        if (step + 1u < steps) multiply(step + 1u, std::integral_constant<int, CH - 1>{});
-        if constexpr (KIND != F32_PLAIN) flush();
+        if (step + 1u < steps) multiply(step + 1u, std::integral_constant<int, 1>{});
     }
     __syncthreads();
 #pragma unroll
     for (int m = 0; m < MR; ++m)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            float4_t v;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = KIND != F32_PLAIN ? (float)(total[m][t][i] + low[m][t][i]) : high[0][m][t][i] + high[CH - 1][m][t][i] + low[m][t][i];
-            (&lds[0][0][0])[(wave * MR * MT + m * MT + t) * 64u + lane] = v;
-        }
+        for (int t = 0; t < MT; ++t) (&lds[0][0][0])[(wave * MR * MT + m * MT + t) * 64u + lane] = high[0][m][t] + high[1][m][t] + low[m][t];
     __syncthreads();
     // a thread: four consecutive rows of a token (D[i = 4q .. 4q + 3][j = r])
     for (uint32_t o = tid; o < (swiglu ? MR / 2u : MR) * MT * 64u; o += 512u) {
@@ -355,8 +334,8 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
 }
 
 // The tile that costs least: rounds of the device (256 compute units) times what a round of workgroups of it takes, 18, 10 and 7 us for 2048
-// columns of 64 x 32, 32 x 32 and 32 x 16 outputs (gate/up of 512 tokens 19.7 / 23.4 / 26.4 us, of 77 tokens 16.2 / 10.8 / 7.9, down of 77 tokens, 512
-// columns, 6.7 / 4.7 / 5.1, router of 512 tokens 16.9 / 11.8 / 14.2).
+// columns of 64 x 32, 32 x 32 and 32 x 16 outputs (gate/up of 512 tokens 20 / 22.5 / 29 us, of 77 tokens 16.7 / 11.1 / 8.2, down of 77 tokens, 512
+// columns, 7.1 / 5.0 / 5.5, router of 512 tokens 18.5 / 12.7 / 16).
 template <F32Kind KIND>
 hipError_t f32_tiles(const float *w, const float *extra_row, const float *x, uint32_t ntok, uint32_t K, uint32_t n_rows, float *out, uint32_t out_stride, void *xh, void *xl,
                      int *xexp, hipStream_t s) {

@@ -9,8 +9,9 @@ from dwarfstar_red_lite_amd.moe import ResidentMoe
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
-# of the rms of a token's outputs: 0.94e-7 was measured over 3000 outputs of 2048 columns (six chains of at most eight additions, each rounded to
-# 2^-25 of a partial sum, and the result's own 2^-25); one token's 48 outputs spread by a third around that
+# of the rms of a token's outputs: 0.74e-7 was measured over 3000 outputs of 2048 columns (eight parts of two chains of four additions, each rounded to
+# 2^-25 of a partial sum, the products left out at 2^-24 of the others, the result's own 2^-25); one token's outputs spread around that, and one product
+# that outweighs the rest shows the last two undiluted: 2^-24 + 2^-25 = 0.9e-7 with the chains' roundings of it, each at most 2^-25, beside them
 TOL = 2e-7
 
 

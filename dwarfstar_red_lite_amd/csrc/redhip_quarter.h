@@ -311,7 +311,8 @@ __device__ __forceinline__ half8_t finish_entry(const Entry &e, half2_t f, const
 #pragma unroll
         for (int i = 0; i < 4; ++i) r.p[i] = r.p[i] * f + off;
     } else {
-        const uint32_t s1 = twice(e.s), s2 = twice(s1), s3 = twice(s2);
+        // (the one-token kernels, which have the small tables, wait for this chain: two doublings at most in a row, the second step a shift)
+        const uint32_t s1 = twice(e.s), s2 = small_tables<SRC>() ? e.s << 2 : twice(s1), s3 = twice(s2);
         if constexpr (fmt<SRC>() == F_XS || small_tables<SRC>()) {     // IQ2_XS entries are signed bytes in general: the sign goes to the (positive) scale
             const uint32_t fb = __builtin_bit_cast(uint32_t, f);
             r.p[0] *= __builtin_bit_cast(half2_t, and_or(e.s, t.sign_bits, fb));

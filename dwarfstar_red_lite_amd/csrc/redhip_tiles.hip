@@ -130,7 +130,10 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
     };
     // Precision. The matrix unit rounds a sum four times per instruction (once per eight products), so what a block's sum loses goes with the
     // length of its chain of instructions: the low halves have a chain of their own, and the high ones one per kChain steps, added up in f32.
-    constexpr uint32_t kChain = layout<SRC>() == L_ROWS ? 2u : 4u;
+    // Narrow tiles also take batches whose fewer tokens are slices (which stop rounding after four instructions), and are no further off than these: with
+    // chains of four steps 1.87e-7 against 1.76e-7 (IQ2_XXS, 2048 x 512, 24 tokens with the routing given), with two and the low halves first 1.74e-7,
+    // at 1 % of a chunk's time; chains of one step lose more in the additions (1.78e-7 against 1.77e-7).
+    constexpr uint32_t kChain = SETS == 1 || layout<SRC>() == L_ROWS ? 2u : 4u;
     H8 xa[2][8], xb[2][8];                                 // SETS 1: [block], SETS 2: [set]
     const auto load_tile = [&](uint32_t tile) {
 #pragma unroll
@@ -166,7 +169,7 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
             const uint32_t e = N < T ? min(tid, N - 1u) : base + tid;      // (surplus threads repeat the last element)
             const uint32_t at = e & 255u, b = __builtin_amdgcn_readfirstlane((e >> 8) % (SETS * NRT)), un = __builtin_amdgcn_readfirstlane((e >> 8) / (SETS * NRT)), set = b % SETS, slot = b / SETS;
             const float *src = pt + un * G::kPart + slot * PK * G::kSums + set * 256u + at;
-            using Sum = std::conditional_t<(PK > 2u), double, float>;      // (a row's parts are added here)
+            using Sum = std::conditional_t<(PK > 1u), double, float>;      // (a row's parts are added here)
             Sum g[PK], u[PK];
 #pragma unroll
             for (uint32_t k = 0; k < PK; ++k) { g[k] = src[k * G::kSums]; u[k] = src[k * G::kSums + SETS * 256u]; }
@@ -237,18 +240,24 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
                 for (uint32_t m = 0; m < 2u; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[SETS == 1 ? m : s][S].v, w[m], low[m][s], 0, 0, 0);
         });
         float *mine = pt + (rt * PK + kp) * G::kSums + 4u * lane;
+        // (the low halves' sums first: what they and the high ones' leave in a result is then rounded once, not twice)
+        if constexpr (SETS == 1) {
+            float4_t &both = acc[0][0];                    // the two blocks
 #pragma unroll
-        for (uint32_t m = 0; m < 2u; ++m)
-#pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) acc[m][s][t] = fmaf(low[m][s][t], 4.8828125e-4f, sum[m][s][t] + acc[m][s][t]) * d[m];
-        if constexpr (SETS == 1) *reinterpret_cast<float4_t *>(mine + up * 256u) = acc[0][0] + acc[1][0];
-        else {
+            for (int t = 0; t < 4; ++t) {
+                const float l = fmaf(low[1][0][t], 4.8828125e-4f * d[1], low[0][0][t] * (4.8828125e-4f * d[0]));
+                both[t] = fmaf(sum[1][0][t] + acc[1][0][t], d[1], fmaf(sum[0][0][t] + acc[0][0][t], d[0], l));
+            }
+            *reinterpret_cast<float4_t *>(mine + up * 256u) = both;
+        } else {
 #pragma unroll
             for (uint32_t m = 0; m < 2u; ++m)
 #pragma unroll
-                for (uint32_t s = 0; s < (uint32_t)SETS; ++s) *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) = acc[m][s];
+                for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) acc[m][s][t] = fmaf(sum[m][s][t] + acc[m][s][t], d[m], low[m][s][t] * (4.8828125e-4f * d[m]));
+                    *reinterpret_cast<float4_t *>(mine + (m * SETS + s) * 256u) = acc[m][s];
+                }
         }
         advance();
         if (++j == upt && u + 1u < u1) { j = 0u; load_tile(++tile); }

@@ -16,6 +16,9 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 // literal among the operands, and for left shifts, bit-field extracts, permutes, and_or, lshl_or and packed fp16, it is 4.3. So the decode
 // keeps its masks in vector registers, shifts left by additions and merges by bitop3.
 __device__ __forceinline__ uint32_t in_vector(uint32_t k) { asm("" : "+v"(k)); return k; }
+// Hides from the compiler that v is the same in every trip of a loop: what is cheap to form again from it must not be kept in registers
+// (which the activations need) across the loop.
+__device__ __forceinline__ uint32_t each_trip(uint32_t v) { asm volatile("" : "+v"(v)); return v; }
 __device__ __forceinline__ uint32_t twice(uint32_t v) { uint32_t r; asm("v_add_u32 %0, %1, %1" : "=v"(r) : "v"(v)); return r; }
 __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0xea); }
 // bits of w, those at position `from` moved to `to`

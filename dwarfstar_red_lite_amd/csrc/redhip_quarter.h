@@ -178,7 +178,7 @@ __device__ __forceinline__ void load_quarter(const uint8_t *tile, const uint8_t 
             v.a = make_uint4(w.x, w.z, (w.y & 0xffffu) | (w.w << 16), __builtin_amdgcn_ubfe(w.y, 16u, 6u) | (__builtin_amdgcn_ubfe(w.w, 16u, 6u) << 6));
         } else
             v.a = *reinterpret_cast<const uint4 *>(tile + chunk * 32u + 16u * (q & 1u));
-        if constexpr (fmt<SRC>() == F_XS) v.c = *reinterpret_cast<const uint16_t *>(scs + chunk * 4u + 2u * (q & 1u));
+        if constexpr (fmt<SRC>() == F_XS) v.c = *reinterpret_cast<const uint16_t *>(scs + each_trip(chunk * 32u + 16u * (q & 1u)) / 8u);      // (no register of its own beside the quarter's)
         d.x = *reinterpret_cast<const uint16_t *>(ds + (kc * 16u + r) * 2u);
     } else if constexpr (layout<SRC>() == L_ROWS) {
         v.a = *reinterpret_cast<const uint4 *>(tile + block * 64u + 16u * q);

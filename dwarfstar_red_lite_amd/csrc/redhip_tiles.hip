@@ -50,10 +50,6 @@ __device__ __forceinline__ void wave_lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
-// Hides from the compiler that v is the same in every trip of a loop: what is cheap to form again from it must not be kept in registers
-// (which the activations need) across the loop.
-__device__ __forceinline__ uint32_t each_trip(uint32_t v) { asm volatile("" : "+v"(v)); return v; }
-
 // exchange of two registers' halves between lanes that differ in bit 4 (16) or 5 (32)
 __device__ __forceinline__ void swap16(uint32_t &a, uint32_t &b) { const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false); a = r[0]; b = r[1]; }
 __device__ __forceinline__ void swap32(uint32_t &a, uint32_t &b) { const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false); a = r[0]; b = r[1]; }

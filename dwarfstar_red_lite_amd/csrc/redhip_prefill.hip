@@ -116,7 +116,9 @@ hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count
 // columns 0.74e-7 (two chains of leading products a wave), 512 columns 0.53e-7, where the fp32 unit with totals in double left 1.04e-7 and 1.1e-7 (and
 // 4.1e-7 in a router's plain chains); gate and up products multiplied by SwiGLU 1.1 .. 1.3e-7, 1.6e-7 before. Terms that are cut instead of rounded are
 // a fifth cheaper to make, but leave out products that all have the sign of the whole: 0.94e-7, and twice that where one product outweighs the rest.
-// An infinity or NaN has no three terms, and an infinite sum may come out as NaN: outputs that are not finite are computed again, product by product.
+// An infinity or NaN has no three terms, and an infinite sum may come out as NaN: a tile with outputs that are not finite multiplies once more, on the
+// fp32 unit, for these. (An output at a time, a thread's 2048 products behind one another, a chunk of 512 tokens of NaN took 3.2 ms an F2 layer; now 0.30,
+// of numbers 0.28. Where only a leading term overflows 3e-7 .. 4e-7 are lost, 6.6e-7 then.)
 // SWIGLU: W holds gate rows, then as many up rows; the upper half of a tile's row blocks are gate rows, the lower half the up rows of the same
 // columns, and out gets silu(gate) * up of them: no pass of its own over the products.
 // Launches with xh get workgroups behind the tiles that write the fp16 halves of the activations (a wave per token, split_token) and multiply them
@@ -199,6 +201,7 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
                                                         _Float16 *xl, int *xexp, uint32_t K, uint32_t n_rows, uint32_t ntok, Beside<KIND> router) {
     constexpr uint32_t BR = 16u * MR, BT = 16u * MT, NB = MR + MT, PIECES = 2u * NB > MR * MT ? 2u * NB : MR * MT;      // KB per wave: 32 columns of the rows and tokens, later its sums
     __shared__ __attribute__((aligned(16))) float4_t lds[8][PIECES][64];
+    __shared__ uint32_t again;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t tok_tiles = (ntok + BT - 1u) / BT, first = KIND == F32_BOTH ? n_rows / BR * tok_tiles : 0u;      // tiles of gate and up rows in front of the router's
     const bool swiglu = KIND == F32_SWIGLU || (KIND == F32_BOTH && blockIdx.x < first);
@@ -254,15 +257,18 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
 #pragma unroll
         for (int t = 0; t < MT; ++t) high[0][m][t] = high[1][m][t] = low[m][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t top = in_vector(0xffff0000u), half = in_vector(0x8000u), at0 = 8u * r + (q ^ (r >> 1)), at1 = 8u * r + ((q + 4u) ^ (r >> 1)), steps = K / 256u;
-    const auto multiply = [&](uint32_t step, auto chain) {
-        constexpr int C = decltype(chain)::value;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this step's columns are in LDS
-        float4_t v[NB][2];
+    const auto fetched = [&](uint32_t step, float4_t (&v)[NB][2]) {      // this step's columns into registers, the next ones requested
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // they are in LDS
 #pragma unroll
         for (uint32_t i = 0; i < NB; ++i) { v[i][0] = mine[128u * i + at0]; v[i][1] = mine[128u * i + at1]; }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // and read, before the next ones take their place
         if (step + 1u < steps) request(step + 1u);
         __builtin_amdgcn_sched_barrier(0);
+    };
+    const auto multiply = [&](uint32_t step, auto chain) {
+        constexpr int C = decltype(chain)::value;
+        float4_t v[NB][2];
+        fetched(step, v);
         ThreeTerms b[MT];
 #pragma unroll
         for (int t = 0; t < MT; ++t) b[t] = three_terms(v[MR + t][0], v[MR + t][1], top, half);
@@ -288,49 +294,79 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
         multiply(step, std::integral_constant<int, 0>{});
         if (step + 1u < steps) multiply(step + 1u, std::integral_constant<int, 1>{});
     }
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < MR; ++m)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) (&lds[0][0][0])[(wave * MR * MT + m * MT + t) * 64u + lane] = high[0][m][t] + high[1][m][t] + low[m][t];
-    __syncthreads();
     // a thread: four consecutive rows of a token (D[i = 4q .. 4q + 3][j = r])
-    for (uint32_t o = tid; o < (swiglu ? MR / 2u : MR) * MT * 64u; o += 512u) {
-        const uint32_t t = (o >> 6) % MT, m = (o >> 6) / MT, l = o & 63u, tok = tile_t * BT + 16u * t + (l & 15u), row = 4u * (l >> 4);
-        if (tok >= ntok) continue;
-        const auto products = [&](uint32_t mm) {
-            double sum[4] = {0.0, 0.0, 0.0, 0.0};
+    const uint32_t t = (tid >> 6) % MT, m = (tid >> 6) / MT, l = tid & 63u, tok = tile_t * BT + 16u * t + (l & 15u), row = 4u * (l >> 4);
+    const bool has = tid < (swiglu ? MR / 2u : MR) * MT * 64u && tok < ntok;
+    static_assert(MR * MT * 64u <= 512u, "four outputs a thread");
+    const auto meet = [&](auto part) {                     // the waves' sums in LDS
+        __syncthreads();
 #pragma unroll
-            for (uint32_t k = 0; k < 8u; ++k) {
-                const float4_t v = (&lds[0][0][0])[(k * MR * MT + mm * MT + t) * 64u + l];
+        for (int mm = 0; mm < MR; ++mm)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) sum[i] += v[i];
-            }
-            float4_t y;
+            for (int tt = 0; tt < MT; ++tt) (&lds[0][0][0])[(wave * MR * MT + mm * MT + tt) * 64u + lane] = part(mm, tt);
+        __syncthreads();
+    };
+    const auto products = [&](uint32_t mm) {
+        double sum[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) {
-                y[i] = (float)sum[i];
-                if (!(fabsf(y[i]) <= 3.402823466e38f) && block_row(mm) + row + i < all_rows) {
-                    const float *wr = matrix_row(block_row(mm) + row + i), *xr = x + (uint64_t)tok * K;
-                    float again = 0.0f;
-                    for (uint32_t c = 0; c < K; ++c) again = fmaf(wr[c], xr[c], again);
-                    y[i] = again;
-                }
-            }
-            return y;
-        };
-        float4_t y = products(m);
-        if (swiglu) {
-            const float4_t u = products(m + MR / 2u);
+        for (uint32_t k = 0; k < 8u; ++k) {
+            const float4_t v = (&lds[0][0][0])[(k * MR * MT + mm * MT + t) * 64u + l];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) y[i] = (y[i] / (1.0f + expf(-y[i]))) * u[i];
-            *reinterpret_cast<float4_t *>(out + (uint64_t)tok * out_stride + block_row(m) + row) = y;
-        } else {
+            for (int i = 0; i < 4; ++i) sum[i] += v[i];
+        }
+        return float4_t{(float)sum[0], (float)sum[1], (float)sum[2], (float)sum[3]};
+    };
+    // stores those of a thread's outputs that `which` names (a bit each) and whose products are finite or `last`; returns the rest
+    const auto store = [&](uint32_t which, bool last) {
+        float4_t y = products(m), u{};
+        if (swiglu) u = products(m + MR / 2u);
+        float *to = out + (uint64_t)tok * out_stride + block_row(m) + row;
+        uint32_t now = 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+            if ((fabsf(y[i]) <= 3.402823466e38f && fabsf(u[i]) <= 3.402823466e38f) || last) now |= which & (1u << i);
+            if (swiglu) y[i] = (y[i] / (1.0f + expf(-y[i]))) * u[i];
+        }
+        if (swiglu && now == 15u) *reinterpret_cast<float4_t *>(to) = y;
+        else {
 #pragma unroll
             for (uint32_t i = 0; i < 4u; ++i)
-                if (block_row(m) + row + i < all_rows) out[(uint64_t)tok * out_stride + block_row(m) + row + i] = y[i];
+                if (now >> i & 1u) to[i] = y[i];
         }
+        which &= ~now;
+        return which;
+    };
+    uint32_t which = 0u;                                   // outputs of this thread that are to be stored
+    if (has) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) which |= swiglu || block_row(m) + row + i < all_rows ? 1u << i : 0u;
     }
+    if (tid == 0u) again = 0u;
+    meet([&](int mm, int tt) { return high[0][mm][tt] + high[1][mm][tt] + low[mm][tt]; });
+    if (which) which = store(which, false);
+    if (which) again = 1u;
+    __syncthreads();
+    if (!again) return;
+    // the tile once more on the fp32 unit, for the others
+    float4_t sum[MR][MT];
+#pragma unroll
+    for (int mm = 0; mm < MR; ++mm)
+#pragma unroll
+        for (int tt = 0; tt < MT; ++tt) sum[mm][tt] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    request(0u);
+    for (uint32_t step = 0; step < steps; ++step) {
+        float4_t v[NB][2];
+        fetched(step, v);
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k)
+#pragma unroll
+            for (int mm = 0; mm < MR; ++mm)
+#pragma unroll
+                for (int tt = 0; tt < MT; ++tt)
+                    sum[mm][tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[mm][k / 4u][k % 4u], v[MR + tt][k / 4u][k % 4u], sum[mm][tt], 0, 0, 0);
+    }
+    meet([&](int mm, int tt) { return sum[mm][tt]; });
+    if (which) store(which, true);
 }
 
 // The tile that costs least: rounds of the device (256 compute units) times what a round of workgroups of it takes, 18, 10 and 7 us for 2048

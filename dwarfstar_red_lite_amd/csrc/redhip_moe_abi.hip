@@ -1,5 +1,6 @@
 // Resident MoE FFN layers: every expert of every layer stays in HBM, one call runs a layer's FFN on a stream.
 // See include/redhip_moe.h for the contract.
+#include <math.h>
 #include <stdarg.h>
 #include <stdlib.h>
 #include <stdio.h>
@@ -140,33 +141,32 @@ struct Moe {
     // 512 pairs behind the layer's own router (own_router: the selection launch sorts that many; a caller's routing is sorted by one more
     // workgroup of the launch that splits the activations, up to 256 pairs)
     static constexpr uint32_t kSmallMaxFused = 16u, kSmallMaxRouted = 32u, kSmallMaxGiven = 24u, kSmallMaxMixed = 32u;
-    // ... unless the tiles are ahead from fewer tokens on. The slices cost a pass per two pairs of an expert, the tiles a decode per distinct expert,
-    // so the line lies lower the cheaper a unit of the tiles' decode is and the larger the experts, which have to fill the tiles' launches; a call
-    // with given routing does not know how it is spread. Slices / tiles, us per layer:
-    // 2048 x 512, 512 experts, ten a token, behind the own router:
-    //   IQ2_XXS 20, 24, 28, 32 tokens 85 / 86, 97 / 94, 109 / 102, 121 / 110; IQ1_M 18, 24: 89 / 85, 108 / 95; IQ3_S down 18, 20, 24: 90 / 92, 97 / 96,
-    //   108 / 102; IQ2_XS 20, 24, 28: 101 / 106, 116 / 114, 130 / 121
-    // given, evenly / on 32 hot experts:
-    //   IQ2_XXS 18, 20: 69 / 72 and 58 / 51, 75 / 75 and 63 / 53; IQ1_M 18: 84 / 80 and 71 / 61; IQ3_S down 18, 20: 86 / 89 and 71 / 63, 93 / 92 and
-    //   77 / 67; IQ2_XS 20, 22, 24: 97 / 99 and 81 / 71, 103 / 103 and 87 / 73, 109 / 106 and 93 / 74
-    // 1024 x 512, 200 experts, eight a token, own router: IQ1_M 24, 32: 61 / 62, 75 / 66; IQ3_S down 60 / 66, 75 / 67; IQ2_XS 63 / 69, 78 / 74; IQ2_XXS
-    //   32: 65 / 65; given 18, 24: IQ1_M 47 / 52 and 44 / 47, 56 / 54 and 52 / 48; IQ3_S down 24: 57 / 58 and 51 / 50; IQ2_XS 58 / 59 and 54 / 52
-    // 2048 x 768 (IQ2_XXS, 128 experts, eight a token): own router 18, 24: 78 / 81, 95 / 87; evenly given 73 / 73, 88 / 80
-    // 1024 x 256, 96 experts, six a token, own router 24, 32: IQ1_M 41 / 47, 49 / 48; IQ3_S down 40 / 50, 48 / 51; IQ2_XS 41 / 51, 50 / 52: the slices
-    uint32_t slices_up_to(bool own_router) const {
-        const size_t weights = (size_t)cfg.hidden * cfg.ffn;
-        if (weights >= (size_t)1024u * 512u && tile_chunk(kSmallMaxRouted)) {
-            const bool large = weights >= (size_t)2048u * 512u;
-            if (fused) {
-                if (large) return own_router ? 22u : 19u;
-            } else if (gu_type == T_IQ1_M)
-                return large ? 16u : own_router ? 25u : 22u;
-            else if (dn_type == T_IQ3_S)
-                return large ? 19u : own_router ? 28u : kSmallMaxGiven;
-            else
-                return large ? (own_router ? 23u : 22u) : own_router ? 30u : kSmallMaxGiven;
-        }
-        return own_router ? (fused ? kSmallMaxRouted : kSmallMaxMixed) : kSmallMaxGiven;
+    // ... unless the tiles are ahead from fewer tokens on. Per layer the slices cost so many us per pass of two pairs of an expert, and per token (the shared
+    // expert, on mixed layouts also the router), the tiles so many per distinct expert, each more for larger matrices, and their launches more than the
+    // slices': both by the tokens' expected spread over the experts. Fitted to 2052 calls timed on both sides: 17 .. 32 tokens, 16 to 512 experts,
+    // two to ten a token, 1024 x 512 to 2048 x 768, own router and routing given (that call does not know how it is spread: a line between even
+    // spread and 32 hot experts). Chosen so, a call is 0.4 % slower than on the quicker side on average. Slices / tiles, us:
+    // own router, 32 tokens of 2048 x 512: 512 experts, ten a token: IQ2_XXS 122 / 112, IQ1_M 135 / 111; four a token 74 / 81 and 84 / 78; 60 experts, two a
+    //   token 45 / 54 and 59 / 55; 32 experts, eight a token 79 / 48 and 95 / 60. 18 tokens: 512 experts, ten a token 80 / 85 and 89 / 88; 32 experts, eight a
+    //   token 53 / 52 and 63 / 57
+    // given, evenly / on 32 hot experts: 20 tokens of 2048 x 512, 512 experts, ten a token: IQ2_XXS 74 / 78 and 62 / 51; 23 tokens, 200 experts, eight a token:
+    //   IQ3_S down 71 / 61 (hot), IQ2_XS 85 / 87 and 74 / 61
+    // Narrower experts (1024 x 256: 32 tokens, 96 experts, six a token 48 / 50 .. 52) stay slices.
+    bool slices_ahead(uint32_t ntok, bool own_router) const {
+        const float E = (float)cfg.n_expert, share = (float)cfg.top_k / E, n = (float)ntok, weights = (float)cfg.hidden * (float)cfg.ffn / (2048.0f * 512.0f);
+        const float distinct = E * (1.0f - powf(1.0f - share, n));
+        const float passes = 0.5f * (n * (float)cfg.top_k + 0.5f * E * (1.0f - powf(1.0f - 2.0f * share, n)));      // (half the pairs, and half a pass for every odd one out)
+        const float launches = (fused ? 19.5f : gu_type == T_IQ1_M ? 22.5f : dn_type == T_IQ3_S ? 26.5f : 27.0f) - (own_router ? 0.0f : 2.2f);
+        return passes * (0.075f + 0.255f * weights) + n * (fused ? 0.22f : 0.57f) <= launches + fmaxf(distinct, 32.0f) * (0.055f + 0.205f * weights);      // (fewer experts do not fill the tiles' launches)
+    }
+    uint32_t slices_own = 0, slices_given = 0;      // batches of up to so many tokens run as slices (set at creation)
+    uint32_t slices_up_to(bool own_router) const { return own_router ? slices_own : slices_given; }
+    uint32_t slices_line(bool own_router) const {
+        const uint32_t most = !own_router ? kSmallMaxGiven : fused ? kSmallMaxRouted : kSmallMaxMixed;
+        if (cfg.ffn < 512u || (size_t)cfg.hidden * cfg.ffn < (size_t)1024u * 512u || !tile_chunk(kSmallMaxRouted)) return most;
+        uint32_t n = kSmallMaxFused;
+        while (n < most && slices_ahead(n + 1u, own_router)) ++n;
+        return n;
     }
     bool dense_routed = false;               // every layer has f32 copies of its router and of the shared expert's gate | up rows (set at creation)
     bool small_batch(uint32_t ntok, bool own_router = false) const {
@@ -556,6 +556,8 @@ redhip_moe_t redhip_moe_create(const redhip_moe_config *cfg) {
                           c.hidden / 512u <= 4u && (nv == 2u || nv == 4u || nv == 8u || nv == 16u);
         m->dense_routed = m->mixed_slices;      // (every mixed layer gets f32 copies of its shared expert, and of its router unless that is f32 already)
     }
+    m->slices_own = m->slices_line(true);
+    m->slices_given = m->slices_line(false);
     m->pk_gate_bytes = packed_matrix_bytes(gu, c.ffn, c.hidden);
     m->packed_stride = m->fused && m->rowmajor_down() ? m->expert_stride : align256(2u * m->pk_gate_bytes);
     m->gu_grid = caller_grid_device(gu);

@@ -1,5 +1,6 @@
 """The sizes where batches of large experts leave the slices for the tile kernels, on both sides of each line, against the CPU path; a token
-gets the same from either."""
+gets the same from either, and each side is the one that it is said to be."""
+import ctypes as C
 import json
 import os
 
@@ -7,6 +8,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as orc
+from dwarfstar_red_lite_amd import load
 from dwarfstar_red_lite_amd import moe as moe_api
 from dwarfstar_red_lite_amd import synth
 from dwarfstar_red_lite_amd.moe import ResidentMoe
@@ -17,9 +19,23 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
-@pytest.mark.parametrize("layout,shape,own,given", [("iq2", (2048, 512, 40, 10), 22, 19), ("iq2", (2048, 768, 24, 8), 22, 19), ("m", (2048, 512, 40, 10), 16, 16),
-                                                    ("f2", (2048, 512, 40, 10), 19, 19), ("xs", (2048, 512, 40, 10), 23, 22), ("m", (1024, 512, 24, 8), 25, 22),
-                                                    ("f2", (1024, 512, 24, 8), 28, 24), ("xs", (1024, 512, 24, 8), 30, 24)])
+def on_tiles(call):
+    """the call's result, and whether the tile kernels made it"""
+    lib = load()
+    n = lib.redhip_profile_stage_count()
+    ms, launches = (C.c_double * n)(), (C.c_uint32 * n)()
+    lib.redhip_profile_begin()
+    out = call().cpu().numpy()
+    lib.redhip_profile_end(ms, launches, n)
+    return out, launches[[lib.redhip_profile_stage_name(i) for i in range(n)].index(b"prefill_gateup")] > 0
+
+
+# experts per layer, experts per token and size all move the lines (most tokens that are slices: behind the own router, with the routing given); layers of
+# few experts per token have none below 32 and 24 tokens
+@pytest.mark.parametrize("layout,shape,own,given", [("iq2", (2048, 512, 64, 6), 24, 22), ("iq2", (2048, 768, 40, 4), 25, 22), ("m", (2048, 512, 48, 5), 21, 19),
+                                                    ("f2", (2048, 512, 48, 5), 24, 22), ("xs", (2048, 512, 64, 6), 23, 21), ("m", (1024, 512, 24, 8), 19, 17),
+                                                    ("f2", (1024, 512, 24, 8), 21, 20), ("xs", (1024, 512, 24, 8), 22, 20), ("iq2", (2048, 512, 40, 10), 16, 16),
+                                                    ("iq2", (2048, 512, 60, 2), 32, 24), ("f2", (2048, 512, 60, 2), 32, 24), ("m", (1024, 512, 60, 4), 28, 24)])
 def test_both_sides_of_the_line(layout, shape, own, given, golden_dir):
     if layout in ("m", "xs"):
         g = json.load(open(os.path.join(golden_dir, "iq_grids.json")))
@@ -34,13 +50,19 @@ def test_both_sides_of_the_line(layout, shape, own, given, golden_dir):
     x = synth.normed_x(np.random.default_rng(96), own + 1, H)
     x_dev = torch.from_numpy(x).cuda()
     want, cids, _, clog = orc.Layer(cfg, **lay).forward(x, threads=8)
-    whole = [m.forward(0, x_dev[:n]).cpu().numpy() for n in (own, own + 1)]
+    whole = []
+    for n in (own, own + 1):
+        out, tiles = on_tiles(lambda: m.forward(0, x_dev[:n]))
+        assert tiles == (n > own)
+        whole.append(out)
     gids, gw, _ = m.last_route(own + 1)
     same = [t for t in range(own) if np.array_equal(gids[t], cids[t])]
     assert all(ids_match_up_to_ties(gids[t], cids[t], clog[t]) for t in range(own + 1)) and len(same) >= own - 1
     ids_dev, w_dev = torch.from_numpy(gids.astype(np.int32)).cuda(), torch.from_numpy(gw).cuda()
     for n in (given, given + 1):
-        whole.append(m.experts(0, x_dev[:n], ids_dev[:n].contiguous(), w_dev[:n].contiguous()).cpu().numpy())
+        out, tiles = on_tiles(lambda: m.experts(0, x_dev[:n], ids_dev[:n].contiguous(), w_dev[:n].contiguous()))
+        assert tiles == (n > given)
+        whole.append(out)
     for got in whole:
         assert max(rel_l2(got[t], want[t]) for t in same if t < len(got)) <= REL_L2_TOL
         assert max(rel_l2(got[t], whole[1][t]) for t in range(len(got))) <= 1e-6      # (either path is 2e-7 off from exact)

@@ -100,11 +100,15 @@ __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *
             for (uint32_t c = 0; c < kCopies; ++c) *reinterpret_cast<uint4 *>(entries + ((size_t)e * kCopies + c) * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
         }
     } else {
-        for (uint32_t e = tid; e < 16u * 512u; e += T) {
-            const uint32_t gw = redhip_iq3s_grid[e & 511u];
-            const float f = (float)(1u + 2u * (e >> 9));
-            *reinterpret_cast<uint2 *>(entries + (size_t)e * 8u) =
-                make_uint2(two_halves(f * (float)(gw & 255u), f * (float)((gw >> 8) & 255u)), two_halves(f * (float)((gw >> 16) & 255u), f * (float)(gw >> 24)));
+        for (uint32_t i = tid; i < 2u * 512u; i += T) {      // (an entry's request is a trip to memory: eight scales for each)
+            const uint32_t gw = redhip_iq3s_grid[i & 511u];
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) {
+                const uint32_t scale = (i >> 9) * 8u + k;
+                const float f = (float)(1u + 2u * scale);
+                *reinterpret_cast<uint2 *>(entries + (size_t)(scale * 512u + (i & 511u)) * 8u) =
+                    make_uint2(two_halves(f * (float)(gw & 255u), f * (float)((gw >> 8) & 255u)), two_halves(f * (float)((gw >> 16) & 255u), f * (float)(gw >> 24)));
+            }
         }
     }
     build_signs<SRC, T>(signs, tid);

@@ -300,7 +300,7 @@ constexpr uint32_t down_waves(int sets) { return sets == 1 ? 12u : 8u; }
 template <int SETS, uint32_t KP> constexpr uint32_t down_tiles_a_pass() { return SETS == 1 && KP <= 2u ? 2u : 1u; }
 template <int SRC, int SETS, uint32_t KP> struct DownLds {
     uint32_t signs[sign_bytes<SRC>() / 4u];
-    uint8_t entries[kEntryBytes];
+    uint8_t entries[small_tables<SRC>() ? small_entry_bytes<SRC>() : kEntryBytes];
     uint8_t x[(SETS == 2 ? 2u : down_tiles_a_pass<SETS, KP>()) * KP * kPanel];      // [tile % 2, or set][block]
     TileInfo tiles[kTileInfos];
     float scales[2u * KP * 16u * (uint32_t)SETS];        // [tile % 2][block][pair]: powers of two that the sums of a pair's block are multiplied with
@@ -325,8 +325,14 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
     const uint32_t ipt = a.rows / 32u, tile0 = i0 / parts, n_info = (i1 - 1u) / parts + 1u - tile0, quads = ((ipt / 4u) << 16) / parts + 1u;      // quads: fours of items per part, 16 bits behind the point
     if (tid < 64u) {
         if (tid < n_info) lds.tiles[tid] = tile_info(a, list, tile0 + tid);
-    } else if (tables)
-        build_staged_tables<SRC, T - 64u>(lds.entries, lds.signs, tid - 64u, a.grid);
+    } else if (tables) {
+        if constexpr (small_tables<SRC>()) {
+            SmallSeeds<SRC, T - 64u> seeds;
+            seeds.request(tid - 64u, a.grid);
+            seeds.store(lds.entries, lds.signs, tid - 64u);
+        } else
+            build_staged_tables<SRC, T - 64u>(lds.entries, lds.signs, tid - 64u, a.grid);
+    }
     __syncthreads();
     const LaneTables lt = lane_tables<SRC>(lds.entries, lds.signs, tid);
     const auto info_of = [&](uint32_t tile) { return uniform_info(lds.tiles[tile - tile0]); };
@@ -516,14 +522,18 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
 // down. Whole chunks measured with and without, by weights in wide tiles: gate/up of 235 to 268 million (512 tokens, Zipf-popular or 32 pairs
 // per expert) 7 to 12 us slower with them, 262 million (250 tiles of 1024 x 512) 0 to 4 us quicker, 315 million 15 us quicker, one of 1000 million
 // 20 to 60 us quicker; down of 117 million 5 to 8 us slower, 131 to 157 million 1 to 3 us slower, 230 million 4 us quicker, 500 million 6 to
-// 24. Down matrices of more than two blocks have none: their tiles of 32 pairs do not fit the LDS.
-template <int SRC, bool DOWN, uint32_t KP> constexpr bool has_wide() { return !DOWN || KP <= 2u; }
+// 24. Wide down tiles of three blocks, and of four IQ3_S ones, fit the LDS beside small tables only; even so 2048 x 768, 128 experts, eight a token, raw
+// rows take at 2048 tokens 239 us instead of 339 (IQ3_S), 196 / 242 (IQ2_XS), 181 / 191 (IQ1_M), whole calls of the pool 507 / 616, 543 / 595, 471 / 492
+// and 467 / 491 (IQ2_XXS). The other formats' four blocks do not fit, and packed rows gain nothing.
+template <int SRC, bool DOWN, uint32_t KP> constexpr bool has_wide() { return !DOWN || KP <= 2u || (layout<SRC>() == L_RAW && (KP == 3u || fmt<SRC>() == F_IQ3)); }
+template <int SRC, int SETS, uint32_t KP> constexpr int down_src() { return SETS == 2 && KP > 2u ? SRC | SMALL_TABLES : SRC; }
 template <int SRC, bool DOWN, uint32_t KP> uint32_t few_wide(uint32_t rows, uint32_t K) {
     return !has_wide<SRC, DOWN, KP>() ? ~0u : (DOWN ? 200000000u : 145000000u) / (rows * K) + 1u;
 }
 template <int SRC, bool DOWN, int SETS, uint32_t KP>
 __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) void staged_tiles_kernel(StagedArgs a) {
-    __shared__ __attribute__((aligned(16))) std::conditional_t<DOWN, DownLds<SRC, SETS, KP>, GateUpLds<SRC, SETS, KP>> lds;
+    __shared__ __attribute__((aligned(16))) std::conditional_t<DOWN, DownLds<down_src<SRC, SETS, KP>(), SETS, KP>, GateUpLds<SRC, SETS, KP>> lds;
+    static_assert(sizeof(lds) <= 160u * 1024u, "what a compute unit has");
     const uint32_t n0 = a.n_tiles[0], n1 = a.n_tiles[1], n2 = a.n_tiles[2];      // (one trip)
     const bool few = n1 < a.few;
     if (SETS == 2 && few) return;
@@ -543,7 +553,7 @@ __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) v
     for (uint32_t from = w0; from < w1;) {                 // (a run of more than kTileInfos tiles in parts)
         const uint32_t to = min(w1, (from / per_tile + kTileInfos) * per_tile);
         if (from != w0) __syncthreads();
-        if constexpr (DOWN) down_items<SRC, SETS, KP>(a, list, per_tile, from, to, lds, from == w0);
+        if constexpr (DOWN) down_items<down_src<SRC, SETS, KP>(), SETS, KP>(a, list, per_tile, from, to, lds, from == w0);
         else gateup_units<SRC, SETS, KP>(a, list, from, to, lds, from == w0);
         from = to;
     }

@@ -1,5 +1,6 @@
 """Down matrices of three and four blocks of 256 columns on raw rows: their tiles are cut into parts (a pass each, fours of 32-row items), as many as the
-busiest workgroup has anyway. Numbers of tiles on both sides of what the device holds at once, against sums in double."""
+busiest workgroup has anyway, and tiles of up to 32 pairs have a launch of their own again. Numbers of tiles on both sides of what the device holds at
+once, against sums in double."""
 import ctypes as C
 import json
 import os
@@ -61,6 +62,20 @@ def test_narrow_tiles(layout, ffn, hidden, used, n, golden_dir):
     got = m.experts(0, x, ids, w).to(torch.float64)
     want = routed_in_double(lay, cfg, x, ids, w)
     assert float((got - want).norm() / want.norm()) <= F32_CHUNK
+    m.close()
+
+
+# 30 pairs an expert beside some of 31 and 32; weights in wide tiles above the line of 200 million
+@pytest.mark.parametrize("layout,hidden,ffn,used", [("f2", 2048, 768, 136), ("xs", 2048, 768, 136), ("m", 2048, 768, 136), ("f2", 2048, 1024, 104)])
+def test_wide_tiles(layout, hidden, ffn, used, golden_dir):
+    n = used * 30 // 4 + 11
+    cfg, lay, m = layer(layout, hidden, ffn, used, n, golden_dir)
+    x = torch.from_numpy(synth.normed_x(np.random.default_rng(74), n, hidden)).cuda()
+    ids, w = evenly(n, used, 75)
+    out = []
+    assert down_stage(lambda: out.append(m.experts(0, x, ids, w)))[1] == 2      # a launch for wide and one for narrow tiles
+    want = routed_in_double(lay, cfg, x, ids, w)
+    assert float((out[0].to(torch.float64) - want).norm() / want.norm()) <= F32_CHUNK
     m.close()
 
 

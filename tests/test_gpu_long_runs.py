@@ -22,9 +22,9 @@ def grids(golden_dir):
     return xs, m
 
 
-# 22000 pairs an expert: 688 tiles of 32, 8256 in all (and the shared expert's), 33 and more in a run of 256; 24 experts of 5500 pairs: 344 tiles of
-# 16 each (a down matrix of three blocks has no wide ones)
-@pytest.mark.parametrize("layout,ffn,n_expert,ntok", [("iq2", 256, 12, 66000), ("m", 768, 24, 33000)])
+# 22000 pairs an expert: 688 tiles of 32, 8256 in all (and the shared expert's), 33 and more in a run of 256; 24 experts of 11000 pairs: 344 tiles of
+# 32 each, a down matrix of three blocks (half as many: 17 a run)
+@pytest.mark.parametrize("layout,ffn,n_expert,ntok", [("iq2", 256, 12, 66000), ("m", 768, 24, 33000), ("m", 768, 24, 66000)])
 def test_more_tiles_than_infos(grids, layout, ffn, n_expert, ntok):
     from dwarfstar_red_lite_amd import moe as moe_api
     hidden, top_k = 512, 4

@@ -163,7 +163,11 @@ struct Moe {
     uint32_t slices_up_to(bool own_router) const { return own_router ? slices_own : slices_given; }
     uint32_t slices_line(bool own_router) const {
         const uint32_t most = !own_router ? kSmallMaxGiven : fused ? kSmallMaxRouted : kSmallMaxMixed;
-        if (cfg.ffn < 512u || (size_t)cfg.hidden * cfg.ffn < (size_t)1024u * 512u || !tile_chunk(kSmallMaxRouted)) return most;
+        const size_t weights = (size_t)cfg.hidden * cfg.ffn;
+        if (cfg.ffn < 512u || weights < (size_t)1024u * 512u || !tile_chunk(kSmallMaxRouted)) return most;
+        // (and 1024 x 512 where the tiles are further off from sums in double than the slices, 1.75e-7 against 1.72e-7; behind the own router of a mixed
+        // layout they are not, with the tiles' router)
+        if (weights < (size_t)2048u * 512u && (fused || (!own_router && gu_type != T_IQ1_M))) return most;
         uint32_t n = kSmallMaxFused;
         while (n < most && slices_ahead(n + 1u, own_router)) ++n;
         return n;
@@ -556,8 +560,9 @@ redhip_moe_t redhip_moe_create(const redhip_moe_config *cfg) {
                           c.hidden / 512u <= 4u && (nv == 2u || nv == 4u || nv == 8u || nv == 16u);
         m->dense_routed = m->mixed_slices;      // (every mixed layer gets f32 copies of its shared expert, and of its router unless that is f32 already)
     }
-    m->slices_own = m->slices_line(true);
     m->slices_given = m->slices_line(false);
+    m->slices_own = m->slices_line(true);
+    if (m->slices_own < m->slices_given) m->slices_own = m->slices_given;      // (a batch of given routing is checked against both)
     m->pk_gate_bytes = packed_matrix_bytes(gu, c.ffn, c.hidden);
     m->packed_stride = m->fused && m->rowmajor_down() ? m->expert_stride : align256(2u * m->pk_gate_bytes);
     m->gu_grid = caller_grid_device(gu);

@@ -34,8 +34,8 @@ def on_tiles(call):
 # few experts per token have none below 32 and 24 tokens
 @pytest.mark.parametrize("layout,shape,own,given", [("iq2", (2048, 512, 64, 6), 24, 22), ("iq2", (2048, 768, 40, 4), 25, 22), ("m", (2048, 512, 48, 5), 21, 19),
                                                     ("f2", (2048, 512, 48, 5), 24, 22), ("xs", (2048, 512, 64, 6), 23, 21), ("m", (1024, 512, 24, 8), 19, 17),
-                                                    ("f2", (1024, 512, 24, 8), 21, 20), ("xs", (1024, 512, 24, 8), 22, 20), ("iq2", (2048, 512, 40, 10), 16, 16),
-                                                    ("iq2", (2048, 512, 60, 2), 32, 24), ("f2", (2048, 512, 60, 2), 32, 24), ("m", (1024, 512, 60, 4), 28, 24)])
+                                                    ("f2", (1024, 512, 24, 8), 24, 24), ("xs", (1024, 512, 24, 8), 24, 24), ("iq2", (2048, 512, 40, 10), 16, 16),
+                                                    ("iq2", (1024, 512, 24, 8), 32, 24), ("iq2", (2048, 512, 60, 2), 32, 24), ("f2", (2048, 512, 60, 2), 32, 24), ("m", (1024, 512, 60, 4), 28, 24)])
 def test_both_sides_of_the_line(layout, shape, own, given, golden_dir):
     if layout in ("m", "xs"):
         g = json.load(open(os.path.join(golden_dir, "iq_grids.json")))

@@ -57,3 +57,21 @@ def test_tiles_against_slices(layout, hidden, ffn, golden_dir):
     slices, tiles = np.sqrt(err / norm)
     print("%s %d x %d: slices %.3e, tiles %.3e" % (layout, hidden, ffn, slices, tiles))
     assert slices <= 2.1e-7 and tiles <= slices, (slices, tiles)      # (2.1e-7: what f32 products of such a layer give)
+
+
+# where 32 tokens with the routing given would be further off on the tiles than as slices, 24 still are slices, however few the experts
+@pytest.mark.parametrize("layout", ["iq2", "f2", "xs"])
+def test_small_experts_stay_slices(layout, golden_dir):
+    from test_gpu_batch_lines import on_tiles
+    if layout == "xs":
+        g = json.load(open(os.path.join(golden_dir, "iq_grids.json")))
+        moe_api.set_codebooks(*(np.frombuffer(bytes.fromhex(g[k]), np.int8) for k in ("iq2_xs", "iq1_m")))
+    cfg = synth.layer_config(hidden=1024, ffn=512, n_expert=24, top_k=8, layout=layout)
+    m = ResidentMoe(cfg, n_layer=1, max_tokens=32)
+    m.load_layer(0, synth.make_layer(3, cfg))
+    x = torch.from_numpy(synth.normed_x(np.random.default_rng(4), 32, 1024)).cuda()
+    ids = torch.from_numpy(np.stack([np.random.default_rng(t).permutation(24)[:8] for t in range(32)]).astype(np.int32)).cuda()
+    w = torch.full((32, 8), 0.125, device="cuda")
+    for n in (17, 24, 25):
+        assert on_tiles(lambda: m.experts(0, x[:n].contiguous(), ids[:n].contiguous(), w[:n].contiguous()))[1] == (n > 24)
+    m.close()

@@ -278,6 +278,7 @@ struct StagedChunk {                        // the pair sort of the call, its ti
     TileLists tl;
     uint32_t ntok, top_k, n_expert;
     uint32_t wide_tiles = kWideUnknown;     // tiles of more than kPrefillTile pairs, where the host knows their number
+    bool batch = false;                     // so few tokens that still fewer run as expert slices: the sums of the tiles as exact as theirs
 };
 bool staged_gateup_supported(uint32_t type, RowLayout lay, uint32_t hidden, uint32_t ffn);
 bool staged_down_supported(uint32_t type, RowLayout lay, uint32_t hidden, uint32_t ffn);

@@ -404,7 +404,7 @@ int experts_enqueue(Moe *m, uint32_t layer, const float *x, uint32_t ntok, const
             const uint8_t *plain = m->fused ? L.packed : L.experts;
             const StagedMatrices gu{m->gu_type, tiles_gu ? RowLayout::tiled : rows, tiles_gu ? L.tiled : plain, tiles_gu ? L.shared_tiled : L.shared_packed,
                                     tiles_gu ? m->tiled_stride() : m->fused ? m->packed_stride : m->expert_stride, tiles_gu ? m->pk_gate_bytes : m->gate_bytes, m->gu_grid};
-            const StagedChunk chunk{m->pair_token, tl, ntok, c.top_k, c.n_expert};
+            const StagedChunk chunk{m->pair_token, tl, ntok, c.top_k, c.n_expert, kWideUnknown, ntok <= Moe::kSmallMaxRouted};
             if (!gu.experts) { moe_err("internal: no rows for the tile kernels (layer %u)", layer); return 0; }
             HIP_OK(launch_staged_gateup(gu, chunk, m->xh, m->xl, m->xexp, m->act, c.hidden, c.ffn, s), "gate/up tile launch");
             const uint8_t *dn_rows = m->fused ? (tiles_dn ? L.tiled : L.packed) + 2u * m->gate_bytes : tiles_dn ? L.tiled_down : L.experts ? L.experts + 2u * m->gate_bytes : nullptr;

@@ -97,7 +97,7 @@ template <int SRC, int SETS, uint32_t KP> struct GateUpLds {
 };
 
 // units u0 .. u1 - 1 (unit = tile * units per tile + unit of the tile) of a tile list
-template <int SRC, int SETS, uint32_t KP>
+template <int SRC, int SETS, uint32_t KP, bool SHORT>
 __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList &list, uint32_t u0, uint32_t u1, GateUpLds<SRC, SETS, KP> &lds, bool tables) {
     using G = GateUp<SETS, KP>;
     constexpr uint32_t PK = G::PK, NRT = G::NRT, K = 256u * KP, PAIRS = 16u * SETS, T = kGateUpThreads, UB = G::kUnits;
@@ -126,10 +126,10 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
     };
     // Precision. The matrix unit rounds a sum four times per instruction (once per eight products), so what a block's sum loses goes with the
     // length of its chain of instructions: the low halves have a chain of their own, and the high ones one per kChain steps, added up in f32.
-    // Narrow tiles also take batches whose fewer tokens are slices (which stop rounding after four instructions), and are no further off than these: with
-    // chains of four steps 1.87e-7 against 1.76e-7 (IQ2_XXS, 2048 x 512, 24 tokens with the routing given), with two and the low halves first 1.74e-7,
-    // at 1 % of a chunk's time; chains of one step lose more in the additions (1.78e-7 against 1.77e-7).
-    constexpr uint32_t kChain = SETS == 1 || layout<SRC>() == L_ROWS ? 2u : 4u;
+    // (SHORT: of two steps.) The low halves go first into a result, so that it is rounded once for both. Of a chunk 1.82e-7 is lost so, 1.74e-7 with short
+    // chains, in 1 to 2 % more time; batches of fewer tokens are slices, which lose 1.76e-7, so these have short ones and are no further off on the
+    // tiles (IQ2_XXS, 2048 x 512, 24 tokens with the routing given; chains of one step lose more in the additions).
+    constexpr uint32_t kChain = SHORT || layout<SRC>() == L_ROWS ? 2u : 4u;
     H8 xa[2][8], xb[2][8];                                 // SETS 1: [block], SETS 2: [set]
     const auto load_tile = [&](uint32_t tile) {
 #pragma unroll
@@ -236,7 +236,6 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
                 for (uint32_t m = 0; m < 2u; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[SETS == 1 ? m : s][S].v, w[m], low[m][s], 0, 0, 0);
         });
         float *mine = pt + (rt * PK + kp) * G::kSums + 4u * lane;
-        // (the low halves' sums first: what they and the high ones' leave in a result is then rounded once, not twice)
         if constexpr (SETS == 1) {
             float4_t &both = acc[0][0];                    // the two blocks
 #pragma unroll
@@ -530,7 +529,7 @@ template <int SRC, int SETS, uint32_t KP> constexpr int down_src() { return SETS
 template <int SRC, bool DOWN, uint32_t KP> uint32_t few_wide(uint32_t rows, uint32_t K) {
     return !has_wide<SRC, DOWN, KP>() ? ~0u : (DOWN ? 200000000u : 145000000u) / (rows * K) + 1u;
 }
-template <int SRC, bool DOWN, int SETS, uint32_t KP>
+template <int SRC, bool DOWN, int SETS, uint32_t KP, bool SHORT>
 __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) void staged_tiles_kernel(StagedArgs a) {
     __shared__ __attribute__((aligned(16))) std::conditional_t<DOWN, DownLds<down_src<SRC, SETS, KP>(), SETS, KP>, GateUpLds<SRC, SETS, KP>> lds;
     static_assert(sizeof(lds) <= 160u * 1024u, "what a compute unit has");
@@ -554,39 +553,41 @@ __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) v
         const uint32_t to = min(w1, (from / per_tile + kTileInfos) * per_tile);
         if (from != w0) __syncthreads();
         if constexpr (DOWN) down_items<down_src<SRC, SETS, KP>(), SETS, KP>(a, list, per_tile, from, to, lds, from == w0);
-        else gateup_units<SRC, SETS, KP>(a, list, from, to, lds, from == w0);
+        else gateup_units<SRC, SETS, KP, SHORT>(a, list, from, to, lds, from == w0);
         from = to;
     }
 }
 
-template <int SRC, bool DOWN, int SETS, uint32_t KP>
+template <int SRC, bool DOWN, int SETS, uint32_t KP, bool SHORT = false>
 hipError_t launch_staged_list(const StagedArgs &a, uint32_t grid, hipStream_t s) {
-    REDHIP_LAUNCH((staged_tiles_kernel<SRC, DOWN, SETS, KP>), dim3(grid), dim3(DOWN ? 64u * down_waves(SETS) : kGateUpThreads), 0, s, a);
+    REDHIP_LAUNCH((staged_tiles_kernel<SRC, DOWN, SETS, KP, SHORT>), dim3(grid), dim3(DOWN ? 64u * down_waves(SETS) : kGateUpThreads), 0, s, a);
     return hipGetLastError();
 }
-// wide: wide tiles that the chunk is expected to have
+// wide: wide tiles that the chunk is expected to have; batch: it has so few tokens that still fewer would be slices
 template <int SRC, bool DOWN, uint32_t KP>
-hipError_t launch_staged_lists(StagedArgs a, uint32_t grid, uint32_t wide, hipStream_t s) {
+hipError_t launch_staged_lists(StagedArgs a, uint32_t grid, uint32_t wide, bool batch, hipStream_t s) {
     a.few = few_wide<SRC, DOWN, KP>(a.rows, 256u * KP);
     hipError_t e = hipSuccess;
     if (wide < a.few) a.few = ~0u;                         // (without a wide launch the narrow one takes everything)
     if constexpr (has_wide<SRC, DOWN, KP>()) {
         if (a.few != ~0u) e = launch_staged_list<SRC, DOWN, 2, KP>(a, grid, s);
     }
+    if constexpr (!DOWN && layout<SRC>() == L_TILED && KP >= 4u)
+        if (batch) return e == hipSuccess ? launch_staged_list<SRC, DOWN, 1, KP, true>(a, grid, s) : e;
     return e == hipSuccess ? launch_staged_list<SRC, DOWN, 1, KP>(a, grid, s) : e;
 }
 template <int SRC>
-hipError_t staged_gateup(const StagedArgs &a, uint32_t hidden, uint32_t grid, uint32_t wide, hipStream_t s) {
-    return hidden == 512u    ? launch_staged_lists<SRC, false, 2>(a, grid, wide, s)
-           : hidden == 1024u ? launch_staged_lists<SRC, false, 4>(a, grid, wide, s)
-                             : launch_staged_lists<SRC, false, 8>(a, grid, wide, s);
+hipError_t staged_gateup(const StagedArgs &a, uint32_t hidden, uint32_t grid, uint32_t wide, bool batch, hipStream_t s) {
+    return hidden == 512u    ? launch_staged_lists<SRC, false, 2>(a, grid, wide, batch, s)
+           : hidden == 1024u ? launch_staged_lists<SRC, false, 4>(a, grid, wide, batch, s)
+                             : launch_staged_lists<SRC, false, 8>(a, grid, wide, batch, s);
 }
 template <int SRC>
 hipError_t staged_down(const StagedArgs &a, uint32_t ffn, uint32_t grid, uint32_t wide, hipStream_t s) {
-    if (ffn == 256u) return launch_staged_lists<SRC, true, 1>(a, grid, wide, s);
-    if (ffn == 512u) return launch_staged_lists<SRC, true, 2>(a, grid, wide, s);
+    if (ffn == 256u) return launch_staged_lists<SRC, true, 1>(a, grid, wide, false, s);
+    if (ffn == 512u) return launch_staged_lists<SRC, true, 2>(a, grid, wide, false, s);
     if constexpr (layout<SRC>() == L_TILED) return hipErrorInvalidValue;      // (tile-major copies are made for ffn <= 512)
-    else return ffn == 768u ? launch_staged_lists<SRC, true, 3>(a, grid, wide, s) : launch_staged_lists<SRC, true, 4>(a, grid, wide, s);
+    else return ffn == 768u ? launch_staged_lists<SRC, true, 3>(a, grid, wide, false, s) : launch_staged_lists<SRC, true, 4>(a, grid, wide, false, s);
 }
 
 int staged_src(uint32_t type, RowLayout lay) {
@@ -649,13 +650,13 @@ hipError_t launch_staged_gateup(const StagedMatrices &m, const StagedChunk &c, c
     const uint32_t wide = staged_wide(c);
     prof_set_stage(ST_PREFILL_GATEUP);
     switch (staged_src(m.type, m.layout)) {
-        case S_XXS: return staged_gateup<S_XXS>(a, hidden, grid, wide, s);
-        case S_XS: return staged_gateup<S_XS>(a, hidden, grid, wide, s);
-        case S_M: return staged_gateup<S_M>(a, hidden, grid, wide, s);
-        case S_ROWS_XXS: return staged_gateup<S_ROWS_XXS>(a, hidden, grid, wide, s);
-        case S_TILED_XXS: return staged_gateup<S_TILED_XXS>(a, hidden, grid, wide, s);
-        case S_TILED_XS: return staged_gateup<S_TILED_XS>(a, hidden, grid, wide, s);
-        case S_TILED_M: return staged_gateup<S_TILED_M>(a, hidden, grid, wide, s);
+        case S_XXS: return staged_gateup<S_XXS>(a, hidden, grid, wide, c.batch, s);
+        case S_XS: return staged_gateup<S_XS>(a, hidden, grid, wide, c.batch, s);
+        case S_M: return staged_gateup<S_M>(a, hidden, grid, wide, c.batch, s);
+        case S_ROWS_XXS: return staged_gateup<S_ROWS_XXS>(a, hidden, grid, wide, c.batch, s);
+        case S_TILED_XXS: return staged_gateup<S_TILED_XXS>(a, hidden, grid, wide, c.batch, s);
+        case S_TILED_XS: return staged_gateup<S_TILED_XS>(a, hidden, grid, wide, c.batch, s);
+        case S_TILED_M: return staged_gateup<S_TILED_M>(a, hidden, grid, wide, c.batch, s);
     }
     return hipErrorInvalidValue;
 }

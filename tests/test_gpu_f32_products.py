@@ -41,6 +41,21 @@ def test_logits(hidden, n_expert, tokens):
     m.close()
 
 
+@pytest.mark.parametrize("hidden,outweigh", [(512, 1.0), (2048, 1.0), (512, 1e5), (2048, 1e5)])
+def test_terms_are_rounded(hidden, outweigh):
+    """Terms that are cut instead of rounded leave out products that all have the sign of the whole: sums come out 3e-8 .. 4e-8 too small in magnitude
+    (the products left out, by themselves; rounded 1e-10), which a bound on the error itself does not see. Rounding errors of either sign, 1e-7 of each of
+    513 x 256 outputs (a token's share one factor where a product outweighs the rest), leave less than 1e-8 of a mean."""
+    m, rows = layer(hidden, 256)
+    x = synth.normed_x(np.random.default_rng(9), 513, hidden)
+    x[:, 11] *= np.float32(outweigh)
+    logits, want = m.route(0, torch.from_numpy(x).cuda())[2].cpu().numpy(), x.astype(np.float64) @ rows.T.astype(np.float64)
+    bias = ((logits - want) * np.sign(want)).mean() / np.abs(want).mean()
+    print("%d columns, outweighed %g: %.1e" % (hidden, outweigh, bias))
+    assert abs(bias) <= 1e-8
+    m.close()
+
+
 @pytest.mark.parametrize("shift", [1, 2, 3])
 def test_activations_at_any_float(shift):
     m, rows = layer(1024, 48)

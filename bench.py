@@ -6,7 +6,7 @@ A step is one pass of the hot path over one batch: router GEMV -> softmax top-k 
 (distinct weights, so the 256 MB Infinity Cache cannot hold the working set) and through a pool of activations, so
 the router picks different experts every step. Inputs are resident in HBM before the timed region starts.
 
-Prints one JSON line (metric: microseconds per token for one MoE layer; lower is better), with
+Prints one JSON line (metric: microseconds per token for one MoE layer; lower is better; of the sweeps the times, --details FILE has the rest), with
   roofline       the dominant kernel's algorithmic bytes per launch / its measured launch duration, vs 8 TB/s
   cpu_baseline   the CPU oracle (a port of the reference's scalar double-accumulating path) on this host's cores
   batch_sweep    the ragged small batches (B = 2, 4, 8): drawn hot routing as an input, and the layer's own router
@@ -36,6 +36,45 @@ HBM_PEAK_GBS = 8000.0
 MFMA_F16_PEAK_TFLOPS = 2500.0
 
 
+def short_line(result):
+    """The record with every sweep entry cut down to its time (and error): a line that a log's last 6 KB hold whole."""
+    def step(e):
+        return "%s%d %s" % (e["layout"] + " " if "layout" in e else "", e["batch"], e["routing"])
+
+    def chunk(e):
+        return "%s %d %s" % (e["layout"], e["tokens"], e["routing"])
+
+    def steps(entries):
+        return {step(e): e["us_per_step"] for e in entries}
+    out, errors = {}, []
+    for k, v in result.items():
+        if k == "batch_sweep" or k == "mid_sweep":
+            errors += [e["rel_l2_vs_cpu_oracle"] for e in v]
+            out[k] = {"us_per_step": steps(v)}
+        elif k.endswith("_sweep") and "runs" in v:
+            errors += [e["rel_l2_vs_cpu_oracle"] for e in v["runs"]]
+            out[k] = {"us_per_step": steps(v["runs"])}
+        elif k == "prefill_sweep":
+            errors += [e["rel_l2_vs_cpu_oracle"] for e in v]
+            out[k] = {"us_per_chunk": {chunk(e): e["us_per_chunk"] for e in v}, "gateup_tflops": {chunk(e): (e["roofline"] or {}).get("achieved") for e in v}}
+        elif k == "stack":
+            errors += [e["rel_l2_vs_cpu_oracle_layer0_block"] for e in v]
+            out[k] = {"us_per_token": {e["layout"]: e["us_per_token"] for e in v}, "gbps": {e["layout"]: e["gbps"] for e in v}}
+        elif k == "yardsticks":
+            out[k] = {"streaming_read_gbps": v["streaming_read"]["gbps"], "copy_gbps": v["copy"]["gbps_in_plus_out"], "mfma_f16_tflops": v["mfma_f16_16x16x32"]["tflops"]}
+        elif k == "microbench":
+            out[k] = {n: {f: x for f, x in e.items() if f != "note"} for n, e in v.items()}
+        elif k == "topk_pool":
+            def pool(e):
+                return {m: {f: x for f, x in e[m].items() if f.endswith("_us")} for m in ("raw", "fast") if m in e}
+            out[k] = dict(pool(v), **({"iq2_xs_experts": pool(v["iq2_xs_experts"])} if "iq2_xs_experts" in v else {}))
+        elif k != "launch_floor_note":
+            out[k] = v
+    if errors:
+        out["parity"] = dict(out["parity"], largest_rel_l2_of_the_sweeps=max(errors))
+    return out
+
+
 def parse():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -62,6 +101,7 @@ def parse():
     ap.add_argument("--prefill-layers", type=int, default=8, help="resident layers of the chunk handles (a chunk reads about 0.4 GB of experts per layer)")
     ap.add_argument("--no-yardsticks", action="store_true", help="skip the streaming-read and matrix-core yardsticks")
     ap.add_argument("--no-pool", action="store_true", help="skip the file-backed top-k pool entries that the default run appends")
+    ap.add_argument("--details", metavar="FILE", help="also write the whole record (stages, bytes, rooflines and errors of every sweep entry) to FILE")
     ap.add_argument("--prime", type=int, default=2000, help="untimed steps before the warm-up that bring the clocks up (reported as clock_priming_steps)")
     return ap.parse_args()
 
@@ -767,7 +807,10 @@ def main():
                                   "sample": "%d forwards of layer 0 (same weights and activations as the GPU run), rows split over %d pthreads "
                                             "per matvec like the reference; 1 thread: %.0f us/token" % (reps, cores, one_us),
                                   "gpu_speedup": round(cpu_us / us_per_token, 1)}
-    print(json.dumps(result))
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(result, f, indent=1)
+    print(json.dumps(short_line(result)))
     moe.close()
 
 

@@ -24,6 +24,13 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t b, uint32_t c) {
 // bits of w, those at position `from` moved to `to`
 template <uint32_t FROM, uint32_t TO> __device__ __forceinline__ uint32_t moved(uint32_t w) { return FROM >= TO ? w >> (FROM >= TO ? FROM - TO : 0u) : w << (FROM < TO ? TO - FROM : 0u); }
 
+// a barrier that waits for LDS only: loads and stores of device memory stay in flight
+__device__ __forceinline__ void wave_lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // power-of-two pre-scale: largest |v| lands in [2^13, 2^14); beside an infinity every finite value stays below 2^13
 __device__ __forceinline__ int prescale_exp(float amax) {
     if (!(amax > 0.0f)) return 0;

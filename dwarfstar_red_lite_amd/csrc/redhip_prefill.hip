@@ -345,7 +345,7 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
     meet([&](int mm, int tt) { return high[0][mm][tt] + high[1][mm][tt] + low[mm][tt]; });
     if (which) which = store(which, false);
     if (which) again = 1u;
-    __syncthreads();
+    wave_lds_barrier();                                    // (not for the stores)
     if (!again) return;
     // the tile once more on the fp32 unit, for the others
     float4_t sum[MR][MT];

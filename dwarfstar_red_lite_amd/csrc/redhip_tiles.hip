@@ -44,12 +44,6 @@ struct StagedArgs {
     uint32_t few;                          // wide tiles that are not worth a launch: fewer than this many
 };
 
-__device__ __forceinline__ void wave_lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 // exchange of two registers' halves between lanes that differ in bit 4 (16) or 5 (32)
 __device__ __forceinline__ void swap16(uint32_t &a, uint32_t &b) { const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false); a = r[0]; b = r[1]; }
 __device__ __forceinline__ void swap32(uint32_t &a, uint32_t &b) { const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false); a = r[0]; b = r[1]; }

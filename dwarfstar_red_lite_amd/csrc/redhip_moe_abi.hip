@@ -143,7 +143,7 @@ struct Moe {
     static constexpr uint32_t kSmallMaxFused = 16u, kSmallMaxRouted = 32u, kSmallMaxGiven = 24u, kSmallMaxMixed = 32u;
     // ... unless the tiles are ahead from fewer tokens on. Per layer the slices cost so many us per pass of two pairs of an expert, and per token (the shared
     // expert, on mixed layouts also the router), the tiles so many per distinct expert, each more for larger matrices, and their launches more than the
-    // slices': both by the tokens' expected spread over the experts. Fitted to 2052 calls timed on both sides: 17 .. 32 tokens, 16 to 512 experts,
+    // slices': both by the tokens' expected spread over the experts. Fitted to 1332 calls timed on both sides: 17 .. 32 tokens, 16 to 512 experts,
     // two to ten a token, 1024 x 512 to 2048 x 768, own router and routing given (that call does not know how it is spread: a line between even
     // spread and 32 hot experts). Chosen so, a call is 0.4 % slower than on the quicker side on average. Slices / tiles, us:
     // own router, 32 tokens of 2048 x 512: 512 experts, ten a token: IQ2_XXS 122 / 112, IQ1_M 135 / 111; four a token 74 / 81 and 84 / 78; 60 experts, two a

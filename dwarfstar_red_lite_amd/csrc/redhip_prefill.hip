@@ -101,7 +101,7 @@ hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count
 
 // out[tok][row] = W[row] . x[tok] for an f32 matrix W (a router, the dense shared expert of mixed layouts) and a chunk of activations. Every f32
 // is the sum of three bf16 numbers, exactly (the nearest one, the nearest to the rest, and what is left), and of the
-// nine products of such sums the six that reach 2^-24 of the largest go through v_mfma_f32_16x16x32_bf16: six of those are 96 cycles for 32 columns
+// nine products of such sums (a published way to f32 products: Henry, Tang, Heinecke, ARITH 2019) the six that reach 2^-24 of the largest go through v_mfma_f32_16x16x32_bf16: six of those are 96 cycles for 32 columns
 // where the fp32 unit takes 256. The products of the leading terms have accumulators of their own, the other five share one.
 // A workgroup owns BR = 16 MR rows x BT = 16 MT tokens, each of its eight waves an eighth of k for all of them; the eight sums meet in LDS, in
 // double. A wave fetches 32 columns of every row and token straight into LDS (full 128-byte lines: sixteen lanes of a load that name sixteen rows

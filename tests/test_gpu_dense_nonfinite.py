@@ -64,7 +64,8 @@ def test_leading_terms_that_overflow(n, given):
     m.close()
 
 
-def test_infinite_and_nan_tokens():
+@pytest.mark.parametrize("shift", [0, 1])      # (activations at any float: fetched by another way)
+def test_infinite_and_nan_tokens(shift):
     cfg, lay = shared_only_layer(53)
     n = 600
     m = ResidentMoe(cfg, n_layer=1, max_tokens=n)
@@ -73,7 +74,10 @@ def test_infinite_and_nan_tokens():
     plain = m.forward(0, torch.from_numpy(x).cuda()).cpu().numpy()
     y = x.copy()
     y[7, 300], y[41, 20], y[599, 511] = np.nan, np.inf, -np.inf
-    got = m.forward(0, torch.from_numpy(y).cuda()).cpu().numpy()
+    room = torch.zeros(n * H + 1, device="cuda")
+    at = room[shift:shift + n * H].reshape(n, H)
+    at.copy_(torch.from_numpy(y))
+    got = m.forward(0, at).cpu().numpy()
     rest = [t for t in range(n) if t not in (7, 41, 599)]
     assert np.array_equal(got[rest], plain[rest]) and not np.isfinite(got[[7, 41, 599]]).any()
     m.close()

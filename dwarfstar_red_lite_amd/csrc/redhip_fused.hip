@@ -1749,7 +1749,9 @@ __device__ __forceinline__ void signed_weights_lut(const LaneTables &t, uint2 q,
     constexpr uint32_t kLutShift = LR == 8 ? 5u : LR == 16 ? 6u : 7u;      // log2 of the bytes per sign field
     // bytes of the magnitude address: [low byte of the lane's base, index byte L of q.x, upper two bytes of the lane's base]
     const uint32_t mag_at = __builtin_amdgcn_perm(q.x, t.mag_lane, 0x03020000u | ((4u + L) << 8));
-    const uint32_t lut_at = and_or(moved<7u * L, kLutShift>(q.y), t.lut_mask, t.lut_lane);
+    // one token (LR 32) waits for its chain, and and_or adds to it: masks as literals there (12.6 .. 12.9 us a pool call instead of 12.8 .. 13.0)
+    constexpr bool kChain = LR == 32;
+    const uint32_t field = moved<7u * L, kLutShift>(q.y), lut_at = kChain ? (field & (127u << kLutShift)) | t.lut_lane : and_or(field, t.lut_mask, t.lut_lane);
 #ifdef REDHIP_ABLATE_NO_LDS      // measurement builds only (build.py --ablate): the table reads replaced by register moves, results wrong
     const lds_u32x4 m = {mag_at, lut_at, mag_at ^ 0x1234u, lut_at + 7u};
     const uint32_t e = lut_at ^ mag_at;
@@ -1760,11 +1762,12 @@ __device__ __forceinline__ void signed_weights_lut(const LaneTables &t, uint2 q,
 #ifdef REDHIP_ABLATE_NO_SIGN     // ... the sign placement left out
     b0.u[0] = m.x ^ e; b0.u[1] = m.y; b1.u[0] = m.z; b1.u[1] = m.w;
 #else
-    const uint32_t e1 = twice(e), e2 = e << 2, e3 = twice(e2);      // (three doublings in a row are 0.3 % of a decode step: it waits for its chain)
-    b0.u[0] = and_or(e, t.sign_bits, m.x);
-    b0.u[1] = and_or(e1, t.sign_bits, m.y);
-    b1.u[0] = and_or(e2, t.sign_bits, m.z);
-    b1.u[1] = and_or(e3, t.sign_bits, m.w);
+    const uint32_t e1 = kChain ? e << 1 : twice(e), e2 = e << 2, e3 = kChain ? e << 3 : twice(e2);
+    const auto place = [&](uint32_t signs, uint32_t m4) { return kChain ? (signs & 0x80008000u) | m4 : and_or(signs, t.sign_bits, m4); };
+    b0.u[0] = place(e, m.x);
+    b0.u[1] = place(e1, m.y);
+    b1.u[0] = place(e2, m.z);
+    b1.u[1] = place(e3, m.w);
 #endif
 }
 template <int REP, int LR, uint32_t L>

@@ -295,8 +295,8 @@ __global__ __launch_bounds__(512) void f32_tiles_kernel(const float *w, const fl
         if (step + 1u < steps) multiply(step + 1u, std::integral_constant<int, 1>{});
     }
     // a thread: four consecutive rows of a token (D[i = 4q .. 4q + 3][j = r])
-    const uint32_t t = (tid >> 6) % MT, m = (tid >> 6) / MT, l = tid & 63u, tok = tile_t * BT + 16u * t + (l & 15u), row = 4u * (l >> 4);
-    const bool has = tid < (swiglu ? MR / 2u : MR) * MT * 64u && tok < ntok;
+    const uint32_t at = each_trip(tid), t = (at >> 6) % MT, m = (at >> 6) / MT, l = at & 63u, tok = tile_t * BT + 16u * t + (l & 15u), row = 4u * (l >> 4);      // (nothing of it in front of the first request)
+    const bool has = at < (swiglu ? MR / 2u : MR) * MT * 64u && tok < ntok;
     static_assert(MR * MT * 64u <= 512u, "four outputs a thread");
     const auto meet = [&](auto part) {                     // the waves' sums in LDS
         __syncthreads();

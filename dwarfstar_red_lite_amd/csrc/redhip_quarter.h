@@ -45,78 +45,117 @@ template <int SRC> constexpr uint32_t sign_shift() { return sign_copies<SRC>() =
 template <int SRC> constexpr uint32_t sign_bytes() { return (is_iq3<SRC>() ? 256u : 128u) * sign_copies<SRC>() * 4u; }
 constexpr uint32_t kEntryBytes = 65536u;
 
-__device__ __forceinline__ uint32_t two_halves(float lo, float hi) {
-    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
+template <int SRC> constexpr uint32_t codebook_entries() { return fmt<SRC>() == F_XXS ? 256u : fmt<SRC>() == F_M ? 2048u : 512u; }
+
+// Bytes B and B + 1 of w as two fp16 halves: 1024 + byte by a permute (100 0100 of the exponent above it), minus 1024, exact. Signed bytes: flipped to
+// 0 .. 255 before, minus another 128.
+template <uint32_t B, bool SIGNED> __device__ __forceinline__ half2_t byte_halves(uint32_t w) {
+    const half2_t v = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, SIGNED ? w ^ 0x80808080u : w, 0x04000400u | B | ((B + 1u) << 16)));
+    constexpr _Float16 off = SIGNED ? 1152.0f : 1024.0f;
+    return v - half2_t{off, off};
+}
+template <bool SIGNED> __device__ __forceinline__ H8 entry_halves(uint64_t e) {
+    H8 r;
+    r.p[0] = byte_halves<0u, SIGNED>((uint32_t)e);
+    r.p[1] = byte_halves<2u, SIGNED>((uint32_t)e);
+    r.p[2] = byte_halves<0u, SIGNED>((uint32_t)(e >> 32));
+    r.p[3] = byte_halves<2u, SIGNED>((uint32_t)(e >> 32));
+    return r;
+}
+__device__ __forceinline__ half2_t odd_halves(uint32_t s) {      // 2 s + 1 twice, exact
+    const half2_t big = __builtin_bit_cast(half2_t, (0x6401u + 2u * s) * 0x10001u);
+    return big - half2_t{(_Float16)1024.0f, (_Float16)1024.0f};
 }
 
 template <int SRC, uint32_t T>          // by T threads
 __device__ __forceinline__ void build_signs(uint32_t *signs, uint32_t tid) {
     if constexpr (fmt<SRC>() != F_M) {
-        constexpr uint32_t R = sign_copies<SRC>(), N = sign_bytes<SRC>() / 4u;
+        constexpr uint32_t R = sign_copies<SRC>(), W = R < 4u ? R : 4u, N = sign_bytes<SRC>() / (4u * W);      // W copies a store
         for (uint32_t i = tid; i < N; i += T) {
-            const uint32_t s = i / R, s8 = is_iq3<SRC>() ? s : s | ((__popc(s) & 1u) << 7);
-            uint32_t w = 0u;
-#pragma unroll
-            for (uint32_t k = 0; k < 4u; ++k) w |= (((s8 >> (2u * k)) & 1u) << (15u - k)) | (((s8 >> (2u * k + 1u)) & 1u) << (31u - k));
-            signs[i] = w;
+            const uint32_t s = i * W / R, s8 = is_iq3<SRC>() ? s : s | ((__popc(s) & 1u) << 7);
+            uint32_t y = ((s8 >> 1) & 0x55u) | ((s8 & 0x55u) << 16);      // odd weights' signs in the low half, even ones' in the high half, side by side, then in reverse
+            y = (y | (y >> 1)) & 0x00330033u;
+            y = (y | (y >> 2)) & 0x000f000fu;
+            const uint32_t w = __brev(y);
+            if constexpr (W == 4u) reinterpret_cast<uint4 *>(signs)[i] = make_uint4(w, w, w, w);
+            else reinterpret_cast<uint2 *>(signs)[i] = make_uint2(w, w);
         }
     }
 }
 
+// The large tables, by T threads: a thread's codebook entries are requested together (a trip to memory), every further one is packed fp16 arithmetic, exact.
+// Where a thread writes four entries side by side, in an order that differs between the fours of lanes: sixteen lanes then write to different
+// banks. (Entry by entry in f32, each behind a trip of its own, the tables of IQ2_XXS took 8000 cycles of every launch, 20000 of the 91000 of a batch
+// of 24 tokens until the first products with what waits for them.)
 template <int SRC, uint32_t T>
 __device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *signs, uint32_t tid, const int8_t *grid) {
-    if constexpr (fmt<SRC>() == F_XXS) {
-        for (uint32_t e4 = tid; e4 < 4u * 256u; e4 += T) {
-            const uint64_t ge = redhip_iq2xxs_grid[e4 >> 2];
+    if constexpr (fmt<SRC>() == F_XXS || fmt<SRC>() == F_XS) {
+        constexpr uint32_t PER = fmt<SRC>() == F_XXS ? 4u : 2u, kItems = PER * codebook_entries<SRC>(), N = (kItems + T - 1u) / T;      // four scales or copies each
+        uint64_t ge[N];
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n) {
+            const uint32_t e = min(tid + n * T, kItems - 1u) / PER;      // (surplus threads repeat the last)
+            if constexpr (fmt<SRC>() == F_XXS) ge[n] = redhip_iq2xxs_grid[e];
+            else ge[n] = reinterpret_cast<const uint64_t *>(grid)[e];
+        }
+        build_signs<SRC, T>(signs, tid);
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n) {
+            const uint32_t i = min(tid + n * T, kItems - 1u);
+            const H8 base = entry_halves<fmt<SRC>() == F_XS>(ge[n]);
 #pragma unroll
             for (uint32_t k = 0; k < 4u; ++k) {
-                const uint32_t e = 4u * e4 + k;
-                const float f = (float)(2u * (e & 15u) + 1u);
-                uint32_t w4[4];
+                const uint32_t at = 4u * i + ((k + (i >> 2)) & 3u);
+                H8 v = base;
+                if constexpr (fmt<SRC>() == F_XXS) {
+                    const half2_t f = odd_halves(at & 15u);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) w4[i] = two_halves(f * (float)((uint32_t)(ge >> (16 * i)) & 255u), f * (float)((uint32_t)(ge >> (16 * i + 8)) & 255u));
-                *reinterpret_cast<uint4 *>(entries + (size_t)e * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+                    for (int p = 0; p < 4; ++p) v.p[p] = base.p[p] * f;
+                }
+                *reinterpret_cast<uint4 *>(entries + at * 16u) = v.u;
             }
         }
     } else if constexpr (fmt<SRC>() == F_M) {
-        for (uint32_t e = tid; e < 2048u; e += T) {
-            const uint64_t ge = reinterpret_cast<const uint64_t *>(grid)[e];
+        constexpr uint32_t kItems = codebook_entries<SRC>(), N = (kItems + T - 1u) / T;
+        uint64_t ge[N];
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n) ge[n] = reinterpret_cast<const uint64_t *>(grid)[min(tid + n * T, kItems - 1u)];
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n) {
+            const uint32_t i = min(tid + n * T, kItems - 1u);
+            const H8 base = entry_halves<true>(ge[n]);
 #pragma unroll
             for (uint32_t neg = 0; neg < 2u; ++neg) {
-                const float off = neg ? -0.125f : 0.125f;      // (exact: a byte and three bits behind the point)
-                uint32_t w4[4];
+                const _Float16 off = neg ? -0.125f : 0.125f;      // (exact: a byte and three bits behind the point)
+                H8 v;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) w4[i] = two_halves((float)(int8_t)(ge >> (16 * i)) + off, (float)(int8_t)(ge >> (16 * i + 8)) + off);
-                *reinterpret_cast<uint4 *>(entries + neg * 32768u + e * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+                for (int p = 0; p < 4; ++p) v.p[p] = base.p[p] + half2_t{off, off};
+                *reinterpret_cast<uint4 *>(entries + neg * 32768u + i * 16u) = v.u;
             }
         }
-    } else if constexpr (fmt<SRC>() == F_XS) {
-        constexpr uint32_t kCopies = 8u, kEntries = kEntryBytes / (16u * kCopies);
-        for (uint32_t e = tid; e < kEntries; e += T) {
-            const uint64_t ge = reinterpret_cast<const uint64_t *>(grid)[e];
-            uint32_t w4[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) w4[i] = two_halves((float)(int8_t)(ge >> (16 * i)), (float)(int8_t)(ge >> (16 * i + 8)));
-            for (uint32_t c = 0; c < kCopies; ++c) *reinterpret_cast<uint4 *>(entries + ((size_t)e * kCopies + c) * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
-        }
     } else {
-        for (uint32_t i = tid; i < 2u * 512u; i += T) {      // (an entry's request is a trip to memory: eight scales for each)
-            const uint32_t gw = redhip_iq3s_grid[i & 511u];
+        constexpr uint32_t kItems = 2u * 512u, N = (kItems + T - 1u) / T;      // eight scales each
+        uint32_t gw[N];
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n) gw[n] = redhip_iq3s_grid[min(tid + n * T, kItems - 1u) & 511u];
+        build_signs<SRC, T>(signs, tid);
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n) {
+            const uint32_t i = min(tid + n * T, kItems - 1u);
+            const half2_t a = byte_halves<0u, false>(gw[n]), b = byte_halves<2u, false>(gw[n]);
 #pragma unroll
             for (uint32_t k = 0; k < 8u; ++k) {
                 const uint32_t scale = (i >> 9) * 8u + k;
-                const float f = (float)(1u + 2u * scale);
-                *reinterpret_cast<uint2 *>(entries + (size_t)(scale * 512u + (i & 511u)) * 8u) =
-                    make_uint2(two_halves(f * (float)(gw & 255u), f * (float)((gw >> 8) & 255u)), two_halves(f * (float)((gw >> 16) & 255u), f * (float)(gw >> 24)));
+                const half2_t f = odd_halves(scale);
+                *reinterpret_cast<uint2 *>(entries + (scale * 512u + (i & 511u)) * 8u) =
+                    make_uint2(__builtin_bit_cast(uint32_t, a * f), __builtin_bit_cast(uint32_t, b * f));
             }
         }
     }
-    build_signs<SRC, T>(signs, tid);
 }
 
 // The small tables, by T threads in two parts: a thread's codebook entries are requested (before the rows, which the second part must not
 // wait for), then written. Tables with copies are written by two threads per entry, half of the copies each.
-template <int SRC> constexpr uint32_t codebook_entries() { return fmt<SRC>() == F_XXS ? 256u : fmt<SRC>() == F_M ? 2048u : 512u; }
 template <int SRC> constexpr uint32_t small_copies() { return fmt<SRC>() == F_XXS ? 8u : fmt<SRC>() == F_M ? 1u : 4u; }
 template <int SRC> constexpr uint32_t entry_shift() { return !small_tables<SRC>() ? (fmt<SRC>() == F_M ? 4u : 7u) : fmt<SRC>() == F_XXS ? 7u : fmt<SRC>() == F_XS ? 6u : fmt<SRC>() == F_M ? 4u : 5u; }
 template <int SRC> constexpr uint32_t small_entry_bytes() { return codebook_entries<SRC>() << entry_shift<SRC>(); }
@@ -138,19 +177,13 @@ template <int SRC, uint32_t T> struct SmallSeeds {
         for (uint32_t n = 0; n < N; ++n) {
             const uint32_t i = min(tid + n * T, kItems - 1u), first = ((i / kHalves) * kCopies + (i % kHalves) * kMine);      // (surplus threads repeat the last)
             if constexpr (is_iq3<SRC>()) {
-                const uint32_t g = (uint32_t)e[n];
-                const uint2 v = make_uint2(two_halves((float)(g & 255u), (float)((g >> 8) & 255u)), two_halves((float)((g >> 16) & 255u), (float)(g >> 24)));
+                const uint2 v = make_uint2(__builtin_bit_cast(uint32_t, byte_halves<0u, false>((uint32_t)e[n])), __builtin_bit_cast(uint32_t, byte_halves<2u, false>((uint32_t)e[n])));
 #pragma unroll
                 for (uint32_t c = 0; c < kMine; ++c) *reinterpret_cast<uint2 *>(entries + (size_t)(first + c) * 8u) = v;
             } else {
-                uint32_t w4[4];
+                const H8 v = entry_halves<fmt<SRC>() != F_XXS>(e[n]);
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if constexpr (fmt<SRC>() == F_XXS) w4[k] = two_halves((float)((uint32_t)(e[n] >> (16 * k)) & 255u), (float)((uint32_t)(e[n] >> (16 * k + 8)) & 255u));
-                    else w4[k] = two_halves((float)(int8_t)(e[n] >> (16 * k)), (float)(int8_t)(e[n] >> (16 * k + 8)));
-                }
-#pragma unroll
-                for (uint32_t c = 0; c < kMine; ++c) *reinterpret_cast<uint4 *>(entries + (size_t)(first + c) * 16u) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+                for (uint32_t c = 0; c < kMine; ++c) *reinterpret_cast<uint4 *>(entries + (size_t)(first + c) * 16u) = v.u;
             }
         }
         build_signs<SRC, T>(signs, tid);

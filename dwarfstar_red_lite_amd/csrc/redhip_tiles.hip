@@ -133,9 +133,10 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
             const uint64_t base = (uint64_t)tok * K + 256u * (SETS == 1 ? 2u * kp + x : kp) + 8u * q;
             const _Float16 *hp = a.xh + base, *lp = a.xl + base;
             // four lanes of a pair take 64 bytes side by side; the exchange makes them each lane's own run
+            // (the two halves of a line of 128 bytes one behind the other: with others between them the second was another trip to L2)
 #pragma unroll
-            for (uint32_t g = 0; g < 8u; ++g) {
-                const uint32_t at = 8u * (16u * ((g >> 1) & 1u) + 8u * (g & 1u) + 4u * (g >> 2));
+            for (uint32_t n = 0; n < 8u; ++n) {
+                const uint32_t g = (n >> 1) + 4u * (n & 1u), at = 8u * (16u * ((g >> 1) & 1u) + 8u * (g & 1u) + 4u * (g >> 2));
                 xa[x][g].u = *reinterpret_cast<const uint4 *>(hp + at);
                 xb[x][g].u = *reinterpret_cast<const uint4 *>(lp + at);
             }

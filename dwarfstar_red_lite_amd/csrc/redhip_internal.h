@@ -205,12 +205,12 @@ hipError_t launch_tile_iq3s(const void *raw, uint64_t raw_stride, uint32_t count
 // Tile lists of a chunk for the tile kernels. Groups 0..U-1 are the distinct routed experts (pairs expert_start[u] ..
 // expert_start[u + 1]), the last is the shared expert with pairs P .. P + shared_ntok (0: no shared tiles). A tile = (expert id or
 // kSharedTile, first pair, number of pairs). Three lists in the same arrays, list l from entry l * list_stride on (list_stride = prefill_tile_bound of the call),
-// its length in n_tiles[l]:
+// its length in n_tiles[l]; a list's tiles of up to kPrefillSmallTile pairs are its last ones, n_tiles[3] and n_tiles[4] = the number of the others in lists 0 and 2:
 //   0  tiles of kPrefillTile pairs
 //   1  "wide" tiles of 17 .. kPrefillWideTile pairs: a group's runs of 32 pairs, and its remainder when that is more than 16
 //   2  "narrow" tiles: the remainders of 1 .. 16 pairs
 // List 0 covers every pair once, and so do lists 1 and 2 together: wide tiles multiply two sets of 16 pairs with every decoded weight.
-constexpr uint32_t kPrefillTile = 16u, kPrefillWideTile = 32u, kSharedTile = 0xffffffffu;
+constexpr uint32_t kPrefillSmallTile = 8u, kPrefillTile = 16u, kPrefillWideTile = 32u, kSharedTile = 0xffffffffu;
 struct TileLists {
     uint32_t *tile_expert, *tile_pair0, *tile_n, *n_tiles;
     uint32_t list_stride, shared_ntok;
@@ -220,11 +220,13 @@ struct TileLists {
 // wave_total: LDS scratch. Exclusive prefix sums of the tiles per group, then every group writes its tiles.
 __device__ __forceinline__ void build_tile_lists(uint32_t expert, uint32_t p0, uint32_t n, uint32_t P, const TileLists &tl, uint32_t (*wave_total)[16]) {
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
-    auto counts = [](uint32_t m, uint32_t *c) {            // tiles of m pairs in the three lists
-        const uint32_t rem = m % kPrefillWideTile;
-        c[0] = (m + kPrefillTile - 1u) / kPrefillTile;
+    // tiles of m pairs in the three lists; a small one (a group has at most one, its last) counts kSmall, so that one sum has both numbers
+    constexpr uint32_t kSmall = 1u << 21, kOthers = kSmall - 1u;
+    auto counts = [](uint32_t m, uint32_t *c) {
+        const uint32_t rem = m % kPrefillWideTile, rem16 = m % kPrefillTile;
+        c[0] = m / kPrefillTile + (rem16 > kPrefillSmallTile ? 1u : rem16 ? kSmall : 0u);
         c[1] = m / kPrefillWideTile + (rem > kPrefillTile ? 1u : 0u);
-        c[2] = rem > 0u && rem <= kPrefillTile ? 1u : 0u;
+        c[2] = rem > kPrefillTile || !rem ? 0u : rem > kPrefillSmallTile ? 1u : kSmall;
     };
     uint32_t mine[3], scan[3];
     counts(n, mine);
@@ -243,9 +245,9 @@ __device__ __forceinline__ void build_tile_lists(uint32_t expert, uint32_t p0, u
     counts(tl.shared_ntok, sh);
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
-        uint32_t base = 0u, routed_tiles = 0u;
-        for (uint32_t w = 0; w < 16u; ++w) { if (w < wave) base += wave_total[l][w]; routed_tiles += wave_total[l][w]; }
-        const uint32_t off = (uint32_t)l * tl.list_stride, first = off + base + scan[l] - mine[l];
+        uint32_t base = scan[l] - mine[l], routed = 0u;
+        for (uint32_t w = 0; w < 16u; ++w) { if (w < wave) base += wave_total[l][w]; routed += wave_total[l][w]; }
+        const uint32_t off = (uint32_t)l * tl.list_stride, others = (routed & kOthers) + (sh[l] & kOthers);
         // tile t of a run of m pairs that starts at pair q0, in list l
         auto put = [&](uint32_t at, uint32_t e, uint32_t q0, uint32_t m, uint32_t t) {
             const uint32_t size = l == 0 ? kPrefillTile : kPrefillWideTile, start = l == 2 ? m - m % kPrefillWideTile : size * t;
@@ -253,9 +255,15 @@ __device__ __forceinline__ void build_tile_lists(uint32_t expert, uint32_t p0, u
             tl.tile_pair0[at] = q0 + start;
             tl.tile_n[at] = m - start < size ? m - start : size;
         };
-        for (uint32_t t = 0; t < mine[l]; ++t) put(first + t, expert, p0, n, t);
-        for (uint32_t t = tid; t < sh[l]; t += 1024u) put(off + routed_tiles + t, kSharedTile, P, tl.shared_ntok, t);
-        if (tid == 0u) tl.n_tiles[l] = routed_tiles + sh[l];
+        const uint32_t big = mine[l] & kOthers, sh_big = sh[l] & kOthers;
+        for (uint32_t t = 0; t < big; ++t) put(off + (base & kOthers) + t, expert, p0, n, t);
+        if (mine[l] >= kSmall) put(off + others + base / kSmall, expert, p0, n, big);
+        for (uint32_t t = tid; t < sh_big; t += 1024u) put(off + (routed & kOthers) + t, kSharedTile, P, tl.shared_ntok, t);
+        if (tid == 0u) {
+            if (sh[l] >= kSmall) put(off + others + routed / kSmall, kSharedTile, P, tl.shared_ntok, sh_big);
+            tl.n_tiles[l] = others + (routed + sh[l]) / kSmall;
+            if (l != 1) tl.n_tiles[l == 0 ? 3 : 4] = others;
+        }
     }
 }
 #endif

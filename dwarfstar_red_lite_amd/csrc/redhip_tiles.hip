@@ -73,6 +73,9 @@ __device__ __forceinline__ void request_quarter(const StagedArgs &a, const uint8
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pair_rows(float *base, uint32_t n, uint32_t rows) { return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)(n * rows * 4u), 0x00027000); }
 
 // ---- gate/up ----
+// SMALL: a tile of up to eight pairs, whose high and low halves are rows 0 .. 7 and 8 .. 15 of one operand: half the matrix instructions, half the
+// activations. Tiles end with what is left of an expert's pairs, so these are a third (ten pairs an expert) to all (batches) of a chunk's: 77 tokens of
+// IQ1_M layers 311 -> 286 us for two layers, a batch of 24 on IQ2_XXS 290 -> 271 for three, 512 tokens of a pool 204 -> 197.
 // Eight waves. A wave keeps the activations of its columns for the whole tile in registers, as fp16 halves: of two blocks of 256 columns for
 // sixteen pairs (SETS 1; it multiplies the gate or the up rows with them), of one block for 32 (SETS 2; both rows). PK such parts make the
 // columns, NRT row tiles of 16 rows are in work beside each other: a unit is the gate and the up rows of 16 NRT FFN columns.
@@ -91,10 +94,11 @@ template <int SRC, int SETS, uint32_t KP> struct GateUpLds {
 };
 
 // units u0 .. u1 - 1 (unit = tile * units per tile + unit of the tile) of a tile list
-template <int SRC, int SETS, uint32_t KP, bool SHORT>
+template <int SRC, int SETS, uint32_t KP, bool SHORT, bool SMALL>
 __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList &list, uint32_t u0, uint32_t u1, GateUpLds<SRC, SETS, KP> &lds, bool tables) {
     using G = GateUp<SETS, KP>;
-    constexpr uint32_t PK = G::PK, NRT = G::NRT, K = 256u * KP, PAIRS = 16u * SETS, T = kGateUpThreads, UB = G::kUnits;
+    constexpr uint32_t PK = G::PK, NRT = G::NRT, K = 256u * KP, PAIRS = SMALL ? kPrefillSmallTile : 16u * SETS, T = kGateUpThreads, UB = G::kUnits;
+    static_assert(!SMALL || SETS == 1, "");
     const uint32_t tid = each_trip(threadIdx.x), lane = tid & 63u, r = lane & 15u, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t kp = wave % PK, rt = (wave / PK) % NRT, up = wave / (PK * NRT);      // up: SETS 1, the wave has the up rows
     const uint32_t upt = a.rows / (16u * NRT), tile0 = u0 / upt, n_info = (u1 - 1u) / upt + 1u - tile0;
@@ -124,21 +128,22 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
     // chains, in 1 to 2 % more time; batches of fewer tokens are slices, which lose 1.76e-7, so these have short ones and are no further off on the
     // tiles (IQ2_XXS, 2048 x 512, 24 tokens with the routing given; chains of one step lose more in the additions).
     constexpr uint32_t kChain = SHORT || layout<SRC>() == L_ROWS ? 2u : 4u;
-    H8 xa[2][8], xb[2][8];                                 // SETS 1: [block], SETS 2: [set]
+    H8 xa[2][8], xb[SMALL ? 1 : 2][8];                     // SETS 1: [block], SETS 2: [set]; high and low halves (SMALL: both in xa)
+    const float row_scale = SMALL && q >= 2u ? 4.8828125e-4f : 1.0f;      // of the lane's rows of the products
     const auto load_tile = [&](uint32_t tile) {
 #pragma unroll
         for (uint32_t x = 0; x < 2u; ++x) {
             __builtin_amdgcn_sched_barrier(0);             // one at a time: both at once do not fit the registers
-            const uint32_t tok = lds.tokens[(tile - tile0) * PAIRS + (SETS == 1 ? 0u : 16u * x) + r];
+            const uint32_t tok = lds.tokens[(tile - tile0) * PAIRS + (SETS == 1 ? 0u : 16u * x) + (SMALL ? r & 7u : r)];
             const uint64_t base = (uint64_t)tok * K + 256u * (SETS == 1 ? 2u * kp + x : kp) + 8u * q;
-            const _Float16 *hp = a.xh + base, *lp = a.xl + base;
+            const _Float16 *hp = (SMALL && r >= 8u ? a.xl : a.xh) + base, *lp = a.xl + base;
             // four lanes of a pair take 64 bytes side by side; the exchange makes them each lane's own run
             // (the two halves of a line of 128 bytes one behind the other: with others between them the second was another trip to L2)
 #pragma unroll
             for (uint32_t n = 0; n < 8u; ++n) {
                 const uint32_t g = (n >> 1) + 4u * (n & 1u), at = 8u * (16u * ((g >> 1) & 1u) + 8u * (g & 1u) + 4u * (g >> 2));
                 xa[x][g].u = *reinterpret_cast<const uint4 *>(hp + at);
-                xb[x][g].u = *reinterpret_cast<const uint4 *>(lp + at);
+                if constexpr (!SMALL) xb[x][g].u = *reinterpret_cast<const uint4 *>(lp + at);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -146,26 +151,31 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
         for (uint32_t x = 0; x < 2u; ++x) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (uint32_t g = 0; g < 8u; g += 2u) { swap16(xa[x][g].u, xa[x][g + 1u].u); swap16(xb[x][g].u, xb[x][g + 1u].u); }
+            for (uint32_t g = 0; g < 8u; g += 2u) { swap16(xa[x][g].u, xa[x][g + 1u].u); if constexpr (!SMALL) swap16(xb[x][g].u, xb[x][g + 1u].u); }
 #pragma unroll
-            for (uint32_t g = 0; g < 8u; ++g) if (!(g & 2u)) { swap32(xa[x][g].u, xa[x][g + 2u].u); swap32(xb[x][g].u, xb[x][g + 2u].u); }
+            for (uint32_t g = 0; g < 8u; ++g) if (!(g & 2u)) { swap32(xa[x][g].u, xa[x][g + 2u].u); if constexpr (!SMALL) swap32(xb[x][g].u, xb[x][g + 2u].u); }
         }
     };
     // The sums of UNITS units, the first of them number fj of tile ft, and their SwiGLU. No wave and no lane may skip a store: the loads of the next units are in flight in front of it, and the
     // compiler, which waits for them by counting memory operations in order, can count only what every path issues.
     const auto reduce = [&](auto units, uint32_t ft, uint32_t fj, const float *pt) {
-        constexpr uint32_t UNITS = decltype(units)::value, N = 256u * SETS * NRT * UNITS;
+        constexpr uint32_t UNITS = decltype(units)::value, OUT = 16u * (SMALL ? 8u : 16u), N = OUT * SETS * NRT * UNITS;      // OUT: a row tile's outputs, of sixteen pairs or of eight
 #pragma unroll
         for (uint32_t base = 0; base < N; base += T) {
             const uint32_t e = N < T ? min(tid, N - 1u) : base + tid;      // (surplus threads repeat the last element)
-            const uint32_t at = e & 255u, b = __builtin_amdgcn_readfirstlane((e >> 8) % (SETS * NRT)), un = __builtin_amdgcn_readfirstlane((e >> 8) / (SETS * NRT)), set = b % SETS, slot = b / SETS;
+            const uint32_t at = e % OUT, b = __builtin_amdgcn_readfirstlane((e / OUT) % (SETS * NRT)), un = __builtin_amdgcn_readfirstlane((e / OUT) / (SETS * NRT)), set = b % SETS, slot = b / SETS;
             const float *src = pt + un * G::kPart + slot * PK * G::kSums + set * 256u + at;
-            using Sum = std::conditional_t<(PK > 1u), double, float>;      // (a row's parts are added here)
-            Sum g[PK], u[PK];
+            constexpr uint32_t PARTS = SMALL ? 2u * PK : PK;      // SMALL: the sums over high and over low halves apart
+            using Sum = std::conditional_t<(PARTS > 1u), double, float>;      // (a row's parts are added here)
+            Sum g[PARTS], u[PARTS];
 #pragma unroll
-            for (uint32_t k = 0; k < PK; ++k) { g[k] = src[k * G::kSums]; u[k] = src[k * G::kSums + SETS * 256u]; }
+            for (uint32_t k = 0; k < PARTS; ++k) {
+                const uint32_t off = (k % PK) * G::kSums + (k / PK) * OUT;
+                g[k] = src[off];
+                u[k] = src[off + SETS * 256u];
+            }
 #pragma unroll
-            for (uint32_t n = PK / 2u; n; n /= 2u)
+            for (uint32_t n = PARTS / 2u; n; n /= 2u)
 #pragma unroll
                 for (uint32_t k = 0; k < n; ++k) { g[k] += g[k + n]; u[k] += u[k + n]; }
             uint32_t dt = ft - tile0, dj = fj + un;
@@ -194,6 +204,7 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
 #pragma unroll
         for (uint32_t m = 0; m < 2u; ++m) {
             d[m] = quarter_d<SRC>(c.d[m]);
+            if constexpr (SMALL) d[m] *= row_scale;
             e[m] = fetch_entry<SRC, 0u>(c.v[m], lt);
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s) acc[m][s] = low[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -225,18 +236,23 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
                 for (uint32_t m = 0; m < 2u; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[SETS == 1 ? m : s][S].v, w[m], acc[m][s], 0, 0, 0);
+            if constexpr (!SMALL) {
 #pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
+                for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
-                for (uint32_t m = 0; m < 2u; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[SETS == 1 ? m : s][S].v, w[m], low[m][s], 0, 0, 0);
+                    for (uint32_t m = 0; m < 2u; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[SETS == 1 ? m : s][S].v, w[m], low[m][s], 0, 0, 0);
+            }
         });
         float *mine = pt + (rt * PK + kp) * G::kSums + 4u * lane;
         if constexpr (SETS == 1) {
             float4_t &both = acc[0][0];                    // the two blocks
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const float l = fmaf(low[1][0][t], 4.8828125e-4f * d[1], low[0][0][t] * (4.8828125e-4f * d[0]));
-                both[t] = fmaf(sum[1][0][t] + acc[1][0][t], d[1], fmaf(sum[0][0][t] + acc[0][0][t], d[0], l));
+                if constexpr (SMALL) both[t] = fmaf(sum[1][0][t] + acc[1][0][t], d[1], (sum[0][0][t] + acc[0][0][t]) * d[0]);
+                else {
+                    const float l = fmaf(low[1][0][t], 4.8828125e-4f * d[1], low[0][0][t] * (4.8828125e-4f * d[0]));
+                    both[t] = fmaf(sum[1][0][t] + acc[1][0][t], d[1], fmaf(sum[0][0][t] + acc[0][0][t], d[0], l));
+                }
             }
             *reinterpret_cast<float4_t *>(mine + up * 256u) = both;
         } else {
@@ -528,27 +544,38 @@ template <int SRC, bool DOWN, int SETS, uint32_t KP, bool SHORT>
 __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) void staged_tiles_kernel(StagedArgs a) {
     __shared__ __attribute__((aligned(16))) std::conditional_t<DOWN, DownLds<down_src<SRC, SETS, KP>(), SETS, KP>, GateUpLds<SRC, SETS, KP>> lds;
     static_assert(sizeof(lds) <= 160u * 1024u, "what a compute unit has");
-    const uint32_t n0 = a.n_tiles[0], n1 = a.n_tiles[1], n2 = a.n_tiles[2];      // (one trip)
+    const uint32_t n0 = a.n_tiles[0], n1 = a.n_tiles[1], n2 = a.n_tiles[2], b0 = a.n_tiles[3], b2 = a.n_tiles[4];      // (one trip)
     const bool few = n1 < a.few;
     if (SETS == 2 && few) return;
     const uint32_t l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
-    const uint32_t n_tiles = SETS == 2 ? n1 : few ? n0 : n2;
+    const uint32_t n_tiles = SETS == 2 ? n1 : few ? n0 : n2, n_big = DOWN || SETS == 2 ? n_tiles : few ? b0 : b2;      // the others are small ones
     uint32_t per_tile = a.rows / (DOWN ? 32u : 16u * GateUp<SETS, DOWN ? 2u : KP>::NRT);
     if constexpr (DOWN && down_tiles_a_pass<SETS, KP>() == 1u) {
         // as many passes a tile as fill the rounds that the busiest workgroup has anyway
         const uint32_t least = (per_tile + down_waves(SETS) - 1u) / down_waves(SETS), rounds = (n_tiles * least + gridDim.x - 1u) / gridDim.x;
         per_tile = n_tiles ? min(per_tile / 4u, rounds * gridDim.x / n_tiles) : least;
     }
-    const uint32_t work = n_tiles * per_tile;
     const TileList list{a.tile_expert + off, a.tile_pair0 + off, a.tile_n + off};
     // workgroups are dealt round-robin over the eight XCDs: neighbouring runs (which share tiles) go to one XCD's L2
     const uint32_t G = gridDim.x, at = G % 8u == 0u ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
-    const uint32_t w0 = (uint32_t)((uint64_t)at * work / G), w1 = (uint32_t)((uint64_t)(at + 1u) * work / G);
-    for (uint32_t from = w0; from < w1;) {                 // (a run of more than kTileInfos tiles in parts)
-        const uint32_t to = min(w1, (from / per_tile + kTileInfos) * per_tile);
+    // equal shares of the time: a unit of a small tile takes kSmallCost / kBigCost of another one's
+    constexpr uint32_t kBigCost = 5u, kSmallCost = 4u;
+    const uint32_t w_big = n_big * per_tile;
+    const uint64_t cost = (uint64_t)w_big * kBigCost + (uint64_t)(n_tiles - n_big) * per_tile * kSmallCost;
+    const auto border = [&](uint32_t i) {
+        const uint64_t c = i * cost / G, big = (uint64_t)w_big * kBigCost;
+        return c <= big ? (uint32_t)(c / kBigCost) : w_big + (uint32_t)((c - big) / kSmallCost);
+    };
+    const uint32_t w0 = border(at), w1 = border(at + 1u);
+    for (uint32_t from = w0; from < w1;) {                 // (a run of more than kTileInfos tiles in parts, small tiles apart)
+        const bool small = from >= w_big;
+        const uint32_t to = min(small ? w1 : min(w1, w_big), (from / per_tile + kTileInfos) * per_tile);
         if (from != w0) __syncthreads();
         if constexpr (DOWN) down_items<down_src<SRC, SETS, KP>(), SETS, KP>(a, list, per_tile, from, to, lds, from == w0);
-        else gateup_units<SRC, SETS, KP, SHORT>(a, list, from, to, lds, from == w0);
+        else if constexpr (SETS == 1) {
+            if (small) gateup_units<SRC, SETS, KP, SHORT, true>(a, list, from, to, lds, from == w0);
+            else gateup_units<SRC, SETS, KP, SHORT, false>(a, list, from, to, lds, from == w0);
+        } else gateup_units<SRC, SETS, KP, SHORT, false>(a, list, from, to, lds, from == w0);
         from = to;
     }
 }

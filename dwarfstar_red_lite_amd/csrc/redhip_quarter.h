@@ -83,76 +83,56 @@ __device__ __forceinline__ void build_signs(uint32_t *signs, uint32_t tid) {
     }
 }
 
-// The large tables, by T threads: a thread's codebook entries are requested together (a trip to memory), every further one is packed fp16 arithmetic, exact.
+// The large tables, by T threads in two parts: a thread's codebook entries are requested together (a trip to memory, beside whatever is requested behind
+// them), then written: every further entry is packed fp16 arithmetic, exact.
 // Where a thread writes four entries side by side, in an order that differs between the fours of lanes: sixteen lanes then write to different
-// banks. (Entry by entry in f32, each behind a trip of its own, the tables of IQ2_XXS took 8000 cycles of every launch, 20000 of the 91000 of a batch
-// of 24 tokens until the first products with what waits for them.)
-template <int SRC, uint32_t T>
-__device__ __forceinline__ void build_staged_tables(uint8_t *entries, uint32_t *signs, uint32_t tid, const int8_t *grid) {
-    if constexpr (fmt<SRC>() == F_XXS || fmt<SRC>() == F_XS) {
-        constexpr uint32_t PER = fmt<SRC>() == F_XXS ? 4u : 2u, kItems = PER * codebook_entries<SRC>(), N = (kItems + T - 1u) / T;      // four scales or copies each
-        uint64_t ge[N];
+// banks. (Entry by entry in f32, each behind a trip of its own, the tables of IQ2_XXS took 8000 cycles of every launch, of the 91000 of a batch
+// of 24 tokens.)
+template <int SRC, uint32_t T> struct TableSeeds {
+    // items: XXS four scales of an entry, XS four copies, M an entry with both offsets, IQ3 eight scales of an entry
+    static constexpr uint32_t kPer = fmt<SRC>() == F_XXS ? 4u : fmt<SRC>() == F_M ? 1u : 2u, kItems = kPer * codebook_entries<SRC>(), N = (kItems + T - 1u) / T;
+    std::conditional_t<is_iq3<SRC>(), uint32_t, uint64_t> e[N];
+    static __device__ __forceinline__ uint32_t item(uint32_t tid, uint32_t n) { return min(tid + n * T, kItems - 1u); }      // (surplus threads repeat the last)
+    __device__ __forceinline__ void request(uint32_t tid, const int8_t *grid) {
 #pragma unroll
         for (uint32_t n = 0; n < N; ++n) {
-            const uint32_t e = min(tid + n * T, kItems - 1u) / PER;      // (surplus threads repeat the last)
-            if constexpr (fmt<SRC>() == F_XXS) ge[n] = redhip_iq2xxs_grid[e];
-            else ge[n] = reinterpret_cast<const uint64_t *>(grid)[e];
+            const uint32_t i = item(tid, n);
+            if constexpr (is_iq3<SRC>()) e[n] = redhip_iq3s_grid[i & 511u];
+            else if constexpr (fmt<SRC>() == F_XXS) e[n] = redhip_iq2xxs_grid[i / kPer];
+            else e[n] = reinterpret_cast<const uint64_t *>(grid)[i / kPer];
         }
+    }
+    __device__ __forceinline__ void store(uint8_t *entries, uint32_t *signs, uint32_t tid) const {
         build_signs<SRC, T>(signs, tid);
 #pragma unroll
         for (uint32_t n = 0; n < N; ++n) {
-            const uint32_t i = min(tid + n * T, kItems - 1u);
-            const H8 base = entry_halves<fmt<SRC>() == F_XS>(ge[n]);
+            const uint32_t i = item(tid, n);
+            if constexpr (is_iq3<SRC>()) {
+                const half2_t a = byte_halves<0u, false>(e[n]), b = byte_halves<2u, false>(e[n]);
 #pragma unroll
-            for (uint32_t k = 0; k < 4u; ++k) {
-                const uint32_t at = 4u * i + ((k + (i >> 2)) & 3u);
-                H8 v = base;
-                if constexpr (fmt<SRC>() == F_XXS) {
-                    const half2_t f = odd_halves(at & 15u);
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) v.p[p] = base.p[p] * f;
+                for (uint32_t k = 0; k < 8u; ++k) {
+                    const uint32_t scale = (i >> 9) * 8u + k;
+                    const half2_t f = odd_halves(scale);
+                    *reinterpret_cast<uint2 *>(entries + (scale * 512u + (i & 511u)) * 8u) =
+                        make_uint2(__builtin_bit_cast(uint32_t, a * f), __builtin_bit_cast(uint32_t, b * f));
                 }
-                *reinterpret_cast<uint4 *>(entries + at * 16u) = v.u;
-            }
-        }
-    } else if constexpr (fmt<SRC>() == F_M) {
-        constexpr uint32_t kItems = codebook_entries<SRC>(), N = (kItems + T - 1u) / T;
-        uint64_t ge[N];
+            } else {
+                const H8 base = entry_halves<fmt<SRC>() != F_XXS>(e[n]);
 #pragma unroll
-        for (uint32_t n = 0; n < N; ++n) ge[n] = reinterpret_cast<const uint64_t *>(grid)[min(tid + n * T, kItems - 1u)];
+                for (uint32_t k = 0; k < (fmt<SRC>() == F_M ? 2u : 4u); ++k) {
+                    const uint32_t at = fmt<SRC>() == F_M ? 2048u * k + i : 4u * i + ((k + (i >> 2)) & 3u);
+                    H8 v = base;
 #pragma unroll
-        for (uint32_t n = 0; n < N; ++n) {
-            const uint32_t i = min(tid + n * T, kItems - 1u);
-            const H8 base = entry_halves<true>(ge[n]);
-#pragma unroll
-            for (uint32_t neg = 0; neg < 2u; ++neg) {
-                const _Float16 off = neg ? -0.125f : 0.125f;      // (exact: a byte and three bits behind the point)
-                H8 v;
-#pragma unroll
-                for (int p = 0; p < 4; ++p) v.p[p] = base.p[p] + half2_t{off, off};
-                *reinterpret_cast<uint4 *>(entries + neg * 32768u + i * 16u) = v.u;
-            }
-        }
-    } else {
-        constexpr uint32_t kItems = 2u * 512u, N = (kItems + T - 1u) / T;      // eight scales each
-        uint32_t gw[N];
-#pragma unroll
-        for (uint32_t n = 0; n < N; ++n) gw[n] = redhip_iq3s_grid[min(tid + n * T, kItems - 1u) & 511u];
-        build_signs<SRC, T>(signs, tid);
-#pragma unroll
-        for (uint32_t n = 0; n < N; ++n) {
-            const uint32_t i = min(tid + n * T, kItems - 1u);
-            const half2_t a = byte_halves<0u, false>(gw[n]), b = byte_halves<2u, false>(gw[n]);
-#pragma unroll
-            for (uint32_t k = 0; k < 8u; ++k) {
-                const uint32_t scale = (i >> 9) * 8u + k;
-                const half2_t f = odd_halves(scale);
-                *reinterpret_cast<uint2 *>(entries + (scale * 512u + (i & 511u)) * 8u) =
-                    make_uint2(__builtin_bit_cast(uint32_t, a * f), __builtin_bit_cast(uint32_t, b * f));
+                    for (int p = 0; p < 4; ++p) {
+                        if constexpr (fmt<SRC>() == F_XXS) { const half2_t f = odd_halves(at & 15u); v.p[p] = base.p[p] * f; }
+                        if constexpr (fmt<SRC>() == F_M) { const _Float16 off = k ? -0.125f : 0.125f; v.p[p] = base.p[p] + half2_t{off, off}; }      // (exact: a byte and three bits behind the point)
+                    }
+                    *reinterpret_cast<uint4 *>(entries + at * 16u) = v.u;
+                }
             }
         }
     }
-}
+};
 
 // The small tables, by T threads in two parts: a thread's codebook entries are requested (before the rows, which the second part must not
 // wait for), then written. Tables with copies are written by two threads per entry, half of the copies each.

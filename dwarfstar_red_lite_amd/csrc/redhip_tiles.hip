@@ -54,14 +54,8 @@ __device__ __forceinline__ void swap32(uint4 &a, uint4 &b) { swap32(a.x, b.x); s
 constexpr uint32_t kTileInfos = 32u;
 struct TileInfo { uint64_t mat; uint32_t p0, n; };      // mat: distance of the expert's first matrix from StagedArgs::experts
 struct TileList { const uint32_t *expert, *pair0, *n; };
-__device__ __forceinline__ TileInfo tile_info(const StagedArgs &a, const TileList &l, uint32_t tile) {
-    const uint32_t e = l.expert[tile];
-    return TileInfo{e == kSharedTile ? (uint64_t)(a.shared - a.experts) : (uint64_t)e * a.stride, l.pair0[tile], l.n[tile]};
-}
-__device__ __forceinline__ TileInfo uniform_info(const TileInfo &t) {
-    const auto one = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane(v); };
-    return TileInfo{((uint64_t)one((uint32_t)(t.mat >> 32)) << 32) | one((uint32_t)t.mat), one(t.p0), one(t.n)};
-}
+__device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ TileInfo uniform_info(const TileInfo &t) { return TileInfo{((uint64_t)uni((uint32_t)(t.mat >> 32)) << 32) | uni((uint32_t)t.mat), uni(t.p0), uni(t.n)}; }
 // the lane's quarter of block kc of row tile `row_tile` of a matrix of `rows` rows
 template <int SRC, uint32_t KP>
 __device__ __forceinline__ void request_quarter(const StagedArgs &a, const uint8_t *mat, uint32_t row_tile, uint32_t r, uint32_t kc, uint32_t q, Quarter &v, uint2 &d) {
@@ -102,17 +96,32 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
     const uint32_t tid = each_trip(threadIdx.x), lane = tid & 63u, r = lane & 15u, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t kp = wave % PK, rt = (wave / PK) % NRT, up = wave / (PK * NRT);      // up: SETS 1, the wave has the up rows
     const uint32_t upt = a.rows / (16u * NRT), tile0 = u0 / upt, n_info = (u1 - 1u) / upt + 1u - tile0;
-    if (tid < 64u) {
-        if (tid < n_info) lds.tiles[tid] = tile_info(a, list, tile0 + tid);
-        for (uint32_t k = tid; k < n_info * PAIRS; k += 64u) {      // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
-            const uint32_t t = tile0 + k / PAIRS, i = k % PAIRS, p = list.pair0[t] + (i < list.n[t] ? i : 0u), tok = p < a.P ? a.pair_token[p] : p - a.P;
-            lds.tokens[k] = tok;
-            lds.scales[k] = format_scale<SRC>() * exp2i(a.xexp[tok]);
-        }
-    } else if (tables)
-        build_staged_tables<SRC, T - 64u>(lds.entries, lds.signs, tid - 64u, a.grid);
-    __syncthreads();
-    const LaneTables lt = lane_tables<SRC>(lds.entries, lds.signs, tid);
+    // Everything that the first products wait for is on its way before the tables are built: the codebook, the run's tiles, their tokens, the first units'
+    // rows, the first tile's activations, each behind what names it. (Fetched behind the tables and a barrier, the first products of a batch of 24
+    // tokens began 13800 cycles into a launch of 89000.) Every thread requests the same number of loads, so that the waits can count them.
+    TableSeeds<SRC, T> seeds;
+    if (tables) seeds.request(tid, a.grid);
+    constexpr uint32_t NI = (kTileInfos * PAIRS + T - 1u) / T;      // pairs of the run's tiles per thread
+    struct { uint32_t e, p0, n, tok; int exp; } info[NI];
+    const auto at_info = [&](uint32_t n) { return min(tid + n * T, n_info * PAIRS - 1u); };
+#pragma unroll
+    for (uint32_t n = 0; n < NI; ++n) {
+        const uint32_t t = tile0 + at_info(n) / PAIRS;
+        info[n].e = list.expert[t]; info[n].p0 = list.pair0[t]; info[n].n = list.n[t];
+    }
+    const auto mat_of = [&](uint32_t e) { return e == kSharedTile ? (uint64_t)(a.shared - a.experts) : (uint64_t)e * a.stride; };
+    const uint32_t e0 = uni(list.expert[tile0]), e1 = uni(list.expert[tile0 + min(1u, n_info - 1u)]), first_p0 = uni(list.pair0[tile0]), first_n = uni(list.n[tile0]);
+    const auto token_of = [&](uint32_t p0, uint32_t n, uint32_t i) {      // (pairs beyond the tile's n repeat its first one: their rows of the product are never stored)
+        const uint32_t p = p0 + (i < n ? i : 0u), tok = a.pair_token[min(p, a.P - 1u)];
+        return p < a.P ? tok : p - a.P;
+    };
+    const uint32_t pair = SMALL ? r & 7u : r;              // the lane's row of the activations
+    uint32_t first_tok[SETS];
+#pragma unroll
+    for (uint32_t s = 0; s < (uint32_t)SETS; ++s) first_tok[s] = token_of(first_p0, first_n, 16u * s + pair);
+#pragma unroll
+    for (uint32_t n = 0; n < NI; ++n) info[n].tok = token_of(info[n].p0, info[n].n, at_info(n) % PAIRS);
+    __builtin_amdgcn_sched_barrier(0);
     // the lane's two quarters of a unit (SETS 1: of the two blocks, SETS 2: of the gate and the up row), and what their d are made from
     struct Carried { Quarter v[2]; uint2 d[2]; };
     const auto request = [&](Carried &c, uint64_t mat, uint32_t j) {
@@ -122,6 +131,22 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
             request_quarter<SRC, KP>(a, mm, j * NRT + rt, r, SETS == 1 ? 2u * kp + m : kp, q, c.v[m], c.d[m]);
         }
     };
+    constexpr uint32_t kCarried = SETS == 2 && fmt<SRC>() != F_XXS ? 1u : 2u;      // units on their way: two where the registers hold them
+    Carried c[kCarried];
+    uint32_t tile = tile0, j = u0 % upt, ftile = tile0, fj = j, fleft = u1 - u0;      // f..: the unit to be requested next
+    uint64_t fmat = mat_of(e0);
+    request(c[0], fmat, fj);
+    if constexpr (kCarried == 2u) {                        // (a tile has two units at least)
+        if (fleft > 1u) {
+            --fleft;
+            if (++fj == upt) { fj = 0u; ++ftile; fmat = mat_of(e1); }
+        }
+        request(c[1], fmat, fj);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (uint32_t n = 0; n < NI; ++n) info[n].exp = a.xexp[info[n].tok];
+    __builtin_amdgcn_sched_barrier(0);
     // Precision. The matrix unit rounds a sum four times per instruction (once per eight products), so what a block's sum loses goes with the
     // length of its chain of instructions: the low halves have a chain of their own, and the high ones one per kChain steps, added up in f32.
     // (SHORT: of two steps.) The low halves go first into a result, so that it is rounded once for both. Of a chunk 1.82e-7 is lost so, 1.74e-7 with short
@@ -130,23 +155,19 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
     constexpr uint32_t kChain = SHORT || layout<SRC>() == L_ROWS ? 2u : 4u;
     H8 xa[2][8], xb[SMALL ? 1 : 2][8];                     // SETS 1: [block], SETS 2: [set]; high and low halves (SMALL: both in xa)
     const float row_scale = SMALL && q >= 2u ? 4.8828125e-4f : 1.0f;      // of the lane's rows of the products
-    const auto load_tile = [&](uint32_t tile) {
+    const auto fetch_block = [&](uint32_t x, uint32_t tok) {
+        const uint64_t base = (uint64_t)tok * K + 256u * (SETS == 1 ? 2u * kp + x : kp) + 8u * q;
+        const _Float16 *hp = (SMALL && r >= 8u ? a.xl : a.xh) + base, *lp = a.xl + base;
+        // four lanes of a pair take 64 bytes side by side; the exchange makes them each lane's own run
 #pragma unroll
-        for (uint32_t x = 0; x < 2u; ++x) {
-            __builtin_amdgcn_sched_barrier(0);             // one at a time: both at once do not fit the registers
-            const uint32_t tok = lds.tokens[(tile - tile0) * PAIRS + (SETS == 1 ? 0u : 16u * x) + (SMALL ? r & 7u : r)];
-            const uint64_t base = (uint64_t)tok * K + 256u * (SETS == 1 ? 2u * kp + x : kp) + 8u * q;
-            const _Float16 *hp = (SMALL && r >= 8u ? a.xl : a.xh) + base, *lp = a.xl + base;
-            // four lanes of a pair take 64 bytes side by side; the exchange makes them each lane's own run
-            // (the two halves of a line of 128 bytes one behind the other: with others between them the second was another trip to L2)
-#pragma unroll
-            for (uint32_t n = 0; n < 8u; ++n) {
-                const uint32_t g = (n >> 1) + 4u * (n & 1u), at = 8u * (16u * ((g >> 1) & 1u) + 8u * (g & 1u) + 4u * (g >> 2));
-                xa[x][g].u = *reinterpret_cast<const uint4 *>(hp + at);
-                if constexpr (!SMALL) xb[x][g].u = *reinterpret_cast<const uint4 *>(lp + at);
-            }
+        for (uint32_t g = 0; g < 8u; ++g) {
+            const uint32_t at = 8u * (16u * ((g >> 1) & 1u) + 8u * (g & 1u) + 4u * (g >> 2));
+            xa[x][g].u = *reinterpret_cast<const uint4 *>(hp + at);
+            if constexpr (!SMALL) xb[x][g].u = *reinterpret_cast<const uint4 *>(lp + at);
         }
-        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_sched_barrier(0);                 // one block at a time: the addresses of both do not fit the registers
+    };
+    const auto arrange_blocks = [&] {
 #pragma unroll
         for (uint32_t x = 0; x < 2u; ++x) {
             __builtin_amdgcn_sched_barrier(0);
@@ -156,6 +177,32 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
             for (uint32_t g = 0; g < 8u; ++g) if (!(g & 2u)) { swap32(xa[x][g].u, xa[x][g + 2u].u); if constexpr (!SMALL) swap32(xb[x][g].u, xb[x][g + 2u].u); }
         }
     };
+    const auto load_tile = [&](uint32_t tile) {
+#pragma unroll
+        for (uint32_t x = 0; x < 2u; ++x) {
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_block(x, lds.tokens[(tile - tile0) * PAIRS + (SETS == 1 ? 0u : 16u * x) + (each_trip(threadIdx.x) & (SMALL ? 7u : 15u))]);
+        }
+        arrange_blocks();
+    };
+    const auto fill_lds = [&] {
+        if (tables) seeds.store(lds.entries, lds.signs, tid);
+#pragma unroll
+        for (uint32_t n = 0; n < NI; ++n) {
+            const uint32_t k = at_info(n);                 // (surplus threads repeat the last)
+            lds.tokens[k] = info[n].tok;
+            lds.scales[k] = format_scale<SRC>() * exp2i(info[n].exp);
+            if (k % PAIRS == 0u) lds.tiles[k / PAIRS] = TileInfo{mat_of(info[n].e), info[n].p0, info[n].n};
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (SETS == 2) fill_lds();                   // (the registers do not hold the seeds beside the activations)
+#pragma unroll
+    for (uint32_t x = 0; x < 2u; ++x) fetch_block(x, first_tok[SETS == 1 ? 0u : x]);
+    if constexpr (SETS == 1) fill_lds();
+    wave_lds_barrier();
+    const LaneTables lt = lane_tables<SRC>(lds.entries, lds.signs, tid);
+    arrange_blocks();
     // The sums of UNITS units, the first of them number fj of tile ft, and their SwiGLU. No wave and no lane may skip a store: the loads of the next units are in flight in front of it, and the
     // compiler, which waits for them by counting memory operations in order, can count only what every path issues.
     const auto reduce = [&](auto units, uint32_t ft, uint32_t fj, const float *pt) {
@@ -187,8 +234,6 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
                                                   4u * (i * a.rows + dj * 16u * NRT + 16u * slot + ((at >> 2) & 15u)), 0, 0);
         }
     };
-    uint32_t tile = tile0, j = u0 % upt, ftile = tile0, fj = j, fleft = u1 - u0;      // f..: the unit to be requested next
-    uint64_t fmat = uniform_info(lds.tiles[0]).mat;
     const auto request_rows = [&](Carried &c) { request(c, fmat, fj); };
     const auto advance = [&] {                             // (the last units fetch theirs again: registers filled under a condition would be live all around the loop)
         if (fleft <= 1u) return;
@@ -268,14 +313,7 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
         advance();
         if (++j == upt && u + 1u < u1) { j = 0u; load_tile(++tile); }
     };
-    constexpr uint32_t kCarried = SETS == 2 && fmt<SRC>() != F_XXS ? 1u : 2u;      // units on their way: two where the registers hold them
-    Carried c[kCarried];
-#pragma unroll
-    for (uint32_t k = 0; k < kCarried; ++k) {
-        request_rows(c[k]);
-        advance();
-    }
-    load_tile(tile);
+    advance();
     // A buffer of partial sums is written again two barriers after its sums were complete; whoever adds them has passed one in between.
     constexpr std::integral_constant<uint32_t, 1u> one{};
     constexpr std::integral_constant<uint32_t, UB> all{};
@@ -328,24 +366,13 @@ __device__ __forceinline__ float row_max(float v) {
 // Where a pass is of one tile: parts. A tile is `parts` passes, a run whole passes; cut by items, a run that crosses tiles has up to two passes more
 // than its share, with waves idle in both (IQ3_S, 1024 x 768, 60 tiles: 46 us, now 35; 2048 x 768, 122 tiles: 58 -> 48). A part is a number of fours of
 // items, one for each SIMD: 12 + 12 + 8 items are 2 % quicker than 11 + 11 + 10.
-template <int SRC, int SETS, uint32_t KP>
+template <int SRC, int SETS, uint32_t KP, bool SMALL>
 __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &list, uint32_t parts, uint32_t i0, uint32_t i1, DownLds<SRC, SETS, KP> &lds, bool tables) {
-    constexpr uint32_t WV = down_waves(SETS), T = 64u * WV, PAIRS = 16u * SETS, K = 256u * KP, kPassTiles = down_tiles_a_pass<SETS, KP>();
+    constexpr uint32_t WV = down_waves(SETS), T = 64u * WV, PAIRS = SMALL ? kPrefillSmallTile : 16u * SETS, K = 256u * KP, kPassTiles = down_tiles_a_pass<SETS, KP>();
+    constexpr uint32_t PANEL = SMALL ? kPanel / 2u : kPanel;
+    static_assert(!SMALL || SETS == 1, "");
     const uint32_t tid = each_trip(threadIdx.x), lane = tid & 63u, r = lane & 15u, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t ipt = a.rows / 32u, tile0 = i0 / parts, n_info = (i1 - 1u) / parts + 1u - tile0, quads = ((ipt / 4u) << 16) / parts + 1u;      // quads: fours of items per part, 16 bits behind the point
-    if (tid < 64u) {
-        if (tid < n_info) lds.tiles[tid] = tile_info(a, list, tile0 + tid);
-    } else if (tables) {
-        if constexpr (small_tables<SRC>()) {
-            SmallSeeds<SRC, T - 64u> seeds;
-            seeds.request(tid - 64u, a.grid);
-            seeds.store(lds.entries, lds.signs, tid - 64u);
-        } else
-            build_staged_tables<SRC, T - 64u>(lds.entries, lds.signs, tid - 64u, a.grid);
-    }
-    __syncthreads();
-    const LaneTables lt = lane_tables<SRC>(lds.entries, lds.signs, tid);
-    const auto info_of = [&](uint32_t tile) { return uniform_info(lds.tiles[tile - tile0]); };
     // A pass: an item per wave, of up to kPassTiles tiles
     struct Pass { uint32_t i, tile, j, n; };               // first item or part, its tile, the first item's number in the tile, items
     const auto pass_at = [&](uint32_t i, uint32_t tile, uint32_t at) {      // at: number of the item or part in the tile
@@ -367,32 +394,52 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
         }
     };
     const auto second = [&](const Pass &p) { return kPassTiles == 2u && p.j + min(wave, p.n - 1u) >= ipt ? 1u : 0u; };      // the wave's item is of the pass's second tile
+    const auto last_tile = [&](const Pass &p) { return p.tile + (p.j + p.n > ipt ? 1u : 0u); };
+    Pass p = pass_at(i0, tile0, i0 - tile0 * parts);
+    // As in gate/up, what the first products wait for is on its way before the tables are built, and no thread skips a request: the codebook, the run's tiles, the
+    // first pass's rows, the activations of the run's first two tiles.
+    TableSeeds<SRC, T> seeds;
+    SmallSeeds<SRC, T> small_seeds;
+    if (tables) {
+        if constexpr (small_tables<SRC>()) small_seeds.request(tid, a.grid);
+        else seeds.request(tid, a.grid);
+    }
+    const uint32_t info_at = min(tid, n_info - 1u), info_e = list.expert[tile0 + info_at], info_p0 = list.pair0[tile0 + info_at], info_n = list.n[tile0 + info_at];
+    const auto mat_of = [&](uint32_t e) { return e == kSharedTile ? (uint64_t)(a.shared - a.experts) : (uint64_t)e * a.stride; };
+    const auto listed = [&](uint32_t t) { return TileInfo{mat_of(uni(list.expert[t])), uni(list.pair0[t]), uni(list.n[t])}; };
+    const TileInfo first[2] = {listed(tile0), listed(tile0 + min(1u, n_info - 1u))};
     // the lane's quarters of a block of the wave's two row tiles, and what their d are made from
     struct Carried { Quarter v[2]; uint2 d[2]; };
-    struct { Pass p; uint64_t mat; uint32_t kb; } ahead;   // the block to be requested next
-    ahead.p = pass_at(i0, tile0, i0 - tile0 * parts);
-    ahead.mat = info_of(tile0 + second(ahead.p)).mat;
-    ahead.kb = 0u;
-    Pass p = ahead.p;
-    const auto request = [&](Carried &c) {                 // (a wave without an item requests the pass's last)
-        const uint32_t item = ahead.p.j + min(wave, ahead.p.n - 1u) - second(ahead.p) * ipt;
+    const auto request_block = [&](Carried &c, const Pass &p, uint64_t mat, uint32_t kb) {      // (a wave without an item requests the pass's last)
+        const uint32_t item = p.j + min(wave, p.n - 1u) - second(p) * ipt;
 #pragma unroll
-        for (uint32_t m = 0; m < 2u; ++m) request_quarter<SRC, KP>(a, a.experts + ahead.mat, 2u * item + m, r, ahead.kb, q, c.v[m], c.d[m]);
-        if (++ahead.kb < KP) return;
-        ahead.kb = 0u;
-        ahead.p = following(ahead.p);
-        ahead.mat = info_of(ahead.p.tile + second(ahead.p)).mat;
+        for (uint32_t m = 0; m < 2u; ++m) request_quarter<SRC, KP>(a, a.experts + mat, 2u * item + m, r, kb, q, c.v[m], c.d[m]);
     };
-    // f32 activations of four pairs and a block per wave: one exponent for a pair's block, then the fp16 halves
-    const auto stage = [&](uint32_t tile) {
-        const TileInfo ti = info_of(tile);
-        for (uint32_t w = wave; w < KP * SETS * 4u; w += WV) {
-            const uint32_t block = w / (SETS * 4u), i = (w % (SETS * 4u)) * 4u + q;
-            const float *src = a.act + (uint64_t)(i < ti.n ? ti.p0 + i : ti.p0) * K + 256u * block + 4u * r;
-            float4 v[4];
-            float amax = 0.0f;
+    Carried c[2];
+    TileInfo now = first[second(p)];                       // the tile of the wave's item of pass p
+    struct { Pass p; TileInfo info, before; uint32_t kb; } ahead{p, now, now, KP > 1u ? 2u % KP : 1u % KP};      // the block to be requested next; `before`: of the pass before it
+    request_block(c[0], p, now.mat, 0u);
+    if constexpr (KP > 1u) request_block(c[1], p, now.mat, 1u);
+    __builtin_amdgcn_sched_barrier(0);
+    // f32 activations of four pairs and a block per wave: one exponent for a pair's block, then the fp16 halves. Requested a tile ahead, kept in registers.
+    constexpr uint32_t NS = (KP * PAIRS / 4u + WV - 1u) / WV;
+    struct Staged { float4 v[NS][4]; };
+    const auto fetch_tile = [&](Staged &st, uint32_t p0, uint32_t n) {
 #pragma unroll
-            for (uint32_t k = 0; k < 4u; ++k) v[k] = *reinterpret_cast<const float4 *>(src + 64u * k);
+        for (uint32_t x = 0; x < NS; ++x) {
+            const uint32_t w = min(wave + x * WV, KP * PAIRS / 4u - 1u), block = w / (PAIRS / 4u), i = (w % (PAIRS / 4u)) * 4u + q;
+            const float *src = a.act + (uint64_t)(i < n ? p0 + i : p0) * K + 256u * block + 4u * r;
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) st.v[x][k] = *reinterpret_cast<const float4 *>(src + 64u * k);
+        }
+    };
+    const auto put_tile = [&](const Staged &st, uint32_t tile) {
+#pragma unroll
+        for (uint32_t x = 0; x < NS; ++x) {
+            const uint32_t w = wave + x * WV, block = w / (PAIRS / 4u), i = (w % (PAIRS / 4u)) * 4u + q;
+            if (w >= KP * PAIRS / 4u) break;
+            const float4 *v = st.v[x];
+            float amax = 0.0f;
 #pragma unroll
             for (uint32_t k = 0; k < 4u; ++k) amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[k].x), fabsf(v[k].y)), fmaxf(fabsf(v[k].z), fabsf(v[k].w))));
             const int e = prescale_exp(row_max(amax));
@@ -410,14 +457,53 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
                 }
                 // columns 64 k + 4 r .. + 3: eight of step s and lane quarter sq, their half r % 2
                 const uint32_t c8 = 8u * k + r / 2u, s = fmt<SRC>() == F_IQ3_WORDS ? 4u * (c8 >> 4) + ((c8 >> 2) & 3u) : c8 & 7u, sq = fmt<SRC>() == F_IQ3_WORDS ? c8 & 3u : c8 >> 3;
-                uint8_t *at = lds.x + ((SETS == 2 ? i / 16u : kPassTiles == 2u ? tile & 1u : 0u) * KP + block) * kPanel + (s * 64u + sq * 16u + (i & 15u)) * 16u + (r & 1u) * 8u;
+                uint8_t *at = lds.x + ((SETS == 2 ? i / 16u : kPassTiles == 2u ? tile & 1u : 0u) * KP + block) * PANEL + (s * 64u + sq * 16u + (i & 15u)) * 16u + (r & 1u) * 8u;
                 *reinterpret_cast<uint2 *>(at) = hi.u;
-                *reinterpret_cast<uint2 *>(at + 8192u) = lo.u;
+                *reinterpret_cast<uint2 *>(at + (SMALL ? 8u * 16u : 8192u)) = lo.u;      // (SMALL: the operand's rows 8 .. 15)
             }
         }
     };
+    constexpr bool kAhead = NS <= (uint32_t)SETS;          // as far as the registers hold them
+    Staged next;                                           // of tile `staged`
+    uint32_t staged = tile0;                               // tiles below it are in LDS or were
+    {
+        Staged st;
+        fetch_tile(st, first[0].p0, first[0].n);
+        if constexpr (kAhead) fetch_tile(next, first[1].p0, first[1].n);
+        __builtin_amdgcn_sched_barrier(0);
+        if (tables) {
+            if constexpr (small_tables<SRC>()) small_seeds.store(lds.entries, lds.signs, tid);
+            else seeds.store(lds.entries, lds.signs, tid);
+        }
+        if (tid < n_info) lds.tiles[tid] = TileInfo{mat_of(info_e), info_p0, info_n};
+        put_tile(st, staged++);
+    }
+    if constexpr (kPassTiles == 2u) {
+        if (staged <= last_tile(p)) {
+            if constexpr (!kAhead) fetch_tile(next, first[1].p0, first[1].n);
+            put_tile(next, staged++);
+        }
+    }
+    wave_lds_barrier();
+    const LaneTables lt = lane_tables<SRC>(lds.entries, lds.signs, tid);
+    const auto info_of = [&](uint32_t tile) { return uniform_info(lds.tiles[tile - tile0]); };
+    const auto fetch_next = [&] { const TileInfo t = info_of(min(staged, tile0 + n_info - 1u)); fetch_tile(next, t.p0, t.n); };
+    const auto advance = [&] {
+        ahead.kb = 0u;
+        ahead.p = following(ahead.p);
+        ahead.before = ahead.info;
+        ahead.info = info_of(ahead.p.tile + second(ahead.p));
+    };
+    const auto request = [&](Carried &c) {
+        request_block(c, ahead.p, ahead.info.mat, ahead.kb);
+        if (++ahead.kb == KP) advance();
+    };
+    if constexpr (KP <= 2u) advance();
+    if constexpr (KP == 1u) request(c[1]);
+    if constexpr (kAhead) { if (staged > tile0 + 1u) fetch_next(); }
     // Precision: as in gate/up, but a row's blocks are added up in f32, so the chains are half as long.
     constexpr uint32_t kChain = 2u;
+    const float row_scale = SMALL && q >= 2u ? 4.8828125e-4f : 1.0f;      // of the lane's rows of the products
     float4_t sum[2][SETS];
     const auto clear = [&] {
 #pragma unroll
@@ -427,7 +513,7 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
     };
     // adds the products of the block whose rows are in c
     const auto multiply = [&](const Carried &c, const uint8_t *x, const float *pair_scale) {
-        const auto operand = [&](uint32_t s, uint32_t half, uint32_t step) { return *reinterpret_cast<const half8_t *>(x + s * KP * kPanel + half * 8192u + 1024u * step); };
+        const auto operand = [&](uint32_t s, uint32_t half, uint32_t step) { return *reinterpret_cast<const half8_t *>(x + s * KP * PANEL + half * 8192u + 1024u * step); };
         float4_t acc[2][SETS], low[2][SETS], block[2][SETS];
         float d[2];
         Entry e[2];
@@ -435,6 +521,7 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
 #pragma unroll
         for (uint32_t m = 0; m < 2u; ++m) {
             d[m] = quarter_d<SRC>(c.d[m]);
+            if constexpr (SMALL) d[m] *= row_scale;
             e[m] = fetch_entry<SRC, 0u>(c.v[m], lt);
 #pragma unroll
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s) acc[m][s] = low[m][s] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -445,7 +532,7 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
             __builtin_amdgcn_sched_barrier(0);
             half8_t w[2], xh[SETS], xl[SETS];
 #pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) { xh[s] = operand(s, 0u, S); xl[s] = operand(s, 1u, S); }
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s) { xh[s] = operand(s, 0u, S); if constexpr (!SMALL) xl[s] = operand(s, 1u, S); }
 #pragma unroll
             for (uint32_t m = 0; m < 2u; ++m) {
                 if constexpr (steps_per_scale<SRC>() != 0u) { if constexpr (S % steps_per_scale<SRC>() == 0u) f[m] = step_scale<SRC, S>(c.v[m]); }
@@ -467,48 +554,56 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
             for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
                 for (uint32_t m = 0; m < 2u; ++m) acc[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[s], w[m], acc[m][s], 0, 0, 0);
+            if constexpr (!SMALL) {
 #pragma unroll
-            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
+                for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
-                for (uint32_t m = 0; m < 2u; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[s], w[m], low[m][s], 0, 0, 0);
+                    for (uint32_t m = 0; m < 2u; ++m) low[m][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[s], w[m], low[m][s], 0, 0, 0);
+            }
         });
 #pragma unroll
         for (uint32_t s = 0; s < (uint32_t)SETS; ++s) {
-            const float4_t ps = *reinterpret_cast<const float4_t *>(pair_scale + 16u * s + 4u * q);
+            const float4_t ps = *reinterpret_cast<const float4_t *>(pair_scale + 16u * s + 4u * (SMALL ? q & 1u : q));
 #pragma unroll
             for (uint32_t m = 0; m < 2u; ++m)
 #pragma unroll
-                for (int t = 0; t < 4; ++t) sum[m][s][t] = fmaf(fmaf(low[m][s][t], 4.8828125e-4f, block[m][s][t] + acc[m][s][t]), d[m] * ps[t], sum[m][s][t]);
+                for (int t = 0; t < 4; ++t) {
+                    const float both = SMALL ? block[m][s][t] + acc[m][s][t] : fmaf(low[m][s][t], 4.8828125e-4f, block[m][s][t] + acc[m][s][t]);
+                    sum[m][s][t] = fmaf(both, d[m] * ps[t], sum[m][s][t]);
+                }
         }
     };
-    // No wave may skip a store (as in gate/up): of a wave without an item every one falls out of the range.
+    // No wave may skip a store (as in gate/up): of a wave without an item every one falls out of the range. A lane's distance from the first output of
+    // the item is the same for every item. SMALL: the sums over high halves (lanes 0 .. 31) and over low ones meet, of the first row tile in the lower
+    // lanes and of the second in the upper ones.
+    const uint32_t out_at = 4u * ((SMALL ? 4u * (q & 1u) : 4u * q) * a.rows + (SMALL ? 16u * (q >> 1) : 0u) + r);
     const auto store_pass = [&] {
-        const uint32_t over = second(p), item = p.j + wave - over * ipt;
-        const TileInfo ti = info_of(p.tile + over);
-        const auto buf = pair_rows(ti.p0 < a.P ? a.tmp + (uint64_t)ti.p0 * a.rows : a.sh_tmp + (uint64_t)(ti.p0 - a.P) * a.rows, wave < p.n ? ti.n : 0u, a.rows);      // (a tile is routed or shared as a whole)
+        const uint32_t item = p.j + wave - second(p) * ipt;
+        const auto buf = pair_rows(now.p0 < a.P ? a.tmp + (uint64_t)now.p0 * a.rows : a.sh_tmp + (uint64_t)(now.p0 - a.P) * a.rows, wave < p.n ? now.n : 0u, a.rows);      // (a tile is routed or shared as a whole)
+        const uint32_t first_row = 4u * 32u * (wave < p.n ? item : 0u);
+        if constexpr (SMALL) {
 #pragma unroll
-        for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
+            for (uint32_t t = 0; t < 4u; ++t) {
+                uint32_t x = __float_as_uint(sum[0][0][t]), y = __float_as_uint(sum[1][0][t] );
+                swap32(x, y);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(__uint_as_float(x) + __uint_as_float(y)), buf, out_at + 4u * t * a.rows, first_row, 0);
+            }
+        } else {
 #pragma unroll
-            for (uint32_t m = 0; m < 2u; ++m)
+            for (uint32_t s = 0; s < (uint32_t)SETS; ++s)
 #pragma unroll
                 for (uint32_t t = 0; t < 4u; ++t)
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sum[m][s][t]), buf, 4u * ((16u * s + 4u * q + t) * a.rows + (2u * item + m) * 16u + r), 0, 0);
+#pragma unroll
+                    for (uint32_t m = 0; m < 2u; ++m)
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sum[m][s][t]), buf, out_at + 4u * (16u * s + t) * a.rows, first_row + 64u * m, 0);
+        }
     };
-    Carried c[2];
-    request(c[0]);
-    request(c[1]);
     const uint8_t *x_lane = lds.x + 16u * lane;
-    uint32_t kb = 0u, staged = tile0;                      // staged: tiles below it are in LDS or were
-    const auto last_tile = [&] { return p.tile + (p.j + p.n > ipt ? 1u : 0u); };
-    const auto stage_pass = [&] {
-        for (; staged <= last_tile(); ++staged) stage(staged);
-        wave_lds_barrier();
-    };
+    uint32_t kb = 0u;
     clear();
-    stage_pass();
     const auto block = [&](Carried &cc) {                  // false: the last one is done
         const uint32_t odd = (p.tile + second(p)) & 1u;
-        if (wave < p.n) multiply(cc, x_lane + ((kPassTiles == 2u ? odd : 0u) * KP + kb) * kPanel, lds.scales + (odd * KP + kb) * PAIRS);
+        if (wave < p.n) multiply(cc, x_lane + ((kPassTiles == 2u ? odd : 0u) * KP + kb) * PANEL, lds.scales + (odd * KP + kb) * PAIRS);
         request(cc);
         if (++kb < KP) return true;
         kb = 0u;
@@ -516,9 +611,14 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
         clear();
         if (last(p)) return false;
         p = following(p);
-        if (last_tile() >= staged) {
+        now = KP == 1u ? info_of(p.tile + second(p)) : KP == 2u ? ahead.before : ahead.info;
+        if (last_tile(p) >= staged) {
             wave_lds_barrier();                            // (nobody needs the tiles before the pass's any more)
-            stage_pass();
+            if constexpr (!kAhead) fetch_next();
+            put_tile(next, staged++);
+            if constexpr (kPassTiles == 2u) while (staged <= last_tile(p)) { fetch_next(); put_tile(next, staged++); }
+            wave_lds_barrier();
+            if constexpr (kAhead) fetch_next();
         }
         return true;
     };
@@ -548,7 +648,7 @@ __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) v
     const bool few = n1 < a.few;
     if (SETS == 2 && few) return;
     const uint32_t l = SETS == 2 ? 1u : few ? 0u : 2u, off = l * a.list_stride;
-    const uint32_t n_tiles = SETS == 2 ? n1 : few ? n0 : n2, n_big = DOWN || SETS == 2 ? n_tiles : few ? b0 : b2;      // the others are small ones
+    const uint32_t n_tiles = SETS == 2 ? n1 : few ? n0 : n2, n_big = SETS == 2 ? n_tiles : few ? b0 : b2;      // the others are small ones
     uint32_t per_tile = a.rows / (DOWN ? 32u : 16u * GateUp<SETS, DOWN ? 2u : KP>::NRT);
     if constexpr (DOWN && down_tiles_a_pass<SETS, KP>() == 1u) {
         // as many passes a tile as fill the rounds that the busiest workgroup has anyway
@@ -558,8 +658,9 @@ __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) v
     const TileList list{a.tile_expert + off, a.tile_pair0 + off, a.tile_n + off};
     // workgroups are dealt round-robin over the eight XCDs: neighbouring runs (which share tiles) go to one XCD's L2
     const uint32_t G = gridDim.x, at = G % 8u == 0u ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
-    // equal shares of the time: a unit of a small tile takes kSmallCost / kBigCost of another one's
-    constexpr uint32_t kBigCost = 5u, kSmallCost = 4u;
+    // Equal shares of the time: a unit of a small tile takes 0.8 of another one's (gate/up 1830 and 2250 cycles on IQ1_M, 2140 and 2290 on IQ2_XXS, down 2360
+    // and 2870). Parts are too few for that: six a workgroup, five or seven of which would last longer.
+    constexpr uint32_t kBigCost = 5u, kSmallCost = DOWN && down_tiles_a_pass<SETS, KP>() == 1u ? kBigCost : 4u;
     const uint32_t w_big = n_big * per_tile;
     const uint64_t cost = (uint64_t)w_big * kBigCost + (uint64_t)(n_tiles - n_big) * per_tile * kSmallCost;
     const auto border = [&](uint32_t i) {
@@ -571,8 +672,12 @@ __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) v
         const bool small = from >= w_big;
         const uint32_t to = min(small ? w1 : min(w1, w_big), (from / per_tile + kTileInfos) * per_tile);
         if (from != w0) __syncthreads();
-        if constexpr (DOWN) down_items<down_src<SRC, SETS, KP>(), SETS, KP>(a, list, per_tile, from, to, lds, from == w0);
-        else if constexpr (SETS == 1) {
+        if constexpr (DOWN) {
+            constexpr int DSRC = down_src<SRC, SETS, KP>();
+            if constexpr (SETS == 2) down_items<DSRC, SETS, KP, false>(a, list, per_tile, from, to, lds, from == w0);
+            else if (small) down_items<DSRC, SETS, KP, true>(a, list, per_tile, from, to, lds, from == w0);
+            else down_items<DSRC, SETS, KP, false>(a, list, per_tile, from, to, lds, from == w0);
+        } else if constexpr (SETS == 1) {
             if (small) gateup_units<SRC, SETS, KP, SHORT, true>(a, list, from, to, lds, from == w0);
             else gateup_units<SRC, SETS, KP, SHORT, false>(a, list, from, to, lds, from == w0);
         } else gateup_units<SRC, SETS, KP, SHORT, false>(a, list, from, to, lds, from == w0);

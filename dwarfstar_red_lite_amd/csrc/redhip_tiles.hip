@@ -63,6 +63,14 @@ __device__ __forceinline__ void request_quarter(const StagedArgs &a, const uint8
     load_quarter<SRC, KP>(mat + (uint64_t)row_tile * tile_bytes, mat + a.d_off + row_tile * (KP * 32u),
                           fmt<SRC>() == F_XS ? mat + a.d_off + (uint64_t)a.rows * KP * 2u + row_tile * (KP * 128u) : nullptr, r, kc, q, v, d);
 }
+// g / (1 + exp(-g)). The exponent's product with log2(e) as two floats, so that the result is as good as the exponential instruction; the quotient from the
+// reciprocal and one step on what it leaves over, infinities and NaN as a division gives them. A third of the instructions of expf and a division, and no
+// further off from double (both 0.4 units in the last place on average).
+__device__ __forceinline__ float silu(float g) {
+    const float c = __builtin_amdgcn_fmed3f(g, -128.0f, 128.0f), h = c * -1.44269502f, l = fmaf(c, -1.92596303e-8f, fmaf(c, -1.44269502f, -h));
+    const float e = __builtin_amdgcn_exp2f(h) * fmaf(l, 0.693147182f, 1.0f), d = 1.0f + e, r = __builtin_amdgcn_rcpf(d), x = g * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-x, d, g), r, x), d, g);
+}
 // rows `rows` long of the pairs of a tile: stores of pairs beyond n fall out of the range
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pair_rows(float *base, uint32_t n, uint32_t rows) { return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)(n * rows * 4u), 0x00027000); }
 
@@ -131,7 +139,7 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
             request_quarter<SRC, KP>(a, mm, j * NRT + rt, r, SETS == 1 ? 2u * kp + m : kp, q, c.v[m], c.d[m]);
         }
     };
-    constexpr uint32_t kCarried = SETS == 2 && fmt<SRC>() != F_XXS ? 1u : 2u;      // units on their way: two where the registers hold them
+    constexpr uint32_t kCarried = SETS == 2 && (fmt<SRC>() != F_XXS || layout<SRC>() == L_ROWS) ? 1u : 2u;      // units on their way: two where the registers hold them
     Carried c[kCarried];
     uint32_t tile = tile0, j = u0 % upt, ftile = tile0, fj = j, fleft = u1 - u0;      // f..: the unit to be requested next
     uint64_t fmat = mat_of(e0);
@@ -205,12 +213,15 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
     arrange_blocks();
     // The sums of UNITS units, the first of them number fj of tile ft, and their SwiGLU. No wave and no lane may skip a store: the loads of the next units are in flight in front of it, and the
     // compiler, which waits for them by counting memory operations in order, can count only what every path issues.
-    const auto reduce = [&](auto units, uint32_t ft, uint32_t fj, const float *pt) {
+    // (What is done for every output is counted here too: a thread's outputs are the same place of different units, so their pair, its distance in `act` and
+    // its scale are found once, and the tile stands in scalar registers.)
+    TileInfo here{fmat, first_p0, first_n};                // the tile of the unit that is multiplied
+    const auto reduce = [&](auto units, const TileInfo &of, uint32_t ft, uint32_t fj, const float *pt) {
         constexpr uint32_t UNITS = decltype(units)::value, OUT = 16u * (SMALL ? 8u : 16u), N = OUT * SETS * NRT * UNITS;      // OUT: a row tile's outputs, of sixteen pairs or of eight
+        const uint32_t at = each_trip(threadIdx.x) % OUT, pair0 = 4u * (at >> 6) + (at & 3u), out_at = 4u * (pair0 * a.rows + ((at >> 2) & 15u));
 #pragma unroll
         for (uint32_t base = 0; base < N; base += T) {
-            const uint32_t e = N < T ? min(tid, N - 1u) : base + tid;      // (surplus threads repeat the last element)
-            const uint32_t at = e % OUT, b = __builtin_amdgcn_readfirstlane((e / OUT) % (SETS * NRT)), un = __builtin_amdgcn_readfirstlane((e / OUT) / (SETS * NRT)), set = b % SETS, slot = b / SETS;
+            const uint32_t b = uni(((base + threadIdx.x) % N) / OUT), un = b / (SETS * NRT), set = b % SETS, slot = (b / SETS) % NRT;      // (surplus threads repeat others' outputs)
             const float *src = pt + un * G::kPart + slot * PK * G::kSums + set * 256u + at;
             constexpr uint32_t PARTS = SMALL ? 2u * PK : PK;      // SMALL: the sums over high and over low halves apart
             using Sum = std::conditional_t<(PARTS > 1u), double, float>;      // (a row's parts are added here)
@@ -221,17 +232,19 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
                 g[k] = src[off];
                 u[k] = src[off + SETS * 256u];
             }
+            uint32_t dt = ft - tile0, dj = fj + un;
+            TileInfo d = of;
+            if (dj >= upt) {
+                while (dj >= upt) { dj -= upt; ++dt; }
+                d = uniform_info(lds.tiles[dt]);
+            }
+            const float scale = lds.scales[dt * PAIRS + 16u * set + pair0];
 #pragma unroll
             for (uint32_t n = PARTS / 2u; n; n /= 2u)
 #pragma unroll
                 for (uint32_t k = 0; k < n; ++k) { g[k] += g[k + n]; u[k] += u[k + n]; }
-            uint32_t dt = ft - tile0, dj = fj + un;
-            while (dj >= upt) { dj -= upt; ++dt; }
-            const TileInfo d = uniform_info(lds.tiles[dt]);
-            const uint32_t i = 16u * set + 4u * (at >> 6) + (at & 3u);
-            const float scale = lds.scales[dt * PAIRS + i], gate = (float)g[0] * scale;
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((gate / (1.0f + expf(-gate))) * ((float)u[0] * scale)), pair_rows(a.act + (uint64_t)d.p0 * a.rows, d.n, a.rows),
-                                                  4u * (i * a.rows + dj * 16u * NRT + 16u * slot + ((at >> 2) & 15u)), 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(silu((float)g[0] * scale) * ((float)u[0] * scale)), pair_rows(a.act + (uint64_t)d.p0 * a.rows, d.n, a.rows),
+                                                  out_at + 64u * set * a.rows, 4u * (dj * 16u * NRT + 16u * slot), 0);
         }
     };
     const auto request_rows = [&](Carried &c) { request(c, fmat, fj); };
@@ -311,7 +324,7 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
                 }
         }
         advance();
-        if (++j == upt && u + 1u < u1) { j = 0u; load_tile(++tile); }
+        if (++j == upt && u + 1u < u1) { j = 0u; here = uniform_info(lds.tiles[++tile - tile0]); load_tile(tile); }
     };
     advance();
     // A buffer of partial sums is written again two barriers after its sums were complete; whoever adds them has passed one in between.
@@ -322,17 +335,19 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
     const auto turn = [&] { pt = pt == lds.part ? lds.part + UB * G::kPart : lds.part; };
     for (; UB > 1u && u + UB <= u1; u += UB) {
         const uint32_t t = tile, j0 = j;
+        const TileInfo of = here;
 #pragma unroll
         for (uint32_t k = 0; k < UB; ++k) unit(u + k, c[k % kCarried], pt + k * G::kPart);
         wave_lds_barrier();
-        reduce(all, t, j0, pt);
+        reduce(all, of, t, j0, pt);
         turn();
     }
     const auto single = [&](Carried &cc) {
         const uint32_t t = tile, j0 = j;
+        const TileInfo of = here;
         unit(u, cc, pt);
         wave_lds_barrier();
-        reduce(one, t, j0, pt);
+        reduce(one, of, t, j0, pt);
         turn();
         return ++u < u1;
     };

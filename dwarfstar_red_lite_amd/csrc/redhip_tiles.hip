@@ -72,7 +72,10 @@ __device__ __forceinline__ float silu(float g) {
     return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-x, d, g), r, x), d, g);
 }
 // rows `rows` long of the pairs of a tile: stores of pairs beyond n fall out of the range
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t pair_rows(float *base, uint32_t n, uint32_t rows) { return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)(n * rows * 4u), 0x00027000); }
+// (base and n are the same in every lane; said again here, or the store would be in a loop over the lanes that have the same ones)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pair_rows(float *rows_of_all, uint32_t p0, uint32_t n, uint32_t rows) {
+    return __builtin_amdgcn_make_buffer_rsrc(rows_of_all + (uint64_t)uni(p0) * rows, 0, (int)(uni(n) * rows * 4u), 0x00027000);
+}
 
 // ---- gate/up ----
 // SMALL: a tile of up to eight pairs, whose high and low halves are rows 0 .. 7 and 8 .. 15 of one operand: half the matrix instructions, half the
@@ -243,7 +246,7 @@ __device__ __forceinline__ void gateup_units(const StagedArgs &a, const TileList
             for (uint32_t n = PARTS / 2u; n; n /= 2u)
 #pragma unroll
                 for (uint32_t k = 0; k < n; ++k) { g[k] += g[k + n]; u[k] += u[k + n]; }
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(silu((float)g[0] * scale) * ((float)u[0] * scale)), pair_rows(a.act + (uint64_t)d.p0 * a.rows, d.n, a.rows),
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(silu((float)g[0] * scale) * ((float)u[0] * scale)), pair_rows(a.act, d.p0, d.n, a.rows),
                                                   out_at + 64u * set * a.rows, 4u * (dj * 16u * NRT + 16u * slot), 0);
         }
     };
@@ -594,7 +597,8 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
     const uint32_t out_at = 4u * ((SMALL ? 4u * (q & 1u) : 4u * q) * a.rows + (SMALL ? 16u * (q >> 1) : 0u) + r);
     const auto store_pass = [&] {
         const uint32_t item = p.j + wave - second(p) * ipt;
-        const auto buf = pair_rows(now.p0 < a.P ? a.tmp + (uint64_t)now.p0 * a.rows : a.sh_tmp + (uint64_t)(now.p0 - a.P) * a.rows, wave < p.n ? now.n : 0u, a.rows);      // (a tile is routed or shared as a whole)
+        const bool routed = uni(now.p0) < a.P;                 // (a tile is routed or shared as a whole)
+        const auto buf = pair_rows(routed ? a.tmp : a.sh_tmp, routed ? now.p0 : now.p0 - a.P, wave < p.n ? now.n : 0u, a.rows);
         const uint32_t first_row = 4u * 32u * (wave < p.n ? item : 0u);
         if constexpr (SMALL) {
 #pragma unroll

@@ -216,10 +216,22 @@ struct TileLists {
     uint32_t list_stride, shared_ntok;
 };
 #ifdef __HIPCC__
+// Prefix sums (each lane's own value included) of the sixteen lanes of a row and of a wave: DPP additions, no trip to LDS as a shuffle is.
+__device__ __forceinline__ uint32_t row_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);      // row_shr 1, 2, 4, 8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+}
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v = row_scan(v);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);      // row_bcast 15 into rows 1 and 3, row_bcast 31 into rows 2 and 3
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
+}
 // By all 1024 threads of one workgroup: thread u < U brings its group's expert and run (first pair p0, n pairs), the others n = 0;
 // wave_total: LDS scratch. Exclusive prefix sums of the tiles per group, then every group writes its tiles.
 __device__ __forceinline__ void build_tile_lists(uint32_t expert, uint32_t p0, uint32_t n, uint32_t P, const TileLists &tl, uint32_t (*wave_total)[16]) {
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
+    const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63u;
     // tiles of m pairs in the three lists; a small one (a group has at most one, its last) counts kSmall, so that one sum has both numbers
     constexpr uint32_t kSmall = 1u << 21, kOthers = kSmall - 1u;
     auto counts = [](uint32_t m, uint32_t *c) {
@@ -232,21 +244,16 @@ __device__ __forceinline__ void build_tile_lists(uint32_t expert, uint32_t p0, u
     counts(n, mine);
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
-        scan[l] = mine[l];
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t up = __shfl_up(scan[l], o, 64);
-            if (lane >= (uint32_t)o) scan[l] += up;
-        }
+        scan[l] = wave_scan(mine[l]);
         if (lane == 63u) wave_total[l][wave] = scan[l];
     }
     __syncthreads();
     uint32_t sh[3];
     counts(tl.shared_ntok, sh);
+    const uint32_t waves = row_scan(wave_total[min(lane >> 4, 2u)][lane & 15u]);      // list l in row l
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
-        uint32_t base = scan[l] - mine[l], routed = 0u;
-        for (uint32_t w = 0; w < 16u; ++w) { if (w < wave) base += wave_total[l][w]; routed += wave_total[l][w]; }
+        const uint32_t routed = __builtin_amdgcn_readlane(waves, 16 * l + 15), base = scan[l] - mine[l] + (wave ? __builtin_amdgcn_readlane(waves, 16 * l + wave - 1) : 0u);
         const uint32_t off = (uint32_t)l * tl.list_stride, others = (routed & kOthers) + (sh[l] & kOthers);
         // tile t of a run of m pairs that starts at pair q0, in list l
         auto put = [&](uint32_t at, uint32_t e, uint32_t q0, uint32_t m, uint32_t t) {

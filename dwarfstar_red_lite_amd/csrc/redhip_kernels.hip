@@ -845,131 +845,140 @@ hipError_t launch_weighted_sum(const float *tmp, const float *weights, uint32_t 
 
 // ---------------------------------------------------------------- token grouping (pair sort)
 
-// exclusive prefix sum over the 1024 threads of a workgroup (16 waves): in-wave shuffles, then the 16 wave totals
-__device__ __forceinline__ uint32_t block_scan_1024(uint32_t v, uint32_t *wave_tot /* [17] */, uint32_t &total) {
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint32_t inc = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) { const uint32_t n = __shfl_up(inc, o, 64); if (lane >= (uint32_t)o) inc += n; }
+// exclusive prefix sum over the 1024 threads of a workgroup (16 waves); wave_tot: read until the next barrier
+__device__ __forceinline__ uint32_t block_scan_1024(uint32_t v, uint32_t *wave_tot /* [16] */, uint32_t &total) {
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), inc = wave_scan(v);
     if (lane == 63u) wave_tot[wave] = inc;
     __syncthreads();
-    if (threadIdx.x == 0u) {
-        uint32_t acc = 0u;
-#pragma unroll
-        for (int w = 0; w < 16; ++w) { const uint32_t t = wave_tot[w]; wave_tot[w] = acc; acc += t; }
-        wave_tot[16] = acc;
-    }
-    __syncthreads();
-    total = wave_tot[16];
-    const uint32_t ex = wave_tot[wave] + inc - v;
-    __syncthreads();                               // wave_tot may be reused right away
-    return ex;
+    const uint32_t waves = row_scan(wave_tot[lane & 15u]);
+    total = __builtin_amdgcn_readlane(waves, 15);
+    return (wave ? __builtin_amdgcn_readlane(waves, wave - 1u) : 0u) + inc - v;
 }
 
-// One workgroup. For every (token, k) pair p = t * top_k + k:
+// One workgroup, up to 512 tokens. For every (token, k) pair p = t * top_k + k:
 //   first[e]   = smallest p that names expert e            -> experts numbered in first-appearance order
 //   member[e]  = bitmap over tokens that selected e        -> rank of a pair inside its expert = popcount below t
-// which gives the stable counting sort of the host loop it replaces without a serial pass. All of it runs on one
-// compute unit, so the instruction count is what it costs: the token of a pair comes from a multiply-high by
-// ceil(2^32 / top_k) (exact while pairs * top_k < 2^32), and with PREFIX the bit counts of the words below a token's word come
-// from a table made once per expert (which also yields the expert's pair count) instead of a loop per pair.
+// which gives the stable counting sort of the host loop it replaces without a serial pass. All of it runs on one compute unit behind nothing
+// that could hide it, so what it costs is the trips to LDS that follow one another and the instruction count: the token of a pair comes from a
+// multiply-high by ceil(2^32 / top_k) (exact while pairs * top_k < 2^32), the bit counts of the words below a token's word from a table made
+// once per expert (which also yields the expert's pair count), the number of an expert from a bitmap of the first pairs and the counts below
+// its words, an expert's start stands with the expert, prefix sums are DPP additions, and no read-back of an LDS atomic is waited for before
+// the last one is on its way.
 // An expert's words lie an odd number of words behind the last one's: the pairs of a wave belong to tokens near each other, so they all
 // use the same word of their experts, and with sixteen words per expert (512 tokens) these were in a few LDS banks.
-template <bool PREFIX>
+constexpr uint32_t kGroupTokens = 512u, kGroupPairs = 8192u;      // most tokens, most pairs (eight per thread, 256 words of first pairs)
+static __host__ __device__ uint32_t group_member_words(uint32_t n_expert, uint32_t ntok) { return (n_expert * (((ntok + 31u) / 32u) | 1u) + 3u) & ~3u; }
+static size_t group_pairs_lds(uint32_t n_expert, uint32_t ntok, uint32_t P) {
+    const size_t sorted = sizeof(uint2) * P, tables = sizeof(uint32_t) * ((size_t)2u * group_member_words(n_expert, ntok) + 2u * n_expert + 2u * 1024u + 2u * (kGroupPairs / 32u) + 4u + 16u);
+    return sorted > tables ? sorted : tables;
+}
 __global__ __launch_bounds__(1024) void group_pairs_kernel(const uint32_t *ids, const float *weights, uint32_t ntok, uint32_t top_k, uint32_t top_k_magic,
                                                            uint32_t n_expert, uint32_t *uid, uint32_t *expert_start,
                                                            uint32_t *pair_token, float *pair_weight, uint32_t *tok_pair,
-                                                           uint32_t *n_unique, uint32_t *status, uint32_t cache_ids, TileLists tiles) {
-    extern __shared__ uint32_t sm[];
+                                                           uint32_t *n_unique, uint32_t *status, TileLists tiles) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t sm[];
     __shared__ uint32_t tile_tot[3][16];
-    const uint32_t words = (ntok + 31u) / 32u, stride = words | 1u, P = ntok * top_k, tid = threadIdx.x;
-    uint32_t *first = sm;                          // [n_expert]
-    uint32_t *count = first + n_expert;            // [n_expert]
-    uint32_t *dense = count + n_expert;            // [n_expert]
-    uint32_t *start = dense + n_expert;            // [n_expert + 1] by dense index
-    uint32_t *uid_l = start + n_expert + 1u;       // [1024] experts by dense index (n_expert <= 1024)
-    uint32_t *wave_tot = uid_l + 1024u;            // [17]
-    uint32_t *member = wave_tot + 17u;             // [n_expert][stride]
-    uint32_t *below = member + n_expert * stride;  // [n_expert][stride] when PREFIX: members in the words before this one
-    uint32_t *ids_l = cache_ids ? below + (PREFIX ? n_expert * stride : 0u) : nullptr;      // [P] the clamped ids, when LDS has room: the later passes need no second trip to device memory
+    constexpr uint32_t FW = kGroupPairs / 32u, N = kGroupPairs / 1024u;
+    const uint32_t words = (ntok + 31u) / 32u, stride = words | 1u, P = ntok * top_k, tid = threadIdx.x, lane = tid & 63u, mw = group_member_words(n_expert, ntok);
+    uint32_t *member = sm;                         // [n_expert][stride]
+    uint32_t *below = member + mw;                 // [n_expert][stride] members in the words before this one
+    uint32_t *first = below + mw;                  // [n_expert]
+    uint32_t *base = first + n_expert;             // [n_expert] the expert's first place
+    uint32_t *uid_l = base + n_expert;             // [1024] experts in first-appearance order (n_expert <= 1024)
+    uint32_t *count = uid_l + 1024u;               // [1024] their pairs
+    uint32_t *firsts = count + 1024u;              // [FW] bitmap of the pairs that are their expert's first
+    uint32_t *before = firsts + FW;                // [FW] first pairs in the words of the same 64 before this one
+    uint32_t *first_tot = before + FW;             // [4] of each 64 words
+    uint32_t *wave_tot = first_tot + 4u;           // [16]
     auto token_of = [&](uint32_t p) { return top_k == 1u ? p : __umulhi(p, top_k_magic); };
-    // the ids are the caller's: clamped into the tables (reported once, in the first pass)
-    auto id_of = [&](uint32_t p) { if (ids_l) return ids_l[p]; const uint32_t e = ids[p]; return e < n_expert ? e : n_expert - 1u; };
-    // Up to eight pairs per thread (chunks of up to 8192 pairs) are requested here, ids and weights, before anything else: read inside the
-    // passes below, each would be a round trip of its own (the stores of the last pass keep the loads of the next pair behind them).
-    constexpr uint32_t kRegPairs = 8u;
-    const bool in_regs = P <= kRegPairs * 1024u;
-    uint32_t ereg[kRegPairs];
-    float wreg[kRegPairs];
-    if (in_regs) {
+    // A thread's pairs, ids and weights, are requested here, before anything else: read inside the passes below, each would be a round trip of
+    // its own (the stores of the last pass keep the loads of the next pair behind them).
+    uint32_t ereg[N];
+    float wreg[N];
 #pragma unroll
-        for (uint32_t j = 0; j < kRegPairs; ++j) {
-            const uint32_t p = tid + 1024u * j;
-            ereg[j] = p < P ? ids[p] : 0u;
-            wreg[j] = p < P ? weights[p] : 0.0f;
+    for (uint32_t j = 0; j < N; ++j) {
+        const uint32_t p = tid + 1024u * j;
+        ereg[j] = p < P ? ids[p] : 0u;
+        wreg[j] = p < P ? weights[p] : 0.0f;
+    }
+    for (uint32_t i = tid; i < mw / 4u; i += 1024u) reinterpret_cast<uint4 *>(member)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (tid < n_expert) first[tid] = 0xffffffffu;
+    if (tid < FW) firsts[tid] = 0u;
+    __syncthreads();
+    uint32_t bad = 0u;                             // bit 0: an id out of range (clamped), bit 1: the token names this expert twice
+    uint32_t old[N];
+#pragma unroll
+    for (uint32_t j = 0; j < N; ++j) {
+        const uint32_t p = tid + 1024u * j, t = token_of(p);
+        old[j] = 0u;
+        if (p < P) {
+            if (ereg[j] >= n_expert) { bad |= 1u; ereg[j] = n_expert - 1u; }
+            atomicMin(&first[ereg[j]], p);
+            old[j] = atomicOr(&member[ereg[j] * stride + (t >> 5)], 1u << (t & 31u));
         }
     }
-    for (uint32_t i = tid; i < n_expert; i += 1024u) { first[i] = 0xffffffffu; count[i] = 0u; dense[i] = 0u; }
-    for (uint32_t i = tid; i < n_expert * stride; i += 1024u) member[i] = 0u;
-    __syncthreads();
-    auto enter = [&](uint32_t p, uint32_t raw) {
-        const uint32_t e = guarded_id(raw, n_expert, status), t = token_of(p);
-        if (ids_l) ids_l[p] = e;
-        atomicMin(&first[e], p);
-        if constexpr (!PREFIX) atomicAdd(&count[e], 1u);
-        if ((atomicOr(&member[e * stride + (t >> 5)], 1u << (t & 31u)) & (1u << (t & 31u))) && status) atomicOr(status, 2u);      // the token names this expert twice
-        return e;
-    };
-    if (in_regs) {
 #pragma unroll
-        for (uint32_t j = 0; j < kRegPairs; ++j) { const uint32_t p = tid + 1024u * j; if (p < P) ereg[j] = enter(p, ereg[j]); }
-    } else {
-        for (uint32_t p = tid; p < P; p += 1024u) enter(p, ids[p]);
-    }
+    for (uint32_t j = 0; j < N; ++j) bad |= __builtin_amdgcn_ubfe(old[j], token_of(tid + 1024u * j) & 31u, 1u) << 1;
+    if (bad && status) atomicOr(status, bad);
     __syncthreads();
-    if constexpr (PREFIX) {
-        for (uint32_t e = tid; e < n_expert; e += 1024u) {
-            uint32_t run = 0u;
-            for (uint32_t w = 0; w < words; ++w) { below[e * stride + w] = run; run += __popc(member[e * stride + w]); }
-            count[e] = run;
+    uint32_t mine = 0u, my_first = 0xffffffffu;      // of expert tid: pairs, first pair
+    if (tid < n_expert) {
+        my_first = first[tid];
+        if (my_first != 0xffffffffu) atomicOr(&firsts[my_first >> 5], 1u << (my_first & 31u));
+        for (uint32_t w0 = 0; w0 < words; w0 += 4u) {
+            uint32_t m[4];
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; ++i) m[i] = w0 + i < words ? member[tid * stride + w0 + i] : 0u;
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; ++i) {
+                if (w0 + i < words) below[tid * stride + w0 + i] = mine;
+                mine += __popc(m[i]);
+            }
         }
     }
-    // exclusive scan of "pair p is the first appearance of its expert", P elements in per-thread runs
-    const uint32_t per = (P + 1023u) / 1024u;
-    uint32_t mine = 0u;
-    for (uint32_t j = 0; j < per; ++j) { const uint32_t p = tid * per + j; if (p < P && first[id_of(p)] == p) ++mine; }
-    uint32_t U = 0u;
-    uint32_t run = block_scan_1024(mine, wave_tot, U);
-    for (uint32_t j = 0; j < per; ++j) {
-        const uint32_t p = tid * per + j;
-        if (p < P && first[id_of(p)] == p) { const uint32_t e = id_of(p); dense[e] = run; uid_l[run] = e; uid[run] = e; ++run; }
+    __syncthreads();
+    if (tid < FW) {
+        const uint32_t n = __popc(firsts[tid]), inc = wave_scan(n);
+        before[tid] = inc - n;
+        if (lane == 63u) first_tot[tid >> 6] = inc;
     }
     __syncthreads();
-    // exclusive scan of the per-expert pair counts in dense order (U <= n_expert <= 1024: one per thread)
+    static_assert(FW == 4u * 64u, "");
+    const uint32_t n0 = first_tot[0], n1 = n0 + first_tot[1], n2 = n1 + first_tot[2], U = n2 + first_tot[3];
+    if (my_first != 0xffffffffu) {
+        const uint32_t word = my_first >> 5, seg = word >> 6;
+        const uint32_t d = (seg == 0u ? 0u : seg == 1u ? n0 : seg == 2u ? n1 : n2) + before[word] + __popc(firsts[word] & ((1u << (my_first & 31u)) - 1u));
+        uid_l[d] = tid; uid[d] = tid; count[d] = mine;
+    }
+    __syncthreads();
+    const uint32_t my_expert = tid < U ? uid_l[tid] : 0u, my_count = tid < U ? count[tid] : 0u;      // of expert number tid
     uint32_t all = 0u;
-    const uint32_t my_start = block_scan_1024(tid < U ? count[uid_l[tid]] : 0u, wave_tot, all);
-    if (tid < U) { start[tid] = my_start; expert_start[tid] = my_start; }
-    if (tid == 0u) { start[U] = all; expert_start[U] = all; n_unique[0] = U; }
+    const uint32_t my_start = block_scan_1024(my_count, wave_tot, all);
+    if (tid < U) { base[my_expert] = my_start; expert_start[tid] = my_start; }
+    if (tid == 0u) { expert_start[U] = all; n_unique[0] = U; }
     __syncthreads();
-    auto place = [&](uint32_t p, uint32_t e, float wt) {
-        const uint32_t t = token_of(p);
-        const uint32_t *bits = member + e * stride;
-        uint32_t rank = __popc(bits[t >> 5] & ((1u << (t & 31u)) - 1u));
-        if constexpr (PREFIX) rank += below[e * stride + (t >> 5)];
-        else for (uint32_t w = 0; w < (t >> 5); ++w) rank += __popc(bits[w]);
-        const uint32_t pos = start[dense[e]] + rank;
-        pair_token[pos] = t;
-        pair_weight[pos] = wt;
-        tok_pair[p] = pos;
-    };
-    if (in_regs) {
+    // sorted in LDS (where the tables were) and stored side by side: one compute unit stores 64 places far apart in 64 cycles
+    uint2 *sorted = reinterpret_cast<uint2 *>(sm);
+    uint32_t pos[N];
 #pragma unroll
-        for (uint32_t j = 0; j < kRegPairs; ++j) { const uint32_t p = tid + 1024u * j; if (p < P) place(p, ereg[j], wreg[j]); }
-    } else {
-        for (uint32_t p = tid; p < P; p += 1024u) place(p, id_of(p), weights[p]);
+    for (uint32_t j = 0; j < N; ++j) {
+        const uint32_t p = tid + 1024u * j, t = token_of(p), at = ereg[j] * stride + (t >> 5);
+        if (p < P) tok_pair[p] = pos[j] = base[ereg[j]] + below[at] + __popc(member[at] & ((1u << (t & 31u)) - 1u));
     }
-    // the tile lists of the prefill kernels, from the group starts still in LDS: no launch of their own
-    if (tiles.tile_expert) build_tile_lists(tid < U ? uid_l[tid] : 0u, tid < U ? start[tid] : 0u, tid < U ? start[tid + 1u] - start[tid] : 0u, P, tiles, tile_tot);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < N; ++j) {
+        const uint32_t p = tid + 1024u * j;
+        if (p < P) sorted[pos[j]] = make_uint2(token_of(p), __float_as_uint(wreg[j]));
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < all; i += 1024u) {          // (`all` is less than P where a token names an expert twice)
+        const uint2 v = sorted[i];
+        pair_token[i] = v.x;
+        pair_weight[i] = __uint_as_float(v.y);
+    }
+    // the tile lists of the prefill kernels: no launch of their own
+    if (tiles.tile_expert) build_tile_lists(my_expert, my_start, my_count, P, tiles, tile_tot);
 }
 
 // The same sort for chunks of more than 512 tokens, whose token bitmaps per expert would not fit the LDS (2048 tokens x 512 experts: 128
@@ -977,7 +986,7 @@ __global__ __launch_bounds__(1024) void group_pairs_kernel(const uint32_t *ids, 
 // appearances and the pair counts of the experts come from one pass over all pairs, then the pairs are placed block by block of 512
 // tokens - bitmaps and prefix counts of one block (32 KB each), a cursor per expert that advances by the block's count. Same outputs in
 // the same (stable) order; one workgroup, the time grows with the number of blocks.
-constexpr uint32_t kGroupBlockTokens = 512u, kGroupBlockWords = kGroupBlockTokens / 32u;
+constexpr uint32_t kGroupBlockTokens = kGroupTokens, kGroupBlockWords = kGroupBlockTokens / 32u;
 __global__ __launch_bounds__(1024) void group_pairs_blocked_kernel(const uint32_t *ids, const float *weights, uint32_t ntok, uint32_t top_k, uint32_t top_k_magic,
                                                                    uint32_t n_expert, uint32_t *uid, uint32_t *expert_start,
                                                                    uint32_t *pair_token, float *pair_weight, uint32_t *tok_pair,
@@ -1194,18 +1203,8 @@ hipError_t launch_group_pairs(const uint32_t *ids, const float *weights, uint32_
                               uint32_t *tok_pair, uint32_t *n_unique, hipStream_t s, const TileLists *tiles, const GroupScratch *scratch) {
     if (!ntok || !top_k || !n_expert || n_expert > 1024u || (uint64_t)ntok * top_k * top_k >= (1ull << 32)) return hipErrorInvalidValue;
     const TileLists tl = tiles ? *tiles : TileLists{};
-    const uint32_t words = (ntok + 31u) / 32u;
-    const size_t lds = sizeof(uint32_t) * ((size_t)4u * n_expert + 1u + 1024u + 17u + (size_t)n_expert * (words | 1u));
     constexpr size_t kGroupDynLds = 159u * 1024u;      // (the kernel has a little static LDS beside it)
-    const size_t lds_prefix = lds + sizeof(uint32_t) * (size_t)n_expert * (words | 1u);
     const uint32_t magic = (uint32_t)(((1ull << 32) + top_k - 1u) / top_k);      // top_k == 1 needs none (and would not fit)
-    static bool attr_set = false;
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(group_pairs_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGroupDynLds);
-        if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(group_pairs_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGroupDynLds);
-        if (e != hipSuccess) return e;
-        attr_set = true;
-    }
     if (scratch && ntok > kGroupBlockTokens && (ntok + kGroupSpan - 1u) / kGroupSpan <= scratch->blocks && top_k <= 16u) {      // many workgroups, three launches
         const uint32_t nb = (ntok + kGroupSpan - 1u) / kGroupSpan;
         REDHIP_LAUNCH(group_count_kernel, dim3(nb), dim3(256), 0, s, ids, ntok, top_k, n_expert, *scratch, route_guard().status);
@@ -1216,7 +1215,8 @@ hipError_t launch_group_pairs(const uint32_t *ids, const float *weights, uint32_
     }
     const size_t ids_bytes = sizeof(uint32_t) * (size_t)ntok * top_k;
     const size_t lds_blocked = sizeof(uint32_t) * ((size_t)5u * n_expert + 1u + 1024u + 17u + (size_t)2u * n_expert * kGroupBlockWords);
-    if (ntok > kGroupBlockTokens && lds_blocked <= kGroupDynLds) {       // larger chunks: block by block
+    if (ntok > kGroupTokens) {                           // larger chunks: block by block
+        if (lds_blocked > kGroupDynLds) return hipErrorInvalidValue;      // (1024 experts take 155 KB)
         static bool blocked_attr = false;
         if (!blocked_attr) {
             const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(group_pairs_blocked_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGroupDynLds);
@@ -1228,16 +1228,16 @@ hipError_t launch_group_pairs(const uint32_t *ids, const float *weights, uint32_
                       pair_token, pair_weight, tok_pair, n_unique, route_guard().status, cache ? 1u : 0u, tl);
         return hipGetLastError();
     }
-    if (lds > kGroupDynLds) return hipErrorInvalidValue;
-    if (lds_prefix <= kGroupDynLds) {
-        const bool cache = lds_prefix + ids_bytes <= kGroupDynLds;
-        REDHIP_LAUNCH(group_pairs_kernel<true>, dim3(1), dim3(1024), lds_prefix + (cache ? ids_bytes : 0u), s, ids, weights, ntok, top_k, magic, n_expert, uid, expert_start, pair_token,
-                      pair_weight, tok_pair, n_unique, route_guard().status, cache ? 1u : 0u, tl);
-    } else {
-        const bool cache = lds + ids_bytes <= kGroupDynLds;
-        REDHIP_LAUNCH(group_pairs_kernel<false>, dim3(1), dim3(1024), lds + (cache ? ids_bytes : 0u), s, ids, weights, ntok, top_k, magic, n_expert, uid, expert_start, pair_token,
-                      pair_weight, tok_pair, n_unique, route_guard().status, cache ? 1u : 0u, tl);
+    const size_t lds = group_pairs_lds(n_expert, ntok, ntok * top_k);
+    if (ntok * top_k > kGroupPairs || lds > kGroupDynLds) return hipErrorInvalidValue;      // (16 a token at most; 1024 experts and 512 tokens take 158 KB)
+    static bool attr_set = false;
+    if (!attr_set) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(group_pairs_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGroupDynLds);
+        if (e != hipSuccess) return e;
+        attr_set = true;
     }
+    REDHIP_LAUNCH(group_pairs_kernel, dim3(1), dim3(1024), lds, s, ids, weights, ntok, top_k, magic, n_expert, uid, expert_start, pair_token, pair_weight, tok_pair, n_unique,
+                  route_guard().status, tl);
     return hipGetLastError();
 }
 

@@ -206,3 +206,18 @@ def test_grouping_numbers_late_experts(ntok, E, K):
     for got, want in zip(m.group(dev(ids.astype(np.int32)), dev(w)), orc.group_pairs(ids, w, E)):
         assert np.array_equal(got.cpu().numpy().view(want.dtype), want)
     m.close()
+
+
+# one workgroup's sort: the smallest, the most pairs (8192: the sorted list is larger than the tables of few experts), the widest table with experts that first
+# appear in the last words of the first pairs
+@pytest.mark.parametrize("ntok,E,K", [(1, 1, 1), (9, 3, 2), (512, 16, 16), (511, 24, 16), (512, 1024, 16), (128, 1024, 16), (33, 1000, 1)])
+def test_grouping_by_one_workgroup(ntok, E, K):
+    from dwarfstar_red_lite_amd import moe
+    m = moe.ResidentMoe(synth.layer_config(hidden=256, ffn=256, n_expert=E, top_k=K), n_layer=1, max_tokens=ntok)
+    rng = np.random.default_rng(ntok + K)
+    ids = np.argsort(rng.random((ntok, max(K, E - 70))), axis=1)[:, :K].astype(np.uint32)
+    if E - 70 > K: ids[-1] = E - 1 - np.arange(K)      # never named before
+    w = rng.random((ntok, K)).astype(np.float32)
+    for got, want in zip(m.group(dev(ids.astype(np.int32)), dev(w)), orc.group_pairs(ids, w, E)):
+        assert np.array_equal(got.cpu().numpy().view(want.dtype), want)
+    m.close()

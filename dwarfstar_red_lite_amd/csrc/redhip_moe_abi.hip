@@ -660,8 +660,8 @@ redhip_moe_t redhip_moe_create(const redhip_moe_config *cfg) {
     m->act_l = w; w += align256(2u * TA * (c.top_k + 1u) * c.ffn);
     m->act_exp = reinterpret_cast<int *>(w); w += align256(4u * TA * (c.top_k + 1u) * (c.ffn / 32u));
     if (T > 8u && m->mixed) {
-        if (hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking) != hipSuccess || hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&m->ev_join, hipEventDisableTiming) != hipSuccess) {
+        if (hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking) != hipSuccess || hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess ||
+            hipEventCreateWithFlags(&m->ev_join, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) {
             moe_err("failed to create the side stream of the shared expert");
             redhip_moe_destroy(m);
             return nullptr;

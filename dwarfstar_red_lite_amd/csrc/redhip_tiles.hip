@@ -677,16 +677,30 @@ __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) v
     const TileList list{a.tile_expert + off, a.tile_pair0 + off, a.tile_n + off};
     // workgroups are dealt round-robin over the eight XCDs: neighbouring runs (which share tiles) go to one XCD's L2
     const uint32_t G = gridDim.x, at = G % 8u == 0u ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
-    // Equal shares of the time: a unit of a small tile takes 0.8 of another one's (gate/up 1830 and 2250 cycles on IQ1_M, 2140 and 2290 on IQ2_XXS, down 2360
-    // and 2870). Parts are too few for that: six a workgroup, five or seven of which would last longer.
-    constexpr uint32_t kBigCost = 5u, kSmallCost = DOWN && down_tiles_a_pass<SETS, KP>() == 1u ? kBigCost : 4u;
-    const uint32_t w_big = n_big * per_tile;
-    const uint64_t cost = (uint64_t)w_big * kBigCost + (uint64_t)(n_tiles - n_big) * per_tile * kSmallCost;
-    const auto border = [&](uint32_t i) {
-        const uint64_t c = i * cost / G, big = (uint64_t)w_big * kBigCost;
-        return c <= big ? (uint32_t)(c / kBigCost) : w_big + (uint32_t)((c - big) / kSmallCost);
-    };
-    const uint32_t w0 = border(at), w1 = border(at + 1u);
+    // Equal shares of the time, small tiles and others on workgroups of their own: one that went from the others to the small ones began again with an empty
+    // pipeline, 4 to 8 us behind all the rest (batch of 24 tokens, gate/up: ends at 41.6 us, the others at 34.4 on average). A unit of another tile takes 1.25
+    // to 1.6 times as long as a small one's: gate/up, 2048 columns 2.10 and 1.61 us IQ2_XXS, 1.95 and 1.46 IQ1_M, 2.43 and 1.96 IQ2_XS, 1024 columns 2.07 and
+    // 1.39; with popular experts, whose rows are at hand, 1.70 and 1.17; down 0.51 and 0.42, 0.49 and 0.38, 0.61 and 0.53, popular 0.48 and 0.45. Parts
+    // are too few for that: six a workgroup, five or seven of which would last longer; there whole rounds are dealt.
+    const uint32_t w_big = n_big * per_tile, w_small = (n_tiles - n_big) * per_tile;
+    uint32_t g_big = 0u;                                   // workgroups of the others; G: no such parting (no small tiles, or none but these)
+    if (SETS == 2 || !w_small) g_big = G;
+    else if constexpr (DOWN && down_tiles_a_pass<SETS, KP>() == 1u) {
+        const uint32_t rounds = (w_big + w_small + G - 1u) / G;
+        g_big = (w_big + rounds - 1u) / rounds;
+        if (g_big + (w_small + rounds - 1u) / rounds > G) g_big = G;
+    } else if (w_big) {
+        constexpr float kCost = DOWN ? 1.15f : KP == 8u ? 1.35f : 1.45f;
+        const float big = kCost * (float)w_big, small = (float)w_small;
+        const uint32_t g = min(max((uint32_t)((float)G * big / (big + small)), 1u), G - 1u), more = min(g + 1u, G - 1u);
+        const auto longest = [&](uint32_t n) { return fmaxf(big / (float)n, small / (float)(G - n)); };
+        g_big = G == 1u ? G : longest(more) < longest(g) ? more : g;
+    }
+    const bool parted = g_big < G, mine_small = parted && at >= g_big;
+    const uint32_t part_first = mine_small ? w_big : 0u, part = !parted ? w_big + w_small : mine_small ? w_small : w_big;
+    const uint32_t part_at = mine_small ? at - g_big : at, part_groups = !parted ? G : mine_small ? G - g_big : g_big;
+    const auto border = [&](uint32_t i) { return part_first + (uint32_t)((uint64_t)i * part / part_groups); };
+    const uint32_t w0 = border(part_at), w1 = border(part_at + 1u);
     for (uint32_t from = w0; from < w1;) {                 // (a run of more than kTileInfos tiles in parts, small tiles apart)
         const bool small = from >= w_big;
         const uint32_t to = min(small ? w1 : min(w1, w_big), (from / per_tile + kTileInfos) * per_tile);

@@ -145,19 +145,21 @@ struct Moe {
     // expert, on mixed layouts also the router), the tiles so many per distinct expert, each more for larger matrices, and their launches more than the
     // slices': both by the tokens' expected spread over the experts. Fitted to 1332 calls timed on both sides: 17 .. 32 tokens, 16 to 512 experts,
     // two to ten a token, 1024 x 512 to 2048 x 768, own router and routing given (that call does not know how it is spread: a line between even
-    // spread and 32 hot experts). Chosen so, a call is 0.4 % slower than on the quicker side on average. Slices / tiles, us:
-    // own router, 32 tokens of 2048 x 512: 512 experts, ten a token: IQ2_XXS 122 / 112, IQ1_M 135 / 111; four a token 74 / 81 and 84 / 78; 60 experts, two a
-    //   token 45 / 54 and 59 / 55; 32 experts, eight a token 79 / 48 and 95 / 60. 18 tokens: 512 experts, ten a token 80 / 85 and 89 / 88; 32 experts, eight a
-    //   token 53 / 52 and 63 / 57
-    // given, evenly / on 32 hot experts: 20 tokens of 2048 x 512, 512 experts, ten a token: IQ2_XXS 74 / 78 and 62 / 51; 23 tokens, 200 experts, eight a token:
-    //   IQ3_S down 71 / 61 (hot), IQ2_XS 85 / 87 and 74 / 61
+    // spread and 32 hot experts), and 746 more of 10 .. 32 tokens once small tiles cost half their matrix instructions. Beyond 64 experts one more costs the
+    // tiles 0.7 of one below: with fewer, workgroups wait for the longest run. Slices / tiles, us:
+    // own router, 2048 x 512: 512 experts, ten a token: 16 tokens IQ2_XXS 73 / 72, IQ1_M 79 / 74, IQ3_S down 80 / 81; 18 tokens 80 / 75, 89 / 76 and 88 / 83; 24 tokens
+    //   97 / 85, 108 / 86 and 109 / 93; four a token, 28 tokens 67 / 69, 79 / 65 and 79 / 70; 60 experts, two a token, 32 tokens 45 / 49, 61 / 48 and 60 / 52;
+    //   32 experts, eight a token, 18 tokens 53 / 48, 64 / 58 and 64 / 56
+    // given, evenly / on 32 hot experts: 18 tokens of 2048 x 512, 512 experts, ten a token: IQ2_XXS 70 / 67 and 58 / 50; 300 experts, six a token, 20 tokens: 53 / 55
+    //   and 45 / 40, IQ3_S down 70 / 66 and 58 / 50, IQ2_XS 73 / 70 and 60 / 51
     // Narrower experts (1024 x 256: 32 tokens, 96 experts, six a token 48 / 50 .. 52) stay slices.
     bool slices_ahead(uint32_t ntok, bool own_router) const {
         const float E = (float)cfg.n_expert, share = (float)cfg.top_k / E, n = (float)ntok, weights = (float)cfg.hidden * (float)cfg.ffn / (2048.0f * 512.0f);
         const float distinct = E * (1.0f - powf(1.0f - share, n));
         const float passes = 0.5f * (n * (float)cfg.top_k + 0.5f * E * (1.0f - powf(1.0f - 2.0f * share, n)));      // (half the pairs, and half a pass for every odd one out)
         const float launches = (fused ? 19.5f : gu_type == T_IQ1_M ? 22.5f : dn_type == T_IQ3_S ? 26.5f : 27.0f) - (own_router ? 0.0f : 2.2f);
-        return passes * (0.075f + 0.255f * weights) + n * (fused ? 0.22f : 0.57f) <= launches + fmaxf(distinct, 32.0f) * (0.055f + 0.205f * weights);      // (fewer experts do not fill the tiles' launches)
+        const float decoded = fminf(fmaxf(distinct, 32.0f), 64.0f) + 0.7f * fmaxf(distinct - 64.0f, 0.0f);      // (fewer than 32 experts do not fill the tiles' launches)
+        return passes * (0.075f + 0.255f * weights) + n * (fused ? 0.22f : 0.57f) <= launches + decoded * (0.055f + 0.205f * weights);
     }
     uint32_t slices_own = 0, slices_given = 0;      // batches of up to so many tokens run as slices (set at creation)
     uint32_t slices_up_to(bool own_router) const { return own_router ? slices_own : slices_given; }

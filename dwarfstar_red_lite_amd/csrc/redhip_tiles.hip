@@ -18,8 +18,8 @@
 // columns, and adds the waves' sums up in LDS; the 512 columns of a down tile fit the LDS, so there every wave has whole rows and nothing
 // is added up (with whole rows and the activations of 2048 columns passing through LDS block by block, gate/up took 171 instead of 144 us).
 // The SwiGLU activations go to the down kernel as f32, so work is cut at any unit, not at groups of columns that share an exponent.
-// 512 raw IQ2_XXS experts of 2048 x 512 with ten pairs each: gate/up 144 us (sixteen waves of one block, and the decode on full instruction rate
-// only: 166), down 83 (99, activations in registers too); 77 tokens of IQ1_M layers 96 + 48 (112 + 68).
+// 512 raw IQ2_XXS experts of 2048 x 512 with ten pairs each: gate/up 130 us (small tiles as full ones 144; sixteen waves of one block, and the decode on full
+// instruction rate only: 166), down 74 (83; 99, activations in registers too); 77 tokens of IQ1_M layers 70 + 40 (96 + 48; 112 + 68).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -681,16 +681,13 @@ __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) v
     // pipeline, 4 to 8 us behind all the rest (batch of 24 tokens, gate/up: ends at 41.6 us, the others at 34.4 on average). A unit of another tile takes 1.25
     // to 1.6 times as long as a small one's: gate/up, 2048 columns 2.10 and 1.61 us IQ2_XXS, 1.95 and 1.46 IQ1_M, 2.43 and 1.96 IQ2_XS, 1024 columns 2.07 and
     // 1.39; with popular experts, whose rows are at hand, 1.70 and 1.17; down 0.51 and 0.42, 0.49 and 0.38, 0.61 and 0.53, popular 0.48 and 0.45. Parts
-    // are too few for that: six a workgroup, five or seven of which would last longer; there whole rounds are dealt.
+    // are too few for that: four to six a workgroup, one more of which lasts longer (150 tokens of 2048 x 768: 158 us undivided, 161 divided by whole rounds).
     const uint32_t w_big = n_big * per_tile, w_small = (n_tiles - n_big) * per_tile;
     uint32_t g_big = 0u;                                   // workgroups of the others; G: no such parting (no small tiles, or none but these)
     if (SETS == 2 || !w_small) g_big = G;
-    else if constexpr (DOWN && down_tiles_a_pass<SETS, KP>() == 1u) {
-        const uint32_t rounds = (w_big + w_small + G - 1u) / G;
-        g_big = (w_big + rounds - 1u) / rounds;
-        if (g_big + (w_small + rounds - 1u) / rounds > G) g_big = G;
-    } else if (w_big) {
-        constexpr float kCost = DOWN ? 1.15f : KP == 8u ? 1.35f : 1.45f;
+    else if constexpr (DOWN && down_tiles_a_pass<SETS, KP>() == 1u) g_big = G;
+    else if (w_big) {
+        constexpr float kCost = DOWN ? 1.15f : KP == 8u ? 1.3f : 1.45f;
         const float big = kCost * (float)w_big, small = (float)w_small;
         const uint32_t g = min(max((uint32_t)((float)G * big / (big + small)), 1u), G - 1u), more = min(g + 1u, G - 1u);
         const auto longest = [&](uint32_t n) { return fmaxf(big / (float)n, small / (float)(G - n)); };

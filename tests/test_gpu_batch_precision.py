@@ -9,6 +9,8 @@ import pytest
 from dwarfstar_red_lite_amd import moe as moe_api
 from dwarfstar_red_lite_amd import synth
 from dwarfstar_red_lite_amd.moe import ResidentMoe
+from test_gpu_batch_lines import on_tiles
+from test_gpu_staged_tiles import routing_with
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -59,10 +61,41 @@ def test_tiles_against_slices(layout, hidden, ffn, golden_dir):
     assert slices <= 2.1e-7 and tiles <= slices, (slices, tiles)      # (2.1e-7: what f32 products of such a layer give)
 
 
+# Where many experts are named nearly every tile has one to eight pairs, whose high and low halves are rows of one operand and are rounded apart. (16 tokens are
+# slices with the routing given, ten a token of 128 experts.)
+@pytest.mark.parametrize("layout,ffn", [("iq2", 512), ("f2", 512), ("xs", 512), ("m", 512), ("iq2", 768)])
+def test_small_tiles_against_slices(layout, ffn, golden_dir):
+    if layout in ("m", "xs"):
+        g = json.load(open(os.path.join(golden_dir, "iq_grids.json")))
+        moe_api.set_codebooks(*(np.frombuffer(bytes.fromhex(g[k]), np.int8) for k in ("iq2_xs", "iq1_m")))
+    hidden, E, K = 2048, 128, 10
+    cfg = synth.layer_config(hidden=hidden, ffn=ffn, n_expert=E, top_k=K, layout=layout)
+    err, norm = np.zeros(2), 0.0
+    lay = synth.make_layer(7, cfg)
+    lay["sh_down"] = np.zeros_like(lay["sh_down"])      # the routed experts alone
+    m = ResidentMoe(cfg, n_layer=1, max_tokens=32)
+    m.load_layer(0, lay)
+    for seed in range(6):
+        rng = np.random.default_rng(200 + seed)
+        x = torch.from_numpy(synth.normed_x(rng, 32, hidden)).cuda()
+        ids = routing_with([8] * 8 + [7] * 8 + [6] * 8 + [2] * 48 + [1] * 56, 32, K, rng)
+        ids = torch.from_numpy(ids.astype(np.int32)).cuda()
+        w = torch.from_numpy((rng.random((32, K)) + 0.1).astype(np.float32)).cuda()
+        want = routed_in_double(lay, cfg, x[:16], ids[:16], w[:16])
+        for i, n in enumerate((16, 32)):
+            got, tiles = on_tiles(lambda: m.experts(0, x[:n].contiguous(), ids[:n].contiguous(), w[:n].contiguous())[:16])
+            assert tiles == (n == 32)
+            err[i] += float((torch.from_numpy(got).cuda().to(torch.float64) - want).square().sum())
+        norm += float(want.square().sum())
+    m.close()
+    slices, tiles = np.sqrt(err / norm)
+    print("%s 2048 x %d, small tiles: slices %.3e, tiles %.3e" % (layout, ffn, slices, tiles))
+    assert slices <= 2.1e-7 and tiles <= slices, (slices, tiles)
+
+
 # where 32 tokens with the routing given would be further off on the tiles than as slices, 24 still are slices, however few the experts
 @pytest.mark.parametrize("layout", ["iq2", "f2", "xs"])
 def test_small_experts_stay_slices(layout, golden_dir):
-    from test_gpu_batch_lines import on_tiles
     if layout == "xs":
         g = json.load(open(os.path.join(golden_dir, "iq_grids.json")))
         moe_api.set_codebooks(*(np.frombuffer(bytes.fromhex(g[k]), np.int8) for k in ("iq2_xs", "iq1_m")))

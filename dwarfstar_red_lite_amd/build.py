@@ -11,7 +11,7 @@ OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libredmetal_hip.so")
 SOURCES = ["redhip_kernels.hip", "redhip_fused.hip", "redhip_prefill.hip", "redhip_tiles.hip", "redhip_token.hip", "redhip_pool_abi.hip", "redhip_moe_abi.hip",
            "redhip_gguf.hip", "redhip_profile.hip", "redhip_topk_abi.hip"]
-# -packed-fp32-ops off: v_pk_*_f32 forms are not used on this pool of machines
+# -packed-fp32-ops off: some v_pk_*_f32 forms have given wrong results now and then, so none are made
 # -amdgpu-kernarg-preload-count: the leading scalar / pointer arguments of a kernel (up to 14 dwords) are handed to every wave in
 # registers at its start instead of being fetched from the argument block in memory; the latency-bound kernels name what their first
 # requests need in leading arguments for this reason (one-token layer 16.4 -> 15.5 us)

@@ -146,13 +146,15 @@ struct Moe {
     // slices': both by the tokens' expected spread over the experts. Fitted to 1332 calls timed on both sides: 17 .. 32 tokens, 16 to 512 experts,
     // two to ten a token, 1024 x 512 to 2048 x 768, own router and routing given (that call does not know how it is spread: a line between even
     // spread and 32 hot experts), and 746 more of 10 .. 32 tokens once small tiles cost half their matrix instructions. Beyond 64 experts one more costs the
-    // tiles 0.7 of one below: with fewer, workgroups wait for the longest run. Slices / tiles, us:
+    // tiles 0.7 of one below: that is the fit's, no cause of it was measured, and the fit is over all of these calls: single ones lie on the slower side (60 experts,
+    // two a token, 32 tokens with IQ3_S down stay slices at 60 us, tiles 52; 300 experts, six a token, 20 tokens on hot experts given stay slices at 45, tiles 40). Slices / tiles, us:
     // own router, 2048 x 512: 512 experts, ten a token: 16 tokens IQ2_XXS 73 / 72, IQ1_M 79 / 74, IQ3_S down 80 / 81; 18 tokens 80 / 75, 89 / 76 and 88 / 83; 24 tokens
     //   97 / 85, 108 / 86 and 109 / 93; four a token, 28 tokens 67 / 69, 79 / 65 and 79 / 70; 60 experts, two a token, 32 tokens 45 / 49, 61 / 48 and 60 / 52;
     //   32 experts, eight a token, 18 tokens 53 / 48, 64 / 58 and 64 / 56
     // given, evenly / on 32 hot experts: 18 tokens of 2048 x 512, 512 experts, ten a token: IQ2_XXS 70 / 67 and 58 / 50; 300 experts, six a token, 20 tokens: 53 / 55
     //   and 45 / 40, IQ3_S down 70 / 66 and 58 / 50, IQ2_XS 73 / 70 and 60 / 51
-    // Narrower experts (1024 x 256: 32 tokens, 96 experts, six a token 48 / 50 .. 52) stay slices.
+    // Narrower experts (1024 x 256: 32 tokens, 96 experts, six a token 48 / 50 .. 52) stay slices, and so do up to 16 tokens of any layer: behind the own router the two
+    // are level there at best for all formats but one (512 experts, ten a token, above: IQ1_M 6 % behind; hot experts given 63 / 56), and fewer experts favour the slices.
     bool slices_ahead(uint32_t ntok, bool own_router) const {
         const float E = (float)cfg.n_expert, share = (float)cfg.top_k / E, n = (float)ntok, weights = (float)cfg.hidden * (float)cfg.ffn / (2048.0f * 512.0f);
         const float distinct = E * (1.0f - powf(1.0f - share, n));
@@ -167,8 +169,8 @@ struct Moe {
         const uint32_t most = !own_router ? kSmallMaxGiven : fused ? kSmallMaxRouted : kSmallMaxMixed;
         const size_t weights = (size_t)cfg.hidden * cfg.ffn;
         if (cfg.ffn < 512u || weights < (size_t)1024u * 512u || !tile_chunk(kSmallMaxRouted)) return most;
-        // (and 1024 x 512 where the tiles are further off from sums in double than the slices, 1.75e-7 against 1.72e-7; behind the own router of a mixed
-        // layout they are not, with the tiles' router)
+        // (and 1024 x 512 where the tiles are further off from sums in double than the slices: IQ2_XXS 1.726e-7 against 1.714e-7, IQ2_XS 1.713e-7 against 1.704e-7,
+        // F2 level, 1.711e-7 against 1.716e-7; IQ1_M is nearer, 1.690e-7 against 1.714e-7, and behind the own router of a mixed layout they are not further, with the tiles' router)
         if (weights < (size_t)2048u * 512u && (fused || (!own_router && gu_type != T_IQ1_M))) return most;
         uint32_t n = kSmallMaxFused;
         while (n < most && slices_ahead(n + 1u, own_router)) ++n;

@@ -650,10 +650,13 @@ __device__ __forceinline__ void down_items(const StagedArgs &a, const TileList &
 // A launch that finds few wide tiles leaves them: the narrow one then takes every pair in tiles of 16 (list 0). Two launches where one would
 // do cost 10 to 20 us (tables, the first tiles' activations, compute units without work at both ends); a wide tile saves a second decoding
 // of its rows, which goes with their weights. So the line is a number of weights in wide tiles: 290 million for gate/up, 200 million for
-// down. Whole chunks measured with and without, by weights in wide tiles: gate/up of 235 to 268 million (512 tokens, Zipf-popular or 32 pairs
-// per expert) 7 to 12 us slower with them, 262 million (250 tiles of 1024 x 512) 0 to 4 us quicker, 315 million 15 us quicker, one of 1000 million
-// 20 to 60 us quicker; down of 117 million 5 to 8 us slower, 131 to 157 million 1 to 3 us slower, 230 million 4 us quicker, 500 million 6 to
-// 24. Wide down tiles of three blocks, and of four IQ3_S ones, fit the LDS beside small tables only; even so 2048 x 768, 128 experts, eight a token, raw
+// down, fitted while a tile of up to eight pairs cost as much as one of sixteen. Whole chunks since, us, by the line / never wide / wide wherever there are any:
+//   gate/up  2048 x 768, 128 experts, eight a token: IQ2_XXS 300 tokens 160 / 149 / 160, 400 164 / 167 / 162, 700 246 / 252 / 245; F2 300 208 / 208 / 218, 512 297 / 292 / 298
+//            1024 x 512, 200 experts, eight a token: IQ2_XXS 500 tokens 106 / 106 / 115, F2 700 151 / 152 / 162, IQ1_M 1000 183 / 182 / 194
+//            2048 x 512, 512 experts, ten a token, Zipf: IQ2_XXS 512 tokens 232 / 236 / 233, 800 284 / 290 / 281; F2 512 266 / 264 / 272; own router, F2 1024 405 / 412 / 410
+//   down     the same: 300 F2 208 / 206 / 214; 500 106 / 106 / 112, 700 F2 151 / 152 / 157; Zipf 512 F2 266 / 268 / 273, 1024 F2 405 / 413 / 408
+// (runs of one side differ by 1 to 2 %). It lies right but for chunks whose wide tiles hold few pairs beyond sixteen (the first: 19 an expert), where a full tile
+// and a small one are quicker: 7 % there. Wide down tiles of three blocks, and of four IQ3_S ones, fit the LDS beside small tables only; even so 2048 x 768, 128 experts, eight a token, raw
 // rows take at 2048 tokens 239 us instead of 339 (IQ3_S), 196 / 242 (IQ2_XS), 181 / 191 (IQ1_M), whole calls of the pool 507 / 616, 543 / 595, 471 / 492
 // and 467 / 491 (IQ2_XXS). The other formats' four blocks do not fit, and packed rows gain nothing.
 template <int SRC, bool DOWN, uint32_t KP> constexpr bool has_wide() { return !DOWN || KP <= 2u || (layout<SRC>() == L_RAW && (KP == 3u || fmt<SRC>() == F_IQ3)); }
@@ -680,9 +683,11 @@ __global__ __launch_bounds__((DOWN ? 64u * down_waves(SETS) : kGateUpThreads)) v
     // workgroups are dealt round-robin over the eight XCDs: neighbouring runs (which share tiles) go to one XCD's L2
     const uint32_t G = gridDim.x, at = G % 8u == 0u ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
     // Equal shares of the time, small tiles and others on workgroups of their own: one that went from the others to the small ones began again with an empty
-    // pipeline, 4 to 8 us behind all the rest (batch of 24 tokens, gate/up: ends at 41.6 us, the others at 34.4 on average). A unit of another tile takes 1.25
-    // to 1.6 times as long as a small one's: gate/up, 2048 columns 2.10 and 1.61 us IQ2_XXS, 1.95 and 1.46 IQ1_M, 2.43 and 1.96 IQ2_XS, 1024 columns 2.07 and
-    // 1.39; with popular experts, whose rows are at hand, 1.70 and 1.17; down 0.51 and 0.42, 0.49 and 0.38, 0.61 and 0.53, popular 0.48 and 0.45. Parts
+    // pipeline, 4 to 8 us behind all the rest (batch of 24 tokens, gate/up: ends at 41.6 us, the others at 34.4 on average). A unit of another tile takes 1.24
+    // to 1.49 times as long as a small one's in gate/up and 1.07 to 1.29 times in down: gate/up, 2048 columns 2.10 and 1.61 us IQ2_XXS, 1.95 and 1.46 IQ1_M, 2.43 and
+    // 1.96 IQ2_XS, 1024 columns 2.07 and 1.39; with popular experts, whose rows are at hand, 1.70 and 1.17; down 0.51 and 0.42, 0.49 and 0.38, 0.61 and 0.53, popular
+    // 0.48 and 0.45. No one ratio fits all, so kCost is chosen among these by whole chunks: at 2048 columns 1.3, not 1.45 (F2, 512 tokens Zipf, two layers 521 and 547 us; the same
+    // of IQ2_XXS, its pool chunk, 24 and 77 tokens within 2 %), at 1024 1.45 (150 tokens IQ1_M and 300 IQ2_XXS the same at 1.3); 512 columns as 1024, not measured. Parts
     // are too few for that: four to six a workgroup, one more of which lasts longer (150 tokens of 2048 x 768: 158 us undivided, 161 divided by whole rounds).
     const uint32_t w_big = n_big * per_tile, w_small = (n_tiles - n_big) * per_tile;
     uint32_t g_big = 0u;                                   // workgroups of the others; G: no such parting (no small tiles, or none but these)
